@@ -1,0 +1,8 @@
+#include "dcn_backward_input_host.h"
+
+namespace dcn {
+
+#define INSTANTIATE(T, ND, S) template int backward_input_offset<T, ND, S>(const Geometry&, const S*, const S*, const S*, const S*, T*, T*, void*, size_t, hipStream_t, unsigned, bool*);
+INSTANTIATE(double, 2, double) INSTANTIATE(double, 3, double)
+
+}  // namespace dcn

@@ -1,0 +1,429 @@
+// Host side of the backward pass to input and offset: plans and launches.
+#pragma once
+#include "dcn_host.h"
+
+namespace dcn {
+
+template <typename T>
+int absmax(const T* w, size_t n, float* out, hipStream_t s) {
+    hipLaunchKernelGGL(fill_zero_kernel<float>, dim3(1), dim3(64), 0, s, out, (size_t)1);
+    if (int rc = check_launch("fill_zero_kernel")) return rc;
+    const unsigned blocks = (unsigned)((n + 1023) / 1024 > 128 ? 128 : (n + 1023) / 1024);
+    hipLaunchKernelGGL(absmax_kernel<T>, dim3(blocks ? blocks : 1), dim3(256), 0, s, w, n, out);
+    return check_launch("absmax_kernel");
+}
+// out[0] = max |w|, out[1] = largest norm over the output channels of a group of an (input channel, tap)
+// column; `out` was cleared by the pack_weight_kernel launched before
+template <typename T>
+int weight_bounds(const Params& P, const T* w, float* out, hipStream_t s) {
+    const size_t cols = (size_t)P.Cg * P.kV;
+    if (P.G > 65535) return fail(DCN_E_ARGUMENT, "more than 65535 convolution groups");
+    hipLaunchKernelGGL(weight_bounds_kernel<T>, dim3((unsigned)((cols + 63) / 64), (unsigned)P.G), dim3(512), 0, s, w, P.M, cols, out);
+    return check_launch("weight_bounds_kernel");
+}
+
+// S = T: the float32 / float64 operator.  S = Bf16 / Fp16 (T = float): input, weight, offset and
+// grad_output are in that storage format (the gradients are float), and only the fused kernel with
+// its grad_output operand in registers serves them, on the 16-bit matrix instructions; where it
+// cannot, *declined is set and nothing is launched: the caller then widens the tensors and runs the
+// float32 operator.
+template <typename T, int ND, typename S>
+int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* off, const S* gout, T* gin,
+                          T* goff, void* ws, size_t ws_bytes, hipStream_t s, unsigned flags, bool* declined) {
+    constexpr bool S16 = !std::is_same<S, T>::value;
+    Params P;
+    if (int rc = validate(g, P)) return rc;
+    if (flags & ~(unsigned)(DCN_FLAG_OOB_OFFSET_GRAD_ZERO | FLAG_INPUT_ONLY)) return fail(DCN_E_ARGUMENT, "unknown flag");
+    if (int rc = device_info(nullptr)) return rc;
+    P.oob_zero = (flags & DCN_FLAG_OOB_OFFSET_GRAD_ZERO) ? 1 : 0;
+    // grad_input alone (the plain convolution's backward-to-input, which is not given the input): the
+    // scatter kernels need no input values; `goff` is then scratch for the one kernel that writes it anyway
+    const bool input_only = (flags & FLAG_INPUT_ONLY) != 0;
+    if ((!in && !input_only) || !w || !off || !gout || !gin || !goff) return fail(DCN_E_ARGUMENT, "null tensor pointer");
+    bwd_data_weight_pad<T>(P.M, P.Cg, P.Mp, P.Cgp);
+    const size_t wbytes = bwd_data_weight_bytes<T>(P.M, P.Cg, P.kV, P.G, P.cpg);
+    const size_t tbytes = align256((size_t)P.N * P.C_in * P.inV * sizeof(T));
+    if (!ws || ws_bytes < wbytes + 2 * tbytes) return fail(DCN_E_WORKSPACE, "workspace too small");
+    S* wt = static_cast<S*>(ws);
+    T* in_cl = reinterpret_cast<T*>(static_cast<char*>(ws) + wbytes);
+    T* gin_cl = reinterpret_cast<T*>(static_cast<char*>(ws) + wbytes + tbytes);
+    const int TN = Mma<T>::TN;
+    const int mk = bwd_data_mk<T>(P.M);
+    // weight bounds (two floats) and, 64 bytes further, the plan chosen on the device: in the last whole
+    // 256-byte block of the workspace when that lies behind the two channels-last regions
+    // (dcn_workspace_bytes counts it), else at the start of the channels-last gradient, which the LDS
+    // paths do not use
+    const size_t tail_at = ws_bytes >= 256 ? (ws_bytes - 256) / 256 * 256 : 0;
+    const bool tail_words = tail_at >= wbytes + 2 * tbytes;
+    float* wmax = tail_words ? reinterpret_cast<float*>(static_cast<char*>(ws) + tail_at) : reinterpret_cast<float*>(gin_cl);
+    const dim3 tgrid((P.inV + 31) / 32, (unsigned)(P.C_in + 31) / 32, (unsigned)P.N), tblock(32, 8);
+
+    // 1) one kernel: scatter privatised in LDS + coordinate gradient from an LDS input halo
+    // A halo of up to FUSED_HS cells gets the variant with that compile-time plane stride (the four
+    // planes of either kind then lie within the 64 KB reach of an LDS instruction's offset field).
+    // Eight wavefronts per workgroup; four (half the positions, in the block shape with the smallest
+    // halo) where only that fits, e.g. under stride 2.
+    constexpr int FUSED_HS = sizeof(T) == 4 ? 2720 : 2112;
+    constexpr int FUSED_HS8 = 2016;     // plane stride of the 8-channel float instantiation with compile-time halo extents
+    using Kern = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const S*, const S*, const float*, T*, T*, int, unsigned, int);
+    struct FusedPlan {
+        Params Ph;
+        Kern kern;
+        int nw, cch, csplit, goff_atomic;
+        bool zero_goff;
+        bool wide;
+        long long whole, items, slots;
+        size_t lds;
+        const S* wt;
+    };
+    const int seg = P.cpg < P.Cg ? P.cpg : P.Cg;
+    // Plans the fused kernel for a halo of margin m; false when none of its shapes fits.
+    // (attempts: eight wavefronts on the default block, eight on the block shape with the smallest
+    // halo, four on the block shape with the smallest halo)
+    auto plan_fused = [&](int m, FusedPlan& fp) {
+        for (int attempt = fused_first_waves() == 8 ? 0 : 2; attempt < 3; ++attempt) {
+            const int nw = attempt < 2 ? 8 : 4;
+            const bool smallest = attempt > 0;
+            Params Ph = P;
+            // float32: two channels per LDS cell as 32-bit fixed point while the terms one cell can receive
+            // (positions of the block x taps) leave at least 17 bits below the largest possible term
+            const bool pair = sizeof(T) == 4 && fused_pair() && (long long)nw * TN * P.kV <= (1 << 14);
+            const size_t chb = (pair ? 4 : 8) + sizeof(T);      // LDS bytes per channel and halo voxel: cell + input value
+            // Channels per chunk: 8 where that takes fewer MFMA passes per channel (a pass holds TN / CCH
+            // taps: the 9 taps of a 3x3 kernel are 2 float passes per 4 channels or 3 per 8; the 27 of a
+            // 3x3x3 kernel 4 or 7) and the planes of 8 channels fit: the small halos of 2-D layers, and
+            // 3-D ones with paired cells.  16 (2-D, float, paired cells): two taps per pass -- the 9 taps of
+            // a 3x3 kernel are 5 passes per 16 channels instead of 6.  The float kernel with 8 channels
+            // per chunk keeps the input values bank-swizzled and wants the innermost halo extent a
+            // multiple of the four-channel groups per voxel.
+            auto passes = [&](int c) { const int tp = Mma<T>::TN / c; return (P.kV + tp - 1) / tp; };
+            int cch = 0;
+            size_t tables = 0;
+            bool fixed = false, special = false;
+            for (int cand = 16; cand >= 4 && !cch; cand /= 2) {
+                if (cand >= 8 && !((ND == 2 || pair) && nw == 8 && fused_chunk8() && seg >= 8 && passes(8) * 4 < passes(4) * 8)) continue;
+                if (cand == 16 && !(ND == 2 && pair && fused_chunk16() && seg >= 16 && passes(16) * 8 < passes(8) * 16)) continue;
+                Params Pc = P;
+                const int wmult = cand == 16 ? 1 : cand == 8 ? swizzle_groups<T, 8>() : 1;
+                if (!plan_halo<T, ND>(Pc, scatter_budget(), m, 8, chb, nw, smallest, 0, nullptr, wmult)) continue;
+                const size_t tb = (size_t)Pc.hvol * 4;      // halo table
+                if ((long long)Pc.N * Pc.tiles * Pc.DG * 4 > 0x7fffffffLL) continue;
+                if (cand >= 8) {
+                    if ((scatter_budget() - tb) / ((size_t)Pc.hstride * chb) < (size_t)cand) continue;
+                } else {
+                    // A halo of up to FUSED_HS cells gets the variant with that compile-time plane stride
+                    fixed = fused_fixed_stride() && Pc.hvol <= FUSED_HS && (size_t)4 * FUSED_HS * chb + tb <= scatter_budget();
+                    if (!fixed && (scatter_budget() - tb) / ((size_t)Pc.hstride * chb) < 4) continue;
+                }
+                Ph = Pc;
+                tables = tb;
+                cch = cand;
+            }
+            if (!cch) continue;
+            const bool sixteen = cch == 16, eight = cch >= 8;
+            Ph.cchunk = cch;
+            if (fixed && !eight) Ph.hstride = FUSED_HS;
+            // grad_output operand held in registers when its reduction steps fit: 32 per pass
+            // (M <= 64 float, 128 double with 4-channel chunks)
+            // (16-bit storage: a reduction step takes 8 output channels and an operand batch half as many steps)
+            const int KS = GcolGemm<T, S>::KS, halve = S16 ? 2 : 1;
+            const int ksteps = (P.M + KS - 1) / KS;
+            const bool wide = eight && !sixteen && pair && ksteps <= 32 / halve;                     // the kernel's WIDE
+            const int slot_regs = (wide || sixteen) ? 8 : (Mma<T>::row(1, 0) - Mma<T>::row(0, 0) == 1) ? 4 : cch / 4;      // the kernel's RPS
+            const bool breg = ksteps <= Mma<T>::NACC / slot_regs * ((wide || sixteen) ? 16 : 8) / halve;
+            // float, 4-channel chunks: a second set of 32 registers takes the operand of up to 128 output channels (16-bit: 256)
+            const bool breg2 = sizeof(T) == 4 && !eight && !breg && ksteps <= 64 / halve && fused_breg2();
+            special = ND == 3 && eight && !sixteen && pair && wide && breg && fused_fixed_stride() && Ph.hext[1] == 14 && Ph.hext[2] == 14 &&
+                      Ph.hstride <= FUSED_HS8;
+            if (special) Ph.hstride = FUSED_HS8;
+            const size_t lds = (size_t)cch * Ph.hstride * chb + tables;
+            Kern kern = nullptr;
+#define DCN_FUSED_C(CCH_, BREG_, HS_, NW_, PAIR_) backward_input_halo_kernel<T, ND, CCH_, true, (BREG_) || S16, HS_, NW_, true, PAIR_, 1, 0, 0, S>
+#define DCN_FUSED_B2(HS_, NW_, PAIR_) backward_input_halo_kernel<T, ND, 4, true, true, HS_, NW_, true, PAIR_, 2, 0, 0, S>
+            auto pick = [&](auto pair_tag) {
+                constexpr bool PR = decltype(pair_tag)::value;
+                if (sixteen) {
+                    if constexpr (ND == 2 && PR && sizeof(T) == 4) kern = breg ? DCN_FUSED_C(16, true, 0, 8, PR) : DCN_FUSED_C(16, false, 0, 8, PR);
+                } else if (eight) {
+                    if constexpr (ND == 2 || PR) kern = breg ? DCN_FUSED_C(8, true, 0, 8, PR) : DCN_FUSED_C(8, false, 0, 8, PR);
+                    // the halo of a 3x3x3 kernel at stride 1 and margin 2 under the default block of positions:
+                    // inner extents 14 x 14 and the plane stride fixed at compile time
+                    if constexpr (ND == 3 && PR && sizeof(T) == 4) {
+                        if (special) kern = backward_input_halo_kernel<T, ND, 8, true, true, FUSED_HS8, 8, true, true, 1, 14, 14, S>;
+                    }
+                } else if (breg2) {
+                    if constexpr (sizeof(T) == 4) {
+                        if (nw == 8) kern = fixed ? DCN_FUSED_B2(FUSED_HS, 8, PR) : DCN_FUSED_B2(0, 8, PR);
+                        else kern = fixed ? DCN_FUSED_B2(FUSED_HS, 4, PR) : DCN_FUSED_B2(0, 4, PR);
+                    }
+                } else if (nw == 8)
+                    kern = fixed && breg ? DCN_FUSED_C(4, true, FUSED_HS, 8, PR) : fixed ? DCN_FUSED_C(4, false, FUSED_HS, 8, PR) : DCN_FUSED_C(4, false, 0, 8, PR);
+                else
+                    kern = fixed && breg ? DCN_FUSED_C(4, true, FUSED_HS, 4, PR) : fixed ? DCN_FUSED_C(4, false, FUSED_HS, 4, PR) : DCN_FUSED_C(4, false, 0, 4, PR);
+            };
+            if constexpr (sizeof(T) == 4) {
+                if (pair) pick(std::true_type{});
+                else pick(std::false_type{});
+            } else
+                pick(std::false_type{});
+#undef DCN_FUSED_B2
+#undef DCN_FUSED_C
+            if (!kern) continue;
+            if (S16 && !breg && !breg2) continue;       // 16-bit operands come from registers only
+            // Work items are (tile, deformable group) pairs, each a run of nchunks channel chunks.  `slots`
+            // workgroups run at once, so the items take whole rounds plus a partly filled last one.  Either
+            // every item is split over 1, 2 or 4 workgroups (workgroup cz takes every csplit-th chunk), or
+            // the items of the whole rounds stay unsplit and only those of the last round are split, as
+            // finely as fills the device; they come last in the launch.  A workgroup's fixed part
+            // (grad_output operand, halo table, offsets) costs about a quarter of a chunk, which the
+            // estimate charges per split.  The workgroups that share an item add their grad_offset parts with
+            // float atomics on a zero-filled buffer; the only owner of an item stores running sums.
+            const int nchunks = (seg + cch - 1) / cch;
+            const long long items = (long long)Ph.N * Ph.tiles * Ph.DG;
+            const long long slots = forced_slots() ? forced_slots() : resident_workgroups(reinterpret_cast<const void*>(kern), nw * 64, lds);
+            auto item_cost = [&](double chunks_per_wg, int wgs) { return wgs * (chunks_per_wg + 0.25) / nchunks; };
+            int csplit = 1;
+            long long whole = 0;                              // unsplit items at the start of the launch
+            double best = 1e30;
+            for (int cs = 1; cs <= 4 && cs <= nchunks; cs *= 2) {
+                const double rounds = (double)((items * cs + slots - 1) / slots) / cs * item_cost((double)nchunks / cs, cs);
+                if (rounds < best) { best = rounds; csplit = cs; }
+            }
+            if (fused_tail_split() && items > slots && items % slots) {
+                const long long rest = items % slots;
+                const long long cs = slots / rest < nchunks ? slots / rest : nchunks;
+                if (cs >= 2) {
+                    const double rounds = (double)(items / slots) * item_cost(nchunks, 1) + item_cost((double)((nchunks + cs - 1) / cs), 1);
+                    if (rounds < best) { best = rounds; csplit = (int)cs; whole = items - rest; }
+                }
+            }
+            if (forced_csplit()) { csplit = forced_csplit(); whole = 0; }
+            if (csplit > nchunks) csplit = nchunks;
+            if (whole + (items - whole) * csplit > 0x7fffffffLL) continue;
+            fp.Ph = Ph; fp.kern = kern; fp.nw = nw; fp.cch = cch; fp.csplit = csplit;
+            // grad_offset over the chunks of an item that one workgroup owns: the running sum through plain
+            // loads and stores in the 3-D kernels (float atomics run at about 3e11 per second over the device,
+            // and a 3x3x3 layer has 81 grad_offset elements per position and chunk); atomics in the 2-D ones
+            fp.goff_atomic = ND == 2 && nchunks > 1 ? 1 : 0;
+            fp.zero_goff = fp.goff_atomic || csplit > 1;
+            fp.wide = wide; fp.whole = whole; fp.items = items; fp.slots = slots; fp.lds = lds; fp.wt = nullptr;
+            return true;
+        }
+        return false;
+    };
+    FusedPlan fp[MAX_PLANS];
+    int margins[MAX_PLANS];
+    const int nmargins = plan_margins(ND, margins);
+    if (S16 && !(scatter_in_lds() && fused_coord() && !input_only && native16())) {
+        if (declined) *declined = true;
+        return DCN_OK;
+    }
+    if (scatter_in_lds() && fused_coord() && !input_only && plan_fused(margins[0], fp[0])) {
+        // Wider halos for offsets that reach further; the choice is made on the device, see
+        // PlanChoice.  A plan whose weights want another lane order gets a packed copy of its own in
+        // the region of the channels-last input, which this path does not use.
+        PlanChoice pc = {};
+        pc.nplans = 1;
+        pc.nd = ND;
+        pc.margin[0] = margins[0];
+        pc.base[0] = 1.f;
+        pc.far_sample = ND == 3 ? 4.5f : 1.f;       // a sample beyond the halo scatters with global atomics
+        pc.far_steep = ND == 3 ? 25.f : 0.f;        // (c4, margin 2: 3.0, 4.1, 10.4, 26.6 times the time at 49, 70, 87.5, 96 % of the samples beyond the halo)
+        // 3-D: when most samples leave even the widest halo, the path without LDS tiling (coalesced
+        // atomics on a channels-last copy; about 6.5 times the fused kernel's time on small offsets,
+        // whatever the offsets) is the cheaper one: offered as a fourth choice, its kernels launched
+        // behind the fused ones and gated on the choice (DCN_GLOBAL_PLAN=0: not offered)
+        const bool offer_global = !S16 && ND == 3 && tail_words && global_plan() && (long long)P.N * ((P.outV + WAVES * TN - 1) / (WAVES * TN)) <= 0x7fffffffLL &&
+                                  P.DG <= 65535;
+        int copies = 1;                             // packed weight copies
+        fp[0].wt = wt;
+        for (int k = 1; k < nmargins; ++k) {
+            FusedPlan& c = fp[pc.nplans];
+            if (!plan_fused(margins[k], c) || c.Ph.hvol > 3 * fp[0].Ph.hvol) continue;
+            for (int e = 0; e < pc.nplans && !c.wt; ++e)
+                if (fp[e].cch == c.cch && fp[e].wide == c.wide) c.wt = fp[e].wt;
+            if (!c.wt) {
+                if ((size_t)copies * wbytes > tbytes) continue;
+                c.wt = reinterpret_cast<const S*>(reinterpret_cast<const char*>(in_cl) + (size_t)(copies - 1) * wbytes);
+                ++copies;
+            }
+            pc.margin[pc.nplans] = margins[k];
+            // flush, staging and the per-chunk passes grow with the halo: most of the kernel's time in 3-D, little in 2-D
+            // (a quarter more where only the shape with half the wavefronts fits)
+            pc.base[pc.nplans] = (1.f + (ND == 3 ? 0.9f : 0.05f) * ((float)c.Ph.hvol / (float)fp[0].Ph.hvol - 1.f)) * (c.nw < fp[0].nw ? 1.25f : 1.f);
+            ++pc.nplans;
+        }
+        for (int k = pc.nplans; k < MAX_PLANS; ++k) {
+            pc.margin[k] = pc.margin[pc.nplans - 1];
+            pc.base[k] = 1e30f;
+        }
+        unsigned* sel = (pc.nplans > 1 || offer_global) ? reinterpret_cast<unsigned*>(wmax + 16) : nullptr;
+        pc.sel = sel;
+        pc.global_cost = offer_global ? 6.5f : 0.f;
+        const size_t n_off = (size_t)P.N * P.DG * P.kV * ND * P.outV;
+        // weights in the lane order of the kernel's operand loads, one slab per channel chunk; the
+        // first launch clears the weight bounds and chooses the plan
+        for (int k = 0; k < pc.nplans; ++k) {
+            bool packed = false;
+            for (int e = 0; e < k; ++e) packed = packed || fp[e].wt == fp[k].wt;
+            if (packed) continue;
+            const bool sixteen = fp[k].cch == 16, eight = fp[k].cch == 8, wide = fp[k].wide;
+            const size_t total = packed_weight_elems<T, S>(P.M, P.kV, (size_t)(sixteen ? chunk_candidates<16>(P.cpg, P.Cg, P.C_in)
+                                                                            : eight ? chunk_candidates<8>(P.cpg, P.Cg, P.C_in)
+                                                                                    : chunk_candidates<4>(P.cpg, P.Cg, P.C_in)), fp[k].cch);
+            const unsigned blocks = (unsigned)((total + 255) / 256 > 8192 ? 8192 : (total + 255) / 256);
+            PlanChoice pk = pc;
+            if (k > 0) pk.sel = nullptr;
+            float* bounds = k == 0 ? wmax : nullptr;
+            S* dst = const_cast<S*>(fp[k].wt);
+            const dim3 pgrid(blocks + (pk.sel ? 1 : 0));
+            // (wide: row order that leaves the eight channels of a tap in one lane)
+            if (sixteen) hipLaunchKernelGGL((pack_weight_kernel<T, 16, false, S>), pgrid, dim3(256), 0, s, P, w, dst, bounds, pk, off, n_off);
+            else if (wide) hipLaunchKernelGGL((pack_weight_kernel<T, 8, true, S>), pgrid, dim3(256), 0, s, P, w, dst, bounds, pk, off, n_off);
+            else if (eight) hipLaunchKernelGGL((pack_weight_kernel<T, 8, false, S>), pgrid, dim3(256), 0, s, P, w, dst, bounds, pk, off, n_off);
+            else hipLaunchKernelGGL((pack_weight_kernel<T, 4, false, S>), pgrid, dim3(256), 0, s, P, w, dst, bounds, pk, off, n_off);
+            if (int rc = check_launch("pack_weight_kernel")) return rc;
+        }
+        if (int rc = weight_bounds<S>(P, w, wmax, s)) return rc;
+        bool any_atomic = false;
+        for (int k = 0; k < pc.nplans; ++k) any_atomic = any_atomic || fp[k].zero_goff;
+        if (any_atomic) {
+            const size_t nel = (size_t)P.N * P.DG * P.kV * ND * P.outV;
+            const unsigned fb = (unsigned)((nel + 1023) / 1024 > 8192 ? 8192 : (nel + 1023) / 1024);
+            hipLaunchKernelGGL(fill_zero_kernel<T>, dim3(fb), dim3(256), 0, s, goff, nel);
+            if (int rc = check_launch("fill_zero_kernel")) return rc;
+        }
+        // one launch per set of plans that differ in nothing but the halo
+        unsigned launched = 0;
+        for (int k = 0; k < pc.nplans; ++k) {
+            if ((launched >> k) & 1u) continue;
+            // (the kernel takes plan 0 as its Params argument: a launch that does not serve plan 0 gets
+            // the Params of its first plan there, which its mask never selects as such)
+            PlanSet alts;
+            alts.mask = 0;
+            size_t lds = 0;
+            for (int e = 1; e < MAX_PLANS; ++e) alts.alt[e - 1] = halo_plan_of(fp[k].Ph);
+            for (int e = k; e < pc.nplans; ++e) {
+                const bool same = fp[e].kern == fp[k].kern && fp[e].wt == fp[k].wt && fp[e].csplit == fp[k].csplit && fp[e].whole == fp[k].whole &&
+                                  fp[e].items == fp[k].items && fp[e].goff_atomic == fp[k].goff_atomic && fp[e].nw == fp[k].nw &&
+                                  fp[e].slots == fp[k].slots && same_blocks(fp[e].Ph, fp[k].Ph);      // (as many workgroups per CU with the larger LDS)
+                if (!same) continue;
+                if (e > 0) alts.alt[e - 1] = halo_plan_of(fp[e].Ph);
+                alts.mask |= 1u << e;
+                if (fp[e].lds > lds) lds = fp[e].lds;
+            }
+            launched |= alts.mask;
+            if (trace_plans()) {
+                fprintf(stderr, "dcn backward_input_offset: launch for plans %#x: %d wavefronts, %d channels per chunk%s, grid %lld (%lld unsplit, rest x %d), LDS %zu\n",
+                        alts.mask, fp[k].nw, fp[k].cch, fp[k].wide ? " (wide)" : "", fp[k].whole + (fp[k].items - fp[k].whole) * fp[k].csplit, fp[k].whole,
+                        fp[k].csplit, lds);
+                for (int e = 0; e < pc.nplans; ++e)
+                    if ((alts.mask >> e) & 1u)
+                        fprintf(stderr, "  plan %d: margin %d, halo %d x %d x %d, base cost %.3f\n", e, pc.margin[e], fp[e].Ph.hext[0], fp[e].Ph.hext[1],
+                                fp[e].Ph.hext[2], pc.base[e]);
+            }
+            if (lds > 48 * 1024)
+                if (int rc = raise_lds_limit(reinterpret_cast<const void*>(fp[k].kern), lds)) return rc;
+            hipLaunchKernelGGL(fp[k].kern, dim3((unsigned)(fp[k].whole + (fp[k].items - fp[k].whole) * fp[k].csplit)), dim3(fp[k].nw * 64), lds, s,
+                               fp[k].Ph, alts, (const unsigned*)sel, in, off, fp[k].wt, gout, (const float*)wmax, gin, goff, fp[k].csplit, (unsigned)fp[k].whole,
+                               fp[k].goff_atomic);
+            if (int rc = check_launch("backward_input_halo_kernel")) return rc;
+        }
+        if constexpr (!S16) if (offer_global) {
+            // the fourth choice: three launches that return at once unless *sel == MAX_PLANS.  They reuse
+            // the weight region and the channels-last regions, which the fused kernels no longer read then.
+            Params Pg = P;
+            Pg.tiles = (P.outV + WAVES * TN - 1) / (WAVES * TN);
+            const size_t total_w = (size_t)P.G * P.kV * P.Mp * P.Cgp, pad_w = (size_t)TAP_PAD * P.Mp * P.Cgp;
+            const size_t nelem = (size_t)P.N * P.C_in * P.inV;
+            const unsigned nb_w = (unsigned)((total_w + pad_w + 255) / 256 > 1024 ? 1024 : (total_w + pad_w + 255) / 256);
+            const unsigned nb_z = (unsigned)((nelem + 1023) / 1024 > 4096 ? 4096 : (nelem + 1023) / 1024);
+            const size_t ntiles = (size_t)P.N * ((P.C_in + 31) / 32) * ((P.inV + 31) / 32);
+            const unsigned nb_t = (unsigned)(ntiles > 16384 ? 16384 : ntiles);
+            if (trace_plans()) fprintf(stderr, "dcn backward_input_offset: path without LDS tiling offered at cost %.2f\n", pc.global_cost);
+            hipLaunchKernelGGL(global_path_prepare_kernel<T>, dim3(nb_w + nb_z + nb_t), dim3(256), 0, s, Pg, w, wt, pad_w, gin_cl, in, in_cl,
+                               nb_w, nb_z, (const unsigned*)sel, (unsigned)MAX_PLANS);
+            if (int rc = check_launch("global_path_prepare_kernel")) return rc;
+            hipLaunchKernelGGL((backward_data_kernel<T, ND, true, 0>), dim3((unsigned)Pg.N * Pg.tiles, (unsigned)P.DG), dim3(WG), 0, s, Pg,
+                               (const T*)in_cl, off, (const T*)wt, gout, gin_cl, goff, (const unsigned*)sel, (unsigned)MAX_PLANS);
+            if (int rc = check_launch("backward_data_kernel")) return rc;
+            hipLaunchKernelGGL(add_from_channels_last_kernel<T>, tgrid, tblock, 0, s, (const T*)gin_cl, gin, P.C_in, P.inV,
+                               (const unsigned*)sel, (unsigned)MAX_PLANS);
+            if (int rc = check_launch("add_from_channels_last_kernel")) return rc;
+        }
+        return DCN_OK;
+    }
+    if constexpr (S16) {
+        if (declined) *declined = true;
+        return DCN_OK;
+    } else {
+
+    // 2) grad_offset from the channels-last kernel, grad_input from the LDS-privatised scatter
+    if (int rc = relayout<T>(P, w, wt, 1, s)) return rc;
+    {   // zero tap slabs behind the last group
+        const size_t used = (size_t)P.G * P.kV * P.Mp * P.Cgp, pad = (size_t)TAP_PAD * P.Mp * P.Cgp;
+        hipLaunchKernelGGL(fill_zero_kernel<T>, dim3((unsigned)((pad + 255) / 256)), dim3(256), 0, s, wt + used, pad);
+        if (int rc = check_launch("fill_zero_kernel")) return rc;
+    }
+    if (!input_only) {
+        hipLaunchKernelGGL(to_channels_last_kernel<T>, tgrid, tblock, 0, s, in, in_cl, P.C_in, P.inV);
+        if (int rc = check_launch("to_channels_last_kernel")) return rc;
+    }
+    Params Ph = P;
+    bool halo = scatter_in_lds() && plan_halo<T, ND>(Ph, scatter_budget(), default_margin(), 8, 8);
+    if (halo && (long long)Ph.N * Ph.tiles * Ph.DG > 0x7fffffffLL) halo = false;
+    if (halo) {                                     // the scatter kernel packs 4 or 8 channels per MFMA tile
+        const size_t fit = (scatter_budget() - (size_t)Ph.hvol * 4) / ((size_t)Ph.hstride * 8);
+        if (fit >= 8) Ph.cchunk = 8;
+        else if (fit >= 4) Ph.cchunk = 4;
+        else halo = false;
+    }
+    P.tiles = (P.outV + WAVES * TN - 1) / (WAVES * TN);
+    if ((long long)P.N * P.tiles > 0x7fffffffLL || P.DG > 65535)
+        return fail(DCN_E_ARGUMENT, "layer too large for the kernel without the fused LDS halo (more than 65535 deformable groups)");
+    const dim3 grid((unsigned)P.N * P.tiles, (unsigned)P.DG);
+    if (halo) {
+        T* none = nullptr;
+        if (!input_only)
+        switch (mk) {      // register-resident grad_output slab when M is small enough
+            case 8: hipLaunchKernelGGL((backward_data_kernel<T, ND, false, 8>), grid, dim3(WG), 0, s, P, in_cl, off, wt, gout, none, goff); break;
+            case 16: hipLaunchKernelGGL((backward_data_kernel<T, ND, false, 16>), grid, dim3(WG), 0, s, P, in_cl, off, wt, gout, none, goff); break;
+            case 32: hipLaunchKernelGGL((backward_data_kernel<T, ND, false, 32>), grid, dim3(WG), 0, s, P, in_cl, off, wt, gout, none, goff); break;
+            default: hipLaunchKernelGGL((backward_data_kernel<T, ND, false, 0>), grid, dim3(WG), 0, s, P, in_cl, off, wt, gout, none, goff); break;
+        }
+        if (!input_only)
+            if (int rc = check_launch("backward_data_kernel")) return rc;
+        const size_t lds = (size_t)Ph.cchunk * Ph.hstride * 8 + (size_t)Ph.hvol * 4;
+        if (int rc = absmax<T>(w, (size_t)P.C_out * P.Cg * P.kV, wmax, s)) return rc;
+        const dim3 hgrid((unsigned)Ph.N * Ph.tiles * Ph.DG);
+        T* nogoff = nullptr;
+        PlanSet alts;
+        for (int e = 1; e < MAX_PLANS; ++e) alts.alt[e - 1] = halo_plan_of(Ph);
+        alts.mask = 1u;
+        const unsigned* nosel = nullptr;
+        if (Ph.cchunk == 8)
+            return launch_halo(backward_input_halo_kernel<T, ND, 8, false, false, 0, WAVESH>, "backward_input_halo_kernel", hgrid, WGH, lds, s,
+                               Ph, alts, nosel, in, off, (const T*)wt, gout, (const float*)wmax, gin, nogoff, 1, 0u, 0);
+        if (Ph.cchunk == 4)
+            return launch_halo(backward_input_halo_kernel<T, ND, 4, false, false, 0, WAVESH>, "backward_input_halo_kernel", hgrid, WGH, lds, s,
+                               Ph, alts, nosel, in, off, (const T*)wt, gout, (const float*)wmax, gin, nogoff, 1, 0u, 0);
+        return fail(DCN_E_LAUNCH, "no scatter kernel for this channel chunk");
+    }
+    // halo does not fit in LDS: scatter with global atomics on the channels-last copy
+    const size_t nelem = (size_t)P.N * P.C_in * P.inV;
+    const unsigned fblocks = (unsigned)((nelem + 1023) / 1024 > 8192 ? 8192 : (nelem + 1023) / 1024);
+    hipLaunchKernelGGL(fill_zero_kernel<T>, dim3(fblocks), dim3(256), 0, s, gin_cl, nelem);
+    if (int rc = check_launch("fill_zero_kernel")) return rc;
+    if (input_only) {       // the kernel reads input values for the grad_offset it also writes (into scratch here)
+        hipLaunchKernelGGL(fill_zero_kernel<T>, dim3(fblocks), dim3(256), 0, s, in_cl, nelem);
+        if (int rc = check_launch("fill_zero_kernel")) return rc;
+    }
+    hipLaunchKernelGGL((backward_data_kernel<T, ND, true, 0>), grid, dim3(WG), 0, s, P, in_cl, off, wt, gout, gin_cl, goff);
+    if (int rc = check_launch("backward_data_kernel")) return rc;
+    hipLaunchKernelGGL(add_from_channels_last_kernel<T>, tgrid, tblock, 0, s, gin_cl, gin, P.C_in, P.inV);
+    return check_launch("add_from_channels_last_kernel");
+    }
+}
+
+
+}  // namespace dcn

@@ -1,0 +1,8 @@
+#include "dcn_forward_host.h"
+
+namespace dcn {
+
+#define INSTANTIATE(T, ND, S) template int forward<T, ND, S>(const Geometry&, const S*, const S*, const S*, const S*, S*, void*, size_t, hipStream_t, bool*);
+INSTANTIATE(float, 2, float) INSTANTIATE(float, 3, float)
+
+}  // namespace dcn

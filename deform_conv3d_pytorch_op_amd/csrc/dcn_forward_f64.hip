@@ -1,0 +1,8 @@
+#include "dcn_forward_host.h"
+
+namespace dcn {
+
+#define INSTANTIATE(T, ND, S) template int forward<T, ND, S>(const Geometry&, const S*, const S*, const S*, const S*, S*, void*, size_t, hipStream_t, bool*);
+INSTANTIATE(double, 2, double) INSTANTIATE(double, 3, double)
+
+}  // namespace dcn

@@ -1,0 +1,291 @@
+// Host side of the forward pass: plans and launches.
+#pragma once
+#include "dcn_host.h"
+#include "dcn_forward.h"
+
+namespace dcn {
+
+// S = T: the float32 / float64 operator.  S = Bf16 / Fp16 (T = float): the tensors are in that
+// storage format and only the LDS-halo kernel serves them; where it cannot (halo too large, a layer
+// that wants the input-channel split), *declined is set and nothing is launched: the caller then
+// widens the tensors and runs the float32 operator.
+template <typename T, int ND, typename S>
+int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* bias, S* out, void* ws,
+            size_t ws_bytes, hipStream_t s, bool* declined) {
+    constexpr bool S16 = !std::is_same<S, T>::value;
+    Params P;
+    if (int rc = validate(g, P)) return rc;
+    if (!in || !w || !off || !out) return fail(DCN_E_ARGUMENT, "null tensor pointer");
+    if (int rc = device_info(nullptr)) return rc;
+    int MT;
+    fwd_weight_pad<T>(P.M, P.Cg, MT, P.mchunks, P.Mp, P.Cgp);
+    if (!ws || (!S16 && ws_bytes < (size_t)P.G * P.kV * P.Mp * P.Cgp * sizeof(T))) return fail(DCN_E_WORKSPACE, "workspace too small");
+    S* wt = static_cast<S*>(ws);
+    const int TN = Mma<T>::TN;
+    // Too few position blocks to give every CU a workgroup.  First the input channels of a block are
+    // split over up to FWD_MAX_SPLIT workgroups (each samples its own channels once; their partial
+    // outputs are joined by a second kernel), as far as the workspace holds the partial outputs.
+    // Then fewer row tiles per wavefront: more output-channel chunks, each sampling for itself.
+    int fsplit = 1;
+    const int mtiles_all = (P.M + TN - 1) / TN;
+    const size_t out_bytes = (size_t)P.N * P.C_out * P.outV * sizeof(T);
+    const size_t wq_bound = align256(((size_t)chunk_slot<FQ>(P.cpg, P.Cg, P.C_in - 1) + 1) *
+                                     forward_slab_elems<T>(P.kV, (mtiles_all + 7) / 8 * 8 * TN) * sizeof(T));
+    {
+        Params Pt = P;
+        const bool tiled = plan_halo<T, ND>(Pt, 144 * 1024, default_margin(), 1 << 30, sizeof(T), WAVESH, false, FQ);
+        const long long tiles = tiled ? (long long)Pt.N * Pt.tiles : (long long)P.N * ((P.outV + WAVES * TN - 1) / (WAVES * TN));
+        // (eight row tiles per wavefront only pay when the grid is full anyway: measured slower than
+        // four with twice the sampling)
+        if (MT == 8 && tiles * P.G * P.mchunks < cu_count()) {
+            MT = 4;
+            P.mchunks = (mtiles_all + MT - 1) / MT;
+        }
+        if (!S16 && tiled && forward_split() > 1 && (size_t)P.N * P.outV < FWD_SPLIT_POSITIONS && ws_bytes > wq_bound) {
+            const size_t room = ws_bytes - wq_bound < FWD_PARTIAL_CAP ? ws_bytes - wq_bound : FWD_PARTIAL_CAP;
+            while (fsplit * 2 <= FWD_MAX_SPLIT && fsplit * 2 <= forward_split() && tiles * P.G * P.mchunks * fsplit * 2 <= cu_count() &&
+                   (size_t)fsplit * 2 * out_bytes <= room && fsplit * 2 * 16 <= P.Cg)      // at least 16 channels per part
+                fsplit *= 2;
+        }
+        while (MT > 1 && tiles * P.G * P.mchunks * fsplit < cu_count()) {
+            MT /= 2;
+            P.mchunks = (mtiles_all + MT - 1) / MT;
+        }
+        P.Mp = P.mchunks * MT * TN;
+    }
+    // Halo kernel: four channels of a voxel side by side in LDS (forward_quad_kernel).  Few
+    // accumulators (MT <= 2): one 1024-thread workgroup per CU with the whole LDS, if its larger halo
+    // fits and leaves 8 channels per pass.  Otherwise 512 threads: two workgroups per CU when that
+    // still leaves 8 channels per LDS pass, else one large one.  Returns the wavefronts per
+    // workgroup, 0 when no halo of margin m fits.
+    auto plan_for = [&](int m, Params& Ph) {
+        Ph = P;
+        int nw = 0;
+        // (the 3-D double instance of the 1024-thread shape does not fit its 128 registers)
+        if (MT <= 2 && wide_forward() && !(sizeof(T) == 8 && ND == 3)) {
+            Params Pw = P;
+            if (plan_halo<T, ND>(Pw, 144 * 1024, m, 1 << 30, sizeof(T), 16, false, FQ) &&
+                (long long)Pw.N * Pw.tiles * Pw.G * Pw.mchunks <= 0x7fffffffLL &&
+                (wide_forward() == 2 || (Pw.cchunk >= 8 && (long long)Pw.N * Pw.tiles * Pw.G * Pw.mchunks >= cu_count()))) {
+                Ph = Pw;
+                nw = 16;
+            }
+        }
+        if (!nw) {
+            bool tiled = plan_halo<T, ND>(Ph, LDS_BUDGET, m, 1 << 30, sizeof(T), WAVESH, false, FQ);
+            if ((!tiled || Ph.cchunk < 8) && LDS_BUDGET < 144 * 1024)
+                tiled = plan_halo<T, ND>(Ph, 144 * 1024, m, 1 << 30, sizeof(T), WAVESH, false, FQ) || tiled;
+            if (!tiled || Ph.cchunk < 8) {       // strided layers: the block shape with the smallest halo may hold 8 channels
+                Params Ps = P;
+                if (plan_halo<T, ND>(Ps, 144 * 1024, m, 1 << 30, sizeof(T), WAVESH, true, FQ) && (!tiled || Ps.cchunk > Ph.cchunk)) {
+                    Ph = Ps;
+                    tiled = true;
+                }
+            }
+            if (tiled && (long long)Ph.N * Ph.tiles * Ph.G * Ph.mchunks <= 0x7fffffffLL) nw = WAVESH;
+        }
+        return nw;
+    };
+    {
+        int margins[MAX_PLANS];
+        const int nmargins = plan_margins(ND, margins);
+        Params plans[MAX_PLANS];
+        const int nw = plan_for(margins[0], plans[0]);
+        const size_t slabs = (size_t)chunk_slot<FQ>(P.cpg, P.Cg, P.C_in - 1) + 1;
+        const size_t wq_bytes = slabs * forward_slab_elems<T>(P.kV, P.Mp) * sizeof(S);
+        if (nw == 16 || ws_bytes < align256(wq_bytes) + (size_t)fsplit * out_bytes) fsplit = 1;
+        if (nw && ws_bytes >= wq_bytes) {
+            // channels per LDS pass such that every workgroup of a block gets the same number of passes
+            auto even_passes = [&](Params& Ph) {
+                auto chunks_of_group0 = [&](int cc) {
+                    int n = 0;
+                    for (int dg = 0; dg <= (P.Cg - 1) / P.cpg; ++dg) {
+                        const int len = (P.Cg < (dg + 1) * P.cpg ? P.Cg : (dg + 1) * P.cpg) - dg * P.cpg;
+                        n += (len + cc - 1) / cc;
+                    }
+                    return n;
+                };
+                for (int cc = Ph.cchunk; cc >= FQ; cc -= FQ)
+                    if (chunks_of_group0(cc) % fsplit == 0) { Ph.cchunk = cc; break; }
+            };
+            if (fsplit > 1) even_passes(plans[0]);
+            // Wider halos that one launch of the same kernel can serve as well (same workgroup shape and
+            // position blocks); the choice among them is made on the device, see PlanChoice.  The
+            // chosen index lives in the last 256 bytes of the workspace.
+            PlanChoice pc = {};
+            pc.nplans = 1;
+            pc.nd = ND;
+            pc.margin[0] = margins[0];
+            pc.base[0] = 1.f;
+            // a wavefront with a sample beyond the halo walks every channel of the pass once more, and each
+            // such sample gathers its corners from global memory (fitted to timings at c4 and c3)
+            pc.far_wave = ND == 3 ? 0.5f : 0.1f;
+            pc.far_sample = ND == 3 ? 2.2f : 5.f;
+            const size_t used = align256(wq_bytes) + (fsplit > 1 ? (size_t)fsplit * out_bytes : 0);
+            if (nmargins > 1 && ws_bytes >= used + 512) {
+                // (within the LDS of the first plan, which fixes how many workgroups share a CU; all of it
+                // when the grid gives a CU one workgroup at most)
+                const long long wgs = (long long)plans[0].N * plans[0].tiles * plans[0].G * plans[0].mchunks * fsplit;
+                size_t lds0 = (size_t)plans[0].cchunk * plans[0].hstride * sizeof(T) + (size_t)plans[0].hvol * 4;
+                if (wgs <= cu_count() && lds0 < 144 * 1024) lds0 = 144 * 1024;
+                for (int k = 1; k < nmargins; ++k) {
+                    Params& Pk = plans[pc.nplans];
+                    Pk = P;
+                    if (!plan_halo<T, ND>(Pk, lds0, margins[k], 1 << 30, sizeof(T), nw, false, FQ, plans[0].tdim)) continue;
+                    if (!same_blocks(Pk, plans[0]) || Pk.hvol > 3 * plans[0].hvol) continue;
+                    if (fsplit > 1) even_passes(Pk);
+                    pc.margin[pc.nplans] = margins[k];
+                    // staging and the per-pass geometry grow with the halo: about a third of the kernel's time in 3-D, an eighth in 2-D
+                    pc.base[pc.nplans] = 1.f + (ND == 3 ? 0.3f : 0.12f) * ((float)Pk.hvol / (float)plans[0].hvol - 1.f);
+                    ++pc.nplans;
+                }
+                if (pc.nplans > 1) pc.sel = reinterpret_cast<unsigned*>(static_cast<char*>(ws) + (ws_bytes - 256) / 256 * 256);
+            }
+            for (int k = pc.nplans; k < MAX_PLANS; ++k) {
+                plans[k] = plans[0];
+                pc.margin[k] = pc.margin[pc.nplans - 1];
+                pc.base[k] = 1e30f;
+            }
+            PlanSet alts;
+            for (int k = 1; k < MAX_PLANS; ++k) alts.alt[k - 1] = halo_plan_of(plans[k]);
+            alts.mask = (1u << pc.nplans) - 1;
+            {
+                const size_t total = (size_t)chunk_candidates<FQ>(P.cpg, P.Cg, P.C_in) * forward_slab_elems<T>(P.kV, P.Mp);
+                const unsigned blocks = (unsigned)((total + 255) / 256 > 8192 ? 8192 : (total + 255) / 256);
+                const size_t n_off = (size_t)P.N * P.DG * P.kV * ND * P.outV;
+                hipLaunchKernelGGL((pack_forward_weight_kernel<T, S>), dim3(blocks + (pc.sel ? 1 : 0)), dim3(256), 0, s, plans[0], w, wt, pc, off, n_off);
+                if (int rc = check_launch("pack_forward_weight_kernel")) return rc;
+            }
+            size_t lds = 0;
+            for (int k = 0; k < pc.nplans; ++k) {
+                const size_t l = (size_t)plans[k].cchunk * plans[k].hstride * sizeof(T) + (size_t)plans[k].hvol * 4;
+                if (l > lds) lds = l;
+            }
+            const Params& Ph = plans[0];
+            using Kern = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const S*, const S*, S*, T*, int, unsigned, TailSplit);
+            Kern kern;
+            if (nw == 16) kern = MT == 1 ? forward_quad_kernel<T, ND, 1, 16, S> : forward_quad_kernel<T, ND, 2, 16, S>;
+            else kern = MT == 1 ? forward_quad_kernel<T, ND, 1, WAVESH, S> : MT == 2 ? forward_quad_kernel<T, ND, 2, WAVESH, S>
+                      : MT == 4 ? forward_quad_kernel<T, ND, 4, WAVESH, S> : forward_quad_kernel<T, ND, 8, WAVESH, S>;
+            T* part = reinterpret_cast<T*>(static_cast<char*>(ws) + align256(wq_bytes));      // partial sums, in the arithmetic type
+            // A grid that ends in a partly filled round of workgroups: the units of that round, last in
+            // the launch, are split over several workgroups each (every tsplit-th channel pass), so that
+            // the round fills the device; forward_join_tail_kernel adds their partial sums.  Either all
+            // of them tsplit ways, or -- when that leaves the last of the resulting short rounds partly
+            // empty -- as many of them tsplit + 1 ways as make the workgroup count a whole number of
+            // rounds (TailSplit: the units split tsplit ways come first, so that the longer workgroups
+            // start first).  Cost of a workgroup: per channel pass one part for the tap geometry and one
+            // per four channels, plus 5 % of a unit for its fixed part (halo table, offsets, output).
+            const long long units = (long long)Ph.N * Ph.tiles * Ph.G * Ph.mchunks;
+            int tsplit = 1;
+            long long whole = 0;
+            TailSplit ts = {0u, 0, 0};
+            if (fsplit == 1 && forward_tail_split()) {
+                const long long slots = forward_slots() ? forward_slots() : resident_workgroups(reinterpret_cast<const void*>(kern), nw * 64, lds);
+                const long long rest = units % slots;
+                constexpr double GEO = 0.45;    // tap geometry of a pass, in units of four channels' sampling and contraction
+                // cost of the longest workgroup when the passes of a unit (cch channels each) are dealt to cs workgroups
+                auto wg_cost = [&](int cs, int cch, int* npasses) {
+                    double load[64] = {0};
+                    int k = 0;
+                    for (int dg = 0; dg <= (P.Cg - 1) / P.cpg; ++dg) {
+                        const int len = (P.Cg < (dg + 1) * P.cpg ? P.Cg : (dg + 1) * P.cpg) - dg * P.cpg;
+                        for (int c0 = 0; c0 < len; c0 += cch, ++k) load[k % cs] += GEO + (double)(((len - c0 < cch ? len - c0 : cch) + FQ - 1) / FQ);
+                    }
+                    if (npasses) *npasses = k;
+                    double worst = 0;
+                    for (int z = 0; z < cs; ++z) worst = load[z] > worst ? load[z] : worst;
+                    return worst;
+                };
+                int passes = 0;                 // channel passes of a unit under the first plan
+                const double unit_cost = wg_cost(1, Ph.cchunk, &passes);
+                const size_t end = pc.sel ? (ws_bytes - 256) / 256 * 256 : ws_bytes;
+                const size_t room = end > align256(wq_bytes) ? end - align256(wq_bytes) : 0;
+                const size_t per_wg = (size_t)MT * TN * nw * TN * sizeof(T);
+                if (units > slots && rest) {
+                    double best = 0.9;          // of the time of an unsplit last round; a tenth must be gained
+                    for (int cs = 2; cs <= 8 && cs <= passes; ++cs) {
+                        if (forward_tail_split() > 1 && cs != forward_tail_split()) continue;
+                        const long long rounds = (rest * cs + slots - 1) / slots;
+                        const double ta = wg_cost(cs, Ph.cchunk, nullptr) / unit_cost + 0.05;
+                        {
+                            const double t = (double)rounds * ta;
+                            const size_t bytes = (size_t)rest * cs * per_wg;
+                            if ((t < best || forward_tail_split() > 1) && bytes <= room && bytes <= FWD_PARTIAL_CAP) {
+                                best = t; tsplit = cs; ts = TailSplit{0u, 0, 0};
+                            }
+                        }
+                        // two runs: nb units cs + 1 ways, the others cs ways, rounds * slots workgroups in all;
+                        // the cs-way workgroups must fit the first round
+                        const long long nb = rounds * slots - rest * cs;
+                        if (!forward_tail_two_runs() || cs + 1 > 8 || nb <= 0 || nb >= rest || (rest - nb) * cs > slots) continue;
+                        double tb = 1e30;
+                        int cchb = Ph.cchunk;
+                        for (int cch = Ph.cchunk; cch >= FQ; cch -= FQ) {
+                            int np = 0;
+                            const double c = wg_cost(cs + 1, cch, &np) / unit_cost + 0.05;
+                            if (np >= cs + 1 && c < tb) { tb = c; cchb = cch; }
+                        }
+                        const double t = ta + (double)(rounds - 1) * tb;
+                        const size_t bytes = (size_t)(rounds * slots) * per_wg;
+                        if (t < best && bytes <= room && bytes <= FWD_PARTIAL_CAP) {
+                            best = t; tsplit = cs; ts = TailSplit{(unsigned)(rest - nb), cs + 1, cchb};
+                        }
+                    }
+                    if (tsplit > 1) whole = units - rest;
+                }
+            }
+            const long long wgs = tsplit > 1 ? whole + (ts.splitB ? (long long)ts.unitsA * tsplit + (units - whole - ts.unitsA) * ts.splitB : (units - whole) * tsplit)
+                                             : units * fsplit;
+            if (wgs > 0x7fffffffLL) return fail(DCN_E_ARGUMENT, "too many workgroups for one launch");
+            const dim3 grid((unsigned)wgs);
+            if (trace_plans()) {
+                fprintf(stderr, "dcn forward: %d wavefronts, MT %d, grid %u (%lld unsplit, rest x %d), LDS %zu, every unit split x %d\n", nw, MT, grid.x,
+                        tsplit > 1 ? whole : 0LL, tsplit, lds, fsplit);
+                if (ts.splitB) fprintf(stderr, "  of the rest: %u units x %d, the others x %d with %d channels per pass\n", ts.unitsA, tsplit, ts.splitB, ts.cchB);
+                for (int k = 0; k < pc.nplans; ++k)
+                    fprintf(stderr, "  plan %d: margin %d, halo %d x %d x %d, %d channels per pass, base cost %.3f\n", k, pc.margin[k],
+                            plans[k].hext[0], plans[k].hext[1], plans[k].hext[2], plans[k].cchunk, pc.base[k]);
+            }
+            const unsigned* sel = pc.sel;
+            if (int rc = launch_halo(kern, "forward_quad_kernel", grid, nw * 64, lds, s, Ph, alts, sel, in, off, (const S*)wt, bias, out, part,
+                                     tsplit > 1 ? tsplit : fsplit, (unsigned)whole, ts))
+                return rc;
+            if (fsplit == 1 && tsplit == 1) return DCN_OK;
+            if (tsplit > 1) {
+                using Join = void (*)(Params, PlanSet, const unsigned*, const T*, const S*, S*, int, unsigned, TailSplit);
+                Join join;
+                if (nw == 16) join = MT == 1 ? forward_join_tail_kernel<T, ND, 1, 16, S> : forward_join_tail_kernel<T, ND, 2, 16, S>;
+                else join = MT == 1 ? forward_join_tail_kernel<T, ND, 1, WAVESH, S> : MT == 2 ? forward_join_tail_kernel<T, ND, 2, WAVESH, S>
+                          : MT == 4 ? forward_join_tail_kernel<T, ND, 4, WAVESH, S> : forward_join_tail_kernel<T, ND, 8, WAVESH, S>;
+                hipLaunchKernelGGL(join, dim3((unsigned)((units - whole) * (MT * TN / JOIN_ROWS))), dim3(nw * TN), 0, s, Ph, alts, sel, (const T*)part, bias, out, tsplit, (unsigned)whole, ts);
+                return check_launch("forward_join_tail_kernel");
+            }
+            if constexpr (!S16) {
+                const size_t total = (size_t)P.N * P.C_out * P.outV;
+                const unsigned jb = (unsigned)((total + 255) / 256 > 4096 ? 4096 : (total + 255) / 256);
+                hipLaunchKernelGGL(forward_join_partials_kernel<T>, dim3(jb), dim3(256), 0, s, part, bias, out, fsplit, total, P.C_out, P.outV);
+                return check_launch("forward_join_partials_kernel");
+            }
+        }
+    }
+    if constexpr (S16) {
+        if (declined) *declined = true;
+        return DCN_OK;
+    } else {
+    if (int rc = relayout<T>(P, w, wt, 0, s)) return rc;
+    // geometry whose halo does not fit in LDS: gather straight from global memory
+    P.tiles = (P.outV + WAVES * TN - 1) / (WAVES * TN);
+    if ((long long)P.N * P.tiles > 0x7fffffffLL || (long long)P.G * P.mchunks > 65535)
+        return fail(DCN_E_ARGUMENT, "layer too large for the kernel without LDS tiling (groups x output-channel chunks > 65535)");
+    const dim3 grid((unsigned)P.N * P.tiles, (unsigned)P.G * P.mchunks);
+    switch (MT) {
+        case 1: hipLaunchKernelGGL((forward_kernel<T, ND, 1>), grid, dim3(WG), 0, s, P, in, off, wt, bias, out); break;
+        case 2: hipLaunchKernelGGL((forward_kernel<T, ND, 2>), grid, dim3(WG), 0, s, P, in, off, wt, bias, out); break;
+        case 4: hipLaunchKernelGGL((forward_kernel<T, ND, 4>), grid, dim3(WG), 0, s, P, in, off, wt, bias, out); break;
+        default: hipLaunchKernelGGL((forward_kernel<T, ND, 8>), grid, dim3(WG), 0, s, P, in, off, wt, bias, out); break;
+    }
+    return check_launch("forward_kernel");
+    }
+}
+}  // namespace dcn

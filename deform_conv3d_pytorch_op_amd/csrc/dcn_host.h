@@ -1,0 +1,471 @@
+// Host side shared by the translation units of libdcn_amd.so: argument validation, workspace layout,
+// tuning knobs, halo tiling plans, launch helpers, and the operator functions behind the C ABI.
+#pragma once
+#include "../../include/dcn_amd.h"
+#include "dcn_kernels.h"
+#include "dcn_forward.h"
+
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <map>
+#include <mutex>
+#include <string>
+#include <type_traits>
+#include <utility>
+
+namespace dcn {
+
+inline thread_local std::string g_err;
+
+inline int fail(int code, const char* msg) {
+    g_err = msg;
+    return code;
+}
+
+
+// Largest re-laid-out weight any call needs; see relayout_weight_kernel for the two layouts.
+template <typename T> inline void fwd_weight_pad(int M, int Cg, int& MT, int& mchunks, int& Mp, int& Cgp) {
+    const int TN = Mma<T>::TN, KL = Mma<T>::KL;
+    const int mtiles = (M + TN - 1) / TN;
+    MT = mtiles >= 8 ? 8 : (mtiles > 2 ? 4 : mtiles);          // 1, 2, 4 or 8 tiles per wavefront
+    mchunks = (mtiles + MT - 1) / MT;
+    Mp = mchunks * MT * TN;
+    Cgp = Cg + 2 * KL;       // the kernels read up to one reduction step past the last channel
+}
+// backward-data layout.  MK = reduction steps over output channels whose grad_output values
+// backward_data_kernel keeps in registers (0: M too large, the kernel re-reads grad_output per tap).
+template <typename T> inline int bwd_data_mk(int M) {
+    const int steps = (M + Mma<T>::KL - 1) / Mma<T>::KL;
+    for (int mk = 8; mk <= 64; mk *= 2)
+        if (steps <= mk) return mk;
+    return 0;
+}
+template <typename T> inline void bwd_data_weight_pad(int M, int Cg, int& Mp, int& Cgp) {
+    // rows: reduction steps are consumed in batches of 8; the coordinate kernel reads up to KL rows further
+    const int KL = Mma<T>::KL;
+    const int steps = ((M + KL - 1) / KL + 7) / 8 * 8;
+    Mp = steps * KL + KL;
+    const int mk = bwd_data_mk<T>(M) * KL;
+    if (mk > Mp) Mp = mk;
+    Cgp = Cg + Mma<T>::TN;
+}
+inline size_t align256(size_t v) { return (v + 255) / 256 * 256; }
+
+constexpr int TAP_PAD = 8;      // zero tap slabs behind the last group: an MFMA pass may start up to 7 taps before the end
+// Elements of the per-chunk weight slabs of the fused backward kernel (pack_weight_kernel, chunks of
+// `cch` channels) for `slabs` slabs.
+template <typename T, typename S = T> inline size_t packed_weight_elems(int M, int kV, size_t slabs, int cch) {
+    const int TP = Mma<T>::TN / cch;
+    return slabs * ((kV + TP - 1) / TP) * (size_t)gcol_slab_steps<T, S>(M) * 64 * (std::is_same<S, T>::value ? 1 : 4);
+}
+// Upper bound of chunk_slot<cch>(cpg, Cg, c) + 1 over the channels: the slabs a per-chunk weight
+// layout occupies.  cpg = 0: the channels per deformable group are not known (the first workspace
+// query is not told them) and the bound assumes their largest possible number of groups, C_in.
+inline size_t slab_bound(size_t C_in, int G, int cpg, int cch) { return C_in / cch + (cpg > 0 ? C_in / cpg : C_in) + G + 1; }
+// Either weight layout of backward_input_offset fits.
+template <typename T> inline size_t bwd_data_weight_bytes(int M, int Cg, int kV, int G, int cpg = 0) {
+    int Mp, Cgp;
+    bwd_data_weight_pad<T>(M, Cg, Mp, Cgp);
+    const size_t plain = ((size_t)G * kV + TAP_PAD) * Mp * Cgp;
+    const size_t C_in = (size_t)Cg * G;
+    const size_t packed4 = packed_weight_elems<T>(M, kV, slab_bound(C_in, G, cpg, 4), 4);
+    const size_t packed8 = packed_weight_elems<T>(M, kV, slab_bound(C_in, G, cpg, 8), 8);
+    const size_t packed16 = packed_weight_elems<T>(M, kV, slab_bound(C_in, G, cpg, 16), 16);
+    size_t packed = packed4 > packed8 ? packed4 : packed8;
+    if (packed16 > packed) packed = packed16;
+    return align256((plain > packed ? plain : packed) * sizeof(T));
+}
+// Partial outputs of a forward pass that splits the input channels of a position block over several
+// workgroups: only layers of few positions do (too few blocks to fill the device), with at most
+// FWD_MAX_SPLIT parts and FWD_PARTIAL_CAP bytes.
+constexpr int FWD_MAX_SPLIT = 16;
+constexpr size_t FWD_PARTIAL_CAP = (size_t)64 << 20;
+constexpr size_t FWD_SPLIT_POSITIONS = 256 * 512;      // no split from this many positions on: they fill the device anyway
+inline size_t forward_partial_bound(int N, int C_out, size_t outV, size_t elem) {
+    if ((size_t)N * outV >= FWD_SPLIT_POSITIONS) return 0;
+    const size_t all = (size_t)FWD_MAX_SPLIT * N * C_out * outV * elem;
+    return align256(all < FWD_PARTIAL_CAP ? all : FWD_PARTIAL_CAP) + 256;
+}
+template <typename T> inline size_t workspace_need(int N, int C_in, int C_out, size_t inV, size_t outV, int kV, int G, int cpg = 0) {
+    const int M = C_out / G, Cg = C_in / G;
+    int MT, mchunks, Mp, Cgp;
+    fwd_weight_pad<T>(M, Cg, MT, mchunks, Mp, Cgp);
+    // forward: [g][tap][c][m] for the kernel without LDS tiling, or one slab per four channels for the
+    // halo kernel (its row padding is at most eight tiles' worth)
+    const int TNf = Mma<T>::TN;
+    const int Mp8 = ((M + TNf - 1) / TNf + 7) / 8 * 8 * TNf;
+    const size_t fwd_plain = (size_t)G * kV * (Mp > Mp8 ? Mp : Mp8) * Cgp * sizeof(T);
+    const size_t fwd_quad = slab_bound((size_t)C_in, G, cpg, FQ) * forward_slab_elems<T>(kV, Mp8) * sizeof(T);
+    const size_t fwd = (fwd_plain > fwd_quad ? fwd_plain : fwd_quad) + forward_partial_bound(N, C_out, outV, sizeof(T));
+    // (+ the last whole 256-byte block of the workspace: weight bounds and the plan the device chose)
+    const size_t bwd = bwd_data_weight_bytes<T>(M, Cg, kV, G, cpg) + 2 * align256((size_t)N * C_in * inV * sizeof(T)) + 512;
+    // backward_weight: two channels-last copies + one partial weight per position split (at most 256 splits,
+    // and never more than about 4096 workgroups: see bww_plan)
+    const int TNq = Mma<T>::TN;
+    const long long tiles_lb = (long long)kV * ((C_in + TNq - 1) / TNq);           // lower bound of kV * nct * mchunks
+    long long split_ub = (4096 + tiles_lb - 1) / tiles_lb;
+    if (split_ub > 256) split_ub = 256;
+    if (split_ub < 1) split_ub = 1;
+    const size_t bww = align256((size_t)N * C_in * inV * sizeof(T)) + align256((size_t)N * C_out * outV * sizeof(T)) +
+                       align256((size_t)split_ub * kV * C_out * Cg * sizeof(T));
+    size_t need = fwd > bwd ? fwd : bwd;
+    return need > bww ? need : bww;
+}
+
+struct Geometry {   // the reference's argument list, 2-D mapped onto slots 1,2 with a unit length axis
+    int nd, N, C_in, C_out, in[3], out[3], k[3], pad[3], stride[3], dil[3], cpg, G;
+};
+
+// Mirrors shape_check of the reference as far as it can be stated without tensor handles
+// (deform3d/lib/deform_conv3d_cuda.cpp:24-87): the extents must be consistent with each other and
+// with the output-size formula.  Rank and per-tensor size checks live in the Python front end,
+// which owns the tensors.
+inline int validate(const Geometry& g, Params& P) {
+    if (g.N <= 0 || g.C_in <= 0 || g.C_out <= 0) return fail(DCN_E_ARGUMENT, "batch / channel extents must be positive");
+    if (g.G <= 0 || g.C_in % g.G || g.C_out % g.G) return fail(DCN_E_ARGUMENT, "input c != kernel c");
+    if (g.cpg <= 0 || g.C_in % g.cpg) return fail(DCN_E_ARGUMENT, "off channel");
+    static const char* const omsg[3] = {"error output ll", "error outhh", "error outww"};
+    for (int a = 3 - g.nd; a < 3; ++a) {
+        if (g.in[a] <= 0 || g.k[a] <= 0 || g.stride[a] <= 0 || g.dil[a] <= 0 || g.pad[a] < 0)
+            return fail(DCN_E_ARGUMENT, "input / kernel / stride / dilation extents must be positive, pad non-negative");
+        if (g.in[a] + 2 * g.pad[a] - g.k[a] < 0) return fail(DCN_E_ARGUMENT, omsg[a]);
+        // the reference's dilation-blind output size, or the usual dilation-aware one (the sampler
+        // gives every position a meaning, so both are served)
+        const int blind = (g.in[a] + 2 * g.pad[a] - g.k[a]) / g.stride[a] + 1;
+        const int span = g.in[a] + 2 * g.pad[a] - g.dil[a] * (g.k[a] - 1) - 1;
+        const int standard = span >= 0 ? span / g.stride[a] + 1 : 0;
+        if (g.out[a] != blind && !(standard >= 1 && g.out[a] == standard)) return fail(DCN_E_ARGUMENT, omsg[a]);
+    }
+    const long long inV = (long long)g.in[0] * g.in[1] * g.in[2], outV = (long long)g.out[0] * g.out[1] * g.out[2];
+    // per-channel offsets are 32-bit inside the kernels (including a bias of up to 4 channels)
+    if (inV > (1ll << 27) || outV > (1ll << 27)) return fail(DCN_E_ARGUMENT, "a single channel exceeds 2^27 voxels");
+    // channels-last voxel*channel offsets of one sample are 32-bit as well
+    if (inV * g.C_in > (1ll << 31)) return fail(DCN_E_ARGUMENT, "one input sample exceeds 2^31 elements");
+    if (g.N > 65535) return fail(DCN_E_ARGUMENT, "batch exceeds 65535");
+    P.oob_zero = 0;
+    P.nd = g.nd; P.N = g.N; P.C_in = g.C_in; P.C_out = g.C_out; P.G = g.G; P.cpg = g.cpg; P.DG = g.C_in / g.cpg;
+    P.M = g.C_out / g.G; P.Cg = g.C_in / g.G;
+    for (int a = 0; a < 3; ++a) {
+        P.in[a] = g.in[a]; P.out[a] = g.out[a]; P.k[a] = g.k[a];
+        P.pad[a] = g.pad[a]; P.stride[a] = g.stride[a]; P.dil[a] = g.dil[a];
+    }
+    P.inV = (unsigned)inV; P.outV = (unsigned)outV; P.kV = g.k[0] * g.k[1] * g.k[2];
+    P.tiles = P.mchunks = P.Mp = P.Cgp = P.nsplit = P.nctiles = 0;
+    return DCN_OK;
+}
+
+inline int check_launch(const char* what) {
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess) {
+        g_err = std::string(what) + ": " + hipGetErrorString(e);
+        return DCN_E_LAUNCH;
+    }
+    return DCN_OK;
+}
+
+template <typename T>
+inline int relayout(const Params& P, const T* w, T* wt, int channel_fastest, hipStream_t s) {
+    const size_t total = (size_t)P.G * P.kV * P.Mp * P.Cgp;
+    const int blocks = (int)((total + 255) / 256 > 4096 ? 4096 : (total + 255) / 256);
+    hipLaunchKernelGGL(relayout_weight_kernel<T>, dim3(blocks), dim3(256), 0, s, P, w, wt, channel_fastest);
+    return check_launch("relayout_weight_kernel");
+}
+
+// ---------------------------------------------------------------------------------------------
+// Halo tiling plan: block of output positions per workgroup, halo extents, channels per LDS pass.
+// Returns false when the geometry does not suit (halo too large for the staging table or LDS).
+// Tuning knobs (environment, read once per process):
+//   DCN_HALO_MARGIN        voxels of halo beyond the integer tap span on each side: one fixed margin instead of
+//                          the choice on the device among 2, 3, 4 (3-D) or 2, 4, 6 (2-D)
+//   DCN_ADAPTIVE_MARGIN=0  always the smallest of those margins (2)
+//   DCN_TRACE_PLANS=1      print the halo plans and launches of every call on stderr
+//   DCN_LDS_BUDGET_KB      LDS per 512-thread workgroup of the forward halo kernel (default 72: two per CU)
+//   DCN_FORWARD_WG=512     never use the 1024-thread forward variant; =1024 use it whenever its halo fits
+//   DCN_FORWARD_SPLIT=n    forward pass: split the input channels of a position block over at most n workgroups (0: never)
+//   DCN_FORWARD_TAIL=0     forward pass: never split only the units of the last, partly filled round of workgroups (n > 1: n ways)
+//   DCN_FORWARD_TAIL2=0    forward pass: the split units of the last round all the same number of ways, never in two runs
+//   DCN_FORWARD_SLOTS=n    forward pass: plan the launch as if n workgroups ran at once (test hook)
+//   DCN_SCATTER_BUDGET_KB  LDS per workgroup of the privatised scatter kernel (default 144)
+//   DCN_SCATTER=global     scatter grad-input with global atomics instead of the LDS-privatised kernel
+//   DCN_COORD=separate     grad_offset from the channels-last kernel instead of the fused LDS-halo kernel
+//   DCN_FUSED_WAVES=4      fused backward kernel with four wavefronts per workgroup even where eight fit
+//   DCN_FUSED_CHUNK=4      fused backward kernel with 4-channel chunks also where it would take 8 or 16; =8: never 16 (2-D layers)
+//   DCN_FUSED_TAIL=0       fused backward kernel: all items split alike, never only those of the last round
+//   DCN_CSPLIT=n           fused backward kernel: every item split over n workgroups
+//   DCN_FUSED_SLOTS=n      fused backward kernel: plan the launch as if n workgroups ran at once (test hook)
+//   DCN_FUSED_FIXED=0      fused backward kernel: runtime plane stride even where the compile-time one fits
+//   DCN_FUSED_PAIR=0       fused backward kernel, float32: one channel per 64-bit LDS cell instead of two 32-bit halves
+//   DCN_FUSED_BREG2=0      fused backward kernel: no second register set for the grad_output operand of 64 < M <= 128
+//   DCN_GLOBAL_PLAN=0      backward_input_offset (3-D): the device is not offered the path without LDS tiling
+//   DCN_NATIVE16=0         16-bit entry points: always widen to float32 and run the float32 kernels
+static size_t env_kb(const char* name, int dflt) {
+    const char* e = getenv(name);
+    const int v = e ? atoi(e) : dflt;
+    return (size_t)(v > 0 ? v : dflt) * 1024;
+}
+static size_t lds_budget() { static const size_t v = env_kb("DCN_LDS_BUDGET_KB", 72); return v; }
+static size_t scatter_budget() { static const size_t v = env_kb("DCN_SCATTER_BUDGET_KB", 144); return v; }
+static bool fused_coord() {
+    static const int v = [] { const char* e = getenv("DCN_COORD"); return (e && strcmp(e, "separate") == 0) ? 0 : 1; }();
+    return v != 0;
+}
+// What the library needs to know about a GPU, looked up once per device ordinal.
+struct DeviceInfo { int state = 0; int cus = 256; };      // state: 0 not looked up, 1 usable, -1 not a gfx950
+constexpr int MAX_DEVICES = 64;
+inline std::mutex g_device_lock;
+inline DeviceInfo g_device[MAX_DEVICES];
+
+// Fills `out` for the current device; DCN_E_DEVICE when there is none or it is not a gfx950.
+inline int device_info(const DeviceInfo** out, int* ordinal = nullptr) {
+    int dev = -1;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= MAX_DEVICES) {
+        (void)hipGetLastError();
+        return fail(DCN_E_DEVICE, "no current HIP device (or its ordinal is beyond 63)");
+    }
+    std::lock_guard<std::mutex> lock(g_device_lock);
+    DeviceInfo& d = g_device[dev];
+    if (d.state == 0) {
+        hipDeviceProp_t prop;
+        if (hipGetDeviceProperties(&prop, dev) != hipSuccess) {
+            (void)hipGetLastError();
+            return fail(DCN_E_DEVICE, "hipGetDeviceProperties failed");
+        }
+        d.state = strncmp(prop.gcnArchName, "gfx950", 6) == 0 ? 1 : -1;
+        if (prop.multiProcessorCount > 0) d.cus = prop.multiProcessorCount;
+    }
+    if (d.state < 0) return fail(DCN_E_DEVICE, "the current device is not a gfx950 GPU");
+    if (out) *out = &d;
+    if (ordinal) *ordinal = dev;
+    return DCN_OK;
+}
+static int cu_count() {      // of the current device (every entry point has called device_info by then)
+    const DeviceInfo* d = nullptr;
+    return device_info(&d) == DCN_OK ? d->cus : 256;
+}
+static int wide_forward() {      // 0 never, 1 when it pays, 2 whenever the halo fits
+    static const int v = [] {
+        const char* e = getenv("DCN_FORWARD_WG");
+        return !e ? 1 : atoi(e) == 512 ? 0 : atoi(e) == 1024 ? 2 : 1;
+    }();
+    return v;
+}
+static bool fused_chunk16() {     // DCN_FUSED_CHUNK=8 (or 4): never take 16-channel chunks in the fused backward kernel
+    static const int v = [] { const char* e = getenv("DCN_FUSED_CHUNK"); return (e && (atoi(e) == 8 || atoi(e) == 4)) ? 0 : 1; }();
+    return v != 0;
+}
+static bool fused_chunk8() {      // DCN_FUSED_CHUNK=4: never take 8-channel chunks in the fused backward kernel
+    static const int v = [] { const char* e = getenv("DCN_FUSED_CHUNK"); return (e && atoi(e) == 4) ? 0 : 1; }();
+    return v != 0;
+}
+static int fused_first_waves() {
+    static const int v = [] { const char* e = getenv("DCN_FUSED_WAVES"); return (e && atoi(e) == 4) ? 4 : 8; }();
+    return v;
+}
+static bool fused_fixed_stride() {      // DCN_FUSED_FIXED=0: runtime plane stride even where the compile-time one fits
+    static const int v = [] { const char* e = getenv("DCN_FUSED_FIXED"); return (e && atoi(e) == 0) ? 0 : 1; }();
+    return v != 0;
+}
+static bool fused_tail_split() {        // DCN_FUSED_TAIL=0: the fused backward kernel never splits only the items of the last round
+    static const int v = [] { const char* e = getenv("DCN_FUSED_TAIL"); return (e && atoi(e) == 0) ? 0 : 1; }();
+    return v != 0;
+}
+static int forced_slots() {             // DCN_FUSED_SLOTS=n (test hook): plan the fused backward launch as if n workgroups ran at once
+    static const int v = [] { const char* e = getenv("DCN_FUSED_SLOTS"); return e && atoi(e) > 0 ? atoi(e) : 0; }();
+    return v;
+}
+static int forward_split() {            // DCN_FORWARD_SPLIT=n: the forward pass splits the input channels of a position block at most n ways
+    static const int v = [] { const char* e = getenv("DCN_FORWARD_SPLIT"); return e ? atoi(e) : 1 << 20; }();
+    return v;
+}
+static int forward_slots() {            // DCN_FORWARD_SLOTS=n (test hook): plan the forward launch as if n workgroups ran at once
+    static const int v = [] { const char* e = getenv("DCN_FORWARD_SLOTS"); return e && atoi(e) > 0 ? atoi(e) : 0; }();
+    return v;
+}
+static int forward_tail_split() {       // DCN_FORWARD_TAIL=0: the forward pass never splits the units of its last round of workgroups; n > 1: n ways
+    static const int v = [] { const char* e = getenv("DCN_FORWARD_TAIL"); return e ? atoi(e) : 1; }();
+    return v;
+}
+static bool forward_tail_two_runs() {    // DCN_FORWARD_TAIL2=0: the split units of the forward pass's last round are all split the same number of ways
+    static const int v = [] { const char* e = getenv("DCN_FORWARD_TAIL2"); return (e && atoi(e) == 0) ? 0 : 1; }();
+    return v != 0;
+}
+static bool fused_pair() {              // DCN_FUSED_PAIR=0: float32 LDS cells of the fused backward kernel hold one channel each (64-bit)
+    static const int v = [] { const char* e = getenv("DCN_FUSED_PAIR"); return (e && atoi(e) == 0) ? 0 : 1; }();
+    return v != 0;
+}
+static bool fused_breg2() {             // DCN_FUSED_BREG2=0: grad_output operand in registers only up to 32 reduction steps
+    static const int v = [] { const char* e = getenv("DCN_FUSED_BREG2"); return (e && atoi(e) == 0) ? 0 : 1; }();
+    return v != 0;
+}
+static bool native16() {                // DCN_NATIVE16=0: the 16-bit entry points always widen to float32 first
+    static const int v = [] { const char* e = getenv("DCN_NATIVE16"); return (e && atoi(e) == 0) ? 0 : 1; }();
+    return v != 0;
+}
+static bool global_plan() {             // DCN_GLOBAL_PLAN=0: the device never chooses the path without LDS tiling
+    static const int v = [] { const char* e = getenv("DCN_GLOBAL_PLAN"); return (e && atoi(e) == 0) ? 0 : 1; }();
+    return v != 0;
+}
+static bool scatter_in_lds() {
+    static const int v = [] { const char* e = getenv("DCN_SCATTER"); return (e && strcmp(e, "global") == 0) ? 0 : 1; }();
+    return v != 0;
+}
+#define LDS_BUDGET lds_budget()
+static int halo_margin() {      // DCN_HALO_MARGIN: one fixed margin; -1 when not set
+    static const int v = [] {
+        const char* e = getenv("DCN_HALO_MARGIN");
+        if (!e) return -1;
+        const int m = atoi(e);
+        return m < 0 ? 0 : m;
+    }();
+    return v;
+}
+// Halo margins to plan for, ascending; the first is the one taken when nothing can be chosen.
+static int plan_margins(int nd, int* m) {
+    static const int adaptive = [] { const char* e = getenv("DCN_ADAPTIVE_MARGIN"); return (e && atoi(e) == 0) ? 0 : 1; }();
+    if (halo_margin() >= 0) { m[0] = halo_margin(); return 1; }
+    m[0] = 2;
+    if (!adaptive) return 1;
+    m[1] = nd == 3 ? 3 : 4;
+    m[2] = nd == 3 ? 4 : 6;
+    return MAX_PLANS;
+}
+static_assert(MAX_PLANS == 3, "plan_margins fills three margins");
+static bool trace_plans() {             // DCN_TRACE_PLANS=1: the halo plans and launches of every call on stderr
+    static const int v = [] { const char* e = getenv("DCN_TRACE_PLANS"); return (e && atoi(e) != 0) ? 1 : 0; }();
+    return v != 0;
+}
+static int default_margin() { return halo_margin() >= 0 ? halo_margin() : 2; }
+static int forced_csplit() {    // DCN_CSPLIT=n: workgroups per (tile, deformable group) of the fused backward kernel
+    static const int v = [] { const char* e = getenv("DCN_CSPLIT"); return e && atoi(e) > 0 ? atoi(e) : 0; }();
+    return v;
+}
+
+template <typename T, int ND>
+inline bool plan_halo(Params& P, size_t budget, int m, int max_chunk = 1 << 30, size_t cell_bytes = sizeof(T), int waves = WAVESH,
+               bool smallest_halo = false, int chunk_mult = 0, const int* blocks = nullptr, int wmult = 1) {
+    const int npos = waves * Mma<T>::TN;        // positions per workgroup, one column tile per wavefront
+    int td[3] = {1, 1, 1};
+    if (ND == 3) { td[1] = 8; td[2] = 8; td[0] = npos / 64; }
+    else         { td[2] = 16; td[1] = npos / 16; }
+    if (blocks) {                               // the block shape of another plan
+        for (int a = 0; a < 3; ++a) td[a] = blocks[a];
+    } else if (smallest_halo) {
+        // the block shape (powers of two, at least 4 positions along the fastest axis) with the
+        // smallest halo: strided geometries want blocks that are short along the strided axes
+        long long best = -1;
+        for (int a = 1; a <= npos; a *= 2)
+            for (int b = 1; a * b <= npos; b *= 2) {
+                const int c = npos / (a * b);
+                if (c < 4 || (ND == 2 && a != 1)) continue;
+                const int cand[3] = {a, b, c};
+                long long hv = 1;
+                for (int x = 3 - ND; x < 3; ++x) hv *= (cand[x] - 1) * P.stride[x] + (P.k[x] - 1) * P.dil[x] + 1 + 2 * m;
+                if (best < 0 || hv < best) { best = hv; td[0] = a; td[1] = b; td[2] = c; }
+            }
+    }
+    long long hvol = 1, tiles = 1;
+    for (int a = 0; a < 3; ++a) {
+        P.tdim[a] = td[a];
+        P.ntile[a] = (P.out[a] + td[a] - 1) / td[a];
+        const bool used = a >= 3 - ND;
+        P.mlo[a] = used ? m : 0;
+        // lowest corner: base - m; highest corner: base + m (the high corner of a sample at base + m - eps)
+        P.hext[a] = used ? (td[a] - 1) * P.stride[a] + (P.k[a] - 1) * P.dil[a] + 1 + 2 * m : 1;
+        // (wmult: the innermost extent rounded up to a multiple, for kernels whose LDS layout depends on
+        // the position of a halo voxel modulo that number; the extra cells lie on the high side)
+        if (a == 2 && wmult > 1) P.hext[a] = (P.hext[a] + wmult - 1) / wmult * wmult;
+        hvol *= P.hext[a];
+        tiles *= P.ntile[a];
+    }
+    if (hvol > MAX_HVOL) return false;
+    P.hvol = (int)hvol;
+    P.hstride = ((int)hvol + 63) / 64 * 64 + 32;
+    const int KL = chunk_mult > 0 ? chunk_mult : Mma<T>::KL;      // channels per pass come in multiples of this
+    if (budget <= (size_t)hvol * 4) return false;
+    long long cc = (long long)((budget - (size_t)hvol * 4) / ((size_t)P.hstride * cell_bytes));
+    cc = cc / KL * KL;
+    const int seg = P.cpg < P.Cg ? P.cpg : P.Cg;          // longest run of channels sharing offsets and group
+    const int seg_up = (seg + KL - 1) / KL * KL;
+    if (cc > seg_up) cc = seg_up;
+    if (cc > max_chunk) cc = max_chunk / KL * KL;
+    if (cc < KL) return false;
+    P.cchunk = (int)cc;
+    if (tiles * P.N > 0x7fffffffLL) return false;
+    P.tiles = (int)tiles;
+    return true;
+}
+
+// Raises a kernel's dynamic LDS limit; the runtime is asked only when a kernel needs more than it
+// was last granted on the current device.
+inline int raise_lds_limit(const void* kern, size_t lds) {
+    static std::mutex lock;
+    static std::map<std::pair<int, const void*>, size_t> granted;
+    int dev = 0;
+    if (device_info(nullptr, &dev) != DCN_OK) return DCN_E_DEVICE;
+    std::lock_guard<std::mutex> guard(lock);
+    size_t& have = granted[std::make_pair(dev, kern)];
+    if (lds <= have) return DCN_OK;
+    if (hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess) {
+        (void)hipGetLastError();
+        return fail(DCN_E_LAUNCH, "cannot raise the dynamic LDS limit");
+    }
+    have = lds;
+    return DCN_OK;
+}
+
+// Workgroups of a kernel that the current device holds at once (one per CU if the query fails).
+inline long long resident_workgroups(const void* kern, int threads, size_t lds) {
+    static std::mutex lock;
+    static std::map<std::pair<const void*, size_t>, int> per_cu_of;
+    int per_cu = 0;
+    {
+        std::lock_guard<std::mutex> guard(lock);
+        int& v = per_cu_of[std::make_pair(kern, lds)];
+        if (v == 0) {
+            if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&v, kern, threads, lds) != hipSuccess || v < 1) {
+                (void)hipGetLastError();
+                v = 1;
+            }
+        }
+        per_cu = v;
+    }
+    return (long long)per_cu * cu_count();
+}
+
+static HaloPlan halo_plan_of(const Params& P) {
+    HaloPlan h;
+    for (int a = 0; a < 3; ++a) { h.hext[a] = P.hext[a]; h.mlo[a] = P.mlo[a]; }
+    h.hvol = P.hvol; h.hstride = P.hstride; h.cchunk = P.cchunk;
+    return h;
+}
+static bool same_blocks(const Params& a, const Params& b) {
+    for (int x = 0; x < 3; ++x)
+        if (a.tdim[x] != b.tdim[x] || a.ntile[x] != b.ntile[x]) return false;
+    return a.tiles == b.tiles;
+}
+
+template <typename K, typename... Args>
+inline int launch_halo(K kern, const char* name, dim3 grid, int threads, size_t lds, hipStream_t s, Args... args) {
+    if (lds > 48 * 1024)
+        if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kern), lds)) return rc;
+    hipLaunchKernelGGL(kern, grid, dim3(threads), lds, s, args...);
+    return check_launch(name);
+}
+
+// ---------------------------------------------------------------------------------------------
+// The operators, each instantiated in a translation unit of its own (they compile in parallel).
+constexpr unsigned FLAG_INPUT_ONLY = 0x100u;     // internal: see backward_input_offset
+template <typename T, int ND, typename S = T>
+int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* bias, S* out, void* ws, size_t ws_bytes,
+            hipStream_t s, bool* declined = nullptr);
+template <typename T, int ND, typename S = T>
+int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* off, const S* gout, T* gin, T* goff, void* ws,
+                          size_t ws_bytes, hipStream_t s, unsigned flags = 0, bool* declined = nullptr);
+template <typename T, int ND>
+int backward_weight(const Geometry& g, const T* in, const T* off, const T* gout, T* gw, void* ws, size_t ws_bytes, hipStream_t s);
+template <typename S, int ND>
+int backward_weight_native16(const Params& Pin, const S* in, const S* off, const S* gout, float* fgw, void* ws, size_t ws_bytes,
+                             hipStream_t s, bool* declined);
+
+}  // namespace dcn
