@@ -185,11 +185,13 @@ Geometry geo2(int batch, int input_c, int output_c, int input_h, int input_w, in
 
 // ---------------------------------------------------------------------------------------------
 // Scratch of the allocation-free entry point: the re-laid-out weight of one forward call.  A
-// file-scope device array, so every GPU the library runs on holds DCN_NOALLOC_SCRATCH_BYTES of it
+// file-scope device array, so every GPU the library runs on holds SCRATCH_BYTES of it
 // until the process ends.  In host code the array's name is only a handle for
 // hipGetSymbolAddress: the device address is looked up once per device and kept, and host code
 // passes that address, never the name, to kernels.
-static __device__ __align__(256) unsigned char scratch[DCN_NOALLOC_SCRATCH_BYTES];
+// (twice the accepted size of the float32 layout: the kernel's packed weights are half as large again)
+constexpr size_t SCRATCH_BYTES = 2 * (size_t)DCN_NOALLOC_SCRATCH_BYTES;
+static __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
 
 std::mutex g_scratch_lock;
 void* g_scratch_ptr[MAX_DEVICES] = {};
@@ -269,7 +271,7 @@ int dcn3d_forward_noalloc_f32(const float* input, const float* weight, const flo
     }
     void* ws = nullptr;
     if (int rc = scratch_address(&ws)) return rc;
-    return forward<float, 3>(g, input, weight, offset, bias, output, ws, DCN_NOALLOC_SCRATCH_BYTES,
+    return forward<float, 3>(g, input, weight, offset, bias, output, ws, SCRATCH_BYTES,
                              static_cast<hipStream_t>(stream));
 }
 

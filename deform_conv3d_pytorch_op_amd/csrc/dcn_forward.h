@@ -1,4 +1,4 @@
-// Forward kernel with the input halo in LDS, four channels of a voxel side by side.
+// Forward kernel of the float64 operator: input halo in LDS, four channels of a voxel side by side.
 //
 //   out[n][g*M + m][pos] = sum_{cl,tap} W[g*M+m][cl][tap] * sample(in[n][g*Cg+cl], tap, pos)  (+ bias)
 //
@@ -34,9 +34,9 @@ __host__ __device__ inline size_t forward_slab_elems(int kV, int Mp) {
 }
 
 // With pc.sel set the launch has one block more, which chooses the halo plan from the offsets.
-template <typename T, typename S = T>
-__global__ void pack_forward_weight_kernel(Params P, const S* __restrict__ W, S* __restrict__ Wq, PlanChoice pc,
-                                           const S* __restrict__ off, size_t n_off) {
+template <typename T>
+__global__ void pack_forward_weight_kernel(Params P, const T* __restrict__ W, T* __restrict__ Wq, PlanChoice pc,
+                                           const T* __restrict__ off, size_t n_off) {
     using MM = Mma<T>;
     constexpr int TN = MM::TN, KL = MM::KL;
     const unsigned pack_blocks = pc.sel ? gridDim.x - 1 : gridDim.x;
@@ -59,7 +59,7 @@ __global__ void pack_forward_weight_kernel(Params P, const S* __restrict__ W, S*
         const int tile = (int)(r % mtiles);
         const int tg = (int)(r / mtiles);
         const int m = tile * TN + j, tap = tg * KL + q, c = c0 + e, g = c0 / P.Cg;
-        S v = S();
+        T v = 0;
         if (m < P.M && tap < P.kV && c < seg_e) v = W[(((size_t)g * P.M + m) * P.Cg + (c - g * P.Cg)) * P.kV + tap];
         Wq[(size_t)chunk_slot<FQ>(P.cpg, P.Cg, c0) * per_slab + i % per_slab] = v;
     }
@@ -68,8 +68,8 @@ __global__ void pack_forward_weight_kernel(Params P, const S* __restrict__ W, S*
 // Stage `nch` channels of the halo as groups of four: sIn[group][halo voxel][4].  Missing channels
 // of a short last group and halo voxels outside the volume hold zero (a sample in the rim reads
 // the latter with weight zero).
-template <typename T, int WGS, typename S = T>
-__device__ inline void halo_stage_quads(const Params& P, const HaloPlan& H, const S* __restrict__ chan0, int nch,
+template <typename T, int WGS>
+__device__ inline void halo_stage_quads(const Params& P, const HaloPlan& H, const T* __restrict__ chan0, int nch,
                                         const unsigned* __restrict__ sTab, T* __restrict__ sIn, int* __restrict__ nonfinite) {
     const int ngrp = (nch + FQ - 1) / FQ;
     bool bad = false;                  // a NaN or an infinity among the staged values (see halo_nonfinite)
@@ -79,7 +79,7 @@ __device__ inline void halo_stage_quads(const Params& P, const HaloPlan& H, cons
         for (int grp = 0; grp < ngrp; ++grp) {
             T val[FQ];
 #pragma unroll
-            for (int e = 0; e < FQ; ++e) val[e] = Store<S>::ld(chan0[(size_t)min(grp * FQ + e, nch - 1) * P.inV + g]);
+            for (int e = 0; e < FQ; ++e) val[e] = chan0[(size_t)min(grp * FQ + e, nch - 1) * P.inV + g];
 #pragma unroll
             for (int e = 0; e < FQ; ++e) bad = bad || !(fabs(val[e]) <= std::numeric_limits<T>::max());
 #pragma unroll
@@ -103,20 +103,16 @@ __device__ inline void halo_stage_quads(const Params& P, const HaloPlan& H, cons
 //     the last round fills the device; their partial sums go to part as
 //     [split workgroup][row of the chunk][position of the block] in launch order, i.e.
 //     [unit - whole][cz] within each of the two runs of TailSplit (forward_join_tail_kernel).
-// (few accumulators: four wavefronts per SIMD, i.e. at most 128 registers, also for the 512-thread
-// shape, so that two of its workgroups share a CU)
-// S: storage format of the tensors (see Store); T is float with a 16-bit format, and partial sums are always T.
-template <typename T, int ND, int MT, int NW, typename S = T>
-__global__ __launch_bounds__(NW * 64, (MT <= 2 && sizeof(T) == 4) ? 4 : 1) void forward_quad_kernel(Params P, PlanSet alts, const unsigned* __restrict__ sel,
-                                                           const S* __restrict__ in,
-                                                           const S* __restrict__ off, const S* __restrict__ Wq,
-                                                           const S* __restrict__ bias, S* __restrict__ out,
+template <typename T, int ND, int MT, int NW>
+__global__ __launch_bounds__(NW * 64, 1) void forward_quad_kernel(Params P, PlanSet alts, const unsigned* __restrict__ sel,
+                                                           const T* __restrict__ in,
+                                                           const T* __restrict__ off, const T* __restrict__ Wq,
+                                                           const T* __restrict__ bias, T* __restrict__ out,
                                                            T* __restrict__ part, int csplit, unsigned whole, TailSplit ts) {
     HaloPlan H;
     if (!chosen_halo(P, alts, sel, H)) return;          // another launch runs the chosen plan
     using MM = Mma<T>;
     constexpr int TN = MM::TN, KL = MM::KL, NC = 1 << ND, WGS = NW * 64;
-    constexpr bool S16 = sizeof(S) == 2;                // 16-bit storage: 16-bit matrix instructions
     typedef T V4 __attribute__((ext_vector_type(4)));
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ int sNonFinite;
@@ -186,15 +182,15 @@ __global__ __launch_bounds__(NW * 64, (MT <= 2 && sizeof(T) == 4) ? 4 : 1) void 
     int chunk_no = 0;
     for (int dg = cg0 / P.cpg; dg <= (cg1 - 1) / P.cpg; ++dg) {
         const int cb = max(cg0, dg * P.cpg), ce = min(cg1, (dg + 1) * P.cpg);
-        const S* off_dg = off + ((size_t)n * P.DG + dg) * P.kV * ND * P.outV;
+        const T* off_dg = off + ((size_t)n * P.DG + dg) * P.kV * ND * P.outV;
         for (int cc0 = cb; cc0 < ce; cc0 += cch) {
             if ((chunk_no++) % csplit != cz) continue;                     // another workgroup's chunk (uniform)
             const int nch = min(cch, ce - cc0);
             const int ngrp = (nch + FQ - 1) / FQ;
-            const S* chan0 = in + ((size_t)n * P.C_in + cc0) * P.inV;      // workgroup-uniform
+            const T* chan0 = in + ((size_t)n * P.C_in + cc0) * P.inV;      // workgroup-uniform
             if (threadIdx.x == 0) sNonFinite = 0;
             __syncthreads();                                               // readers of the previous chunk are done
-            halo_stage_quads<T, WGS, S>(P, H, chan0, nch, sTab, sIn, &sNonFinite);
+            halo_stage_quads<T, WGS>(P, H, chan0, nch, sTab, sIn, &sNonFinite);
             __syncthreads();
             // Non-finite input values in this halo: the branch-free sampler reads the cell next to a
             // collapsed corner with weight 0, and 0 * inf would be NaN where the reference never
@@ -204,17 +200,17 @@ __global__ __launch_bounds__(NW * 64, (MT <= 2 && sizeof(T) == 4) ? 4 : 1) void 
             const bool halo_nonfinite = sNonFinite != 0;                   // uniform
             // slabs of consecutive groups of one segment are consecutive.  Uniform base (scalar
             // registers); the lanes add the 32-bit offset w_lane.
-            const S* wchunk = Wq + (size_t)chunk_slot<FQ>(P.cpg, P.Cg, cc0) * per_slab;
+            const T* wchunk = Wq + (size_t)chunk_slot<FQ>(P.cpg, P.Cg, cc0) * per_slab;
 
             // kernel coordinates of this lane's tap, counted up with the tap groups
             int kq[ND];
             decode_tap<ND>(P, q, kq);
             T o_buf[2][ND];
             auto load_offsets_of = [&](int tgi, T* dst) {                  // offsets of tap tgi*KL + q (clamped to a legal tap)
-                const S* ob = off_dg + (size_t)tgi * KL * ND * P.outV;     // uniform
+                const T* ob = off_dg + (size_t)tgi * KL * ND * P.outV;     // uniform
                 const unsigned lo = (unsigned)min(q, P.kV - 1 - tgi * KL) * ND * P.outV + pos;
 #pragma unroll
-                for (int a = 0; a < ND; ++a) dst[a] = Store<S>::ld((ob + (size_t)a * P.outV)[lo]);
+                for (int a = 0; a < ND; ++a) dst[a] = (ob + (size_t)a * P.outV)[lo];
             };
             load_offsets_of(0, o_buf[0]);
 
@@ -278,13 +274,12 @@ __global__ __launch_bounds__(NW * 64, (MT <= 2 && sizeof(T) == 4) ? 4 : 1) void 
                     kq[0] += carry;
                 }
                 const V4* hp = reinterpret_cast<const V4*>(sIn) + base;
-                const S* wp = wchunk + (size_t)tgi * w_tg;
+                const T* wp = wchunk + (size_t)tgi * w_tg;
                 for (int grp = 0; grp < ngrp; ++grp) {
-                    // this lane's weights of the group's four channels: one 16- (32-, 8-) byte load per row tile
-                    typedef typename std::conditional<S16, typename Mma16<typename std::conditional<S16, S, Bf16>::type>::Vec, V4>::type A4;
-                    A4 a4[MT];
+                    // this lane's weights of the group's four channels: 32 contiguous bytes per row tile
+                    V4 a4[MT];
 #pragma unroll
-                    for (int mt = 0; mt < MT; ++mt) a4[mt] = *reinterpret_cast<const A4*>(wp + (w_lane + mt * w_tile));
+                    for (int mt = 0; mt < MT; ++mt) a4[mt] = *reinterpret_cast<const V4*>(wp + (w_lane + mt * w_tile));
                     // weighted corner sum, four corners at a time (all eight in flight would cost 32
                     // registers that the 16-wavefront shape does not have)
                     // (element by element: a vector times scalar product would hold four copies of
@@ -312,22 +307,11 @@ __global__ __launch_bounds__(NW * 64, (MT <= 2 && sizeof(T) == 4) ? 4 : 1) void 
 #pragma unroll
                             for (int i = 0; i < 4; ++i) val[e] += c4[i][e] * cw[4 + i];
                     }
-                    if constexpr (S16) {
-                        // the four channels are the four reduction elements this lane supplies to one
-                        // 32x32x8 instruction (lane group q: elements 4q .. 4q + 3, its tap)
-                        float b4[FQ];
 #pragma unroll
-                        for (int e = 0; e < FQ; ++e) b4[e] = near ? val[e] : 0.f;
-                        const auto bv = Mma16<S>::pack(b4);
+                    for (int e = 0; e < FQ; ++e) {
+                        const T b = near ? val[e] : (T)0;
 #pragma unroll
-                        for (int mt = 0; mt < MT; ++mt) acc[mt] = Mma16<S>::mma(a4[mt], bv, acc[mt]);
-                    } else {
-#pragma unroll
-                        for (int e = 0; e < FQ; ++e) {
-                            const T b = near ? val[e] : (T)0;
-#pragma unroll
-                            for (int mt = 0; mt < MT; ++mt) acc[mt] = MM::mma(a4[mt][e], b, acc[mt]);
-                        }
+                        for (int mt = 0; mt < MT; ++mt) acc[mt] = MM::mma(a4[mt][e], b, acc[mt]);
                     }
                     hp += H.hstride;
                     wp += per_slab;
@@ -345,20 +329,18 @@ __global__ __launch_bounds__(NW * 64, (MT <= 2 && sizeof(T) == 4) ? 4 : 1) void 
                         t.f[a] = pa - (T)l;
                     }
                     tap_corner_idx<T, ND>(P, t);
-                    const S* wf = wchunk + (size_t)tgi * w_tg;
+                    const T* wf = wchunk + (size_t)tgi * w_tg;
                     for (int c = 0; c < nch; ++c) {
                         T b = 0;
                         if (far) {
                             T cc[NC];
 #pragma unroll
-                            for (int i = 0; i < NC; ++i) cc[i] = Store<S>::ld((chan0 + (size_t)c * P.inV)[t.idx[i]]);
+                            for (int i = 0; i < NC; ++i) cc[i] = (chan0 + (size_t)c * P.inV)[t.idx[i]];
                             b = interp<T, ND>(cc, t.f);
-                            if constexpr (S16) b = Store<S>::ld(Store<S>::st(b));      // rounded like the samples of the halo path
                         }
-                        const S* wc = wf + (size_t)(c / FQ) * per_slab + c % FQ;
-                        // (one channel at a time through the float instruction: same accumulator layout)
+                        const T* wc = wf + (size_t)(c / FQ) * per_slab + c % FQ;
 #pragma unroll
-                        for (int mt = 0; mt < MT; ++mt) acc[mt] = MM::mma((T)Store<S>::ld(wc[w_lane + mt * w_tile]), b, acc[mt]);
+                        for (int mt = 0; mt < MT; ++mt) acc[mt] = MM::mma(wc[w_lane + mt * w_tile], b, acc[mt]);
                     }
                 }
             };
@@ -397,8 +379,8 @@ __global__ __launch_bounds__(NW * 64, (MT <= 2 && sizeof(T) == 4) ? 4 : 1) void 
                 T v = acc[mt][r];
                 if (split) pdst[at] = v;
                 else {
-                    if (bias) v += Store<S>::ld(bias[g * P.M + m]);
-                    out[at] = Store<S>::st(v);
+                    if (bias) v += bias[g * P.M + m];
+                    out[at] = v;
                 }
             }
         }

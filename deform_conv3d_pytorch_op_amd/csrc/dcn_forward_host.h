@@ -2,6 +2,7 @@
 #pragma once
 #include "dcn_host.h"
 #include "dcn_forward.h"
+#include "dcn_forward_shared.h"
 
 namespace dcn {
 
@@ -13,6 +14,14 @@ template <typename T, int ND, typename S>
 int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* bias, S* out, void* ws,
             size_t ws_bytes, hipStream_t s, bool* declined) {
     constexpr bool S16 = !std::is_same<S, T>::value;
+    constexpr bool MX = sizeof(T) == 4;                 // forward_split_kernel; float64: forward_quad_kernel
+    constexpr size_t MAX_LDS = MX ? 160 * 1024 - 256 : 144 * 1024;      // dynamic LDS of the only workgroup of a CU
+    constexpr int CM = MX ? FG : FQ;                    // channels of a weight slab
+    using WE = typename std::conditional<MX, typename Parts<typename std::conditional<MX, S, float>::type>::Elem, S>::type;      // packed weight element
+    auto slab_bytes = [](int kV, int Mp) {
+        if constexpr (MX) return split_slab_elems<S>(kV, Mp) * sizeof(WE);
+        else return forward_slab_elems<T>(kV, Mp) * sizeof(T);
+    };
     Params P;
     if (int rc = validate(g, P)) return rc;
     if (!in || !w || !off || !out) return fail(DCN_E_ARGUMENT, "null tensor pointer");
@@ -20,7 +29,6 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
     int MT;
     fwd_weight_pad<T>(P.M, P.Cg, MT, P.mchunks, P.Mp, P.Cgp);
     if (!ws || (!S16 && ws_bytes < (size_t)P.G * P.kV * P.Mp * P.Cgp * sizeof(T))) return fail(DCN_E_WORKSPACE, "workspace too small");
-    S* wt = static_cast<S*>(ws);
     const int TN = Mma<T>::TN;
     // Too few position blocks to give every CU a workgroup.  First the input channels of a block are
     // split over up to FWD_MAX_SPLIT workgroups (each samples its own channels once; their partial
@@ -28,16 +36,26 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
     // Then fewer row tiles per wavefront: more output-channel chunks, each sampling for itself.
     int fsplit = 1;
     const int mtiles_all = (P.M + TN - 1) / TN;
+    // More than 64 output channels, 2-D (in 3-D a block of 128 positions stages twice the halo per position:
+    // 1.27 against 0.97 ms for 128 -> 128 channels at stride 2): forward_shared_kernel, units of 128 positions and MT = 4 or 8 row tiles.
+    // Per 16 reduction slots and 32 positions a row tile costs its matrix instructions and every chunk of
+    // row tiles samples for itself: the cheaper of the two.
+    bool shared = MX && ND == 2 && mtiles_all > 2 && forward_shared();
+    if (shared) {
+        auto cost = [&](int rt) { const int mc = (mtiles_all + rt - 1) / rt; return mc * (rt * (S16 ? 1 : 6) + 10); };
+        MT = mtiles_all > 4 && cost(8) <= cost(4) ? 8 : 4;
+        P.mchunks = (mtiles_all + MT - 1) / MT;
+    }
+    const int nwp = shared ? SHARED_COLS : WAVESH;      // column tiles of a block
     const size_t out_bytes = (size_t)P.N * P.C_out * P.outV * sizeof(T);
-    const size_t wq_bound = align256(((size_t)chunk_slot<FQ>(P.cpg, P.Cg, P.C_in - 1) + 1) *
-                                     forward_slab_elems<T>(P.kV, (mtiles_all + 7) / 8 * 8 * TN) * sizeof(T));
+    const size_t wq_bound = align256(((size_t)chunk_slot<CM>(P.cpg, P.Cg, P.C_in - 1) + 1) * slab_bytes(P.kV, (mtiles_all + 7) / 8 * 8 * TN));
     {
         Params Pt = P;
-        const bool tiled = plan_halo<T, ND>(Pt, 144 * 1024, default_margin(), 1 << 30, sizeof(T), WAVESH, false, FQ);
+        const bool tiled = plan_halo<T, ND>(Pt, MAX_LDS, default_margin(), 1 << 30, MX ? sizeof(S) : sizeof(T), nwp, false, FQ, nullptr, 1, !MX);
         const long long tiles = tiled ? (long long)Pt.N * Pt.tiles : (long long)P.N * ((P.outV + WAVES * TN - 1) / (WAVES * TN));
         // (eight row tiles per wavefront only pay when the grid is full anyway: measured slower than
         // four with twice the sampling)
-        if (MT == 8 && tiles * P.G * P.mchunks < cu_count()) {
+        if (MT == 8 && !shared && (MX || tiles * P.G * P.mchunks < cu_count())) {
             MT = 4;
             P.mchunks = (mtiles_all + MT - 1) / MT;
         }
@@ -47,7 +65,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                    (size_t)fsplit * 2 * out_bytes <= room && fsplit * 2 * 16 <= P.Cg)      // at least 16 channels per part
                 fsplit *= 2;
         }
-        while (MT > 1 && tiles * P.G * P.mchunks * fsplit < cu_count()) {
+        while (MT > 1 && !shared && tiles * P.G * P.mchunks * fsplit < cu_count()) {
             MT /= 2;
             P.mchunks = (mtiles_all + MT - 1) / MT;
         }
@@ -58,26 +76,39 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
     // fits and leaves 8 channels per pass.  Otherwise 512 threads: two workgroups per CU when that
     // still leaves 8 channels per LDS pass, else one large one.  Returns the wavefronts per
     // workgroup, 0 when no halo of margin m fits.
+    // channels per LDS pass: multiples of eight for forward_split_kernel, where they fit
+    auto plan_shape = [&](Params& Ph, size_t budget, int m, int waves, bool smallest, const int* blocks = nullptr) {
+        if constexpr (MX)
+            if (plan_halo<T, ND>(Ph, budget, m, 1 << 30, sizeof(S), waves, smallest, FG, blocks, 1, false)) return true;
+        return !S16 && plan_halo<T, ND>(Ph, budget, m, MX ? 4 : 1 << 30, sizeof(T), waves, smallest, FQ, blocks, 1, !MX);
+    };
     auto plan_for = [&](int m, Params& Ph) {
         Ph = P;
         int nw = 0;
+        if (shared) {
+            const size_t room = MAX_LDS - shared_column_bytes<typename std::conditional<MX, S, float>::type>();
+            bool tiled = plan_halo<T, ND>(Ph, room, m, 1 << 30, sizeof(S), SHARED_COLS, false, FG, nullptr, 1, false);
+            if (!tiled || Ph.cchunk < 16) {
+                Params Ps = P;
+                if (plan_halo<T, ND>(Ps, room, m, 1 << 30, sizeof(S), SHARED_COLS, true, FG, nullptr, 1, false) && (!tiled || Ps.cchunk > Ph.cchunk)) { Ph = Ps; tiled = true; }
+            }
+            return tiled && (long long)Ph.N * Ph.tiles * Ph.G * Ph.mchunks <= 0x7fffffffLL ? SHARED_COLS : 0;
+        }
         // (the 3-D double instance of the 1024-thread shape does not fit its 128 registers)
         if (MT <= 2 && wide_forward() && !(sizeof(T) == 8 && ND == 3)) {
             Params Pw = P;
-            if (plan_halo<T, ND>(Pw, 144 * 1024, m, 1 << 30, sizeof(T), 16, false, FQ) &&
-                (long long)Pw.N * Pw.tiles * Pw.G * Pw.mchunks <= 0x7fffffffLL &&
+            if (plan_shape(Pw, MAX_LDS, m, 16, false) && (long long)Pw.N * Pw.tiles * Pw.G * Pw.mchunks <= 0x7fffffffLL &&
                 (wide_forward() == 2 || (Pw.cchunk >= 8 && (long long)Pw.N * Pw.tiles * Pw.G * Pw.mchunks >= cu_count()))) {
                 Ph = Pw;
                 nw = 16;
             }
         }
         if (!nw) {
-            bool tiled = plan_halo<T, ND>(Ph, LDS_BUDGET, m, 1 << 30, sizeof(T), WAVESH, false, FQ);
-            if ((!tiled || Ph.cchunk < 8) && LDS_BUDGET < 144 * 1024)
-                tiled = plan_halo<T, ND>(Ph, 144 * 1024, m, 1 << 30, sizeof(T), WAVESH, false, FQ) || tiled;
+            bool tiled = plan_shape(Ph, LDS_BUDGET, m, WAVESH, false);
+            if ((!tiled || Ph.cchunk < 8) && LDS_BUDGET < MAX_LDS) tiled = plan_shape(Ph, MAX_LDS, m, WAVESH, false) || tiled;
             if (!tiled || Ph.cchunk < 8) {       // strided layers: the block shape with the smallest halo may hold 8 channels
                 Params Ps = P;
-                if (plan_halo<T, ND>(Ps, 144 * 1024, m, 1 << 30, sizeof(T), WAVESH, true, FQ) && (!tiled || Ps.cchunk > Ph.cchunk)) {
+                if (plan_shape(Ps, MAX_LDS, m, WAVESH, true) && (!tiled || Ps.cchunk > Ph.cchunk)) {
                     Ph = Ps;
                     tiled = true;
                 }
@@ -90,9 +121,17 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
         int margins[MAX_PLANS];
         const int nmargins = plan_margins(ND, margins);
         Params plans[MAX_PLANS];
-        const int nw = plan_for(margins[0], plans[0]);
-        const size_t slabs = (size_t)chunk_slot<FQ>(P.cpg, P.Cg, P.C_in - 1) + 1;
-        const size_t wq_bytes = slabs * forward_slab_elems<T>(P.kV, P.Mp) * sizeof(S);
+        int nw = plan_for(margins[0], plans[0]);
+        if (shared && !nw) {       // (no halo of 128 positions holds eight channels)
+            shared = false;
+            MT = 4;
+            P.mchunks = (mtiles_all + MT - 1) / MT;
+            P.Mp = P.mchunks * MT * TN;
+            nw = plan_for(margins[0], plans[0]);
+        }
+        const size_t col_bytes = shared ? shared_column_bytes<typename std::conditional<MX, S, float>::type>() : 0;
+        const size_t wq_bytes = ((size_t)chunk_slot<CM>(P.cpg, P.Cg, P.C_in - 1) + 1) * slab_bytes(P.kV, P.Mp) + 256;      // (+: operands read from four elements further on)
+        auto halo_lds = [=](const Params& Ph) { return col_bytes + (size_t)Ph.cchunk * Ph.hstride * (MX ? sizeof(S) : sizeof(T)) + (MX ? 0 : (size_t)Ph.hvol * 4); };
         if (nw == 16 || ws_bytes < align256(wq_bytes) + (size_t)fsplit * out_bytes) fsplit = 1;
         if (nw && ws_bytes >= wq_bytes) {
             // channels per LDS pass such that every workgroup of a block gets the same number of passes
@@ -105,7 +144,8 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                     }
                     return n;
                 };
-                for (int cc = Ph.cchunk; cc >= FQ; cc -= FQ)
+                const int step = Ph.cchunk % CM == 0 ? CM : FQ;
+                for (int cc = Ph.cchunk; cc >= step; cc -= step)
                     if (chunks_of_group0(cc) % fsplit == 0) { Ph.cchunk = cc; break; }
             };
             if (fsplit > 1) even_passes(plans[0]);
@@ -126,12 +166,13 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                 // (within the LDS of the first plan, which fixes how many workgroups share a CU; all of it
                 // when the grid gives a CU one workgroup at most)
                 const long long wgs = (long long)plans[0].N * plans[0].tiles * plans[0].G * plans[0].mchunks * fsplit;
-                size_t lds0 = (size_t)plans[0].cchunk * plans[0].hstride * sizeof(T) + (size_t)plans[0].hvol * 4;
-                if (wgs <= cu_count() && lds0 < 144 * 1024) lds0 = 144 * 1024;
+                size_t lds0 = halo_lds(plans[0]);
+                if ((wgs <= cu_count() || shared) && lds0 < MAX_LDS) lds0 = MAX_LDS;
                 for (int k = 1; k < nmargins; ++k) {
                     Params& Pk = plans[pc.nplans];
                     Pk = P;
-                    if (!plan_halo<T, ND>(Pk, lds0, margins[k], 1 << 30, sizeof(T), nw, false, FQ, plans[0].tdim)) continue;
+                    if (shared ? !plan_halo<T, ND>(Pk, lds0 - col_bytes, margins[k], 1 << 30, sizeof(S), nw, false, FG, plans[0].tdim, 1, false)
+                               : !plan_shape(Pk, lds0, margins[k], nw, false, plans[0].tdim)) continue;
                     if (!same_blocks(Pk, plans[0]) || Pk.hvol > 3 * plans[0].hvol) continue;
                     if (fsplit > 1) even_passes(Pk);
                     pc.margin[pc.nplans] = margins[k];
@@ -150,23 +191,34 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             for (int k = 1; k < MAX_PLANS; ++k) alts.alt[k - 1] = halo_plan_of(plans[k]);
             alts.mask = (1u << pc.nplans) - 1;
             {
-                const size_t total = (size_t)chunk_candidates<FQ>(P.cpg, P.Cg, P.C_in) * forward_slab_elems<T>(P.kV, P.Mp);
+                size_t total = (size_t)chunk_candidates<CM>(P.cpg, P.Cg, P.C_in);
+                if constexpr (MX) total *= (size_t)((P.kV + 1) / 2) * P.Mp * 2;          // one thread per operand of a lane
+                else total *= forward_slab_elems<T>(P.kV, P.Mp);
                 const unsigned blocks = (unsigned)((total + 255) / 256 > 8192 ? 8192 : (total + 255) / 256);
                 const size_t n_off = (size_t)P.N * P.DG * P.kV * ND * P.outV;
-                hipLaunchKernelGGL((pack_forward_weight_kernel<T, S>), dim3(blocks + (pc.sel ? 1 : 0)), dim3(256), 0, s, plans[0], w, wt, pc, off, n_off);
-                if (int rc = check_launch("pack_forward_weight_kernel")) return rc;
+                const dim3 pgrid(blocks + (pc.sel ? 1 : 0));
+                if constexpr (MX) hipLaunchKernelGGL(pack_split_weight_kernel<S>, pgrid, dim3(256), 0, s, plans[0], w, static_cast<WE*>(ws), pc, off, n_off);
+                else hipLaunchKernelGGL(pack_forward_weight_kernel<T>, pgrid, dim3(256), 0, s, plans[0], w, static_cast<T*>(ws), pc, off, n_off);
+                if (int rc = check_launch("forward weight packing")) return rc;
             }
             size_t lds = 0;
             for (int k = 0; k < pc.nplans; ++k) {
-                const size_t l = (size_t)plans[k].cchunk * plans[k].hstride * sizeof(T) + (size_t)plans[k].hvol * 4;
+                const size_t l = halo_lds(plans[k]);
                 if (l > lds) lds = l;
             }
             const Params& Ph = plans[0];
-            using Kern = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const S*, const S*, S*, T*, int, unsigned, TailSplit);
-            Kern kern;
-            if (nw == 16) kern = MT == 1 ? forward_quad_kernel<T, ND, 1, 16, S> : forward_quad_kernel<T, ND, 2, 16, S>;
-            else kern = MT == 1 ? forward_quad_kernel<T, ND, 1, WAVESH, S> : MT == 2 ? forward_quad_kernel<T, ND, 2, WAVESH, S>
-                      : MT == 4 ? forward_quad_kernel<T, ND, 4, WAVESH, S> : forward_quad_kernel<T, ND, 8, WAVESH, S>;
+            using Kern = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const WE*, const S*, S*, T*, int, unsigned, TailSplit);
+            Kern kern = nullptr;
+            if constexpr (MX) {
+                if (shared) { if constexpr (ND == 2) kern = MT == 8 ? forward_shared_kernel<ND, 8, S> : forward_shared_kernel<ND, 4, S>; }
+                else if (nw == 16) kern = MT == 1 ? forward_split_kernel<ND, 1, 16, S> : forward_split_kernel<ND, 2, 16, S>;
+                else kern = MT == 1 ? forward_split_kernel<ND, 1, WAVESH, S> : MT == 2 ? forward_split_kernel<ND, 2, WAVESH, S>
+                                                                             : forward_split_kernel<ND, 4, WAVESH, S>;
+            } else {
+                if (nw == 16) kern = MT == 1 ? forward_quad_kernel<T, ND, 1, 16> : forward_quad_kernel<T, ND, 2, 16>;
+                else kern = MT == 1 ? forward_quad_kernel<T, ND, 1, WAVESH> : MT == 2 ? forward_quad_kernel<T, ND, 2, WAVESH>
+                          : MT == 4 ? forward_quad_kernel<T, ND, 4, WAVESH> : forward_quad_kernel<T, ND, 8, WAVESH>;
+            }
             T* part = reinterpret_cast<T*>(static_cast<char*>(ws) + align256(wq_bytes));      // partial sums, in the arithmetic type
             // A grid that ends in a partly filled round of workgroups: the units of that round, last in
             // the launch, are split over several workgroups each (every tsplit-th channel pass), so that
@@ -181,7 +233,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             long long whole = 0;
             TailSplit ts = {0u, 0, 0};
             if (fsplit == 1 && forward_tail_split()) {
-                const long long slots = forward_slots() ? forward_slots() : resident_workgroups(reinterpret_cast<const void*>(kern), nw * 64, lds);
+                const long long slots = forward_slots() ? forward_slots() : resident_workgroups(reinterpret_cast<const void*>(kern), (shared ? SHARED_WAVES : nw) * 64, lds);
                 const long long rest = units % slots;
                 constexpr double GEO = 0.45;    // tap geometry of a pass, in units of four channels' sampling and contraction
                 // cost of the longest workgroup when the passes of a unit (cch channels each) are dealt to cs workgroups
@@ -221,7 +273,8 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                         if (!forward_tail_two_runs() || cs + 1 > 8 || nb <= 0 || nb >= rest || (rest - nb) * cs > slots) continue;
                         double tb = 1e30;
                         int cchb = Ph.cchunk;
-                        for (int cch = Ph.cchunk; cch >= FQ; cch -= FQ) {
+                        const int step = Ph.cchunk % CM == 0 ? CM : FQ;
+                        for (int cch = Ph.cchunk; cch >= step; cch -= step) {
                             int np = 0;
                             const double c = wg_cost(cs + 1, cch, &np) / unit_cost + 0.05;
                             if (np >= cs + 1 && c < tb) { tb = c; cchb = cch; }
@@ -248,16 +301,17 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                             plans[k].hext[0], plans[k].hext[1], plans[k].hext[2], plans[k].cchunk, pc.base[k]);
             }
             const unsigned* sel = pc.sel;
-            if (int rc = launch_halo(kern, "forward_quad_kernel", grid, nw * 64, lds, s, Ph, alts, sel, in, off, (const S*)wt, bias, out, part,
+            if (int rc = launch_halo(kern, "forward halo kernel", grid, (shared ? SHARED_WAVES : nw) * 64, lds, s, Ph, alts, sel, in, off, (const WE*)ws, bias, out, part,
                                      tsplit > 1 ? tsplit : fsplit, (unsigned)whole, ts))
                 return rc;
             if (fsplit == 1 && tsplit == 1) return DCN_OK;
             if (tsplit > 1) {
                 using Join = void (*)(Params, PlanSet, const unsigned*, const T*, const S*, S*, int, unsigned, TailSplit);
                 Join join;
-                if (nw == 16) join = MT == 1 ? forward_join_tail_kernel<T, ND, 1, 16, S> : forward_join_tail_kernel<T, ND, 2, 16, S>;
+                if (shared) join = MT == 8 ? forward_join_tail_kernel<T, ND, 8, SHARED_COLS, S> : forward_join_tail_kernel<T, ND, 4, SHARED_COLS, S>;
+                else if (nw == 16) join = MT == 1 ? forward_join_tail_kernel<T, ND, 1, 16, S> : forward_join_tail_kernel<T, ND, 2, 16, S>;
                 else join = MT == 1 ? forward_join_tail_kernel<T, ND, 1, WAVESH, S> : MT == 2 ? forward_join_tail_kernel<T, ND, 2, WAVESH, S>
-                          : MT == 4 ? forward_join_tail_kernel<T, ND, 4, WAVESH, S> : forward_join_tail_kernel<T, ND, 8, WAVESH, S>;
+                          : MT == 4 || MX ? forward_join_tail_kernel<T, ND, 4, WAVESH, S> : forward_join_tail_kernel<T, ND, MX ? 4 : 8, WAVESH, S>;
                 hipLaunchKernelGGL(join, dim3((unsigned)((units - whole) * (MT * TN / JOIN_ROWS))), dim3(nw * TN), 0, s, Ph, alts, sel, (const T*)part, bias, out, tsplit, (unsigned)whole, ts);
                 return check_launch("forward_join_tail_kernel");
             }
@@ -273,6 +327,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
         if (declined) *declined = true;
         return DCN_OK;
     } else {
+    T* wt = static_cast<T*>(ws);
     if (int rc = relayout<T>(P, w, wt, 0, s)) return rc;
     // geometry whose halo does not fit in LDS: gather straight from global memory
     P.tiles = (P.outV + WAVES * TN - 1) / (WAVES * TN);

@@ -1,0 +1,624 @@
+// Forward kernel of the float32 and 16-bit operators: input halo in LDS, contraction on the 16-bit
+// matrix instructions.
+//
+//   out[n][g*M + m][pos] = sum_{cl,tap} W[g*M+m][cl][tap] * sample(in[n][g*Cg+cl], tap, pos)  (+ bias)
+//
+// replaces deformable_im2col + the per-group Sgemm of the reference
+// (deform3d/lib/deform_conv3d_cuda.cpp:110-148, deform2d_double/lib/deform_conv2d_cuda.cpp:102-138).
+//
+// Contraction of float32 operands.  A float32 value is the exact sum of three bfloat16 values: the
+// value rounded to bfloat16, the remainder rounded to bfloat16, and what is left (24 significant bits
+// = 3 x 8; each remainder is formed without rounding).  A product of two values is then nine products
+// of parts, each exact in float32, of which the three smallest (below 2^-24 of the product together)
+// are left out; the other six are summed by v_mfma_f32_32x32x16_bf16 into float32 accumulators,
+// smallest first.  Against float64, sums of 64 to 6912 products come out with 10 to 30 % less error
+// than from v_mfma_f32_32x32x2_f32, which rounds after every second product where this rounds
+// after every sixteenth.  Six instructions reduce over 16 slots in 93 ns per SIMD where the float32 ones
+// take 239 ns, and unlike those they run next to vector instructions.
+// Non-finite operands have no such parts (inf - inf): a workgroup whose result is not finite
+// everywhere works its block out once more through the float32 instructions, which also gives an
+// overflow of the parts the float32 meaning.
+//
+// Lane roles.  A wavefront owns 32 output positions; lane (j, q) works on position j and supplies
+// eight of the 16 reduction slots of an instruction: eight channels of tap tg*2 + q.  Every lane derives
+// the geometry of ONE (tap, position) per tap pair and no two lanes repeat each other's work; the halo
+// holds four channels of a voxel in 16 consecutive bytes, so that one wide LDS read per corner fetches
+// four of the lane's values.
+#pragma once
+#include <limits>
+#include "dcn_kernels.h"
+#include "dcn_forward.h"
+
+namespace dcn {
+
+constexpr int FG = 8;              // channels per reduction group: what a lane supplies to one matrix instruction
+
+// The 16-bit matrix instruction with 16 reduction slots, and how a lane's eight values become operands.
+template <typename S> struct Parts;
+template <> struct Parts<float> {
+    static constexpr int NP = 3;   // bfloat16 parts of a value
+    typedef __bf16 Vec __attribute__((ext_vector_type(8)));
+    static __device__ inline void split(const float v[8], Vec p[NP]) {
+        typedef __bf16 B2 __attribute__((ext_vector_type(2)));
+        typedef float F2 __attribute__((ext_vector_type(2)));
+        typedef unsigned U4 __attribute__((ext_vector_type(4)));
+        U4 out[NP];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            float a = v[2 * i], b = v[2 * i + 1];
+#pragma unroll
+            for (int k = 0; k < NP; ++k) {
+                const unsigned u = __builtin_bit_cast(unsigned, __builtin_convertvector(F2{a, b}, B2));
+                out[k][i] = u;
+                a -= __uint_as_float(u << 16);
+                b -= __uint_as_float(u & 0xffff0000u);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NP; ++k) p[k] = __builtin_bit_cast(Vec, out[k]);
+    }
+    static __device__ inline float join(const Vec p[NP], int e) { return ((float)p[2][e] + (float)p[1][e]) + (float)p[0][e]; }
+    // parts of one value for the packed weights; infinities and NaN stay in the first part, and so that
+    // a value near the largest float does not round to infinity its first part is then cut off instead
+    static __device__ inline void split1(float v, __bf16 p[NP]) {
+        p[0] = (__bf16)v;
+        if (!(fabsf((float)p[0]) <= std::numeric_limits<float>::max())) {
+            if (!(fabsf(v) <= std::numeric_limits<float>::max())) { p[1] = p[2] = (__bf16)0.f; return; }
+            p[0] = (__bf16)__uint_as_float(__float_as_uint(v) & 0xffff0000u);
+        }
+        p[1] = (__bf16)(v - (float)p[0]);
+        p[2] = (__bf16)((v - (float)p[0]) - (float)p[1]);
+    }
+    typedef __bf16 Elem;
+    static __device__ inline Mma<float>::Acc mma(Vec a, Vec b, Mma<float>::Acc c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+};
+template <> struct Parts<Bf16> {
+    static constexpr int NP = 1;
+    typedef __bf16 Vec __attribute__((ext_vector_type(8)));
+    typedef __bf16 Elem;
+    static __device__ inline void split(const float v[8], Vec p[NP]) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) p[0][e] = (__bf16)v[e];            // round to nearest even
+    }
+    static __device__ inline float join(const Vec p[NP], int e) { return (float)p[0][e]; }
+    static __device__ inline void split1(Bf16 v, __bf16 p[NP]) { p[0] = __builtin_bit_cast(__bf16, v.bits); }
+    static __device__ inline Mma<float>::Acc mma(Vec a, Vec b, Mma<float>::Acc c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+};
+template <> struct Parts<Fp16> {
+    static constexpr int NP = 1;
+    typedef _Float16 Vec __attribute__((ext_vector_type(8)));
+    typedef _Float16 Elem;
+    static __device__ inline void split(const float v[8], Vec p[NP]) {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) p[0][e] = (_Float16)v[e];
+    }
+    static __device__ inline float join(const Vec p[NP], int e) { return (float)p[0][e]; }
+    static __device__ inline void split1(Fp16 v, _Float16 p[NP]) { p[0] = v.v; }
+    static __device__ inline Mma<float>::Acc mma(Vec a, Vec b, Mma<float>::Acc c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
+};
+// acc[mt] += A[mt] * B for MT row tiles: the products of parts i, j with i + j < NP, smallest first
+template <typename S, int MT>
+__device__ inline void mma_parts(const typename Parts<S>::Vec a[MT][Parts<S>::NP], const typename Parts<S>::Vec b[Parts<S>::NP],
+                                 Mma<float>::Acc acc[MT]) {
+    constexpr int NP = Parts<S>::NP;
+#pragma unroll
+    for (int sum = NP - 1; sum >= 0; --sum)
+#pragma unroll
+        for (int i = 0; i <= sum; ++i)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) acc[mt] = Parts<S>::mma(a[mt][i], b[sum - i], acc[mt]);
+}
+
+// Packed weights: one slab per group of eight channels (groups start at the first channel of a
+// segment and at every eighth after it), in the order the lanes consume them:
+//   Wq[slab][tap pair][row tile][part][q][j][e] = part of W[m = tile*32 + j][channel = first + e][tap = tg*2 + q]
+// zero past M, past the last tap and past the segment.  An operand is 16 contiguous bytes of a lane and
+// 1 KB of a wavefront.
+template <typename S>
+__host__ __device__ inline size_t split_slab_elems(int kV, int Mp) {
+    return (size_t)((kV + 1) / 2) * Mp * 2 * FG * Parts<S>::NP;
+}
+
+// One thread per operand of a lane.  With pc.sel set the launch has one block more, which chooses the
+// halo plan from the offsets.
+template <typename S>
+__global__ __launch_bounds__(256) void pack_split_weight_kernel(Params P, const S* __restrict__ W, typename Parts<S>::Elem* __restrict__ Wq,
+                                                                PlanChoice pc, const S* __restrict__ off, size_t n_off) {
+    using PT = Parts<S>;
+    constexpr int TN = 32, NP = PT::NP;
+    const unsigned pack_blocks = pc.sel ? gridDim.x - 1 : gridDim.x;
+    if (blockIdx.x == pack_blocks) {
+        choose_plan(pc, off, n_off);
+        return;
+    }
+    const unsigned mtiles = P.Mp / TN, ntg = (P.kV + 1) / 2;
+    const unsigned per_slab = ntg * mtiles * 64;                                    // threads of a slab
+    const size_t total = (size_t)chunk_candidates<FG>(P.cpg, P.Cg, P.C_in) * per_slab;
+    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)pack_blocks * blockDim.x) {
+        const int c0 = chunk_candidate<FG>(P.cpg, P.Cg, (int)(i / per_slab));       // candidate first channel of a group
+        const int seg_b = max(c0 / P.cpg * P.cpg, c0 / P.Cg * P.Cg);
+        if ((c0 - seg_b) % FG) continue;
+        const int seg_e = min((c0 / P.cpg + 1) * P.cpg, (c0 / P.Cg + 1) * P.Cg);
+        unsigned r = (unsigned)(i % per_slab);
+        const int lane = r % 64; r /= 64;
+        const int tile = (int)(r % mtiles), tg = (int)(r / mtiles);
+        const int m = tile * TN + lane % TN, tap = tg * 2 + lane / TN, g = c0 / P.Cg;
+        typename PT::Vec part[NP];
+#pragma unroll
+        for (int e = 0; e < FG; ++e) {
+            S v = S();
+            if (m < P.M && tap < P.kV && c0 + e < seg_e) v = W[(((size_t)g * P.M + m) * P.Cg + (c0 + e - g * P.Cg)) * P.kV + tap];
+            typename PT::Elem p[NP];
+            PT::split1(v, p);
+#pragma unroll
+            for (int k = 0; k < NP; ++k) part[k][e] = p[k];
+        }
+        typename PT::Vec* dst = reinterpret_cast<typename PT::Vec*>(Wq) + (size_t)chunk_slot<FG>(P.cpg, P.Cg, c0) * per_slab * NP +
+                                ((size_t)tg * mtiles + tile) * NP * 64 + lane;
+#pragma unroll
+        for (int k = 0; k < NP; ++k) dst[k * 64] = part[k];
+    }
+}
+
+// Offset of halo voxel v inside a channel of the input, ~0u outside the volume.  The two divisions
+// are float multiplications: exact for the few thousand voxels of a halo.
+template <int ND>
+__device__ inline unsigned halo_voxel(const Params& P, const HaloPlan& H, const TileGeo<ND>& tg, int v, float inv1, float inv2) {
+    const int r = (int)(((float)v + 0.5f) * inv2);
+    int c[ND];
+    c[ND - 1] = v - __mul24(r, H.hext[2]);
+    if constexpr (ND == 3) {
+        c[0] = (int)(((float)r + 0.5f) * inv1);
+        c[1] = r - __mul24(c[0], H.hext[1]);
+    } else
+        c[0] = r;
+    bool inb = true;
+    unsigned lin = 0;
+#pragma unroll
+    for (int a = 0; a < ND; ++a) {
+        c[a] += tg.hb[a];
+        inb = inb && (unsigned)c[a] < (unsigned)P.in[slot<ND>(a)];
+        lin = lin * (unsigned)P.in[slot<ND>(a)] + (unsigned)c[a];
+    }
+    return inb ? lin : ~0u;
+}
+
+// What a workgroup of a forward launch works on: units are (block of positions, group, output-channel
+// chunk), workgroups of one tile are neighbours in an XCD-contiguous order.  The launch splits units as
+// described at forward_quad_kernel: csplit > 1 and whole = 0, every unit; whole > 0, the units from
+// `whole` on, in the two runs of TailSplit.
+struct ForwardUnit {
+    unsigned wg;                // unit
+    unsigned pslot;             // which partial sum of the split runs
+    int cz, cs;                 // this workgroup takes every cs-th channel pass, from the cz-th on
+    int cch;                    // channels per LDS pass
+    bool split;
+};
+__device__ inline ForwardUnit forward_unit(int cchunk, int csplit, unsigned whole, const TailSplit& ts) {
+    ForwardUnit u;
+    u.pslot = 0;
+    u.cz = 0;
+    u.cs = csplit;
+    u.cch = cchunk;
+    u.split = csplit > 1 && blockIdx.x >= whole;
+    if (!u.split) {
+        u.wg = xcd_contiguous(blockIdx.x, csplit > 1 ? whole : gridDim.x);
+        u.cs = 1;
+        return u;
+    }
+    const unsigned rel = blockIdx.x - whole, all = gridDim.x - whole;
+    const unsigned wgsA = ts.splitB ? ts.unitsA * (unsigned)csplit : all;
+    unsigned first = whole, r;
+    if (rel < wgsA) {
+        r = xcd_contiguous(rel, wgsA);
+        u.pslot = r;
+    } else {
+        r = xcd_contiguous(rel - wgsA, all - wgsA);
+        u.cs = ts.splitB;
+        first = whole + ts.unitsA;
+        u.pslot = wgsA + r;
+        u.cch = min(cchunk, ts.cchB);
+    }
+    u.wg = first + r / (unsigned)u.cs;
+    u.cz = (int)(r % (unsigned)u.cs);
+    return u;
+}
+
+// The halo in LDS: 16-byte cells [cell plane][halo voxel] that hold the next few channels of a voxel in
+// their storage format, four float32 or eight 16-bit ones: one wide read fetches them all.  (16-bit values
+// are widened after the read: half the LDS reads and twice the channels per pass of a float halo.)
+template <typename S> struct HaloCell {
+    static constexpr int CH = 16 / sizeof(S);
+    typedef typename std::conditional<sizeof(S) == 4, float, typename Parts<S>::Elem>::type V;
+    typedef V Vec __attribute__((ext_vector_type(CH)));
+    static __device__ inline V raw(S v) { return __builtin_bit_cast(V, v); }
+};
+
+// Stages `nch` channels of the halo, planes of hstride cells; missing channels of a short last group
+// and voxels outside the volume hold zero.  Returns whether the thread met a non-finite value (CHECK).
+template <int ND, int WGS, bool CHECK, typename S>
+__device__ inline bool stage_halo(const Params& P, const HaloPlan& H, const TileGeo<ND>& tg, const S* __restrict__ chan0, int nch,
+                                  typename HaloCell<S>::Vec* __restrict__ sIn) {
+    constexpr int CH = HaloCell<S>::CH;
+    // an item is a cell: consecutive threads take consecutive voxels, several items of a thread are in flight
+    const int items = (nch + CH - 1) / CH * H.hvol;
+    const float inv2 = 1.f / (float)H.hext[2], inv1 = 1.f / (float)H.hext[1], inv = 1.f / (float)H.hvol;
+    const size_t step = (size_t)P.inV * sizeof(S);
+    bool bad = false;
+#pragma unroll 4
+    for (int it = threadIdx.x; it < items; it += WGS) {
+        const int grp = (int)(((float)it + 0.5f) * inv), v = it - __mul24(grp, H.hvol);
+        const unsigned t = halo_voxel<ND>(P, H, tg, v, inv1, inv2);
+        const char* cp = reinterpret_cast<const char*>(chan0) + (size_t)(t == ~0u ? 0u : t) * sizeof(S) + (size_t)(grp * CH) * step;
+        const int last = nch - 1 - grp * CH;                    // >= CH - 1 but in a short last group
+        typename HaloCell<S>::Vec cell;
+#pragma unroll
+        for (int e = 0; e < CH; ++e) {
+            const S x = *reinterpret_cast<const S*>(cp + (size_t)min(e, last) * step);
+            if constexpr (CHECK) bad = bad || !(fabsf(Store<S>::ld(x)) <= std::numeric_limits<float>::max());
+            cell[e] = HaloCell<S>::raw(x);
+        }
+#pragma unroll
+        for (int e = 0; e < CH; ++e) cell[e] = (e <= last && t != ~0u) ? cell[e] : (typename HaloCell<S>::V)0.f;
+        sIn[(size_t)grp * H.hstride + v] = cell;
+    }
+    return bad;
+}
+
+// Geometry of a lane's (tap, position), following the reference sampler
+// (deform3d/lib/deform_conv3d_cuda_kernel.cu:21-26,40-45,123-124) in a branch-free form: the coordinate
+// is clamped into [0, size - 1]; low corner = floor, fraction toward the high corner = clamped
+// coordinate - floor.  Where the reference collapses the high corner onto the low one (p <= 0,
+// p >= size - 1) the fraction is 0, so the corner one step further carries weight 0 and every sample
+// uses the same eight (four) cells at fixed strides.
+template <int ND> struct SplitTap {
+    float pq[ND];               // coordinate
+    float cw[1 << ND];          // corner weights w_l * w_h * w_w, all zero without a sample in the halo
+    unsigned base;              // low corner's halo cell, 0 without a sample in the halo
+    bool near, far;             // sampled from the halo / reaches past it
+};
+// k0, k1: kernel coordinates of the taps of lane groups 0 and 1 (uniform); rim_far: samples in the
+// collapse zones are not taken from the halo.
+template <int ND>
+__device__ inline void split_geometry(const Params& P, const HaloPlan& H, const TileGeo<ND>& tg, const int ib[ND], int q, const int* k0,
+                                      const int* k1, const float* ofs, bool tap_ok, bool rim_far, SplitTap<ND>& t) {
+    bool inside = tap_ok, inhalo = true;
+    float f[ND];
+    int u[ND];
+#pragma unroll
+    for (int a = 0; a < ND; ++a) {
+        const int sa = slot<ND>(a);
+        const float top = (float)(P.in[sa] - 1);
+        const int kd = k0[a] * P.dil[sa];
+        int dk = k1[a] * P.dil[sa] - kd;
+        asm volatile("" : "+s"(dk));                            // (scalar arithmetic)
+        const float pa = (float)(__mul24(q, dk) + ib[a] + kd) + ofs[a];
+        const float pc = __builtin_amdgcn_fmed3f(pa, 0.f, top);
+        const float fl = floorf(pc);
+        t.pq[a] = pa;
+        f[a] = pc - fl;
+        inside = inside && fabsf(pa - pc) < 1.f;                // -1 < p < size, false for NaN
+        u[a] = (int)fl - tg.hb[a];
+        inhalo = inhalo && (unsigned)u[a] < (unsigned)(H.hext[sa] - 1);
+    }
+    if (rim_far) {
+#pragma unroll
+        for (int a = 0; a < ND; ++a) inhalo = inhalo && t.pq[a] > 0.f && t.pq[a] < (float)(P.in[slot<ND>(a)] - 1);
+    }
+    t.near = inside && inhalo;
+    t.far = inside && !inhalo;
+    unsigned base;
+    if constexpr (ND == 3) base = (unsigned)(__mul24(__mul24(u[0], H.hext[1]) + u[1], H.hext[2]) + u[2]);
+    else base = (unsigned)(__mul24(u[0], H.hext[2]) + u[1]);
+    t.base = t.near ? base : 0u;
+    float* cw = t.cw;
+    if constexpr (ND == 3) {
+        const float fl = t.near ? f[0] : 0.f, gl = t.near ? 1.f - f[0] : 0.f;
+        const float fh = f[1], gh = 1.f - fh, fw = f[2], gw = 1.f - fw;
+        const float a00 = gl * gh, a01 = gl * fh, a10 = fl * gh, a11 = fl * fh;
+        cw[0] = a00 * gw; cw[1] = a00 * fw; cw[2] = a01 * gw; cw[3] = a01 * fw;
+        cw[4] = a10 * gw; cw[5] = a10 * fw; cw[6] = a11 * gw; cw[7] = a11 * fw;
+    } else {
+        const float fh = t.near ? f[0] : 0.f, gh = t.near ? 1.f - f[0] : 0.f, fw = f[1], gw = 1.f - fw;
+        cw[0] = gh * gw; cw[1] = gh * fw; cw[2] = fh * gw; cw[3] = fh * fw;
+    }
+}
+
+// Weighted corner sums of the channels of a cell (element by element: a vector times scalar product
+// would hold four copies of every weight).  The sums are formed here, not where the contraction uses
+// them, so that one cell's corners are in flight at a time.  row, plane: cells between neighbours along h and l.
+template <int ND, typename S>
+__device__ inline void cell_sum(const typename HaloCell<S>::Vec* cell, unsigned row, unsigned plane, const float* cw, float* v) {
+    constexpr int NC = 1 << ND, CH = HaloCell<S>::CH;
+    typename HaloCell<S>::Vec c[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) c[i] = cell[(i >> 2) * plane + ((i >> 1) & 1) * row + (i & 1)];
+#pragma unroll
+    for (int e = 0; e < CH; ++e) {
+#pragma unroll
+        for (int i = 0; i < NC; ++i) v[e] = i ? v[e] + (float)c[i][e] * cw[i] : (float)c[i][e] * cw[i];
+    }
+#pragma unroll
+    for (int e = 0; e < CH; ++e) asm volatile("" : "+v"(v[e]));
+    __builtin_amdgcn_sched_barrier(0);
+}
+// ... of the eight channels of group grp of a chunk of nch channels
+template <int ND, typename S>
+__device__ inline void group_sum8(const typename HaloCell<S>::Vec* sIn, unsigned base, int grp, int nch, int hstride, unsigned row,
+                                  unsigned plane, const float* cw, float val[FG]) {
+    constexpr int CH = HaloCell<S>::CH;
+#pragma unroll
+    for (int e = 0; e < FG; ++e) val[e] = 0.f;
+    const typename HaloCell<S>::Vec* hp = sIn + base + (size_t)grp * (FG / CH) * hstride;
+    cell_sum<ND, S>(hp, row, plane, cw, val);
+    if constexpr (CH == 4)
+        if (grp * FG + 4 < nch) cell_sum<ND, S>(hp + hstride, row, plane, cw, val + 4);
+}
+
+// Samples that reach past the halo: val[e] of such lanes = channels c .. c + 7 of the chunk (below nch)
+// from global memory, with the reference's corner rule on the same coordinate.
+template <int ND, typename S>
+__device__ inline void far_values(const Params& P, const SplitTap<ND>& t, const S* __restrict__ chan0, int c, int nch, float val[FG]) {
+    constexpr int NC = 1 << ND;
+    TapGeo<float, ND> g;
+    g.inside = t.far;
+#pragma unroll
+    for (int a = 0; a < ND; ++a) {
+        float pa = t.pq[a];
+        asm volatile("" : "+v"(pa));       // (worked out here, not hoisted into the common path)
+        const int l = t.far ? (int)pa : 0;
+        g.p[a] = pa;
+        g.lo[a] = l;
+        g.hi[a] = (pa >= (float)(P.in[slot<ND>(a)] - 1) || pa <= 0.f) ? l : l + 1;
+        g.f[a] = pa - (float)l;
+    }
+    tap_corner_idx<float, ND>(P, g);
+#pragma unroll 1
+    for (int e = 0; e < FG; ++e) {
+        float cc[NC];
+        const S* ch = chan0 + (size_t)min(c + e, nch - 1) * P.inV;
+#pragma unroll
+        for (int i = 0; i < NC; ++i) cc[i] = Store<S>::ld(ch[g.idx[i]]);
+        const float v = c + e < nch ? interp<float, ND>(cc, g.f) : 0.f;
+#pragma unroll
+        for (int x = 0; x < FG; ++x) val[x] = t.far && x == e ? v : val[x];
+    }
+}
+
+// kernel coordinates of the next tap (uniform)
+template <int ND>
+__device__ inline void next_tap(const Params& P, int k[ND]) {
+    int carry = 1;
+#pragma unroll
+    for (int a = ND - 1; a > 0; --a) {
+        k[a] += carry;
+        carry = k[a] >= P.k[slot<ND>(a)] ? 1 : 0;
+        k[a] = carry ? 0 : k[a];
+    }
+    k[0] += carry;
+}
+
+// offsets of this lane's tap of pair tgi (tap tgi * 2 + q, clamped to a legal tap) at position pos
+template <int ND, typename S>
+__device__ inline void load_pair_offsets(const Params& P, const S* __restrict__ off_dg, int tgi, int q, unsigned pos, float ofs[ND]) {
+    const char* ob = reinterpret_cast<const char*>(off_dg + (size_t)tgi * 2 * ND * P.outV);      // uniform
+    unsigned lo = ((q && tgi * 2 + 1 < P.kV ? ND * P.outV : 0u) + pos) * (unsigned)sizeof(S);
+    asm volatile("" : "+v"(lo));               // (not hoisted into registers that stay live)
+#pragma unroll
+    for (int a = 0; a < ND; ++a) {
+        ofs[a] = Store<S>::ld(*reinterpret_cast<const S*>(ob + lo));
+        ob += (size_t)P.outV * sizeof(S);
+    }
+}
+
+// The contraction of a lane's values on the float32 instructions, one channel of the tap pair at a
+// time (results that are not finite).  nvalid: how many of the values exist.
+template <typename S, int MT>
+__device__ inline void mma_exact(const typename Parts<S>::Vec a[MT][Parts<S>::NP], const float val[FG], bool live, int nvalid, Mma<float>::Acc acc[MT]) {
+#pragma unroll 1
+    for (int e = 0; e < FG; ++e) {
+        float b = 0.f;
+#pragma unroll
+        for (int x = 0; x < FG; ++x) b = x == e && e < nvalid && live ? val[x] : b;
+        if constexpr (sizeof(S) == 2) b = Store<S>::ld(Store<S>::st(b));
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) {
+            float w = 0.f;
+#pragma unroll
+            for (int x = 0; x < FG; ++x) w = x == e && e < nvalid ? Parts<S>::join(a[mt], x) : w;
+            acc[mt] = Mma<float>::mma(w, b, acc[mt]);
+        }
+    }
+}
+
+// NaN or infinite when a result of the lane is (or when the sum overflows: its workgroup then repeats in vain)
+template <int NT>
+__device__ inline bool all_finite(const Mma<float>::Acc* acc) {
+    float s = 0.f;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < Mma<float>::NACC; ++r) s += fabsf(acc[t][r]);
+    return s <= std::numeric_limits<float>::max();
+}
+
+// Writes a 32 x 32 result tile: row m0 + r of group g's output channels (m0 uniform), this lane's position.
+// dst: the sample's output, or its partial sums (no bias).
+template <typename O, typename S>
+__device__ inline void store_tile(const Params& P, O* __restrict__ dst, const S* __restrict__ bias, int g, int m0, int q, unsigned pos,
+                                  const Mma<float>::Acc& acc) {
+    O* base = dst + ((size_t)g * P.M + m0) * P.outV;                   // uniform
+    const unsigned at = (unsigned)q * 4 * P.outV + pos;
+    const int rows = P.M - m0 - q * 4;
+#pragma unroll
+    for (int r = 0; r < Mma<float>::NACC; ++r) {
+        const int row = Mma<float>::row(r, 0);
+        if (row < rows) {
+            float v = acc[r];
+            if (bias) v += Store<S>::ld(bias[g * P.M + m0 + row + q * 4]);
+            (base + (size_t)row * P.outV)[at] = Store<O>::st(v);
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------
+// Up to four row tiles (128 output channels) per wavefront, each wavefront sampling its own 32
+// positions straight into its operands.  NW wavefronts; dynamic LDS = cchunk * hstride * sizeof(S) bytes,
+// cchunk a multiple of eight (or four, float32: half of the reduction slots then stay empty).
+// Binding: the LDS reads of the corners in 3-D (64 channels, 27 taps, 200 704 positions: 1.2e7 16-byte
+// reads with 46 % bank conflicts of random offsets hold a CU's LDS 0.32 of 0.52 ms; 0.64 ms on the
+// float32 instructions), operand latency in 2-D.
+// (up to two row tiles: four wavefronts per SIMD, i.e. at most 128 registers)
+template <int ND, int MT, int NW, typename S>
+__global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel(Params P, PlanSet alts, const unsigned* __restrict__ sel,
+                                                           const S* __restrict__ in, const S* __restrict__ off,
+                                                           const typename Parts<S>::Elem* __restrict__ Wq, const S* __restrict__ bias,
+                                                           S* __restrict__ out, float* __restrict__ part, int csplit, unsigned whole,
+                                                           TailSplit ts) {
+    HaloPlan H;
+    if (!chosen_halo(P, alts, sel, H)) return;          // another launch runs the chosen plan
+    using PT = Parts<S>;
+    using MM = Mma<float>;
+    typedef typename PT::Vec Vec;
+    typedef typename PT::Elem Elem;
+    constexpr int TN = 32, WGS = NW * 64, NP = PT::NP;
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    __shared__ int sNonFinite, sRedo;
+    typedef typename HaloCell<S>::Vec Cell;
+    Cell* sIn = reinterpret_cast<Cell*>(smem_raw);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int j = lane % TN, q = lane / TN;
+    const ForwardUnit U = forward_unit(H.cchunk, csplit, whole, ts);
+    const unsigned gm = U.wg % (unsigned)(P.G * P.mchunks);
+    const int g = gm / P.mchunks, mchunk = gm % P.mchunks;
+
+    TileGeo<ND> tg;
+    tile_decode<ND>(P, H, U.wg / (unsigned)(P.G * P.mchunks), tg);
+    const int n = tg.n;
+    int ib[ND];
+    unsigned pos;
+    bool valid;
+    {
+        int o[ND];
+        valid = tile_position<ND>(P, tg, wave * TN + j, o, pos);
+#pragma unroll
+        for (int a = 0; a < ND; ++a) ib[a] = o[a] * P.stride[slot<ND>(a)] - P.pad[slot<ND>(a)];
+    }
+
+    typename MM::Acc acc[MT];
+    const int ntg = (P.kV + 1) / 2;
+    const unsigned mtiles = P.Mp / TN;
+    const unsigned per_slab = (unsigned)ntg * mtiles * NP * 64;        // operands (16 bytes) of a slab
+    const unsigned row = (unsigned)H.hext[2], plane = ND == 3 ? (unsigned)(H.hext[1] * H.hext[2]) : 0u;
+    const unsigned a_lane = (unsigned)lane * 16;         // byte offset of this lane's operand
+    const unsigned a_tg = mtiles * NP * 64;
+    constexpr int LINES = (MT * NP * 8 + NW - 1) / NW;             // 128-byte lines of a step's weights per wavefront
+    const unsigned touch_at = (unsigned)min(wave * LINES + min(lane, LINES - 1), MT * NP * 8 - 1) * 128;
+    const int cg0 = g * P.Cg, cg1 = cg0 + P.Cg;
+
+    if (threadIdx.x == 0) sRedo = 0;                    // ordered before the checks by the barriers of the first chunk
+    // exact: the contraction on the float32 instructions, with the reference's treatment of non-finite
+    // input next to the rim.
+    auto work = [&](auto exact_tag) {
+        constexpr bool exact = decltype(exact_tag)::value;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[mt] = acc_zero<float>();
+        int chunk_no = 0;
+        for (int dg = cg0 / P.cpg; dg <= (cg1 - 1) / P.cpg; ++dg) {
+            const int cb = max(cg0, dg * P.cpg), ce = min(cg1, (dg + 1) * P.cpg);
+            const S* off_dg = off + ((size_t)n * P.DG + dg) * P.kV * ND * P.outV;
+            for (int cc0 = cb; cc0 < ce; cc0 += U.cch) {
+                if ((chunk_no++) % U.cs != U.cz) continue;                     // another workgroup's chunk (uniform)
+                const int nch = min(U.cch, ce - cc0);
+                const int ngrp = (nch + FG - 1) / FG;
+                const S* chan0 = in + ((size_t)n * P.C_in + cc0) * P.inV;      // workgroup-uniform
+                float ofs[ND];
+                load_pair_offsets<ND, S>(P, off_dg, 0, q, pos, ofs);
+                if (exact && threadIdx.x == 0) sNonFinite = 0;
+                __syncthreads();                                               // readers of the previous chunk are done
+                if (stage_halo<ND, WGS, exact, S>(P, H, tg, chan0, nch, sIn)) sNonFinite = 1;
+                __syncthreads();
+                // Non-finite input in this halo (a non-finite sample always leads to the second pass): the
+                // branch-free sampler reads the cell next to a collapsed corner with weight 0, and 0 * inf would
+                // be NaN where the reference never touches that voxel
+                // (deform3d/lib/deform_conv3d_cuda_kernel.cu:24-26).  Samples in the collapse zones (p <= 0 or
+                // p >= size - 1 on some axis) are then taken from global memory with the reference's corner rule.
+                const bool rim_far = exact && sNonFinite != 0;                 // uniform
+                // (passes of four channels, where no more fit: every second one takes the upper half of its
+                // group -- the operands from four elements further on, whose last four then meet zeros)
+                const int upper = (cc0 - cb) & 4;
+                const Elem* wchunk = Wq + ((size_t)chunk_slot<FG>(P.cpg, P.Cg, cc0 - upper) * per_slab * FG + (size_t)mchunk * MT * NP * 64 * FG + upper);
+                int k0[ND];                            // kernel coordinates of the tap pair, counted up in scalar registers
+#pragma unroll
+                for (int a = 0; a < ND; ++a) k0[a] = 0;
+                int touched = 0;
+                for (int tgi = 0; tgi < ntg; ++tgi) {
+                    int k1[ND];
+#pragma unroll
+                    for (int a = 0; a < ND; ++a) k1[a] = k0[a];
+                    next_tap<ND>(P, k1);
+                    SplitTap<ND> t;
+                    split_geometry<ND>(P, H, tg, ib, q, k0, k1, ofs, valid && tgi * 2 + q < P.kV, rim_far, t);
+                    const bool any_far = __any(t.far); // rare: some sample of this wave reaches past the halo
+                    const Elem* wp = wchunk + (size_t)tgi * a_tg * FG;
+                    for (int grp = 0; grp < ngrp; ++grp) {
+                        float val[FG];
+                        // The weights of the next step come into the L1 while this one is worked on: every
+                        // wavefront touches its share of their cache lines (128 channels, 3-D: 0.94 ms against 1.19).
+                        asm volatile("" ::"v"(touched));
+                        if constexpr (!exact) {
+                            const Elem* nx = grp + 1 < ngrp ? wp + (size_t)per_slab * FG : wchunk + (size_t)min(tgi + 1, ntg - 1) * a_tg * FG;
+                            touched = *reinterpret_cast<const int*>(reinterpret_cast<const char*>(nx) + touch_at);
+                        }
+                        group_sum8<ND, S>(sIn, t.base, grp, nch, H.hstride, row, plane, t.cw, val);
+                        if (__builtin_expect(any_far, 0)) far_values<ND, S>(P, t, chan0, grp * FG, nch, val);
+                        // the next tap pair's offsets travel behind the contraction (earlier, they would be
+                        // live through the rare branch above, which takes the registers)
+                        if (grp + 1 == ngrp) load_pair_offsets<ND, S>(P, off_dg, min(tgi + 1, ntg - 1), q, pos, ofs);
+                        Vec a8[MT][NP];
+#pragma unroll
+                        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                            for (int k = 0; k < NP; ++k) __builtin_memcpy(&a8[mt][k], reinterpret_cast<const char*>(wp) + (mt * NP + k) * 1024 + a_lane, 16);
+                        __builtin_amdgcn_sched_barrier(0);          // all of them on their way while the operand is split
+                        if constexpr (!exact) {
+                            Vec b8[NP];
+                            PT::split(val, b8);
+                            mma_parts<S, MT>(a8, b8, acc);
+                        } else
+                            mma_exact<S, MT>(a8, val, t.near || t.far, nch - grp * FG, acc);
+                        wp += (size_t)per_slab * FG;
+                    }
+                    next_tap<ND>(P, k1);
+#pragma unroll
+                    for (int a = 0; a < ND; ++a) k0[a] = k1[a];
+                }
+            }
+        }
+    };
+    work(std::false_type{});
+    if (valid && !all_finite<MT>(acc)) sRedo = 1;
+    __syncthreads();
+    if (__builtin_expect(sRedo, 0)) work(std::true_type{});
+
+    if (U.split && whole > 0) {
+        // partial sums of a unit of the last round: [split workgroup][MT * TN rows][NW * TN positions]
+        float* dst = part + (size_t)U.pslot * (MT * TN) * (NW * TN) + q * 4 * (NW * TN) + wave * TN + j;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int r = 0; r < MM::NACC; ++r) dst[(mt * TN + MM::row(r, 0)) * (NW * TN)] = acc[mt][r];
+        return;
+    }
+    if (!valid) return;
+    // unsplit: the output with bias; every unit split: a partial output tensor per cz, the bias is added when they are joined
+    const size_t sample = (size_t)n * P.C_out * P.outV;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int m0 = (mchunk * MT + mt) * TN;
+        if (U.split) store_tile<float, S>(P, part + (size_t)U.cz * P.N * P.C_out * P.outV + sample, nullptr, g, m0, q, pos, acc[mt]);
+        else store_tile<S, S>(P, out + sample, bias, g, m0, q, pos, acc[mt]);
+    }
+}
+
+}  // namespace dcn

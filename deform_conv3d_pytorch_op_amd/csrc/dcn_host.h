@@ -4,6 +4,7 @@
 #include "../../include/dcn_amd.h"
 #include "dcn_kernels.h"
 #include "dcn_forward.h"
+#include "dcn_forward_split.h"
 
 #include <cstdio>
 #include <cstdlib>
@@ -91,12 +92,13 @@ template <typename T> inline size_t workspace_need(int N, int C_in, int C_out, s
     const int M = C_out / G, Cg = C_in / G;
     int MT, mchunks, Mp, Cgp;
     fwd_weight_pad<T>(M, Cg, MT, mchunks, Mp, Cgp);
-    // forward: [g][tap][c][m] for the kernel without LDS tiling, or one slab per four channels for the
-    // halo kernel (its row padding is at most eight tiles' worth)
+    // forward: [g][tap][c][m] for the kernel without LDS tiling, or one slab per four (float64) or eight
+    // channels for the halo kernels (their row padding is at most eight tiles' worth)
     const int TNf = Mma<T>::TN;
     const int Mp8 = ((M + TNf - 1) / TNf + 7) / 8 * 8 * TNf;
     const size_t fwd_plain = (size_t)G * kV * (Mp > Mp8 ? Mp : Mp8) * Cgp * sizeof(T);
-    const size_t fwd_quad = slab_bound((size_t)C_in, G, cpg, FQ) * forward_slab_elems<T>(kV, Mp8) * sizeof(T);
+    const size_t fwd_quad = sizeof(T) == 4 ? slab_bound((size_t)C_in, G, cpg, FG) * split_slab_elems<float>(kV, Mp8) * 2
+                                           : slab_bound((size_t)C_in, G, cpg, FQ) * forward_slab_elems<T>(kV, Mp8) * sizeof(T);
     const size_t fwd = (fwd_plain > fwd_quad ? fwd_plain : fwd_quad) + forward_partial_bound(N, C_out, outV, sizeof(T));
     // (+ the last whole 256-byte block of the workspace: weight bounds and the plan the device chose)
     const size_t bwd = bwd_data_weight_bytes<T>(M, Cg, kV, G, cpg) + 2 * align256((size_t)N * C_in * inV * sizeof(T)) + 512;
@@ -186,6 +188,7 @@ inline int relayout(const Params& P, const T* w, T* wt, int channel_fastest, hip
 //   DCN_FORWARD_TAIL=0     forward pass: never split only the units of the last, partly filled round of workgroups (n > 1: n ways)
 //   DCN_FORWARD_TAIL2=0    forward pass: the split units of the last round all the same number of ways, never in two runs
 //   DCN_FORWARD_SLOTS=n    forward pass: plan the launch as if n workgroups ran at once (test hook)
+//   DCN_FORWARD_SHARED=0   forward pass, float32 and 16-bit: never share the sampled columns of a block among wavefronts
 //   DCN_SCATTER_BUDGET_KB  LDS per workgroup of the privatised scatter kernel (default 144)
 //   DCN_SCATTER=global     scatter grad-input with global atomics instead of the LDS-privatised kernel
 //   DCN_COORD=separate     grad_offset from the channels-last kernel instead of the fused LDS-halo kernel
@@ -290,6 +293,10 @@ static bool forward_tail_two_runs() {    // DCN_FORWARD_TAIL2=0: the split units
     static const int v = [] { const char* e = getenv("DCN_FORWARD_TAIL2"); return (e && atoi(e) == 0) ? 0 : 1; }();
     return v != 0;
 }
+static bool forward_shared() {           // DCN_FORWARD_SHARED=0: the forward pass always samples in every wavefront (forward_split_kernel)
+    static const int v = [] { const char* e = getenv("DCN_FORWARD_SHARED"); return (e && atoi(e) == 0) ? 0 : 1; }();
+    return v != 0;
+}
 static bool fused_pair() {              // DCN_FUSED_PAIR=0: float32 LDS cells of the fused backward kernel hold one channel each (64-bit)
     static const int v = [] { const char* e = getenv("DCN_FUSED_PAIR"); return (e && atoi(e) == 0) ? 0 : 1; }();
     return v != 0;
@@ -343,7 +350,7 @@ static int forced_csplit() {    // DCN_CSPLIT=n: workgroups per (tile, deformabl
 
 template <typename T, int ND>
 inline bool plan_halo(Params& P, size_t budget, int m, int max_chunk = 1 << 30, size_t cell_bytes = sizeof(T), int waves = WAVESH,
-               bool smallest_halo = false, int chunk_mult = 0, const int* blocks = nullptr, int wmult = 1) {
+               bool smallest_halo = false, int chunk_mult = 0, const int* blocks = nullptr, int wmult = 1, bool table = true) {
     const int npos = waves * Mma<T>::TN;        // positions per workgroup, one column tile per wavefront
     int td[3] = {1, 1, 1};
     if (ND == 3) { td[1] = 8; td[2] = 8; td[0] = npos / 64; }
@@ -380,10 +387,12 @@ inline bool plan_halo(Params& P, size_t budget, int m, int max_chunk = 1 << 30, 
     }
     if (hvol > MAX_HVOL) return false;
     P.hvol = (int)hvol;
-    P.hstride = ((int)hvol + 63) / 64 * 64 + 32;
+    // (table: the kernel keeps an offset per halo voxel in LDS and channel planes of its own stride)
+    P.hstride = table ? ((int)hvol + 63) / 64 * 64 + 32 : (int)hvol;
+    const size_t tbytes = table ? (size_t)hvol * 4 : 0;
     const int KL = chunk_mult > 0 ? chunk_mult : Mma<T>::KL;      // channels per pass come in multiples of this
-    if (budget <= (size_t)hvol * 4) return false;
-    long long cc = (long long)((budget - (size_t)hvol * 4) / ((size_t)P.hstride * cell_bytes));
+    if (budget <= tbytes) return false;
+    long long cc = (long long)((budget - tbytes) / ((size_t)P.hstride * cell_bytes));
     cc = cc / KL * KL;
     const int seg = P.cpg < P.Cg ? P.cpg : P.Cg;          // longest run of channels sharing offsets and group
     const int seg_up = (seg + KL - 1) / KL * KL;
