@@ -6,13 +6,17 @@ There is no fallback: if the shared library is missing the import of an operator
 error that says how to build it.
 """
 import ctypes
+import importlib.machinery
+import importlib.util
 import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 SO_PATH = os.path.join(_HERE, "csrc", "libdcn_amd.so")
+NATIVE_PATH = os.path.join(_HERE, "_native.so")
 
 _c_int, _c_vp, _c_sz = ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t
 _lib = None
+_native = None
 
 N_GEOM = {3: 23, 2: 17}     # number of int arguments of DCN3D_GEOMETRY / DCN2D_GEOMETRY
 N_CONV2D_GEOM = 16          # ... of CONV2D_GEOMETRY
@@ -68,6 +72,24 @@ def load():
         raise ImportError("libdcn_amd.so has ABI version %d, expected 1" % L.dcn_version())
     _lib = L
     return L
+
+
+def native():
+    """The C++ extension with the autograd layer (csrc/dcn_torch.cpp), on the same libdcn_amd.so."""
+    global _native
+    if _native is None:
+        load()
+        if not os.path.exists(NATIVE_PATH):
+            raise ImportError("_native.so is not built (expected at %s). Build it with "
+                              "`python -m deform_conv3d_pytorch_op_amd.build`; there is no fallback." % NATIVE_PATH)
+        import torch  # noqa: F401  (its libraries have to be there first)
+        loader = importlib.machinery.ExtensionFileLoader(__package__ + "._native", NATIVE_PATH)
+        spec = importlib.util.spec_from_loader(loader.name, loader)
+        module = importlib.util.module_from_spec(spec)
+        loader.exec_module(module)
+        module.set_error(DcnError)
+        _native = module
+    return _native
 
 
 def check(rc):

@@ -1,5 +1,5 @@
-"""Builds csrc/libdcn_amd.so with hipcc for gfx950 (in-tree, no JIT cache).  The translation units
-compile side by side.
+"""Builds csrc/libdcn_amd.so with hipcc for gfx950 and the C++ extension _native.so on top of it
+(in-tree, no JIT cache).  The translation units compile side by side.
 
     python -m deform_conv3d_pytorch_op_amd.build
 """
@@ -7,12 +7,14 @@ import glob
 import os
 import subprocess
 import sys
+import sysconfig
 import tempfile
 from concurrent.futures import ThreadPoolExecutor
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 SO = os.path.join(CSRC, "libdcn_amd.so")
+NATIVE = os.path.join(HERE, "_native.so")
 
 HIPCC_FLAGS = [
     "--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC",
@@ -34,15 +36,34 @@ def _run(cmd, verbose):
         print(out)
 
 
+def _torch_flags():
+    import torch
+    root = os.path.dirname(torch.__file__)
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    include = [os.path.join(root, "include"), os.path.join(root, "include", "torch", "csrc", "api", "include"),
+               os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]
+    compile_flags = ["-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1",
+                     "-D_GLIBCXX_USE_CXX11_ABI=%d" % int(torch._C._GLIBCXX_USE_CXX11_ABI)] + ["-I" + d for d in include]
+    link_flags = ["-L" + os.path.join(root, "lib"), "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip",
+                  "-L" + CSRC, "-ldcn_amd", "-Wl,-rpath,$ORIGIN/csrc"]
+    return compile_flags, link_flags
+
+
 def build(verbose=False):
     hipcc = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
+    cxx = os.environ.get("CXX", "g++")
     sources = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
-    jobs = min(len(sources), int(os.environ.get("MAX_JOBS", 0) or os.cpu_count() or 1))
+    jobs = min(len(sources) + 1, int(os.environ.get("MAX_JOBS", 0) or os.cpu_count() or 1))
+    compile_flags, link_flags = _torch_flags()
     with tempfile.TemporaryDirectory() as tmp:
         objects = [os.path.join(tmp, os.path.basename(s) + ".o") for s in sources]
+        native = os.path.join(tmp, "dcn_torch.o")
+        commands = [[cxx] + compile_flags + ["-c", "-o", native, os.path.join(CSRC, "dcn_torch.cpp")]]
+        commands += [[hipcc] + HIPCC_FLAGS + ["-c", "-o", o, s] for s, o in zip(sources, objects)]
         with ThreadPoolExecutor(jobs) as pool:
-            list(pool.map(lambda so: _run([hipcc] + HIPCC_FLAGS + ["-c", "-o", so[1], so[0]], verbose), zip(sources, objects)))
+            list(pool.map(lambda c: _run(c, verbose), commands))
         _run([hipcc] + HIPCC_FLAGS + ["-shared", "-o", SO] + objects, verbose)
+        _run([cxx, "-shared", "-o", NATIVE, native] + link_flags, verbose)
     return SO
 
 
