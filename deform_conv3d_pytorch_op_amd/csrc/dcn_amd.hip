@@ -47,6 +47,21 @@ size_t copies16_bytes(int N, int C_in, int C_out, size_t inV, size_t outV, int k
     return 2 * align256(in * 4) + 2 * align256(w * 4) + 2 * align256(off * 4) + align256(out * 4) + align256((size_t)C_out * 4);
 }
 
+// grad_weight alone, added to what it holds
+template <typename T, int ND>
+int backward_weight(const Geometry& g, const T* in, const T* off, const T* gout, T* gw, void* ws, size_t ws_bytes, hipStream_t s) {
+    Params P;
+    if (int rc = validate(g, P)) return rc;
+    if (!in || !off || !gout || !gw) return fail(DCN_E_ARGUMENT, "null tensor pointer");
+    if (int rc = device_info(nullptr)) return rc;
+    WeightCall<T, T> call;
+    Prep prep;
+    const PlanChoice none = {};
+    if (int rc = backward_weight_plan<T, ND, T>(P, in, gout, ws, ws_bytes, false, call, prep, nullptr)) return rc;
+    if (int rc = launch_prepare<T, T>(P, none, prep, static_cast<const T*>(nullptr), off, 0, s)) return rc;
+    return backward_weight_run<T, ND, T>(call, off, gw, nullptr, true, s);
+}
+
 template <typename S, int ND>
 int forward16(const Geometry& g, const S* in, const S* w, const S* off, const S* bias, S* out, void* ws, size_t ws_bytes,
               hipStream_t s) {
@@ -112,8 +127,16 @@ int backward_weight16(const Geometry& g, const S* in, const S* off, const S* gou
     if (!fin || !foff || !fgout || !fgw) return fail(DCN_E_WORKSPACE, "workspace too small");
     if (int rc = widen(gw, fgw, z.w, s)) return rc;               // grad_weight is accumulated into
     bool declined = true;
-    if (native16())
-        if (int rc = backward_weight_native16<S, ND>(P, in, off, gout, fgw, c.p, c.left, s, &declined)) return rc;
+    if (native16()) {
+        WeightCall<float, S> call;
+        Prep prep;
+        const PlanChoice none = {};
+        if (int rc = backward_weight_plan<float, ND, S>(P, in, gout, c.p, c.left, false, call, prep, &declined)) return rc;
+        if (!declined) {
+            if (int rc = launch_prepare<float, S>(P, none, prep, static_cast<const S*>(nullptr), off, 0, s)) return rc;
+            if (int rc = backward_weight_run<float, ND, S>(call, off, fgw, nullptr, true, s)) return rc;
+        }
+    }
     if (declined) {
         if (int rc = widen(in, fin, z.in, s)) return rc;
         if (int rc = widen(off, foff, z.off, s)) return rc;
@@ -121,6 +144,103 @@ int backward_weight16(const Geometry& g, const S* in, const S* off, const S* gou
         if (int rc = backward_weight<float, ND>(g, fin, foff, fgout, fgw, c.p, c.left, s)) return rc;
     }
     return narrow(fgw, gw, z.w, s);
+}
+
+// ---------------------------------------------------------------------------------------------
+// The backward pass of a layer in one call: the gradients asked for (null: not wanted), written, not
+// added.  What the operators need beforehand -- cleared buffers, packed weights, channels-last copies,
+// the sums for grad_bias -- is one launch (backward_prepare_kernel).
+// Workspace: [ 16-bit storage: float gradients | backward_input_offset | backward_weight ].
+template <typename S> struct Wide { typedef float type; };
+template <> struct Wide<double> { typedef double type; };
+template <typename S>
+__global__ __launch_bounds__(256) void narrow_gradients_kernel(const float* __restrict__ a, S* __restrict__ da, size_t na, const float* __restrict__ b,
+                                                               S* __restrict__ db, size_t nb, const float* __restrict__ c, S* __restrict__ dc, size_t nc,
+                                                               const float* __restrict__ d, S* __restrict__ dd, size_t nd) {
+    const size_t step = (size_t)gridDim.x * 256, first = (size_t)blockIdx.x * 256 + threadIdx.x;
+    for (size_t i = first; i < na; i += step) da[i] = S::narrow(a[i]);
+    for (size_t i = first; i < nb; i += step) db[i] = S::narrow(b[i]);
+    for (size_t i = first; i < nc; i += step) dc[i] = S::narrow(c[i]);
+    for (size_t i = first; i < nd; i += step) dd[i] = S::narrow(d[i]);
+}
+template <typename S, int ND>
+int layer_backward(const Geometry& g, const S* in, const S* w, const S* off, const S* gout, S* gin, S* goff, S* gw, S* gb, void* ws, size_t ws_bytes,
+                   hipStream_t s, unsigned flags) {
+    typedef typename Wide<S>::type T;
+    constexpr bool S16 = !std::is_same<S, T>::value;
+    Params P;
+    if (int rc = validate(g, P)) return rc;
+    const bool data = gin || goff;
+    if (!in || !w || !off || !gout || (data && (!gin || !goff)) || (gb && !gw)) return fail(DCN_E_ARGUMENT, "null tensor pointer");
+    if (int rc = device_info(nullptr)) return rc;
+    const Sizes16 z = sizes16(P, ND);
+    char* p = static_cast<char*>(ws);
+    size_t left = ws ? ws_bytes : 0;
+    auto take = [&](size_t bytes) -> void* {
+        bytes = align256(bytes);
+        if (bytes > left) return nullptr;
+        void* r = p;
+        p += bytes;
+        left -= bytes;
+        return r;
+    };
+    T *tgin, *tgoff, *tgw, *tgb;
+    if constexpr (S16) {
+        tgin = data ? static_cast<T*>(take(z.in * 4)) : nullptr;
+        tgoff = data ? static_cast<T*>(take(z.off * 4)) : nullptr;
+        tgw = gw ? static_cast<T*>(take(z.w * 4)) : nullptr;
+        tgb = gb ? static_cast<T*>(take((size_t)P.C_out * 4)) : nullptr;
+        if ((data && (!tgin || !tgoff)) || (gw && !tgw) || (gb && !tgb)) return fail(DCN_E_WORKSPACE, "workspace too small");
+    } else {
+        tgin = gin; tgoff = goff; tgw = gw; tgb = gb;
+    }
+    const size_t dbytes = backward_data_need<T>(P.N, P.C_in, P.C_out, P.inV, P.kV, P.G, P.cpg);
+    const size_t wbytes = backward_weight_need<T>(P.N, P.C_in, P.C_out, P.inV, P.outV, P.kV, P.G);
+    void *dws = data ? take(dbytes) : nullptr, *wws = gw ? take(wbytes) : nullptr;
+    if ((data && !dws) || (gw && !wws)) return fail(DCN_E_WORKSPACE, "workspace too small");
+    Prep prep;
+    WeightCall<T, S> call;
+    const PlanChoice none = {};
+    if (data) prep.zero(tgin, z.in * sizeof(T));
+    // (16-bit storage: the kernels that read it may decline a layer, which then runs on widened copies)
+    bool wdeclined = S16 && !native16(), ddeclined = wdeclined;
+    if (gw && !wdeclined)
+        if (int rc = backward_weight_plan<T, ND, S>(P, in, gout, wws, wbytes, gb != nullptr, call, prep, S16 ? &wdeclined : nullptr)) return rc;
+    if (data && !ddeclined)
+        if (int rc = backward_input_offset<T, ND, S>(g, in, w, off, gout, tgin, tgoff, dws, dbytes, s, flags, S16 ? &ddeclined : nullptr, &prep)) return rc;
+    if (!data || ddeclined)
+        if (int rc = launch_prepare<T, S>(P, none, prep, w, off, 0, s)) return rc;
+    const T *fin = nullptr, *fw = nullptr, *foff = nullptr, *fgout = nullptr;
+    if constexpr (S16) {
+        if ((data && ddeclined) || (gw && wdeclined)) {
+            float* copy[4] = {static_cast<float*>(take(z.in * 4)), static_cast<float*>(take(z.w * 4)), static_cast<float*>(take(z.off * 4)), static_cast<float*>(take(z.out * 4))};
+            if (!copy[0] || !copy[1] || !copy[2] || !copy[3]) return fail(DCN_E_WORKSPACE, "workspace too small");
+            if (int rc = widen(in, copy[0], z.in, s)) return rc;
+            if (int rc = widen(w, copy[1], z.w, s)) return rc;
+            if (int rc = widen(off, copy[2], z.off, s)) return rc;
+            if (int rc = widen(gout, copy[3], z.out, s)) return rc;
+            fin = copy[0]; fw = copy[1]; foff = copy[2]; fgout = copy[3];
+        }
+    }
+    if (data && ddeclined)
+        if (int rc = backward_input_offset<T, ND>(g, fin, fw, foff, fgout, tgin, tgoff, dws, dbytes, s, flags)) return rc;
+    if (gw && !wdeclined) {
+        if (int rc = backward_weight_run<T, ND, S>(call, off, tgw, tgb, false, s)) return rc;
+    } else if (gw) {
+        WeightCall<T, T> wide;
+        Prep wprep;
+        if (int rc = backward_weight_plan<T, ND, T>(P, fin, fgout, wws, wbytes, gb != nullptr, wide, wprep, nullptr)) return rc;
+        if (int rc = launch_prepare<T, T>(P, none, wprep, fw, foff, 0, s)) return rc;
+        if (int rc = backward_weight_run<T, ND, T>(wide, foff, tgw, tgb, false, s)) return rc;
+    }
+    if constexpr (S16) {
+        const size_t na = data ? z.in : 0, nb = data ? z.off : 0, nc = gw ? z.w : 0, nd = gb ? (size_t)P.C_out : 0, most = na + nb + nc;
+        const unsigned blocks = (unsigned)((most + 1023) / 1024 > 8192 ? 8192 : (most + 1023) / 1024 + 1);
+        hipLaunchKernelGGL(narrow_gradients_kernel<S>, dim3(blocks), dim3(256), 0, s, (const float*)tgin, gin, na, (const float*)tgoff, goff, nb, (const float*)tgw, gw,
+                           nc, (const float*)tgb, gb, nd);
+        return check_launch("narrow_gradients_kernel");
+    }
+    return DCN_OK;
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -250,6 +370,45 @@ size_t dcn_workspace_bytes_for(int elem_size, int batch, int input_c, int output
     return elem_size == 8
                ? workspace_need<double>(batch, input_c, output_c, input_volume, output_volume, kernel_volume, group, cpg)
                : workspace_need<float>(batch, input_c, output_c, input_volume, output_volume, kernel_volume, group, cpg);
+}
+
+size_t dcn_layer_backward_workspace_bytes(int elem_size, int nd, int batch, int input_c, int output_c, size_t input_volume, size_t output_volume,
+                                          int kernel_volume, int group, int channel_per_deformable_group) {
+    if (group <= 0 || batch <= 0 || input_c <= 0 || output_c <= 0 || kernel_volume <= 0 || input_volume == 0 || output_volume == 0 ||
+        channel_per_deformable_group <= 0 || input_c % channel_per_deformable_group || input_c % group || output_c % group || nd < 2 || nd > 3)
+        return 0;
+    const int cpg = channel_per_deformable_group;
+    if (elem_size == 8)
+        return align256(backward_data_need<double>(batch, input_c, output_c, input_volume, kernel_volume, group, cpg)) +
+               align256(backward_weight_need<double>(batch, input_c, output_c, input_volume, output_volume, kernel_volume, group));
+    return align256(backward_data_need<float>(batch, input_c, output_c, input_volume, kernel_volume, group, cpg)) +
+           align256(backward_weight_need<float>(batch, input_c, output_c, input_volume, output_volume, kernel_volume, group)) +
+           (elem_size == 2 ? copies16_bytes(batch, input_c, output_c, input_volume, output_volume, kernel_volume, group, cpg) : 0);
+}
+
+int dcn_layer_backward(int nd, int dtype, const void* input, const void* weight, const void* offset, const void* grad_output, void* grad_input, void* grad_offset,
+                       void* grad_weight, void* grad_bias, const int* geometry, void* workspace, size_t workspace_bytes, void* stream, unsigned flags) {
+    if (!geometry || (nd != 2 && nd != 3)) return fail(DCN_E_ARGUMENT, "two or three axes and their geometry");
+    if (flags & ~(unsigned)DCN_FLAG_OOB_OFFSET_GRAD_ZERO) return fail(DCN_E_ARGUMENT, "unknown flag");
+    if (flags && dtype >= 2) return fail(DCN_E_ARGUMENT, "oob_offset_grad='zero' is available in float32 and float64 only");
+    const int* v = geometry;
+    Geometry g{nd, v[0], v[1], v[2], {1, 1, 1}, {1, 1, 1}, {1, 1, 1}, {0, 0, 0}, {1, 1, 1}, {1, 1, 1}, 0, 0};
+    v += 3;
+    for (int* axis : {g.in, g.out, g.k, g.pad, g.stride, g.dil})
+        for (int a = 3 - nd; a < 3; ++a) axis[a] = *v++;
+    g.cpg = v[0];
+    g.G = v[1];
+#define LAYER(S, ND)                                                                                                                              \
+    layer_backward<S, ND>(g, (const S*)input, (const S*)weight, (const S*)offset, (const S*)grad_output, (S*)grad_input, (S*)grad_offset,         \
+                          (S*)grad_weight, (S*)grad_bias, workspace, workspace_bytes, static_cast<hipStream_t>(stream), flags)
+    switch (dtype) {
+        case 0: return nd == 3 ? LAYER(float, 3) : LAYER(float, 2);
+        case 1: return nd == 3 ? LAYER(double, 3) : LAYER(double, 2);
+        case 2: return nd == 3 ? LAYER(Bf16, 3) : LAYER(Bf16, 2);
+        case 3: return nd == 3 ? LAYER(Fp16, 3) : LAYER(Fp16, 2);
+        default: return fail(DCN_E_ARGUMENT, "unknown data type");
+    }
+#undef LAYER
 }
 
 int dcn3d_forward_noalloc_f32(const float* input, const float* weight, const float* offset, const float* bias,

@@ -2,7 +2,7 @@
 
 namespace dcn {
 
-#define INSTANTIATE(T, ND, S) template int backward_input_offset<T, ND, S>(const Geometry&, const S*, const S*, const S*, const S*, T*, T*, void*, size_t, hipStream_t, unsigned, bool*);
+#define INSTANTIATE(T, ND, S) template int backward_input_offset<T, ND, S>(const Geometry&, const S*, const S*, const S*, const S*, T*, T*, void*, size_t, hipStream_t, unsigned, bool*, Prep*);
 INSTANTIATE(float, 2, float)
 
 }  // namespace dcn

@@ -4,24 +4,6 @@
 
 namespace dcn {
 
-template <typename T>
-int absmax(const T* w, size_t n, float* out, hipStream_t s) {
-    hipLaunchKernelGGL(fill_zero_kernel<float>, dim3(1), dim3(64), 0, s, out, (size_t)1);
-    if (int rc = check_launch("fill_zero_kernel")) return rc;
-    const unsigned blocks = (unsigned)((n + 1023) / 1024 > 128 ? 128 : (n + 1023) / 1024);
-    hipLaunchKernelGGL(absmax_kernel<T>, dim3(blocks ? blocks : 1), dim3(256), 0, s, w, n, out);
-    return check_launch("absmax_kernel");
-}
-// out[0] = max |w|, out[1] = largest norm over the output channels of a group of an (input channel, tap)
-// column; `out` was cleared by the pack_weight_kernel launched before
-template <typename T>
-int weight_bounds(const Params& P, const T* w, float* out, hipStream_t s) {
-    const size_t cols = (size_t)P.Cg * P.kV;
-    if (P.G > 65535) return fail(DCN_E_ARGUMENT, "more than 65535 convolution groups");
-    hipLaunchKernelGGL(weight_bounds_kernel<T>, dim3((unsigned)((cols + 63) / 64), (unsigned)P.G), dim3(512), 0, s, w, P.M, cols, out);
-    return check_launch("weight_bounds_kernel");
-}
-
 // S = T: the float32 / float64 operator.  S = Bf16 / Fp16 (T = float): input, weight, offset and
 // grad_output are in that storage format (the gradients are float), and only the fused kernel with
 // its grad_output operand in registers serves them, on the 16-bit matrix instructions; where it
@@ -29,7 +11,7 @@ int weight_bounds(const Params& P, const T* w, float* out, hipStream_t s) {
 // float32 operator.
 template <typename T, int ND, typename S>
 int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* off, const S* gout, T* gin,
-                          T* goff, void* ws, size_t ws_bytes, hipStream_t s, unsigned flags, bool* declined) {
+                          T* goff, void* ws, size_t ws_bytes, hipStream_t s, unsigned flags, bool* declined, Prep* given) {
     constexpr bool S16 = !std::is_same<S, T>::value;
     Params P;
     if (int rc = validate(g, P)) return rc;
@@ -49,13 +31,15 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
     T* gin_cl = reinterpret_cast<T*>(static_cast<char*>(ws) + wbytes + tbytes);
     const int TN = Mma<T>::TN;
     const int mk = bwd_data_mk<T>(P.M);
-    // weight bounds (two floats) and, 64 bytes further, the plan chosen on the device: in the last whole
-    // 256-byte block of the workspace when that lies behind the two channels-last regions
-    // (dcn_workspace_bytes counts it), else at the start of the channels-last gradient, which the LDS
-    // paths do not use
-    const size_t tail_at = ws_bytes >= 256 ? (ws_bytes - 256) / 256 * 256 : 0;
+    // weight bounds and, 64 bytes into the block behind them, the plan chosen on the device: in the last whole
+    // 256-byte blocks of the workspace when those lie behind the two channels-last regions (dcn_workspace_bytes counts them),
+    // else at the start of the channels-last gradient, which the LDS paths do not use
+    const size_t tail_at = ws_bytes >= BWD_TAIL ? (ws_bytes - 256) / 256 * 256 - (BWD_TAIL - 256) : 0;
     const bool tail_words = tail_at >= wbytes + 2 * tbytes;
-    float* wmax = tail_words ? reinterpret_cast<float*>(static_cast<char*>(ws) + tail_at) : reinterpret_cast<float*>(gin_cl);
+    if (!tail_words && tbytes < BWD_TAIL) return fail(DCN_E_WORKSPACE, "workspace too small");
+    float* bounds = tail_words ? reinterpret_cast<float*>(static_cast<char*>(ws) + tail_at) : reinterpret_cast<float*>(gin_cl);
+    Prep own;
+    Prep& prep = given ? *given : own;
     const dim3 tgrid((P.inV + 31) / 32, (unsigned)(P.C_in + 31) / 32, (unsigned)P.N), tblock(32, 8);
 
     // 1) one kernel: scatter privatised in LDS + coordinate gradient from an LDS input halo
@@ -257,42 +241,30 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             pc.margin[k] = pc.margin[pc.nplans - 1];
             pc.base[k] = 1e30f;
         }
-        unsigned* sel = (pc.nplans > 1 || offer_global) ? reinterpret_cast<unsigned*>(wmax + 16) : nullptr;
+        unsigned* sel = (pc.nplans > 1 || offer_global) ? reinterpret_cast<unsigned*>(bounds + 2 * BOUND_BLOCKS + 16) : nullptr;
         pc.sel = sel;
         pc.global_cost = offer_global ? 6.5f : 0.f;
         const size_t n_off = (size_t)P.N * P.DG * P.kV * ND * P.outV;
-        // weights in the lane order of the kernel's operand loads, one slab per channel chunk; the
-        // first launch clears the weight bounds and chooses the plan
+        // one launch prepares: weights in the lane order of the kernel's operand loads, one slab per channel
+        // chunk (variant 9: the row order that leaves the eight channels of a tap in one lane), their bounds,
+        // the choice of the plan, grad_offset cleared where it is added to, and the caller's jobs
+        if (sel) prep.add(PREP_PLAN, 1);
         for (int k = 0; k < pc.nplans; ++k) {
             bool packed = false;
             for (int e = 0; e < k; ++e) packed = packed || fp[e].wt == fp[k].wt;
             if (packed) continue;
-            const bool sixteen = fp[k].cch == 16, eight = fp[k].cch == 8, wide = fp[k].wide;
-            const size_t total = packed_weight_elems<T, S>(P.M, P.kV, (size_t)(sixteen ? chunk_candidates<16>(P.cpg, P.Cg, P.C_in)
-                                                                            : eight ? chunk_candidates<8>(P.cpg, P.Cg, P.C_in)
-                                                                                    : chunk_candidates<4>(P.cpg, P.Cg, P.C_in)), fp[k].cch);
-            const unsigned blocks = (unsigned)((total + 255) / 256 > 8192 ? 8192 : (total + 255) / 256);
-            PlanChoice pk = pc;
-            if (k > 0) pk.sel = nullptr;
-            float* bounds = k == 0 ? wmax : nullptr;
-            S* dst = const_cast<S*>(fp[k].wt);
-            const dim3 pgrid(blocks + (pk.sel ? 1 : 0));
-            // (wide: row order that leaves the eight channels of a tap in one lane)
-            if (sixteen) hipLaunchKernelGGL((pack_weight_kernel<T, 16, false, S>), pgrid, dim3(256), 0, s, P, w, dst, bounds, pk, off, n_off);
-            else if (wide) hipLaunchKernelGGL((pack_weight_kernel<T, 8, true, S>), pgrid, dim3(256), 0, s, P, w, dst, bounds, pk, off, n_off);
-            else if (eight) hipLaunchKernelGGL((pack_weight_kernel<T, 8, false, S>), pgrid, dim3(256), 0, s, P, w, dst, bounds, pk, off, n_off);
-            else hipLaunchKernelGGL((pack_weight_kernel<T, 4, false, S>), pgrid, dim3(256), 0, s, P, w, dst, bounds, pk, off, n_off);
-            if (int rc = check_launch("pack_weight_kernel")) return rc;
+            const size_t total = packed_weight_elems<T, S>(P.M, P.kV, (size_t)(fp[k].cch == 16 ? chunk_candidates<16>(P.cpg, P.Cg, P.C_in)
+                                                                            : fp[k].cch == 8 ? chunk_candidates<8>(P.cpg, P.Cg, P.C_in)
+                                                                                             : chunk_candidates<4>(P.cpg, P.Cg, P.C_in)), fp[k].cch);
+            PrepJob& job = prep.add(PREP_PACK, (unsigned)((total + 255) / 256 > 8192 ? 8192 : (total + 255) / 256));
+            job.variant = fp[k].wide ? 9 : fp[k].cch;
+            job.dst = const_cast<S*>(fp[k].wt);
         }
-        if (int rc = weight_bounds<S>(P, w, wmax, s)) return rc;
+        prep.add(PREP_BOUNDS, BOUND_BLOCKS).dst = bounds;
         bool any_atomic = false;
         for (int k = 0; k < pc.nplans; ++k) any_atomic = any_atomic || fp[k].zero_goff;
-        if (any_atomic) {
-            const size_t nel = (size_t)P.N * P.DG * P.kV * ND * P.outV;
-            const unsigned fb = (unsigned)((nel + 1023) / 1024 > 8192 ? 8192 : (nel + 1023) / 1024);
-            hipLaunchKernelGGL(fill_zero_kernel<T>, dim3(fb), dim3(256), 0, s, goff, nel);
-            if (int rc = check_launch("fill_zero_kernel")) return rc;
-        }
+        if (any_atomic) prep.zero(goff, n_off * sizeof(T));
+        if (int rc = launch_prepare<T, S>(P, pc, prep, w, off, n_off, s)) return rc;
         // one launch per set of plans that differ in nothing but the halo
         unsigned launched = 0;
         for (int k = 0; k < pc.nplans; ++k) {
@@ -325,7 +297,7 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             if (lds > 48 * 1024)
                 if (int rc = raise_lds_limit(reinterpret_cast<const void*>(fp[k].kern), lds)) return rc;
             hipLaunchKernelGGL(fp[k].kern, dim3((unsigned)(fp[k].whole + (fp[k].items - fp[k].whole) * fp[k].csplit)), dim3(fp[k].nw * 64), lds, s,
-                               fp[k].Ph, alts, (const unsigned*)sel, in, off, fp[k].wt, gout, (const float*)wmax, gin, goff, fp[k].csplit, (unsigned)fp[k].whole,
+                               fp[k].Ph, alts, (const unsigned*)sel, in, off, fp[k].wt, gout, (const float*)bounds, gin, goff, fp[k].csplit, (unsigned)fp[k].whole,
                                fp[k].goff_atomic);
             if (int rc = check_launch("backward_input_halo_kernel")) return rc;
         }
@@ -359,6 +331,11 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
     } else {
 
     // 2) grad_offset from the channels-last kernel, grad_input from the LDS-privatised scatter
+    {
+        prep.add(PREP_BOUNDS, BOUND_BLOCKS).dst = bounds;
+        PlanChoice none = {};
+        if (int rc = launch_prepare<T, S>(P, none, prep, w, off, 0, s)) return rc;
+    }
     if (int rc = relayout<T>(P, w, wt, 1, s)) return rc;
     {   // zero tap slabs behind the last group
         const size_t used = (size_t)P.G * P.kV * P.Mp * P.Cgp, pad = (size_t)TAP_PAD * P.Mp * P.Cgp;
@@ -394,7 +371,6 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
         if (!input_only)
             if (int rc = check_launch("backward_data_kernel")) return rc;
         const size_t lds = (size_t)Ph.cchunk * Ph.hstride * 8 + (size_t)Ph.hvol * 4;
-        if (int rc = absmax<T>(w, (size_t)P.C_out * P.Cg * P.kV, wmax, s)) return rc;
         const dim3 hgrid((unsigned)Ph.N * Ph.tiles * Ph.DG);
         T* nogoff = nullptr;
         PlanSet alts;
@@ -403,10 +379,10 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
         const unsigned* nosel = nullptr;
         if (Ph.cchunk == 8)
             return launch_halo(backward_input_halo_kernel<T, ND, 8, false, false, 0, WAVESH>, "backward_input_halo_kernel", hgrid, WGH, lds, s,
-                               Ph, alts, nosel, in, off, (const T*)wt, gout, (const float*)wmax, gin, nogoff, 1, 0u, 0);
+                               Ph, alts, nosel, in, off, (const T*)wt, gout, (const float*)bounds, gin, nogoff, 1, 0u, 0);
         if (Ph.cchunk == 4)
             return launch_halo(backward_input_halo_kernel<T, ND, 4, false, false, 0, WAVESH>, "backward_input_halo_kernel", hgrid, WGH, lds, s,
-                               Ph, alts, nosel, in, off, (const T*)wt, gout, (const float*)wmax, gin, nogoff, 1, 0u, 0);
+                               Ph, alts, nosel, in, off, (const T*)wt, gout, (const float*)bounds, gin, nogoff, 1, 0u, 0);
         return fail(DCN_E_LAUNCH, "no scatter kernel for this channel chunk");
     }
     // halo does not fit in LDS: scatter with global atomics on the channels-last copy

@@ -5,6 +5,7 @@
 #include "dcn_kernels.h"
 #include "dcn_forward.h"
 #include "dcn_forward_split.h"
+#include "dcn_prepare.h"
 
 #include <cstdio>
 #include <cstdlib>
@@ -88,30 +89,39 @@ inline size_t forward_partial_bound(int N, int C_out, size_t outV, size_t elem) 
     const size_t all = (size_t)FWD_MAX_SPLIT * N * C_out * outV * elem;
     return align256(all < FWD_PARTIAL_CAP ? all : FWD_PARTIAL_CAP) + 256;
 }
-template <typename T> inline size_t workspace_need(int N, int C_in, int C_out, size_t inV, size_t outV, int kV, int G, int cpg = 0) {
+// last bytes of a backward_input_offset workspace: bounds of the weights, and the plan chosen on the device
+constexpr size_t BWD_TAIL = BOUND_BLOCKS * 2 * sizeof(float) + 256;
+template <typename T> inline size_t forward_need(int N, int C_in, int C_out, size_t outV, int kV, int G, int cpg = 0) {
     const int M = C_out / G, Cg = C_in / G;
     int MT, mchunks, Mp, Cgp;
     fwd_weight_pad<T>(M, Cg, MT, mchunks, Mp, Cgp);
-    // forward: [g][tap][c][m] for the kernel without LDS tiling, or one slab per four (float64) or eight
+    // [g][tap][c][m] for the kernel without LDS tiling, or one slab per four (float64) or eight
     // channels for the halo kernels (their row padding is at most eight tiles' worth)
     const int TNf = Mma<T>::TN;
     const int Mp8 = ((M + TNf - 1) / TNf + 7) / 8 * 8 * TNf;
     const size_t fwd_plain = (size_t)G * kV * (Mp > Mp8 ? Mp : Mp8) * Cgp * sizeof(T);
     const size_t fwd_quad = sizeof(T) == 4 ? slab_bound((size_t)C_in, G, cpg, FG) * split_slab_elems<float>(kV, Mp8) * 2
                                            : slab_bound((size_t)C_in, G, cpg, FQ) * forward_slab_elems<T>(kV, Mp8) * sizeof(T);
-    const size_t fwd = (fwd_plain > fwd_quad ? fwd_plain : fwd_quad) + forward_partial_bound(N, C_out, outV, sizeof(T));
-    // (+ the last whole 256-byte block of the workspace: weight bounds and the plan the device chose)
-    const size_t bwd = bwd_data_weight_bytes<T>(M, Cg, kV, G, cpg) + 2 * align256((size_t)N * C_in * inV * sizeof(T)) + 512;
-    // backward_weight: two channels-last copies + one partial weight per position split (at most 256 splits,
-    // and never more than about 4096 workgroups: see bww_plan)
+    return (fwd_plain > fwd_quad ? fwd_plain : fwd_quad) + forward_partial_bound(N, C_out, outV, sizeof(T)) + 1024;
+}
+template <typename T> inline size_t backward_data_need(int N, int C_in, int C_out, size_t inV, int kV, int G, int cpg = 0) {
+    return bwd_data_weight_bytes<T>(C_out / G, C_in / G, kV, G, cpg) + 2 * align256((size_t)N * C_in * inV * sizeof(T)) + BWD_TAIL + 512;
+}
+// two channels-last copies + one partial weight per position split (at most 256 splits, and never more
+// than about 4096 workgroups: see bww_plan) + the strips of grad_output's sums
+template <typename T> inline size_t backward_weight_need(int N, int C_in, int C_out, size_t inV, size_t outV, int kV, int G) {
     const int TNq = Mma<T>::TN;
     const long long tiles_lb = (long long)kV * ((C_in + TNq - 1) / TNq);           // lower bound of kV * nct * mchunks
     long long split_ub = (4096 + tiles_lb - 1) / tiles_lb;
     if (split_ub > 256) split_ub = 256;
     if (split_ub < 1) split_ub = 1;
-    const size_t bww = align256((size_t)N * C_in * inV * sizeof(T)) + align256((size_t)N * C_out * outV * sizeof(T)) +
-                       align256((size_t)split_ub * kV * C_out * Cg * sizeof(T));
-    size_t need = fwd > bwd ? fwd : bwd;
+    return align256((size_t)N * C_in * inV * sizeof(T)) + align256((size_t)N * C_out * outV * sizeof(T)) +
+           align256((size_t)split_ub * kV * C_out * (C_in / G) * sizeof(T)) + align256((size_t)N * last_strips((unsigned)outV) * C_out * sizeof(T));
+}
+template <typename T> inline size_t workspace_need(int N, int C_in, int C_out, size_t inV, size_t outV, int kV, int G, int cpg = 0) {
+    const size_t fwd = forward_need<T>(N, C_in, C_out, outV, kV, G, cpg), bwd = backward_data_need<T>(N, C_in, C_out, inV, kV, G, cpg),
+                 bww = backward_weight_need<T>(N, C_in, C_out, inV, outV, kV, G);
+    const size_t need = fwd > bwd ? fwd : bwd;
     return need > bww ? need : bww;
 }
 
@@ -468,13 +478,29 @@ constexpr unsigned FLAG_INPUT_ONLY = 0x100u;     // internal: see backward_input
 template <typename T, int ND, typename S = T>
 int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* bias, S* out, void* ws, size_t ws_bytes,
             hipStream_t s, bool* declined = nullptr);
+// prep: jobs that belong to the caller, done in the launch that prepares this operator
 template <typename T, int ND, typename S = T>
 int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* off, const S* gout, T* gin, T* goff, void* ws,
-                          size_t ws_bytes, hipStream_t s, unsigned flags = 0, bool* declined = nullptr);
-template <typename T, int ND>
-int backward_weight(const Geometry& g, const T* in, const T* off, const T* gout, T* gw, void* ws, size_t ws_bytes, hipStream_t s);
-template <typename S, int ND>
-int backward_weight_native16(const Params& Pin, const S* in, const S* off, const S* gout, float* fgw, void* ws, size_t ws_bytes,
-                             hipStream_t s, bool* declined);
+                          size_t ws_bytes, hipStream_t s, unsigned flags = 0, bool* declined = nullptr, Prep* prep = nullptr);
+// backward_weight in two halves: where its operands go (jobs for the preparing launch), and the kernels.
+// T arithmetic, S storage (T, or 16 bits: channel pairs, see backward_weight16_kernel).
+template <typename T, typename S> struct WeightCall {
+    Params P;
+    int MT;
+    S *in_cl, *gout_cl;
+    T *partial, *sums;
+    int nsums;
+};
+template <typename T, int ND, typename S>
+int backward_weight_plan(const Params& P, const S* in, const S* gout, void* ws, size_t ws_bytes, bool bias, WeightCall<T, S>& c, Prep& prep, bool* declined);
+template <typename T, int ND, typename S>
+int backward_weight_run(const WeightCall<T, S>& c, const S* off, T* gw, T* gb, bool accumulate, hipStream_t s);
+
+template <typename T, typename S>
+inline int launch_prepare(const Params& P, const PlanChoice& pc, const Prep& prep, const S* w, const S* off, size_t n_off, hipStream_t s) {
+    if (prep.jobs.n == 0) return DCN_OK;
+    hipLaunchKernelGGL((backward_prepare_kernel<T, S>), dim3(prep.blocks), dim3(256), 0, s, P, pc, prep.jobs, w, off, n_off);
+    return check_launch("backward_prepare_kernel");
+}
 
 }  // namespace dcn

@@ -218,27 +218,19 @@ __device__ inline void choose_plan(const PlanChoice& pc, const S* __restrict__ o
 // WIDE (float, CCH = 8): row j of a pass holds (tap, channel) = (2 * (j / 16) + (j / 4) % 2,
 // 4 * ((j / 8) % 2) + j % 4) instead of (j / CCH, j % CCH): the MFMA then leaves all eight channels
 // of a tap in one lane (fused_row_tap / fused_row_channel).
-// `bounds` (two floats, may be null) is cleared for the weight_bounds_kernel that follows.
-// With pc.sel set the launch has one block more, which chooses the halo plan from the offsets.
 // S = Bf16 / Fp16: Wp[slab][pass][k][lane][r] = W[m = 8 * k + 4 * q + r][...], four values per lane and step.
+// Block `block` of `blocks` blocks of 256 threads.
 template <typename T, int CCH, bool WIDE = false, typename S = T>
-__global__ void pack_weight_kernel(Params P, const S* __restrict__ W, S* __restrict__ Wp, float* __restrict__ bounds,
-                                   PlanChoice pc, const S* __restrict__ off, size_t n_off) {
+__device__ inline void pack_backward_weight(const Params& P, const S* __restrict__ W, S* __restrict__ Wp, unsigned block, unsigned blocks) {
     using MM = Mma<T>;
     constexpr bool S16 = !std::is_same<S, T>::value;
     constexpr int PER = S16 ? 4 : 1;                    // values per lane and reduction step
-    const unsigned pack_blocks = pc.sel ? gridDim.x - 1 : gridDim.x;
-    if (blockIdx.x == pack_blocks) {
-        choose_plan(pc, off, n_off);
-        return;
-    }
-    if (bounds && blockIdx.x == 0 && threadIdx.x < 2) bounds[threadIdx.x] = 0.f;
     constexpr int TN = MM::TN, KL = MM::KL, TP = TN / CCH;
     const int npass = (P.kV + TP - 1) / TP;
     const int kst = gcol_slab_steps<T, S>(P.M);                 // operand batches are 8 or 16 (16-bit: 4 or 8) reduction steps
     const size_t per_chunk = (size_t)npass * kst * 64 * PER;
     const size_t total = (size_t)chunk_candidates<CCH>(P.cpg, P.Cg, P.C_in) * per_chunk;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)pack_blocks * blockDim.x) {
+    for (size_t i = (size_t)block * 256 + threadIdx.x; i < total; i += (size_t)blocks * 256) {
         const int c0 = chunk_candidate<CCH>(P.cpg, P.Cg, (int)(i / per_chunk));      // candidate first channel of a chunk
         const int seg_b = max(c0 / P.cpg * P.cpg, c0 / P.Cg * P.Cg);
         if ((c0 - seg_b) % CCH) continue;
@@ -867,63 +859,12 @@ template <> struct LdsCell<double> {
     __device__ static inline double value(type c, double) { return c; }
 };
 
-// max |w| over a small tensor (used for the fixed-point exponent), NaN if any element is NaN.  Each
-// workgroup reduces a strided share and joins the result with an integer atomic max: non-negative
-// floats order like their bit patterns.  `out` must hold 0 beforehand.
-template <typename T>
-__global__ void absmax_kernel(const T* __restrict__ w, size_t n, float* __restrict__ out) {
-    __shared__ float red[256];
-    // maxima are taken on the bit patterns: |NaN| has the largest pattern, so a NaN survives (fmaxf drops it)
-    unsigned m = 0u;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-        m = max(m, __float_as_uint(fabsf((float)w[i])));
-    unsigned* redu = reinterpret_cast<unsigned*>(red);
-    redu[threadIdx.x] = m;
-    __syncthreads();
-    for (int sft = blockDim.x / 2; sft > 0; sft >>= 1) {
-        if ((int)threadIdx.x < sft) redu[threadIdx.x] = max(redu[threadIdx.x], redu[threadIdx.x + sft]);
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) atomicMax(reinterpret_cast<unsigned*>(out), redu[0]);
-}
-
-// out[0] = max |w| and out[1] = max over the weight's (input channel, tap) columns of the Euclidean
-// norm over the output channels of one convolution group, NaN if any element is NaN: |grad column|
-// <= that norm times the norm of grad_output over the output channels at the position
-// (Cauchy-Schwarz).  W is [G*M][Cg][kV]; grid (ceil(Cg*kV / 64), G); joined like absmax_kernel.
-// `out` must hold two zeros beforehand.
-template <typename T>
-__global__ __launch_bounds__(512) void weight_bounds_kernel(const T* __restrict__ w, int M, size_t cols, float* __restrict__ out) {
-    // workgroup = 64 neighbouring columns of one group (blockIdx.y) x 8 slices of its rows
-    __shared__ float part[8][64];
-    __shared__ unsigned amax[8];
-    const int cx = threadIdx.x & 63, sl = threadIdx.x >> 6;
-    const size_t col = (size_t)blockIdx.x * 64 + cx;
-    float ss = 0.f;
-    unsigned am = 0u;
-    if (col < cols) {
-        const T* p = w + (size_t)blockIdx.y * M * cols + col;
-#pragma unroll 8
-        for (int r = sl; r < M; r += 8) {
-            const float v = offset_value(p[(size_t)r * cols]);
-            ss += v * v;
-            am = max(am, __float_as_uint(fabsf(v)));
-        }
-    }
-    for (int sh = 1; sh < 64; sh <<= 1) am = max(am, (unsigned)__shfl_xor((int)am, sh));
-    part[sl][cx] = ss;
-    if (cx == 0) amax[sl] = am;
-    __syncthreads();
-    if (sl == 0) {
-#pragma unroll
-        for (int k = 1; k < 8; ++k) { ss += part[k][cx]; am = max(am, amax[k]); }
-        unsigned m = __float_as_uint(fabsf(sqrtf(ss)));       // NaN keeps the largest pattern
-        for (int sh = 1; sh < 64; sh <<= 1) m = max(m, (unsigned)__shfl_xor((int)m, sh));
-        if (cx == 0) {
-            atomicMax(reinterpret_cast<unsigned*>(out), am);          // out[0] = max |w|
-            atomicMax(reinterpret_cast<unsigned*>(out) + 1, m);       // out[1] = largest column norm
-        }
-    }
+// Maximum over the blocks of backward_prepare_kernel that worked out the bounds of the weights: which = 0
+// max |w|, 1 the largest column norm (see prep_bounds); one bound per lane.
+__device__ inline float weight_bound(const float* __restrict__ bounds, int which) {
+    unsigned m = __float_as_uint(bounds[2 * (threadIdx.x & 63) + which]);
+    for (int sh = 1; sh < 64; sh <<= 1) m = max(m, (unsigned)__shfl_xor((int)m, sh));
+    return __uint_as_float(m);
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -966,7 +907,6 @@ __global__ __launch_bounds__(512) void weight_bounds_kernel(const T* __restrict_
 // half the LDS atomics and two thirds of the LDS bytes per channel.  The terms are scaled such
 // that (positions of the block x taps) of the largest possible one -- all that a cell can receive
 // -- still fit 31 bits; the host allows it only while that leaves enough bits below that term.
-// wmax[1] then holds the largest column norm of the weight (colnorm_max_kernel).
 // S: storage format of input, offset, weight and grad_output (Bf16 / Fp16 with T = float: the grad-column
 // GEMM then runs on the 16-bit matrix instructions, see GcolGemm; requires BREG and PACKW); the
 // gradients are written as T.
@@ -977,7 +917,7 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
                                                                   const S* __restrict__ off,
                                                                   const S* __restrict__ Wt,
                                                                   const S* __restrict__ gout,
-                                                                  const float* __restrict__ wmax,
+                                                                  const float* __restrict__ bounds,
                                                                   T* __restrict__ gin, T* __restrict__ goff, int csplit,
                                                                   unsigned whole, int goff_atomic) {
     HaloPlan H;
@@ -1035,6 +975,7 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
         cz = r % (unsigned)cs;
     }
     const unsigned nt = (unsigned)P.N * P.tiles;
+    const float wbound = weight_bound(bounds, PAIR ? 1 : 0);
     const int dg = item / nt;
     // an item that several workgroups share needs the atomics (the host has zero-filled grad_offset);
     // the only owner of an item stores the running sum over its chunks instead, unless the host asks for
@@ -1184,12 +1125,12 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
         int ex = 0;
         // paired cells: |term| <= largest column norm of W x largest norm of grad_output over the
         // output channels (0.1 % slack for the rounding of those two and of the MFMA sums)
-        const float bound = PAIR ? 1.001f * wmax[1] * sqrtf(__uint_as_float(smaxb)) : 8.f * wmax[0] * __uint_as_float(smaxb);
+        const float bound = PAIR ? 1.001f * wbound * sqrtf(__uint_as_float(smaxb)) : 8.f * wbound * __uint_as_float(smaxb);
         // paired cells: all that one cell can receive.  A (tap, position) spreads at most |grad column| over
         // its corners (their weights add up to one), so a cell's terms add up to at most the sum over the
         // block's positions and the taps of that bound -- far less than (number of terms) x (largest term)
         // when a few positions carry most of grad_output
-        const float bound_cell = PAIR ? 1.001f * wmax[1] * (float)P.kV * ssum : 0.f;
+        const float bound_cell = PAIR ? 1.001f * wbound * (float)P.kV * ssum : 0.f;
         // the LDS cells need a finite bound; without one this workgroup scatters through the far path
         // (float cells need the exponent; and with either cell type a corner that carries weight zero
         // would receive 0 * inf = NaN where the reference adds nothing)
@@ -2171,17 +2112,28 @@ __global__ __launch_bounds__(WG) void backward_weight16_kernel(Params P, const S
         }
 }
 
-// grad_weight[g*M+m][cl][tap] += sum over splits of partial[split][tap][g*M+m][cl]
+// grad_weight[g*M+m][cl][tap] (+)= sum over splits of partial[split][tap][g*M+m][cl]
 // 256 threads = 64 consecutive elements x 4 lanes of splits: lane l adds the splits l, l + 4, ...
 // (loads of a lane independent of each other), then the four sums are added in the order of l, so
-// the result does not depend on timing.
+// the result does not depend on timing.  The blocks from `wblocks` on add up the strips of
+// grad_output's sums (backward_prepare_kernel), a wavefront per output channel: grad_bias.
 template <typename T>
 __global__ __launch_bounds__(256) void reduce_weight_partials_kernel(const T* __restrict__ partial, T* __restrict__ gw, int nsplit, int kV,
-                                                                     size_t rows_x_cg /* C_out * Cg */) {
+                                                                     size_t rows_x_cg /* C_out * Cg */, int accumulate, unsigned wblocks,
+                                                                     const T* __restrict__ sums, T* __restrict__ gb, int C_out, int nsums) {
+    if (blockIdx.x >= wblocks) {
+        const int c = (int)(blockIdx.x - wblocks) * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+        if (c >= C_out) return;
+        T s = 0;
+        for (int i = lane; i < nsums; i += 64) s += sums[(size_t)c * nsums + i];
+        for (int sh = 1; sh < 64; sh <<= 1) s += __shfl_xor(s, sh);
+        if (lane == 0) gb[c] = s;
+        return;
+    }
     __shared__ T part[4][64];
     const size_t total = (size_t)kV * rows_x_cg;
     const int e = threadIdx.x & 63, l = threadIdx.x >> 6;
-    for (size_t i0 = (size_t)blockIdx.x * 64; i0 < total; i0 += (size_t)gridDim.x * 64) {
+    for (size_t i0 = (size_t)blockIdx.x * 64; i0 < total; i0 += (size_t)wblocks * 64) {
         const size_t i = i0 + e;
         T sum = 0;
         if (i < total) {
@@ -2197,37 +2149,10 @@ __global__ __launch_bounds__(256) void reduce_weight_partials_kernel(const T* __
         __syncthreads();
         if (l == 0 && i < total) {
             const size_t tap = i / rows_x_cg, rc = i % rows_x_cg;     // rc = (g*M + m) * Cg + cl
-            gw[rc * kV + tap] += ((part[0][e] + part[1][e]) + part[2][e]) + part[3][e];
+            const T v = ((part[0][e] + part[1][e]) + part[2][e]) + part[3][e];
+            gw[rc * kV + tap] = accumulate ? gw[rc * kV + tap] + v : v;
         }
         __syncthreads();
-    }
-}
-
-// Both layout changes of backward_weight in one launch: z < N copies tensor A, z >= N tensor B
-// (grid: the larger of the two extents along x and y, 2 * N along z).
-template <typename T>
-__global__ void to_channels_last_pair_kernel(const T* __restrict__ srcA, T* __restrict__ dstA, int CA, unsigned VA,
-                                             const T* __restrict__ srcB, T* __restrict__ dstB, int CB, unsigned VB, int N) {
-    __shared__ T tile[32][33];
-    const bool second = (int)blockIdx.z >= N;
-    const T* src = second ? srcB : srcA;
-    T* dst = second ? dstB : dstA;
-    const int C = second ? CB : CA;
-    const unsigned V = second ? VB : VA;
-    const unsigned v0 = blockIdx.x * 32;
-    const int c0 = blockIdx.y * 32;
-    if (v0 >= V || c0 >= C) return;                 // uniform for the block
-    const size_t base = (size_t)(second ? blockIdx.z - N : blockIdx.z) * C * V;
-    for (int i = threadIdx.y; i < 32; i += 8) {
-        const int c = c0 + i;
-        const unsigned v = v0 + threadIdx.x;
-        if (c < C && v < V) tile[i][threadIdx.x] = src[base + (size_t)c * V + v];
-    }
-    __syncthreads();
-    for (int i = threadIdx.y; i < 32; i += 8) {
-        const unsigned v = v0 + i;
-        const int c = c0 + threadIdx.x;
-        if (c < C && v < V) dst[base + (size_t)v * C + c] = tile[threadIdx.x][i];
     }
 }
 

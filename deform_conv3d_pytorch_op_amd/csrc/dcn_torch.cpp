@@ -250,24 +250,35 @@ Gradients conv_offset_backward(const Config& c, const Tensor& input, const Tenso
     const Geometry g = geometry(c, input, weight, out);
     const Tensor in = input.contiguous(), off = offset.contiguous(), w = weight.contiguous(), go = grad_output.contiguous();
     const int dt = dtype_index(in.scalar_type());
+    check(!(c.nd == 3 && c.oob_zero && need_data && dt >= 2), "oob_offset_grad='zero' is available in float32 and float64 only");
     const hipStream_t main = c10::hip::getCurrentHIPStream(in.device().index()).stream();
     Gradients r;
     const bool two = need_data && need_weight && overlap_backward();
-    const Tensor ws = workspace_tensor(in, g.ws_bytes), ws_w = two ? workspace_tensor(in, g.ws_bytes) : ws;
-    if (need_weight) r.weight = at::zeros_like(w);       // beta = 1 accumulation, as in the reference
+    if (need_weight) r.weight = two ? at::zeros_like(w) : at::empty_like(w);
     if (need_data) {
-        // the kernels accumulate into grad_input (as the reference's atomicAdd does) and store every element of grad_offset
-        r.input = at::zeros_like(in);
+        r.input = two ? at::zeros_like(in) : at::empty_like(in);
         r.offset = at::empty_like(off);
     }
-    hipStream_t side = main;
     if (two) {
-        side = side_stream(in.device().index()).stream();
+        const Tensor ws = workspace_tensor(in, g.ws_bytes), ws_w = workspace_tensor(in, g.ws_bytes);
+        const hipStream_t side = side_stream(in.device().index()).stream();
         wait_for(side, main);                            // the operands and the zero fills above are ready
+        check_rc(run_backward_data(c.nd, dt, c.oob_zero, in, w, off, go, r.input, r.offset, g.v, workspace(ws, g.ws_bytes, main)));
+        check_rc(run_backward_weight(c.nd, dt, in, off, go, r.weight, g.v, workspace(ws_w, g.ws_bytes, side)));
+        wait_for(main, side);                            // everything issued later on the caller's stream sees grad_weight
+    } else if (need_data || need_weight) {
+        size_t in_v = 1, out_v = 1;
+        int kv = 1;
+        for (int a = 0; a < c.nd; ++a) { in_v *= in.size(2 + a); out_v *= out[a]; kv *= (int)w.size(2 + a); }
+        const size_t bytes = dcn_layer_backward_workspace_bytes((int)in.element_size(), c.nd, g.v[0], g.v[1], g.v[2], in_v, out_v, kv, c.group, c.cpg);
+        const Tensor ws = workspace_tensor(in, bytes);
+        const bool bias_too = need_bias && need_weight;
+        if (bias_too) r.bias = at::empty({w.size(0)}, w.options());
+        auto p = [](const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; };
+        check_rc(dcn_layer_backward(c.nd, dt, cptr<void>(in), cptr<void>(w), cptr<void>(off), cptr<void>(go), p(r.input), p(r.offset), p(r.weight), p(r.bias), g.v,
+                                    ws.data_ptr(), bytes, main, c.nd == 3 && c.oob_zero ? DCN_FLAG_OOB_OFFSET_GRAD_ZERO : 0u));
+        if (bias_too) return r;
     }
-    if (need_data) check_rc(run_backward_data(c.nd, dt, c.oob_zero, in, w, off, go, r.input, r.offset, g.v, workspace(ws, g.ws_bytes, main)));
-    if (need_weight) check_rc(run_backward_weight(c.nd, dt, in, off, go, r.weight, g.v, workspace(ws_w, g.ws_bytes, side)));
-    if (two) wait_for(main, side);                       // everything issued later on the caller's stream sees grad_weight
     if (need_bias) {
         static const int64_t dims[2][4] = {{0, 2, 3, 0}, {0, 2, 3, 4}};
         r.bias = go.sum(at::IntArrayRef(dims[c.nd - 2], c.nd + 1));

@@ -201,6 +201,20 @@ int conv2d_backward_weight_f32(const float *input, const float *grad_output, flo
 int conv2d_backward_weight_f64(const double *input, const double *grad_output, double *grad_weight, CONV2D_GEOMETRY,
                                void *workspace, size_t workspace_bytes, void *stream);
 
+/* ---- the backward pass of a layer in one call ------------------------------------------------
+ * No counterpart in the reference, whose Functions call backward_input_offset and backward_weight and
+ * add up grad_bias themselves (deform3d/deform_conv3d_functions/deform_conv3d_function.py:44-77).  Gradients that
+ * are not wanted are null (grad_input and grad_offset come together; grad_bias only beside grad_weight);
+ * the others are WRITTEN, not accumulated.  nd: 2 or 3; dtype: 0 float32, 1 float64, 2 bfloat16, 3
+ * binary16; geometry: the integers of DCN2D_GEOMETRY / DCN3D_GEOMETRY in their order; flags: as
+ * dcn3d_backward_input_offset_flags_f32 (float32 and float64 only).  Same kernels and accuracy as the separate
+ * calls, with one launch instead of up to ten in front of them. */
+size_t dcn_layer_backward_workspace_bytes(int elem_size, int nd, int batch, int input_c, int output_c, size_t input_volume,
+                                          size_t output_volume, int kernel_volume, int group, int channel_per_deformable_group);
+int dcn_layer_backward(int nd, int dtype, const void *input, const void *weight, const void *offset, const void *grad_output,
+                       void *grad_input, void *grad_offset, void *grad_weight, void *grad_bias, const int *geometry,
+                       void *workspace, size_t workspace_bytes, void *stream, unsigned flags);
+
 /* ---- 16-bit storage, float32 accumulation ----------------------------------------------------
  * No counterpart in the reference, which instantiates float only
  * (deform3d/lib/deform_conv3d_cuda_kernel.cu:162-172).  Every tensor (input, weight, offset, bias,
