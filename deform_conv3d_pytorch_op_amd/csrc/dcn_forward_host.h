@@ -46,7 +46,27 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
         MT = mtiles_all > 4 && cost(8) <= cost(4) ? 8 : 4;
         P.mchunks = (mtiles_all + MT - 1) / MT;
     }
-    const int nwp = shared ? SHARED_COLS : WAVESH;      // column tiles of a block
+    // Few positions: forward_split_kernel in blocks of 64 positions, four wavefronts to a position, as long as
+    // that gives no more than two workgroups per CU.
+    bool small = false;
+    // (a single tap leaves too few steps to share in 3-D: the halo of 64 positions costs more to stage than it saves)
+    if (MX && shared) {       // ... unless it fills half of the device, with the input channels split
+        Params Pt = P;
+        if (plan_halo<T, ND>(Pt, MAX_LDS, default_margin(), 1 << 30, sizeof(S), SHARED_COLS, false, FG, nullptr, 1, false) &&
+            (long long)Pt.N * Pt.tiles * P.G * P.mchunks * (P.Cg >= 32 ? P.Cg / 16 : 1) * 2 < cu_count())
+            shared = false;
+    }
+    if (MX && !shared && (ND == 2 || P.kV > 1) && forward_small() && forward_slots() == 0) {
+        Params Pt = P;
+        const int mt = mtiles_all > 2 ? 4 : mtiles_all, mc = (mtiles_all + mt - 1) / mt;
+        if (plan_halo<T, ND>(Pt, MAX_LDS, default_margin(), 1 << 30, sizeof(S), 2, false, FG, nullptr, 1, false) &&
+            (long long)Pt.N * Pt.tiles * P.G * mc <= (mt == 4 ? 1 : 2) * cu_count()) {
+            small = true;
+            MT = mt;
+            P.mchunks = mc;
+        }
+    }
+    const int nwp = shared ? SHARED_COLS : small ? 2 : WAVESH;      // column tiles of a block
     const size_t out_bytes = (size_t)P.N * P.C_out * P.outV * sizeof(T);
     const size_t wq_bound = align256(((size_t)chunk_slot<CM>(P.cpg, P.Cg, P.C_in - 1) + 1) * slab_bytes(P.kV, (mtiles_all + 7) / 8 * 8 * TN));
     {
@@ -61,11 +81,12 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
         }
         if (!S16 && tiled && forward_split() > 1 && (size_t)P.N * P.outV < FWD_SPLIT_POSITIONS && ws_bytes > wq_bound) {
             const size_t room = ws_bytes - wq_bound < FWD_PARTIAL_CAP ? ws_bytes - wq_bound : FWD_PARTIAL_CAP;
-            while (fsplit * 2 <= FWD_MAX_SPLIT && fsplit * 2 <= forward_split() && tiles * P.G * P.mchunks * fsplit * 2 <= cu_count() &&
-                   (size_t)fsplit * 2 * out_bytes <= room && fsplit * 2 * 16 <= P.Cg)      // at least 16 channels per part
+            while (fsplit * 2 <= FWD_MAX_SPLIT && fsplit * 2 <= forward_split() && tiles * P.G * P.mchunks * fsplit * 2 <= (small && MT < 4 ? 2 : 1) * cu_count() &&
+                   (size_t)fsplit * 2 * out_bytes <= room && fsplit * 2 * (small ? 8 : 16) <= P.Cg)      // at least 16 channels per part (8: four wavefronts share them)
                 fsplit *= 2;
         }
-        while (MT > 1 && !shared && tiles * P.G * P.mchunks * fsplit < cu_count()) {
+        // (forward_split_kernel fills a CU with two wavefronts per position before that pays)
+        while (MT > 1 && !shared && !small && tiles * P.G * P.mchunks * fsplit < cu_count() / (MX ? 2 : 1)) {
             MT /= 2;
             P.mchunks = (mtiles_all + MT - 1) / MT;
         }
@@ -94,8 +115,15 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             }
             return tiled && (long long)Ph.N * Ph.tiles * Ph.G * Ph.mchunks <= 0x7fffffffLL ? SHARED_COLS : 0;
         }
-        // (the 3-D double instance of the 1024-thread shape does not fit its 128 registers)
-        if (MT <= 2 && wide_forward() && !(sizeof(T) == 8 && ND == 3)) {
+        if (small) {
+            // (half of the LDS: two workgroups share a CU)
+            const bool tiled = plan_halo<T, ND>(Ph, MT == 4 ? MAX_LDS : MAX_LDS / 2, m, 1 << 30, sizeof(S), 2, false, FG, nullptr, 1, false) ||
+                               plan_halo<T, ND>(Ph, MAX_LDS, m, 1 << 30, sizeof(S), 2, false, FG, nullptr, 1, false);
+            return tiled ? 2 : 0;
+        }
+        // (the 3-D double instance of the 1024-thread shape does not fit its 128 registers; short segments
+        // have short passes, and two workgroups per CU then cover each other's staging)
+        if (MT <= 2 && wide_forward() && !(sizeof(T) == 8 && ND == 3) && (!MX || wide_forward() == 2 || (P.cpg >= 16 && P.Cg >= 16))) {
             Params Pw = P;
             if (plan_shape(Pw, MAX_LDS, m, 16, false) && (long long)Pw.N * Pw.tiles * Pw.G * Pw.mchunks <= 0x7fffffffLL &&
                 (wide_forward() == 2 || (Pw.cchunk >= 8 && (long long)Pw.N * Pw.tiles * Pw.G * Pw.mchunks >= cu_count()))) {
@@ -129,6 +157,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             P.Mp = P.mchunks * MT * TN;
             nw = plan_for(margins[0], plans[0]);
         }
+        if (small && !nw) return fail(DCN_E_LAUNCH, "no halo plan");      // (planned above)
         const size_t col_bytes = shared ? shared_column_bytes<typename std::conditional<MX, S, float>::type>() : 0;
         const size_t wq_bytes = ((size_t)chunk_slot<CM>(P.cpg, P.Cg, P.C_in - 1) + 1) * slab_bytes(P.kV, P.Mp) + 256;      // (+: operands read from four elements further on)
         auto halo_lds = [=](const Params& Ph) { return col_bytes + (size_t)Ph.cchunk * Ph.hstride * (MX ? sizeof(S) : sizeof(T)) + (MX ? 0 : (size_t)Ph.hvol * 4); };
@@ -168,10 +197,11 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                 const long long wgs = (long long)plans[0].N * plans[0].tiles * plans[0].G * plans[0].mchunks * fsplit;
                 size_t lds0 = halo_lds(plans[0]);
                 if ((wgs <= cu_count() || shared) && lds0 < MAX_LDS) lds0 = MAX_LDS;
+                if (small && wgs > cu_count() && lds0 < MAX_LDS / 2) lds0 = MAX_LDS / 2;
                 for (int k = 1; k < nmargins; ++k) {
                     Params& Pk = plans[pc.nplans];
                     Pk = P;
-                    if (shared ? !plan_halo<T, ND>(Pk, lds0 - col_bytes, margins[k], 1 << 30, sizeof(S), nw, false, FG, plans[0].tdim, 1, false)
+                    if (shared || small ? !plan_halo<T, ND>(Pk, lds0 - col_bytes, margins[k], 1 << 30, sizeof(S), nw, false, FG, plans[0].tdim, 1, false)
                                : !plan_shape(Pk, lds0, margins[k], nw, false, plans[0].tdim)) continue;
                     if (!same_blocks(Pk, plans[0]) || Pk.hvol > 3 * plans[0].hvol) continue;
                     if (fsplit > 1) even_passes(Pk);
@@ -201,7 +231,11 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                 else hipLaunchKernelGGL(pack_forward_weight_kernel<T>, pgrid, dim3(256), 0, s, plans[0], w, static_cast<T*>(ws), pc, off, n_off);
                 if (int rc = check_launch("forward weight packing")) return rc;
             }
-            size_t lds = 0;
+            // a grid of at most one workgroup per CU: sixteen wavefronts to its 256 positions, two to a position
+            const bool pairs = MX && !small && !shared && nw == WAVESH && MT <= 2 && P.kV > 1 && forward_small() && forward_slots() == 0 &&
+                               (long long)plans[0].N * plans[0].tiles * plans[0].G * plans[0].mchunks * fsplit <= cu_count();
+            // (the sums of the wavefronts that share positions)
+            size_t lds = small ? (size_t)3 * 2 * MT * 4096 : pairs ? (size_t)WAVESH * MT * 4096 : 0;
             for (int k = 0; k < pc.nplans; ++k) {
                 const size_t l = halo_lds(plans[k]);
                 if (l > lds) lds = l;
@@ -210,10 +244,12 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             using Kern = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const WE*, const S*, S*, T*, int, unsigned, TailSplit);
             Kern kern = nullptr;
             if constexpr (MX) {
-                if (shared) { if constexpr (ND == 2) kern = MT == 8 ? forward_shared_kernel<ND, 8, S> : forward_shared_kernel<ND, 4, S>; }
-                else if (nw == 16) kern = MT == 1 ? forward_split_kernel<ND, 1, 16, S> : forward_split_kernel<ND, 2, 16, S>;
-                else kern = MT == 1 ? forward_split_kernel<ND, 1, WAVESH, S> : MT == 2 ? forward_split_kernel<ND, 2, WAVESH, S>
-                                                                             : forward_split_kernel<ND, 4, WAVESH, S>;
+                if (pairs) kern = MT == 1 ? forward_split_kernel<ND, 1, 16, 2, S> : forward_split_kernel<ND, 2, 16, 2, S>;
+                else if (small) kern = MT == 1 ? forward_split_kernel<ND, 1, 8, 4, S> : MT == 2 ? forward_split_kernel<ND, 2, 8, 4, S> : forward_split_kernel<ND, 4, 8, 4, S>;
+                else if (shared) { if constexpr (ND == 2) kern = MT == 8 ? forward_shared_kernel<ND, 8, S> : forward_shared_kernel<ND, 4, S>; }
+                else if (nw == 16) kern = MT == 1 ? forward_split_kernel<ND, 1, 16, 1, S> : forward_split_kernel<ND, 2, 16, 1, S>;
+                else kern = MT == 1 ? forward_split_kernel<ND, 1, WAVESH, 1, S> : MT == 2 ? forward_split_kernel<ND, 2, WAVESH, 1, S>
+                                                                             : forward_split_kernel<ND, 4, WAVESH, 1, S>;
             } else {
                 if (nw == 16) kern = MT == 1 ? forward_quad_kernel<T, ND, 1, 16> : forward_quad_kernel<T, ND, 2, 16>;
                 else kern = MT == 1 ? forward_quad_kernel<T, ND, 1, WAVESH> : MT == 2 ? forward_quad_kernel<T, ND, 2, WAVESH>
@@ -233,7 +269,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             long long whole = 0;
             TailSplit ts = {0u, 0, 0};
             if (fsplit == 1 && forward_tail_split()) {
-                const long long slots = forward_slots() ? forward_slots() : resident_workgroups(reinterpret_cast<const void*>(kern), (shared ? SHARED_WAVES : nw) * 64, lds);
+                const long long slots = forward_slots() ? forward_slots() : resident_workgroups(reinterpret_cast<const void*>(kern), (pairs ? 16 : shared || small ? 8 : nw) * 64, lds);
                 const long long rest = units % slots;
                 constexpr double GEO = 0.45;    // tap geometry of a pass, in units of four channels' sampling and contraction
                 // cost of the longest workgroup when the passes of a unit (cch channels each) are dealt to cs workgroups
@@ -301,14 +337,15 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                             plans[k].hext[0], plans[k].hext[1], plans[k].hext[2], plans[k].cchunk, pc.base[k]);
             }
             const unsigned* sel = pc.sel;
-            if (int rc = launch_halo(kern, "forward halo kernel", grid, (shared ? SHARED_WAVES : nw) * 64, lds, s, Ph, alts, sel, in, off, (const WE*)ws, bias, out, part,
+            if (int rc = launch_halo(kern, "forward halo kernel", grid, (pairs ? 16 : shared || small ? 8 : nw) * 64, lds, s, Ph, alts, sel, in, off, (const WE*)ws, bias, out, part,
                                      tsplit > 1 ? tsplit : fsplit, (unsigned)whole, ts))
                 return rc;
             if (fsplit == 1 && tsplit == 1) return DCN_OK;
             if (tsplit > 1) {
                 using Join = void (*)(Params, PlanSet, const unsigned*, const T*, const S*, S*, int, unsigned, TailSplit);
                 Join join;
-                if (shared) join = MT == 8 ? forward_join_tail_kernel<T, ND, 8, SHARED_COLS, S> : forward_join_tail_kernel<T, ND, 4, SHARED_COLS, S>;
+                if (small) join = MT == 1 ? forward_join_tail_kernel<T, ND, 1, 2, S> : MT == 2 ? forward_join_tail_kernel<T, ND, 2, 2, S> : forward_join_tail_kernel<T, ND, 4, 2, S>;
+                else if (shared) join = MT == 8 ? forward_join_tail_kernel<T, ND, 8, SHARED_COLS, S> : forward_join_tail_kernel<T, ND, 4, SHARED_COLS, S>;
                 else if (nw == 16) join = MT == 1 ? forward_join_tail_kernel<T, ND, 1, 16, S> : forward_join_tail_kernel<T, ND, 2, 16, S>;
                 else join = MT == 1 ? forward_join_tail_kernel<T, ND, 1, WAVESH, S> : MT == 2 ? forward_join_tail_kernel<T, ND, 2, WAVESH, S>
                           : MT == 4 || MX ? forward_join_tail_kernel<T, ND, 4, WAVESH, S> : forward_join_tail_kernel<T, ND, MX ? 4 : 8, WAVESH, S>;

@@ -245,8 +245,7 @@ __device__ inline bool stage_halo(const Params& P, const HaloPlan& H, const Tile
     const float inv2 = 1.f / (float)H.hext[2], inv1 = 1.f / (float)H.hext[1], inv = 1.f / (float)H.hvol;
     const size_t step = (size_t)P.inV * sizeof(S);
     bool bad = false;
-#pragma unroll 4
-    for (int it = threadIdx.x; it < items; it += WGS) {
+    auto stage = [&](int it, auto full_tag) {
         const int grp = (int)(((float)it + 0.5f) * inv), v = it - __mul24(grp, H.hvol);
         const unsigned t = halo_voxel<ND>(P, H, tg, v, inv1, inv2);
         const char* cp = reinterpret_cast<const char*>(chan0) + (size_t)(t == ~0u ? 0u : t) * sizeof(S) + (size_t)(grp * CH) * step;
@@ -254,13 +253,23 @@ __device__ inline bool stage_halo(const Params& P, const HaloPlan& H, const Tile
         typename HaloCell<S>::Vec cell;
 #pragma unroll
         for (int e = 0; e < CH; ++e) {
-            const S x = *reinterpret_cast<const S*>(cp + (size_t)min(e, last) * step);
-            if constexpr (CHECK) bad = bad || !(fabsf(Store<S>::ld(x)) <= std::numeric_limits<float>::max());
-            cell[e] = HaloCell<S>::raw(x);
+            cell[e] = (typename HaloCell<S>::V)0.f;
+            if (decltype(full_tag)::value || e < nch) {         // (uniform)
+                const S x = *reinterpret_cast<const S*>(cp + (size_t)min(e, last) * step);
+                if constexpr (CHECK) bad = bad || !(fabsf(Store<S>::ld(x)) <= std::numeric_limits<float>::max());
+                cell[e] = HaloCell<S>::raw(x);
+            }
         }
 #pragma unroll
         for (int e = 0; e < CH; ++e) cell[e] = (e <= last && t != ~0u) ? cell[e] : (typename HaloCell<S>::V)0.f;
         sIn[(size_t)grp * H.hstride + v] = cell;
+    };
+    if (nch >= CH) {
+#pragma unroll 4
+        for (int it = threadIdx.x; it < items; it += WGS) stage(it, std::true_type{});
+    } else {                                                    // a segment shorter than a cell loads what it has
+#pragma unroll 4
+        for (int it = threadIdx.x; it < items; it += WGS) stage(it, std::false_type{});
     }
     return bad;
 }
@@ -327,19 +336,24 @@ __device__ inline void split_geometry(const Params& P, const HaloPlan& H, const 
 // Weighted corner sums of the channels of a cell (element by element: a vector times scalar product
 // would hold four copies of every weight).  The sums are formed here, not where the contraction uses
 // them, so that one cell's corners are in flight at a time.  row, plane: cells between neighbours along h and l.
+// `more` (uniform): also the channels from the fifth on of a 16-bit cell.
 template <int ND, typename S>
-__device__ inline void cell_sum(const typename HaloCell<S>::Vec* cell, unsigned row, unsigned plane, const float* cw, float* v) {
+__device__ inline void cell_sum(const typename HaloCell<S>::Vec* cell, unsigned row, unsigned plane, const float* cw, float* v, bool more) {
     constexpr int NC = 1 << ND, CH = HaloCell<S>::CH;
     typename HaloCell<S>::Vec c[NC];
 #pragma unroll
     for (int i = 0; i < NC; ++i) c[i] = cell[(i >> 2) * plane + ((i >> 1) & 1) * row + (i & 1)];
 #pragma unroll
-    for (int e = 0; e < CH; ++e) {
+    for (int h = 0; h < CH; h += 4)
+        if (h == 0 || more) {
 #pragma unroll
-        for (int i = 0; i < NC; ++i) v[e] = i ? v[e] + (float)c[i][e] * cw[i] : (float)c[i][e] * cw[i];
-    }
+            for (int e = h; e < h + 4; ++e) {
 #pragma unroll
-    for (int e = 0; e < CH; ++e) asm volatile("" : "+v"(v[e]));
+                for (int i = 0; i < NC; ++i) v[e] = i ? v[e] + (float)c[i][e] * cw[i] : (float)c[i][e] * cw[i];
+            }
+#pragma unroll
+            for (int e = h; e < h + 4; ++e) asm volatile("" : "+v"(v[e]));
+        }
     __builtin_amdgcn_sched_barrier(0);
 }
 // ... of the eight channels of group grp of a chunk of nch channels
@@ -350,9 +364,9 @@ __device__ inline void group_sum8(const typename HaloCell<S>::Vec* sIn, unsigned
 #pragma unroll
     for (int e = 0; e < FG; ++e) val[e] = 0.f;
     const typename HaloCell<S>::Vec* hp = sIn + base + (size_t)grp * (FG / CH) * hstride;
-    cell_sum<ND, S>(hp, row, plane, cw, val);
+    cell_sum<ND, S>(hp, row, plane, cw, val, grp * FG + 4 < nch);
     if constexpr (CH == 4)
-        if (grp * FG + 4 < nch) cell_sum<ND, S>(hp + hstride, row, plane, cw, val + 4);
+        if (grp * FG + 4 < nch) cell_sum<ND, S>(hp + hstride, row, plane, cw, val + 4, false);
 }
 
 // Samples that reach past the halo: val[e] of such lanes = channels c .. c + 7 of the chunk (below nch)
@@ -373,15 +387,24 @@ __device__ inline void far_values(const Params& P, const SplitTap<ND>& t, const 
         g.f[a] = pa - (float)l;
     }
     tap_corner_idx<float, ND>(P, g);
+    // 16 gathers in flight (channel by channel, a layer with one offset in ten beyond its halo waited
+    // eight times per step; 32 in 3-D cost the common path its registers)
+    constexpr int B = 16 / NC;
 #pragma unroll 1
-    for (int e = 0; e < FG; ++e) {
-        float cc[NC];
-        const S* ch = chan0 + (size_t)min(c + e, nch - 1) * P.inV;
+    for (int e0 = 0; e0 < FG; e0 += B) {
+        float cc[B][NC];
 #pragma unroll
-        for (int i = 0; i < NC; ++i) cc[i] = Store<S>::ld(ch[g.idx[i]]);
-        const float v = c + e < nch ? interp<float, ND>(cc, g.f) : 0.f;
+        for (int e = 0; e < B; ++e) {
+            const S* ch = chan0 + (size_t)min(c + e0 + e, nch - 1) * P.inV;
 #pragma unroll
-        for (int x = 0; x < FG; ++x) val[x] = t.far && x == e ? v : val[x];
+            for (int i = 0; i < NC; ++i) cc[e][i] = Store<S>::ld(ch[g.idx[i]]);
+        }
+#pragma unroll
+        for (int e = 0; e < B; ++e) {
+            const float v = c + e0 + e < nch ? interp<float, ND>(cc[e], g.f) : 0.f;
+#pragma unroll
+            for (int x = e; x < FG; x += B) val[x] = t.far && x == e0 + e ? v : val[x];
+        }
     }
 }
 
@@ -468,8 +491,11 @@ __device__ inline void store_tile(const Params& P, O* __restrict__ dst, const S*
 // Binding: the LDS reads of the corners in 3-D (64 channels, 27 taps, 200 704 positions: 1.2e7 16-byte
 // reads with 46 % bank conflicts of random offsets hold a CU's LDS 0.32 of 0.52 ms; 0.64 ms on the
 // float32 instructions), operand latency in 2-D.
+// TS > 1 (layers too small to fill the device otherwise): TS wavefronts share 32 positions, each takes a
+// contiguous share of a pass's (tap pair, channel group) steps, and their sums meet in LDS -- a step
+// takes a lone wavefront 1 to 1.5 us of latencies, so a small layer's time is the length of that chain.
 // (up to two row tiles: four wavefronts per SIMD, i.e. at most 128 registers)
-template <int ND, int MT, int NW, typename S>
+template <int ND, int MT, int NW, int TS, typename S>
 __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel(Params P, PlanSet alts, const unsigned* __restrict__ sel,
                                                            const S* __restrict__ in, const S* __restrict__ off,
                                                            const typename Parts<S>::Elem* __restrict__ Wq, const S* __restrict__ bias,
@@ -482,11 +508,12 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
     typedef typename PT::Vec Vec;
     typedef typename PT::Elem Elem;
     constexpr int TN = 32, WGS = NW * 64, NP = PT::NP;
+    constexpr bool EARLY = MT == 4;                     // weights requested before the step's samples: there are registers for it
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ int sNonFinite, sRedo;
     typedef typename HaloCell<S>::Vec Cell;
     Cell* sIn = reinterpret_cast<Cell*>(smem_raw);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = TS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     const int j = lane % TN, q = lane / TN;
     const ForwardUnit U = forward_unit(H.cchunk, csplit, whole, ts);
     const unsigned gm = U.wg % (unsigned)(P.G * P.mchunks);
@@ -500,7 +527,7 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
     bool valid;
     {
         int o[ND];
-        valid = tile_position<ND>(P, tg, wave * TN + j, o, pos);
+        valid = tile_position<ND>(P, tg, wave / TS * TN + j, o, pos);
 #pragma unroll
         for (int a = 0; a < ND; ++a) ib[a] = o[a] * P.stride[slot<ND>(a)] - P.pad[slot<ND>(a)];
     }
@@ -512,8 +539,6 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
     const unsigned row = (unsigned)H.hext[2], plane = ND == 3 ? (unsigned)(H.hext[1] * H.hext[2]) : 0u;
     const unsigned a_lane = (unsigned)lane * 16;         // byte offset of this lane's operand
     const unsigned a_tg = mtiles * NP * 64;
-    constexpr int LINES = (MT * NP * 8 + NW - 1) / NW;             // 128-byte lines of a step's weights per wavefront
-    const unsigned touch_at = (unsigned)min(wave * LINES + min(lane, LINES - 1), MT * NP * 8 - 1) * 128;
     const int cg0 = g * P.Cg, cg1 = cg0 + P.Cg;
 
     if (threadIdx.x == 0) sRedo = 0;                    // ordered before the checks by the barriers of the first chunk
@@ -532,8 +557,11 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
                 const int nch = min(U.cch, ce - cc0);
                 const int ngrp = (nch + FG - 1) / FG;
                 const S* chan0 = in + ((size_t)n * P.C_in + cc0) * P.inV;      // workgroup-uniform
+                // this wavefront's steps of the pass: [first, last) of the (tap pair, group) list
+                const int steps = ntg * ngrp, first = TS > 1 ? steps * (wave % TS) / TS : 0, last = TS > 1 ? steps * (wave % TS + 1) / TS : steps;
+                const int tg_first = TS > 1 ? first / ngrp : 0, tg_end = TS > 1 ? (last + ngrp - 1) / ngrp : ntg;
                 float ofs[ND];
-                load_pair_offsets<ND, S>(P, off_dg, 0, q, pos, ofs);
+                load_pair_offsets<ND, S>(P, off_dg, min(tg_first, ntg - 1), q, pos, ofs);
                 if (exact && threadIdx.x == 0) sNonFinite = 0;
                 __syncthreads();                                               // readers of the previous chunk are done
                 if (stage_halo<ND, WGS, exact, S>(P, H, tg, chan0, nch, sIn)) sNonFinite = 1;
@@ -551,36 +579,34 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
                 int k0[ND];                            // kernel coordinates of the tap pair, counted up in scalar registers
 #pragma unroll
                 for (int a = 0; a < ND; ++a) k0[a] = 0;
-                int touched = 0;
-                for (int tgi = 0; tgi < ntg; ++tgi) {
+                if constexpr (TS > 1) decode_tap<ND>(P, 2 * tg_first, k0);
+                for (int tgi = tg_first; tgi < tg_end; ++tgi) {
                     int k1[ND];
 #pragma unroll
                     for (int a = 0; a < ND; ++a) k1[a] = k0[a];
                     next_tap<ND>(P, k1);
                     SplitTap<ND> t;
                     split_geometry<ND>(P, H, tg, ib, q, k0, k1, ofs, valid && tgi * 2 + q < P.kV, rim_far, t);
+                    // the next tap pair's offsets travel through this one's steps
+                    load_pair_offsets<ND, S>(P, off_dg, min(tgi + 1, ntg - 1), q, pos, ofs);
                     const bool any_far = __any(t.far); // rare: some sample of this wave reaches past the halo
                     const Elem* wp = wchunk + (size_t)tgi * a_tg * FG;
-                    for (int grp = 0; grp < ngrp; ++grp) {
+                    const int g0 = TS > 1 ? max(first - tgi * ngrp, 0) : 0, g1 = TS > 1 ? min(last - tgi * ngrp, ngrp) : ngrp;
+                    if constexpr (TS > 1) wp += (size_t)g0 * per_slab * FG;
+                    for (int grp = g0; grp < g1; ++grp) {
                         float val[FG];
-                        // The weights of the next step come into the L1 while this one is worked on: every
-                        // wavefront touches its share of their cache lines (128 channels, 3-D: 0.94 ms against 1.19).
-                        asm volatile("" ::"v"(touched));
-                        if constexpr (!exact) {
-                            const Elem* nx = grp + 1 < ngrp ? wp + (size_t)per_slab * FG : wchunk + (size_t)min(tgi + 1, ntg - 1) * a_tg * FG;
-                            touched = *reinterpret_cast<const int*>(reinterpret_cast<const char*>(nx) + touch_at);
-                        }
+                        Vec a8[MT][NP];
+                        auto load_a = [&]() {
+#pragma unroll
+                            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                                for (int k = 0; k < NP; ++k) __builtin_memcpy(&a8[mt][k], reinterpret_cast<const char*>(wp) + (mt * NP + k) * 1024 + a_lane, 16);
+                            __builtin_amdgcn_sched_barrier(0);      // all of them on their way while the operand is made
+                        };
+                        if constexpr (EARLY) load_a();
                         group_sum8<ND, S>(sIn, t.base, grp, nch, H.hstride, row, plane, t.cw, val);
                         if (__builtin_expect(any_far, 0)) far_values<ND, S>(P, t, chan0, grp * FG, nch, val);
-                        // the next tap pair's offsets travel behind the contraction (earlier, they would be
-                        // live through the rare branch above, which takes the registers)
-                        if (grp + 1 == ngrp) load_pair_offsets<ND, S>(P, off_dg, min(tgi + 1, ntg - 1), q, pos, ofs);
-                        Vec a8[MT][NP];
-#pragma unroll
-                        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                            for (int k = 0; k < NP; ++k) __builtin_memcpy(&a8[mt][k], reinterpret_cast<const char*>(wp) + (mt * NP + k) * 1024 + a_lane, 16);
-                        __builtin_amdgcn_sched_barrier(0);          // all of them on their way while the operand is split
+                        if constexpr (!EARLY) load_a();
                         if constexpr (!exact) {
                             Vec b8[NP];
                             PT::split(val, b8);
@@ -600,14 +626,34 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
     if (valid && !all_finite<MT>(acc)) sRedo = 1;
     __syncthreads();
     if (__builtin_expect(sRedo, 0)) work(std::true_type{});
+    if constexpr (TS > 1) {
+        // the sums of a position's TS wavefronts, added in their order: [TS - 1][position tile][register][lane]
+        __syncthreads();
+        float* sum = reinterpret_cast<float*>(smem_raw);
+        const int part_of = wave % TS, tile = wave / TS;
+        if (part_of) {
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int r = 0; r < MM::NACC; ++r) sum[((((part_of - 1) * (NW / TS) + tile) * MT + mt) * MM::NACC + r) * 64 + lane] = acc[mt][r];
+        }
+        __syncthreads();
+        if (part_of) return;
+        for (int k = 0; k < TS - 1; ++k)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int r = 0; r < MM::NACC; ++r) acc[mt][r] += sum[(((k * (NW / TS) + tile) * MT + mt) * MM::NACC + r) * 64 + lane];
+    }
 
     if (U.split && whole > 0) {
         // partial sums of a unit of the last round: [split workgroup][MT * TN rows][NW * TN positions]
-        float* dst = part + (size_t)U.pslot * (MT * TN) * (NW * TN) + q * 4 * (NW * TN) + wave * TN + j;
+        constexpr int NP_ = NW / TS * TN;
+        float* dst = part + (size_t)U.pslot * (MT * TN) * NP_ + q * 4 * NP_ + wave / TS * TN + j;
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-            for (int r = 0; r < MM::NACC; ++r) dst[(mt * TN + MM::row(r, 0)) * (NW * TN)] = acc[mt][r];
+            for (int r = 0; r < MM::NACC; ++r) dst[(mt * TN + MM::row(r, 0)) * NP_] = acc[mt][r];
         return;
     }
     if (!valid) return;

@@ -199,6 +199,7 @@ inline int relayout(const Params& P, const T* w, T* wt, int channel_fastest, hip
 //   DCN_FORWARD_TAIL2=0    forward pass: the split units of the last round all the same number of ways, never in two runs
 //   DCN_FORWARD_SLOTS=n    forward pass: plan the launch as if n workgroups ran at once (test hook)
 //   DCN_FORWARD_SHARED=0   forward pass, float32 and 16-bit: never share the sampled columns of a block among wavefronts
+//   DCN_FORWARD_SMALL=0    forward pass, float32 and 16-bit: never several wavefronts to a position
 //   DCN_SCATTER_BUDGET_KB  LDS per workgroup of the privatised scatter kernel (default 144)
 //   DCN_SCATTER=global     scatter grad-input with global atomics instead of the LDS-privatised kernel
 //   DCN_COORD=separate     grad_offset from the channels-last kernel instead of the fused LDS-halo kernel
@@ -307,6 +308,10 @@ static bool forward_shared() {           // DCN_FORWARD_SHARED=0: the forward pa
     static const int v = [] { const char* e = getenv("DCN_FORWARD_SHARED"); return (e && atoi(e) == 0) ? 0 : 1; }();
     return v != 0;
 }
+static bool forward_small() {            // DCN_FORWARD_SMALL=0: the forward pass never lets several wavefronts share a position
+    static const int v = [] { const char* e = getenv("DCN_FORWARD_SMALL"); return (e && atoi(e) == 0) ? 0 : 1; }();
+    return v != 0;
+}
 static bool fused_pair() {              // DCN_FUSED_PAIR=0: float32 LDS cells of the fused backward kernel hold one channel each (64-bit)
     static const int v = [] { const char* e = getenv("DCN_FUSED_PAIR"); return (e && atoi(e) == 0) ? 0 : 1; }();
     return v != 0;
@@ -364,7 +369,7 @@ inline bool plan_halo(Params& P, size_t budget, int m, int max_chunk = 1 << 30, 
     const int npos = waves * Mma<T>::TN;        // positions per workgroup, one column tile per wavefront
     int td[3] = {1, 1, 1};
     if (ND == 3) { td[1] = 8; td[2] = 8; td[0] = npos / 64; }
-    else         { td[2] = 16; td[1] = npos / 16; }
+    else         { td[2] = npos >= 128 ? 16 : 8; td[1] = npos / td[2]; }
     if (blocks) {                               // the block shape of another plan
         for (int a = 0; a < 3; ++a) td[a] = blocks[a];
     } else if (smallest_halo) {

@@ -1,5 +1,9 @@
 """The float32 contraction from bfloat16 parts: edges of its tiles and groups, its accuracy, and the
 results that are not finite (worked out on the float32 instructions)."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -65,3 +69,18 @@ def test_results_that_are_not_finite(spec, what):
     fin = torch.isfinite(want)
     assert fin.any() and (what == "huge" or not fin.all())
     assert ((got - want)[fin].double().norm() / want[fin].double().norm()).item() <= 1e-5
+
+
+@pytest.mark.parametrize("knob", ["DCN_FORWARD_SMALL", "DCN_FORWARD_SHARED"])
+def test_larger_shapes_of_the_kernels(knob):
+    """Layers this small are worked on by several wavefronts to a position, and wide ones share their
+    columns: the same layers through the shapes that larger ones take (one process per setting: the
+    knobs are read once)."""
+    print("knob", knob, flush=True)
+    env = dict(os.environ, **{knob: "0"})
+    r = subprocess.run([sys.executable, "-u", "-m", "pytest", __file__, os.path.join(os.path.dirname(__file__), "test_gpu_parity.py"),
+                        "-q", "-x", "-m", "gpu", "-k", "(edges or not_finite or small_cases or random_medium) and f32 or edges or not_finite",
+                        "--timeout", "120", "--timeout-method", "thread"],
+                       cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), env=env, stdout=subprocess.PIPE, stderr=subprocess.STDOUT,
+                       text=True, timeout=300)
+    assert r.returncode == 0, r.stdout[-3000:]
