@@ -103,6 +103,7 @@ EXPORTS = ["dcn_version", "dcn_arch", "dcn_last_error", "dcn_workspace_bytes", "
     for suf in ("f32", "f64", "bf16", "f16")] + [
     "dcn3d_backward_input_offset_flags_f32", "dcn3d_backward_input_offset_flags_f64",
     "dcn_layer_backward", "dcn_layer_backward_workspace_bytes", "dcn3d_forward_noalloc_f32", "conv2d_workspace_bytes"] + [
-    "conv2d_%s_%s" % (op, suf) for op in ("forward", "backward_input", "backward_weight") for suf in ("f32", "f64")]
+    "conv2d_layer_backward_workspace_bytes"] + [
+    "conv2d_%s_%s" % (op, suf) for op in ("forward", "backward_input", "backward_weight", "layer_backward") for suf in ("f32", "f64")]
 NOALLOC_SCRATCH_BYTES = 8 << 20
 FLAG_OOB_OFFSET_GRAD_ZERO = 1

@@ -2,7 +2,7 @@
 
 namespace dcn {
 
-#define INSTANTIATE(T, ND, S) template int forward<T, ND, S>(const Geometry&, const S*, const S*, const S*, const S*, S*, void*, size_t, hipStream_t, bool*);
+#define INSTANTIATE(T, ND, S) template int forward<T, ND, S>(const Geometry&, const S*, const S*, const S*, const S*, S*, void*, size_t, hipStream_t, bool*, bool);
 INSTANTIATE(float, 2, float) INSTANTIATE(float, 3, float)
 
 }  // namespace dcn

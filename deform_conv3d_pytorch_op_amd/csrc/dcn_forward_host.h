@@ -12,7 +12,7 @@ namespace dcn {
 // widens the tensors and runs the float32 operator.
 template <typename T, int ND, typename S>
 int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* bias, S* out, void* ws,
-            size_t ws_bytes, hipStream_t s, bool* declined) {
+            size_t ws_bytes, hipStream_t s, bool* declined, bool transposed) {
     constexpr bool S16 = !std::is_same<S, T>::value;
     constexpr bool MX = sizeof(T) == 4;                 // forward_split_kernel; float64: forward_quad_kernel
     constexpr size_t MAX_LDS = MX ? 160 * 1024 - 256 : 144 * 1024;      // dynamic LDS of the only workgroup of a CU
@@ -24,7 +24,8 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
     };
     Params P;
     if (int rc = validate(g, P)) return rc;
-    if (!in || !w || !off || !out) return fail(DCN_E_ARGUMENT, "null tensor pointer");
+    if (!in || !w || (!off && !MX) || !out) return fail(DCN_E_ARGUMENT, "null tensor pointer");
+    P.transposed = transposed ? 1 : 0;
     if (int rc = device_info(nullptr)) return rc;
     int MT;
     fwd_weight_pad<T>(P.M, P.Cg, MT, P.mchunks, P.Mp, P.Cgp);
@@ -147,7 +148,11 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
     };
     {
         int margins[MAX_PLANS];
-        const int nmargins = plan_margins(ND, margins);
+        int nmargins = plan_margins(ND, margins);
+        if (!off && halo_margin() < 0) {       // samples at integer coordinates: their high corners are one voxel on
+            nmargins = 1;
+            margins[0] = 1;
+        }
         Params plans[MAX_PLANS];
         int nw = plan_for(margins[0], plans[0]);
         if (shared && !nw) {       // (no halo of 128 positions holds eight channels)
@@ -365,6 +370,11 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
         return DCN_OK;
     } else {
     T* wt = static_cast<T*>(ws);
+    if (!off || transposed) {         // (the caller has another way)
+        if (!declined) return fail(DCN_E_ARGUMENT, "null tensor pointer");
+        *declined = true;
+        return DCN_OK;
+    }
     if (int rc = relayout<T>(P, w, wt, 0, s)) return rc;
     // geometry whose halo does not fit in LDS: gather straight from global memory
     P.tiles = (P.outV + WAVES * TN - 1) / (WAVES * TN);

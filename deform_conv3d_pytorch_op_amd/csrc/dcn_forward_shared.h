@@ -86,7 +86,7 @@ __global__ __launch_bounds__(SHARED_WAVES * 64, 2) void forward_shared_kernel(Pa
                 const S* chan0 = in + ((size_t)n * P.C_in + cc0) * P.inV;      // workgroup-uniform
                 const Elem* wchunk = Wq + ((size_t)chunk_slot<FG>(P.cpg, P.Cg, cc0) * per_slab + ((size_t)mchunk * RT + rw * RW) * NP * 64) * FG;
                 float ofs[ND];
-                load_pair_offsets<ND, S>(P, off_dg, 0, q, pos, ofs);
+                load_pair_offsets<ND, S>(P, off_dg, 0, q, pos, ofs, off == nullptr);
                 if (exact && threadIdx.x == 0) sNonFinite = 0;
                 __syncthreads();                                               // readers of the previous chunk are done
                 if (stage_halo<ND, WGS, exact, S>(P, H, tg, chan0, nch, sIn)) sNonFinite = 1;
@@ -122,7 +122,7 @@ __global__ __launch_bounds__(SHARED_WAVES * 64, 2) void forward_shared_kernel(Pa
                         next_tap<ND>(P, k1);
 #pragma unroll
                         for (int a = 0; a < ND; ++a) k0[a] = k1[a];
-                        load_pair_offsets<ND, S>(P, off_dg, min(tgi + 1, ntg - 1), q, pos, ofs);
+                        load_pair_offsets<ND, S>(P, off_dg, min(tgi + 1, ntg - 1), q, pos, ofs, off == nullptr);
                     }
                     const int grp = 2 * gp + half;
                     if (grp >= ngrp) return;

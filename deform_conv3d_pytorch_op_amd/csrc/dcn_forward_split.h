@@ -147,7 +147,10 @@ __global__ __launch_bounds__(256) void pack_split_weight_kernel(Params P, const 
 #pragma unroll
         for (int e = 0; e < FG; ++e) {
             S v = S();
-            if (m < P.M && tap < P.kV && c0 + e < seg_e) v = W[(((size_t)g * P.M + m) * P.Cg + (c0 + e - g * P.Cg)) * P.kV + tap];
+            if (m < P.M && tap < P.kV && c0 + e < seg_e) {
+                const size_t cl = (size_t)(c0 + e - g * P.Cg);
+                v = P.transposed ? W[(((size_t)g * P.Cg + cl) * P.M + m) * P.kV + (P.kV - 1 - tap)] : W[(((size_t)g * P.M + m) * P.Cg + cl) * P.kV + tap];
+            }
             typename PT::Elem p[NP];
             PT::split1(v, p);
 #pragma unroll
@@ -423,7 +426,12 @@ __device__ inline void next_tap(const Params& P, int k[ND]) {
 
 // offsets of this lane's tap of pair tgi (tap tgi * 2 + q, clamped to a legal tap) at position pos
 template <int ND, typename S>
-__device__ inline void load_pair_offsets(const Params& P, const S* __restrict__ off_dg, int tgi, int q, unsigned pos, float ofs[ND]) {
+__device__ inline void load_pair_offsets(const Params& P, const S* __restrict__ off_dg, int tgi, int q, unsigned pos, float ofs[ND], bool none) {
+    if (none) {                                // (uniform: a plain convolution)
+#pragma unroll
+        for (int a = 0; a < ND; ++a) ofs[a] = 0.f;
+        return;
+    }
     const char* ob = reinterpret_cast<const char*>(off_dg + (size_t)tgi * 2 * ND * P.outV);      // uniform
     unsigned lo = ((q && tgi * 2 + 1 < P.kV ? ND * P.outV : 0u) + pos) * (unsigned)sizeof(S);
     asm volatile("" : "+v"(lo));               // (not hoisted into registers that stay live)
@@ -561,7 +569,7 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
                 const int steps = ntg * ngrp, first = TS > 1 ? steps * (wave % TS) / TS : 0, last = TS > 1 ? steps * (wave % TS + 1) / TS : steps;
                 const int tg_first = TS > 1 ? first / ngrp : 0, tg_end = TS > 1 ? (last + ngrp - 1) / ngrp : ntg;
                 float ofs[ND];
-                load_pair_offsets<ND, S>(P, off_dg, min(tg_first, ntg - 1), q, pos, ofs);
+                load_pair_offsets<ND, S>(P, off_dg, min(tg_first, ntg - 1), q, pos, ofs, off == nullptr);
                 if (exact && threadIdx.x == 0) sNonFinite = 0;
                 __syncthreads();                                               // readers of the previous chunk are done
                 if (stage_halo<ND, WGS, exact, S>(P, H, tg, chan0, nch, sIn)) sNonFinite = 1;
@@ -588,7 +596,7 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
                     SplitTap<ND> t;
                     split_geometry<ND>(P, H, tg, ib, q, k0, k1, ofs, valid && tgi * 2 + q < P.kV, rim_far, t);
                     // the next tap pair's offsets travel through this one's steps
-                    load_pair_offsets<ND, S>(P, off_dg, min(tgi + 1, ntg - 1), q, pos, ofs);
+                    load_pair_offsets<ND, S>(P, off_dg, min(tgi + 1, ntg - 1), q, pos, ofs, off == nullptr);
                     const bool any_far = __any(t.far); // rare: some sample of this wave reaches past the halo
                     const Elem* wp = wchunk + (size_t)tgi * a_tg * FG;
                     const int g0 = TS > 1 ? max(first - tgi * ngrp, 0) : 0, g1 = TS > 1 ? min(last - tgi * ngrp, ngrp) : ngrp;

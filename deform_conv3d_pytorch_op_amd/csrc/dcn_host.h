@@ -155,7 +155,7 @@ inline int validate(const Geometry& g, Params& P) {
     // channels-last voxel*channel offsets of one sample are 32-bit as well
     if (inV * g.C_in > (1ll << 31)) return fail(DCN_E_ARGUMENT, "one input sample exceeds 2^31 elements");
     if (g.N > 65535) return fail(DCN_E_ARGUMENT, "batch exceeds 65535");
-    P.oob_zero = 0;
+    P.oob_zero = P.transposed = 0;
     P.nd = g.nd; P.N = g.N; P.C_in = g.C_in; P.C_out = g.C_out; P.G = g.G; P.cpg = g.cpg; P.DG = g.C_in / g.cpg;
     P.M = g.C_out / g.G; P.Cg = g.C_in / g.G;
     for (int a = 0; a < 3; ++a) {
@@ -481,8 +481,10 @@ inline int launch_halo(K kern, const char* name, dim3 grid, int threads, size_t 
 // The operators, each instantiated in a translation unit of its own (they compile in parallel).
 constexpr unsigned FLAG_INPUT_ONLY = 0x100u;     // internal: see backward_input_offset
 template <typename T, int ND, typename S = T>
+// off = null (float32): every offset is zero.  transposed: the weight of the convolution that this call is
+// the backward pass of.
 int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* bias, S* out, void* ws, size_t ws_bytes,
-            hipStream_t s, bool* declined = nullptr);
+            hipStream_t s, bool* declined = nullptr, bool transposed = false);
 // prep: jobs that belong to the caller, done in the launch that prepares this operator
 template <typename T, int ND, typename S = T>
 int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* off, const S* gout, T* gin, T* goff, void* ws,

@@ -1792,7 +1792,11 @@ __global__ __launch_bounds__(WG) void backward_weight_kernel(Params P, const T* 
         TapGeo<T, ND> t;
         {
             T offv[ND];
-            load_offsets<T, ND>(P, off + (((size_t)n * P.DG + dg) * P.kV + tap) * ND * P.outV, posc, offv);
+            if (off) load_offsets<T, ND>(P, off + (((size_t)n * P.DG + dg) * P.kV + tap) * ND * P.outV, posc, offv);
+            else {                                 // a plain convolution
+#pragma unroll
+                for (int a = 0; a < ND; ++a) offv[a] = 0;
+            }
             tap_setup_noidx<T, ND>(P, offv, ib, kd, t);
         }
         const bool live = valid && t.inside;

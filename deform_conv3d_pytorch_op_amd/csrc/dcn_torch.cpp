@@ -293,22 +293,21 @@ Gradients conv2d_backward(const Config& c, const Tensor& input, const Tensor& we
     const int* g = geo.v;
     const Tensor in = input.contiguous(), w = weight.contiguous(), go = grad_output.contiguous();
     const hipStream_t stream = c10::hip::getCurrentHIPStream(in.device().index()).stream();
-    check(geo.ws_bytes > 0, "inconsistent convolution geometry");
-    const Tensor wst = workspace_tensor(in, geo.ws_bytes);
-    const Workspace ws = workspace(wst, geo.ws_bytes, stream);
-    const bool f32 = in.scalar_type() == at::kFloat;
+    const size_t bytes = conv2d_layer_backward_workspace_bytes((int)in.element_size(), g[0], g[1], g[2], (size_t)(in.size(2) * in.size(3)), (size_t)(out[0] * out[1]),
+                                                               (int)(w.size(2) * w.size(3)), c.group);
+    check(bytes > 0, "inconsistent convolution geometry");
     Gradients r;
-    if (need_data) {
-        r.input = at::zeros_like(in);
-        check_rc(f32 ? conv2d_backward_input_f32(cptr<float>(w), cptr<float>(go), mptr<float>(r.input), GEOC(g), ws.p, ws.n, ws.stream)
-                     : conv2d_backward_input_f64(cptr<double>(w), cptr<double>(go), mptr<double>(r.input), GEOC(g), ws.p, ws.n, ws.stream));
+    if (need_data) r.input = at::empty_like(in);
+    if (need_weight) r.weight = at::empty_like(w);
+    if (need_weight && need_bias) r.bias = at::empty({w.size(0)}, w.options());
+    if (need_data || need_weight) {
+        const Tensor ws = workspace_tensor(in, bytes);
+        auto p = [](const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; };
+#define CALL(SUF, T) conv2d_layer_backward_##SUF(cptr<T>(in), cptr<T>(w), cptr<T>(go), (T*)p(r.input), (T*)p(r.weight), (T*)p(r.bias), GEOC(g), ws.data_ptr(), bytes, stream)
+        check_rc(in.scalar_type() == at::kFloat ? CALL(f32, float) : CALL(f64, double));
+#undef CALL
     }
-    if (need_weight) {
-        r.weight = at::zeros_like(w);
-        check_rc(f32 ? conv2d_backward_weight_f32(cptr<float>(in), cptr<float>(go), mptr<float>(r.weight), GEOC(g), ws.p, ws.n, ws.stream)
-                     : conv2d_backward_weight_f64(cptr<double>(in), cptr<double>(go), mptr<double>(r.weight), GEOC(g), ws.p, ws.n, ws.stream));
-    }
-    if (need_bias) r.bias = go.sum(at::IntArrayRef({0, 2, 3}));
+    if (need_bias && !need_weight) r.bias = go.sum(at::IntArrayRef({0, 2, 3}));
     return r;
 }
 

@@ -200,6 +200,16 @@ int conv2d_backward_weight_f32(const float *input, const float *grad_output, flo
                                void *workspace, size_t workspace_bytes, void *stream);
 int conv2d_backward_weight_f64(const double *input, const double *grad_output, double *grad_weight, CONV2D_GEOMETRY,
                                void *workspace, size_t workspace_bytes, void *stream);
+/* The backward pass in one call: the gradients that are not null (grad_bias only beside grad_weight) are
+ * WRITTEN, not accumulated. */
+size_t conv2d_layer_backward_workspace_bytes(int elem_size, int batch, int input_c, int output_c, size_t input_volume,
+                                             size_t output_volume, int kernel_volume, int group);
+int conv2d_layer_backward_f32(const float *input, const float *weight, const float *grad_output, float *grad_input,
+                              float *grad_weight, float *grad_bias, CONV2D_GEOMETRY, void *workspace,
+                              size_t workspace_bytes, void *stream);
+int conv2d_layer_backward_f64(const double *input, const double *weight, const double *grad_output, double *grad_input,
+                              double *grad_weight, double *grad_bias, CONV2D_GEOMETRY, void *workspace,
+                              size_t workspace_bytes, void *stream);
 
 /* ---- the backward pass of a layer in one call ------------------------------------------------
  * No counterpart in the reference, whose Functions call backward_input_offset and backward_weight and
