@@ -13,15 +13,33 @@ float64 on one MI355X; there is no CPU path.
 import torch
 import torch.nn as nn
 from torch.autograd import Function
+from torch.autograd.function import once_differentiable
 from torch.nn.modules.utils import _pair
 
 from . import _lib
 
 
 class Conv2dFunction(Function):
+    @classmethod
+    def apply(cls, inputs, weight, bias=None, stride=(1, 1), padding=(0, 0), dilation=(1, 1), group=1):
+        if cls is Conv2dFunction:       # (a derived class: through PyTorch's own apply, see functions.py)
+            return _lib.native().conv2d(inputs, weight, bias, stride, padding, dilation, group)
+        return super().apply(inputs, weight, bias, stride, padding, dilation, group)
+
     @staticmethod
-    def apply(inputs, weight, bias=None, stride=(1, 1), padding=(0, 0), dilation=(1, 1), group=1):
-        return _lib.native().conv2d(inputs, weight, bias, stride, padding, dilation, group)
+    def forward(ctx, inputs, weight, bias=None, stride=(1, 1), padding=(0, 0), dilation=(1, 1), group=1):
+        ctx.layer = (stride, padding, dilation, group)
+        ctx.has_bias = bias is not None
+        ctx.save_for_backward(inputs, weight)
+        return _lib.native().conv2d_forward(inputs, weight, bias, *ctx.layer)
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad_output):
+        inputs, weight = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        gi, gw, gb = _lib.native().conv2d_backward(inputs, weight, grad_output, *ctx.layer, need[0], need[1], ctx.has_bias and need[2])
+        return gi, gw, gb, None, None, None, None
 
 
 class Conv2d(nn.Module):

@@ -1,5 +1,6 @@
 // The autograd layer of the package in C++: `_native.conv_offset` and `_native.conv2d` check a call, run
-// the operators of libdcn_amd.so on the current stream and record the backward node.  In Python these
+// the operators of libdcn_amd.so on the current stream and record the backward node; the `_forward` and
+// `_backward` entries are their halves without a node, for the package's Python Functions.  In Python these
 // steps cost more than the kernels of a small layer: every operator call converted some thirty arguments,
 // and the backward half ran on the autograd engine's own thread, which had to take turns for the
 // interpreter lock with the thread that waits for it (2 images of 16 x 16, 8 -> 8 channels, forward and
@@ -382,45 +383,39 @@ Tensor with_history(const Config& c, const Tensor& out, const Tensor& input, con
     return out;
 }
 
-Tensor conv_offset(const Config& c, const Tensor& input, const Tensor& offset, const Tensor& weight, const Tensor& bias) {
+Tensor conv_offset_forward(const Config& c, const Tensor& input, const Tensor& offset, const Tensor& weight, const Tensor& bias) {
     device_check(input, {&offset, &weight, &bias});
     int64_t out[3];
     shape_check(c, input, weight, offset, out);
     const Geometry g = geometry(c, input, weight, out);
     if (bias.defined()) check(bias.dim() == 1 && bias.size(0) == weight.size(0), "bias size");
-    Tensor output;
-    {
-        c10::AutoGradMode no_grad(false);
-        const c10::OptionalDeviceGuard guard(input.device());
-        const Tensor in = input.contiguous(), off = offset.contiguous(), w = weight.contiguous(), b = bias.defined() ? bias.contiguous() : Tensor();
-        int64_t sizes[5] = {input.size(0), weight.size(0), out[0], out[1], c.nd == 3 ? out[2] : 1};
-        output = at::empty(at::IntArrayRef(sizes, c.nd + 2), in.options());
-        const Tensor ws = workspace_tensor(in, g.ws_bytes);
-        check_rc(run_forward(c.nd, dtype_index(in.scalar_type()), in, w, off, b, output, g.v,
-                             workspace(ws, g.ws_bytes, c10::hip::getCurrentHIPStream(in.device().index()).stream())));
-    }
-    return with_history(c, output, input, offset, weight, bias);
+    c10::AutoGradMode no_grad(false);
+    const c10::OptionalDeviceGuard guard(input.device());
+    const Tensor in = input.contiguous(), off = offset.contiguous(), w = weight.contiguous(), b = bias.defined() ? bias.contiguous() : Tensor();
+    int64_t sizes[5] = {input.size(0), weight.size(0), out[0], out[1], c.nd == 3 ? out[2] : 1};
+    Tensor output = at::empty(at::IntArrayRef(sizes, c.nd + 2), in.options());
+    const Tensor ws = workspace_tensor(in, g.ws_bytes);
+    check_rc(run_forward(c.nd, dtype_index(in.scalar_type()), in, w, off, b, output, g.v,
+                         workspace(ws, g.ws_bytes, c10::hip::getCurrentHIPStream(in.device().index()).stream())));
+    return output;
 }
 
-Tensor conv2d(const Config& c, const Tensor& input, const Tensor& weight, const Tensor& bias) {
+Tensor conv2d_forward(const Config& c, const Tensor& input, const Tensor& weight, const Tensor& bias) {
     int64_t out[3];
     conv_check(c, input, weight, bias, out);
     const Geometry geo = geometry(c, input, weight, out);
     const int* g = geo.v;
     check(geo.ws_bytes > 0, "inconsistent convolution geometry");
-    Tensor output;
-    {
-        c10::AutoGradMode no_grad(false);
-        const c10::OptionalDeviceGuard guard(input.device());
-        const Tensor in = input.contiguous(), w = weight.contiguous(), b = bias.defined() ? bias.contiguous() : Tensor();
-        output = at::empty({input.size(0), weight.size(0), out[0], out[1]}, in.options());
-        const Tensor wst = workspace_tensor(in, geo.ws_bytes);
-        const Workspace ws = workspace(wst, geo.ws_bytes, c10::hip::getCurrentHIPStream(in.device().index()).stream());
-        check_rc(in.scalar_type() == at::kFloat
-                     ? conv2d_forward_f32(cptr<float>(in), cptr<float>(w), cptr<float>(b), mptr<float>(output), GEOC(g), ws.p, ws.n, ws.stream)
-                     : conv2d_forward_f64(cptr<double>(in), cptr<double>(w), cptr<double>(b), mptr<double>(output), GEOC(g), ws.p, ws.n, ws.stream));
-    }
-    return with_history(c, output, input, Tensor(), weight, bias);
+    c10::AutoGradMode no_grad(false);
+    const c10::OptionalDeviceGuard guard(input.device());
+    const Tensor in = input.contiguous(), w = weight.contiguous(), b = bias.defined() ? bias.contiguous() : Tensor();
+    Tensor output = at::empty({input.size(0), weight.size(0), out[0], out[1]}, in.options());
+    const Tensor wst = workspace_tensor(in, geo.ws_bytes);
+    const Workspace ws = workspace(wst, geo.ws_bytes, c10::hip::getCurrentHIPStream(in.device().index()).stream());
+    check_rc(in.scalar_type() == at::kFloat
+                 ? conv2d_forward_f32(cptr<float>(in), cptr<float>(w), cptr<float>(b), mptr<float>(output), GEOC(g), ws.p, ws.n, ws.stream)
+                 : conv2d_forward_f64(cptr<double>(in), cptr<double>(w), cptr<double>(b), mptr<double>(output), GEOC(g), ws.p, ws.n, ws.stream));
+    return output;
 }
 
 // ---- Python entry points -------------------------------------------------------------------
@@ -465,46 +460,114 @@ Tensor as_tensor(PyObject* o, const char* what, bool optional = false) {
     return THPVariable_Unpack(o);
 }
 
-// conv_offset(nd, inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group, standard, oob_zero)
-PyObject* py_conv_offset(PyObject*, PyObject* const* a, Py_ssize_t n) {
+PyObject* wrap(const Tensor& t) {
+    if (!t.defined()) Py_RETURN_NONE;
+    return THPVariable_Wrap(t);
+}
+PyObject* wrap(const Gradients& g, bool deform) {
+    const Tensor* ts[4] = {&g.input, deform ? &g.offset : &g.weight, deform ? &g.weight : &g.bias, &g.bias};
+    const Py_ssize_t n = deform ? 4 : 3;
+    PyObject* r = PyTuple_New(n);
+    if (!r) throw python_error();
+    for (Py_ssize_t i = 0; i < n; ++i) PyTuple_SET_ITEM(r, i, wrap(*ts[i]));
+    return r;
+}
+// stride, padding, dilation, channel_per_group, group, standard, oob_zero
+Config layer_config(int nd, PyObject* const* a) {
+    Config c;
+    c.nd = nd;
+    as_ints(a[0], nd, c.stride);
+    as_ints(a[1], nd, c.pad);
+    as_ints(a[2], nd, c.dil);
+    c.cpg = as_int(a[3]);
+    c.group = as_int(a[4]);
+    c.standard = PyObject_IsTrue(a[5]) == 1;
+    c.oob_zero = PyObject_IsTrue(a[6]) == 1;
+    check(c.cpg > 0, "off channel");
+    return c;
+}
+// stride, padding, dilation, group
+Config conv_config(PyObject* const* a) {
+    Config c;
+    c.nd = 2;
+    as_ints(a[0], 2, c.stride);
+    as_ints(a[1], 2, c.pad);
+    as_ints(a[2], 2, c.dil);
+    c.group = as_int(a[3]);
+    return c;
+}
+int axes(PyObject* o) {
+    const int nd = as_int(o);
+    check(nd == 2 || nd == 3, "two or three axes");
+    return nd;
+}
+
+// conv_offset(nd, inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group, standard, oob_zero):
+// the layer with its backward node
+template <bool HISTORY> PyObject* py_conv_offset(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     check(n == 12, "conv_offset takes 12 arguments");
-    Config c;
-    c.nd = as_int(a[0]);
+    const int nd = axes(a[0]);
     const Tensor input = as_tensor(a[1], "inputs"), offset = as_tensor(a[2], "offset"), weight = as_tensor(a[3], "weight"), bias = as_tensor(a[4], "bias", true);
-    as_ints(a[5], c.nd, c.stride);
-    as_ints(a[6], c.nd, c.pad);
-    as_ints(a[7], c.nd, c.dil);
-    c.cpg = as_int(a[8]);
-    c.group = as_int(a[9]);
-    c.standard = PyObject_IsTrue(a[10]) == 1;
-    c.oob_zero = PyObject_IsTrue(a[11]) == 1;
-    check(c.cpg > 0, "off channel");
+    const Config c = layer_config(nd, a + 5);
     Tensor out;
     {
         pybind11::gil_scoped_release nogil;
-        out = conv_offset(c, input, offset, weight, bias);
+        out = conv_offset_forward(c, input, offset, weight, bias);
+        if (HISTORY) out = with_history(c, out, input, offset, weight, bias);
     }
     return THPVariable_Wrap(out);
     END_HANDLE_TH_ERRORS
 }
-// conv2d(inputs, weight, bias, stride, padding, dilation, group)
-PyObject* py_conv2d(PyObject*, PyObject* const* a, Py_ssize_t n) {
+// conv_offset_backward(nd, inputs, offset, weight, grad_output, stride, padding, dilation, channel_per_group, group, standard,
+// oob_zero, need_data, need_weight, need_bias): the gradients of inputs, offset, weight, bias, None where not needed
+PyObject* py_conv_offset_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    check(n == 15, "conv_offset_backward takes 15 arguments");
+    const int nd = axes(a[0]);
+    const Tensor input = as_tensor(a[1], "inputs"), offset = as_tensor(a[2], "offset"), weight = as_tensor(a[3], "weight"), go = as_tensor(a[4], "grad_output");
+    const Config c = layer_config(nd, a + 5);
+    const bool data = PyObject_IsTrue(a[12]) == 1, w = PyObject_IsTrue(a[13]) == 1, b = PyObject_IsTrue(a[14]) == 1;
+    Gradients g;
+    {
+        pybind11::gil_scoped_release nogil;
+        c10::AutoGradMode no_grad(false);
+        const c10::OptionalDeviceGuard guard(input.device());
+        g = conv_offset_backward(c, input, offset, weight, go, data, w, b);
+    }
+    return wrap(g, true);
+    END_HANDLE_TH_ERRORS
+}
+// conv2d(inputs, weight, bias, stride, padding, dilation, group): the layer with its backward node
+template <bool HISTORY> PyObject* py_conv2d(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     check(n == 7, "conv2d takes 7 arguments");
-    Config c;
-    c.nd = 2;
     const Tensor input = as_tensor(a[0], "inputs"), weight = as_tensor(a[1], "weight"), bias = as_tensor(a[2], "bias", true);
-    as_ints(a[3], 2, c.stride);
-    as_ints(a[4], 2, c.pad);
-    as_ints(a[5], 2, c.dil);
-    c.group = as_int(a[6]);
+    const Config c = conv_config(a + 3);
     Tensor out;
     {
         pybind11::gil_scoped_release nogil;
-        out = conv2d(c, input, weight, bias);
+        out = conv2d_forward(c, input, weight, bias);
+        if (HISTORY) out = with_history(c, out, input, Tensor(), weight, bias);
     }
     return THPVariable_Wrap(out);
+    END_HANDLE_TH_ERRORS
+}
+// conv2d_backward(inputs, weight, grad_output, stride, padding, dilation, group, need_data, need_weight, need_bias)
+PyObject* py_conv2d_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    check(n == 10, "conv2d_backward takes 10 arguments");
+    const Tensor input = as_tensor(a[0], "inputs"), weight = as_tensor(a[1], "weight"), go = as_tensor(a[2], "grad_output");
+    const Config c = conv_config(a + 3);
+    const bool data = PyObject_IsTrue(a[7]) == 1, w = PyObject_IsTrue(a[8]) == 1, b = PyObject_IsTrue(a[9]) == 1;
+    Gradients g;
+    {
+        pybind11::gil_scoped_release nogil;
+        c10::AutoGradMode no_grad(false);
+        const c10::OptionalDeviceGuard guard(input.device());
+        g = conv2d_backward(c, input, weight, go, data, w, b);
+    }
+    return wrap(g, false);
     END_HANDLE_TH_ERRORS
 }
 // set_error(type): the exception class for calls that the library rejects
@@ -515,8 +578,14 @@ PyObject* py_set_error(PyObject*, PyObject* type) {
     Py_RETURN_NONE;
 }
 
-PyMethodDef methods[] = {{"conv_offset", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_conv_offset)), METH_FASTCALL, nullptr},
-                         {"conv2d", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_conv2d)), METH_FASTCALL, nullptr},
+using FastCall = PyObject* (*)(PyObject*, PyObject* const*, Py_ssize_t);
+PyCFunction method(FastCall f) { return reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(f)); }
+PyMethodDef methods[] = {{"conv_offset", method(py_conv_offset<true>), METH_FASTCALL, nullptr},
+                         {"conv_offset_forward", method(py_conv_offset<false>), METH_FASTCALL, nullptr},
+                         {"conv_offset_backward", method(py_conv_offset_backward), METH_FASTCALL, nullptr},
+                         {"conv2d", method(py_conv2d<true>), METH_FASTCALL, nullptr},
+                         {"conv2d_forward", method(py_conv2d<false>), METH_FASTCALL, nullptr},
+                         {"conv2d_backward", method(py_conv2d_backward), METH_FASTCALL, nullptr},
                          {"set_error", py_set_error, METH_O, nullptr},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -17,10 +17,12 @@ not required come back as None instead of crashing (the reference wraps None in 
 All tensors must live on one MI355X; there is no CPU path.
 
 `apply` hands over to the C++ extension (csrc/dcn_torch.cpp), which checks the call, runs the
-operators and records the backward node; `shape_check` restates its checks in Python.
+operators and records the backward node; a class derived from one of the Functions goes through
+PyTorch's own `Function.apply` and its `forward` and `backward`, which run the same operators.
 """
 import torch
 from torch.autograd import Function
+from torch.autograd.function import once_differentiable
 
 from . import _lib
 
@@ -95,25 +97,75 @@ def _workspace(inputs, weight, group, out_sizes, channel_per_group):
     return torch.empty(max(nbytes, 1), dtype=torch.uint8, device=inputs.device), nbytes
 
 
-def _apply(nd, inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group, standard_output_size,
-           oob_offset_grad):
+def _oob_zero(oob_offset_grad):
     if oob_offset_grad not in ("reference", "zero"):
         raise ValueError("oob_offset_grad must be 'reference' or 'zero'")
-    return _lib.native().conv_offset(nd, inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group,
-                                     standard_output_size, oob_offset_grad == "zero")
+    return oob_offset_grad == "zero"
 
 
-class ConvOffset3dFunction(Function):
-    @staticmethod
-    def apply(inputs, offset, weight, bias=None, stride=(1, 1, 1), padding=(0, 0, 0), dilation=(1, 1, 1),
+class _ConvOffsetNdFunction(Function):
+    ND = 0
+
+    @classmethod
+    def _fwd(cls, ctx, inputs, offset, weight, bias, *layer):
+        ctx.layer = layer[:-1] + (_oob_zero(layer[-1]),)
+        ctx.has_bias = bias is not None
+        ctx.save_for_backward(inputs, offset, weight)
+        return _lib.native().conv_offset_forward(cls.ND, inputs, offset, weight, bias, *ctx.layer)
+
+    @classmethod
+    def _bwd(cls, ctx, grad_output):
+        inputs, offset, weight = ctx.saved_tensors
+        need = ctx.needs_input_grad
+        # grad_input and grad_offset come out of one kernel, as in the reference (:52)
+        gi, go, gw, gb = _lib.native().conv_offset_backward(cls.ND, inputs, offset, weight, grad_output, *ctx.layer, need[0] or need[1],
+                                                            need[2], ctx.has_bias and need[3])
+        return (gi if need[0] else None, go if need[1] else None, gw, gb) + (None,) * 7
+
+
+class ConvOffset3dFunction(_ConvOffsetNdFunction):
+    ND = 3
+
+    @classmethod
+    def apply(cls, inputs, offset, weight, bias=None, stride=(1, 1, 1), padding=(0, 0, 0), dilation=(1, 1, 1),
               channel_per_group=1, group=1, standard_output_size=False, oob_offset_grad="reference"):
-        return _apply(3, inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group,
-                      standard_output_size, oob_offset_grad)
+        if cls is ConvOffset3dFunction:
+            return _lib.native().conv_offset(3, inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group,
+                                             standard_output_size, _oob_zero(oob_offset_grad))
+        return super().apply(inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group,
+                             standard_output_size, oob_offset_grad)
 
-
-class ConvOffset2dFunction(Function):
     @staticmethod
-    def apply(inputs, offset, weight, bias=None, stride=(1, 1), padding=(0, 0), dilation=(1, 1),
+    def forward(ctx, inputs, offset, weight, bias=None, stride=(1, 1, 1), padding=(0, 0, 0), dilation=(1, 1, 1),
+                channel_per_group=1, group=1, standard_output_size=False, oob_offset_grad="reference"):
+        return ConvOffset3dFunction._fwd(ctx, inputs, offset, weight, bias, stride, padding, dilation,
+                                         channel_per_group, group, standard_output_size, oob_offset_grad)
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad_output):
+        return ConvOffset3dFunction._bwd(ctx, grad_output)
+
+
+class ConvOffset2dFunction(_ConvOffsetNdFunction):
+    ND = 2
+
+    @classmethod
+    def apply(cls, inputs, offset, weight, bias=None, stride=(1, 1), padding=(0, 0), dilation=(1, 1),
               channel_per_group=1, group=1, standard_output_size=False, oob_offset_grad="reference"):
-        return _apply(2, inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group,
-                      standard_output_size, oob_offset_grad)
+        if cls is ConvOffset2dFunction:
+            return _lib.native().conv_offset(2, inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group,
+                                             standard_output_size, _oob_zero(oob_offset_grad))
+        return super().apply(inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group,
+                             standard_output_size, oob_offset_grad)
+
+    @staticmethod
+    def forward(ctx, inputs, offset, weight, bias=None, stride=(1, 1), padding=(0, 0), dilation=(1, 1),
+                channel_per_group=1, group=1, standard_output_size=False, oob_offset_grad="reference"):
+        return ConvOffset2dFunction._fwd(ctx, inputs, offset, weight, bias, stride, padding, dilation,
+                                         channel_per_group, group, standard_output_size, oob_offset_grad)
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, grad_output):
+        return ConvOffset2dFunction._bwd(ctx, grad_output)

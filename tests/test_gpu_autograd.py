@@ -1,0 +1,43 @@
+"""The package's Functions beside backward: derived classes, tracing, forward mode, saved-tensor hooks,
+undefined and misshapen gradients."""
+import pytest
+import torch
+
+from tests.cases import make_case
+
+pytestmark = pytest.mark.gpu
+
+LAYERS = {"2d": (2, 1, 8, 6, (7, 9), 3, 1, 1, 1, 4, 2, 1.5), "3d": (3, 1, 4, 6, (4, 5, 6), 3, 1, 1, 1, 4, 1, 1.5), "conv2d": None}
+
+
+def _layer(name):
+    """The Function, its arguments (leaves on the GPU that need gradients first) and a grad_output."""
+    import deform_conv3d_pytorch_op_amd as dcn
+    if name == "conv2d":
+        g = torch.Generator().manual_seed(5)
+        leaves = [torch.randn(s, generator=g).cuda().requires_grad_() for s in ((2, 6, 8, 7), (4, 3, 3, 3), (4,))]
+        return dcn.Conv2dFunction, leaves, ((1, 1), (1, 1), (1, 1), 2), torch.randn((2, 4, 8, 7), generator=g).cuda()
+    c = make_case(*LAYERS[name], dtype=torch.float32, seed=5)
+    fn = dcn.ConvOffset3dFunction if c["nd"] == 3 else dcn.ConvOffset2dFunction
+    leaves = [c[k].cuda().requires_grad_() for k in ("x", "off", "w", "b")]
+    return fn, leaves, (c["stride"], c["pad"], c["dil"], c["cpg"], c["groups"]), c["gout"].cuda()
+
+
+def _results(fn, leaves, cfg, gout):
+    out = fn.apply(*leaves, *cfg)
+    return [out] + list(torch.autograd.grad(out, leaves, gout))
+
+
+def _same(got, want):
+    """Equal but for the float atomics that grad_input and grad_offset end in."""
+    for g, w in zip(got, want):
+        assert g.shape == w.shape and (g - w).norm().item() <= 1e-5 * w.norm().item()
+
+
+@pytest.mark.parametrize("name", LAYERS)
+def test_derived_class_matches_the_function(name):
+    print("derived", name, flush=True)
+    fn, leaves, cfg, gout = _layer(name)
+    derived = type("Derived", (fn,), {})
+    assert derived.apply(*leaves, *cfg).grad_fn.name() == "DerivedBackward"
+    _same(_results(derived, leaves, cfg, gout), _results(fn, leaves, cfg, gout))
