@@ -22,8 +22,10 @@ from . import _lib
 class Conv2dFunction(Function):
     @classmethod
     def apply(cls, inputs, weight, bias=None, stride=(1, 1), padding=(0, 0), dilation=(1, 1), group=1):
-        if cls is Conv2dFunction:       # (a derived class: through PyTorch's own apply, see functions.py)
-            return _lib.native().conv2d(inputs, weight, bias, stride, padding, dilation, group)
+        if cls is Conv2dFunction:       # (otherwise through PyTorch's own apply, see functions.py)
+            out = _lib.native().conv2d(inputs, weight, bias, stride, padding, dilation, group)
+            if out is not NotImplemented:
+                return out
         return super().apply(inputs, weight, bias, stride, padding, dilation, group)
 
     @staticmethod

@@ -21,6 +21,7 @@
 #include <torch/csrc/autograd/functions/utils.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/autograd/saved_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 
 #include <cstdlib>
 #include <cstring>
@@ -502,13 +503,25 @@ int axes(PyObject* o) {
     return nd;
 }
 
+// Whether a call has to go through PyTorch's Function.apply, because more than backward has to know about it: a
+// trace being recorded (the tracer sees no operator of libdcn_amd.so and would keep the allocation of the output alone).
+bool wants_function() {
+    return torch::jit::tracer::isTracing();
+}
+PyObject* py_wants_function(PyObject*, PyObject*) {
+    HANDLE_TH_ERRORS
+    return PyBool_FromLong(wants_function());
+    END_HANDLE_TH_ERRORS
+}
+
 // conv_offset(nd, inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group, standard, oob_zero):
-// the layer with its backward node
+// the layer with its backward node; NotImplemented when the call has to go through Function.apply
 template <bool HISTORY> PyObject* py_conv_offset(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     check(n == 12, "conv_offset takes 12 arguments");
     const int nd = axes(a[0]);
     const Tensor input = as_tensor(a[1], "inputs"), offset = as_tensor(a[2], "offset"), weight = as_tensor(a[3], "weight"), bias = as_tensor(a[4], "bias", true);
+    if (HISTORY && wants_function()) Py_RETURN_NOTIMPLEMENTED;
     const Config c = layer_config(nd, a + 5);
     Tensor out;
     {
@@ -538,11 +551,12 @@ PyObject* py_conv_offset_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return wrap(g, true);
     END_HANDLE_TH_ERRORS
 }
-// conv2d(inputs, weight, bias, stride, padding, dilation, group): the layer with its backward node
+// conv2d(inputs, weight, bias, stride, padding, dilation, group): the layer with its backward node, or NotImplemented
 template <bool HISTORY> PyObject* py_conv2d(PyObject*, PyObject* const* a, Py_ssize_t n) {
     HANDLE_TH_ERRORS
     check(n == 7, "conv2d takes 7 arguments");
     const Tensor input = as_tensor(a[0], "inputs"), weight = as_tensor(a[1], "weight"), bias = as_tensor(a[2], "bias", true);
+    if (HISTORY && wants_function()) Py_RETURN_NOTIMPLEMENTED;
     const Config c = conv_config(a + 3);
     Tensor out;
     {
@@ -586,6 +600,7 @@ PyMethodDef methods[] = {{"conv_offset", method(py_conv_offset<true>), METH_FAST
                          {"conv2d", method(py_conv2d<true>), METH_FASTCALL, nullptr},
                          {"conv2d_forward", method(py_conv2d<false>), METH_FASTCALL, nullptr},
                          {"conv2d_backward", method(py_conv2d_backward), METH_FASTCALL, nullptr},
+                         {"wants_function", py_wants_function, METH_NOARGS, nullptr},
                          {"set_error", py_set_error, METH_O, nullptr},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

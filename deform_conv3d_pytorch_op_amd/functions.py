@@ -17,8 +17,9 @@ not required come back as None instead of crashing (the reference wraps None in 
 All tensors must live on one MI355X; there is no CPU path.
 
 `apply` hands over to the C++ extension (csrc/dcn_torch.cpp), which checks the call, runs the
-operators and records the backward node; a class derived from one of the Functions goes through
-PyTorch's own `Function.apply` and its `forward` and `backward`, which run the same operators.
+operators and records the backward node.  A call under `torch.jit.trace` and a class derived from one of
+the Functions go through PyTorch's own `Function.apply` and the class's `forward` and `backward`, which run
+the same operators.
 """
 import torch
 from torch.autograd import Function
@@ -130,8 +131,10 @@ class ConvOffset3dFunction(_ConvOffsetNdFunction):
     def apply(cls, inputs, offset, weight, bias=None, stride=(1, 1, 1), padding=(0, 0, 0), dilation=(1, 1, 1),
               channel_per_group=1, group=1, standard_output_size=False, oob_offset_grad="reference"):
         if cls is ConvOffset3dFunction:
-            return _lib.native().conv_offset(3, inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group,
-                                             standard_output_size, _oob_zero(oob_offset_grad))
+            out = _lib.native().conv_offset(3, inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group,
+                                            standard_output_size, _oob_zero(oob_offset_grad))
+            if out is not NotImplemented:
+                return out
         return super().apply(inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group,
                              standard_output_size, oob_offset_grad)
 
@@ -154,8 +157,10 @@ class ConvOffset2dFunction(_ConvOffsetNdFunction):
     def apply(cls, inputs, offset, weight, bias=None, stride=(1, 1), padding=(0, 0), dilation=(1, 1),
               channel_per_group=1, group=1, standard_output_size=False, oob_offset_grad="reference"):
         if cls is ConvOffset2dFunction:
-            return _lib.native().conv_offset(2, inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group,
-                                             standard_output_size, _oob_zero(oob_offset_grad))
+            out = _lib.native().conv_offset(2, inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group,
+                                            standard_output_size, _oob_zero(oob_offset_grad))
+            if out is not NotImplemented:
+                return out
         return super().apply(inputs, offset, weight, bias, stride, padding, dilation, channel_per_group, group,
                              standard_output_size, oob_offset_grad)
 

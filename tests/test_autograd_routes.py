@@ -31,3 +31,37 @@ def test_derived_classes_run_their_own_forward_and_backward(fn):
     assert torch.equal(y.detach(), 2 * x.detach())
     y.sum().backward()
     assert torch.equal(x.grad, torch.full((4,), 2.0))
+
+
+def test_a_trace_being_recorded_goes_through_function_apply():
+    """... which the tracer records; it sees nothing of the operators themselves."""
+    from deform_conv3d_pytorch_op_amd import _lib
+    native, seen = _lib.native(), []
+
+    def f(x):
+        seen.append(native.wants_function())
+        return x + 1
+    f(torch.zeros(2))
+    torch.jit.trace(f, torch.zeros(2), check_trace=False)
+    f(torch.zeros(2))
+    assert seen == [False, True, False]
+
+
+@pytest.mark.parametrize("fn", _functions(), ids=lambda f: f.__name__)
+def test_a_traced_call_is_recorded_as_the_function(fn):
+    """On the CPU the call itself is refused (there is no CPU path), by the Function's own forward."""
+    import deform_conv3d_pytorch_op_amd as dcn
+    nd = 3 if fn is dcn.ConvOffset3dFunction else 2
+    x, w = torch.zeros((1, 2) + (4,) * nd), torch.zeros((2, 2) + (1,) * nd)
+    args = (x, w) if fn is dcn.Conv2dFunction else (x, torch.zeros((1, 2 * nd) + (4,) * nd), w)
+    calls, forward = [], fn.forward
+    fn.forward = staticmethod(lambda *a: calls.append(len(a)) or forward(*a))
+    try:
+        with pytest.raises(RuntimeError, match="GPU"):
+            fn.apply(*args)
+        assert calls == []
+        with pytest.raises(RuntimeError, match="GPU|float32"):
+            torch.jit.trace(lambda *t: fn.apply(*t), args, check_trace=False)
+        assert len(calls) == 1
+    finally:
+        fn.forward = forward

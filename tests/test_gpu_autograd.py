@@ -41,3 +41,27 @@ def test_derived_class_matches_the_function(name):
     derived = type("Derived", (fn,), {})
     assert derived.apply(*leaves, *cfg).grad_fn.name() == "DerivedBackward"
     _same(_results(derived, leaves, cfg, gout), _results(fn, leaves, cfg, gout))
+
+
+@pytest.mark.parametrize("name", LAYERS)
+def test_trace_replays_the_layer(name):
+    """A recorded layer gives the layer's results on other inputs, and its gradients."""
+    print("trace", name, flush=True)
+    fn, leaves, cfg, gout = _layer(name)
+    traced = torch.jit.trace(lambda *t: fn.apply(*t, *cfg) * 2, [t.detach() for t in leaves], check_trace=False)
+    assert fn.__name__ in str(traced.graph)
+    for k in range(2):
+        other = [(t.detach() * (1 + k) + 0.25).requires_grad_() for t in leaves]
+        out = traced(*other)
+        want = fn.apply(*other, *cfg) * 2
+        assert torch.equal(out, want)
+        _same(torch.autograd.grad(out, other, gout), torch.autograd.grad(want, other, gout))
+
+
+def test_traced_module():
+    import deform_conv3d_pytorch_op_amd as dcn
+    print("traced module", flush=True)
+    m = torch.nn.Sequential(dcn.ConvOffset2dPack(4, 6, 3, padding=1, channel_per_group=4), torch.nn.ReLU()).cuda()
+    x = torch.randn(2, 4, 9, 8, generator=torch.Generator().manual_seed(1)).cuda()
+    traced = torch.jit.trace(m, x)
+    assert torch.equal(traced(x), m(x)) and torch.equal(traced(x + 1), m(x + 1))
