@@ -503,14 +503,27 @@ int axes(PyObject* o) {
     return nd;
 }
 
-// Whether a call has to go through PyTorch's Function.apply, because more than backward has to know about it: a
-// trace being recorded (the tracer sees no operator of libdcn_amd.so and would keep the allocation of the output alone).
-bool wants_function() {
-    return torch::jit::tracer::isTracing();
+// Whether a call has to go through PyTorch's Function.apply, because more than backward has to know about it:
+// - a trace being recorded: the tracer sees no operator of libdcn_amd.so and would keep the allocation of the output alone;
+// - an argument with a forward-mode tangent, which the node here would drop without a word (Function.apply refuses it);
+// - functorch transforms (vmap, torch.func.grad, ...), likewise refused there, and wrappers that outlived one.
+bool wants_function(std::initializer_list<const Tensor*> args) {
+    using c10::DispatchKey;
+    using c10::DispatchKeySet;
+    if (torch::jit::tracer::isTracing()) return true;
+    if (c10::impl::tls_local_dispatch_key_set().included_.has_any(
+            DispatchKeySet({DispatchKey::FuncTorchDynamicLayerFrontMode, DispatchKey::FuncTorchDynamicLayerBackMode})))
+        return true;
+    for (const Tensor* t : args)
+        if (t->defined() && (t->_fw_grad(0).defined() ||
+                             t->key_set().has_any(DispatchKeySet({DispatchKey::FuncTorchGradWrapper, DispatchKey::FuncTorchBatched}))))
+            return true;
+    return false;
 }
-PyObject* py_wants_function(PyObject*, PyObject*) {
+PyObject* py_wants_function(PyObject*, PyObject* arg) {
     HANDLE_TH_ERRORS
-    return PyBool_FromLong(wants_function());
+    const Tensor t = as_tensor(arg, "argument");
+    return PyBool_FromLong(wants_function({&t}));
     END_HANDLE_TH_ERRORS
 }
 
@@ -521,7 +534,7 @@ template <bool HISTORY> PyObject* py_conv_offset(PyObject*, PyObject* const* a, 
     check(n == 12, "conv_offset takes 12 arguments");
     const int nd = axes(a[0]);
     const Tensor input = as_tensor(a[1], "inputs"), offset = as_tensor(a[2], "offset"), weight = as_tensor(a[3], "weight"), bias = as_tensor(a[4], "bias", true);
-    if (HISTORY && wants_function()) Py_RETURN_NOTIMPLEMENTED;
+    if (HISTORY && wants_function({&input, &offset, &weight, &bias})) Py_RETURN_NOTIMPLEMENTED;
     const Config c = layer_config(nd, a + 5);
     Tensor out;
     {
@@ -556,7 +569,7 @@ template <bool HISTORY> PyObject* py_conv2d(PyObject*, PyObject* const* a, Py_ss
     HANDLE_TH_ERRORS
     check(n == 7, "conv2d takes 7 arguments");
     const Tensor input = as_tensor(a[0], "inputs"), weight = as_tensor(a[1], "weight"), bias = as_tensor(a[2], "bias", true);
-    if (HISTORY && wants_function()) Py_RETURN_NOTIMPLEMENTED;
+    if (HISTORY && wants_function({&input, &weight, &bias})) Py_RETURN_NOTIMPLEMENTED;
     const Config c = conv_config(a + 3);
     Tensor out;
     {
@@ -600,7 +613,7 @@ PyMethodDef methods[] = {{"conv_offset", method(py_conv_offset<true>), METH_FAST
                          {"conv2d", method(py_conv2d<true>), METH_FASTCALL, nullptr},
                          {"conv2d_forward", method(py_conv2d<false>), METH_FASTCALL, nullptr},
                          {"conv2d_backward", method(py_conv2d_backward), METH_FASTCALL, nullptr},
-                         {"wants_function", py_wants_function, METH_NOARGS, nullptr},
+                         {"wants_function", py_wants_function, METH_O, nullptr},
                          {"set_error", py_set_error, METH_O, nullptr},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -19,7 +19,8 @@ All tensors must live on one MI355X; there is no CPU path.
 `apply` hands over to the C++ extension (csrc/dcn_torch.cpp), which checks the call, runs the
 operators and records the backward node.  A call under `torch.jit.trace` and a class derived from one of
 the Functions go through PyTorch's own `Function.apply` and the class's `forward` and `backward`, which run
-the same operators.
+the same operators; so do arguments with forward-mode tangents and calls under functorch transforms, which
+`Function.apply` refuses (the layers have no forward-mode derivative).
 """
 import torch
 from torch.autograd import Function

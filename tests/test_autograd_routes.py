@@ -39,7 +39,7 @@ def test_a_trace_being_recorded_goes_through_function_apply():
     native, seen = _lib.native(), []
 
     def f(x):
-        seen.append(native.wants_function())
+        seen.append(native.wants_function(x))
         return x + 1
     f(torch.zeros(2))
     torch.jit.trace(f, torch.zeros(2), check_trace=False)
@@ -65,3 +65,30 @@ def test_a_traced_call_is_recorded_as_the_function(fn):
         assert len(calls) == 1
     finally:
         fn.forward = forward
+
+
+@pytest.mark.parametrize("fn", _functions(), ids=lambda f: f.__name__)
+@pytest.mark.parametrize("at", range(4))
+def test_forward_mode_tangents_are_refused(fn, at):
+    """A tangent on any argument: refused by Function.apply, not dropped."""
+    import torch.autograd.forward_ad as fwad
+    forward = fn.forward
+    fn.forward = staticmethod(lambda ctx, inputs, *rest: inputs * 2)       # (needs no GPU)
+    try:
+        args = [torch.ones(3) for _ in range(3 if fn.__name__ == "Conv2dFunction" else 4)]
+        at = min(at, len(args) - 1)
+        with fwad.dual_level():
+            args[at] = fwad.make_dual(args[at], torch.ones(3))
+            with pytest.raises(NotImplementedError, match="jvp"):
+                fn.apply(*args)
+    finally:
+        fn.forward = forward
+
+
+@pytest.mark.parametrize("fn", _functions(), ids=lambda f: f.__name__)
+def test_functorch_transforms_are_refused_by_name(fn):
+    args = [torch.ones(3) for _ in range(2 if fn.__name__ == "Conv2dFunction" else 3)]
+    for call in (lambda: torch.vmap(lambda t: fn.apply(t, *args[1:]))(torch.ones(2, 3)),
+                 lambda: torch.func.grad(lambda t: fn.apply(t, *args[1:]).sum())(args[0])):
+        with pytest.raises(RuntimeError, match="functorch transforms"):
+            call()

@@ -65,3 +65,17 @@ def test_traced_module():
     x = torch.randn(2, 4, 9, 8, generator=torch.Generator().manual_seed(1)).cuda()
     traced = torch.jit.trace(m, x)
     assert torch.equal(traced(x), m(x)) and torch.equal(traced(x + 1), m(x + 1))
+
+
+@pytest.mark.parametrize("name", LAYERS)
+def test_forward_mode_is_refused(name):
+    import torch.autograd.forward_ad as fwad
+    print("forward mode", name, flush=True)
+    fn, leaves, cfg, _ = _layer(name)
+    for at in range(len(leaves)):
+        with fwad.dual_level():
+            args = [t.detach() for t in leaves]
+            args[at] = fwad.make_dual(args[at], torch.ones_like(args[at]))
+            with pytest.raises(NotImplementedError, match="jvp"):
+                fn.apply(*args, *cfg)
+    assert fn.apply(*leaves, *cfg).grad_fn is not None
