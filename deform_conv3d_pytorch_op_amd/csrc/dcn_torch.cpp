@@ -331,7 +331,8 @@ struct LayerBackward : public Node {
         const bool deform = cfg.cpg > 0;
         const size_t at_w = deform ? 2 : 1, n = at_w + 1 + (has_bias ? 1 : 0);
         variable_list res(n);
-        if (!grads[0].defined()) return res;
+        // (a gradient that is not defined is zeros, as for a Function)
+        const Tensor grad_output = grads[0].defined() ? grads[0] : input_metadata(0).zeros_like();
         const Tensor input = input_.unpack(), weight = weight_.unpack(), offset = deform ? offset_.unpack() : Tensor();
         const bool need_in = task_should_compute_output(0), need_off = deform && task_should_compute_output(1);
         const bool need_w = task_should_compute_output(at_w), need_b = has_bias && task_should_compute_output(at_w + 1);
@@ -339,14 +340,14 @@ struct LayerBackward : public Node {
         {
             c10::AutoGradMode off_mode(false);
             const c10::OptionalDeviceGuard guard(input.device());
-            Gradients g = deform ? conv_offset_backward(cfg, input, offset, weight, grads[0], need_in || need_off, need_w, need_b)
-                                 : conv2d_backward(cfg, input, weight, grads[0], need_in, need_w, need_b);
+            Gradients g = deform ? conv_offset_backward(cfg, input, offset, weight, grad_output, need_in || need_off, need_w, need_b)
+                                 : conv2d_backward(cfg, input, weight, grad_output, need_in, need_w, need_b);
             if (need_in) res[0] = std::move(g.input);
             if (need_off) res[1] = std::move(g.offset);
             if (need_w) res[at_w] = std::move(g.weight);
             if (need_b) res[at_w + 1] = std::move(g.bias);
         }
-        if (create_graph && grads[0].requires_grad()) {
+        if (create_graph && grad_output.requires_grad()) {
             // no second derivative: results that say so when they are differentiated
             auto fail = std::make_shared<torch::autograd::DelayedError>(
                 "trying to differentiate twice a function that was marked with @once_differentiable", (int64_t)n);

@@ -79,3 +79,23 @@ def test_forward_mode_is_refused(name):
             with pytest.raises(NotImplementedError, match="jvp"):
                 fn.apply(*args, *cfg)
     assert fn.apply(*leaves, *cfg).grad_fn is not None
+
+
+class _NoGradient(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, t):
+        return t.sum()
+
+    @staticmethod
+    def backward(ctx, grad_output):
+        return None
+
+
+@pytest.mark.parametrize("name", LAYERS)
+def test_an_undefined_gradient_is_zeros(name):
+    """... as it is for a Function: the gradients are there, and zero."""
+    print("undefined gradient", name, flush=True)
+    fn, leaves, cfg, _ = _layer(name)
+    _NoGradient.apply(fn.apply(*leaves, *cfg)).backward()
+    for t in leaves:
+        assert t.grad is not None and t.grad.shape == t.shape and not t.grad.any()
