@@ -120,8 +120,8 @@ Geometry geometry(const Config& c, const Tensor& input, const Tensor& weight, co
     return g;
 }
 
-// The checks of the reference's shape_check with its messages.
-void shape_check(const Config& c, const Tensor& input, const Tensor& weight, const Tensor& offset, int64_t* out) {
+// The checks of the reference's shape_check with its messages; `shape`: of grad_output, in the backward pass.
+void shape_check(const Config& c, const Tensor& input, const Tensor& weight, const Tensor& offset, int64_t* out, const at::IntArrayRef* shape = nullptr) {
     static const char* const out_msg[2][3] = {{"error outhh", "error outww", ""}, {"error output ll", "error outhh", "error outww"}};
     static const char* const off_msg[2][3] = {{"off h", "off w", ""}, {"off l", "off h", "off w"}};
     const int nd = c.nd;
@@ -129,15 +129,20 @@ void shape_check(const Config& c, const Tensor& input, const Tensor& weight, con
     check(weight.dim() == nd + 2, "kernel dim");
     output_size(c, input, weight, c.standard, out);
     check(input.size(1) == weight.size(1) * c.group, "input c != kernel c");
+    if (shape) {
+        check((int)shape->size() == nd + 2, "output dim");
+        check((*shape)[0] == input.size(0), "output b != input b");
+        check((*shape)[1] == weight.size(0), "ou c != ker c");
+    }
     check(offset.dim() == nd + 2, "off dim");
     check(offset.size(0) == input.size(0), "off batch");
     int64_t kv = 1;
     for (int a = 0; a < nd; ++a) kv *= weight.size(2 + a);
     check(c.cpg > 0 && input.size(1) % c.cpg == 0, "off channel");
     check(offset.size(1) == input.size(1) / c.cpg * nd * kv, "off channel");
-    for (int a = 0; a < nd; ++a) check(offset.size(2 + a) == out[a], off_msg[nd - 2][a]);
+    for (int a = 0; a < nd; ++a) check(offset.size(2 + a) == (shape ? (*shape)[2 + a] : out[a]), off_msg[nd - 2][a]);
     for (int a = 0; a < nd; ++a)
-        check(input.size(2 + a) + 2 * c.pad[a] - weight.size(2 + a) >= 0 && out[a] >= 1, out_msg[nd - 2][a]);
+        check(input.size(2 + a) + 2 * c.pad[a] - weight.size(2 + a) >= 0 && out[a] >= 1 && (!shape || (*shape)[2 + a] == out[a]), out_msg[nd - 2][a]);
     check(c.group > 0 && weight.size(0) % c.group == 0, "ou c != ker c");
 }
 void conv_check(const Config& c, const Tensor& input, const Tensor& weight, const Tensor& bias, int64_t* out) {
@@ -248,7 +253,8 @@ Gradients conv_offset_backward(const Config& c, const Tensor& input, const Tenso
                                bool need_weight, bool need_bias) {
     device_check(input, {&offset, &weight, &grad_output});
     int64_t out[3];
-    shape_check(c, input, weight, offset, out);
+    const at::IntArrayRef shape = grad_output.sizes();
+    shape_check(c, input, weight, offset, out, &shape);
     const Geometry g = geometry(c, input, weight, out);
     const Tensor in = input.contiguous(), off = offset.contiguous(), w = weight.contiguous(), go = grad_output.contiguous();
     const int dt = dtype_index(in.scalar_type());
@@ -291,6 +297,11 @@ Gradients conv_offset_backward(const Config& c, const Tensor& input, const Tenso
 Gradients conv2d_backward(const Config& c, const Tensor& input, const Tensor& weight, const Tensor& grad_output, bool need_data, bool need_weight, bool need_bias) {
     int64_t out[3];
     conv_check(c, input, weight, grad_output, out);
+    check(grad_output.dim() == 4, "output dim");
+    check(grad_output.size(0) == input.size(0), "output b != input b");
+    check(grad_output.size(1) == weight.size(0), "ou c != ker c");
+    check(grad_output.size(2) == out[0], "error outhh");
+    check(grad_output.size(3) == out[1], "error outww");
     const Geometry geo = geometry(c, input, weight, out);
     const int* g = geo.v;
     const Tensor in = input.contiguous(), w = weight.contiguous(), go = grad_output.contiguous();
@@ -598,6 +609,27 @@ PyObject* py_conv2d_backward(PyObject*, PyObject* const* a, Py_ssize_t n) {
     return wrap(g, false);
     END_HANDLE_TH_ERRORS
 }
+// shape_check(nd, inputs, weight, offset, output_shape, stride, padding, dilation, channel_per_group, group, standard)
+PyObject* py_shape_check(PyObject*, PyObject* const* a, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    check(n == 11, "shape_check takes 11 arguments");
+    Config c;
+    c.nd = axes(a[0]);
+    const Tensor input = as_tensor(a[1], "inputs"), weight = as_tensor(a[2], "weight"), offset = as_tensor(a[3], "offset");
+    std::vector<int64_t> sizes;
+    for (const auto& v : pybind11::reinterpret_borrow<pybind11::sequence>(a[4])) sizes.push_back(v.cast<int64_t>());
+    as_ints(a[5], c.nd, c.stride);
+    as_ints(a[6], c.nd, c.pad);
+    as_ints(a[7], c.nd, c.dil);
+    c.cpg = as_int(a[8]);
+    c.group = as_int(a[9]);
+    c.standard = PyObject_IsTrue(a[10]) == 1;
+    const at::IntArrayRef shape(sizes);
+    int64_t out[3];
+    shape_check(c, input, weight, offset, out, &shape);
+    Py_RETURN_NONE;
+    END_HANDLE_TH_ERRORS
+}
 // set_error(type): the exception class for calls that the library rejects
 PyObject* py_set_error(PyObject*, PyObject* type) {
     Py_INCREF(type);
@@ -615,6 +647,7 @@ PyMethodDef methods[] = {{"conv_offset", method(py_conv_offset<true>), METH_FAST
                          {"conv2d_forward", method(py_conv2d<false>), METH_FASTCALL, nullptr},
                          {"conv2d_backward", method(py_conv2d_backward), METH_FASTCALL, nullptr},
                          {"wants_function", py_wants_function, METH_O, nullptr},
+                         {"shape_check", method(py_shape_check), METH_FASTCALL, nullptr},
                          {"set_error", py_set_error, METH_O, nullptr},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module_def = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

@@ -29,11 +29,6 @@ from torch.autograd.function import once_differentiable
 from . import _lib
 
 
-def _check(cond, msg):
-    if not cond:
-        raise RuntimeError(msg)
-
-
 def output_size(in_sizes, kernel, stride, padding, dilation=None, standard=False):
     """The reference formula, dilation not included (deform3d/lib/deform_conv3d_cuda.cpp:15-17;
     deform_conv3d_function.py:26-27).  `standard=True` gives the usual dilation-aware size
@@ -47,35 +42,14 @@ def output_size(in_sizes, kernel, stride, padding, dilation=None, standard=False
     return tuple((i + 2 * p - k) // s + 1 for i, k, s, p in zip(in_sizes, kernel, stride, padding))
 
 
-_OUT_MSG = {3: ("error output ll", "error outhh", "error outww"), 2: ("error outhh", "error outww")}
-_OFF_MSG = {3: ("off l", "off h", "off w"), 2: ("off h", "off w")}
-
-
 def shape_check(nd, inputs, weight, offset, output_shape, channel_per_group, group, stride, padding,
                 dilation=None, standard=False):
-    """Python restatement of the reference's shape_check with its messages."""
-    _check(weight.dim() == nd + 2, "kernel dim")
-    _check(inputs.dim() == nd + 2, "input dim")
-    _check(inputs.size(1) == weight.size(1) * group, "input c != kernel c")
-    _check(len(output_shape) == nd + 2, "output dim")
-    _check(output_shape[0] == inputs.size(0), "output b != input b")
-    _check(output_shape[1] == weight.size(0), "ou c != ker c")
-    _check(offset.dim() == nd + 2, "off dim")
-    _check(offset.size(0) == inputs.size(0), "off batch")
-    kV = 1
-    for k in weight.shape[2:]:
-        kV *= k
-    _check(channel_per_group > 0 and inputs.size(1) % channel_per_group == 0, "off channel")
-    _check(offset.size(1) == inputs.size(1) // channel_per_group * nd * kV, "off channel")
-    for a in range(nd):
-        _check(offset.size(2 + a) == output_shape[2 + a], _OFF_MSG[nd][a])
-    want = output_size(inputs.shape[2:], weight.shape[2:], stride, padding, dilation, standard)
-    for a in range(nd):
-        _check(inputs.size(2 + a) + 2 * padding[a] - weight.size(2 + a) >= 0 and want[a] >= 1 and
-               want[a] == output_shape[2 + a], _OUT_MSG[nd][a])
-    _check(group > 0 and weight.size(0) % group == 0, "ou c != ker c")
+    """The reference's shape_check with its messages: the checks that every call of a layer goes through."""
+    _lib.native().shape_check(nd, inputs, weight, offset, output_shape, stride, padding, 1 if dilation is None else dilation,
+                              channel_per_group, group, standard)
 
 
+# Arguments and workspace of a C-ABI call, for callers of libdcn_amd.so itself.
 def _geom(nd, inputs, weight, out_sizes, stride, padding, dilation, channel_per_group, group):
     return ([inputs.size(0), inputs.size(1), weight.size(0)] + list(inputs.shape[2:]) + list(out_sizes) +
             list(weight.shape[2:]) + list(padding) + list(stride) + list(dilation) + [channel_per_group, group])

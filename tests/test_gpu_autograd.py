@@ -99,3 +99,19 @@ def test_an_undefined_gradient_is_zeros(name):
     _NoGradient.apply(fn.apply(*leaves, *cfg)).backward()
     for t in leaves:
         assert t.grad is not None and t.grad.shape == t.shape and not t.grad.any()
+
+
+def test_misshapen_grad_output_is_refused():
+    """backward called by hand: no kernel runs on a grad_output that is not the output's shape."""
+    import deform_conv3d_pytorch_op_amd as dcn
+    from deform_conv3d_pytorch_op_amd import _lib
+    for name in LAYERS:
+        fn, leaves, cfg, gout = _layer(name)
+        leaves = [t.detach() for t in leaves[:-1]]
+        for bad, msg in ((gout[:1, :, :-1], "output b|off|outhh|output ll"), (gout[:, :-1], "ou c != ker c"), (gout[..., :-1], "off w|outww"), (gout[0], "output dim")):
+            print("misshapen", name, tuple(bad.shape), flush=True)
+            with pytest.raises(RuntimeError, match=msg):
+                if fn is dcn.Conv2dFunction:
+                    _lib.native().conv2d_backward(*leaves, bad, *cfg, True, True, True)
+                else:
+                    _lib.native().conv_offset_backward(3 if name == "3d" else 2, *leaves, bad, *cfg, False, False, True, True, True)
