@@ -359,13 +359,11 @@ Geometry geo2(int batch, int input_c, int output_c, int input_h, int input_w, in
 
 // ---------------------------------------------------------------------------------------------
 // Scratch of the allocation-free entry point: the re-laid-out weight of one forward call.  A
-// file-scope device array, so every GPU the library runs on holds SCRATCH_BYTES of it
+// file-scope device array, so every GPU the library runs on holds NOALLOC_ARRAY_BYTES of it
 // until the process ends.  In host code the array's name is only a handle for
 // hipGetSymbolAddress: the device address is looked up once per device and kept, and host code
 // passes that address, never the name, to kernels.
-// (twice the accepted size of the float32 layout: the kernel's packed weights are half as large again)
-constexpr size_t SCRATCH_BYTES = 2 * (size_t)DCN_NOALLOC_SCRATCH_BYTES;
-static __device__ __align__(256) unsigned char scratch[SCRATCH_BYTES];
+static __device__ __align__(256) unsigned char scratch[NOALLOC_ARRAY_BYTES];
 
 std::mutex g_scratch_lock;
 void* g_scratch_ptr[MAX_DEVICES] = {};
@@ -470,21 +468,16 @@ int dcn3d_forward_noalloc_f32(const float* input, const float* weight, const flo
     const Geometry g = geo3(G3_ARGS);
     Params P;
     if (int rc = validate(g, P)) return rc;
-    // what forward() asks of a workspace: either weight layout must fit the fixed array
-    int MT, mchunks, Mp, Cgp;
-    fwd_weight_pad<float>(P.M, P.Cg, MT, mchunks, Mp, Cgp);
-    const int Mp8 = ((P.M + 31) / 32 + 7) / 8 * 8 * 32;
-    const size_t plain = (size_t)P.G * P.kV * (Mp > Mp8 ? Mp : Mp8) * Cgp * sizeof(float);
-    const size_t quad = ((size_t)chunk_slot<FQ>(P.cpg, P.Cg, P.C_in - 1) + 1) * forward_slab_elems<float>(P.kV, Mp8) * sizeof(float);
-    if (plain > DCN_NOALLOC_SCRATCH_BYTES || quad > DCN_NOALLOC_SCRATCH_BYTES) {
+    const size_t need = noalloc_weight_bytes(P);
+    if (need > DCN_NOALLOC_SCRATCH_BYTES) {
         char msg[200];
         snprintf(msg, sizeof msg, "layer too large for the allocation-free entry point: its re-laid-out weight takes %zu bytes, "
-                 "the fixed scratch holds %zu", plain > quad ? plain : quad, (size_t)DCN_NOALLOC_SCRATCH_BYTES);
+                 "the fixed scratch holds %zu", need, (size_t)DCN_NOALLOC_SCRATCH_BYTES);
         return fail(DCN_E_WORKSPACE, msg);
     }
     void* ws = nullptr;
     if (int rc = scratch_address(&ws)) return rc;
-    return forward<float, 3>(g, input, weight, offset, bias, output, ws, SCRATCH_BYTES,
+    return forward<float, 3>(g, input, weight, offset, bias, output, ws, NOALLOC_ARRAY_BYTES,
                              static_cast<hipStream_t>(stream));
 }
 

@@ -181,7 +181,9 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
         }
         if (small && !nw) return fail(DCN_E_LAUNCH, "no halo plan");      // (planned above)
         const size_t col_bytes = shared ? shared_column_bytes<typename std::conditional<MX, S, float>::type>() : 0;
-        const size_t wq_bytes = ((size_t)chunk_slot<CM>(P.cpg, P.Cg, P.C_in - 1) + 1) * slab_bytes(P.kV, P.Mp) + 256;      // (+: operands read from four elements further on)
+        size_t wq_bytes;
+        if constexpr (MX) wq_bytes = split_weight_bytes<S>(P, P.Mp);
+        else wq_bytes = ((size_t)chunk_slot<CM>(P.cpg, P.Cg, P.C_in - 1) + 1) * slab_bytes(P.kV, P.Mp) + 256;
         auto halo_lds = [=](const Params& Ph) { return col_bytes + (size_t)Ph.cchunk * Ph.hstride * (MX ? sizeof(S) : sizeof(T)) + (MX ? 0 : (size_t)Ph.hvol * 4); };
         if (nw == 16 || ws_bytes < align256(wq_bytes) + (size_t)fsplit * out_bytes) fsplit = 1;
         if (nw && ws_bytes >= wq_bytes) {

@@ -104,6 +104,24 @@ template <typename T> inline size_t forward_need(int N, int C_in, int C_out, siz
                                            : slab_bound((size_t)C_in, G, cpg, FQ) * forward_slab_elems<T>(kV, Mp8) * sizeof(T);
     return (fwd_plain > fwd_quad ? fwd_plain : fwd_quad) + forward_partial_bound(N, C_out, outV, sizeof(T)) + 1024;
 }
+// The allocation-free entry point accepts a layer by the size of its weight re-laid out as float32 (the larger of
+// [g][tap][c][m] and one slab per four channels).  What the halo kernels then store is three bfloat16 parts per
+// weight in slabs of eight channels: half as much again, and three times as much where the deformable groups have
+// four channels, each of which takes a slab.  The array holds that for every layer accepted (behind it 256 bytes
+// that operands of half a group are read past the end, and the block of the plan word).
+constexpr size_t NOALLOC_ARRAY_BYTES = 3 * (size_t)DCN_NOALLOC_SCRATCH_BYTES + 4096;
+inline size_t noalloc_weight_bytes(const Params& P) {
+    int MT, mchunks, Mp, Cgp;
+    fwd_weight_pad<float>(P.M, P.Cg, MT, mchunks, Mp, Cgp);
+    const int Mp8 = ((P.M + 31) / 32 + 7) / 8 * 8 * 32;
+    const size_t plain = (size_t)P.G * P.kV * (Mp > Mp8 ? Mp : Mp8) * Cgp * sizeof(float);
+    const size_t quad = ((size_t)chunk_slot<FQ>(P.cpg, P.Cg, P.C_in - 1) + 1) * forward_slab_elems<float>(P.kV, Mp8) * sizeof(float);
+    return plain > quad ? plain : quad;
+}
+// Bytes of the halo kernels' packed weights (float32: three parts, 16-bit storage: one).
+template <typename S> inline size_t split_weight_bytes(const Params& P, int Mp) {
+    return ((size_t)chunk_slot<FG>(P.cpg, P.Cg, P.C_in - 1) + 1) * split_slab_elems<S>(P.kV, Mp) * 2 + 256;      // (+: operands read from four elements further on)
+}
 template <typename T> inline size_t backward_data_need(int N, int C_in, int C_out, size_t inV, int kV, int G, int cpg = 0) {
     return bwd_data_weight_bytes<T>(C_out / G, C_in / G, kV, G, cpg) + 2 * align256((size_t)N * C_in * inV * sizeof(T)) + BWD_TAIL + 512;
 }

@@ -111,7 +111,7 @@ int dcn3d_backward_input_offset_f64(const double *input, const double *weight, c
  * dcn3d_forward_f32 without the workspace pair; the re-laid-out weight (and, for a layer of few
  * positions, as many partial outputs as still fit; in the last 256 bytes the halo size chosen for
  * the call) goes into a fixed device array
- * of twice DCN_NOALLOC_SCRATCH_BYTES inside the library, which every GPU the library runs on holds until
+ * of three times DCN_NOALLOC_SCRATCH_BYTES (and 4 KB) inside the library, which every GPU the library runs on holds until
  * the process ends.  A layer whose weight, re-laid out as float32, is larger than
  * DCN_NOALLOC_SCRATCH_BYTES (roughly: 4 * kernel volume * output_c rounded up to 256 * (input_c / group + 4) bytes) is rejected with DCN_E_WORKSPACE.  All
  * calls on one GPU share that array: calls that overlap there (two streams, two threads) race on it

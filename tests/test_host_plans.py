@@ -1,0 +1,22 @@
+"""Rules of the library's host side over random layers: host_plans.hip compiled for the CPU alone."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="module")
+def probe(tmp_path_factory):
+    exe = str(tmp_path_factory.mktemp("plans") / "host_plans")
+    r = subprocess.run([os.environ.get("HIPCC", "/opt/rocm/bin/hipcc"), "--offload-host-only", "-std=c++17", "-O1", "-w",
+                        os.path.join(HERE, "host_plans.hip"), "-o", exe], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    assert r.returncode == 0, r.stdout
+    return exe
+
+
+@pytest.mark.parametrize("what", ["noalloc", "native16"])
+def test_rule(probe, what):
+    r = subprocess.run([probe, what, "7", "20000"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
