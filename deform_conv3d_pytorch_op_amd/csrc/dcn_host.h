@@ -523,6 +523,7 @@ int backward_weight_run(const WeightCall<T, S>& c, const S* off, T* gw, T* gb, b
 
 template <typename T, typename S>
 inline int launch_prepare(const Params& P, const PlanChoice& pc, const Prep& prep, const S* w, const S* off, size_t n_off, hipStream_t s) {
+    if (prep.full) return fail(DCN_E_LAUNCH, "too many jobs for the preparing launch");
     if (prep.jobs.n == 0) return DCN_OK;
     hipLaunchKernelGGL((backward_prepare_kernel<T, S>), dim3(prep.blocks), dim3(256), 0, s, P, pc, prep.jobs, w, off, n_off);
     return check_launch("backward_prepare_kernel");

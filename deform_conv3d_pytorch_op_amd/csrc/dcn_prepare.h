@@ -158,8 +158,13 @@ __global__ __launch_bounds__(256) void backward_prepare_kernel(Params P, PlanCho
 struct Prep {
     PrepJobs jobs;
     unsigned blocks = 0;
+    bool full = false;                          // a job too many was added: launch_prepare then refuses
     Prep() { jobs.n = 0; }
     PrepJob& add(int kind, unsigned nblocks) {
+        if (jobs.n == MAX_PREP) {
+            full = true;
+            return spare;
+        }
         PrepJob& j = jobs.job[jobs.n++];
         j = PrepJob{kind, 0, blocks, nullptr, nullptr, nullptr, 0, 0, 0, 0};
         blocks += nblocks;
@@ -175,6 +180,9 @@ struct Prep {
         PrepJob& j = add(PREP_LAST, last_strips(V) * (((unsigned)C + 31) / 32) * (unsigned)N);
         j.src = src; j.dst = dst; j.C = C; j.V = V; j.N = N; j.sums = sums;
     }
+
+private:
+    PrepJob spare;
 };
 
 }  // namespace dcn

@@ -51,6 +51,13 @@ int main(int argc, char** argv) {
     if (argc != 4) return 2;
     const std::string what = argv[1];
     rng.seed((unsigned)atoi(argv[2]));
+    if (what == "jobs") {           // the list of the preparing launch takes no job too many and says so
+        Prep prep;
+        for (int i = 0; i < MAX_PREP; ++i) prep.add(PREP_PLAN, 1);
+        const bool ok = !prep.full && prep.jobs.n == MAX_PREP && prep.blocks == (unsigned)MAX_PREP;
+        prep.add(PREP_PLAN, 1);
+        return ok && prep.full && prep.jobs.n == MAX_PREP ? 0 : 1;
+    }
     int layers = 0, hits = 0;
     for (const int count = atoi(argv[3]); layers < count;) {
         Params P;
