@@ -265,8 +265,9 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                 if (l > lds) lds = l;
             }
             const Params& Ph = plans[0];
-            using Kern = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const WE*, const S*, S*, T*, int, unsigned, TailSplit);
-            Kern kern = nullptr;
+            using KernMx = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const WE*, const S*, const S*, S*, T*, int, unsigned, TailSplit);
+            using KernQuad = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const WE*, const S*, S*, T*, int, unsigned, TailSplit);
+            typename std::conditional<MX, KernMx, KernQuad>::type kern = nullptr;
             if constexpr (MX) {
                 if (pairs) kern = MT == 1 ? forward_split_kernel<ND, 1, 16, 2, S> : forward_split_kernel<ND, 2, 16, 2, S>;
                 else if (small) kern = MT == 1 ? forward_split_kernel<ND, 1, 8, 4, S> : MT == 2 ? forward_split_kernel<ND, 2, 8, 4, S> : forward_split_kernel<ND, 4, 8, 4, S>;
@@ -361,9 +362,11 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                             plans[k].hext[0], plans[k].hext[1], plans[k].hext[2], plans[k].cchunk, pc.base[k]);
             }
             const unsigned* sel = pc.sel;
-            if (int rc = launch_halo(kern, "forward halo kernel", grid, (pairs ? 16 : shared || small ? 8 : nw) * 64, lds, s, Ph, alts, sel, in, off, (const WE*)ws, bias, out, part,
-                                     tsplit > 1 ? tsplit : fsplit, (unsigned)whole, ts))
-                return rc;
+            const int threads = (pairs ? 16 : shared || small ? 8 : nw) * 64, splits = tsplit > 1 ? tsplit : fsplit;
+            int rc;
+            if constexpr (MX) rc = launch_halo(kern, "forward halo kernel", grid, threads, lds, s, Ph, alts, sel, in, off, (const WE*)ws, w, bias, out, part, splits, (unsigned)whole, ts);
+            else rc = launch_halo(kern, "forward halo kernel", grid, threads, lds, s, Ph, alts, sel, in, off, (const WE*)ws, bias, out, part, splits, (unsigned)whole, ts);
+            if (rc) return rc;
             if (fsplit == 1 && tsplit == 1) return DCN_OK;
             if (tsplit > 1) {
                 using Join = void (*)(Params, PlanSet, const unsigned*, const T*, const S*, S*, int, unsigned, TailSplit);

@@ -27,9 +27,9 @@ template <typename S> __host__ __device__ inline constexpr size_t shared_column_
 template <int ND, int RT, typename S>
 __global__ __launch_bounds__(SHARED_WAVES * 64, 2) void forward_shared_kernel(Params P, PlanSet alts, const unsigned* __restrict__ sel,
                                                            const S* __restrict__ in, const S* __restrict__ off,
-                                                           const typename Parts<S>::Elem* __restrict__ Wq, const S* __restrict__ bias,
-                                                           S* __restrict__ out, float* __restrict__ part, int csplit, unsigned whole,
-                                                           TailSplit ts) {
+                                                           const typename Parts<S>::Elem* __restrict__ Wq, const S* __restrict__ W,
+                                                           const S* __restrict__ bias, S* __restrict__ out, float* __restrict__ part, int csplit,
+                                                           unsigned whole, TailSplit ts) {
     HaloPlan H;
     if (!chosen_halo(P, alts, sel, H)) return;          // another launch runs the chosen plan
     using PT = Parts<S>;
@@ -102,7 +102,7 @@ __global__ __launch_bounds__(SHARED_WAVES * 64, 2) void forward_shared_kernel(Pa
                             for (int k = 0; k < NP; ++k) a8[ks][r][k] = *reinterpret_cast<const Vec*>(wp + (r * NP + k) * 1024 + a_lane);
                     }
                 };
-                load_a(0, 0);
+                if constexpr (!(exact && sizeof(S) == 4)) load_a(0, 0);
                 __syncthreads();
                 const bool rim_far = exact && sNonFinite != 0;                 // uniform, see forward_split_kernel
                 int k0[ND];                            // kernel coordinates of the next tap pair
@@ -142,7 +142,7 @@ __global__ __launch_bounds__(SHARED_WAVES * 64, 2) void forward_shared_kernel(Pa
                     }
                 };
                 // this wavefront's row tiles times its column tiles of buffer b
-                auto consume = [&](int gp, int b) {
+                auto consume = [&](int tgi, int gp, int b) {
                     const bool two = 2 * gp + 1 < ngrp;                        // uniform
                     if constexpr (exact) {
 #pragma unroll
@@ -154,7 +154,8 @@ __global__ __launch_bounds__(SHARED_WAVES * 64, 2) void forward_shared_kernel(Pa
                                     float val[FG];
 #pragma unroll
                                     for (int e = 0; e < FG; ++e) val[e] = src[e];
-                                    mma_exact<S, RW>(a8[ks], val, true, nch - (2 * gp + ks) * FG, acc + c * RW);
+                                    mma_exact<S, RW>(P, W, g, (mchunk * RT + rw * RW) * TN + j, tgi * 2 + q, (size_t)(cc0 - cg0 + (2 * gp + ks) * FG), a8[ks], val, true,
+                                                     nch - (2 * gp + ks) * FG, acc + c * RW);
                                 }
                     } else {
                         // all columns of the phase are requested before the first matrix instruction
@@ -182,14 +183,14 @@ __global__ __launch_bounds__(SHARED_WAVES * 64, 2) void forward_shared_kernel(Pa
                     const int gn = gp + 1 < npair ? gp + 1 : 0, tn = gn ? tgi : tgi + 1;
                     const bool more = tn < ntg;                                // uniform
                     if constexpr (exact) {
-                        consume(gp, 0);
+                        consume(tgi, gp, 0);
                         if (!more) break;
-                        load_a(tn, gn);
+                        if constexpr (sizeof(S) == 2) load_a(tn, gn);
                         __syncthreads();
                         produce(tn, gn, 0);
                     } else {
                         if (more && half == 0) produce(tn, gn, b ^ 1);
-                        consume(gp, b);
+                        consume(tgi, gp, b);
                         if (!more) break;
                         load_a(tn, gn);
                         if (half != 0) produce(tn, gn, b ^ 1);
@@ -210,7 +211,7 @@ __global__ __launch_bounds__(SHARED_WAVES * 64, 2) void forward_shared_kernel(Pa
     for (int c = 0; c < CW; ++c) {
         int o[ND];
         ok[c] = tile_position<ND>(P, tg, (cwv * CW + c) * TN + j, o, opos[c]);
-        if (ok[c] && !all_finite<RW>(acc + c * RW)) sRedo = 1;
+        if (ok[c] && !results_stand<RW, S>(acc + c * RW)) sRedo = 1;
     }
     __syncthreads();
     if (__builtin_expect(sRedo, 0)) work(std::true_type{});

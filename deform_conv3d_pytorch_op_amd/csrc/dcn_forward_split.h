@@ -15,9 +15,14 @@
 // than from v_mfma_f32_32x32x2_f32, which rounds after every second product where this rounds
 // after every sixteenth.  Six instructions reduce over 16 slots in 93 ns per SIMD where the float32 ones
 // take 239 ns, and unlike those they run next to vector instructions.
-// Non-finite operands have no such parts (inf - inf): a workgroup whose result is not finite
-// everywhere works its block out once more through the float32 instructions, which also gives an
-// overflow of the parts the float32 meaning.
+// Operands without such parts: a workgroup works its block out once more through the float32
+// instructions, on the weights as they are, when a result
+//   - is not finite (inf - inf in the parts; this also gives an overflow of the parts the float32 meaning), or
+//   - lies below 2^-80 without being zero.  The third part of a value below 2^-110 is subnormal and loses bits,
+//     up to 2^-134 per value: more than float32 sums round away only where a result is below 2^-110 times
+//     the sum of the other operand's magnitudes.  With sums of up to 2^30 that never goes unnoticed (x around
+//     2^-116, weights around 2^10: 3.6e-6 from float64 without the second look, 4e-7 with it).
+//     Samples below 2^-133 (float32 subnormals) count as zero where the result is not looked at again.
 //
 // Lane roles.  A wavefront owns 32 output positions; lane (j, q) works on position j and supplies
 // eight of the 16 reduction slots of an instruction: eight channels of tap tg*2 + q.  Every lane derives
@@ -57,11 +62,12 @@ template <> struct Parts<float> {
 #pragma unroll
         for (int k = 0; k < NP; ++k) p[k] = __builtin_bit_cast(Vec, out[k]);
     }
-    static __device__ inline float join(const Vec p[NP], int e) { return ((float)p[2][e] + (float)p[1][e]) + (float)p[0][e]; }
     // parts of one value for the packed weights; infinities and NaN stay in the first part, and so that
     // a value near the largest float does not round to infinity its first part is then cut off instead
+    // nor does a nonzero weight round to zero: results made of it are too small not to be looked at again
     static __device__ inline void split1(float v, __bf16 p[NP]) {
         p[0] = (__bf16)v;
+        if (v != 0.f && (float)p[0] == 0.f) p[0] = (__bf16)copysignf(0x1p-133f, v);
         if (!(fabsf((float)p[0]) <= std::numeric_limits<float>::max())) {
             if (!(fabsf(v) <= std::numeric_limits<float>::max())) { p[1] = p[2] = (__bf16)0.f; return; }
             p[0] = (__bf16)__uint_as_float(__float_as_uint(v) & 0xffff0000u);
@@ -80,7 +86,6 @@ template <> struct Parts<Bf16> {
 #pragma unroll
         for (int e = 0; e < 8; ++e) p[0][e] = (__bf16)v[e];            // round to nearest even
     }
-    static __device__ inline float join(const Vec p[NP], int e) { return (float)p[0][e]; }
     static __device__ inline void split1(Bf16 v, __bf16 p[NP]) { p[0] = __builtin_bit_cast(__bf16, v.bits); }
     static __device__ inline Mma<float>::Acc mma(Vec a, Vec b, Mma<float>::Acc c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
 };
@@ -92,7 +97,6 @@ template <> struct Parts<Fp16> {
 #pragma unroll
         for (int e = 0; e < 8; ++e) p[0][e] = (_Float16)v[e];
     }
-    static __device__ inline float join(const Vec p[NP], int e) { return (float)p[0][e]; }
     static __device__ inline void split1(Fp16 v, _Float16 p[NP]) { p[0] = v.v; }
     static __device__ inline Mma<float>::Acc mma(Vec a, Vec b, Mma<float>::Acc c) { return __builtin_amdgcn_mfma_f32_32x32x16_f16(a, b, c, 0, 0, 0); }
 };
@@ -117,6 +121,11 @@ __device__ inline void mma_parts(const typename Parts<S>::Vec a[MT][Parts<S>::NP
 template <typename S>
 __host__ __device__ inline size_t split_slab_elems(int kV, int Mp) {
     return (size_t)((kV + 1) / 2) * Mp * 2 * FG * Parts<S>::NP;
+}
+
+// weight of output channel m and input channel cl of group g
+template <typename S> __device__ inline S weight_at(const Params& P, const S* __restrict__ W, int g, int m, size_t cl, int tap) {
+    return P.transposed ? W[(((size_t)g * P.Cg + cl) * P.M + m) * P.kV + (P.kV - 1 - tap)] : W[(((size_t)g * P.M + m) * P.Cg + cl) * P.kV + tap];
 }
 
 // One thread per operand of a lane.  With pc.sel set the launch has one block more, which chooses the
@@ -147,10 +156,7 @@ __global__ __launch_bounds__(256) void pack_split_weight_kernel(Params P, const 
 #pragma unroll
         for (int e = 0; e < FG; ++e) {
             S v = S();
-            if (m < P.M && tap < P.kV && c0 + e < seg_e) {
-                const size_t cl = (size_t)(c0 + e - g * P.Cg);
-                v = P.transposed ? W[(((size_t)g * P.Cg + cl) * P.M + m) * P.kV + (P.kV - 1 - tap)] : W[(((size_t)g * P.M + m) * P.Cg + cl) * P.kV + tap];
-            }
+            if (m < P.M && tap < P.kV && c0 + e < seg_e) v = weight_at<S>(P, W, g, m, (size_t)(c0 + e - g * P.Cg), tap);
             typename PT::Elem p[NP];
             PT::split1(v, p);
 #pragma unroll
@@ -443,9 +449,12 @@ __device__ inline void load_pair_offsets(const Params& P, const S* __restrict__ 
 }
 
 // The contraction of a lane's values on the float32 instructions, one channel of the tap pair at a
-// time (results that are not finite).  nvalid: how many of the values exist.
+// time (results that need a second look).  The weights: in float32 the tensor's own, whose parts may not add
+// up to them -- the lane's rows are m0, m0 + 32, ..., its tap is `tap`, its channels cl .. cl + nvalid - 1 of group
+// g --, in 16-bit storage the packed ones in `a`.
 template <typename S, int MT>
-__device__ inline void mma_exact(const typename Parts<S>::Vec a[MT][Parts<S>::NP], const float val[FG], bool live, int nvalid, Mma<float>::Acc acc[MT]) {
+__device__ inline void mma_exact(const Params& P, const S* __restrict__ W, int g, int m0, int tap, size_t cl, const typename Parts<S>::Vec a[MT][Parts<S>::NP],
+                                 const float val[FG], bool live, int nvalid, Mma<float>::Acc acc[MT]) {
 #pragma unroll 1
     for (int e = 0; e < FG; ++e) {
         float b = 0.f;
@@ -455,22 +464,32 @@ __device__ inline void mma_exact(const typename Parts<S>::Vec a[MT][Parts<S>::NP
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) {
             float w = 0.f;
+            if constexpr (sizeof(S) == 4) {
+                const int m = m0 + mt * Mma<float>::TN;
+                if (e < nvalid && tap < P.kV && m < P.M) w = weight_at<S>(P, W, g, m, cl + e, tap);
+            } else {
 #pragma unroll
-            for (int x = 0; x < FG; ++x) w = x == e && e < nvalid ? Parts<S>::join(a[mt], x) : w;
+                for (int x = 0; x < FG; ++x) w = x == e && e < nvalid ? (float)a[mt][0][x] : w;
+            }
             acc[mt] = Mma<float>::mma(w, b, acc[mt]);
         }
     }
 }
 
-// NaN or infinite when a result of the lane is (or when the sum overflows: its workgroup then repeats in vain)
-template <int NT>
-__device__ inline bool all_finite(const Mma<float>::Acc* acc) {
+// Whether the lane's results are what they should be: finite (also false when their sum overflows: the workgroup
+// then repeats in vain) and, in float32, zero or not too small (see the top of the file).
+template <int NT, typename S>
+__device__ inline bool results_stand(const Mma<float>::Acc* acc) {
     float s = 0.f;
+    unsigned least = ~0u;                               // bits of the least magnitude that is not zero, less one
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
-        for (int r = 0; r < Mma<float>::NACC; ++r) s += fabsf(acc[t][r]);
-    return s <= std::numeric_limits<float>::max();
+        for (int r = 0; r < Mma<float>::NACC; ++r) {
+            s += fabsf(acc[t][r]);
+            if constexpr (sizeof(S) == 4) least = min(least, __float_as_uint(fabsf(acc[t][r])) - 1u);
+        }
+    return s <= std::numeric_limits<float>::max() && least >= __float_as_uint(0x1p-80f) - 1u;
 }
 
 // Writes a 32 x 32 result tile: row m0 + r of group g's output channels (m0 uniform), this lane's position.
@@ -506,9 +525,9 @@ __device__ inline void store_tile(const Params& P, O* __restrict__ dst, const S*
 template <int ND, int MT, int NW, int TS, typename S>
 __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel(Params P, PlanSet alts, const unsigned* __restrict__ sel,
                                                            const S* __restrict__ in, const S* __restrict__ off,
-                                                           const typename Parts<S>::Elem* __restrict__ Wq, const S* __restrict__ bias,
-                                                           S* __restrict__ out, float* __restrict__ part, int csplit, unsigned whole,
-                                                           TailSplit ts) {
+                                                           const typename Parts<S>::Elem* __restrict__ Wq, const S* __restrict__ W,
+                                                           const S* __restrict__ bias, S* __restrict__ out, float* __restrict__ part, int csplit,
+                                                           unsigned whole, TailSplit ts) {
     HaloPlan H;
     if (!chosen_halo(P, alts, sel, H)) return;          // another launch runs the chosen plan
     using PT = Parts<S>;
@@ -611,16 +630,16 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
                                 for (int k = 0; k < NP; ++k) __builtin_memcpy(&a8[mt][k], reinterpret_cast<const char*>(wp) + (mt * NP + k) * 1024 + a_lane, 16);
                             __builtin_amdgcn_sched_barrier(0);      // all of them on their way while the operand is made
                         };
-                        if constexpr (EARLY) load_a();
+                        if constexpr (EARLY && !(exact && sizeof(S) == 4)) load_a();
                         group_sum8<ND, S>(sIn, t.base, grp, nch, H.hstride, row, plane, t.cw, val);
                         if (__builtin_expect(any_far, 0)) far_values<ND, S>(P, t, chan0, grp * FG, nch, val);
-                        if constexpr (!EARLY) load_a();
+                        if constexpr (!EARLY && !(exact && sizeof(S) == 4)) load_a();
                         if constexpr (!exact) {
                             Vec b8[NP];
                             PT::split(val, b8);
                             mma_parts<S, MT>(a8, b8, acc);
                         } else
-                            mma_exact<S, MT>(a8, val, t.near || t.far, nch - grp * FG, acc);
+                            mma_exact<S, MT>(P, W, g, mchunk * MT * TN + j, tgi * 2 + q, (size_t)(cc0 - cg0 + grp * FG), a8, val, t.near || t.far, nch - grp * FG, acc);
                         wp += (size_t)per_slab * FG;
                     }
                     next_tap<ND>(P, k1);
@@ -631,7 +650,7 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
         }
     };
     work(std::false_type{});
-    if (valid && !all_finite<MT>(acc)) sRedo = 1;
+    if (valid && !results_stand<MT, S>(acc)) sRedo = 1;
     __syncthreads();
     if (__builtin_expect(sRedo, 0)) work(std::true_type{});
     if constexpr (TS > 1) {
