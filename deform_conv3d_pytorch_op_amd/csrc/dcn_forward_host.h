@@ -68,10 +68,13 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
     // that gives no more than two workgroups per CU.
     bool small = false;
     // (a single tap leaves too few steps to share in 3-D: the halo of 64 positions costs more to stage than it saves)
-    if (MX && shared) {       // ... unless it fills half of the device, with the input channels split
+    // Shared columns only where they can fill half of the device: with a workgroup for every 16 input channels in
+    // float32, whose channels can be split, and without in 16-bit storage, whose cannot (256 -> 256 channels, 3x3, 2 x 28 x 28
+    // positions in bfloat16: 16 units, 105 us shared and 60 with several wavefronts to a position).
+    if (MX && shared) {
         Params Pt = P;
         if (plan_halo<T, ND>(Pt, MAX_LDS, default_margin(), 1 << 30, sizeof(S), SHARED_COLS, false, FG, nullptr, 1, false) &&
-            (long long)Pt.N * Pt.tiles * P.G * P.mchunks * (P.Cg >= 32 ? P.Cg / 16 : 1) * 2 < cu_count())
+            (long long)Pt.N * Pt.tiles * P.G * P.mchunks * (!S16 && P.Cg >= 32 ? P.Cg / 16 : 1) * 2 < cu_count())
             shared = false;
     }
     if (MX && !shared && (ND == 2 || P.kV > 1) && forward_small() && forward_slots() == 0) {

@@ -1,5 +1,6 @@
 """16-bit storage at the edges of what the 16-bit kernels serve themselves: layers whose halo just fits a block
-of 256 positions and layers past that, which run the float32 operator on widened tensors, and values that are not finite."""
+of 256 positions or whose positions are too few to share their columns, layers past that halo, which run the float32
+operator on widened tensors, and values that are not finite."""
 import pytest
 import torch
 
@@ -15,7 +16,8 @@ ROUNDING = {torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}
 
 # (nd, N, C_in, C_out, ins, k, stride, pad, dil, cpg, groups, reach)
 FITS = [(3, 1, 16, 24, (9, 21, 22), 3, 2, 1, 1, 8, 1, 1.5), (3, 2, 12, 40, (6, 17, 18), 3, 1, 3, 3, 12, 1, 1.5), (3, 1, 8, 16, (5, 19, 20), 3, (1, 2, 2), 2, 2, 8, 1, 1.5),
-        (2, 1, 24, 72, (70, 62), 5, 3, 6, 3, 24, 1, 2.0), (2, 2, 16, 130, (30, 33), 3, 2, 2, 2, 16, 2, 2.0)]
+        (2, 1, 24, 72, (70, 62), 5, 3, 6, 3, 24, 1, 2.0), (2, 1, 256, 96, (30, 27), 3, 1, 1, 1, 64, 1, 1.5), (2, 1, 48, 264, (21, 90), 3, 1, 1, 1, 48, 1, 2.0),
+        (2, 2, 16, 130, (30, 33), 3, 2, 2, 2, 16, 2, 2.0)]
 PAST = [(3, 1, 16, 32, (20, 30, 30), 3, 2, 2, 2, 16, 1, 1.5), (3, 1, 24, 72, (9, 16, 17), 3, 1, 4, 4, 12, 1, 1.5),
         (2, 1, 16, 48, (60, 50), 5, 4, 8, 4, 16, 1, 2.0), (2, 1, 32, 96, (60, 60), 5, 4, 8, 4, 32, 1, 2.0)]
 
@@ -33,7 +35,7 @@ def _id(s):
 
 @pytest.mark.parametrize("dtype", DTYPES.values(), ids=DTYPES)
 @pytest.mark.parametrize("spec", FITS, ids=_id)
-def test_strides_and_dilation_that_fit(spec, dtype):
+def test_layers_that_fit(spec, dtype):
     print("fits", spec, dtype, flush=True)
     _compare(make_case(*spec, dtype=dtype, seed=41), dtype, "fits")
 
