@@ -213,17 +213,25 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             pc.nd = ND;
             pc.margin[0] = margins[0];
             pc.base[0] = 1.f;
-            // a wavefront with a sample beyond the halo walks every channel of the pass once more, and each
-            // such sample gathers its corners from global memory (fitted to timings at c4 and c3)
-            pc.far_wave = ND == 3 ? 0.5f : 0.1f;
-            pc.far_sample = ND == 3 ? 2.2f : 5.f;
+            // How the time grows with the halo, and what samples beyond it cost, in times of a launch without any
+            // (PlanChoice).  forward_split_kernel and forward_shared_kernel, offsets U[-r, r], us per margin (64 -> 64 channels,
+            // 3x3x3, 4 x 16 x 28 x 28 positions; 256 -> 256, 3x3, 8 x 56 x 56):
+            //   3-D, margins 2 / 3 / 4   r = 2: 161 / 169 / 177   r = 2.5: 376 / 169 / 177   r = 5: 688 / 543 / 378   r = 8: 924 / 808 / 683
+            //   2-D, margins 2 / 4 / 6   r = 2: 238 / 250 / 262   r = 2.5: 336 / 250 / 262   r = 5: 380 / 349 / 262   r = 8: 430 / 408 / 374
+            // A pass of four channels (3-D, where the wider halo holds no eight) leaves half of the reduction slots empty: 1.55
+            // times the time.  float64: forward_quad_kernel walks the channels of a wavefront with such a sample once more.
+            const float grow = MX ? (ND == 3 ? 0.1f : 0.12f) : ND == 3 ? 0.3f : 0.12f;
+            pc.far_wave = MX ? (ND == 3 ? 0.6f : 0.4f) : ND == 3 ? 0.5f : 0.1f;
+            pc.far_sample = MX ? (ND == 3 ? 1.3f : 0.4f) : ND == 3 ? 2.2f : 5.f;
+            pc.far_steep = MX ? (ND == 3 ? 2.5f : 0.4f) : 0.f;
             const size_t used = align256(wq_bytes) + (fsplit > 1 ? (size_t)fsplit * out_bytes : 0);
             if (nmargins > 1 && ws_bytes >= used + 512) {
                 // (within the LDS of the first plan, which fixes how many workgroups share a CU; all of it
                 // when the grid gives a CU one workgroup at most)
                 const long long wgs = (long long)plans[0].N * plans[0].tiles * plans[0].G * plans[0].mchunks * fsplit;
                 size_t lds0 = halo_lds(plans[0]);
-                if ((wgs <= cu_count() || shared) && lds0 < MAX_LDS) lds0 = MAX_LDS;
+                // (... or its registers allow no more: 16 wavefronts of up to 128)
+                if ((wgs <= cu_count() || shared || (MX && nw == 16)) && lds0 < MAX_LDS) lds0 = MAX_LDS;
                 if (small && wgs > cu_count() && lds0 < MAX_LDS / 2) lds0 = MAX_LDS / 2;
                 for (int k = 1; k < nmargins; ++k) {
                     Params& Pk = plans[pc.nplans];
@@ -233,8 +241,8 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                     if (!same_blocks(Pk, plans[0]) || Pk.hvol > 3 * plans[0].hvol) continue;
                     if (fsplit > 1) even_passes(Pk);
                     pc.margin[pc.nplans] = margins[k];
-                    // staging and the per-pass geometry grow with the halo: about a third of the kernel's time in 3-D, an eighth in 2-D
-                    pc.base[pc.nplans] = 1.f + (ND == 3 ? 0.3f : 0.12f) * ((float)Pk.hvol / (float)plans[0].hvol - 1.f);
+                    pc.base[pc.nplans] = 1.f + grow * ((float)Pk.hvol / (float)plans[0].hvol - 1.f);
+                    if (MX && Pk.cchunk % FG && plans[0].cchunk % FG == 0) pc.base[pc.nplans] *= 1.55f;
                     ++pc.nplans;
                 }
                 if (pc.nplans > 1) pc.sel = reinterpret_cast<unsigned*>(static_cast<char*>(ws) + (ws_bytes - 256) / 256 * 256);
