@@ -212,7 +212,7 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
         pc.margin[0] = margins[0];
         pc.base[0] = 1.f;
         pc.far_sample = ND == 3 ? 4.5f : 1.f;       // a sample beyond the halo scatters with global atomics
-        pc.far_steep = ND == 3 ? 25.f : 0.f;        // (c4, margin 2: 3.0, 4.1, 10.4, 26.6 times the time at 49, 70, 87.5, 96 % of the samples beyond the halo)
+        pc.far_steep = ND == 3 ? 25.f : 0.f;        // (64 -> 64 channels, 4 x 16 x 56 x 56, margin 2: 3.0, 4.1, 10.4, 26.6 times the time at 49, 70, 87.5, 96 % of the samples beyond the halo)
         // 3-D: when most samples leave even the widest halo, the path without LDS tiling (coalesced
         // atomics on a channels-last copy; about 6.5 times the fused kernel's time on small offsets,
         // whatever the offsets) is the cheaper one: offered as a fourth choice, its kernels launched

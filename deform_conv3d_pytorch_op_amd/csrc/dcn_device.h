@@ -32,7 +32,7 @@ struct Params {
     int hstride;                  // LDS elements between the planes of two channels (>= hvol)
     int cchunk;                   // channels staged per pass
     int oob_zero;                 // 3-D backward: 1 = no grad_offset term for out-of-range samples
-    int transposed;               // forward: the weight is [C_in][C_out / G][taps in reverse] (see conv2d_backward_input)
+    int transposed;               // forward: the weight is [C_in][C_out / G][taps in reverse] (see conv2d_layer_backward)
 };
 
 // Halo margin chosen on the device.  How far the LDS halo of a position block must reach depends on

@@ -386,7 +386,7 @@ __global__ __launch_bounds__(NW * 64, 1) void forward_quad_kernel(Params P, Plan
         }
 }
 
-// Joins the partial sums of the units that forward_quad_kernel split in its last round: one
+// Joins the partial sums of the units that a forward halo kernel split in its last round: one
 // workgroup of NW * TN threads per unit and slice of JOIN_ROWS output channels, thread = position of
 // the block; out = bias + the csplit partial sums, added in the order of cz.
 constexpr int JOIN_ROWS = 8;
@@ -431,7 +431,7 @@ __global__ __launch_bounds__(NW * 64) void forward_join_tail_kernel(Params P, Pl
     }
 }
 
-// out = bias + the sum of `parts` partial outputs of forward_quad_kernel, added in the order of the
+// out = bias + the sum of `parts` partial outputs of a forward halo kernel, added in the order of the
 // parts (the result does not depend on which workgroup finished first).
 template <typename T>
 __global__ void forward_join_partials_kernel(const T* __restrict__ part, const T* __restrict__ bias, T* __restrict__ out,

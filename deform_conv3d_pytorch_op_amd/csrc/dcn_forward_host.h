@@ -54,20 +54,29 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
     // Then fewer row tiles per wavefront: more output-channel chunks, each sampling for itself.
     int fsplit = 1;
     const int mtiles_all = (P.M + TN - 1) / TN;
-    // More than 64 output channels, 2-D (in 3-D a block of 128 positions stages twice the halo per position:
-    // 1.27 against 0.97 ms for 128 -> 128 channels at stride 2): forward_shared_kernel, units of 128 positions and MT = 4 or 8 row tiles.
-    // Per 16 reduction slots and 32 positions a row tile costs its matrix instructions and every chunk of
-    // row tiles samples for itself: the cheaper of the two.
+    // Which shape of the float32 / 16-bit kernels; times in us, float32 and 3x3 unless said otherwise.
+    // Shared columns (forward_shared_kernel; units of 128 positions, MT = 4 or 8 row tiles): more than 64 output channels,
+    // 2-D.  256 -> 256 channels, 8 x 56 x 56 positions: 239, and 277 where every wavefront samples for itself; 64 -> 512: 138 / 157;
+    // in bfloat16 115 / 126 and 71 / 74.  3-D layers are not offered it: a block of 128 positions stages twice the halo
+    // per position, 128 -> 128 channels at stride (1, 2, 2), 2 x 16 x 56 x 56 positions, 981 us and 1265 with shared columns (more output
+    // channels or stride 1 would gain: -> 256 1807 / 1684, 64 -> 128 at stride 1, 2 x 16 x 28 x 28, 144 / 130).
+    // Per 16 reduction slots and 32 positions a row tile costs its matrix instructions, and every chunk of row tiles
+    // samples for itself (10 of the same unit): the cheaper of 4 and 8.  160 to 256 output channels, 8 samples: 238 with 8,
+    // 289 with 4 row tiles.  (The number does not look at how far the
+    // units fill the device: 3 samples of 64 -> 256, 84 units of 8 row tiles, take 73 where 168 of 4 take 48.)
     bool shared = MX && ND == 2 && mtiles_all > 2 && forward_shared();
     if (shared) {
         auto cost = [&](int rt) { const int mc = (mtiles_all + rt - 1) / rt; return mc * (rt * (S16 ? 1 : 6) + 10); };
         MT = mtiles_all > 4 && cost(8) <= cost(4) ? 8 : 4;
         P.mchunks = (mtiles_all + MT - 1) / MT;
     }
-    // Few positions: forward_split_kernel in blocks of 64 positions, four wavefronts to a position, as long as
-    // that gives no more than two workgroups per CU.
+    // Few positions (`small`): forward_split_kernel in blocks of 64 positions, four wavefronts to a position, as long as
+    // that gives a CU no more workgroups than it holds (two; one of four row tiles).  One sample, with / without:
+    // 3x3x3, 64 -> 16 channels, 8 x 14 x 14 positions: 23 / 52; 124 layers of 16 to 256 channels: 0.85 of the time on average, at
+    // worst 1.2 (2-D, 64 -> 64, 75 x 101 positions: 34 / 30).  Limits of half and of twice as many workgroups: the same
+    // on average, single layers 0.7 to 0.8 times as fast.  Not for a single tap in 3-D: the halo of 64 positions costs more to
+    // stage than it saves (128 -> 32 channels, 16 x 28 x 28: 42 with, 29 without).
     bool small = false;
-    // (a single tap leaves too few steps to share in 3-D: the halo of 64 positions costs more to stage than it saves)
     // Shared columns only where they can fill half of the device: with a workgroup for every 16 input channels in
     // float32, whose channels can be split, and without in 16-bit storage, whose cannot (256 -> 256 channels, 3x3, 2 x 28 x 28
     // positions in bfloat16: 16 units, 105 us shared and 60 with several wavefronts to a position).
@@ -100,20 +109,25 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             MT = 4;
             P.mchunks = (mtiles_all + MT - 1) / MT;
         }
+        // Parts of the input channels, as many as the device has room for, at least 16 channels each (8 where four wavefronts
+        // share them; 4 or 16 there: 5 % slower, the same on average).  256 -> 16 channels, 28 x 28 positions: 44 unsplit, 22 split; 3x3x3,
+        // 64 -> 16, 8 x 20 x 20: 71 / 37.  The join and a second workgroup on a CU cost more than short chains gain: 64 -> 64,
+        // 112 x 112: 25 unsplit, 37 in two parts.
         if (!S16 && tiled && forward_split() > 1 && (size_t)P.N * P.outV < FWD_SPLIT_POSITIONS && ws_bytes > wq_bound) {
             const size_t room = ws_bytes - wq_bound < FWD_PARTIAL_CAP ? ws_bytes - wq_bound : FWD_PARTIAL_CAP;
             while (fsplit * 2 <= FWD_MAX_SPLIT && fsplit * 2 <= forward_split() && tiles * P.G * P.mchunks * fsplit * 2 <= (small && MT < 4 ? 2 : 1) * cu_count() &&
-                   (size_t)fsplit * 2 * out_bytes <= room && fsplit * 2 * (small ? 8 : 16) <= P.Cg)      // at least 16 channels per part (8: four wavefronts share them)
+                   (size_t)fsplit * 2 * out_bytes <= room && fsplit * 2 * (small ? 8 : 16) <= P.Cg)
                 fsplit *= 2;
         }
-        // (forward_split_kernel fills a CU with two wavefronts per position before that pays)
+        // Fewer row tiles, more chunks of them, while the grid fills less than half of the device (float64: less than all):
+        // 3x3x3, 16 -> 128 channels, 16 x 40 x 40 positions: 58; limits of all or a quarter of the device: 72, 77.
         while (MT > 1 && !shared && !small && tiles * P.G * P.mchunks * fsplit < cu_count() / (MX ? 2 : 1)) {
             MT /= 2;
             P.mchunks = (mtiles_all + MT - 1) / MT;
         }
         P.Mp = P.mchunks * MT * TN;
     }
-    // Halo kernel: four channels of a voxel side by side in LDS (forward_quad_kernel).  Few
+    // Halo kernel: a workgroup's input neighbourhood in LDS, several channels of a voxel side by side.  Few
     // accumulators (MT <= 2): one 1024-thread workgroup per CU with the whole LDS, if its larger halo
     // fits and leaves 8 channels per pass.  Otherwise 512 threads: two workgroups per CU when that
     // still leaves 8 channels per LDS pass, else one large one.  Returns the wavefronts per
@@ -142,8 +156,8 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                                plan_halo<T, ND>(Ph, MAX_LDS, m, 1 << 30, sizeof(S), 2, false, FG, nullptr, 1, false);
             return tiled ? 2 : 0;
         }
-        // (the 3-D double instance of the 1024-thread shape does not fit its 128 registers; short segments
-        // have short passes, and two workgroups per CU then cover each other's staging)
+        // (the 3-D double instance of the 1024-thread shape does not fit its 128 registers.  float32: the two shapes
+        // measure the same, 64 -> 32 and 64 channels in segments of 4 to 64, 2-D and 3-D: 0.98 to 1.02.)
         if (MT <= 2 && wide_forward() && !(sizeof(T) == 8 && ND == 3) && (!MX || wide_forward() == 2 || (P.cpg >= 16 && P.Cg >= 16))) {
             Params Pw = P;
             if (plan_shape(Pw, MAX_LDS, m, 16, false) && (long long)Pw.N * Pw.tiles * Pw.G * Pw.mchunks <= 0x7fffffffLL &&
@@ -267,6 +281,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                 if (int rc = check_launch("forward weight packing")) return rc;
             }
             // a grid of at most one workgroup per CU: sixteen wavefronts to its 256 positions, two to a position
+            // (224 x 224 positions: 256 -> 16 channels 121, and 137 with one wavefront to a position; 16 -> 64: 28 / 25)
             const bool pairs = MX && !small && !shared && nw == WAVESH && MT <= 2 && P.kV > 1 && forward_small() && forward_slots() == 0 &&
                                (long long)plans[0].N * plans[0].tiles * plans[0].G * plans[0].mchunks * fsplit <= cu_count();
             // (the sums of the wavefronts that share positions)
@@ -307,7 +322,9 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             if (fsplit == 1 && forward_tail_split()) {
                 const long long slots = forward_slots() ? forward_slots() : resident_workgroups(reinterpret_cast<const void*>(kern), (pairs ? 16 : shared || small ? 8 : nw) * 64, lds);
                 const long long rest = units % slots;
-                constexpr double GEO = 0.45;    // tap geometry of a pass, in units of four channels' sampling and contraction
+                // tap geometry of a pass, in units of four channels' sampling and contraction (35 layers of 32 to 128
+                // channels whose last round is partly filled: 0.2 and 0.9 choose splits of the same time, no split takes 1.09 times as long)
+                constexpr double GEO = 0.45;
                 // cost of the longest workgroup when the passes of a unit (cch channels each) are dealt to cs workgroups
                 auto wg_cost = [&](int cs, int cch, int* npasses) {
                     double load[64] = {0};

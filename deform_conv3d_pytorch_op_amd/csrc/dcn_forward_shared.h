@@ -3,8 +3,8 @@
 //
 // Where every wavefront samples into its own operands (forward_split_kernel), 256 output channels mean
 // sampling everything twice and reading 12 KB of weights per 24 matrix instructions and wavefront:
-// the L1 and its latency set the pace (256 -> 256 channels, 3x3, 25 088 positions: 0.33 ms).  Here eight wavefronts
-// share the columns.  A phase is 32 reduction slots -- one tap pair, two groups of eight channels: each
+// the L1 and its latency set the pace (256 -> 256 channels, 3x3, 25 088 positions: 0.277 ms; 0.239 here, with the matrix
+// units of an occupied CU busy 46 % of the cycles, its vector ALUs 23 %).  Here eight wavefronts share the columns.  A phase is 32 reduction slots -- one tap pair, two groups of eight channels: each
 // wavefront samples 32 positions of one group and writes its operand parts to LDS, and multiplies the
 // previous phase's columns by its own row tiles, whose weights (each used by two wavefronts only) come
 // straight from the L2 into registers a phase ahead.  Columns are double buffered, one barrier per phase;

@@ -8,13 +8,13 @@
 //
 // Contraction of float32 operands.  A float32 value is the exact sum of three bfloat16 values: the
 // value rounded to bfloat16, the remainder rounded to bfloat16, and what is left (24 significant bits
-// = 3 x 8; each remainder is formed without rounding).  A product of two values is then nine products
-// of parts, each exact in float32, of which the three smallest (below 2^-24 of the product together)
-// are left out; the other six are summed by v_mfma_f32_32x32x16_bf16 into float32 accumulators,
-// smallest first.  Against float64, sums of 64 to 6912 products come out with 10 to 30 % less error
-// than from v_mfma_f32_32x32x2_f32, which rounds after every second product where this rounds
-// after every sixteenth.  Six instructions reduce over 16 slots in 93 ns per SIMD where the float32 ones
-// take 239 ns, and unlike those they run next to vector instructions.
+// = 3 x 8; each remainder is formed without rounding; values from 2^-110 on, see below).  A product of two
+// values is then nine products of parts, each exact in float32, of which the three smallest (below 2^-24 of the
+// product together) are left out; the other six are summed by v_mfma_f32_32x32x16_bf16 into float32 accumulators,
+// smallest first.  Against float64, sums of 64 / 576 / 6912 products of N(0, 1) values are off by 6.5e-8 / 1.0e-7 /
+// 3.4e-7 (2-norm), by v_mfma_f32_32x32x2_f32, which rounds after every second product where this rounds
+// after every sixteenth, by 9.2e-8 / 2.4e-7 / 5.2e-7.  Six instructions reduce over 16 slots in 81 ns per SIMD
+// (13.5 each) where eight float32 ones take 216 to 239 ns, and unlike those they run next to vector instructions.
 // Operands without such parts: a workgroup works its block out once more through the float32
 // instructions, on the weights as they are, when a result
 //   - is not finite (inf - inf in the parts; this also gives an overflow of the parts the float32 meaning), or
@@ -523,12 +523,14 @@ __device__ inline void store_tile(const Params& P, O* __restrict__ dst, const S*
 // Up to four row tiles (128 output channels) per wavefront, each wavefront sampling its own 32
 // positions straight into its operands.  NW wavefronts; dynamic LDS = cchunk * hstride * sizeof(S) bytes,
 // cchunk a multiple of eight (or four, float32: half of the reduction slots then stay empty).
-// Binding: the LDS reads of the corners in 3-D (64 channels, 27 taps, 200 704 positions: 1.2e7 16-byte
-// reads with 46 % bank conflicts of random offsets hold a CU's LDS 0.32 of 0.52 ms; 0.64 ms on the
-// float32 instructions), operand latency in 2-D.
+// Binding in 3-D: vector instructions, 20 to a matrix instruction, and the LDS reads of the corners beside them (64
+// channels, 27 taps, 200 704 positions, 0.49 ms: while a CU holds a workgroup its vector ALUs are busy 74 % of the cycles, its LDS
+// 53 %, 63 % of that bank conflicts of random offsets, its matrix units 28 %; 0.64 ms on the float32 instructions).  In
+// 2-D: operand latency.
 // TS > 1 (layers too small to fill the device otherwise): TS wavefronts share 32 positions, each takes a
-// contiguous share of a pass's (tap pair, channel group) steps, and their sums meet in LDS -- a step
-// takes a lone wavefront 1 to 1.5 us of latencies, so a small layer's time is the length of that chain.
+// contiguous share of a pass's (tap pair, channel group) steps, and their sums meet in LDS -- a step of a lone
+// wavefront takes 0.8 to 1.8 us in 2-D, 2.0 to 2.4 us in 3-D (one to four row tiles), most of it latencies, so a small
+// layer's time is the length of that chain.
 // (up to two row tiles: four wavefronts per SIMD, i.e. at most 128 registers)
 template <int ND, int MT, int NW, int TS, typename S>
 __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel(Params P, PlanSet alts, const unsigned* __restrict__ sel,

@@ -55,7 +55,7 @@ template <typename T> inline void bwd_data_weight_pad(int M, int Cg, int& Mp, in
 inline size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 
 constexpr int TAP_PAD = 8;      // zero tap slabs behind the last group: an MFMA pass may start up to 7 taps before the end
-// Elements of the per-chunk weight slabs of the fused backward kernel (pack_weight_kernel, chunks of
+// Elements of the per-chunk weight slabs of the fused backward kernel (pack_backward_weight, chunks of
 // `cch` channels) for `slabs` slabs.
 template <typename T, typename S = T> inline size_t packed_weight_elems(int M, int kV, size_t slabs, int cch) {
     const int TP = Mma<T>::TN / cch;
@@ -212,7 +212,7 @@ inline int relayout(const Params& P, const T* w, T* wt, int channel_fastest, hip
 //   DCN_TRACE_PLANS=1      print the halo plans and launches of every call on stderr
 //   DCN_LDS_BUDGET_KB      LDS per 512-thread workgroup of the forward halo kernel (default 72: two per CU)
 //   DCN_FORWARD_WG=512     never use the 1024-thread forward variant; =1024 use it whenever its halo fits
-//   DCN_FORWARD_SPLIT=n    forward pass: split the input channels of a position block over at most n workgroups (0: never)
+//   DCN_FORWARD_SPLIT=n    forward pass, float32 and float64: split the input channels of a position block over at most n workgroups (0: never)
 //   DCN_FORWARD_TAIL=0     forward pass: never split only the units of the last, partly filled round of workgroups (n > 1: n ways)
 //   DCN_FORWARD_TAIL2=0    forward pass: the split units of the last round all the same number of ways, never in two runs
 //   DCN_FORWARD_SLOTS=n    forward pass: plan the launch as if n workgroups ran at once (test hook)
@@ -498,9 +498,9 @@ inline int launch_halo(K kern, const char* name, dim3 grid, int threads, size_t 
 // ---------------------------------------------------------------------------------------------
 // The operators, each instantiated in a translation unit of its own (they compile in parallel).
 constexpr unsigned FLAG_INPUT_ONLY = 0x100u;     // internal: see backward_input_offset
-template <typename T, int ND, typename S = T>
 // off = null (float32): every offset is zero.  transposed: the weight of the convolution that this call is
 // the backward pass of.
+template <typename T, int ND, typename S = T>
 int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* bias, S* out, void* ws, size_t ws_bytes,
             hipStream_t s, bool* declined = nullptr, bool transposed = false);
 // prep: jobs that belong to the caller, done in the launch that prepares this operator

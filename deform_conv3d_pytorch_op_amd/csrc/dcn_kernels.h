@@ -897,7 +897,7 @@ __device__ inline float weight_bound(const float* __restrict__ bounds, int which
 // NW wavefronts per workgroup (8; 4 where only a smaller block of positions has a halo that fits).
 // HS > 0 fixes the plane stride at compile time (the host then plans with hstride = HS): the plane
 // of a channel becomes an immediate offset of the LDS instructions instead of address arithmetic.
-// PACKW: the weights come in the per-chunk lane order of pack_weight_kernel instead of
+// PACKW: the weights come in the per-chunk lane order of pack_backward_weight instead of
 // [g][tap][m][channel].
 // CCH = 16 (float, 2-D layers whose halo leaves room for 16 channel planes): two taps per pass, so the
 // nine taps of a 3x3 kernel take 5 passes per 16 channels instead of 6, with half as many chunks to

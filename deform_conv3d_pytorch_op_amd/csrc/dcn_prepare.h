@@ -3,6 +3,9 @@
 // cleared gradients, channels-last copies with the sums of grad_output for grad_bias -- and each is a
 // few microseconds of work: as launches of their own they cost a small layer more than the kernels they prepare
 // (2 x 8 x 16 x 16 float64: eight launches of 1 to 6 us with gaps of 5 to 17 us between them).
+// Large layers are bound by the copies: 64 -> 64 channels, 3-D, 4 x 16 x 56 x 56 float32, 322 MB in 79 us (4.1 TB/s; a plain
+// copy reaches 5.2), where the jobs one by one took 91 us and the sum of grad_output over two axes 73; 256 -> 256, 2-D,
+// 8 x 56 x 56: 25 against 50 and 12; 128 -> 128, 3-D, 2 x 16 x 112 x 112 -> 56 x 56: 175 against 220 and 42.
 #pragma once
 #include "dcn_kernels.h"
 

@@ -22,7 +22,7 @@ def make_case(nd, N, C_in, C_out, ins, k, stride, pad, dil, cpg, groups, off_sca
     oshape = (N, C_in // cpg * nd * kV) + outs
     if off_dist == "uniform":
         off = (torch.rand(oshape, generator=g, dtype=torch.float64) * 2 - 1) * off_scale
-    else:   # N(0,1) with 10 % of the entries replaced by U[-6,6]  (BASELINE configs[2])
+    else:   # N(0,1) with 10 % of the entries replaced by U[-6,6]
         off = torch.randn(oshape, generator=g, dtype=torch.float64)
         mask = torch.rand(oshape, generator=g, dtype=torch.float64) < 0.1
         wide = (torch.rand(oshape, generator=g, dtype=torch.float64) * 2 - 1) * 6
@@ -41,7 +41,7 @@ SMALL_CASES = {
     "2d_basic": (2, 2, 4, 6, (7, 9), 3, 1, 1, 1, 2, 2, 3.0),
     "2d_rect_kernel_stride_dil": (2, 1, 6, 4, (8, 6), (3, 2), (2, 1), (2, 1), (2, 1), 3, 1, 2.0),
     "2d_ref_gradient_script": (2, 2, 2, 4, 7, 1, 2, 2, 2, 2, 2, 1.0),      # deform2d_double/test_gradient.py:7-19
-    "2d_c1": (2, 2, 8, 8, 16, 3, 1, 1, 1, 8, 1, 1.5),
+    "2d_c1": (2, 2, 8, 8, 16, 3, 1, 1, 1, 8, 1, 1.5),                   
     "2d_wide_m": (2, 1, 40, 72, (9, 11), 3, 1, 1, 1, 20, 1, 2.0),          # several MFMA row tiles, 2 deformable groups
     "2d_many_m_chunks": (2, 1, 6, 300, (6, 7), 3, 1, 1, 1, 6, 1, 1.0),     # M > 8 row tiles of 32
     "2d_c3_like": (2, 1, 16, 8, 10, 3, 1, 2, 2, 4, 2, 3.0),                # groups 2, 4 deformable groups, dilation 2
