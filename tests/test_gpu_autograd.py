@@ -115,3 +115,41 @@ def test_misshapen_grad_output_is_refused():
                     _lib.native().conv2d_backward(*leaves, bad, *cfg, True, True, True)
                 else:
                     _lib.native().conv_offset_backward(3 if name == "3d" else 2, *leaves, bad, *cfg, False, False, True, True, True)
+
+
+@pytest.mark.parametrize("name", LAYERS)
+def test_saved_tensor_hooks(name):
+    """The node saves its tensors through the hooks in force, once each, and gets them back for backward."""
+    print("saved-tensor hooks", name, flush=True)
+    fn, leaves, cfg, gout = _layer(name)
+    want = _results(fn, leaves, cfg, gout)
+    packed = []
+
+    def pack(t):
+        packed.append(t)
+        return t.cpu()
+
+    with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t.cuda()):
+        out = fn.apply(*leaves, *cfg)
+    assert {t.data_ptr() for t in packed} == {t.data_ptr() for t in leaves[:-1]} and len(packed) == len(leaves) - 1
+    _same([out] + list(torch.autograd.grad(out, leaves, gout)), want)
+
+
+@pytest.mark.parametrize("reentrant", [False, True])
+def test_checkpoint(reentrant):
+    import torch.utils.checkpoint as cp
+    print("checkpoint", reentrant, flush=True)
+    fn, leaves, cfg, gout = _layer("3d")
+    out = cp.checkpoint(lambda *t: fn.apply(*t, *cfg).relu(), *leaves, use_reentrant=reentrant)
+    want = fn.apply(*leaves, *cfg).relu()
+    out.backward(gout)
+    _same([t.grad for t in leaves], torch.autograd.grad(want, leaves, gout))
+
+
+def test_saved_tensor_changed_in_place_is_noticed():
+    fn, leaves, cfg, gout = _layer("2d")
+    out = fn.apply(*leaves, *cfg)
+    with torch.no_grad():
+        leaves[2].add_(1.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.backward(gout)
