@@ -480,24 +480,16 @@ __device__ inline void mma_exact(const Params& P, const S* __restrict__ W, int g
 // then repeats in vain) and, in float32, zero or not too small (see the top of the file).
 template <int NT, typename S>
 __device__ inline bool results_stand(const Mma<float>::Acc* acc) {
-    constexpr float SMALL = 0x1p-80f;
-    float s = 0.f, least = SMALL;
+    float s = 0.f;
+    unsigned least = ~0u;                               // twice the bits of the least magnitude that is not zero, less one
 #pragma unroll
     for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int r = 0; r < Mma<float>::NACC; ++r) {
-            const float a = fabsf(acc[t][r]);
-            s += a;
-            if constexpr (sizeof(S) == 4) least = __builtin_amdgcn_fmed3f(least, a, -1.f);       // (the lesser: one instruction a value)
+            s += fabsf(acc[t][r]);
+            if constexpr (sizeof(S) == 4) least = min(least, (__float_as_uint(acc[t][r]) << 1) - 1u);       // (shift-add and half a min3 a value)
         }
-    bool small = false;
-    if (least < SMALL) {                                // zeros (rows past the last channel, positions without a sample) or small ones
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int r = 0; r < Mma<float>::NACC; ++r) small = small || (acc[t][r] != 0.f && fabsf(acc[t][r]) < SMALL);
-    }
-    return s <= std::numeric_limits<float>::max() && !small;
+    return s <= std::numeric_limits<float>::max() && least >= (__float_as_uint(0x1p-80f) << 1) - 1u;
 }
 
 // Writes a 32 x 32 result tile: row m0 + r of group g's output channels (m0 uniform), this lane's position.
