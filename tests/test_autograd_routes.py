@@ -48,41 +48,34 @@ def test_a_trace_being_recorded_goes_through_function_apply():
 
 
 @pytest.mark.parametrize("fn", _functions(), ids=lambda f: f.__name__)
-def test_a_traced_call_is_recorded_as_the_function(fn):
+def test_a_traced_call_is_recorded_as_the_function(fn, monkeypatch):
     """On the CPU the call itself is refused (there is no CPU path), by the Function's own forward."""
     import deform_conv3d_pytorch_op_amd as dcn
     nd = 3 if fn is dcn.ConvOffset3dFunction else 2
     x, w = torch.zeros((1, 2) + (4,) * nd), torch.zeros((2, 2) + (1,) * nd)
     args = (x, w) if fn is dcn.Conv2dFunction else (x, torch.zeros((1, 2 * nd) + (4,) * nd), w)
     calls, forward = [], fn.forward
-    fn.forward = staticmethod(lambda *a: calls.append(len(a)) or forward(*a))
-    try:
-        with pytest.raises(RuntimeError, match="GPU"):
-            fn.apply(*args)
-        assert calls == []
-        with pytest.raises(RuntimeError, match="GPU|float32"):
-            torch.jit.trace(lambda *t: fn.apply(*t), args, check_trace=False)
-        assert len(calls) == 1
-    finally:
-        fn.forward = forward
+    monkeypatch.setattr(fn, "forward", staticmethod(lambda *a: calls.append(len(a)) or forward(*a)))
+    with pytest.raises(RuntimeError, match="GPU"):
+        fn.apply(*args)
+    assert calls == []
+    with pytest.raises(RuntimeError, match="GPU"):
+        torch.jit.trace(lambda *t: fn.apply(*t), args, check_trace=False)
+    assert len(calls) == 1
 
 
 @pytest.mark.parametrize("fn", _functions(), ids=lambda f: f.__name__)
 @pytest.mark.parametrize("at", range(4))
-def test_forward_mode_tangents_are_refused(fn, at):
+def test_forward_mode_tangents_are_refused(fn, at, monkeypatch):
     """A tangent on any argument: refused by Function.apply, not dropped."""
     import torch.autograd.forward_ad as fwad
-    forward = fn.forward
-    fn.forward = staticmethod(lambda ctx, inputs, *rest: inputs * 2)       # (needs no GPU)
-    try:
-        args = [torch.ones(3) for _ in range(3 if fn.__name__ == "Conv2dFunction" else 4)]
-        at = min(at, len(args) - 1)
-        with fwad.dual_level():
-            args[at] = fwad.make_dual(args[at], torch.ones(3))
-            with pytest.raises(NotImplementedError, match="jvp"):
-                fn.apply(*args)
-    finally:
-        fn.forward = forward
+    monkeypatch.setattr(fn, "forward", staticmethod(lambda ctx, inputs, *rest: inputs * 2))       # (needs no GPU)
+    args = [torch.ones(3) for _ in range(3 if fn.__name__ == "Conv2dFunction" else 4)]
+    at = min(at, len(args) - 1)
+    with fwad.dual_level():
+        args[at] = fwad.make_dual(args[at], torch.ones(3))
+        with pytest.raises(NotImplementedError, match="jvp"):
+            fn.apply(*args)
 
 
 @pytest.mark.parametrize("fn", _functions(), ids=lambda f: f.__name__)
