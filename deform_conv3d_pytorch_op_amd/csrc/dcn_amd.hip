@@ -194,7 +194,7 @@ int layer_backward(const Geometry& g, const S* in, const S* w, const S* off, con
     } else {
         tgin = gin; tgoff = goff; tgw = gw; tgb = gb;
     }
-    const size_t dbytes = backward_data_need<T>(P.N, P.C_in, P.C_out, P.inV, P.kV, P.G, P.cpg);
+    const size_t dbytes = backward_data_need<T>(P.N, P.C_in, P.C_out, P.inV, P.outV, P.kV, P.G, P.cpg);
     const size_t wbytes = backward_weight_need<T>(P.N, P.C_in, P.C_out, P.inV, P.outV, P.kV, P.G);
     void *dws = data ? take(dbytes) : nullptr, *wws = gw ? take(wbytes) : nullptr;
     if ((data && !dws) || (gw && !wws)) return fail(DCN_E_WORKSPACE, "workspace too small");
@@ -431,9 +431,9 @@ size_t dcn_layer_backward_workspace_bytes(int elem_size, int nd, int batch, int 
         return 0;
     const int cpg = channel_per_deformable_group;
     if (elem_size == 8)
-        return align256(backward_data_need<double>(batch, input_c, output_c, input_volume, kernel_volume, group, cpg)) +
+        return align256(backward_data_need<double>(batch, input_c, output_c, input_volume, output_volume, kernel_volume, group, cpg)) +
                align256(backward_weight_need<double>(batch, input_c, output_c, input_volume, output_volume, kernel_volume, group));
-    return align256(backward_data_need<float>(batch, input_c, output_c, input_volume, kernel_volume, group, cpg)) +
+    return align256(backward_data_need<float>(batch, input_c, output_c, input_volume, output_volume, kernel_volume, group, cpg)) +
            align256(backward_weight_need<float>(batch, input_c, output_c, input_volume, output_volume, kernel_volume, group)) +
            (elem_size == 2 ? copies16_bytes(batch, input_c, output_c, input_volume, output_volume, kernel_volume, group, cpg) : 0);
 }

@@ -4,11 +4,21 @@
 
 namespace dcn {
 
+// The instantiations of backward_fused_kernel: channels per chunk and position tiles per block.
+template <int ND, typename S>
+using FusedKern = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const typename Parts<S>::Vec*, const S*, const S*, const typename Parts<S>::Vec*,
+                           const float*, float*, float*, int, unsigned, int);
+template <int ND, typename S> inline FusedKern<ND, S> fused_kernel(int cch, int tiles) {
+    if (tiles == 4) return cch == 8 ? backward_fused_kernel<ND, 8, 4, S> : cch == 4 ? backward_fused_kernel<ND, 4, 4, S> : nullptr;
+    if constexpr (ND == 2)
+        if (cch == 16) return backward_fused_kernel<2, 16, 8, S>;
+    return cch == 8 ? backward_fused_kernel<ND, 8, 8, S> : cch == 4 ? backward_fused_kernel<ND, 4, 8, S> : nullptr;
+}
+
 // S = T: the float32 / float64 operator.  S = Bf16 / Fp16 (T = float): input, weight, offset and
-// grad_output are in that storage format (the gradients are float), and only the fused kernel with
-// its grad_output operand in registers serves them, on the 16-bit matrix instructions; where it
-// cannot, *declined is set and nothing is launched: the caller then widens the tensors and runs the
-// float32 operator.
+// grad_output are in that storage format (the gradients are float), and only backward_fused_kernel serves
+// them; where it cannot, *declined is set and nothing is launched: the caller then widens the tensors and
+// runs the float32 operator.
 template <typename T, int ND, typename S>
 int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* off, const S* gout, T* gin,
                           T* goff, void* ws, size_t ws_bytes, hipStream_t s, unsigned flags, bool* declined, Prep* given) {
@@ -42,20 +52,23 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
     Prep& prep = given ? *given : own;
     const dim3 tgrid((P.inV + 31) / 32, (unsigned)(P.C_in + 31) / 32, (unsigned)P.N), tblock(32, 8);
 
-    // 1) one kernel: scatter privatised in LDS + coordinate gradient from an LDS input halo
+    // 1) one kernel: scatter privatised in LDS + coordinate gradient from an LDS input halo.
+    // float32 layers whose LDS cells may be paired and 16-bit storage: backward_fused_kernel, with grad_output in
+    // operand order behind the channels-last regions of the workspace.  Others: backward_input_halo_kernel.
+    const size_t gq_at = wbytes + 2 * tbytes, gq_bytes = fused_gout_need<S>(P.N, P.M, P.G, P.outV);
+    const bool gq_fits = ws_bytes >= gq_at + gq_bytes + (tail_words ? BWD_TAIL + 256 : 0);
     // A halo of up to FUSED_HS cells gets the variant with that compile-time plane stride (the four
     // planes of either kind then lie within the 64 KB reach of an LDS instruction's offset field).
     // Eight wavefronts per workgroup; four (half the positions, in the block shape with the smallest
     // halo) where only that fits, e.g. under stride 2.
     constexpr int FUSED_HS = sizeof(T) == 4 ? 2720 : 2112;
-    constexpr int FUSED_HS8 = 2016;     // plane stride of the 8-channel float instantiation with compile-time halo extents
-    using Kern = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const S*, const S*, const float*, T*, T*, int, unsigned, int);
+    using Kern = void (*)(Params, PlanSet, const unsigned*, const T*, const T*, const T*, const T*, const float*, T*, T*, int, unsigned, int);
     struct FusedPlan {
         Params Ph;
-        Kern kern;
+        Kern kern;                  // null: backward_fused_kernel
+        const void* entry;
         int nw, cch, csplit, goff_atomic;
         bool zero_goff;
-        bool wide;
         long long whole, items, slots;
         size_t lds;
         const S* wt;
@@ -66,33 +79,60 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
     // halo, four on the block shape with the smallest halo)
     auto plan_fused = [&](int m, FusedPlan& fp) {
         for (int attempt = fused_first_waves() == 8 ? 0 : 2; attempt < 3; ++attempt) {
-            const int nw = attempt < 2 ? 8 : 4;
+            int nw = attempt < 2 ? 8 : 4;
             const bool smallest = attempt > 0;
             Params Ph = P;
             // float32: two channels per LDS cell as 32-bit fixed point while the terms one cell can receive
             // (positions of the block x taps) leave at least 17 bits below the largest possible term
-            const bool pair = sizeof(T) == 4 && fused_pair() && (long long)nw * TN * P.kV <= (1 << 14);
-            const size_t chb = (pair ? 4 : 8) + sizeof(T);      // LDS bytes per channel and halo voxel: cell + input value
-            // Channels per chunk: 8 where that takes fewer MFMA passes per channel (a pass holds TN / CCH
-            // taps: the 9 taps of a 3x3 kernel are 2 float passes per 4 channels or 3 per 8; the 27 of a
-            // 3x3x3 kernel 4 or 7) and the planes of 8 channels fit: the small halos of 2-D layers, and
-            // 3-D ones with paired cells.  16 (2-D, float, paired cells): two taps per pass -- the 9 taps of
-            // a 3x3 kernel are 5 passes per 16 channels instead of 6.  The float kernel with 8 channels
-            // per chunk keeps the input values bank-swizzled and wants the innermost halo extent a
-            // multiple of the four-channel groups per voxel.
-            auto passes = [&](int c) { const int tp = Mma<T>::TN / c; return (P.kV + tp - 1) / tp; };
+            const bool pair = sizeof(T) == 4 && fused_pair() && gq_fits && (long long)nw * TN * P.kV <= (1 << 14);
+            if (S16 && !pair) continue;
             int cch = 0;
+            size_t lds = 0;
+            Kern kern = nullptr;
+            const void* entry = nullptr;
+            // tiles of (tap, channel) rows that c channels take
+            auto passes = [&](int c) { const int tp = Mma<T>::TN / c; return (P.kV + tp - 1) / tp; };
+            if constexpr (sizeof(T) == 4) {
+                // Channels per chunk and position tiles per block, the first shape that fits: more channels are fewer passes over
+                // offsets, grad_offset and grad_output, and fewer tap slots (the 9 taps of a 3x3 kernel are 2 tiles per 4 channels, 3
+                // per 8 or 5 per 16, the 27 of a 3x3x3 kernel 4 per 4 or 7 per 8); they are worth half as many positions to a halo
+                // (128 -> 128 channels, 3x3x3, stride 1 2 2: 2.60 ms with 8 channels and 128 positions, 2.80 with 4 and 256).
+                const int shapes[5][2] = {{8, 16}, {8, 8}, {4, 8}, {8, 4}, {4, 4}};
+                for (int k = 0; pair && attempt != 1 && k < 5 && !cch; ++k) {
+                    const int tiles = shapes[k][0], cand = shapes[k][1];
+                    if (tiles > nw) continue;
+                    if (cand >= 8 && !(fused_chunk8() && seg >= 8 && passes(8) * 4 < passes(4) * 8)) continue;
+                    if (cand == 16 && !(ND == 2 && fused_chunk16() && seg >= 16 && passes(16) * 8 < passes(8) * 16)) continue;
+                    const size_t vb = fused_voxel_bytes<S>(cand), budget = fused_budget();
+                    // the usual block, or the one with the smallest halo where that is a tenth smaller: zeroing, staging and flushing grow with it
+                    Params Pc = P, Ps = P;
+                    const bool usual = !smallest && plan_halo<T, ND>(Pc, budget, m, cand, 1, tiles, false, 1, nullptr, 1, false);
+                    if (plan_halo<T, ND>(Ps, budget, m, cand, 1, tiles, true, 1, nullptr, 1, false) && (!usual || Ps.hvol * 10 < Pc.hvol * 9)) Pc = Ps;
+                    else if (!usual) continue;
+                    if ((size_t)Pc.hvol * vb > budget || (long long)Pc.N * Pc.tiles * Pc.DG * 4 > 0x7fffffffLL) continue;
+                    Ph = Pc;
+                    cch = cand;
+                    nw = tiles;
+                    lds = (size_t)Ph.hstride * vb;
+                    entry = reinterpret_cast<const void*>(fused_kernel<ND, S>(cand, tiles));
+                }
+            }
+            if (pair && !cch) continue;
+            if constexpr (!S16) if (!pair) {
+            const size_t chb = 8 + sizeof(T);      // LDS bytes per channel and halo voxel: cell + input value
+            // 8 channels per chunk where that takes fewer MFMA passes per channel and the planes fit: the small halos of
+            // 2-D layers.  The float kernel with 8 channels per chunk keeps the input values bank-swizzled and wants the
+            // innermost halo extent a multiple of the four-channel groups per voxel.
             size_t tables = 0;
-            bool fixed = false, special = false;
-            for (int cand = 16; cand >= 4 && !cch; cand /= 2) {
-                if (cand >= 8 && !((ND == 2 || pair) && nw == 8 && fused_chunk8() && seg >= 8 && passes(8) * 4 < passes(4) * 8)) continue;
-                if (cand == 16 && !(ND == 2 && pair && fused_chunk16() && seg >= 16 && passes(16) * 8 < passes(8) * 16)) continue;
+            bool fixed = false;
+            for (int cand = 8; cand >= 4 && !cch; cand /= 2) {
+                if (cand == 8 && !(ND == 2 && nw == 8 && fused_chunk8() && seg >= 8 && passes(8) * 4 < passes(4) * 8)) continue;
                 Params Pc = P;
-                const int wmult = cand == 16 ? 1 : cand == 8 ? swizzle_groups<T, 8>() : 1;
+                const int wmult = cand == 8 ? swizzle_groups<T, 8>() : 1;
                 if (!plan_halo<T, ND>(Pc, scatter_budget(), m, 8, chb, nw, smallest, 0, nullptr, wmult)) continue;
                 const size_t tb = (size_t)Pc.hvol * 4;      // halo table
                 if ((long long)Pc.N * Pc.tiles * Pc.DG * 4 > 0x7fffffffLL) continue;
-                if (cand >= 8) {
+                if (cand == 8) {
                     if ((scatter_budget() - tb) / ((size_t)Pc.hstride * chb) < (size_t)cand) continue;
                 } else {
                     // A halo of up to FUSED_HS cells gets the variant with that compile-time plane stride
@@ -104,56 +144,36 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
                 cch = cand;
             }
             if (!cch) continue;
-            const bool sixteen = cch == 16, eight = cch >= 8;
-            Ph.cchunk = cch;
+            const bool eight = cch == 8;
             if (fixed && !eight) Ph.hstride = FUSED_HS;
             // grad_output operand held in registers when its reduction steps fit: 32 per pass
             // (M <= 64 float, 128 double with 4-channel chunks)
-            // (16-bit storage: a reduction step takes 8 output channels and an operand batch half as many steps)
-            const int KS = GcolGemm<T, S>::KS, halve = S16 ? 2 : 1;
-            const int ksteps = (P.M + KS - 1) / KS;
-            const bool wide = eight && !sixteen && pair && ksteps <= 32 / halve;                     // the kernel's WIDE
-            const int slot_regs = (wide || sixteen) ? 8 : (Mma<T>::row(1, 0) - Mma<T>::row(0, 0) == 1) ? 4 : cch / 4;      // the kernel's RPS
-            const bool breg = ksteps <= Mma<T>::NACC / slot_regs * ((wide || sixteen) ? 16 : 8) / halve;
-            // float, 4-channel chunks: a second set of 32 registers takes the operand of up to 128 output channels (16-bit: 256)
-            const bool breg2 = sizeof(T) == 4 && !eight && !breg && ksteps <= 64 / halve && fused_breg2();
-            special = ND == 3 && eight && !sixteen && pair && wide && breg && fused_fixed_stride() && Ph.hext[1] == 14 && Ph.hext[2] == 14 &&
-                      Ph.hstride <= FUSED_HS8;
-            if (special) Ph.hstride = FUSED_HS8;
-            const size_t lds = (size_t)cch * Ph.hstride * chb + tables;
-            Kern kern = nullptr;
-#define DCN_FUSED_C(CCH_, BREG_, HS_, NW_, PAIR_) backward_input_halo_kernel<T, ND, CCH_, true, (BREG_) || S16, HS_, NW_, true, PAIR_, 1, 0, 0, S>
-#define DCN_FUSED_B2(HS_, NW_, PAIR_) backward_input_halo_kernel<T, ND, 4, true, true, HS_, NW_, true, PAIR_, 2, 0, 0, S>
-            auto pick = [&](auto pair_tag) {
-                constexpr bool PR = decltype(pair_tag)::value;
-                if (sixteen) {
-                    if constexpr (ND == 2 && PR && sizeof(T) == 4) kern = breg ? DCN_FUSED_C(16, true, 0, 8, PR) : DCN_FUSED_C(16, false, 0, 8, PR);
-                } else if (eight) {
-                    if constexpr (ND == 2 || PR) kern = breg ? DCN_FUSED_C(8, true, 0, 8, PR) : DCN_FUSED_C(8, false, 0, 8, PR);
-                    // the halo of a 3x3x3 kernel at stride 1 and margin 2 under the default block of positions:
-                    // inner extents 14 x 14 and the plane stride fixed at compile time
-                    if constexpr (ND == 3 && PR && sizeof(T) == 4) {
-                        if (special) kern = backward_input_halo_kernel<T, ND, 8, true, true, FUSED_HS8, 8, true, true, 1, 14, 14, S>;
-                    }
-                } else if (breg2) {
-                    if constexpr (sizeof(T) == 4) {
-                        if (nw == 8) kern = fixed ? DCN_FUSED_B2(FUSED_HS, 8, PR) : DCN_FUSED_B2(0, 8, PR);
-                        else kern = fixed ? DCN_FUSED_B2(FUSED_HS, 4, PR) : DCN_FUSED_B2(0, 4, PR);
-                    }
-                } else if (nw == 8)
-                    kern = fixed && breg ? DCN_FUSED_C(4, true, FUSED_HS, 8, PR) : fixed ? DCN_FUSED_C(4, false, FUSED_HS, 8, PR) : DCN_FUSED_C(4, false, 0, 8, PR);
-                else
-                    kern = fixed && breg ? DCN_FUSED_C(4, true, FUSED_HS, 4, PR) : fixed ? DCN_FUSED_C(4, false, FUSED_HS, 4, PR) : DCN_FUSED_C(4, false, 0, 4, PR);
-            };
-            if constexpr (sizeof(T) == 4) {
-                if (pair) pick(std::true_type{});
-                else pick(std::false_type{});
-            } else
-                pick(std::false_type{});
+            const int ksteps = (P.M + Mma<T>::KL - 1) / Mma<T>::KL;
+            const int slot_regs = (Mma<T>::row(1, 0) - Mma<T>::row(0, 0) == 1) ? 4 : cch / 4;      // the kernel's RPS
+            const bool breg = ksteps <= Mma<T>::NACC / slot_regs * 8;
+            // float, 4-channel chunks: a second set of 32 registers takes the operand of up to 128 output channels
+            const bool breg2 = sizeof(T) == 4 && !eight && !breg && ksteps <= 64 && fused_breg2();
+            lds = (size_t)cch * Ph.hstride * chb + tables;
+#define DCN_FUSED_C(CCH_, BREG_, HS_, NW_) backward_input_halo_kernel<T, ND, CCH_, true, BREG_, HS_, NW_, true>
+#define DCN_FUSED_B2(HS_, NW_) backward_input_halo_kernel<T, ND, 4, true, true, HS_, NW_, true, 2>
+            if (eight) {
+                if constexpr (ND == 2) kern = breg ? DCN_FUSED_C(8, true, 0, 8) : DCN_FUSED_C(8, false, 0, 8);
+            } else if (breg2) {
+                if constexpr (sizeof(T) == 4) {
+                    if (nw == 8) kern = fixed ? DCN_FUSED_B2(FUSED_HS, 8) : DCN_FUSED_B2(0, 8);
+                    else kern = fixed ? DCN_FUSED_B2(FUSED_HS, 4) : DCN_FUSED_B2(0, 4);
+                }
+            } else if (nw == 8)
+                kern = fixed && breg ? DCN_FUSED_C(4, true, FUSED_HS, 8) : fixed ? DCN_FUSED_C(4, false, FUSED_HS, 8) : DCN_FUSED_C(4, false, 0, 8);
+            else
+                kern = fixed && breg ? DCN_FUSED_C(4, true, FUSED_HS, 4) : fixed ? DCN_FUSED_C(4, false, FUSED_HS, 4) : DCN_FUSED_C(4, false, 0, 4);
 #undef DCN_FUSED_B2
 #undef DCN_FUSED_C
             if (!kern) continue;
-            if (S16 && !breg && !breg2) continue;       // 16-bit operands come from registers only
+            entry = reinterpret_cast<const void*>(kern);
+            }
+            Ph.cchunk = cch;
+            const int threads = kern ? nw * 64 : FUSED_WAVES * 64;
             // Work items are (tile, deformable group) pairs, each a run of nchunks channel chunks.  `slots`
             // workgroups run at once, so the items take whole rounds plus a partly filled last one.  Either
             // every item is split over 1, 2 or 4 workgroups (workgroup cz takes every csplit-th chunk), or
@@ -164,7 +184,7 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             // float atomics on a zero-filled buffer; the only owner of an item stores running sums.
             const int nchunks = (seg + cch - 1) / cch;
             const long long items = (long long)Ph.N * Ph.tiles * Ph.DG;
-            const long long slots = forced_slots() ? forced_slots() : resident_workgroups(reinterpret_cast<const void*>(kern), nw * 64, lds);
+            const long long slots = forced_slots() ? forced_slots() : resident_workgroups(entry, threads, lds);
             auto item_cost = [&](double chunks_per_wg, int wgs) { return wgs * (chunks_per_wg + 0.25) / nchunks; };
             int csplit = 1;
             long long whole = 0;                              // unsplit items at the start of the launch
@@ -184,13 +204,13 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             if (forced_csplit()) { csplit = forced_csplit(); whole = 0; }
             if (csplit > nchunks) csplit = nchunks;
             if (whole + (items - whole) * csplit > 0x7fffffffLL) continue;
-            fp.Ph = Ph; fp.kern = kern; fp.nw = nw; fp.cch = cch; fp.csplit = csplit;
+            fp.Ph = Ph; fp.kern = kern; fp.entry = entry; fp.nw = nw; fp.cch = cch; fp.csplit = csplit;
             // grad_offset over the chunks of an item that one workgroup owns: the running sum through plain
             // loads and stores in the 3-D kernels (float atomics run at about 3e11 per second over the device,
             // and a 3x3x3 layer has 81 grad_offset elements per position and chunk); atomics in the 2-D ones
             fp.goff_atomic = ND == 2 && nchunks > 1 ? 1 : 0;
             fp.zero_goff = fp.goff_atomic || csplit > 1;
-            fp.wide = wide; fp.whole = whole; fp.items = items; fp.slots = slots; fp.lds = lds; fp.wt = nullptr;
+            fp.whole = whole; fp.items = items; fp.slots = slots; fp.lds = lds; fp.wt = nullptr;
             return true;
         }
         return false;
@@ -223,18 +243,26 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
         fp[0].wt = wt;
         for (int k = 1; k < nmargins; ++k) {
             FusedPlan& c = fp[pc.nplans];
+            c.wt = nullptr;
             if (!plan_fused(margins[k], c) || c.Ph.hvol > 3 * fp[0].Ph.hvol) continue;
             for (int e = 0; e < pc.nplans && !c.wt; ++e)
-                if (fp[e].cch == c.cch && fp[e].wide == c.wide) c.wt = fp[e].wt;
+                if (fp[e].cch == c.cch && !fp[e].kern == !c.kern) c.wt = fp[e].wt;
             if (!c.wt) {
                 if ((size_t)copies * wbytes > tbytes) continue;
                 c.wt = reinterpret_cast<const S*>(reinterpret_cast<const char*>(in_cl) + (size_t)(copies - 1) * wbytes);
                 ++copies;
             }
             pc.margin[pc.nplans] = margins[k];
-            // flush, staging and the per-chunk passes grow with the halo: most of the kernel's time in 3-D, little in 2-D
-            // (a quarter more where only the shape with half the wavefronts fits)
-            pc.base[pc.nplans] = (1.f + (ND == 3 ? 0.9f : 0.05f) * ((float)c.Ph.hvol / (float)fp[0].Ph.hvol - 1.f)) * (c.nw < fp[0].nw ? 1.25f : 1.f);
+            // Flush, staging and the per-chunk passes grow with the halo.  3-D: with its voxels per position r, as 1 + 0.068 r, a tenth more
+            // with narrower chunks (backward_fused_kernel, 64 -> 64 channels, 4 x 16 x 56 x 56: r = 7.7, 18 and 17.7 with 4-channel
+            // chunks at the margins 2, 3, 4 take 1, 1.46 and 1.60); the kernel with single cells as fitted when it served them all.
+            // Little in 2-D.
+            const Params &H0 = fp[0].Ph, &Hk = c.Ph;
+            const float r0 = (float)H0.hvol / (float)(fp[0].nw * TN), rk = (float)Hk.hvol / (float)(c.nw * TN);
+            if (ND == 3 && !c.kern && !fp[0].kern)
+                pc.base[pc.nplans] = (1.f + 0.068f * rk) / (1.f + 0.068f * r0) * (c.cch < fp[0].cch ? 1.1f : 1.f);
+            else
+                pc.base[pc.nplans] = (1.f + (ND == 3 ? 0.9f : 0.05f) * ((float)Hk.hvol / (float)H0.hvol - 1.f)) * (c.nw < fp[0].nw ? 1.25f : 1.f);
             ++pc.nplans;
         }
         for (int k = pc.nplans; k < MAX_PLANS; ++k) {
@@ -246,19 +274,30 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
         pc.global_cost = offer_global ? 6.5f : 0.f;
         const size_t n_off = (size_t)P.N * P.DG * P.kV * ND * P.outV;
         // one launch prepares: weights in the lane order of the kernel's operand loads, one slab per channel
-        // chunk (variant 9: the row order that leaves the eight channels of a tap in one lane), their bounds,
-        // the choice of the plan, grad_offset cleared where it is added to, and the caller's jobs
+        // chunk, grad_output likewise, the bounds of the weights, the choice of the plan, grad_offset cleared where
+        // it is added to, and the caller's jobs
         if (sel) prep.add(PREP_PLAN, 1);
+        bool any_fused = false;
         for (int k = 0; k < pc.nplans; ++k) {
             bool packed = false;
             for (int e = 0; e < k; ++e) packed = packed || fp[e].wt == fp[k].wt;
             if (packed) continue;
-            const size_t total = packed_weight_elems<T, S>(P.M, P.kV, (size_t)(fp[k].cch == 16 ? chunk_candidates<16>(P.cpg, P.Cg, P.C_in)
-                                                                            : fp[k].cch == 8 ? chunk_candidates<8>(P.cpg, P.Cg, P.C_in)
-                                                                                             : chunk_candidates<4>(P.cpg, P.Cg, P.C_in)), fp[k].cch);
-            PrepJob& job = prep.add(PREP_PACK, (unsigned)((total + 255) / 256 > 8192 ? 8192 : (total + 255) / 256));
-            job.variant = fp[k].wide ? 9 : fp[k].cch;
+            const size_t slabs = (size_t)(fp[k].cch == 16 ? chunk_candidates<16>(P.cpg, P.Cg, P.C_in)
+                                          : fp[k].cch == 8 ? chunk_candidates<8>(P.cpg, P.Cg, P.C_in)
+                                                           : chunk_candidates<4>(P.cpg, P.Cg, P.C_in));
+            const size_t total = fp[k].kern ? packed_weight_elems<T>(P.M, P.kV, slabs, fp[k].cch)
+                                            : slabs * fused_tiles(P.kV, fp[k].cch) * fused_steps(P.M) * 64;      // threads
+            PrepJob& job = prep.add(fp[k].kern ? PREP_PACK : PREP_FUSED_PACK, (unsigned)((total + 255) / 256 > 8192 ? 8192 : (total + 255) / 256));
+            job.variant = fp[k].cch;
             job.dst = const_cast<S*>(fp[k].wt);
+            any_fused = any_fused || !fp[k].kern;
+        }
+        char* gq = static_cast<char*>(ws) + gq_at;
+        if (any_fused) {
+            const size_t total = (size_t)P.N * P.G * fused_steps(P.M) * 2 * P.outV;
+            PrepJob& job = prep.add(PREP_GOUT, (unsigned)((total + 255) / 256 > 16384 ? 16384 : (total + 255) / 256));
+            job.src = gout;
+            job.dst = gq;
         }
         prep.add(PREP_BOUNDS, BOUND_BLOCKS).dst = bounds;
         bool any_atomic = false;
@@ -276,7 +315,7 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             size_t lds = 0;
             for (int e = 1; e < MAX_PLANS; ++e) alts.alt[e - 1] = halo_plan_of(fp[k].Ph);
             for (int e = k; e < pc.nplans; ++e) {
-                const bool same = fp[e].kern == fp[k].kern && fp[e].wt == fp[k].wt && fp[e].csplit == fp[k].csplit && fp[e].whole == fp[k].whole &&
+                const bool same = fp[e].entry == fp[k].entry && fp[e].wt == fp[k].wt && fp[e].csplit == fp[k].csplit && fp[e].whole == fp[k].whole &&
                                   fp[e].items == fp[k].items && fp[e].goff_atomic == fp[k].goff_atomic && fp[e].nw == fp[k].nw &&
                                   fp[e].slots == fp[k].slots && same_blocks(fp[e].Ph, fp[k].Ph);      // (as many workgroups per CU with the larger LDS)
                 if (!same) continue;
@@ -286,8 +325,8 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             }
             launched |= alts.mask;
             if (trace_plans()) {
-                fprintf(stderr, "dcn backward_input_offset: launch for plans %#x: %d wavefronts, %d channels per chunk%s, grid %lld (%lld unsplit, rest x %d), LDS %zu\n",
-                        alts.mask, fp[k].nw, fp[k].cch, fp[k].wide ? " (wide)" : "", fp[k].whole + (fp[k].items - fp[k].whole) * fp[k].csplit, fp[k].whole,
+                fprintf(stderr, "dcn backward_input_offset: launch for plans %#x: %d position tiles, %d channels per chunk%s, grid %lld (%lld unsplit, rest x %d), LDS %zu\n",
+                        alts.mask, fp[k].nw, fp[k].cch, fp[k].kern ? " (single cells)" : "", fp[k].whole + (fp[k].items - fp[k].whole) * fp[k].csplit, fp[k].whole,
                         fp[k].csplit, lds);
                 for (int e = 0; e < pc.nplans; ++e)
                     if ((alts.mask >> e) & 1u)
@@ -295,11 +334,21 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
                                 fp[e].Ph.hext[2], pc.base[e]);
             }
             if (lds > 48 * 1024)
-                if (int rc = raise_lds_limit(reinterpret_cast<const void*>(fp[k].kern), lds)) return rc;
-            hipLaunchKernelGGL(fp[k].kern, dim3((unsigned)(fp[k].whole + (fp[k].items - fp[k].whole) * fp[k].csplit)), dim3(fp[k].nw * 64), lds, s,
-                               fp[k].Ph, alts, (const unsigned*)sel, in, off, fp[k].wt, gout, (const float*)bounds, gin, goff, fp[k].csplit, (unsigned)fp[k].whole,
-                               fp[k].goff_atomic);
-            if (int rc = check_launch("backward_input_halo_kernel")) return rc;
+                if (int rc = raise_lds_limit(fp[k].entry, lds)) return rc;
+            const dim3 grid((unsigned)(fp[k].whole + (fp[k].items - fp[k].whole) * fp[k].csplit));
+            if (fp[k].kern) {
+                if constexpr (!S16)
+                    hipLaunchKernelGGL(fp[k].kern, grid, dim3(fp[k].nw * 64), lds, s, fp[k].Ph, alts, (const unsigned*)sel, in, off, fp[k].wt, gout,
+                                       (const float*)bounds, gin, goff, fp[k].csplit, (unsigned)fp[k].whole, fp[k].goff_atomic);
+            } else {
+                if constexpr (sizeof(T) == 4) {
+                    typedef const typename Parts<S>::Vec* Ops;
+                    hipLaunchKernelGGL((fused_kernel<ND, S>(fp[k].cch, fp[k].nw)), grid, dim3(FUSED_WAVES * 64), lds, s, fp[k].Ph, alts, (const unsigned*)sel, in, off,
+                                       reinterpret_cast<Ops>(fp[k].wt), w, gout, reinterpret_cast<Ops>(gq), (const float*)bounds, gin, goff, fp[k].csplit,
+                                       (unsigned)fp[k].whole, fp[k].goff_atomic);
+                }
+            }
+            if (int rc = check_launch(fp[k].kern ? "backward_input_halo_kernel" : "backward_fused_kernel")) return rc;
         }
         if constexpr (!S16) if (offer_global) {
             // the fourth choice: three launches that return at once unless *sel == MAX_PLANS.  They reuse

@@ -57,9 +57,9 @@ inline size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 constexpr int TAP_PAD = 8;      // zero tap slabs behind the last group: an MFMA pass may start up to 7 taps before the end
 // Elements of the per-chunk weight slabs of the fused backward kernel (pack_backward_weight, chunks of
 // `cch` channels) for `slabs` slabs.
-template <typename T, typename S = T> inline size_t packed_weight_elems(int M, int kV, size_t slabs, int cch) {
+template <typename T> inline size_t packed_weight_elems(int M, int kV, size_t slabs, int cch) {
     const int TP = Mma<T>::TN / cch;
-    return slabs * ((kV + TP - 1) / TP) * (size_t)gcol_slab_steps<T, S>(M) * 64 * (std::is_same<S, T>::value ? 1 : 4);
+    return slabs * ((kV + TP - 1) / TP) * (size_t)gcol_slab_steps<T>(M) * 64;
 }
 // Upper bound of chunk_slot<cch>(cpg, Cg, c) + 1 over the channels: the slabs a per-chunk weight
 // layout occupies.  cpg = 0: the channels per deformable group are not known (the first workspace
@@ -73,10 +73,13 @@ template <typename T> inline size_t bwd_data_weight_bytes(int M, int Cg, int kV,
     const size_t C_in = (size_t)Cg * G;
     const size_t packed4 = packed_weight_elems<T>(M, kV, slab_bound(C_in, G, cpg, 4), 4);
     const size_t packed8 = packed_weight_elems<T>(M, kV, slab_bound(C_in, G, cpg, 8), 8);
-    const size_t packed16 = packed_weight_elems<T>(M, kV, slab_bound(C_in, G, cpg, 16), 16);
-    size_t packed = packed4 > packed8 ? packed4 : packed8;
-    if (packed16 > packed) packed = packed16;
-    return align256((plain > packed ? plain : packed) * sizeof(T));
+    const size_t packed = packed4 > packed8 ? packed4 : packed8;
+    size_t bytes = (plain > packed ? plain : packed) * sizeof(T);
+    for (int cch = 4; sizeof(T) == 4 && cch <= 16; cch *= 2) {
+        const size_t parts = slab_bound(C_in, G, cpg, cch) * fused_slab_ops<float>(M, kV, cch) * 16;
+        if (parts > bytes) bytes = parts;
+    }
+    return align256(bytes);
 }
 // Partial outputs of a forward pass that splits the input channels of a position block over several
 // workgroups: only layers of few positions do (too few blocks to fill the device), with at most
@@ -122,8 +125,15 @@ inline size_t noalloc_weight_bytes(const Params& P) {
 template <typename S> inline size_t split_weight_bytes(const Params& P, int Mp) {
     return ((size_t)chunk_slot<FG>(P.cpg, P.Cg, P.C_in - 1) + 1) * split_slab_elems<S>(P.kV, Mp) * 2 + 256;      // (+: operands read from four elements further on)
 }
-template <typename T> inline size_t backward_data_need(int N, int C_in, int C_out, size_t inV, int kV, int G, int cpg = 0) {
-    return bwd_data_weight_bytes<T>(C_out / G, C_in / G, kV, G, cpg) + 2 * align256((size_t)N * C_in * inV * sizeof(T)) + BWD_TAIL + 512;
+// grad_output in the operand order of backward_fused_kernel (float64: another kernel)
+template <typename S> inline size_t fused_gout_need(int N, int M, int G, size_t outV) {
+    if constexpr (sizeof(S) == 8) return 0;
+    else return align256(fused_gout_bytes<S>(N, M, G, outV));
+}
+// packed weights, two channels-last tensors, grad_output in operand order (float32 and 16-bit storage), the tail
+template <typename T> inline size_t backward_data_need(int N, int C_in, int C_out, size_t inV, size_t outV, int kV, int G, int cpg = 0) {
+    return bwd_data_weight_bytes<T>(C_out / G, C_in / G, kV, G, cpg) + 2 * align256((size_t)N * C_in * inV * sizeof(T)) +
+           fused_gout_need<T>(N, C_out / G, G, outV) + BWD_TAIL + 512;
 }
 // two channels-last copies + one partial weight per position split (at most 256 splits, and never more
 // than about 4096 workgroups: see bww_plan) + the strips of grad_output's sums
@@ -137,7 +147,7 @@ template <typename T> inline size_t backward_weight_need(int N, int C_in, int C_
            align256((size_t)split_ub * kV * C_out * (C_in / G) * sizeof(T)) + align256((size_t)N * last_strips((unsigned)outV) * C_out * sizeof(T));
 }
 template <typename T> inline size_t workspace_need(int N, int C_in, int C_out, size_t inV, size_t outV, int kV, int G, int cpg = 0) {
-    const size_t fwd = forward_need<T>(N, C_in, C_out, outV, kV, G, cpg), bwd = backward_data_need<T>(N, C_in, C_out, inV, kV, G, cpg),
+    const size_t fwd = forward_need<T>(N, C_in, C_out, outV, kV, G, cpg), bwd = backward_data_need<T>(N, C_in, C_out, inV, outV, kV, G, cpg),
                  bww = backward_weight_need<T>(N, C_in, C_out, inV, outV, kV, G);
     const size_t need = fwd > bwd ? fwd : bwd;
     return need > bww ? need : bww;
@@ -218,7 +228,7 @@ inline int relayout(const Params& P, const T* w, T* wt, int channel_fastest, hip
 //   DCN_FORWARD_SLOTS=n    forward pass: plan the launch as if n workgroups ran at once (test hook)
 //   DCN_FORWARD_SHARED=0   forward pass, float32 and 16-bit: never share the sampled columns of a block among wavefronts
 //   DCN_FORWARD_SMALL=0    forward pass, float32 and 16-bit: never several wavefronts to a position
-//   DCN_SCATTER_BUDGET_KB  LDS per workgroup of the privatised scatter kernel (default 144)
+//   DCN_SCATTER_BUDGET_KB  LDS per workgroup of the privatised scatter kernels (default 156: backward_fused_kernel, 144: the others)
 //   DCN_SCATTER=global     scatter grad-input with global atomics instead of the LDS-privatised kernel
 //   DCN_COORD=separate     grad_offset from the channels-last kernel instead of the fused LDS-halo kernel
 //   DCN_FUSED_WAVES=4      fused backward kernel with four wavefronts per workgroup even where eight fit
@@ -238,6 +248,8 @@ static size_t env_kb(const char* name, int dflt) {
 }
 static size_t lds_budget() { static const size_t v = env_kb("DCN_LDS_BUDGET_KB", 72); return v; }
 static size_t scatter_budget() { static const size_t v = env_kb("DCN_SCATTER_BUDGET_KB", 144); return v; }
+// backward_fused_kernel: all that a workgroup can have beside what the kernel declares itself
+static size_t fused_budget() { static const size_t v = env_kb("DCN_SCATTER_BUDGET_KB", 156); return v; }
 static bool fused_coord() {
     static const int v = [] { const char* e = getenv("DCN_COORD"); return (e && strcmp(e, "separate") == 0) ? 0 : 1; }();
     return v != 0;
@@ -338,6 +350,7 @@ static bool fused_breg2() {             // DCN_FUSED_BREG2=0: grad_output operan
     static const int v = [] { const char* e = getenv("DCN_FUSED_BREG2"); return (e && atoi(e) == 0) ? 0 : 1; }();
     return v != 0;
 }
+constexpr size_t FUSED_LDS = 157 * 1024;        // dynamic LDS of backward_fused_kernel at most (160 KB less what it declares)
 static bool native16() {                // DCN_NATIVE16=0: the 16-bit entry points always widen to float32 first
     static const int v = [] { const char* e = getenv("DCN_NATIVE16"); return (e && atoi(e) == 0) ? 0 : 1; }();
     return v != 0;

@@ -7,13 +7,13 @@
 // copy reaches 5.2), where the jobs one by one took 91 us and the sum of grad_output over two axes 73; 256 -> 256, 2-D,
 // 8 x 56 x 56: 25 against 50 and 12; 128 -> 128, 3-D, 2 x 16 x 112 x 112 -> 56 x 56: 175 against 220 and 42.
 #pragma once
-#include "dcn_kernels.h"
+#include "dcn_backward_fused.h"
 
 namespace dcn {
 
-enum PrepKind { PREP_PACK, PREP_PLAN, PREP_BOUNDS, PREP_ZERO, PREP_LAST };
+enum PrepKind { PREP_PACK, PREP_FUSED_PACK, PREP_GOUT, PREP_PLAN, PREP_BOUNDS, PREP_ZERO, PREP_LAST };
 struct PrepJob {
-    int kind, variant;          // PACK: channels per chunk, + 1 for the wide row order
+    int kind, variant;          // PACK, FUSED_PACK: channels per chunk
     unsigned first;             // first block; the job's blocks reach to the next job's first
     const void* src;
     void* dst;
@@ -130,11 +130,25 @@ __global__ __launch_bounds__(256) void backward_prepare_kernel(Params P, PlanCho
     const unsigned block = blockIdx.x - job.first, blocks = next - job.first;
     switch (job.kind) {
         case PREP_PACK: {
-            S* dst = static_cast<S*>(job.dst);
-            if (job.variant == 16) { if constexpr (sizeof(T) == 4) pack_backward_weight<T, 16, false, S>(P, W, dst, block, blocks); }
-            else if (job.variant == 9) { if constexpr (sizeof(T) == 4) pack_backward_weight<T, 8, true, S>(P, W, dst, block, blocks); }
-            else if (job.variant == 8) pack_backward_weight<T, 8, false, S>(P, W, dst, block, blocks);
-            else pack_backward_weight<T, 4, false, S>(P, W, dst, block, blocks);
+            if constexpr (std::is_same<S, T>::value) {
+                T* dst = static_cast<T*>(job.dst);
+                if (job.variant == 8) pack_backward_weight<T, 8>(P, W, dst, block, blocks);
+                else pack_backward_weight<T, 4>(P, W, dst, block, blocks);
+            }
+            break;
+        }
+        case PREP_FUSED_PACK: {
+            if constexpr (sizeof(T) == 4) {
+                typename Parts<S>::Vec* dst = static_cast<typename Parts<S>::Vec*>(job.dst);
+                if (job.variant == 16) pack_fused_weight<16, S>(P, W, dst, block, blocks);
+                else if (job.variant == 8) pack_fused_weight<8, S>(P, W, dst, block, blocks);
+                else pack_fused_weight<4, S>(P, W, dst, block, blocks);
+            }
+            break;
+        }
+        case PREP_GOUT: {
+            if constexpr (sizeof(T) == 4)
+                split_grad_output<S>(P, static_cast<const S*>(job.src), static_cast<typename Parts<S>::Vec*>(job.dst), block, blocks);
             break;
         }
         case PREP_PLAN: choose_plan(pc, off, n_off); break;

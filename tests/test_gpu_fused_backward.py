@@ -1,0 +1,91 @@
+"""backward_fused_kernel: edges of its tiles, chunks and block shapes, and the operands that bfloat16 parts do not hold."""
+import pytest
+import torch
+
+from oracle import dcn_oracle as orc
+from tests.cases import make_case
+
+pytestmark = pytest.mark.gpu
+
+# (nd, N, C_in, C_out, ins, k, stride, pad, dil, cpg, groups, reach): steps of 16 output channels and their remainders;
+# chunks of 16, 8 and 4 channels and short ones; one, two and several tiles to a contraction (1, 9, 25 taps); blocks of 128
+# positions (strides in 3-D); wide halos and samples past every halo; a deformable group over two convolution groups
+EDGES = [
+    (2, 1, 16, 1, (17, 16), 3, 1, 1, 1, 16, 1, 1.5), (2, 1, 17, 15, (9, 33), 3, 1, 1, 1, 17, 1, 1.5),
+    (2, 1, 33, 16, (16, 17), 3, 1, 1, 1, 33, 1, 3.5), (2, 2, 15, 17, (11, 12), 3, 1, 1, 1, 15, 1, 1.0),
+    (2, 1, 9, 65, (20, 18), 3, 2, 1, 1, 9, 1, 2.0), (2, 1, 40, 129, (12, 13), 3, 1, 1, 1, 20, 1, 2.0),
+    (2, 1, 24, 34, (18, 18), 5, 1, 2, 1, 24, 1, 2.0), (2, 1, 18, 20, (13, 11), 1, 1, 0, 1, 18, 1, 1.5),
+    (2, 1, 24, 32, (14, 14), 3, 1, 1, 1, 24, 2, 9.0), (2, 1, 8, 8, (24, 24), 3, 3, 1, 2, 2, 1, 2.0),
+    (3, 1, 8, 16, (5, 9, 10), 3, 1, 1, 1, 8, 1, 1.5), (3, 1, 9, 33, (4, 8, 9), 3, 1, 1, 1, 9, 1, 3.5),
+    (3, 1, 12, 80, (9, 21, 19), 3, 2, 1, 1, 12, 1, 2.0), (3, 1, 16, 130, (6, 15, 17), 3, (1, 2, 2), 1, 1, 8, 1, 2.0),
+    (3, 1, 20, 17, (5, 9, 9), 2, 1, 1, 1, 10, 1, 6.0), (3, 1, 8, 24, (9, 9, 9), 3, 1, 2, 2, 4, 2, 2.5),
+    (3, 1, 10, 7, (6, 5, 40), 1, 1, 0, 1, 5, 1, 1.5),
+]
+
+
+def _gradients(c):
+    """grad_input, grad_offset"""
+    import deform_conv3d_pytorch_op_amd as dcn
+    fn = dcn.ConvOffset3dFunction if c["nd"] == 3 else dcn.ConvOffset2dFunction
+    x, off, w = (c[k].cuda().requires_grad_(k != "w") for k in ("x", "off", "w"))
+    fn.apply(x, off, w, None, c["stride"], c["pad"], c["dil"], c["cpg"], c["groups"]).backward(c["gout"].cuda())
+    return x.grad.cpu().double(), off.grad.cpu().double()
+
+
+def _oracle(c):
+    """In float32 with double sums: the coordinates are then those of the kernel."""
+    d = {k: c[k].float() for k in ("x", "off", "w", "gout")}
+    return [t.double() for t in orc.backward(d["x"], d["off"], d["w"], d["gout"], None, c["stride"], c["pad"], c["dil"], c["cpg"], c["groups"])[:2]]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("spec", EDGES, ids=lambda s: "%dd-%d-%d-k%d-cpg%d" % (s[0], s[2], s[3], s[5], s[9]))
+def test_edges(spec, dtype):
+    """2-norm: grad_input is rounded to 32-bit fixed point (1e-4 of its largest values at most), grad_offset a chain of
+    float32 sums over the channels; 16-bit results are rounded once more (2^-9 and 2^-12 of each value)."""
+    print("edges", spec, dtype, flush=True)
+    c = make_case(*spec, dtype=dtype, seed=31, bias=False)
+    once = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}[dtype]
+    for got, want, tol in zip(_gradients(c), _oracle(c), (1e-4, 1e-5)):
+        err = ((got - want).norm() / want.norm()).item()
+        print("  relative 2-norm error %.2e" % err, flush=True)
+        assert err <= tol + once
+
+
+@pytest.mark.parametrize("spec", [EDGES[5], EDGES[10], EDGES[13]], ids=["2d", "3d", "3d-strided"])
+@pytest.mark.parametrize("what,exponent", [("gout", 60), ("gout", 111), ("gout", 118), ("w", 111), ("w", 118), ("w", 126), ("w", 140)])
+def test_small_operands(spec, what, exponent):
+    """One operand times 2^-exponent, the other times a power of two that keeps the gradients normal numbers: as exact as
+    ordinary operands, whose errors test_edges bounds."""
+    print("small", spec, what, exponent, flush=True)
+    c = make_case(*spec, dtype=torch.float32, seed=32, bias=False)
+    c[what] = c[what] * 2.0 ** -exponent
+    other = "w" if what == "gout" else "gout"
+    c[other] = c[other] * 2.0 ** (10 if exponent < 130 else 30)
+    for got, want, tol in zip(_gradients(c), _oracle(c), (1e-4, 1e-5)):
+        assert want.abs().max().item() > 2.0 ** -122
+        err = ((got - want).norm() / want.norm()).item()
+        print("  relative 2-norm error %.2e" % err, flush=True)
+        assert err <= tol
+
+
+def test_one_small_position_beside_ordinary_ones():
+    """grad_offset of positions whose grad_output alone is tiny."""
+    print("small position", flush=True)
+    c = make_case(2, 1, 16, 48, (24, 40), 3, 1, 1, 1, 16, 1, 0.9, dtype=torch.float32, seed=33, bias=False)
+    c["gout"][..., 20:] *= 2.0 ** -119
+    got, want = _gradients(c)[1], _oracle(c)[1]
+    for part in (slice(0, 20), slice(20, None)):
+        g, w = got[..., part], want[..., part]
+        assert ((g - w).norm() / w.norm()).item() <= 1e-5
+
+
+def test_values_whose_parts_round_to_infinity():
+    """Weights just below the largest float with gradients that stay finite."""
+    print("huge", flush=True)
+    c = make_case(3, 1, 12, 20, (4, 9, 9), 3, 1, 1, 1, 12, 1, 1.5, dtype=torch.float32, seed=34, bias=False)
+    c["w"].view(-1)[::5] = 3.395e38
+    c["gout"] *= 1e-6
+    for got, want in zip(_gradients(c), _oracle(c)):
+        assert torch.isfinite(want).all()
+        assert ((got - want).norm() / want.norm()).item() <= 1e-4
