@@ -60,6 +60,8 @@ int launch_bwd_weight(const WeightCall<T, T>& c, const T* off, hipStream_t s) {
     const int TN = Mma<T>::TN;
     const size_t lds = (size_t)WAVES * TN * (TN + 1) * sizeof(T);
     auto kern = backward_weight_kernel<T, ND, MT>;
+    if constexpr (ND == 2)
+        if (!off) kern = backward_weight_kernel<T, ND, MT, true>;
     if (lds > 48 * 1024)
         if (int rc = raise_lds_limit(reinterpret_cast<const void*>(kern), lds)) return rc;
     const dim3 grid((unsigned)P.nsplit * P.kV * P.nctiles * P.mchunks);

@@ -21,6 +21,19 @@ bool forward16_native(const Params& P) {
     return false;
 }
 
+// Channels per LDS pass, at most cchunk and a multiple of step, such that the passes of a group fall evenly on fsplit workgroups.
+inline int even_chunk(const Params& P, int cchunk, int step, int fsplit) {
+    for (int cc = cchunk; cc >= step; cc -= step) {
+        int n = 0;
+        for (int dg = 0; dg <= (P.Cg - 1) / P.cpg; ++dg) {
+            const int len = (P.Cg < (dg + 1) * P.cpg ? P.Cg : (dg + 1) * P.cpg) - dg * P.cpg;
+            n += (len + cc - 1) / cc;
+        }
+        if (n % fsplit == 0) return cc;
+    }
+    return cchunk;
+}
+
 // S = T: the float32 / float64 operator.  S = Bf16 / Fp16 (T = float): the tensors are in that
 // storage format and only the LDS-halo kernel serves them; where it cannot (halo too large, a layer
 // that wants the input-channel split), *declined is set and nothing is launched: the caller then
@@ -32,7 +45,8 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
     constexpr bool MX = sizeof(T) == 4;                 // forward_split_kernel; float64: forward_quad_kernel
     constexpr size_t MAX_LDS = MX ? MAX_FORWARD_LDS : 144 * 1024;       // dynamic LDS of the only workgroup of a CU
     constexpr int CM = MX ? FG : FQ;                    // channels of a weight slab
-    using WE = typename std::conditional<MX, typename Parts<typename std::conditional<MX, S, float>::type>::Elem, S>::type;      // packed weight element
+    using WS = typename std::conditional<MX, S, float>::type;
+    using WE = typename std::conditional<MX, typename Parts<WS>::Elem, S>::type;      // packed weight element
     auto slab_bytes = [](int kV, int Mp) {
         if constexpr (MX) return split_slab_elems<S>(kV, Mp) * sizeof(WE);
         else return forward_slab_elems<T>(kV, Mp) * sizeof(T);
@@ -96,9 +110,54 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             P.mchunks = mc;
         }
     }
-    const int nwp = shared ? SHARED_COLS : small ? 2 : WAVESH;      // column tiles of a block
     const size_t out_bytes = (size_t)P.N * P.C_out * P.outV * sizeof(T);
     const size_t wq_bound = align256(((size_t)chunk_slot<CM>(P.cpg, P.Cg, P.C_in - 1) + 1) * slab_bytes(P.kV, (mtiles_all + 7) / 8 * 8 * TN));
+    // Fewer positions still (`tiny`, position tiles of a block: 1 or 2): sixteen wavefronts to 32 positions or eight each to 64,
+    // and as many parts of the input channels as pay, while that is one workgroup to a CU.  By estimated time: 2.5 us for a pass,
+    // 2.0 (3-D) or 0.8 for a wavefront's step, 0.4 for a thread's cell to stage, 5 for joining parts, 2 for sixteen wavefronts.  One sample,
+    // float32, with / without: 2-D, 64 -> 64, 75 x 101: 20.4 / 33; 48 -> 64, 5x5, 70 x 76: 25 / 49; 3-D, 128 -> 32 at stride 1 2 2, 14 x 20 x 20:
+    // 65 / 102; two samples of 32 -> 16, 15 x 18 x 18: 30 / 55; 70 layers of 8 to 256 channels and 150 to 16 000
+    // positions, 2-D and 3-D, also in bfloat16: 0.85 of the time on average, 49 faster, at worst 1.06.
+    int tiny = 0;
+    if (small && MT <= 2 && forward_tiny()) {
+        const size_t room = ws_bytes > wq_bound ? (ws_bytes - wq_bound < FWD_PARTIAL_CAP ? ws_bytes - wq_bound : FWD_PARTIAL_CAP) : 0;
+        auto parts_fit = [&](int fs) {
+            return fs == 1 || (!S16 && fs <= forward_split() && fs <= FWD_MAX_SPLIT && (size_t)P.N * P.outV < FWD_SPLIT_POSITIONS && (size_t)fs * out_bytes <= room && fs * FG <= P.Cg);
+        };
+        // the longest workgroup of fs to a block of t position tiles, ts wavefronts to a position
+        auto estimate = [&](const Params& Pt, int t, int ts, int fs) {
+            double load[FWD_MAX_SPLIT] = {0}, worst = 0;
+            int k = 0;
+            const int cch = fs > 1 ? even_chunk(P, Pt.cchunk, FG, fs) : Pt.cchunk;
+            for (int dg = 0; dg <= (P.Cg - 1) / P.cpg; ++dg) {
+                const int len = (P.Cg < (dg + 1) * P.cpg ? P.Cg : (dg + 1) * P.cpg) - dg * P.cpg;
+                for (int c0 = 0; c0 < len; c0 += cch, ++k) {
+                    const int n = len - c0 < cch ? len - c0 : cch, steps = (P.kV + 1) / 2 * ((n + FG - 1) / FG), cells = (n + HaloCell<WS>::CH - 1) / HaloCell<WS>::CH;
+                    load[k % fs] += 2.5 + (ND == 3 ? 2.0 : 0.8) * ((steps + ts - 1) / ts) + 0.4 * cells * Pt.hvol / (t * ts * 64);
+                }
+            }
+            for (int z = 0; z < fs; ++z) worst = load[z] > worst ? load[z] : worst;
+            return worst + (fs > 1 ? 5 : 0) + (t * ts == 16 ? 2 : 0);
+        };
+        double best = 1e30;
+        {   // four wavefronts to a position: as many parts as fit, below
+            Params Pt = P;
+            if (plan_halo<T, ND>(Pt, MAX_LDS / 2, default_margin(), 1 << 30, sizeof(S), 2, false, FG, nullptr, 1, false)) {
+                int fs = 1;
+                while (parts_fit(fs * 2) && (long long)Pt.N * Pt.tiles * P.G * P.mchunks * fs * 2 <= 2 * cu_count()) fs *= 2;
+                best = estimate(Pt, 2, 4, fs);
+            }
+        }
+        for (int t = 1; t <= 2; ++t) {
+            Params Pt = P;
+            if (!plan_halo<T, ND>(Pt, MAX_LDS, default_margin(), 1 << 30, sizeof(S), t, true, FG, nullptr, 1, false)) continue;
+            for (int fs = 1; parts_fit(fs) && (long long)Pt.N * Pt.tiles * P.G * P.mchunks * fs <= cu_count(); fs *= 2) {
+                const double e = estimate(Pt, t, 16 / t, fs);
+                if (e < best) { best = e; tiny = t; fsplit = fs; }
+            }
+        }
+    }
+    const int nwp = shared ? SHARED_COLS : tiny ? tiny : small ? 2 : WAVESH;      // column tiles of a block
     {
         Params Pt = P;
         const bool tiled = plan_halo<T, ND>(Pt, MAX_LDS, default_margin(), 1 << 30, MX ? sizeof(S) : sizeof(T), nwp, false, FQ, nullptr, 1, !MX);
@@ -113,7 +172,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
         // share them; 4 or 16 there: 5 % slower, the same on average).  256 -> 16 channels, 28 x 28 positions: 44 unsplit, 22 split; 3x3x3,
         // 64 -> 16, 8 x 20 x 20: 71 / 37.  The join and a second workgroup on a CU cost more than short chains gain: 64 -> 64,
         // 112 x 112: 25 unsplit, 37 in two parts.
-        if (!S16 && tiled && forward_split() > 1 && (size_t)P.N * P.outV < FWD_SPLIT_POSITIONS && ws_bytes > wq_bound) {
+        if (!S16 && tiled && !tiny && forward_split() > 1 && (size_t)P.N * P.outV < FWD_SPLIT_POSITIONS && ws_bytes > wq_bound) {
             const size_t room = ws_bytes - wq_bound < FWD_PARTIAL_CAP ? ws_bytes - wq_bound : FWD_PARTIAL_CAP;
             while (fsplit * 2 <= FWD_MAX_SPLIT && fsplit * 2 <= forward_split() && tiles * P.G * P.mchunks * fsplit * 2 <= (small && MT < 4 ? 2 : 1) * cu_count() &&
                    (size_t)fsplit * 2 * out_bytes <= room && fsplit * 2 * (small ? 8 : 16) <= P.Cg)
@@ -151,6 +210,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             return tiled && (long long)Ph.N * Ph.tiles * Ph.G * Ph.mchunks <= 0x7fffffffLL ? SHARED_COLS : 0;
         }
         if (small) {
+            if (tiny) return plan_halo<T, ND>(Ph, MAX_LDS, m, 1 << 30, sizeof(S), tiny, true, FG, nullptr, 1, false) ? tiny : 0;
             // (half of the LDS: two workgroups share a CU)
             const bool tiled = plan_halo<T, ND>(Ph, MT == 4 ? MAX_LDS : MAX_LDS / 2, m, 1 << 30, sizeof(S), 2, false, FG, nullptr, 1, false) ||
                                plan_halo<T, ND>(Ph, MAX_LDS, m, 1 << 30, sizeof(S), 2, false, FG, nullptr, 1, false);
@@ -205,19 +265,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
         if (nw == 16 || ws_bytes < align256(wq_bytes) + (size_t)fsplit * out_bytes) fsplit = 1;
         if (nw && ws_bytes >= wq_bytes) {
             // channels per LDS pass such that every workgroup of a block gets the same number of passes
-            auto even_passes = [&](Params& Ph) {
-                auto chunks_of_group0 = [&](int cc) {
-                    int n = 0;
-                    for (int dg = 0; dg <= (P.Cg - 1) / P.cpg; ++dg) {
-                        const int len = (P.Cg < (dg + 1) * P.cpg ? P.Cg : (dg + 1) * P.cpg) - dg * P.cpg;
-                        n += (len + cc - 1) / cc;
-                    }
-                    return n;
-                };
-                const int step = Ph.cchunk % CM == 0 ? CM : FQ;
-                for (int cc = Ph.cchunk; cc >= step; cc -= step)
-                    if (chunks_of_group0(cc) % fsplit == 0) { Ph.cchunk = cc; break; }
-            };
+            auto even_passes = [&](Params& Ph) { Ph.cchunk = even_chunk(P, Ph.cchunk, Ph.cchunk % CM == 0 ? CM : FQ, fsplit); };
             if (fsplit > 1) even_passes(plans[0]);
             // Wider halos that one launch of the same kernel can serve as well (same workgroup shape and
             // position blocks); the choice among them is made on the device, see PlanChoice.  The
@@ -285,7 +333,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             const bool pairs = MX && !small && !shared && nw == WAVESH && MT <= 2 && P.kV > 1 && forward_small() && forward_slots() == 0 &&
                                (long long)plans[0].N * plans[0].tiles * plans[0].G * plans[0].mchunks * fsplit <= cu_count();
             // (the sums of the wavefronts that share positions)
-            size_t lds = small ? (size_t)3 * 2 * MT * 4096 : pairs ? (size_t)WAVESH * MT * 4096 : 0;
+            size_t lds = tiny ? (size_t)16 * MT * 4096 : small ? (size_t)3 * 2 * MT * 4096 : pairs ? (size_t)WAVESH * MT * 4096 : 0;
             for (int k = 0; k < pc.nplans; ++k) {
                 const size_t l = halo_lds(plans[k]);
                 if (l > lds) lds = l;
@@ -296,6 +344,8 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             typename std::conditional<MX, KernMx, KernQuad>::type kern = nullptr;
             if constexpr (MX) {
                 if (pairs) kern = MT == 1 ? forward_split_kernel<ND, 1, 16, 2, S> : forward_split_kernel<ND, 2, 16, 2, S>;
+                else if (tiny == 1) kern = MT == 1 ? forward_split_kernel<ND, 1, 16, 16, S> : forward_split_kernel<ND, 2, 16, 16, S>;
+                else if (tiny == 2) kern = MT == 1 ? forward_split_kernel<ND, 1, 16, 8, S> : forward_split_kernel<ND, 2, 16, 8, S>;
                 else if (small) kern = MT == 1 ? forward_split_kernel<ND, 1, 8, 4, S> : MT == 2 ? forward_split_kernel<ND, 2, 8, 4, S> : forward_split_kernel<ND, 4, 8, 4, S>;
                 else if (shared) { if constexpr (ND == 2) kern = MT == 8 ? forward_shared_kernel<ND, 8, S> : forward_shared_kernel<ND, 4, S>; }
                 else if (nw == 16) kern = MT == 1 ? forward_split_kernel<ND, 1, 16, 1, S> : forward_split_kernel<ND, 2, 16, 1, S>;
@@ -319,8 +369,8 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             int tsplit = 1;
             long long whole = 0;
             TailSplit ts = {0u, 0, 0};
-            if (fsplit == 1 && forward_tail_split()) {
-                const long long slots = forward_slots() ? forward_slots() : resident_workgroups(reinterpret_cast<const void*>(kern), (pairs ? 16 : shared || small ? 8 : nw) * 64, lds);
+            if (fsplit == 1 && !tiny && forward_tail_split()) {
+                const long long slots = forward_slots() ? forward_slots() : resident_workgroups(reinterpret_cast<const void*>(kern), (pairs || tiny ? 16 : shared || small ? 8 : nw) * 64, lds);
                 const long long rest = units % slots;
                 // tap geometry of a pass, in units of four channels' sampling and contraction (35 layers of 32 to 128
                 // channels whose last round is partly filled: 0.2 and 0.9 choose splits of the same time, no split takes 1.09 times as long)
@@ -390,7 +440,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                             plans[k].hext[0], plans[k].hext[1], plans[k].hext[2], plans[k].cchunk, pc.base[k]);
             }
             const unsigned* sel = pc.sel;
-            const int threads = (pairs ? 16 : shared || small ? 8 : nw) * 64, splits = tsplit > 1 ? tsplit : fsplit;
+            const int threads = (pairs || tiny ? 16 : shared || small ? 8 : nw) * 64, splits = tsplit > 1 ? tsplit : fsplit;
             int rc;
             if constexpr (MX) rc = launch_halo(kern, "forward halo kernel", grid, threads, lds, s, Ph, alts, sel, in, off, (const WE*)ws, w, bias, out, part, splits, (unsigned)whole, ts);
             else rc = launch_halo(kern, "forward halo kernel", grid, threads, lds, s, Ph, alts, sel, in, off, (const WE*)ws, bias, out, part, splits, (unsigned)whole, ts);

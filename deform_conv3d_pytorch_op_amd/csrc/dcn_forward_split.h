@@ -519,7 +519,7 @@ __device__ inline void store_tile(const Params& P, O* __restrict__ dst, const S*
 // channels, 27 taps, 200 704 positions, 0.49 ms: while a CU holds a workgroup its vector ALUs are busy 74 % of the cycles, its LDS
 // 53 %, 63 % of that bank conflicts of random offsets, its matrix units 28 %; 0.64 ms on the float32 instructions).  In
 // 2-D: operand latency.
-// TS > 1 (layers too small to fill the device otherwise): TS wavefronts share 32 positions, each takes a
+// TS > 1 (layers too small to fill the device otherwise; up to 16): TS wavefronts share 32 positions, each takes a
 // contiguous share of a pass's (tap pair, channel group) steps, and their sums meet in LDS -- a step of a lone
 // wavefront takes 0.8 to 1.8 us in 2-D, 2.0 to 2.4 us in 3-D (one to four row tiles), most of it latencies, so a small
 // layer's time is the length of that chain.
@@ -537,7 +537,7 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
     typedef typename PT::Vec Vec;
     typedef typename PT::Elem Elem;
     constexpr int TN = 32, WGS = NW * 64, NP = PT::NP;
-    constexpr bool EARLY = MT == 4;                     // weights requested before the step's samples: there are registers for it
+    constexpr bool EARLY = MT == 4 || TS >= 8;          // weights requested before the step's samples: there are registers for it
     extern __shared__ __align__(16) unsigned char smem_raw[];
     __shared__ int sNonFinite, sRedo;
     typedef typename HaloCell<S>::Vec Cell;
@@ -588,7 +588,7 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
                 const S* chan0 = in + ((size_t)n * P.C_in + cc0) * P.inV;      // workgroup-uniform
                 // this wavefront's steps of the pass: [first, last) of the (tap pair, group) list
                 const int steps = ntg * ngrp, first = TS > 1 ? steps * (wave % TS) / TS : 0, last = TS > 1 ? steps * (wave % TS + 1) / TS : steps;
-                const int tg_first = TS > 1 ? first / ngrp : 0, tg_end = TS > 1 ? (last + ngrp - 1) / ngrp : ntg;
+                const int tg_first = TS > 1 ? __builtin_amdgcn_readfirstlane(first / ngrp) : 0, tg_end = TS > 1 ? __builtin_amdgcn_readfirstlane((last + ngrp - 1) / ngrp) : ntg;
                 float ofs[ND];
                 load_pair_offsets<ND, S>(P, off_dg, min(tg_first, ntg - 1), q, pos, ofs, off == nullptr);
                 if (exact && threadIdx.x == 0) sNonFinite = 0;
@@ -655,7 +655,34 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
     if (valid && !results_stand<MT, S>(acc)) sRedo = 1;
     __syncthreads();
     if (__builtin_expect(sRedo, 0)) work(std::true_type{});
-    if constexpr (TS > 1) {
+    if constexpr (TS >= 8) {
+        // the sums of a position's TS wavefronts, [wavefront of the position][position tile][register][lane]: each adds up
+        // and writes a share of the registers
+        constexpr int NR = MT * MM::NACC, RW = NR / TS, PTS = NW / TS;
+        __syncthreads();
+        float* sum = reinterpret_cast<float*>(smem_raw);
+        const int part_of = wave % TS, tile = wave / TS;
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int r = 0; r < MM::NACC; ++r) sum[((part_of * PTS + tile) * NR + mt * MM::NACC + r) * 64 + lane] = acc[mt][r];
+        __syncthreads();
+        const size_t at = (size_t)n * P.C_out * P.outV + pos;
+#pragma unroll
+        for (int x = 0; x < RW; ++x) {
+            const int r = part_of * RW + x;                             // uniform
+            float v = 0.f;
+#pragma unroll
+            for (int k = 0; k < TS; ++k) v += sum[((k * PTS + tile) * NR + r) * 64 + lane];
+            const int m = (mchunk * MT + r / MM::NACC) * TN + MM::row(r % MM::NACC, 0) + q * 4;
+            if (valid && m < P.M) {
+                const size_t to = at + ((size_t)g * P.M + m) * P.outV;
+                if (U.split) part[(size_t)U.cz * P.N * P.C_out * P.outV + to] = v;      // (the bias is added when the parts are joined)
+                else out[to] = Store<S>::st(bias ? v + Store<S>::ld(bias[g * P.M + m]) : v);
+            }
+        }
+        return;
+    } else if constexpr (TS > 1) {
         // the sums of a position's TS wavefronts, added in their order: [TS - 1][position tile][register][lane]
         __syncthreads();
         float* sum = reinterpret_cast<float*>(smem_raw);

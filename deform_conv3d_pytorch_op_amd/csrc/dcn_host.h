@@ -228,6 +228,7 @@ inline int relayout(const Params& P, const T* w, T* wt, int channel_fastest, hip
 //   DCN_FORWARD_SLOTS=n    forward pass: plan the launch as if n workgroups ran at once (test hook)
 //   DCN_FORWARD_SHARED=0   forward pass, float32 and 16-bit: never share the sampled columns of a block among wavefronts
 //   DCN_FORWARD_SMALL=0    forward pass, float32 and 16-bit: never several wavefronts to a position
+//   DCN_FORWARD_TINY=0     ... never more than four
 //   DCN_SCATTER_BUDGET_KB  LDS per workgroup of the privatised scatter kernels (default 156: backward_fused_kernel, 144: the others)
 //   DCN_SCATTER=global     scatter grad-input with global atomics instead of the LDS-privatised kernel
 //   DCN_COORD=separate     grad_offset from the channels-last kernel instead of the fused LDS-halo kernel
@@ -342,6 +343,10 @@ static bool forward_small() {            // DCN_FORWARD_SMALL=0: the forward pas
     static const int v = [] { const char* e = getenv("DCN_FORWARD_SMALL"); return (e && atoi(e) == 0) ? 0 : 1; }();
     return v != 0;
 }
+static bool forward_tiny() {             // DCN_FORWARD_TINY=0: at most four wavefronts to a position
+    static const int v = [] { const char* e = getenv("DCN_FORWARD_TINY"); return (e && atoi(e) == 0) ? 0 : 1; }();
+    return v != 0;
+}
 static bool fused_pair() {              // DCN_FUSED_PAIR=0: float32 LDS cells of the fused backward kernel hold one channel each (64-bit)
     static const int v = [] { const char* e = getenv("DCN_FUSED_PAIR"); return (e && atoi(e) == 0) ? 0 : 1; }();
     return v != 0;
@@ -399,7 +404,7 @@ inline bool plan_halo(Params& P, size_t budget, int m, int max_chunk = 1 << 30, 
                bool smallest_halo = false, int chunk_mult = 0, const int* blocks = nullptr, int wmult = 1, bool table = true) {
     const int npos = waves * Mma<T>::TN;        // positions per workgroup, one column tile per wavefront
     int td[3] = {1, 1, 1};
-    if (ND == 3) { td[1] = 8; td[2] = 8; td[0] = npos / 64; }
+    if (ND == 3) { td[1] = td[2] = npos >= 64 ? 8 : 4; td[0] = npos / (td[1] * td[2]); }
     else         { td[2] = npos >= 128 ? 16 : 8; td[1] = npos / td[2]; }
     if (blocks) {                               // the block shape of another plan
         for (int a = 0; a < 3; ++a) td[a] = blocks[a];
