@@ -164,7 +164,6 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
         cz = (int)(r % (unsigned)cs);
     }
     const unsigned nt = (unsigned)P.N * P.tiles;
-    const float wcol = weight_bound(bounds, 1), wmax = weight_bound(bounds, 0);
     const int dg = item / nt;
     goff_atomic = cs > 1 ? 1 : goff_atomic;
 
@@ -248,6 +247,12 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
 
     for (int g = c_lo / P.Cg; g <= (c_hi - 1) / P.Cg; ++g) {
         const int rb = max(c_lo, g * P.Cg), re = min(c_hi, (g + 1) * P.Cg);
+        const int chunks = (re - rb + CCH - 1) / CCH, mine = (cz - chunk_no % cs + cs) % cs;      // this workgroup's: mine, mine + cs, ...
+        chunk_no += chunks;
+        if (mine >= chunks) continue;                                  // (uniform)
+        auto chunk_input = [&](int cc0) { return in + ((size_t)n * P.C_in + cc0) * P.inV; };
+        // (ahead of all else: the first latencies of a workgroup are a third of its time in layers of one chunk)
+        load_x(chunk_input(rb + mine * CCH), min(CCH, re - (rb + mine * CCH)));
         // Scale of the fixed-point terms, from the norms of grad_output over the output channels: a term is at most the
         // largest column norm of W times the largest norm (Cauchy-Schwarz), a cell receives at most kV times the former times the
         // sum of the norms over the block.
@@ -289,7 +294,7 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
         }
 #pragma unroll
         for (int w = 0; w < NW; ++w) gmaxb = max(gmaxb, __float_as_uint(sMax[w]));
-        const float gmax = __uint_as_float(gmaxb);
+        const float gmax = __uint_as_float(gmaxb), wcol = weight_bound(bounds, 1), wmax = weight_bound(bounds, 0);
         const float bound = 1.001f * wcol * __uint_as_float(nmaxb);    // (0.1 % for the rounding of the norms and of the contraction)
         const float bound_cell = 1.001f * wcol * (float)P.kV * nsum;
         // Without a finite bound, or where the squares of tiny weights or of a tiny grad_output underflow, the workgroup scatters
@@ -310,12 +315,8 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
         const double inv_scale = 1.0 / (double)scale;
         const Vec* gqg = gq + ((size_t)n * P.G + g) * steps * NP * 2 * P.outV;
 
-        const int chunks = (re - rb + CCH - 1) / CCH, mine = (cz - chunk_no % cs + cs) % cs;      // this workgroup's: mine, mine + cs, ...
-        chunk_no += chunks;
-        if (mine >= chunks) continue;                                  // (uniform)
         const size_t wslab = (size_t)ntiles * steps * NP * 64;
         auto chunk_weights = [&](int cc0) { return Wq + (size_t)chunk_slot<CCH>(P.cpg, P.Cg, cc0) * wslab; };
-        auto chunk_input = [&](int cc0) { return in + ((size_t)n * P.C_in + cc0) * P.inV; };
 
         Mma<float>::Acc acc[PT];
         float ofs[ND], prev[ND];
@@ -386,7 +387,6 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
                 }
             }
         };
-        load_x(chunk_input(rb + mine * CCH), min(CCH, re - (rb + mine * CCH)));
         contract(rb + mine * CCH, 0);
         store_x(chunk_input(rb + mine * CCH), min(CCH, re - (rb + mine * CCH)));
         __syncthreads();

@@ -16,8 +16,8 @@ template <int ND, typename S> inline FusedKern<ND, S> fused_kernel(int cch, int 
 }
 
 // S = T: the float32 / float64 operator.  S = Bf16 / Fp16 (T = float): input, weight, offset and
-// grad_output are in that storage format (the gradients are float), and only backward_fused_kernel serves
-// them; where it cannot, *declined is set and nothing is launched: the caller then widens the tensors and
+// grad_output are in that storage format (the gradients are float), and only the fused kernels serve
+// them; where they cannot, *declined is set and nothing is launched: the caller then widens the tensors and
 // runs the float32 operator.
 template <typename T, int ND, typename S>
 int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* off, const S* gout, T* gin,
@@ -53,8 +53,8 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
     const dim3 tgrid((P.inV + 31) / 32, (unsigned)(P.C_in + 31) / 32, (unsigned)P.N), tblock(32, 8);
 
     // 1) one kernel: scatter privatised in LDS + coordinate gradient from an LDS input halo.
-    // float32 layers whose LDS cells may be paired and 16-bit storage: backward_fused_kernel, with grad_output in
-    // operand order behind the channels-last regions of the workspace.  Others: backward_input_halo_kernel.
+    // float32 layers whose LDS cells may be paired and 16-bit storage, of more than one tap: backward_fused_kernel, with
+    // grad_output in operand order behind the channels-last regions of the workspace.  Others: backward_input_halo_kernel.
     const size_t gq_at = wbytes + 2 * tbytes, gq_bytes = fused_gout_need<S>(P.N, P.M, P.G, P.outV);
     const bool gq_fits = ws_bytes >= gq_at + gq_bytes + (tail_words ? BWD_TAIL + 256 : 0);
     // A halo of up to FUSED_HS cells gets the variant with that compile-time plane stride (the four
@@ -62,13 +62,14 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
     // Eight wavefronts per workgroup; four (half the positions, in the block shape with the smallest
     // halo) where only that fits, e.g. under stride 2.
     constexpr int FUSED_HS = sizeof(T) == 4 ? 2720 : 2112;
-    using Kern = void (*)(Params, PlanSet, const unsigned*, const T*, const T*, const T*, const T*, const float*, T*, T*, int, unsigned, int);
+    constexpr int FUSED_HS8 = 2016;     // plane stride of the 8-channel float instantiation with compile-time halo extents
+    using Kern = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const S*, const S*, const float*, T*, T*, int, unsigned, int);
     struct FusedPlan {
         Params Ph;
         Kern kern;                  // null: backward_fused_kernel
         const void* entry;
         int nw, cch, csplit, goff_atomic;
-        bool zero_goff;
+        bool zero_goff, wide;
         long long whole, items, slots;
         size_t lds;
         const S* wt;
@@ -84,8 +85,11 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             Params Ph = P;
             // float32: two channels per LDS cell as 32-bit fixed point while the terms one cell can receive
             // (positions of the block x taps) leave at least 17 bits below the largest possible term
-            const bool pair = sizeof(T) == 4 && fused_pair() && gq_fits && (long long)nw * TN * P.kV <= (1 << 14);
-            if (S16 && !pair) continue;
+            const bool pair = sizeof(T) == 4 && fused_pair() && (long long)nw * TN * P.kV <= (1 << 14);
+            // a single tap: a chunk is all staging and flush, which the smaller workgroups of backward_input_halo_kernel overlap
+            // better, and grad_output is used once per chunk (24 layers of one tap: backward_fused_kernel takes 1.09 times as long).
+            // Not where that kernel declines the output channels of a 16-bit layer.
+            const bool split = pair && gq_fits && (P.kV > 1 || (S16 && P.M > 256));
             int cch = 0;
             size_t lds = 0;
             Kern kern = nullptr;
@@ -98,7 +102,7 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
                 // per 8 or 5 per 16, the 27 of a 3x3x3 kernel 4 per 4 or 7 per 8); they are worth half as many positions to a halo
                 // (128 -> 128 channels, 3x3x3, stride 1 2 2: 2.60 ms with 8 channels and 128 positions, 2.80 with 4 and 256).
                 const int shapes[5][2] = {{8, 16}, {8, 8}, {4, 8}, {8, 4}, {4, 4}};
-                for (int k = 0; pair && attempt != 1 && k < 5 && !cch; ++k) {
+                for (int k = 0; split && attempt != 1 && k < 5 && !cch; ++k) {
                     const int tiles = shapes[k][0], cand = shapes[k][1];
                     if (tiles > nw) continue;
                     if (cand >= 8 && !(fused_chunk8() && seg >= 8 && passes(8) * 4 < passes(4) * 8)) continue;
@@ -117,22 +121,28 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
                     entry = reinterpret_cast<const void*>(fused_kernel<ND, S>(cand, tiles));
                 }
             }
-            if (pair && !cch) continue;
-            if constexpr (!S16) if (!pair) {
-            const size_t chb = 8 + sizeof(T);      // LDS bytes per channel and halo voxel: cell + input value
-            // 8 channels per chunk where that takes fewer MFMA passes per channel and the planes fit: the small halos of
-            // 2-D layers.  The float kernel with 8 channels per chunk keeps the input values bank-swizzled and wants the
-            // innermost halo extent a multiple of the four-channel groups per voxel.
+            if (split && !cch) continue;
+            bool wide = false;
+            if (!split) {
+            const size_t chb = (pair ? 4 : 8) + sizeof(T);      // LDS bytes per channel and halo voxel: cell + input value
+            // Channels per chunk: 8 where that takes fewer MFMA passes per channel (a pass holds TN / CCH
+            // taps: the 9 taps of a 3x3 kernel are 2 float passes per 4 channels or 3 per 8; the 27 of a
+            // 3x3x3 kernel 4 or 7) and the planes of 8 channels fit: the small halos of 2-D layers, and
+            // 3-D ones with paired cells.  16 (2-D, float, paired cells): two taps per pass -- the 9 taps of
+            // a 3x3 kernel are 5 passes per 16 channels instead of 6.  The float kernel with 8 channels
+            // per chunk keeps the input values bank-swizzled and wants the innermost halo extent a
+            // multiple of the four-channel groups per voxel.
             size_t tables = 0;
-            bool fixed = false;
-            for (int cand = 8; cand >= 4 && !cch; cand /= 2) {
-                if (cand == 8 && !(ND == 2 && nw == 8 && fused_chunk8() && seg >= 8 && passes(8) * 4 < passes(4) * 8)) continue;
+            bool fixed = false, special = false;
+            for (int cand = 16; cand >= 4 && !cch; cand /= 2) {
+                if (cand >= 8 && !((ND == 2 || pair) && nw == 8 && fused_chunk8() && seg >= 8 && passes(8) * 4 < passes(4) * 8)) continue;
+                if (cand == 16 && !(ND == 2 && pair && fused_chunk16() && seg >= 16 && passes(16) * 8 < passes(8) * 16)) continue;
                 Params Pc = P;
-                const int wmult = cand == 8 ? swizzle_groups<T, 8>() : 1;
+                const int wmult = cand == 16 ? 1 : cand == 8 ? swizzle_groups<T, 8>() : 1;
                 if (!plan_halo<T, ND>(Pc, scatter_budget(), m, 8, chb, nw, smallest, 0, nullptr, wmult)) continue;
                 const size_t tb = (size_t)Pc.hvol * 4;      // halo table
                 if ((long long)Pc.N * Pc.tiles * Pc.DG * 4 > 0x7fffffffLL) continue;
-                if (cand == 8) {
+                if (cand >= 8) {
                     if ((scatter_budget() - tb) / ((size_t)Pc.hstride * chb) < (size_t)cand) continue;
                 } else {
                     // A halo of up to FUSED_HS cells gets the variant with that compile-time plane stride
@@ -144,32 +154,54 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
                 cch = cand;
             }
             if (!cch) continue;
-            const bool eight = cch == 8;
+            const bool sixteen = cch == 16, eight = cch >= 8;
             if (fixed && !eight) Ph.hstride = FUSED_HS;
             // grad_output operand held in registers when its reduction steps fit: 32 per pass
             // (M <= 64 float, 128 double with 4-channel chunks)
-            const int ksteps = (P.M + Mma<T>::KL - 1) / Mma<T>::KL;
-            const int slot_regs = (Mma<T>::row(1, 0) - Mma<T>::row(0, 0) == 1) ? 4 : cch / 4;      // the kernel's RPS
-            const bool breg = ksteps <= Mma<T>::NACC / slot_regs * 8;
-            // float, 4-channel chunks: a second set of 32 registers takes the operand of up to 128 output channels
-            const bool breg2 = sizeof(T) == 4 && !eight && !breg && ksteps <= 64 && fused_breg2();
+            // (16-bit storage: a reduction step takes 8 output channels and an operand batch half as many steps)
+            const int KS = GcolGemm<T, S>::KS, halve = S16 ? 2 : 1;
+            const int ksteps = (P.M + KS - 1) / KS;
+            wide = eight && !sixteen && pair && ksteps <= 32 / halve;                     // the kernel's WIDE
+            const int slot_regs = (wide || sixteen) ? 8 : (Mma<T>::row(1, 0) - Mma<T>::row(0, 0) == 1) ? 4 : cch / 4;      // the kernel's RPS
+            const bool breg = ksteps <= Mma<T>::NACC / slot_regs * ((wide || sixteen) ? 16 : 8) / halve;
+            // float, 4-channel chunks: a second set of 32 registers takes the operand of up to 128 output channels (16-bit: 256)
+            const bool breg2 = sizeof(T) == 4 && !eight && !breg && ksteps <= 64 / halve && fused_breg2();
+            special = ND == 3 && eight && !sixteen && pair && wide && breg && fused_fixed_stride() && Ph.hext[1] == 14 && Ph.hext[2] == 14 &&
+                      Ph.hstride <= FUSED_HS8;
+            if (special) Ph.hstride = FUSED_HS8;
             lds = (size_t)cch * Ph.hstride * chb + tables;
-#define DCN_FUSED_C(CCH_, BREG_, HS_, NW_) backward_input_halo_kernel<T, ND, CCH_, true, BREG_, HS_, NW_, true>
-#define DCN_FUSED_B2(HS_, NW_) backward_input_halo_kernel<T, ND, 4, true, true, HS_, NW_, true, 2>
-            if (eight) {
-                if constexpr (ND == 2) kern = breg ? DCN_FUSED_C(8, true, 0, 8) : DCN_FUSED_C(8, false, 0, 8);
-            } else if (breg2) {
-                if constexpr (sizeof(T) == 4) {
-                    if (nw == 8) kern = fixed ? DCN_FUSED_B2(FUSED_HS, 8) : DCN_FUSED_B2(0, 8);
-                    else kern = fixed ? DCN_FUSED_B2(FUSED_HS, 4) : DCN_FUSED_B2(0, 4);
-                }
-            } else if (nw == 8)
-                kern = fixed && breg ? DCN_FUSED_C(4, true, FUSED_HS, 8) : fixed ? DCN_FUSED_C(4, false, FUSED_HS, 8) : DCN_FUSED_C(4, false, 0, 8);
-            else
-                kern = fixed && breg ? DCN_FUSED_C(4, true, FUSED_HS, 4) : fixed ? DCN_FUSED_C(4, false, FUSED_HS, 4) : DCN_FUSED_C(4, false, 0, 4);
+#define DCN_FUSED_C(CCH_, BREG_, HS_, NW_, PAIR_) backward_input_halo_kernel<T, ND, CCH_, true, (BREG_) || S16, HS_, NW_, true, PAIR_, 1, 0, 0, S>
+#define DCN_FUSED_B2(HS_, NW_, PAIR_) backward_input_halo_kernel<T, ND, 4, true, true, HS_, NW_, true, PAIR_, 2, 0, 0, S>
+            auto pick = [&](auto pair_tag) {
+                constexpr bool PR = decltype(pair_tag)::value;
+                if (sixteen) {
+                    if constexpr (ND == 2 && PR && sizeof(T) == 4) kern = breg ? DCN_FUSED_C(16, true, 0, 8, PR) : DCN_FUSED_C(16, false, 0, 8, PR);
+                } else if (eight) {
+                    if constexpr (ND == 2 || PR) kern = breg ? DCN_FUSED_C(8, true, 0, 8, PR) : DCN_FUSED_C(8, false, 0, 8, PR);
+                    // the halo of a 3x3x3 kernel at stride 1 and margin 2 under the default block of positions:
+                    // inner extents 14 x 14 and the plane stride fixed at compile time
+                    if constexpr (ND == 3 && PR && sizeof(T) == 4) {
+                        if (special) kern = backward_input_halo_kernel<T, ND, 8, true, true, FUSED_HS8, 8, true, true, 1, 14, 14, S>;
+                    }
+                } else if (breg2) {
+                    if constexpr (sizeof(T) == 4) {
+                        if (nw == 8) kern = fixed ? DCN_FUSED_B2(FUSED_HS, 8, PR) : DCN_FUSED_B2(0, 8, PR);
+                        else kern = fixed ? DCN_FUSED_B2(FUSED_HS, 4, PR) : DCN_FUSED_B2(0, 4, PR);
+                    }
+                } else if (nw == 8)
+                    kern = fixed && breg ? DCN_FUSED_C(4, true, FUSED_HS, 8, PR) : fixed ? DCN_FUSED_C(4, false, FUSED_HS, 8, PR) : DCN_FUSED_C(4, false, 0, 8, PR);
+                else
+                    kern = fixed && breg ? DCN_FUSED_C(4, true, FUSED_HS, 4, PR) : fixed ? DCN_FUSED_C(4, false, FUSED_HS, 4, PR) : DCN_FUSED_C(4, false, 0, 4, PR);
+            };
+            if constexpr (sizeof(T) == 4) {
+                if (pair) pick(std::true_type{});
+                else pick(std::false_type{});
+            } else
+                pick(std::false_type{});
 #undef DCN_FUSED_B2
 #undef DCN_FUSED_C
             if (!kern) continue;
+            if (S16 && !breg && !breg2) continue;       // 16-bit operands come from registers only
             entry = reinterpret_cast<const void*>(kern);
             }
             Ph.cchunk = cch;
@@ -210,7 +242,7 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             // and a 3x3x3 layer has 81 grad_offset elements per position and chunk); atomics in the 2-D ones
             fp.goff_atomic = ND == 2 && nchunks > 1 ? 1 : 0;
             fp.zero_goff = fp.goff_atomic || csplit > 1;
-            fp.whole = whole; fp.items = items; fp.slots = slots; fp.lds = lds; fp.wt = nullptr;
+            fp.wide = wide; fp.whole = whole; fp.items = items; fp.slots = slots; fp.lds = lds; fp.wt = nullptr;
             return true;
         }
         return false;
@@ -246,7 +278,7 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             c.wt = nullptr;
             if (!plan_fused(margins[k], c) || c.Ph.hvol > 3 * fp[0].Ph.hvol) continue;
             for (int e = 0; e < pc.nplans && !c.wt; ++e)
-                if (fp[e].cch == c.cch && !fp[e].kern == !c.kern) c.wt = fp[e].wt;
+                if (fp[e].cch == c.cch && fp[e].wide == c.wide && !fp[e].kern == !c.kern) c.wt = fp[e].wt;
             if (!c.wt) {
                 if ((size_t)copies * wbytes > tbytes) continue;
                 c.wt = reinterpret_cast<const S*>(reinterpret_cast<const char*>(in_cl) + (size_t)(copies - 1) * wbytes);
@@ -285,10 +317,10 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             const size_t slabs = (size_t)(fp[k].cch == 16 ? chunk_candidates<16>(P.cpg, P.Cg, P.C_in)
                                           : fp[k].cch == 8 ? chunk_candidates<8>(P.cpg, P.Cg, P.C_in)
                                                            : chunk_candidates<4>(P.cpg, P.Cg, P.C_in));
-            const size_t total = fp[k].kern ? packed_weight_elems<T>(P.M, P.kV, slabs, fp[k].cch)
+            const size_t total = fp[k].kern ? packed_weight_elems<T, S>(P.M, P.kV, slabs, fp[k].cch)
                                             : slabs * fused_tiles(P.kV, fp[k].cch) * fused_steps(P.M) * 64;      // threads
             PrepJob& job = prep.add(fp[k].kern ? PREP_PACK : PREP_FUSED_PACK, (unsigned)((total + 255) / 256 > 8192 ? 8192 : (total + 255) / 256));
-            job.variant = fp[k].cch;
+            job.variant = fp[k].wide ? 9 : fp[k].cch;
             job.dst = const_cast<S*>(fp[k].wt);
             any_fused = any_fused || !fp[k].kern;
         }
@@ -326,7 +358,7 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             launched |= alts.mask;
             if (trace_plans()) {
                 fprintf(stderr, "dcn backward_input_offset: launch for plans %#x: %d position tiles, %d channels per chunk%s, grid %lld (%lld unsplit, rest x %d), LDS %zu\n",
-                        alts.mask, fp[k].nw, fp[k].cch, fp[k].kern ? " (single cells)" : "", fp[k].whole + (fp[k].items - fp[k].whole) * fp[k].csplit, fp[k].whole,
+                        alts.mask, fp[k].nw, fp[k].cch, fp[k].kern ? " (halo kernel)" : "", fp[k].whole + (fp[k].items - fp[k].whole) * fp[k].csplit, fp[k].whole,
                         fp[k].csplit, lds);
                 for (int e = 0; e < pc.nplans; ++e)
                     if ((alts.mask >> e) & 1u)
@@ -337,9 +369,8 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
                 if (int rc = raise_lds_limit(fp[k].entry, lds)) return rc;
             const dim3 grid((unsigned)(fp[k].whole + (fp[k].items - fp[k].whole) * fp[k].csplit));
             if (fp[k].kern) {
-                if constexpr (!S16)
-                    hipLaunchKernelGGL(fp[k].kern, grid, dim3(fp[k].nw * 64), lds, s, fp[k].Ph, alts, (const unsigned*)sel, in, off, fp[k].wt, gout,
-                                       (const float*)bounds, gin, goff, fp[k].csplit, (unsigned)fp[k].whole, fp[k].goff_atomic);
+                hipLaunchKernelGGL(fp[k].kern, grid, dim3(fp[k].nw * 64), lds, s, fp[k].Ph, alts, (const unsigned*)sel, in, off, fp[k].wt, gout,
+                                   (const float*)bounds, gin, goff, fp[k].csplit, (unsigned)fp[k].whole, fp[k].goff_atomic);
             } else {
                 if constexpr (sizeof(T) == 4) {
                     typedef const typename Parts<S>::Vec* Ops;

@@ -57,9 +57,9 @@ inline size_t align256(size_t v) { return (v + 255) / 256 * 256; }
 constexpr int TAP_PAD = 8;      // zero tap slabs behind the last group: an MFMA pass may start up to 7 taps before the end
 // Elements of the per-chunk weight slabs of the fused backward kernel (pack_backward_weight, chunks of
 // `cch` channels) for `slabs` slabs.
-template <typename T> inline size_t packed_weight_elems(int M, int kV, size_t slabs, int cch) {
+template <typename T, typename S = T> inline size_t packed_weight_elems(int M, int kV, size_t slabs, int cch) {
     const int TP = Mma<T>::TN / cch;
-    return slabs * ((kV + TP - 1) / TP) * (size_t)gcol_slab_steps<T>(M) * 64;
+    return slabs * ((kV + TP - 1) / TP) * (size_t)gcol_slab_steps<T, S>(M) * 64 * (std::is_same<S, T>::value ? 1 : 4);
 }
 // Upper bound of chunk_slot<cch>(cpg, Cg, c) + 1 over the channels: the slabs a per-chunk weight
 // layout occupies.  cpg = 0: the channels per deformable group are not known (the first workspace
@@ -73,7 +73,9 @@ template <typename T> inline size_t bwd_data_weight_bytes(int M, int Cg, int kV,
     const size_t C_in = (size_t)Cg * G;
     const size_t packed4 = packed_weight_elems<T>(M, kV, slab_bound(C_in, G, cpg, 4), 4);
     const size_t packed8 = packed_weight_elems<T>(M, kV, slab_bound(C_in, G, cpg, 8), 8);
-    const size_t packed = packed4 > packed8 ? packed4 : packed8;
+    const size_t packed16 = packed_weight_elems<T>(M, kV, slab_bound(C_in, G, cpg, 16), 16);
+    size_t packed = packed4 > packed8 ? packed4 : packed8;
+    if (packed16 > packed) packed = packed16;
     size_t bytes = (plain > packed ? plain : packed) * sizeof(T);
     for (int cch = 4; sizeof(T) == 4 && cch <= 16; cch *= 2) {
         const size_t parts = slab_bound(C_in, G, cpg, cch) * fused_slab_ops<float>(M, kV, cch) * 16;

@@ -125,8 +125,31 @@ __host__ __device__ inline int chunk_candidate(int cpg, int Cg, int y) {     // 
     return y / cps * seg + y % cps * CCH;
 }
 
+// Operands of the grad-column GEMM of the fused backward kernel.  S = T: one value per lane and
+// reduction step, v_mfma_f32_32x32x2_f32 / v_mfma_f64_16x16x4_f64 (KS = KL output channels per
+// step).  S = Bf16 / Fp16 (T = float): four values per lane and step -- the output channels
+// 8 * step + 4 * (lane / 32) + 0..3 -- for v_mfma_f32_32x32x8_bf16 / _f16, which accumulate in float
+// and leave the result in the registers of the float instruction (KS = 8 output channels per step).
+template <typename T, typename S> struct GcolGemm {
+    static constexpr int KS = Mma<T>::KL;
+    typedef T Op;
+    __device__ static inline typename Mma<T>::Acc mma(Op a, Op b, typename Mma<T>::Acc c) { return Mma<T>::mma(a, b, c); }
+};
+template <> struct GcolGemm<float, Bf16> {
+    static constexpr int KS = 8;
+    typedef Mma16<Bf16>::Vec Op;
+    __device__ static inline Mma<float>::Acc mma(Op a, Op b, Mma<float>::Acc c) { return Mma16<Bf16>::mma(a, b, c); }
+};
+template <> struct GcolGemm<float, Fp16> {
+    static constexpr int KS = 8;
+    typedef Mma16<Fp16>::Vec Op;
+    __device__ static inline Mma<float>::Acc mma(Op a, Op b, Mma<float>::Acc c) { return Mma16<Fp16>::mma(a, b, c); }
+};
 // reduction steps of a weight slab's pass: a multiple of the largest operand batch
-template <typename T> __host__ __device__ inline int gcol_slab_steps(int M) { return ((M + Mma<T>::KL - 1) / Mma<T>::KL + 15) / 16 * 16; }
+template <typename T, typename S> __host__ __device__ inline int gcol_slab_steps(int M) {
+    constexpr bool S16 = !std::is_same<S, T>::value;
+    return S16 ? ((M + 7) / 8 + 7) / 8 * 8 : ((M + Mma<T>::KL - 1) / Mma<T>::KL + 15) / 16 * 16;
+}
 
 // One block of 256 threads chooses the halo plan of the launches that follow (see PlanChoice).
 // It reads 32 runs of 256 consecutive offset entries spread evenly over the tensor (all of a small
@@ -192,14 +215,20 @@ __device__ inline void choose_plan(const PlanChoice& pc, const S* __restrict__ o
     }
 }
 
+// WIDE (float, CCH = 8): row j of a pass holds (tap, channel) = (2 * (j / 16) + (j / 4) % 2,
+// 4 * ((j / 8) % 2) + j % 4) instead of (j / CCH, j % CCH): the MFMA then leaves all eight channels
+// of a tap in one lane (fused_row_tap / fused_row_channel).
+// S = Bf16 / Fp16: Wp[slab][pass][k][lane][r] = W[m = 8 * k + 4 * q + r][...], four values per lane and step.
 // Block `block` of `blocks` blocks of 256 threads.
-template <typename T, int CCH>
-__device__ inline void pack_backward_weight(const Params& P, const T* __restrict__ W, T* __restrict__ Wp, unsigned block, unsigned blocks) {
+template <typename T, int CCH, bool WIDE = false, typename S = T>
+__device__ inline void pack_backward_weight(const Params& P, const S* __restrict__ W, S* __restrict__ Wp, unsigned block, unsigned blocks) {
     using MM = Mma<T>;
+    constexpr bool S16 = !std::is_same<S, T>::value;
+    constexpr int PER = S16 ? 4 : 1;                    // values per lane and reduction step
     constexpr int TN = MM::TN, KL = MM::KL, TP = TN / CCH;
     const int npass = (P.kV + TP - 1) / TP;
-    const int kst = gcol_slab_steps<T>(P.M);                    // operand batches are 8 or 16 reduction steps
-    const size_t per_chunk = (size_t)npass * kst * 64;
+    const int kst = gcol_slab_steps<T, S>(P.M);                 // operand batches are 8 or 16 (16-bit: 4 or 8) reduction steps
+    const size_t per_chunk = (size_t)npass * kst * 64 * PER;
     const size_t total = (size_t)chunk_candidates<CCH>(P.cpg, P.Cg, P.C_in) * per_chunk;
     for (size_t i = (size_t)block * 256 + threadIdx.x; i < total; i += (size_t)blocks * 256) {
         const int c0 = chunk_candidate<CCH>(P.cpg, P.Cg, (int)(i / per_chunk));      // candidate first channel of a chunk
@@ -207,10 +236,12 @@ __device__ inline void pack_backward_weight(const Params& P, const T* __restrict
         if ((c0 - seg_b) % CCH) continue;
         const int seg_e = min((c0 / P.cpg + 1) * P.cpg, (c0 / P.Cg + 1) * P.Cg);
         const size_t r = i % per_chunk;
-        const int lane = (int)(r % 64), k = (int)((r / 64) % kst), pass = (int)(r / 64 / kst);
+        const int sub = (int)(r % PER);
+        const int lane = (int)((r / PER) % 64), k = (int)((r / PER / 64) % kst), pass = (int)(r / PER / 64 / kst);
         const int q = lane / TN, j = lane % TN;
-        const int m = k * KL + q, tap = pass * TP + j / CCH, c = c0 + j % CCH, g = c0 / P.Cg;
-        T v = T();
+        const int jt = WIDE ? 2 * (j / 16) + (j / 4) % 2 : j / CCH, jc = WIDE ? 4 * ((j / 8) % 2) + j % 4 : j % CCH;
+        const int m = S16 ? k * 8 + q * 4 + sub : k * KL + q, tap = pass * TP + jt, c = c0 + jc, g = c0 / P.Cg;
+        S v = S();
         if (m < P.M && tap < P.kV && c < seg_e) v = W[(((size_t)g * P.M + m) * P.Cg + (c - g * P.Cg)) * P.kV + tap];
         Wp[(size_t)chunk_slot<CCH>(P.cpg, P.Cg, c0) * per_chunk + r] = v;
     }
@@ -868,13 +899,24 @@ __device__ inline float weight_bound(const float* __restrict__ bounds, int which
 // of a channel becomes an immediate offset of the LDS instructions instead of address arithmetic.
 // PACKW: the weights come in the per-chunk lane order of pack_backward_weight instead of
 // [g][tap][m][channel].
-// (float32 layers whose cells may be paired and 16-bit storage: backward_fused_kernel.)
-template <typename T, int ND, int CCH, bool COORD, bool BREG, int HS, int NW, bool PACKW = false, int BS = 1>
+// CCH = 16 (float, 2-D layers whose halo leaves room for 16 channel planes): two taps per pass, so the
+// nine taps of a 3x3 kernel take 5 passes per 16 channels instead of 6, with half as many chunks to
+// zero, stage and flush; a lane then holds eight channels of each of the two taps (0..3 and 8..11 in
+// lane group 0, 4..7 and 12..15 in lane group 1) and walks them as two tap slots.
+// PAIR (float only): the cells hold two channels each as 32-bit fixed point (LdsCell<float>::add2):
+// half the LDS atomics and two thirds of the LDS bytes per channel.  The terms are scaled such
+// that (positions of the block x taps) of the largest possible one -- all that a cell can receive
+// -- still fit 31 bits; the host allows it only while that leaves enough bits below that term.
+// S: storage format of input, offset, weight and grad_output (Bf16 / Fp16 with T = float: the grad-column
+// GEMM then runs on the 16-bit matrix instructions, see GcolGemm; requires BREG and PACKW); the
+// gradients are written as T.
+template <typename T, int ND, int CCH, bool COORD, bool BREG, int HS, int NW, bool PACKW = false, bool PAIR = false, int BS = 1,
+          int HE1 = 0, int HE2 = 0, typename S = T>
 __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, PlanSet alts, const unsigned* __restrict__ sel,
-                                                                  const T* __restrict__ in,
-                                                                  const T* __restrict__ off,
-                                                                  const T* __restrict__ Wt,
-                                                                  const T* __restrict__ gout,
+                                                                  const S* __restrict__ in,
+                                                                  const S* __restrict__ off,
+                                                                  const S* __restrict__ Wt,
+                                                                  const S* __restrict__ gout,
                                                                   const float* __restrict__ bounds,
                                                                   T* __restrict__ gin, T* __restrict__ goff, int csplit,
                                                                   unsigned whole, int goff_atomic) {
@@ -883,22 +925,37 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
     using MM = Mma<T>;
     using Cell = typename LdsCell<T>::type;
     constexpr int TN = MM::TN, KL = MM::KL, NC = 1 << ND, NACC = MM::NACC;
+    constexpr bool S16 = !std::is_same<S, T>::value;
+    using GG = GcolGemm<T, S>;
+    using Op = typename GG::Op;                         // what a lane supplies to one reduction step
+    constexpr int KS = GG::KS;                          // output channels per reduction step
+    static_assert(!S16 || (BREG && PACKW && sizeof(T) == 4), "16-bit operands: packed weights, grad_output in registers");
     constexpr int TP = TN / CCH;                        // taps per MFMA pass
-    constexpr int RPS = (MM::row(1, 0) - MM::row(0, 0) == 1) ? 4 : CCH / 4;     // registers that share a tap
+    // WIDE (paired cells, 8-channel chunks): the weight rows are ordered such that a lane receives
+    // all eight channels of a tap -- lane group q the taps q and 2 + q of a pass -- instead of four
+    // channels of each of four taps, with the other four in the other lane group: the geometry of a
+    // (tap, position) is then worked out once per eight channels, not once per lane group.
+    constexpr bool WIDE = PAIR && CCH == 8 && BREG;      // (with the grad_output operand in registers: measured slower without)
+    // (16-channel chunks, float: two taps per pass, a lane holds eight channels of each -- 0..3 and 8..11 or 4..7 and 12..15)
+    constexpr int RPS = (WIDE || CCH == 16) ? 8 : (MM::row(1, 0) - MM::row(0, 0) == 1) ? 4 : CCH / 4;   // registers that share a tap
     constexpr int NS = NACC / RPS;                      // tap slots per lane and pass
     // (tap of the pass, channel of the chunk) behind accumulator register r of lane group qq
-    auto row_tap = [](int r, int qq) { return MM::row(r, qq) / CCH; };
-    auto row_ch = [](int r, int qq) { return MM::row(r, qq) % CCH; };
+    auto row_tap = [](int r, int qq) { return WIDE ? 2 * (r / 8) + qq : MM::row(r, qq) / CCH; };
+    auto row_ch = [](int r, int qq) { return WIDE ? r % 8 : MM::row(r, qq) % CCH; };
     static_assert(TN % CCH == 0 && CCH % 4 == 0 && NACC % RPS == 0, "unsupported channel chunk");
-    constexpr int CPL = CCH;                            // cell planes
+    static_assert(!PAIR || (sizeof(T) == 4 && RPS % 2 == 0), "paired cells are a float32 layout");
+    constexpr int CPL = PAIR ? CCH / 2 : CCH;           // cell planes
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int hs = HS ? HS : H.hstride;
-    const int he1 = H.hext[1], he2 = H.hext[2];
+    // HE1, HE2 > 0 fix the two inner halo extents at compile time (the host then launches this
+    // instantiation only for plans with exactly these extents): the distances between the corners of a
+    // sample become immediate offsets of the LDS instructions instead of per-corner address arithmetic
+    const int he1 = HE1 ? HE1 : H.hext[1], he2 = HE2 ? HE2 : H.hext[2];
     Cell* sG = reinterpret_cast<Cell*>(smem_raw);                                       // [CPL][hstride]
     T* sIn = reinterpret_cast<T*>(sG + (size_t)CPL * hs);                               // [hstride][CCH] if COORD: channels of a voxel side by side
     unsigned* sTab = reinterpret_cast<unsigned*>(sIn + (COORD ? (size_t)CCH * hs : 0));   // [hvol]
     constexpr int WGS = NW * 64;                        // threads per workgroup
-    __shared__ float sRed[NW];
+    __shared__ float sRed[NW], sSum[NW], sAmax[NW];
     __shared__ int sNonFinite;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int j = lane % TN, q = lane / TN;
@@ -918,7 +975,7 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
         cz = r % (unsigned)cs;
     }
     const unsigned nt = (unsigned)P.N * P.tiles;
-    const float wbound = weight_bound(bounds, 0);
+    const float wbound = weight_bound(bounds, PAIR ? 1 : 0);
     const int dg = item / nt;
     // an item that several workgroups share needs the atomics (the host has zero-filled grad_offset);
     // the only owner of an item stores the running sum over its chunks instead, unless the host asks for
@@ -942,7 +999,7 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
     for (int a = 0; a < ND; ++a) ibf[a] = (T)ib[a];
 
     const int c_lo = dg * P.cpg, c_hi = c_lo + P.cpg;
-    const T* off_dg = off + ((size_t)n * P.DG + dg) * P.kV * ND * P.outV;
+    const S* off_dg = off + ((size_t)n * P.DG + dg) * P.kV * ND * P.outV;
     T* goff_dg = goff + ((size_t)n * P.DG + dg) * P.kV * ND * P.outV;
     bool first_chunk = true;                        // grad_offset without atomics: the first channel chunk stores, later ones add
     int chunk_no = 0;
@@ -953,10 +1010,10 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
     for (int g = c_lo / P.Cg; g <= (c_hi - 1) / P.Cg; ++g) {
         const int rb = max(c_lo, g * P.Cg), re = min(c_hi, (g + 1) * P.Cg);
         // wave-uniform base (scalar registers) + 32-bit lane offset of the B operand grad_output[m][pos]
-        constexpr int AB = 8;                           // reduction steps per operand batch (NS * AB ride on a pass: 64 output channels)
-        const T* gbase = gout + ((size_t)n * P.C_out + (size_t)g * P.M) * P.outV;
+        constexpr int AB = ((WIDE || CCH == 16) ? 16 : 8) / (S16 ? 2 : 1);      // reduction steps per operand batch (NS * AB ride on a pass: 64 output channels, 16-bit 128)
+        const S* gbase = gout + ((size_t)n * P.C_out + (size_t)g * P.M) * P.outV;
         const unsigned b_off = (unsigned)q * P.outV + pos;
-        const size_t gstep = (size_t)KL * P.outV;
+        const size_t gstep = (size_t)KS * P.outV;
         // Reduction step k of this lane reads grad_output[k * KL + q][pos]: the row base advances in
         // scalar registers, clamped at the last real step (the further steps of a batch meet zero
         // weight rows and re-read that step; a lane whose row of the last step lies past M reads
@@ -965,12 +1022,41 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
         // address arithmetic per lane.  Lanes outside the volume read a clamped position (their
         // columns are never used).  No load is masked: a masked load becomes a conditional one,
         // issued alone with a full wait behind it.
-        const int klast = (P.M + KL - 1) / KL - 1;
+        const int klast = (P.M + KS - 1) / KS - 1;
         const unsigned b_byte = b_off * (unsigned)sizeof(T);
         const unsigned b_byte_last = (klast * KL + q < P.M ? b_off : pos) * (unsigned)sizeof(T);
-        T b_reg[BREG ? NS * AB * BS : 1];
-        float sabs = 0.f;                           // sum_m |grad_output| of this lane's position (its q share)
-        if constexpr (BREG) {
+        Op b_reg[BREG ? NS * AB * BS : 1];
+        float sabs = 0.f;                           // sum_m |grad_output| of this lane's position (its q share); PAIR: of the squares
+        float amax = 0.f;                           // PAIR: largest |grad_output| seen (squares of tiny values underflow)
+        if constexpr (S16) {
+            // four output channels per lane and step: rows 8 * k + 4 * q + r of grad_output at this lane's
+            // position; rows past M (last step only: zero weights there) re-read row M - 1
+            int kl = klast;
+            asm volatile("" : "+s"(kl));
+            unsigned row_off[4], row_off_last[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                row_off[r] = ((unsigned)(4 * q + r) * P.outV + pos) * (unsigned)sizeof(S);
+                const int rl = min(kl * 8 + 4 * q + r, P.M - 1) - kl * 8;
+                row_off_last[r] = ((unsigned)rl * P.outV + pos) * (unsigned)sizeof(S);
+            }
+            const char* gk = reinterpret_cast<const char*>(gbase);
+#pragma unroll
+            for (int k = 0; k < NS * AB * BS; ++k) {
+                float g4[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    g4[r] = Store<S>::ld(*reinterpret_cast<const S*>(gk + (k >= kl ? row_off_last[r] : row_off[r])));
+                gk += k < kl ? gstep * sizeof(S) : (size_t)0;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const bool counts = valid && k <= kl && k * 8 + 4 * q + r < P.M;
+                    sabs += counts ? (PAIR ? g4[r] * g4[r] : fabsf(g4[r])) : 0.f;
+                    if constexpr (PAIR) amax = counts ? fmaxf(amax, fabsf(g4[r])) : amax;
+                }
+                b_reg[k] = Mma16<S>::pack(g4);          // (exact: the values are 16-bit already)
+            }
+        } else if constexpr (BREG) {
             // held unmasked (rows past M meet zero weight rows, columns outside the volume are never
             // used): a masked load becomes a conditional one, issued alone with a full wait behind it
             // (the last step passes through an empty asm: the per-step selects derived from it are
@@ -988,7 +1074,8 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
             for (int k = 0; k < NS * AB * BS; ++k) {
                 const float bk = (float)b_reg[k];
                 const bool counts = valid && (k < kl || (k == kl && kl * KL + q < P.M));
-                sabs += counts ? fabsf(bk) : 0.f;
+                sabs += counts ? (PAIR ? bk * bk : fabsf(bk)) : 0.f;
+                if constexpr (PAIR) amax = counts ? fmaxf(amax, fabsf(bk)) : amax;
             }
         } else {
             // unconditional loads, eight in flight, masked when they are summed (a masked load
@@ -1006,8 +1093,9 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
                     const int kk_ = k0 + k;
                     const float bk = (float)bv[k];
                     const bool counts = valid && (kk_ < klast || (kk_ == klast && klast * KL + q < P.M));
-                    sabs += counts ? fabsf(bk) : 0.f;
-                    }
+                    sabs += counts ? (PAIR ? bk * bk : fabsf(bk)) : 0.f;
+                    if constexpr (PAIR) amax = counts ? fmaxf(amax, fabsf(bk)) : amax;
+                }
             }
         }
         // fixed-point exponent of this (workgroup, convolution group): terms are bounded by
@@ -1018,29 +1106,63 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
         unsigned sbits = __float_as_uint(fabsf(sabs));
 #pragma unroll
         for (int sh = 1; sh < TN; sh <<= 1) sbits = max(sbits, (unsigned)__shfl_xor((int)sbits, sh));
+        // paired cells: also the sum over the block's positions of the norm of grad_output over the
+        // output channels (every lane of a position holds its full sum of squares by now)
+        float nsum = PAIR ? sqrtf(sabs) : 0.f;
+        if constexpr (PAIR) {
+#pragma unroll
+            for (int sh = 1; sh < TN; sh <<= 1) nsum += __shfl_xor(nsum, sh);
+#pragma unroll
+            for (int sh = 1; sh < 64; sh <<= 1) amax = fmaxf(amax, __shfl_xor(amax, sh));
+        }
         __syncthreads();
-        if (lane == 0) sRed[wave] = __uint_as_float(sbits);
+        if (lane == 0) { sRed[wave] = __uint_as_float(sbits); sSum[wave] = nsum; sAmax[wave] = amax; }
         __syncthreads();
         unsigned smaxb = 0u;
+        float ssum = 0.f, gmax = 0.f;
 #pragma unroll
-        for (int w8 = 0; w8 < NW; ++w8) smaxb = max(smaxb, __float_as_uint(sRed[w8]));
+        for (int w8 = 0; w8 < NW; ++w8) { smaxb = max(smaxb, __float_as_uint(sRed[w8])); ssum += sSum[w8]; gmax = fmaxf(gmax, sAmax[w8]); }
         int ex = 0;
-        const float bound = 8.f * wbound * __uint_as_float(smaxb);
+        // paired cells: |term| <= largest column norm of W x largest norm of grad_output over the
+        // output channels (0.1 % slack for the rounding of those two and of the MFMA sums)
+        const float bound = PAIR ? 1.001f * wbound * sqrtf(__uint_as_float(smaxb)) : 8.f * wbound * __uint_as_float(smaxb);
+        // paired cells: all that one cell can receive.  A (tap, position) spreads at most |grad column| over
+        // its corners (their weights add up to one), so a cell's terms add up to at most the sum over the
+        // block's positions and the taps of that bound -- far less than (number of terms) x (largest term)
+        // when a few positions carry most of grad_output
+        const float bound_cell = PAIR ? 1.001f * wbound * (float)P.kV * ssum : 0.f;
         // the LDS cells need a finite bound; without one this workgroup scatters through the far path
         // (float cells need the exponent; and with either cell type a corner that carries weight zero
         // would receive 0 * inf = NaN where the reference adds nothing)
-        const bool cells_ok = bound < 3.0e38f;            // false for NaN
+        // (and a block whose grad_output is so small that its squares underflow: the bound is then not
+        // trustworthy, and the workgroup takes the far path too rather than rounding its gradient away)
+        const bool cells_ok = bound < 3.0e38f && bound_cell < 3.0e38f && !(PAIR && gmax > 0.f && gmax < 1e-18f);            // false for NaN
         if (bound > 0.f && bound < 3.0e38f) (void)frexpf(bound, &ex);
-        const double scale = ldexp(1.0, 30 - ex), inv_scale = ldexp(1.0, ex - 30);
+        double scale = ldexp(1.0, 30 - ex), inv_scale = ldexp(1.0, ex - 30);
+        float scale32 = 1.f;
+        if constexpr (PAIR) {
+            // a single term stays below 2^22 (the float conversion of add2) and all the terms a cell can
+            // receive together below 2^31 (their roundings, half a unit each for at most NW * TN * kV
+            // terms, fit the one per cent of slack)
+            if (bound > 0.f && cells_ok) {
+                const double s_term = 4194304.0 / (double)bound;
+                const double s_cell = bound_cell > 0.f ? 2147483648.0 / (double)bound_cell : s_term;
+                scale = 0.99 * (s_term < s_cell ? s_term : s_cell);
+            } else
+                scale = 1.0;
+            scale32 = (float)(scale < 1e30 ? scale : 1e30);       // (a denormal bound: keep the scale a finite float)
+            scale = (double)scale32;                 // the flush divides by exactly what the terms were multiplied with
+            inv_scale = 1.0 / scale;
+        }
 
         for (int cc0 = rb; cc0 < re; cc0 += CCH) {
             if ((chunk_no++) % cs != cz) continue;          // another workgroup's chunk (uniform)
             const int nch = min(CCH, re - cc0);
             if (threadIdx.x == 0) sNonFinite = 0;
             __syncthreads();                        // the previous chunk's flush is done
-            for (int c = 0; c < nch; ++c)
+            for (int c = 0; c < (PAIR ? (nch + 1) / 2 : nch); ++c)
                 for (int v = threadIdx.x; v < H.hvol; v += WGS) sG[c * hs + v] = 0;      // all-zero bits in either cell type
-            if constexpr (COORD) halo_stage_interleaved<T, CCH, WGS>(P, H, in + ((size_t)n * P.C_in + cc0) * P.inV, nch, sTab, sIn, &sNonFinite);
+            if constexpr (COORD) halo_stage_interleaved<T, CCH, WGS, S>(P, H, in + ((size_t)n * P.C_in + cc0) * P.inV, nch, sTab, sIn, &sNonFinite);
             __syncthreads();
             // Non-finite input values in this halo: the branch-free sampler reads the cell next to a
             // collapsed corner with weight 0, and 0 * inf would be NaN where the reference never
@@ -1055,22 +1177,24 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
             // the matrix pipe works behind the vector work of the scatter instead of before it.
             // Operands arrive in batches of AB reduction steps, loaded one tap slot ahead of use.
             constexpr int MPR = AB / RPS;                              // MFMAs per accumulator register walked
-            const int ksteps = (P.M + KL - 1) / KL;
+            const int ksteps = (P.M + KS - 1) / KS;
+            // (weights are addressed in operands: one value, or with 16-bit storage four values, per lane and step)
+            const Op* Wo = reinterpret_cast<const Op*>(Wt);
             const size_t wstep = PACKW ? (size_t)64 : (size_t)KL * P.Cgp;
-            const size_t wpass = PACKW ? (size_t)gcol_slab_steps<T>(P.M) * 64 : (size_t)TP * P.Mp * P.Cgp;   // weights of one pass
-            const T* wchunk = PACKW ? Wt + (size_t)chunk_slot<CCH>(P.cpg, P.Cg, cc0) * ((P.kV + TP - 1) / TP) * wpass
-                                     : Wt + ((size_t)g * P.kV * P.Mp) * P.Cgp + (cc0 - g * P.Cg);      // uniform; lanes add a_off
+            const size_t wpass = PACKW ? (size_t)gcol_slab_steps<T, S>(P.M) * 64 : (size_t)TP * P.Mp * P.Cgp;   // weights of one pass
+            const Op* wchunk = PACKW ? Wo + (size_t)chunk_slot<CCH>(P.cpg, P.Cg, cc0) * ((P.kV + TP - 1) / TP) * wpass
+                                     : Wo + ((size_t)g * P.kV * P.Mp) * P.Cgp + (cc0 - g * P.Cg);      // uniform; lanes add a_off
             // (k0 passes through an empty asm: what is derived from it is then computed where it is
             // used instead of being hoisted out of the loops into hundreds of long-lived registers)
-            auto load_batch = [&](T* a_nx, T* b_nx, const T* wp, int k0) {      // rows past M are zero padding
+            auto load_batch = [&](Op* a_nx, Op* b_nx, const Op* wp, int k0) {      // rows past M are zero padding
                 asm volatile("" : "+s"(k0));
-                const T* wb = wp + (size_t)k0 * wstep;                // one 64-bit product per batch; the row offsets below are loop invariants
+                const Op* wb = wp + (size_t)k0 * wstep;                // one 64-bit product per batch; the row offsets below are loop invariants
                 const char* gk = reinterpret_cast<const char*>(gbase + (size_t)min(k0, klast) * gstep);
 #pragma unroll
                 for (int k = 0; k < AB; ++k) {
                     a_nx[k] = (wb + (unsigned)k * (unsigned)wstep)[a_off];
                     if constexpr (!BREG) {
-                        b_nx[k] = *reinterpret_cast<const T*>(gk + (k0 + k >= klast ? b_byte_last : b_byte));
+                        b_nx[k] = *reinterpret_cast<const Op*>(gk + (k0 + k >= klast ? b_byte_last : b_byte));
                         gk += k0 + k < klast ? gstep * sizeof(T) : (size_t)0;
                     }
                 }
@@ -1080,8 +1204,8 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
             // (two operand sets that swap roles from batch to batch, two batches per loop trip: copying
             // "next" into "current" costs 2 * AB register moves per batch whenever the register
             // allocator cannot merge the sets, on the same issue port as the MFMAs)
-            auto gemm_tail = [&](typename MM::Acc& dd, const T* wp, int k_begin) {
-                T a_s[2][AB], b_s[2][AB];
+            auto gemm_tail = [&](typename MM::Acc& dd, const Op* wp, int k_begin) {
+                Op a_s[2][AB], b_s[2][AB];
                 load_batch(a_s[0], b_s[0], wp, k_begin);
                 int k0 = k_begin;
                 if (PACKW && ksteps - k_begin >= 96) {
@@ -1096,14 +1220,14 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
                     // grad_output rows: two scalar adds per load instead of a dozen scalar instructions,
                     // which a wavefront has to issue between two MFMAs.
                     const int kfast_end = P.M % KL == 0 ? klast + 1 : klast;      // steps [0, kfast_end) load without a clamp
-                    auto load_fast = [&](T* a_nx, T* b_nx, int k0f) {
+                    auto load_fast = [&](Op* a_nx, Op* b_nx, int k0f) {
                         asm volatile("" : "+s"(k0f));
-                        const T* wb = wp + (size_t)k0f * wstep;
+                        const Op* wb = wp + (size_t)k0f * wstep;
                         const char* gk = reinterpret_cast<const char*>(gbase + (size_t)k0f * gstep);
 #pragma unroll
                         for (int k = 0; k < AB; ++k) {
                             a_nx[k] = (wb + (unsigned)k * (unsigned)wstep)[a_off];
-                            b_nx[k] = *reinterpret_cast<const T*>(gk + b_byte);
+                            b_nx[k] = *reinterpret_cast<const Op*>(gk + b_byte);
                             gk += gstep * sizeof(T);
                         }
                     };
@@ -1120,27 +1244,27 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
                         for (; k0 + 3 * AB <= kfast_end; k0 += 2 * AB) {
                             load_fast(a_s[1], b_s[1], k0 + AB);
 #pragma unroll
-                            for (int k = 0; k < AB; ++k) dd = MM::mma(a_s[0][k], b_s[0][k], dd);
+                            for (int k = 0; k < AB; ++k) dd = GG::mma(a_s[0][k], b_s[0][k], dd);
                             deal();
                             load_fast(a_s[0], b_s[0], k0 + 2 * AB);
 #pragma unroll
-                            for (int k = 0; k < AB; ++k) dd = MM::mma(a_s[1][k], b_s[1][k], dd);
+                            for (int k = 0; k < AB; ++k) dd = GG::mma(a_s[1][k], b_s[1][k], dd);
                             deal();
                         }
                     }
                     for (; k0 + AB < ksteps; k0 += 2 * AB) {
                         load_batch(a_s[1], b_s[1], wp, min(k0 + AB, k_last));
 #pragma unroll
-                        for (int k = 0; k < AB; ++k) dd = MM::mma(a_s[0][k], b_s[0][k], dd);
+                        for (int k = 0; k < AB; ++k) dd = GG::mma(a_s[0][k], b_s[0][k], dd);
                         deal();
                         load_batch(a_s[0], b_s[0], wp, min(k0 + 2 * AB, k_last));
 #pragma unroll
-                        for (int k = 0; k < AB; ++k) dd = MM::mma(a_s[1][k], b_s[1][k], dd);
+                        for (int k = 0; k < AB; ++k) dd = GG::mma(a_s[1][k], b_s[1][k], dd);
                         deal();
                     }
                     if (k0 < ksteps) {
 #pragma unroll
-                        for (int k = 0; k < AB; ++k) dd = MM::mma(a_s[0][k], b_s[0][k], dd);
+                        for (int k = 0; k < AB; ++k) dd = GG::mma(a_s[0][k], b_s[0][k], dd);
                     }
                     return;
                 }
@@ -1148,30 +1272,30 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
                     load_batch(a_s[1], b_s[1], wp, k0 + AB);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int k = 0; k < AB; ++k) dd = MM::mma(a_s[0][k], b_s[0][k], dd);
+                    for (int k = 0; k < AB; ++k) dd = GG::mma(a_s[0][k], b_s[0][k], dd);
                     __builtin_amdgcn_sched_barrier(0);
                     if (k0 + 2 * AB < ksteps) load_batch(a_s[0], b_s[0], wp, k0 + 2 * AB);
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-                    for (int k = 0; k < AB; ++k) dd = MM::mma(a_s[1][k], b_s[1][k], dd);
+                    for (int k = 0; k < AB; ++k) dd = GG::mma(a_s[1][k], b_s[1][k], dd);
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 if (k0 < ksteps) {
 #pragma unroll
-                    for (int k = 0; k < AB; ++k) dd = MM::mma(a_s[0][k], b_s[0][k], dd);
+                    for (int k = 0; k < AB; ++k) dd = GG::mma(a_s[0][k], b_s[0][k], dd);
                 }
             };
             // register-resident operand: the batches of a pass past those that ride on the tap slots
-            auto gemm_tail_reg = [&](typename MM::Acc& dd, const T* wp) {
+            auto gemm_tail_reg = [&](typename MM::Acc& dd, const Op* wp) {
                 if constexpr (BREG && BS > 1) {
-                    T a_x[2][AB];
+                    Op a_x[2][AB];
                     if (NS * AB < ksteps) load_batch(a_x[0], nullptr, wp, NS * AB);
 #pragma unroll
                     for (int kb = NS; kb < NS * BS; ++kb) {
                         if (kb * AB < ksteps) {
                             if ((kb + 1) * AB < ksteps && kb + 1 < NS * BS) load_batch(a_x[(kb + 1 - NS) & 1], nullptr, wp, (kb + 1) * AB);
 #pragma unroll
-                            for (int k = 0; k < AB; ++k) dd = MM::mma(a_x[(kb - NS) & 1][k], b_reg[kb * AB + k], dd);
+                            for (int k = 0; k < AB; ++k) dd = GG::mma(a_x[(kb - NS) & 1][k], b_reg[kb * AB + k], dd);
                         }
                     }
                 }
@@ -1181,10 +1305,10 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
 #pragma unroll
                 for (int ts = 0; ts < NS; ++ts) {
                     if (ts * AB < ksteps) {
-                        T a_cu[AB];
+                        Op a_cu[AB];
                         load_batch(a_cu, nullptr, wchunk, ts * AB);
 #pragma unroll
-                        for (int k = 0; k < AB; ++k) d_next = MM::mma(a_cu[k], b_reg[ts * AB + k], d_next);
+                        for (int k = 0; k < AB; ++k) d_next = GG::mma(a_cu[k], b_reg[ts * AB + k], d_next);
                     }
                 }
                 gemm_tail_reg(d_next, wchunk);
@@ -1223,9 +1347,9 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
                 const int dq = row_tap(ts * RPS, q) - row_tap(ts * RPS, 0);
                 const int dqc = tu + dq < P.kV ? dq : 0;
                 const unsigned lo = (unsigned)dqc * ND * P.outV + pos;
-                const T* ob = off_dg + (size_t)tu * ND * P.outV;
+                const S* ob = off_dg + (size_t)tu * ND * P.outV;
 #pragma unroll
-                for (int a = 0; a < ND; ++a) o_nx[a] = (ob + (size_t)a * P.outV)[lo];
+                for (int a = 0; a < ND; ++a) o_nx[a] = Store<S>::ld((ob + (size_t)a * P.outV)[lo]);
                 if constexpr (RMW) {
                     if (rmw_prev) {
                         const T* gb = goff_dg + (size_t)tu * ND * P.outV;
@@ -1282,7 +1406,7 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
                 const bool more = tap0 + TP < P.kV;                    // a pass follows: its MFMAs ride along
                 int kz = 0;                                            // an opaque zero, for the same reason
                 asm volatile("" : "+s"(kz));
-                const T* wnext = wchunk + (size_t)(tap0 / TP + 1) * wpass;
+                const Op* wnext = wchunk + (size_t)(tap0 / TP + 1) * wpass;
                 if constexpr (!BREG) { if (more && ksteps > NS * AB) gemm_tail(d_next, wnext, NS * AB); }
                 else { if (more) gemm_tail_reg(d_next, wnext); }
 #pragma unroll
@@ -1290,7 +1414,7 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
                     // slots past the last tap (only in the last pass, which feeds no further MFMAs)
                     if (tap0 + row_tap(ts * RPS, 0) >= P.kV) continue;
                     const int tap = tap0 + row_tap(ts * RPS, q);
-                    T a_cu[AB], b_cu[AB];
+                    Op a_cu[AB], b_cu[AB];
                     const T* ofs = o_buf[ts & 1];
                     const T* kdf = kd_buf[ts & 1];
                     const bool do_mma = more && ts * AB < ksteps;      // uniform
@@ -1401,7 +1525,7 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
                         if (do_mma) {
 #pragma unroll
                             for (int k = h * (AB / RH); k < (h + 1) * (AB / RH); ++k)
-                                d_next = MM::mma(a_cu[k], BREG ? b_reg[ts * AB + k] : b_cu[k], d_next);
+                                d_next = GG::mma(a_cu[k], BREG ? b_reg[ts * AB + k] : b_cu[k], d_next);
                         }
                         if constexpr (COORD) {
 #pragma unroll
@@ -1437,12 +1561,22 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
                     }
                     if (near) {
                         Cell* cp = sG + base;
+                        if constexpr (PAIR) {
 #pragma unroll
-                        for (int rr = 0; rr < RPS; ++rr) {
-                            const double gs = LdsCell<T>::pre(gv[rr], scale);
-                            const int cl = row_ch(ts * RPS + rr, q);
+                            for (int rr = 0; rr < RPS; rr += 2) {          // consecutive registers hold consecutive channels
+                                const float g0 = (float)gv[rr] * scale32, g1 = (float)gv[rr + 1] * scale32;
+                                const int pl = row_ch(ts * RPS + rr, q) / 2;
 #pragma unroll
-                            for (int i = 0; i < NC; ++i) LdsCell<T>::add(cp + coff[i] + cl * hs, (double)cw[i], gs);
+                                for (int i = 0; i < NC; ++i) LdsCell<float>::add2(cp + coff[i] + pl * hs, (float)cw[i], g0, g1);
+                            }
+                        } else {
+#pragma unroll
+                            for (int rr = 0; rr < RPS; ++rr) {
+                                const double gs = LdsCell<T>::pre(gv[rr], scale);
+                                const int cl = row_ch(ts * RPS + rr, q);
+#pragma unroll
+                                for (int i = 0; i < NC; ++i) LdsCell<T>::add(cp + coff[i] + cl * hs, (double)cw[i], gs);
+                            }
                         }
                     }
                     if constexpr (COORD && ND == 3) {
@@ -1494,10 +1628,10 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
 #pragma unroll
                                 for (int i = 0; i < NC; ++i) atomic_add(gc + t.idx[i], fcw[i] * g1);
                                 if constexpr (COORD) {
-                                    const T* ic = in + chan;
+                                    const S* ic = in + chan;
                                     T v[NC];
 #pragma unroll
-                                    for (int i = 0; i < NC; ++i) v[i] = g1 * ic[t.idx[i]];
+                                    for (int i = 0; i < NC; ++i) v[i] = g1 * Store<S>::ld(ic[t.idx[i]]);
                                     if constexpr (ND == 3) {
                                         const T fl = t.f[0], gl = (T)1 - fl, fh = t.f[1], gh = (T)1 - fh, fw = t.f[2], gw = (T)1 - fw;
                                         const T c00 = v[0] * gw + v[1] * fw, c01 = v[2] * gw + v[3] * fw;
@@ -1542,10 +1676,23 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
             for (int v = threadIdx.x; v < H.hvol; v += WGS) {
                 const unsigned gv = sTab[v];
                 if (gv == ~0u) continue;            // halo cell outside the volume: never touched
-                for (int c = 0; c < nch; ++c) {
-                    const Cell cell = sG[c * hs + v];
-                    if (cell != (Cell)0)
-                        atomic_add(gin + ((size_t)n * P.C_in + cc0 + c) * P.inV + gv, (T)LdsCell<T>::value(cell, inv_scale));
+                if constexpr (PAIR) {
+                    for (int c = 0; c < nch; c += 2) {
+                        const Cell cell = sG[(c / 2) * hs + v];
+                        if (cell != (Cell)0) {
+                            float v0, v1;
+                            LdsCell<float>::value2(cell, inv_scale, v0, v1);
+                            T* gp = gin + ((size_t)n * P.C_in + cc0 + c) * P.inV + gv;
+                            if (v0 != 0.f) atomic_add(gp, (T)v0);
+                            if (c + 1 < nch && v1 != 0.f) atomic_add(gp + P.inV, (T)v1);
+                        }
+                    }
+                } else {
+                    for (int c = 0; c < nch; ++c) {
+                        const Cell cell = sG[c * hs + v];
+                        if (cell != (Cell)0)
+                            atomic_add(gin + ((size_t)n * P.C_in + cc0 + c) * P.inV + gv, (T)LdsCell<T>::value(cell, inv_scale));
+                    }
                 }
             }
         }

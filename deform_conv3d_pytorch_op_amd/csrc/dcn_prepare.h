@@ -13,7 +13,7 @@ namespace dcn {
 
 enum PrepKind { PREP_PACK, PREP_FUSED_PACK, PREP_GOUT, PREP_PLAN, PREP_BOUNDS, PREP_ZERO, PREP_LAST };
 struct PrepJob {
-    int kind, variant;          // PACK, FUSED_PACK: channels per chunk
+    int kind, variant;          // PACK, FUSED_PACK: channels per chunk; PACK: + 1 for the wide row order
     unsigned first;             // first block; the job's blocks reach to the next job's first
     const void* src;
     void* dst;
@@ -130,11 +130,11 @@ __global__ __launch_bounds__(256) void backward_prepare_kernel(Params P, PlanCho
     const unsigned block = blockIdx.x - job.first, blocks = next - job.first;
     switch (job.kind) {
         case PREP_PACK: {
-            if constexpr (std::is_same<S, T>::value) {
-                T* dst = static_cast<T*>(job.dst);
-                if (job.variant == 8) pack_backward_weight<T, 8>(P, W, dst, block, blocks);
-                else pack_backward_weight<T, 4>(P, W, dst, block, blocks);
-            }
+            S* dst = static_cast<S*>(job.dst);
+            if (job.variant == 16) { if constexpr (sizeof(T) == 4) pack_backward_weight<T, 16, false, S>(P, W, dst, block, blocks); }
+            else if (job.variant == 9) { if constexpr (sizeof(T) == 4) pack_backward_weight<T, 8, true, S>(P, W, dst, block, blocks); }
+            else if (job.variant == 8) pack_backward_weight<T, 8, false, S>(P, W, dst, block, blocks);
+            else pack_backward_weight<T, 4, false, S>(P, W, dst, block, blocks);
             break;
         }
         case PREP_FUSED_PACK: {
