@@ -1,5 +1,6 @@
 // Backward pass to the weight: plans and launches.
 #include "dcn_host.h"
+#include <cmath>
 
 namespace dcn {
 
@@ -37,6 +38,55 @@ void bww_plan(const Params& Pin, int& MT, int& mchunks, int& nct, int& nsplit, l
     if (split > 256) split = 256;
     if (split < 1) split = 1;
     nsplit = (int)split;
+}
+
+// Channel tiles of the convolution group that has the most, times taps.
+inline int split_items(const Params& P) {
+    int most = 0;
+    for (int g = 0; g < P.G; ++g) {
+        int n = 0;
+        for (int dg = g * P.Cg / P.cpg; dg <= ((g + 1) * P.Cg - 1) / P.cpg; ++dg) {
+            const int cb = g * P.Cg > dg * P.cpg ? g * P.Cg : dg * P.cpg, ce = (g + 1) * P.Cg < (dg + 1) * P.cpg ? (g + 1) * P.Cg : (dg + 1) * P.cpg;
+            n += (ce - cb + 31) / 32;
+        }
+        most = n > most ? n : most;
+    }
+    return most * P.kV;
+}
+// backward_weight_split_kernel takes layers of more than 32 output channels to a group, with items for the four wavefronts of a
+// workgroup (not a single tap of few channels) and work for the device: 2.5 slabs to a resident wavefront.  Below, the longer
+// preparation and the fuller grid that backward_weight_kernel makes of few items decide (us of a training step, that kernel against
+// this one: 45 -> 75 channels, one tap, 15 000 positions 699 : 774; 32 -> 432, 5x5, 612 positions 259 : 265; 32 -> 80, 3x3x3, 1176 positions
+// 177 : 184; 96 -> 128, 3x3, 7296 positions 157 : 162); above, this one wins (32 -> 113, 3x3x3, 3456 positions 202 : 183; 16 -> 80, 16 000
+// positions 228 : 203; 12 -> 57, 62 000 positions 750 : 698).  Its wavefronts write a partial tile each: about one round of resident
+// workgroups, as long as the tiles (written and read at about 8 TB/s) cost less than the longer runs of slabs.
+struct SplitPlan { int MT, mchunks, igroups, nsplit; };     // nsplit 0: not a layer for it, or no room
+template <int ND>
+SplitPlan split_plan(const Params& P, size_t room) {
+    SplitPlan c = {};
+    const int items = split_items(P);
+    c.MT = P.M > 64 ? 4 : 2;
+    c.mchunks = ((P.M + 31) / 32 + c.MT - 1) / c.MT;
+    c.igroups = (items + WAVES - 1) / WAVES;
+    const double resident = (double)resident_workgroups(c.MT == 4 ? reinterpret_cast<const void*>(backward_weight_split_kernel<ND, 4>)
+                                                         : reinterpret_cast<const void*>(backward_weight_split_kernel<ND, 2>), WG, 0);
+    const long long nslabs = (long long)P.N * (row_steps(P.outV) / 2);
+    const double other = (double)c.igroups * c.mchunks * P.G;
+    if (P.M <= 32 || items < WAVES || (double)items * c.mchunks * P.G * (double)nslabs < 2.5 * WAVES * resident) return c;
+    const size_t one = (size_t)P.kV * P.C_out * P.Cg * sizeof(float);
+    long long most = (long long)(room / one);
+    if (most > 256) most = 256;
+    if (most > nslabs) most = nslabs;
+    double best = 0;
+    for (long long s = 1; s <= most; ++s) {
+        const double load = other * (double)s / resident, rounds = load > 1 ? ceil(load) : 0.4 + 0.6 * load;
+        const double t = (double)((nslabs + s - 1) / s) * rounds * 4 + (double)s * (double)one * 2 / 8e6;
+        if (s > 1 && t >= best) continue;
+        best = t;
+        c.nsplit = (int)s;
+    }
+    if (other * c.nsplit > 2147483647.0) c.nsplit = 0;
+    return c;
 }
 
 // Workgroups of backward_weight_kernel that the device holds at once (0 if the query fails).
@@ -130,7 +180,19 @@ int backward_weight_plan(const Params& Pin, const S* in, const S* gout, void* ws
         P.nsplit = (int)split;
         if ((long long)P.nsplit * other > 0x7fffffffLL) return DCN_OK;
     }
-    const size_t ibytes = align256((size_t)P.N * P.C_in * P.inV * sizeof(S)), obytes = align256((size_t)P.N * P.C_out * P.outV * sizeof(S));
+    const size_t ibytes = align256((size_t)P.N * P.C_in * P.inV * sizeof(S));
+    size_t obytes = align256((size_t)P.N * P.C_out * P.outV * sizeof(S));
+    c.igroups = 0;
+    c.gout = gout;
+    if constexpr (sizeof(S) == 4) {
+        const size_t rbytes = align256(row_operand_bytes(P.N, P.C_out, P.outV));
+        const size_t used = ibytes + rbytes + (bias ? (size_t)P.N * last_strips(P.outV) * P.C_out * sizeof(T) : 0) + 256;
+        const SplitPlan sp = split_plan<ND>(P, ws && ws_bytes > used ? ws_bytes - used : 0);
+        if (sp.nsplit) {
+            obytes = rbytes;
+            c.MT = sp.MT; c.igroups = sp.igroups; P.mchunks = sp.mchunks; P.nsplit = sp.nsplit;
+        }
+    }
     const size_t pbytes = align256((size_t)P.nsplit * P.kV * P.C_out * P.Cg * sizeof(T));
     c.nsums = (int)(P.N * last_strips(P.outV));
     if (!ws || ws_bytes < ibytes + obytes + pbytes + (bias ? (size_t)c.nsums * P.C_out * sizeof(T) : 0)) return refuse(DCN_E_WORKSPACE, "workspace too small");
@@ -141,16 +203,30 @@ int backward_weight_plan(const Params& Pin, const S* in, const S* gout, void* ws
     c.partial = reinterpret_cast<T*>(p + ibytes + obytes);
     c.sums = bias ? reinterpret_cast<T*>(p + ibytes + obytes + pbytes) : nullptr;
     prep.channels_last(in, c.in_cl, P.C_in, P.inV, P.N, nullptr);
-    prep.channels_last(gout, c.gout_cl, P.C_out, P.outV, P.N, c.sums);
+    if (c.igroups) prep.rows(gout, c.gout_cl, P.C_out, P.outV, P.N, c.sums);
+    else prep.channels_last(gout, c.gout_cl, P.C_out, P.outV, P.N, c.sums);
     return DCN_OK;
+}
+
+template <int ND, int MT>
+int launch_bwd_weight_split(const WeightCall<float, float>& c, const float* off, hipStream_t s) {
+    const Params& P = c.P;
+    const dim3 grid((unsigned)((long long)c.igroups * P.mchunks * P.G * P.nsplit));
+    auto kern = backward_weight_split_kernel<ND, MT>;
+    if constexpr (ND == 2)
+        if (!off) kern = backward_weight_split_kernel<ND, MT, true>;
+    hipLaunchKernelGGL(kern, grid, dim3(WG), 0, s, P, (const float*)c.in_cl, off, c.gout, reinterpret_cast<const Parts<float>::Vec*>(c.gout_cl), c.partial, (unsigned)c.igroups);
+    return check_launch("backward_weight_split_kernel");
 }
 
 template <typename T, int ND, typename S>
 int backward_weight_run(const WeightCall<T, S>& c, const S* off, T* gw, T* gb, bool accumulate, hipStream_t s) {
     const Params& P = c.P;
     if constexpr (std::is_same<S, T>::value) {
-        int rc;
-        switch (c.MT) {
+        int rc = DCN_OK;
+        if constexpr (sizeof(T) == 4)
+            if (c.igroups) rc = c.MT == 4 ? launch_bwd_weight_split<ND, 4>(c, off, s) : launch_bwd_weight_split<ND, 2>(c, off, s);
+        if (!c.igroups) switch (c.MT) {
             case 1: rc = launch_bwd_weight<T, ND, 1>(c, off, s); break;
             case 2: rc = launch_bwd_weight<T, ND, 2>(c, off, s); break;
             default: rc = launch_bwd_weight<T, ND, 4>(c, off, s); break;

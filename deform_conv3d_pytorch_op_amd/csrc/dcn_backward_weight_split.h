@@ -1,0 +1,300 @@
+// Backward pass to the weight of the float32 operator, for layers of more than 32 output channels to a group (split_plan).
+//
+//   gW[g*M+m][cl][tap] += sum_{n,pos} grad_output[n][g*M+m][pos] * sample(in[n][g*Cg+cl], tap, pos)
+//
+// replaces the second deformable_im2col + Sgemm(beta=1) of deform3d/lib/deform_conv3d_cuda.cpp:283-320.
+//
+// The reduction runs over positions.  A wavefront samples 32 channels of one tap: lane (j, q) takes channel c0 + j at eight
+// consecutive positions of a step of 16 -- the input is channels-last, so a corner is one coalesced 128-byte read of the
+// lane group -- and those eight samples are the lane's operand of v_mfma_f32_32x32x16_bf16 as they stand: three bfloat16
+// parts (dcn_forward_split.h).  The other operand, the rows of grad_output, comes from the preparing launch in operand order
+// (prep_rows); the four wavefronts of a workgroup work taps or channel tiles of their own on the same positions and share it
+// through LDS, two steps of it in turn.  The geometry of a slab of 32 positions is worked out once by the position-owning
+// lanes and handed to the channel lanes through a wavefront-private record: byte offset of the low corner and the corner
+// weights.  The low corner is at most size - 2, so that the other corners lie at fixed strides (scalar bases of their own, one
+// address per lane and position for all of them) and a corner past the rim is never read.
+// An accumulator stays in registers for the whole run of a wavefront, which writes one partial tile;
+// reduce_weight_partials_kernel sums the splits (deterministic, no atomics).  Results that are not finite or too small for the
+// parts are formed once more from the values themselves.
+// The instruction cuts what lies below the last places of a product off towards minus infinity, and a chain of hundreds of
+// steps adds that up: the products of a step are summed from zero and then added, and every second split samples with its sign
+// turned round and turns its tile back.  Error of grad_weight against float64 (2-norm; 64 -> 64, 3x3x3, 4 x 16 x 56 x 56, whose rounded
+// coordinates make 2.0e-6 of it; 64 -> 64, 3x3, no offsets): float32 instructions 2.00e-6 and 1.84e-7, one chain 2.39e-6 and
+// 2.51e-7, with sums of a step 2.15e-6 and 3.66e-7, with the signs as well 2.00e-6 and 1.51e-7.
+//
+// What bounds it: the corner reads.  64 -> 64 channels, 3x3x3, 4 x 16 x 56 x 56 positions: 12.2 GB through the vector caches,
+// whose data return is busy 96 % of the time (8.5 GB from L2), the matrix units 20 %, the vector units 40 %.  backward_weight_kernel
+// with the float32 instructions kept the matrix units busy half of the time and read grad_output once per wavefront: with rows
+// straight from L2 this kernel was no faster in 3-D (678 us against 633) and 13 % faster in 2-D.  us, that kernel -> this one: 256 -> 256,
+// 3x3, 8 x 56 x 56: 332 -> 240; 512 -> 512 in two groups, 3x3, 4 x 28 x 28: 105 -> 80; 128 -> 128, 3x3x3, 2 x 16 x 56 x 56
+// (stride 2): 1022 -> 860; 64 -> 64 as above: 633 -> 600; 64 -> 64, 3x3, no offsets, 25 088 positions: 33 -> 25.
+// The preparing launch pays 4 to 30 us of it back (three halves of the bytes of a channels-last copy).
+#pragma once
+#include "dcn_forward_split.h"
+
+namespace dcn {
+
+constexpr unsigned ROW_SLAB = 32;                       // positions of a slab: two steps
+__host__ __device__ inline unsigned row_steps(unsigned V) { return (V + ROW_SLAB - 1) / ROW_SLAB * 2; }
+// grad_output in operand order: [n][step][part][q][output channel], 16 bytes (eight positions) each, zero past the volume
+inline size_t row_operand_bytes(int N, int C_out, size_t V) { return (size_t)N * row_steps((unsigned)V) * Parts<float>::NP * 2 * C_out * 16; }
+
+// MT row tiles to a workgroup.  PLAIN: a plain convolution (off is null): samples at integer coordinates are their low corner alone.
+// Grid: igroups * mchunks * G * nsplit workgroups.  An item is a tap of a channel tile of the convolution group, tap fastest.
+template <int ND, int MT, bool PLAIN = false>
+__global__ __launch_bounds__(WG, MT == 4 ? 3 : 4) void backward_weight_split_kernel(Params P, const float* __restrict__ in_cl, const float* __restrict__ off,
+                                                                                         const float* __restrict__ gout,
+                                                                                         const typename Parts<float>::Vec* __restrict__ rows,
+                                                                                         float* __restrict__ partial, unsigned igroups) {
+    typedef float T;
+    using MM = Mma<float>;
+    using PT = Parts<float>;
+    typedef typename PT::Vec Vec;
+    constexpr int TN = 32, NP = PT::NP, NC = 1 << ND, NR = PLAIN ? 1 : NC;     // corners, corners read
+    __shared__ unsigned sIdx[WAVES][TN];                        // byte offset of the low corner's channel 0 inside the sample
+    __shared__ __align__(16) T sCw[WAVES][TN][NR];              // weight of each corner, 0 where there is no sample
+    __shared__ __align__(16) unsigned char sRow[2][MT * NP * 1024];        // rows of a step of grad_output: [part][q][row]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int j = lane % TN, q = lane / TN;
+
+    // XCD-contiguous order with the items fastest: the workgroups that gather around the same positions share an L2
+    unsigned wg = xcd_contiguous(blockIdx.x, gridDim.x);
+    const int item = (int)(wg % igroups) * WAVES + wave; wg /= igroups;
+    const int mchunk = wg % (unsigned)P.mchunks; wg /= (unsigned)P.mchunks;
+    const int g = wg % (unsigned)P.G, split = wg / (unsigned)P.G;
+    // the item's channel tile: segments are the intersections of the convolution group with deformable groups
+    const int tap = item % P.kV;
+    int z = item / P.kV, dg, c0 = 0, ce = 0;
+    bool works = false;
+    for (dg = g * P.Cg / P.cpg; dg <= ((g + 1) * P.Cg - 1) / P.cpg; ++dg) {
+        const int cb = max(g * P.Cg, dg * P.cpg);
+        ce = min((g + 1) * P.Cg, (dg + 1) * P.cpg);
+        const int nt = (ce - cb + TN - 1) / TN;
+        if (z < nt) { c0 = cb + z * TN; works = true; break; }
+        z -= nt;
+    }
+    if (!works) dg = 0;         // (a wavefront without an item helps with the rows)
+
+    int kk[ND], kd[ND];
+    decode_tap<ND>(P, tap, kk);
+#pragma unroll
+    for (int a = 0; a < ND; ++a) kd[a] = kk[a] * P.dil[slot<ND>(a)];
+
+    const int m_base = mchunk * MT * TN;
+    const unsigned cj = (unsigned)min(c0 + j, P.C_in - 1);      // clamped: lanes past the segment still load legally
+    // 32-bit byte offsets from the sample's base (the host checks that a sample of either tensor stays below 4 GiB)
+    const unsigned cjB = cj * 4u, cinB = (unsigned)P.C_in * 4u;
+    unsigned strB[ND];                                          // from a corner to the next along an axis
+    {
+        unsigned s = cinB;
+#pragma unroll
+        for (int a = ND - 1; a >= 0; --a) {
+            strB[a] = P.in[slot<ND>(a)] > 1 ? s : 0u;
+            s *= (unsigned)P.in[slot<ND>(a)];
+        }
+    }
+    // what this thread copies of a step's rows: 16 bytes each, rows past M as row M - 1
+    constexpr int NROW = MT * NP * 64, NA = (NROW + WG - 1) / WG;
+    unsigned r_at[NA];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+        const int x = i * WG + threadIdx.x, m = x % (MT * TN), pq = min(x / (MT * TN), NP * 2 - 1);
+        r_at[i] = ((unsigned)pq * P.C_out + g * P.M + min(m_base + m, P.M - 1)) * 16u;
+    }
+
+    typename MM::Acc acc[MT];
+    const int slabs_per_sample = (int)(row_steps(P.outV) / 2), nslabs = P.N * slabs_per_sample;
+    // the splits of an XCD take turns in a range of the slabs of their own (all splits in turn over all slabs: 64 -> 64 channels in 3-D
+    // 597 -> 587 us, 128 -> 128 with stride 2 907 -> 838: fewer reads past the L2)
+    const int runs = min(P.nsplit, 8), run = (int)((unsigned)split * runs / (unsigned)P.nsplit);
+    const int s0 = (run * P.nsplit + runs - 1) / runs, s1 = ((run + 1) * P.nsplit + runs - 1) / runs;      // its splits
+    const int first = (int)((long long)nslabs * s0 / P.nsplit) + split - s0, last = (int)((long long)nslabs * s1 / P.nsplit), turn = s1 - s0;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) acc[mt] = acc_zero<T>();
+    const size_t step_bytes = (size_t)NP * 2 * P.C_out * 16;
+    const char* const row0 = reinterpret_cast<const char*>(rows);
+    Vec rv[NA];
+    auto load_rows = [&](size_t step) {                 // of all samples
+        const char* ap = row0 + step * step_bytes;
+#pragma unroll
+        for (int i = 0; i < NA; ++i) rv[i] = *reinterpret_cast<const Vec*>(ap + r_at[i]);
+    };
+    auto put_rows = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < NA; ++i)
+            if ((i + 1) * WG <= NROW || i * WG + threadIdx.x < NROW) *reinterpret_cast<Vec*>(sRow[buf] + (i * WG + threadIdx.x) * 16) = rv[i];
+    };
+    T offv[ND];
+    auto load_off = [&](int slab) {
+        const int n = slab / slabs_per_sample;
+        const unsigned posc = min((unsigned)(slab % slabs_per_sample) * TN + j, P.outV - 1);
+        const T* off_n = PLAIN ? nullptr : off + (((size_t)n * P.DG + dg) * P.kV + tap) * ND * P.outV;
+#pragma unroll
+        for (int a = 0; a < ND; ++a) offv[a] = PLAIN ? 0.f : off_n[(size_t)a * P.outV + posc];
+    };
+    const T sgn = split & 1 ? -1.f : 1.f;               // of this split's samples
+    if (first < last) {
+        load_off(first);
+        load_rows((size_t)first * 2);
+        put_rows(0);
+    }
+    __syncthreads();
+    for (int slab = first; slab < last; slab += turn) {
+        const int n = slab / slabs_per_sample;
+        const unsigned p0 = (unsigned)(slab % slabs_per_sample) * TN;
+        const char* in_n = reinterpret_cast<const char*>(in_cl + (size_t)n * P.inV * P.C_in);        // scalar bases
+        const int next_slab = min(slab + turn, last - 1);
+        const unsigned pos = p0 + j;
+        const bool valid = pos < P.outV;
+        const unsigned posc = valid ? pos : P.outV - 1;
+        int o[ND];
+        decode_pos<ND>(P, posc, o);
+        bool live = valid;
+        T f[ND];
+        unsigned base = 0;
+#pragma unroll
+        for (int a = 0; a < ND; ++a) {
+            const int sa = slot<ND>(a);
+            const T p = (T)(o[a] * P.stride[sa] - P.pad[sa] + kd[a]) + offv[a];
+            const T pc = __builtin_amdgcn_fmed3f(p, 0.f, (T)(P.in[sa] - 1));
+            live = live && fabsf(p - pc) < 1.f;                 // -1 < p < size, false for NaN
+            int lo = (int)pc;
+            if constexpr (!PLAIN) lo = min(lo, max(P.in[sa] - 2, 0));
+            f[a] = pc - (T)lo;
+            base = base * (unsigned)P.in[sa] + (unsigned)lo;
+        }
+        load_off(next_slab);                        // travel through this slab
+        // LDS operations of one wavefront execute in order; the fences only pin the compiler
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        if (q == 0) {
+            T cw[NC];                              // multiplied in the reference's order (w_l * w_h * w_w)
+            if constexpr (ND == 3) {
+                const T fl = f[0], gl = 1.f - fl, fh = f[1], gh = 1.f - fh, fw = f[2], gw = 1.f - fw;
+                cw[0] = gl * gh * gw; cw[1] = gl * gh * fw; cw[2] = gl * fh * gw; cw[3] = gl * fh * fw;
+                cw[4] = fl * gh * gw; cw[5] = fl * gh * fw; cw[6] = fl * fh * gw; cw[7] = fl * fh * fw;
+            } else {
+                const T fh = f[0], gh = 1.f - fh, fw = f[1], gw = 1.f - fw;
+                cw[0] = gh * gw; cw[1] = gh * fw; cw[2] = fh * gw; cw[3] = fh * fw;
+            }
+            sIdx[wave][j] = live ? base * cinB : 0u;
+#pragma unroll
+            for (int i = 0; i < NR; ++i) sCw[wave][j][i] = !live ? 0.f : PLAIN ? sgn : sgn * cw[i];
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+        const char* corner[NR];                     // scalar
+#pragma unroll
+        for (int i = 0; i < NR; ++i) {
+            size_t d = 0;
+#pragma unroll
+            for (int a = 0; a < ND; ++a)
+                if ((i >> (ND - 1 - a)) & 1) d += strB[a];
+            corner[i] = in_n + d;
+        }
+        // position by position; the next one's record and corner values are on their way while this one is added up
+        T cn[NR], wn[NR];
+        auto fetch = [&](int k) {
+            const int pp = (k & 8) * 2 + q * 8 + (k & 7);          // position of the slab this lane group works on
+            const unsigned at = sIdx[wave][pp] + cjB;
+#pragma unroll
+            for (int i = 0; i < NR; ++i) wn[i] = sCw[wave][pp][i];
+#pragma unroll
+            for (int i = 0; i < NR; ++i) cn[i] = *reinterpret_cast<const T*>(corner[i] + at);
+        };
+        if (works) fetch(0);
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+            load_rows(st == 0 ? (size_t)slab * 2 + 1 : (size_t)next_slab * 2);
+            if (works) {
+                float val[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    T cc[NR], wc[NR];
+#pragma unroll
+                    for (int i = 0; i < NR; ++i) { cc[i] = cn[i]; wc[i] = wn[i]; }
+                    if (st * 8 + e + 1 < 16) fetch(st * 8 + e + 1);
+                    __builtin_amdgcn_sched_barrier(0);      // the next position's loads are issued before this one's arithmetic
+                    T v = wc[0] * cc[0];                    // weighted corner sum, as the reference's sampler forms it
+#pragma unroll
+                    for (int i = 1; i < NR; ++i) v += wc[i] * cc[i];
+                    val[e] = v;
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+                // B[k = position][col = channel j]: weight 0 where there is no sample and past the end.  A row of A only reaches
+                // its own row of the tile and a column of B its own column, and rows past M / columns past the segment are not stored.
+                Vec b8[NP];
+                PT::split(val, b8);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    Vec a8[1][NP];
+#pragma unroll
+                    for (int x = 0; x < NP; ++x) a8[0][x] = *reinterpret_cast<const Vec*>(sRow[st] + ((x * 2 + q) * MT * TN + mt * TN + j) * 16);
+                    typename MM::Acc sum[1] = {acc_zero<T>()};
+                    mma_parts<float, 1>(a8, b8, sum);
+                    acc[mt] += sum[0];
+                }
+            }
+            put_rows(st ^ 1);
+            __syncthreads();
+        }
+    }
+    const bool redo = works && __any(!results_stand<MT, float>(acc));
+    // One row tile from the values themselves, two positions at a time, with the reference's corners.  (Its own accumulator, after
+    // the loop above: a second loop over `acc` doubled the registers of the kernel.)
+    auto exact_tile = [&](int mt) {
+        typename MM::Acc x = acc_zero<T>();
+        for (int slab = first; slab < last; slab += turn) {
+            const int n = slab / slabs_per_sample;
+            const unsigned p0 = (unsigned)(slab % slabs_per_sample) * TN;
+            const T* off_n = PLAIN ? nullptr : off + (((size_t)n * P.DG + dg) * P.kV + tap) * ND * P.outV;
+            const char* in_n = reinterpret_cast<const char*>(in_cl + (size_t)n * P.inV * P.C_in);
+#pragma unroll 1
+            for (int ks = 0; ks < TN; ks += 2) {
+                const unsigned pos = p0 + ks + q, posc = min(pos, P.outV - 1);
+                int o[ND], ib[ND];
+                decode_pos<ND>(P, posc, o);
+#pragma unroll
+                for (int a = 0; a < ND; ++a) ib[a] = o[a] * P.stride[slot<ND>(a)] - P.pad[slot<ND>(a)];
+                T offv[ND];
+#pragma unroll
+                for (int a = 0; a < ND; ++a) offv[a] = PLAIN ? 0.f : off_n[(size_t)a * P.outV + posc];
+                TapGeo<T, ND> t;
+                tap_setup_noidx<T, ND>(P, offv, ib, kd, t);
+                const bool live = pos < P.outV && t.inside;
+                unsigned cb[NC];
+                tap_corner_offsets<T, ND>(P, t, live, cinB, cb);
+                T v = 0.f;
+#pragma unroll
+                for (int i = 0; i < NR; ++i) {
+                    T w = 1.f;
+#pragma unroll
+                    for (int a = 0; a < ND; ++a) w *= PLAIN ? 1.f : (i >> (ND - 1 - a)) & 1 ? t.f[a] : 1.f - t.f[a];
+                    v += w * *reinterpret_cast<const T*>(in_n + (cb[i] + cjB));
+                }
+                const T b = live ? v : 0.f;
+                const int m = min(m_base + mt * TN + j, P.M - 1);
+                const T av = pos < P.outV ? gout[((size_t)n * P.C_out + g * P.M + m) * P.outV + posc] : 0.f;
+                x = MM::mma(av, b, x);
+            }
+        }
+        return x;
+    };
+
+    if (!works) return;                                 // (uniform for the wavefront)
+    T* pt = partial + ((size_t)split * P.kV + tap) * P.C_out * P.Cg + (size_t)g * P.M * P.Cg + (c0 + j - g * P.Cg);
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        typename MM::Acc x = acc[mt] * sgn;
+        if (__builtin_expect(redo, 0)) x = exact_tile(mt);
+#pragma unroll
+        for (int r = 0; r < MM::NACC; ++r) {
+            const int m = m_base + mt * TN + MM::row(r, q);
+            if (m < P.M && c0 + j < ce) pt[(size_t)m * P.Cg] = x[r];
+        }
+    }
+}
+
+}  // namespace dcn

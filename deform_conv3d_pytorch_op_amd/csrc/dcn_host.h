@@ -137,7 +137,7 @@ template <typename T> inline size_t backward_data_need(int N, int C_in, int C_ou
     return bwd_data_weight_bytes<T>(C_out / G, C_in / G, kV, G, cpg) + 2 * align256((size_t)N * C_in * inV * sizeof(T)) +
            fused_gout_need<T>(N, C_out / G, G, outV) + BWD_TAIL + 512;
 }
-// two channels-last copies + one partial weight per position split (at most 256 splits, and never more
+// A channels-last copy of the input, grad_output channels-last or (float32) in operand order + one partial weight per position split (at most 256 splits, and never more
 // than about 4096 workgroups: see bww_plan) + the strips of grad_output's sums
 template <typename T> inline size_t backward_weight_need(int N, int C_in, int C_out, size_t inV, size_t outV, int kV, int G) {
     const int TNq = Mma<T>::TN;
@@ -145,7 +145,8 @@ template <typename T> inline size_t backward_weight_need(int N, int C_in, int C_
     long long split_ub = (4096 + tiles_lb - 1) / tiles_lb;
     if (split_ub > 256) split_ub = 256;
     if (split_ub < 1) split_ub = 1;
-    return align256((size_t)N * C_in * inV * sizeof(T)) + align256((size_t)N * C_out * outV * sizeof(T)) +
+    const size_t obytes = (size_t)N * C_out * outV * sizeof(T), rbytes = sizeof(T) == 4 && C_out / G > 32 ? row_operand_bytes(N, C_out, outV) : 0;
+    return align256((size_t)N * C_in * inV * sizeof(T)) + align256(obytes > rbytes ? obytes : rbytes) +
            align256((size_t)split_ub * kV * C_out * (C_in / G) * sizeof(T)) + align256((size_t)N * last_strips((unsigned)outV) * C_out * sizeof(T));
 }
 template <typename T> inline size_t workspace_need(int N, int C_in, int C_out, size_t inV, size_t outV, int kV, int G, int cpg = 0) {
@@ -533,8 +534,10 @@ template <typename T, typename S> struct WeightCall {
     Params P;
     int MT;
     S *in_cl, *gout_cl;
+    const S* gout;
     T *partial, *sums;
     int nsums;
+    int igroups;                    // > 0: backward_weight_split_kernel, and gout_cl is grad_output in its operand order
 };
 template <typename T, int ND, typename S>
 int backward_weight_plan(const Params& P, const S* in, const S* gout, void* ws, size_t ws_bytes, bool bias, WeightCall<T, S>& c, Prep& prep, bool* declined);

@@ -1714,7 +1714,7 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
 // stays in registers; each workgroup writes one partial tile per split and a small second kernel
 // sums the splits into grad_weight (deterministic, no atomics).
 // PLAIN: a plain convolution (off is null): samples at integer coordinates are their low corner alone (64 -> 64 channels, 3x3,
-// 25 088 positions, float32: 38.5 -> 33.4 us).
+// 25 088 positions, float32: 38.5 -> 33.4 us).  float32 layers of many output channels: backward_weight_split_kernel.
 // dynamic LDS = WAVES * TN * (TN+1) * sizeof(T).
 template <typename T, int ND, int MT, bool PLAIN = false>
 __global__ __launch_bounds__(WG) void backward_weight_kernel(Params P, const T* __restrict__ in_cl,

@@ -8,10 +8,11 @@
 // 8 x 56 x 56: 25 against 50 and 12; 128 -> 128, 3-D, 2 x 16 x 112 x 112 -> 56 x 56: 175 against 220 and 42.
 #pragma once
 #include "dcn_backward_fused.h"
+#include "dcn_backward_weight_split.h"
 
 namespace dcn {
 
-enum PrepKind { PREP_PACK, PREP_FUSED_PACK, PREP_GOUT, PREP_PLAN, PREP_BOUNDS, PREP_ZERO, PREP_LAST };
+enum PrepKind { PREP_PACK, PREP_FUSED_PACK, PREP_GOUT, PREP_PLAN, PREP_BOUNDS, PREP_ZERO, PREP_ROWS, PREP_LAST };
 struct PrepJob {
     int kind, variant;          // PACK, FUSED_PACK: channels per chunk; PACK: + 1 for the wide row order
     unsigned first;             // first block; the job's blocks reach to the next job's first
@@ -114,6 +115,52 @@ __device__ inline void prep_channels_last(const PrepJob& job, unsigned block) {
     }
 }
 
+// grad_output in the operand order of backward_weight_split_kernel, and its sums: 32 channels of a strip, 64 positions at a
+// time through LDS, then eight positions of one channel to a thread.
+__device__ inline void prep_rows(const PrepJob& job, unsigned block) {
+    using PT = Parts<float>;
+    __shared__ float tile[32][65];
+    const unsigned strips = last_strips(job.V), ctiles = ((unsigned)job.C + 31) / 32;
+    const unsigned strip = block % strips, c0 = (block / strips) % ctiles * 32, n = block / strips / ctiles;
+    const float* src = static_cast<const float*>(job.src) + (size_t)n * job.C * job.V;
+    const unsigned steps = row_steps(job.V), tx = threadIdx.x & 63, ty = threadIdx.x >> 6, c = c0 + (threadIdx.x & 31), oct = threadIdx.x >> 5;
+    typename PT::Vec* dst = static_cast<typename PT::Vec*>(job.dst) + (size_t)n * steps * PT::NP * 2 * job.C;
+    float sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    for (unsigned v0 = strip * LAST_STRIP; v0 < min((strip + 1) * LAST_STRIP, job.V); v0 += 64) {
+#pragma unroll
+        for (unsigned k = 0; k < 8; ++k) {
+            const unsigned ch = ty + 4 * k, v = v0 + tx;
+            const float x = c0 + ch < (unsigned)job.C && v < job.V ? src[(size_t)(c0 + ch) * job.V + v] : 0.f;
+            tile[ch][tx] = x;
+            sum[k] += x;
+        }
+        __syncthreads();
+        const unsigned step = (v0 >> 4) + (oct >> 1);
+        if (c < (unsigned)job.C && step < steps) {
+            typename PT::Vec p8[PT::NP];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                typename PT::Elem p[PT::NP];
+                PT::split1(tile[threadIdx.x & 31][oct * 8 + e], p);
+#pragma unroll
+                for (int x = 0; x < PT::NP; ++x) p8[x][e] = p[x];
+            }
+#pragma unroll
+            for (int x = 0; x < PT::NP; ++x) dst[((size_t)(step * PT::NP + x) * 2 + (oct & 1)) * job.C + c] = p8[x];
+        }
+        __syncthreads();
+    }
+    if (job.sums) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+#pragma unroll
+            for (int sh = 1; sh < 64; sh <<= 1) sum[k] += __shfl_xor(sum[k], sh);
+            const unsigned ch = c0 + ty + 4 * k;
+            if (tx == 0 && ch < (unsigned)job.C) static_cast<float*>(job.sums)[(size_t)ch * strips * job.N + n * strips + strip] = sum[k];
+        }
+    }
+}
+
 template <typename T, typename S>
 __global__ __launch_bounds__(256) void backward_prepare_kernel(Params P, PlanChoice pc, PrepJobs jobs, const S* __restrict__ W,
                                                                const S* __restrict__ off, size_t n_off) {
@@ -167,6 +214,9 @@ __global__ __launch_bounds__(256) void backward_prepare_kernel(Params P, PlanCho
             }
             break;
         }
+        case PREP_ROWS:
+            if constexpr (sizeof(S) == 4) prep_rows(job, block);
+            break;
         default: prep_channels_last<T, S>(job, block); break;
     }
 }
@@ -195,6 +245,10 @@ struct Prep {
     }
     void channels_last(const void* src, void* dst, int C, unsigned V, int N, void* sums) {
         PrepJob& j = add(PREP_LAST, last_strips(V) * (((unsigned)C + 31) / 32) * (unsigned)N);
+        j.src = src; j.dst = dst; j.C = C; j.V = V; j.N = N; j.sums = sums;
+    }
+    void rows(const void* src, void* dst, int C, unsigned V, int N, void* sums) {
+        PrepJob& j = add(PREP_ROWS, last_strips(V) * (((unsigned)C + 31) / 32) * (unsigned)N);
         j.src = src; j.dst = dst; j.C = C; j.V = V; j.N = N; j.sums = sums;
     }
 

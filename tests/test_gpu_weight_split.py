@@ -1,0 +1,102 @@
+"""backward_weight_split_kernel: layers just large enough for it, with the edges of its tiles, slabs, segments and volumes."""
+import pytest
+import torch
+
+from oracle import dcn_oracle as orc
+from tests.cases import make_case
+
+pytestmark = pytest.mark.gpu
+
+# (nd, N, C_in, C_out, ins, k, stride, pad, dil, cpg, groups, reach): two and four row tiles and their remainders, one and
+# several chunks of them; channel tiles with remainders; deformable groups over two convolution groups; last slabs of 1 and 31
+# positions and whole ones; strides and dilations; an axis of one voxel; one tap of many channels; samples past the volume
+LAYERS = [
+    (2, 1, 33, 65, (97, 161), 3, 1, 1, 1, 33, 1, 1.5), (2, 2, 40, 128, (97, 73), 3, 1, 1, 1, 20, 1, 3.0),
+    (2, 1, 24, 210, (141, 99), 3, 1, 1, 1, 8, 2, 2.0), (2, 3, 33, 33, (85, 89), 3, 1, 1, 1, 33, 1, 1.0),
+    (2, 1, 32, 64, (229, 231), 5, 2, 2, 1, 32, 1, 9.0), (2, 1, 136, 97, (221, 223), 1, 1, 0, 1, 136, 1, 0.9),
+    (3, 1, 16, 80, (9, 32, 32), 3, 1, 1, 1, 16, 1, 1.5), (3, 2, 5, 66, (13, 39, 41), 3, (1, 2, 2), 1, 1, 5, 1, 2.5),
+    (3, 1, 34, 40, (1, 95, 97), 3, 1, 1, 1, 17, 1, 1.0), (3, 1, 12, 70, (23, 21, 25), 3, 1, 2, 2, 12, 2, 2.0),
+]
+IDS = lambda s: "%dd-%d-%d-k%d-g%d" % (s[0], s[2], s[3], s[5], s[10])
+
+
+def _weight_gradient(c):
+    import deform_conv3d_pytorch_op_amd as dcn
+    fn = dcn.ConvOffset3dFunction if c["nd"] == 3 else dcn.ConvOffset2dFunction
+    x, off, w = (c[k].cuda().requires_grad_(k == "w") for k in ("x", "off", "w"))
+    b = torch.zeros(w.shape[0], device="cuda").requires_grad_(True)
+    fn.apply(x, off, w, b, c["stride"], c["pad"], c["dil"], c["cpg"], c["groups"]).backward(c["gout"].cuda())
+    return w.grad.cpu().double(), b.grad.cpu().double()
+
+
+def _oracle(c):
+    """In float32 with double sums: the coordinates are then those of the kernel."""
+    d = {k: c[k].float() for k in ("x", "off", "w", "gout")}
+    return orc.backward(d["x"], d["off"], d["w"], d["gout"], None, c["stride"], c["pad"], c["dil"], c["cpg"], c["groups"])[2].double()
+
+
+@pytest.mark.parametrize("spec", LAYERS, ids=IDS)
+def test_layers(spec):
+    """2-norm: chains of float32 sums over up to a few hundred steps of positions and the splits, each off by half a unit in
+    the last place of a partial sum: below 2^-24 * 64 = 4e-6."""
+    print("weight gradient", spec, flush=True)
+    c = make_case(*spec, dtype=torch.float32, seed=41, bias=False)
+    got, bias = _weight_gradient(c)
+    want = _oracle(c)
+    err = ((got - want).norm() / want.norm()).item()
+    print("  relative 2-norm error %.2e" % err, flush=True)
+    assert err <= 4e-6
+    g64 = c["gout"].double()
+    sums = g64.sum(dim=[0] + list(range(2, g64.dim())))
+    assert ((bias - sums).norm() / sums.norm()).item() <= 4e-6
+
+
+@pytest.mark.parametrize("spec", [LAYERS[0], LAYERS[6]], ids=IDS)
+@pytest.mark.parametrize("what,exponent", [("gout", 90), ("gout", 120), ("x", 100), ("x", 126)])
+def test_small_operands(spec, what, exponent):
+    """Operands whose bfloat16 parts leave the range of normal numbers: the results are formed from the values themselves."""
+    print("small", spec, what, exponent, flush=True)
+    c = make_case(*spec, dtype=torch.float32, seed=42, bias=False)
+    c[what] = c[what] * 2.0 ** -exponent
+    got, _ = _weight_gradient(c)
+    want = _oracle(c)
+    if exponent >= 120:                 # results and partial sums near the smallest normal number, off by a few of its last units
+        assert (got - want).abs().max().item() <= 2.0 ** -149 * 64 + 4e-6 * want.abs().max().item()
+    else:
+        assert ((got - want).norm() / want.norm()).item() <= 4e-6
+
+
+@pytest.mark.parametrize("spec", [LAYERS[0], LAYERS[6]], ids=IDS)
+@pytest.mark.parametrize("what", ["x", "gout", "off"])
+def test_non_finite(spec, what):
+    """Not finite where the oracle's gradient is not, equal to it elsewhere."""
+    print("non-finite", spec, what, flush=True)
+    c = make_case(*spec, dtype=torch.float32, seed=43, bias=False)
+    flat = c[what].view(-1)
+    if what == "x":                     # the last channel alone, in the last rows of the volume: the collapsed corners lie there
+        c["x"][0, -1].view(-1)[-3:] = torch.tensor([float("inf"), float("nan"), -float("inf")])
+    elif what == "gout":
+        c["gout"][0, -1].view(-1)[5:8] = torch.tensor([float("inf"), float("nan"), -float("inf")])
+    else:
+        flat[::997] = float("nan")
+        flat[5::1009] = float("inf")
+    got, _ = _weight_gradient(c)
+    want = _oracle(c)
+    fin = torch.isfinite(want)
+    assert what == "off" or not fin.all()
+    assert torch.equal(torch.isfinite(got), fin)
+    assert ((got - want)[fin].norm() / want[fin].norm()).item() <= 4e-6
+
+
+@pytest.mark.parametrize("n,ci,co,size", [(2, 40, 70, (83, 85)), (4, 33, 64, (73, 91))])
+def test_plain_convolution(n, ci, co, size):
+    """The convolution without offsets, against float64."""
+    import deform_conv3d_pytorch_op_amd as dcn
+    print("plain", n, ci, co, size, flush=True)
+    g = torch.Generator().manual_seed(44)
+    x = torch.randn((n, ci) + size, generator=g)
+    m = dcn.Conv2d(ci, co, 3, 1, 1, 1, device="cuda")
+    gout = torch.randn((n, co) + size, generator=g)
+    m(x.cuda()).backward(gout.cuda())
+    want = torch.nn.grad.conv2d_weight(x.double(), m.weight.shape, gout.double(), stride=1, padding=1)
+    assert ((m.weight.grad.cpu().double() - want).norm() / want.norm()).item() <= 4e-6
