@@ -180,6 +180,7 @@ __global__ __launch_bounds__(NW * 64, 1) void forward_quad_kernel(Params P, Plan
 
     const int cg0 = g * P.Cg, cg1 = cg0 + P.Cg;
     int chunk_no = 0;
+    if (threadIdx.x == 0) sNonFinite = 0;               // (stays set for the chunks that follow, see forward_split_kernel)
     for (int dg = cg0 / P.cpg; dg <= (cg1 - 1) / P.cpg; ++dg) {
         const int cb = max(cg0, dg * P.cpg), ce = min(cg1, (dg + 1) * P.cpg);
         const T* off_dg = off + ((size_t)n * P.DG + dg) * P.kV * ND * P.outV;
@@ -188,11 +189,10 @@ __global__ __launch_bounds__(NW * 64, 1) void forward_quad_kernel(Params P, Plan
             const int nch = min(cch, ce - cc0);
             const int ngrp = (nch + FQ - 1) / FQ;
             const T* chan0 = in + ((size_t)n * P.C_in + cc0) * P.inV;      // workgroup-uniform
-            if (threadIdx.x == 0) sNonFinite = 0;
             __syncthreads();                                               // readers of the previous chunk are done
             halo_stage_quads<T, WGS>(P, H, chan0, nch, sTab, sIn, &sNonFinite);
             __syncthreads();
-            // Non-finite input values in this halo: the branch-free sampler reads the cell next to a
+            // Non-finite input values in this halo or one before it: the branch-free sampler reads the cell next to a
             // collapsed corner with weight 0, and 0 * inf would be NaN where the reference never
             // touches that voxel (deform3d/lib/deform_conv3d_cuda_kernel.cu:24-26).  Samples in the
             // collapse zones (p <= 0 or p >= size - 1 on some axis) then take the pass through global

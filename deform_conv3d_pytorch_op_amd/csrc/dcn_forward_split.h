@@ -570,7 +570,9 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
     const unsigned a_tg = mtiles * NP * 64;
     const int cg0 = g * P.Cg, cg1 = cg0 + P.Cg;
 
-    if (threadIdx.x == 0) sRedo = 0;                    // ordered before the checks by the barriers of the first chunk
+    // Ordered before the checks by the barriers of the first chunk.  sNonFinite stays set for the chunks that follow: cleared for each, it
+    // could be cleared under a wavefront that has not read it yet by one that has no step in this chunk.
+    if (threadIdx.x == 0) sRedo = sNonFinite = 0;
     // exact: the contraction on the float32 instructions, with the reference's treatment of non-finite
     // input next to the rim.
     auto work = [&](auto exact_tag) {
@@ -591,11 +593,10 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
                 const int tg_first = TS > 1 ? __builtin_amdgcn_readfirstlane(first / ngrp) : 0, tg_end = TS > 1 ? __builtin_amdgcn_readfirstlane((last + ngrp - 1) / ngrp) : ntg;
                 float ofs[ND];
                 load_pair_offsets<ND, S>(P, off_dg, min(tg_first, ntg - 1), q, pos, ofs, off == nullptr);
-                if (exact && threadIdx.x == 0) sNonFinite = 0;
                 __syncthreads();                                               // readers of the previous chunk are done
                 if (stage_halo<ND, WGS, exact, S>(P, H, tg, chan0, nch, sIn)) sNonFinite = 1;
                 __syncthreads();
-                // Non-finite input in this halo (a non-finite sample always leads to the second pass): the
+                // Non-finite input in this halo or one before it (a non-finite sample always leads to the second pass): the
                 // branch-free sampler reads the cell next to a collapsed corner with weight 0, and 0 * inf would
                 // be NaN where the reference never touches that voxel
                 // (deform3d/lib/deform_conv3d_cuda_kernel.cu:24-26).  Samples in the collapse zones (p <= 0 or
