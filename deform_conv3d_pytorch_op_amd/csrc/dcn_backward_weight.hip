@@ -41,13 +41,13 @@ void bww_plan(const Params& Pin, int& MT, int& mchunks, int& nct, int& nsplit, l
 }
 
 // Channel tiles of the convolution group that has the most, times taps.
-inline int split_items(const Params& P) {
+inline int split_items(const Params& P, int TC) {
     int most = 0;
     for (int g = 0; g < P.G; ++g) {
         int n = 0;
         for (int dg = g * P.Cg / P.cpg; dg <= ((g + 1) * P.Cg - 1) / P.cpg; ++dg) {
             const int cb = g * P.Cg > dg * P.cpg ? g * P.Cg : dg * P.cpg, ce = (g + 1) * P.Cg < (dg + 1) * P.cpg ? (g + 1) * P.Cg : (dg + 1) * P.cpg;
-            n += (ce - cb + 31) / 32;
+            n += (ce - cb + TC - 1) / TC;
         }
         most = n > most ? n : most;
     }
@@ -61,15 +61,15 @@ inline int split_items(const Params& P) {
 // positions 228 : 203; 12 -> 57, 62 000 positions 750 : 698).  Its wavefronts write a partial tile each: about one round of resident
 // workgroups, as long as the tiles (written and read at about 8 TB/s) cost less than the longer runs of slabs.
 struct SplitPlan { int MT, mchunks, igroups, nsplit; };     // nsplit 0: not a layer for it, or no room
-template <int ND>
+template <int ND, typename S>
 SplitPlan split_plan(const Params& P, size_t room) {
     SplitPlan c = {};
-    const int items = split_items(P);
+    const int items = split_items(P, tile_channels<S>());
     c.MT = P.M > 64 ? 4 : 2;
     c.mchunks = ((P.M + 31) / 32 + c.MT - 1) / c.MT;
     c.igroups = (items + WAVES - 1) / WAVES;
-    const double resident = (double)resident_workgroups(c.MT == 4 ? reinterpret_cast<const void*>(backward_weight_split_kernel<ND, 4>)
-                                                         : reinterpret_cast<const void*>(backward_weight_split_kernel<ND, 2>), WG, 0);
+    const double resident = (double)resident_workgroups(c.MT == 4 ? reinterpret_cast<const void*>(backward_weight_split_kernel<ND, 4, S>)
+                                                         : reinterpret_cast<const void*>(backward_weight_split_kernel<ND, 2, S>), WG, 0);
     const long long nslabs = (long long)P.N * (row_steps(P.outV) / 2);
     const double other = (double)c.igroups * c.mchunks * P.G;
     if (P.M <= 32 || items < WAVES || (double)items * c.mchunks * P.G * (double)nslabs < 2.5 * WAVES * resident) return c;
@@ -184,10 +184,10 @@ int backward_weight_plan(const Params& Pin, const S* in, const S* gout, void* ws
     size_t obytes = align256((size_t)P.N * P.C_out * P.outV * sizeof(S));
     c.igroups = 0;
     c.gout = gout;
-    if constexpr (sizeof(S) == 4) {
-        const size_t rbytes = align256(row_operand_bytes(P.N, P.C_out, P.outV));
+    if constexpr (sizeof(S) <= 4) {
+        const size_t rbytes = align256(row_operand_bytes<S>(P.N, P.C_out, P.outV));
         const size_t used = ibytes + rbytes + (bias ? (size_t)P.N * last_strips(P.outV) * P.C_out * sizeof(T) : 0) + 256;
-        const SplitPlan sp = split_plan<ND>(P, ws && ws_bytes > used ? ws_bytes - used : 0);
+        const SplitPlan sp = split_plan<ND, S>(P, ws && ws_bytes > used ? ws_bytes - used : 0);
         if (sp.nsplit) {
             obytes = rbytes;
             c.MT = sp.MT; c.igroups = sp.igroups; P.mchunks = sp.mchunks; P.nsplit = sp.nsplit;
@@ -208,25 +208,26 @@ int backward_weight_plan(const Params& Pin, const S* in, const S* gout, void* ws
     return DCN_OK;
 }
 
-template <int ND, int MT>
-int launch_bwd_weight_split(const WeightCall<float, float>& c, const float* off, hipStream_t s) {
+template <int ND, int MT, typename S>
+int launch_bwd_weight_split(const WeightCall<float, S>& c, const S* off, hipStream_t s) {
     const Params& P = c.P;
     const dim3 grid((unsigned)((long long)c.igroups * P.mchunks * P.G * P.nsplit));
-    auto kern = backward_weight_split_kernel<ND, MT>;
-    if constexpr (ND == 2)
-        if (!off) kern = backward_weight_split_kernel<ND, MT, true>;
-    hipLaunchKernelGGL(kern, grid, dim3(WG), 0, s, P, (const float*)c.in_cl, off, c.gout, reinterpret_cast<const Parts<float>::Vec*>(c.gout_cl), c.partial, (unsigned)c.igroups);
+    auto kern = backward_weight_split_kernel<ND, MT, S>;
+    if constexpr (ND == 2 && sizeof(S) == 4)
+        if (!off) kern = backward_weight_split_kernel<ND, MT, S, true>;
+    hipLaunchKernelGGL(kern, grid, dim3(WG), 0, s, P, (const S*)c.in_cl, off, c.gout, reinterpret_cast<const typename Parts<S>::Vec*>(c.gout_cl), c.partial, (unsigned)c.igroups);
     return check_launch("backward_weight_split_kernel");
 }
 
 template <typename T, int ND, typename S>
 int backward_weight_run(const WeightCall<T, S>& c, const S* off, T* gw, T* gb, bool accumulate, hipStream_t s) {
     const Params& P = c.P;
-    if constexpr (std::is_same<S, T>::value) {
-        int rc = DCN_OK;
+    if (c.igroups) {
         if constexpr (sizeof(T) == 4)
-            if (c.igroups) rc = c.MT == 4 ? launch_bwd_weight_split<ND, 4>(c, off, s) : launch_bwd_weight_split<ND, 2>(c, off, s);
-        if (!c.igroups) switch (c.MT) {
+            if (int rc = c.MT == 4 ? launch_bwd_weight_split<ND, 4, S>(c, off, s) : launch_bwd_weight_split<ND, 2, S>(c, off, s)) return rc;
+    } else if constexpr (std::is_same<S, T>::value) {
+        int rc;
+        switch (c.MT) {
             case 1: rc = launch_bwd_weight<T, ND, 1>(c, off, s); break;
             case 2: rc = launch_bwd_weight<T, ND, 2>(c, off, s); break;
             default: rc = launch_bwd_weight<T, ND, 4>(c, off, s); break;

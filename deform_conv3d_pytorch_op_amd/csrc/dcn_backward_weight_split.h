@@ -1,13 +1,13 @@
-// Backward pass to the weight of the float32 operator, for layers of more than 32 output channels to a group (split_plan).
+// Backward pass to the weight of the float32 and 16-bit operators, for layers of more than 32 output channels to a group (split_plan).
 //
 //   gW[g*M+m][cl][tap] += sum_{n,pos} grad_output[n][g*M+m][pos] * sample(in[n][g*Cg+cl], tap, pos)
 //
 // replaces the second deformable_im2col + Sgemm(beta=1) of deform3d/lib/deform_conv3d_cuda.cpp:283-320.
 //
-// The reduction runs over positions.  A wavefront samples 32 channels of one tap: lane (j, q) takes channel c0 + j at eight
+// The reduction runs over positions.  A wavefront samples 32 channels of one tap (16-bit storage: 64, two to a lane): lane (j, q) takes channel c0 + j at eight
 // consecutive positions of a step of 16 -- the input is channels-last, so a corner is one coalesced 128-byte read of the
 // lane group -- and those eight samples are the lane's operand of v_mfma_f32_32x32x16_bf16 as they stand: three bfloat16
-// parts (dcn_forward_split.h).  The other operand, the rows of grad_output, comes from the preparing launch in operand order
+// parts or one of the storage format (dcn_forward_split.h).  The other operand, the rows of grad_output, comes from the preparing launch in operand order
 // (prep_rows); the four wavefronts of a workgroup work taps or channel tiles of their own on the same positions and share it
 // through LDS, two steps of it in turn.  The geometry of a slab of 32 positions is worked out once by the position-owning
 // lanes and handed to the channel lanes through a wavefront-private record: byte offset of the low corner and the corner
@@ -29,6 +29,8 @@
 // 3x3, 8 x 56 x 56: 332 -> 240; 512 -> 512 in two groups, 3x3, 4 x 28 x 28: 105 -> 80; 128 -> 128, 3x3x3, 2 x 16 x 56 x 56
 // (stride 2): 1022 -> 860; 64 -> 64 as above: 633 -> 600; 64 -> 64, 3x3, no offsets, 25 088 positions: 33 -> 25.
 // The preparing launch pays 4 to 30 us of it back (three halves of the bytes of a channels-last copy).
+// 16-bit storage, against backward_weight16_kernel, which samples once for every 64 output channels: 256 -> 256 in float16 150 -> 116,
+// 64 -> 64 in 3-D in bfloat16 361 -> 326.
 #pragma once
 #include "dcn_forward_split.h"
 
@@ -37,19 +39,29 @@ namespace dcn {
 constexpr unsigned ROW_SLAB = 32;                       // positions of a slab: two steps
 __host__ __device__ inline unsigned row_steps(unsigned V) { return (V + ROW_SLAB - 1) / ROW_SLAB * 2; }
 // grad_output in operand order: [n][step][part][q][output channel], 16 bytes (eight positions) each, zero past the volume
-inline size_t row_operand_bytes(int N, int C_out, size_t V) { return (size_t)N * row_steps((unsigned)V) * Parts<float>::NP * 2 * C_out * 16; }
+template <typename S> inline size_t row_operand_bytes(int N, int C_out, size_t V) { return (size_t)N * row_steps((unsigned)V) * Parts<S>::NP * 2 * C_out * 16; }
+// channels of a channel tile: those of a 128-byte read by the 32 lanes of a group (16-bit storage: pairs, two columns tiles)
+template <typename S> __host__ __device__ constexpr int tile_channels() { return 128 / (int)sizeof(S); }
+
+// channel u of what a lane reads of a corner
+template <typename S> __device__ inline float channel_of(float v, int) { return v; }
+template <typename S> __device__ inline float channel_of(unsigned v, int u) {
+    if constexpr (std::is_same<S, Bf16>::value) return __uint_as_float(u ? v & 0xffff0000u : v << 16);
+    else return (float)__builtin_bit_cast(_Float16, (unsigned short)(u ? v >> 16 : v));
+}
 
 // MT row tiles to a workgroup.  PLAIN: a plain convolution (off is null): samples at integer coordinates are their low corner alone.
 // Grid: igroups * mchunks * G * nsplit workgroups.  An item is a tap of a channel tile of the convolution group, tap fastest.
-template <int ND, int MT, bool PLAIN = false>
-__global__ __launch_bounds__(WG, MT == 4 ? 3 : 4) void backward_weight_split_kernel(Params P, const float* __restrict__ in_cl, const float* __restrict__ off,
-                                                                                         const float* __restrict__ gout,
-                                                                                         const typename Parts<float>::Vec* __restrict__ rows,
+template <int ND, int MT, typename S, bool PLAIN = false>
+__global__ __launch_bounds__(WG, (MT == 4 ? 3 : 4) - (sizeof(S) == 2)) void backward_weight_split_kernel(Params P, const S* __restrict__ in_cl, const S* __restrict__ off,
+                                                                                         const S* __restrict__ gout,
+                                                                                         const typename Parts<S>::Vec* __restrict__ rows,
                                                                                          float* __restrict__ partial, unsigned igroups) {
     typedef float T;
     using MM = Mma<float>;
-    using PT = Parts<float>;
+    using PT = Parts<S>;
     typedef typename PT::Vec Vec;
+    constexpr int TC = tile_channels<S>(), CT = TC / 32;        // CT channels to a lane
     constexpr int TN = 32, NP = PT::NP, NC = 1 << ND, NR = PLAIN ? 1 : NC;     // corners, corners read
     __shared__ unsigned sIdx[WAVES][TN];                        // byte offset of the low corner's channel 0 inside the sample
     __shared__ __align__(16) T sCw[WAVES][TN][NR];              // weight of each corner, 0 where there is no sample
@@ -69,8 +81,8 @@ __global__ __launch_bounds__(WG, MT == 4 ? 3 : 4) void backward_weight_split_ker
     for (dg = g * P.Cg / P.cpg; dg <= ((g + 1) * P.Cg - 1) / P.cpg; ++dg) {
         const int cb = max(g * P.Cg, dg * P.cpg);
         ce = min((g + 1) * P.Cg, (dg + 1) * P.cpg);
-        const int nt = (ce - cb + TN - 1) / TN;
-        if (z < nt) { c0 = cb + z * TN; works = true; break; }
+        const int nt = (ce - cb + TC - 1) / TC;
+        if (z < nt) { c0 = cb + z * TC; works = true; break; }
         z -= nt;
     }
     if (!works) dg = 0;         // (a wavefront without an item helps with the rows)
@@ -81,9 +93,9 @@ __global__ __launch_bounds__(WG, MT == 4 ? 3 : 4) void backward_weight_split_ker
     for (int a = 0; a < ND; ++a) kd[a] = kk[a] * P.dil[slot<ND>(a)];
 
     const int m_base = mchunk * MT * TN;
-    const unsigned cj = (unsigned)min(c0 + j, P.C_in - 1);      // clamped: lanes past the segment still load legally
+    const unsigned cj = (unsigned)min(c0 + j * CT, P.C_in - CT);      // clamped: lanes past the segment still load legally
     // 32-bit byte offsets from the sample's base (the host checks that a sample of either tensor stays below 4 GiB)
-    const unsigned cjB = cj * 4u, cinB = (unsigned)P.C_in * 4u;
+    const unsigned cjB = cj * (unsigned)sizeof(S), cinB = (unsigned)P.C_in * (unsigned)sizeof(S);
     unsigned strB[ND];                                          // from a corner to the next along an axis
     {
         unsigned s = cinB;
@@ -102,15 +114,17 @@ __global__ __launch_bounds__(WG, MT == 4 ? 3 : 4) void backward_weight_split_ker
         r_at[i] = ((unsigned)pq * P.C_out + g * P.M + min(m_base + m, P.M - 1)) * 16u;
     }
 
-    typename MM::Acc acc[MT];
+    typename MM::Acc acc[CT][MT];
     const int slabs_per_sample = (int)(row_steps(P.outV) / 2), nslabs = P.N * slabs_per_sample;
-    // the splits of an XCD take turns in a range of the slabs of their own (all splits in turn over all slabs: 64 -> 64 channels in 3-D
-    // 597 -> 587 us, 128 -> 128 with stride 2 907 -> 838: fewer reads past the L2)
+    // the splits of an XCD take turns in a range of the slabs of their own (against all splits in turn over all slabs: 64 -> 64 channels in
+    // 3-D 597 -> 587 us, 128 -> 128 with stride 2 907 -> 838: fewer reads past the L2)
     const int runs = min(P.nsplit, 8), run = (int)((unsigned)split * runs / (unsigned)P.nsplit);
     const int s0 = (run * P.nsplit + runs - 1) / runs, s1 = ((run + 1) * P.nsplit + runs - 1) / runs;      // its splits
     const int first = (int)((long long)nslabs * s0 / P.nsplit) + split - s0, last = (int)((long long)nslabs * s1 / P.nsplit), turn = s1 - s0;
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) acc[mt] = acc_zero<T>();
+    for (int u = 0; u < CT; ++u)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[u][mt] = acc_zero<T>();
     const size_t step_bytes = (size_t)NP * 2 * P.C_out * 16;
     const char* const row0 = reinterpret_cast<const char*>(rows);
     Vec rv[NA];
@@ -128,9 +142,9 @@ __global__ __launch_bounds__(WG, MT == 4 ? 3 : 4) void backward_weight_split_ker
     auto load_off = [&](int slab) {
         const int n = slab / slabs_per_sample;
         const unsigned posc = min((unsigned)(slab % slabs_per_sample) * TN + j, P.outV - 1);
-        const T* off_n = PLAIN ? nullptr : off + (((size_t)n * P.DG + dg) * P.kV + tap) * ND * P.outV;
+        const S* off_n = PLAIN ? nullptr : off + (((size_t)n * P.DG + dg) * P.kV + tap) * ND * P.outV;
 #pragma unroll
-        for (int a = 0; a < ND; ++a) offv[a] = PLAIN ? 0.f : off_n[(size_t)a * P.outV + posc];
+        for (int a = 0; a < ND; ++a) offv[a] = PLAIN ? 0.f : Store<S>::ld(off_n[(size_t)a * P.outV + posc]);
     };
     const T sgn = split & 1 ? -1.f : 1.f;               // of this split's samples
     if (first < last) {
@@ -195,61 +209,77 @@ __global__ __launch_bounds__(WG, MT == 4 ? 3 : 4) void backward_weight_split_ker
             corner[i] = in_n + d;
         }
         // position by position; the next one's record and corner values are on their way while this one is added up
-        T cn[NR], wn[NR];
+        typedef typename std::conditional<CT == 1, T, unsigned>::type Word;
+        Word cn[NR];
+        T wn[NR];
         auto fetch = [&](int k) {
             const int pp = (k & 8) * 2 + q * 8 + (k & 7);          // position of the slab this lane group works on
             const unsigned at = sIdx[wave][pp] + cjB;
 #pragma unroll
             for (int i = 0; i < NR; ++i) wn[i] = sCw[wave][pp][i];
 #pragma unroll
-            for (int i = 0; i < NR; ++i) cn[i] = *reinterpret_cast<const T*>(corner[i] + at);
+            for (int i = 0; i < NR; ++i) cn[i] = *reinterpret_cast<const Word*>(corner[i] + at);
         };
         if (works) fetch(0);
 #pragma unroll
         for (int st = 0; st < 2; ++st) {
             load_rows(st == 0 ? (size_t)slab * 2 + 1 : (size_t)next_slab * 2);
             if (works) {
-                float val[8];
+                float val[CT][8];
 #pragma unroll
                 for (int e = 0; e < 8; ++e) {
-                    T cc[NR], wc[NR];
+                    Word cc[NR];
+                    T wc[NR];
 #pragma unroll
                     for (int i = 0; i < NR; ++i) { cc[i] = cn[i]; wc[i] = wn[i]; }
                     if (st * 8 + e + 1 < 16) fetch(st * 8 + e + 1);
                     __builtin_amdgcn_sched_barrier(0);      // the next position's loads are issued before this one's arithmetic
-                    T v = wc[0] * cc[0];                    // weighted corner sum, as the reference's sampler forms it
 #pragma unroll
-                    for (int i = 1; i < NR; ++i) v += wc[i] * cc[i];
-                    val[e] = v;
+                    for (int u = 0; u < CT; ++u) {          // weighted corner sum, as the reference's sampler forms it
+                        T v = wc[0] * channel_of<S>(cc[0], u);
+#pragma unroll
+                        for (int i = 1; i < NR; ++i) v += wc[i] * channel_of<S>(cc[i], u);
+                        val[u][e] = v;
+                    }
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 // B[k = position][col = channel j]: weight 0 where there is no sample and past the end.  A row of A only reaches
                 // its own row of the tile and a column of B its own column, and rows past M / columns past the segment are not stored.
-                Vec b8[NP];
-                PT::split(val, b8);
+                Vec b8[CT][NP];
+#pragma unroll
+                for (int u = 0; u < CT; ++u) PT::split(val[u], b8[u]);
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt) {
                     Vec a8[1][NP];
 #pragma unroll
                     for (int x = 0; x < NP; ++x) a8[0][x] = *reinterpret_cast<const Vec*>(sRow[st] + ((x * 2 + q) * MT * TN + mt * TN + j) * 16);
-                    typename MM::Acc sum[1] = {acc_zero<T>()};
-                    mma_parts<float, 1>(a8, b8, sum);
-                    acc[mt] += sum[0];
+#pragma unroll
+                    for (int u = 0; u < CT; ++u) {
+                        if constexpr (NP > 1) {
+                            typename MM::Acc sum[1] = {acc_zero<T>()};
+                            mma_parts<S, 1>(a8, b8[u], sum);
+                            acc[u][mt] += sum[0];
+                        } else
+                            mma_parts<S, 1>(a8, b8[u], &acc[u][mt]);
+                    }
                 }
             }
             put_rows(st ^ 1);
             __syncthreads();
         }
     }
-    const bool redo = works && __any(!results_stand<MT, float>(acc));
+    bool stands = true;
+#pragma unroll
+    for (int u = 0; u < CT; ++u) stands = stands && results_stand<MT, S>(acc[u]);
+    const bool redo = works && __any(!stands);
     // One row tile from the values themselves, two positions at a time, with the reference's corners.  (Its own accumulator, after
     // the loop above: a second loop over `acc` doubled the registers of the kernel.)
-    auto exact_tile = [&](int mt) {
+    auto exact_tile = [&](int u, int mt) {
         typename MM::Acc x = acc_zero<T>();
         for (int slab = first; slab < last; slab += turn) {
             const int n = slab / slabs_per_sample;
             const unsigned p0 = (unsigned)(slab % slabs_per_sample) * TN;
-            const T* off_n = PLAIN ? nullptr : off + (((size_t)n * P.DG + dg) * P.kV + tap) * ND * P.outV;
+            const S* off_n = PLAIN ? nullptr : off + (((size_t)n * P.DG + dg) * P.kV + tap) * ND * P.outV;
             const char* in_n = reinterpret_cast<const char*>(in_cl + (size_t)n * P.inV * P.C_in);
 #pragma unroll 1
             for (int ks = 0; ks < TN; ks += 2) {
@@ -260,7 +290,7 @@ __global__ __launch_bounds__(WG, MT == 4 ? 3 : 4) void backward_weight_split_ker
                 for (int a = 0; a < ND; ++a) ib[a] = o[a] * P.stride[slot<ND>(a)] - P.pad[slot<ND>(a)];
                 T offv[ND];
 #pragma unroll
-                for (int a = 0; a < ND; ++a) offv[a] = PLAIN ? 0.f : off_n[(size_t)a * P.outV + posc];
+                for (int a = 0; a < ND; ++a) offv[a] = PLAIN ? 0.f : Store<S>::ld(off_n[(size_t)a * P.outV + posc]);
                 TapGeo<T, ND> t;
                 tap_setup_noidx<T, ND>(P, offv, ib, kd, t);
                 const bool live = pos < P.outV && t.inside;
@@ -272,11 +302,12 @@ __global__ __launch_bounds__(WG, MT == 4 ? 3 : 4) void backward_weight_split_ker
                     T w = 1.f;
 #pragma unroll
                     for (int a = 0; a < ND; ++a) w *= PLAIN ? 1.f : (i >> (ND - 1 - a)) & 1 ? t.f[a] : 1.f - t.f[a];
-                    v += w * *reinterpret_cast<const T*>(in_n + (cb[i] + cjB));
+                    v += w * Store<S>::ld(*reinterpret_cast<const S*>(in_n + (cb[i] + cjB + u * (unsigned)sizeof(S))));
                 }
+                if constexpr (CT > 1) v = (T)(typename PT::Elem)v;         // rounded like the operand
                 const T b = live ? v : 0.f;
                 const int m = min(m_base + mt * TN + j, P.M - 1);
-                const T av = pos < P.outV ? gout[((size_t)n * P.C_out + g * P.M + m) * P.outV + posc] : 0.f;
+                const T av = pos < P.outV ? Store<S>::ld(gout[((size_t)n * P.C_out + g * P.M + m) * P.outV + posc]) : 0.f;
                 x = MM::mma(av, b, x);
             }
         }
@@ -284,15 +315,17 @@ __global__ __launch_bounds__(WG, MT == 4 ? 3 : 4) void backward_weight_split_ker
     };
 
     if (!works) return;                                 // (uniform for the wavefront)
-    T* pt = partial + ((size_t)split * P.kV + tap) * P.C_out * P.Cg + (size_t)g * P.M * P.Cg + (c0 + j - g * P.Cg);
+    T* pt = partial + ((size_t)split * P.kV + tap) * P.C_out * P.Cg + (size_t)g * P.M * P.Cg + (c0 + j * CT - g * P.Cg);
+#pragma unroll
+    for (int u = 0; u < CT; ++u)
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) {
-        typename MM::Acc x = acc[mt] * sgn;
-        if (__builtin_expect(redo, 0)) x = exact_tile(mt);
+        typename MM::Acc x = acc[u][mt] * sgn;
+        if (__builtin_expect(redo, 0)) x = exact_tile(u, mt);
 #pragma unroll
         for (int r = 0; r < MM::NACC; ++r) {
             const int m = m_base + mt * TN + MM::row(r, q);
-            if (m < P.M && c0 + j < ce) pt[(size_t)m * P.Cg] = x[r];
+            if (m < P.M && c0 + j * CT + u < ce) pt[(size_t)m * P.Cg + u] = x[r];
         }
     }
 }

@@ -117,12 +117,13 @@ __device__ inline void prep_channels_last(const PrepJob& job, unsigned block) {
 
 // grad_output in the operand order of backward_weight_split_kernel, and its sums: 32 channels of a strip, 64 positions at a
 // time through LDS, then eight positions of one channel to a thread.
+template <typename S>
 __device__ inline void prep_rows(const PrepJob& job, unsigned block) {
-    using PT = Parts<float>;
-    __shared__ float tile[32][65];
+    using PT = Parts<S>;
+    __shared__ S tile[32][sizeof(S) == 4 ? 65 : 66];
     const unsigned strips = last_strips(job.V), ctiles = ((unsigned)job.C + 31) / 32;
     const unsigned strip = block % strips, c0 = (block / strips) % ctiles * 32, n = block / strips / ctiles;
-    const float* src = static_cast<const float*>(job.src) + (size_t)n * job.C * job.V;
+    const S* src = static_cast<const S*>(job.src) + (size_t)n * job.C * job.V;
     const unsigned steps = row_steps(job.V), tx = threadIdx.x & 63, ty = threadIdx.x >> 6, c = c0 + (threadIdx.x & 31), oct = threadIdx.x >> 5;
     typename PT::Vec* dst = static_cast<typename PT::Vec*>(job.dst) + (size_t)n * steps * PT::NP * 2 * job.C;
     float sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -130,9 +131,10 @@ __device__ inline void prep_rows(const PrepJob& job, unsigned block) {
 #pragma unroll
         for (unsigned k = 0; k < 8; ++k) {
             const unsigned ch = ty + 4 * k, v = v0 + tx;
-            const float x = c0 + ch < (unsigned)job.C && v < job.V ? src[(size_t)(c0 + ch) * job.V + v] : 0.f;
+            S x = S();
+            if (c0 + ch < (unsigned)job.C && v < job.V) x = src[(size_t)(c0 + ch) * job.V + v];
             tile[ch][tx] = x;
-            sum[k] += x;
+            sum[k] += Store<S>::ld(x);
         }
         __syncthreads();
         const unsigned step = (v0 >> 4) + (oct >> 1);
@@ -215,7 +217,7 @@ __global__ __launch_bounds__(256) void backward_prepare_kernel(Params P, PlanCho
             break;
         }
         case PREP_ROWS:
-            if constexpr (sizeof(S) == 4) prep_rows(job, block);
+            if constexpr (sizeof(S) <= 4) prep_rows<S>(job, block);
             break;
         default: prep_channels_last<T, S>(job, block); break;
     }

@@ -24,7 +24,7 @@ def _weight_gradient(c):
     import deform_conv3d_pytorch_op_amd as dcn
     fn = dcn.ConvOffset3dFunction if c["nd"] == 3 else dcn.ConvOffset2dFunction
     x, off, w = (c[k].cuda().requires_grad_(k == "w") for k in ("x", "off", "w"))
-    b = torch.zeros(w.shape[0], device="cuda").requires_grad_(True)
+    b = torch.zeros(w.shape[0], device="cuda", dtype=w.dtype).requires_grad_(True)
     fn.apply(x, off, w, b, c["stride"], c["pad"], c["dil"], c["cpg"], c["groups"]).backward(c["gout"].cuda())
     return w.grad.cpu().double(), b.grad.cpu().double()
 
@@ -49,6 +49,36 @@ def test_layers(spec):
     g64 = c["gout"].double()
     sums = g64.sum(dim=[0] + list(range(2, g64.dim())))
     assert ((bias - sums).norm() / sums.norm()).item() <= 4e-6
+
+
+# 16-bit storage: pairs of channels, so even segments
+LAYERS16 = [
+    (2, 1, 34, 70, (129, 161), 3, 1, 1, 1, 34, 1, 1.5), (2, 2, 66, 40, (129, 161), 3, 1, 1, 1, 66, 1, 3.0),
+    (2, 1, 24, 120, (141, 99), 3, 1, 1, 1, 8, 2, 2.0), (3, 1, 20, 64, (9, 32, 33), 3, 1, 1, 1, 10, 1, 1.5),
+    (3, 1, 40, 97, (7, 31, 32), 3, 1, 1, 1, 40, 1, 2.5), (3, 1, 2, 60, (1, 95, 97), 3, 1, 1, 1, 2, 1, 1.0),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("spec", LAYERS16, ids=IDS)
+def test_layers_16bit(spec, dtype):
+    """Samples and results are rounded to the storage format, each off by half a unit in its last place at most: 2-norm
+    below 2^-9 and 2^-12 each.  Non-finite input reaches the elements that it reaches in the oracle."""
+    print("weight gradient", spec, dtype, flush=True)
+    c = make_case(*spec, dtype=dtype, seed=45, bias=False)
+    got, bias = _weight_gradient(c)
+    want = _oracle(c)
+    once = {torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}[dtype]
+    assert ((got - want).norm() / want.norm()).item() <= 2 * once
+    g64 = c["gout"].double()
+    sums = g64.sum(dim=[0] + list(range(2, g64.dim())))
+    assert ((bias - sums).norm() / sums.norm()).item() <= once + 4e-6
+    c["x"][0, -1].view(-1)[-3:] = torch.tensor([float("inf"), float("nan"), -float("inf")])
+    got, _ = _weight_gradient(c)
+    want = _oracle(c)
+    fin = torch.isfinite(want)
+    assert not fin.all() and torch.equal(torch.isfinite(got), fin)
+    assert ((got - want)[fin].norm() / want[fin].norm()).item() <= 2 * once
 
 
 @pytest.mark.parametrize("spec", [LAYERS[0], LAYERS[6]], ids=IDS)
