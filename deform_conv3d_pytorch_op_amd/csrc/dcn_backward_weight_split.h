@@ -4,11 +4,11 @@
 //
 // replaces the second deformable_im2col + Sgemm(beta=1) of deform3d/lib/deform_conv3d_cuda.cpp:283-320.
 //
-// The reduction runs over positions.  A wavefront samples 32 channels of one tap (16-bit storage: 64, two to a lane): lane (j, q) takes channel c0 + j at eight
-// consecutive positions of a step of 16 -- the input is channels-last, so a corner is one coalesced 128-byte read of the
-// lane group -- and those eight samples are the lane's operand of v_mfma_f32_32x32x16_bf16 as they stand: three bfloat16
-// parts or one of the storage format (dcn_forward_split.h).  The other operand, the rows of grad_output, comes from the preparing launch in operand order
-// (prep_rows); the four wavefronts of a workgroup work taps or channel tiles of their own on the same positions and share it
+// The reduction runs over positions.  A wavefront samples 32 channels of one tap (16-bit storage: 64, two to a lane): lane
+// (j, q) takes channel c0 + j at eight consecutive positions of a step of 16 -- the input is channels-last, so a corner is one
+// coalesced 128-byte read of the lane group -- and those eight samples are the lane's operand of v_mfma_f32_32x32x16_bf16 / _f16
+// as they stand: three bfloat16 parts or one of the storage format (dcn_forward_split.h).  The other operand, the rows of
+// grad_output, comes from the preparing launch in operand order (prep_rows); the four wavefronts of a workgroup work taps or channel tiles of their own on the same positions and share it
 // through LDS, two steps of it in turn.  The geometry of a slab of 32 positions is worked out once by the position-owning
 // lanes and handed to the channel lanes through a wavefront-private record: byte offset of the low corner and the corner
 // weights.  The low corner is at most size - 2, so that the other corners lie at fixed strides (scalar bases of their own, one
@@ -28,7 +28,7 @@
 // straight from L2 this kernel was no faster in 3-D (678 us against 633) and 13 % faster in 2-D.  us, that kernel -> this one: 256 -> 256,
 // 3x3, 8 x 56 x 56: 332 -> 240; 512 -> 512 in two groups, 3x3, 4 x 28 x 28: 105 -> 80; 128 -> 128, 3x3x3, 2 x 16 x 56 x 56
 // (stride 2): 1022 -> 860; 64 -> 64 as above: 633 -> 600; 64 -> 64, 3x3, no offsets, 25 088 positions: 33 -> 25.
-// The preparing launch pays 4 to 30 us of it back (three halves of the bytes of a channels-last copy).
+// The preparing launch pays 2 to 20 us of it back (three halves of the bytes of a channels-last copy).
 // 16-bit storage, against backward_weight16_kernel, which samples once for every 64 output channels: 256 -> 256 in float16 150 -> 116,
 // 64 -> 64 in 3-D in bfloat16 361 -> 326.
 #pragma once

@@ -3,9 +3,8 @@
 // cleared gradients, channels-last copies with the sums of grad_output for grad_bias -- and each is a
 // few microseconds of work: as launches of their own they cost a small layer more than the kernels they prepare
 // (2 x 8 x 16 x 16 float64: eight launches of 1 to 6 us with gaps of 5 to 17 us between them).
-// Large layers are bound by the copies: 64 -> 64 channels, 3-D, 4 x 16 x 56 x 56 float32, 322 MB in 79 us (4.1 TB/s; a plain
-// copy reaches 5.2), where the jobs one by one took 91 us and the sum of grad_output over two axes 73; 256 -> 256, 2-D,
-// 8 x 56 x 56: 25 against 50 and 12; 128 -> 128, 3-D, 2 x 16 x 112 x 112 -> 56 x 56: 175 against 220 and 42.
+// Large layers are bound by the copies: 64 -> 64 channels, 3-D, 4 x 16 x 56 x 56 float32, 411 MB in 100 us (4.1 TB/s; a plain
+// copy reaches 5.1); 256 -> 256, 2-D, 8 x 56 x 56: 46 us; 128 -> 128, 3-D, 2 x 16 x 112 x 112 -> 56 x 56: 871 MB in 197.
 #pragma once
 #include "dcn_backward_fused.h"
 #include "dcn_backward_weight_split.h"
@@ -86,17 +85,24 @@ __device__ inline void prep_channels_last(const PrepJob& job, unsigned block) {
     S* dst = static_cast<S*>(job.dst) + base;
     const unsigned tx = threadIdx.x & 31, ty = threadIdx.x >> 5;
     T sum[4] = {0, 0, 0, 0};
-    for (unsigned v0 = strip * LAST_STRIP; v0 < min((strip + 1) * LAST_STRIP, job.V); v0 += 32) {
+    // The next tile's values are on their way while this one is written; clamped, so that no load is masked.  (The launch was bounded
+    // by the round trips to memory; us, a tile at a time -> so: 128 -> 128 channels in 3-D as above 244 -> 197, 64 -> 64 127 -> 100,
+    // 256 -> 256 57 -> 46; a plain convolution of 25 088 positions 20 -> 12.  Tiles of 64 voxels are no faster.)
+    S x[4];
+    auto load = [&](unsigned v0) {
+#pragma unroll
+        for (unsigned k = 0; k < 4; ++k) x[k] = src[(size_t)min(c0 + ty + 8 * k, (unsigned)job.C - 1) * job.V + min(v0 + tx, job.V - 1)];
+    };
+    const unsigned end = min((strip + 1) * LAST_STRIP, job.V);
+    load(strip * LAST_STRIP);
+    for (unsigned v0 = strip * LAST_STRIP; v0 < end; v0 += 32) {
 #pragma unroll
         for (unsigned k = 0; k < 4; ++k) {
-            const unsigned c = c0 + ty + 8 * k, v = v0 + tx;
-            if (c < (unsigned)job.C && v < job.V) {
-                const S x = src[(size_t)c * job.V + v];
-                tile[ty + 8 * k][tx] = x;
-                sum[k] += (T)Store<S>::ld(x);
-            }
+            tile[ty + 8 * k][tx] = x[k];
+            if (v0 + tx < job.V) sum[k] += (T)Store<S>::ld(x[k]);
         }
         __syncthreads();
+        load(v0 + 32);
 #pragma unroll
         for (unsigned k = 0; k < 4; ++k) {
             const unsigned v = v0 + ty + 8 * k, c = c0 + tx;
@@ -127,16 +133,22 @@ __device__ inline void prep_rows(const PrepJob& job, unsigned block) {
     const unsigned steps = row_steps(job.V), tx = threadIdx.x & 63, ty = threadIdx.x >> 6, c = c0 + (threadIdx.x & 31), oct = threadIdx.x >> 5;
     typename PT::Vec* dst = static_cast<typename PT::Vec*>(job.dst) + (size_t)n * steps * PT::NP * 2 * job.C;
     float sum[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    for (unsigned v0 = strip * LAST_STRIP; v0 < min((strip + 1) * LAST_STRIP, job.V); v0 += 64) {
+    S x[8];                                             // (as in prep_channels_last)
+    auto load = [&](unsigned v0) {
+#pragma unroll
+        for (unsigned k = 0; k < 8; ++k) x[k] = src[(size_t)min(c0 + ty + 4 * k, (unsigned)job.C - 1) * job.V + min(v0 + tx, job.V - 1)];
+    };
+    const unsigned end = min((strip + 1) * LAST_STRIP, job.V);
+    load(strip * LAST_STRIP);
+    for (unsigned v0 = strip * LAST_STRIP; v0 < end; v0 += 64) {
 #pragma unroll
         for (unsigned k = 0; k < 8; ++k) {
-            const unsigned ch = ty + 4 * k, v = v0 + tx;
-            S x = S();
-            if (c0 + ch < (unsigned)job.C && v < job.V) x = src[(size_t)(c0 + ch) * job.V + v];
-            tile[ch][tx] = x;
-            sum[k] += Store<S>::ld(x);
+            if (v0 + tx >= job.V) x[k] = S();
+            tile[ty + 4 * k][tx] = x[k];
+            sum[k] += Store<S>::ld(x[k]);
         }
         __syncthreads();
+        load(v0 + 64);
         const unsigned step = (v0 >> 4) + (oct >> 1);
         if (c < (unsigned)job.C && step < steps) {
             typename PT::Vec p8[PT::NP];
