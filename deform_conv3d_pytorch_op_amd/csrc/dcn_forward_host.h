@@ -117,7 +117,9 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
     // 2.0 (3-D) or 0.8 for a wavefront's step, 0.4 for a thread's cell to stage, 5 for joining parts, 2 for sixteen wavefronts.  One sample,
     // float32, with / without: 2-D, 64 -> 64, 75 x 101: 20.4 / 33; 48 -> 64, 5x5, 70 x 76: 25 / 49; 3-D, 128 -> 32 at stride 1 2 2, 14 x 20 x 20:
     // 65 / 102; two samples of 32 -> 16, 15 x 18 x 18: 30 / 55; 70 layers of 8 to 256 channels and 150 to 16 000
-    // positions, 2-D and 3-D, also in bfloat16: 0.85 of the time on average, 49 faster, at worst 1.06.
+    // positions, 2-D and 3-D, also in bfloat16: 0.85 of the time on average.  Only where the estimate falls by a fifth: of 60 layers
+    // below 6e6 samples those taken for less of it are the slower ones (320 -> 16, 3x3 at stride 2, 27 x 25: 25.4 / 27.9; 3-D, 32 -> 49 in
+    // deformable groups of 8, 9 x 13 x 14: 24.5 / 26.2; without the line 0.867 of the time on average, with it 0.862, at worst 1.005).
     int tiny = 0;
     if (small && MT <= 2 && forward_tiny()) {
         const size_t room = ws_bytes > wq_bound ? (ws_bytes - wq_bound < FWD_PARTIAL_CAP ? ws_bytes - wq_bound : FWD_PARTIAL_CAP) : 0;
@@ -153,7 +155,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             if (!plan_halo<T, ND>(Pt, MAX_LDS, default_margin(), 1 << 30, sizeof(S), t, true, FG, nullptr, 1, false)) continue;
             for (int fs = 1; parts_fit(fs) && (long long)Pt.N * Pt.tiles * P.G * P.mchunks * fs <= cu_count(); fs *= 2) {
                 const double e = estimate(Pt, t, 16 / t, fs);
-                if (e < best) { best = e; tiny = t; fsplit = fs; }
+                if (e < (tiny ? best : 0.8 * best)) { best = e; tiny = t; fsplit = fs; }
             }
         }
     }
