@@ -57,7 +57,7 @@ int backward_weight(const Geometry& g, const T* in, const T* off, const T* gout,
     WeightCall<T, T> call;
     Prep prep;
     const PlanChoice none = {};
-    if (int rc = backward_weight_plan<T, ND, T>(P, in, gout, ws, ws_bytes, false, call, prep, nullptr)) return rc;
+    if (int rc = backward_weight_plan<T, ND, T>(P, in, off, gout, ws, ws_bytes, false, call, prep, nullptr)) return rc;
     if (int rc = launch_prepare<T, T>(P, none, prep, static_cast<const T*>(nullptr), off, 0, s)) return rc;
     return backward_weight_run<T, ND, T>(call, off, gw, nullptr, true, s);
 }
@@ -131,7 +131,7 @@ int backward_weight16(const Geometry& g, const S* in, const S* off, const S* gou
         WeightCall<float, S> call;
         Prep prep;
         const PlanChoice none = {};
-        if (int rc = backward_weight_plan<float, ND, S>(P, in, gout, c.p, c.left, false, call, prep, &declined)) return rc;
+        if (int rc = backward_weight_plan<float, ND, S>(P, in, off, gout, c.p, c.left, false, call, prep, &declined)) return rc;
         if (!declined) {
             if (int rc = launch_prepare<float, S>(P, none, prep, static_cast<const S*>(nullptr), off, 0, s)) return rc;
             if (int rc = backward_weight_run<float, ND, S>(call, off, fgw, nullptr, true, s)) return rc;
@@ -205,7 +205,7 @@ int layer_backward(const Geometry& g, const S* in, const S* w, const S* off, con
     // (16-bit storage: the kernels that read it may decline a layer, which then runs on widened copies)
     bool wdeclined = S16 && !native16(), ddeclined = wdeclined;
     if (gw && !wdeclined)
-        if (int rc = backward_weight_plan<T, ND, S>(P, in, gout, wws, wbytes, gb != nullptr, call, prep, S16 ? &wdeclined : nullptr)) return rc;
+        if (int rc = backward_weight_plan<T, ND, S>(P, in, off, gout, wws, wbytes, gb != nullptr, call, prep, S16 ? &wdeclined : nullptr)) return rc;
     if (data && !ddeclined)
         if (int rc = backward_input_offset<T, ND, S>(g, in, w, off, gout, tgin, tgoff, dws, dbytes, s, flags, S16 ? &ddeclined : nullptr, &prep)) return rc;
     if (!data || ddeclined)
@@ -229,7 +229,7 @@ int layer_backward(const Geometry& g, const S* in, const S* w, const S* off, con
     } else if (gw) {
         WeightCall<T, T> wide;
         Prep wprep;
-        if (int rc = backward_weight_plan<T, ND, T>(P, fin, fgout, wws, wbytes, gb != nullptr, wide, wprep, nullptr)) return rc;
+        if (int rc = backward_weight_plan<T, ND, T>(P, fin, foff, fgout, wws, wbytes, gb != nullptr, wide, wprep, nullptr)) return rc;
         if (int rc = launch_prepare<T, T>(P, none, wprep, fw, foff, 0, s)) return rc;
         if (int rc = backward_weight_run<T, ND, T>(wide, foff, tgw, tgb, false, s)) return rc;
     }
@@ -336,7 +336,7 @@ int conv2d_layer_backward(Geometry g, const T* in, const T* w, const T* gout, T*
     Prep prep;
     const PlanChoice none = {};
     const T* off = nullptr;
-    if (int rc = backward_weight_plan<T, 2, T>(P, in, gout, ws, wbytes, gb != nullptr, call, prep, nullptr)) return rc;
+    if (int rc = backward_weight_plan<T, 2, T>(P, in, off, gout, ws, wbytes, gb != nullptr, call, prep, nullptr)) return rc;
     if (int rc = launch_prepare<T, T>(P, none, prep, w, off, 0, s)) return rc;
     return backward_weight_run<T, 2, T>(call, off, gw, gb, false, s);
 }

@@ -40,8 +40,8 @@ void bww_plan(const Params& Pin, int& MT, int& mchunks, int& nct, int& nsplit, l
     nsplit = (int)split;
 }
 
-// Channel tiles of the convolution group that has the most, times taps.
-inline int split_items(const Params& P, int TC) {
+// Channel tiles of TC channels of the convolution group that has the most, times groups of TP taps.
+inline int split_items(const Params& P, int TC, int TP) {
     int most = 0;
     for (int g = 0; g < P.G; ++g) {
         int n = 0;
@@ -51,7 +51,7 @@ inline int split_items(const Params& P, int TC) {
         }
         most = n > most ? n : most;
     }
-    return most * P.kV;
+    return most * ((P.kV + TP - 1) / TP);
 }
 // backward_weight_split_kernel takes layers of more than 32 output channels to a group, with items for the four wavefronts of a
 // workgroup (not a single tap of few channels) and work for the device: 2.5 slabs to a resident wavefront.  Below, the longer
@@ -60,19 +60,53 @@ inline int split_items(const Params& P, int TC) {
 // 177 : 184; 96 -> 128, 3x3, 7296 positions 157 : 162); above, this one wins (32 -> 113, 3x3x3, 3456 positions 202 : 183; 16 -> 80, 16 000
 // positions 228 : 203; 12 -> 57, 62 000 positions 750 : 698).  Its wavefronts write a partial tile each: about one round of resident
 // workgroups, as long as the tiles (written and read at about 8 TB/s) cost less than the longer runs of slabs.
-struct SplitPlan { int MT, mchunks, igroups, nsplit; };     // nsplit 0: not a layer for it, or no room
+template <typename S> using RowOps = typename Parts<S>::Vec;
+template <typename S> using SplitFn = void (*)(Params, const S*, const S*, const S*, const RowOps<S>*, float*, unsigned);
 template <int ND, typename S>
-SplitPlan split_plan(const Params& P, size_t room) {
+SplitFn<S> split_kernel(int MT, int LW, bool plain) {
+    if constexpr (ND == 2 && sizeof(S) == 4)
+        if (plain) return MT == 4 ? backward_weight_split_kernel<ND, 4, 32, S, true> : backward_weight_split_kernel<ND, 2, 32, S, true>;
+    switch (MT * 100 + LW) {
+        case 108: return backward_weight_split_kernel<ND, 1, 8, S>;
+        case 116: return backward_weight_split_kernel<ND, 1, 16, S>;
+        case 208: return backward_weight_split_kernel<ND, 2, 8, S>;
+        case 216: return backward_weight_split_kernel<ND, 2, 16, S>;
+        case 132: case 232: return backward_weight_split_kernel<ND, 2, 32, S>;
+        case 408: return backward_weight_split_kernel<ND, 4, 8, S>;
+        case 416: return backward_weight_split_kernel<ND, 4, 16, S>;
+        default: return backward_weight_split_kernel<ND, 4, 32, S>;
+    }
+}
+// Lanes to a tap: 16 or 8 where a segment fits them and that makes fewer items, at 1.05 and 1.2 items for one of 32: eight lanes read 32
+// bytes of a corner.  (Longer segments read their cache lines in parts then: 80 -> 96, 3-D, 23 600 positions 406 us a step with 32, 431 with 16.)  Layers of up to 32 output channels, too, if it takes a third off them; the
+// first threshold counts items of 32 lanes.  50 training layers, us per step, 32 lanes (or the other
+// kernels) : this: 1.058 times as fast on average, at worst 0.994; 16 -> 38 in groups of 4, 3-D, two samples of 16 700 positions in bfloat16 464 : 322; 20 -> 339 in
+// groups of 5, 7200 positions 301 : 245; 16 -> 14, 165 000 positions in bfloat16 734 : 602; 24 -> 36 in groups of 6, 10 600 positions 184 : 162.
+struct SplitPlan { int MT, LW, mchunks, igroups, nsplit; };     // nsplit 0: not a layer for it, or no room
+template <int ND, typename S>
+SplitPlan split_plan(const Params& P, bool off, size_t room) {
     SplitPlan c = {};
-    const int items = split_items(P, tile_channels<S>());
-    c.MT = P.M > 64 ? 4 : 2;
+    const int whole = split_items(P, 32 * lane_channels<S>(), 1);
+    int items = whole;
+    double least = whole;
+    c.LW = 32;
+    const int longest = P.cpg < P.Cg ? P.cpg : P.Cg;
+    for (int lw : {16, 8}) {
+        if (longest > lw * lane_channels<S>()) continue;
+        const int n = split_items(P, lw * lane_channels<S>(), 32 / lw);
+        const double cost = n * (lw == 8 ? 1.2 : 1.05);
+        if (cost >= least || !off) continue;
+        least = cost;
+        items = n;
+        c.LW = lw;
+    }
+    c.MT = P.M > 64 ? 4 : P.M > 32 ? 2 : 1;
     c.mchunks = ((P.M + 31) / 32 + c.MT - 1) / c.MT;
     c.igroups = (items + WAVES - 1) / WAVES;
-    const double resident = (double)resident_workgroups(c.MT == 4 ? reinterpret_cast<const void*>(backward_weight_split_kernel<ND, 4, S>)
-                                                         : reinterpret_cast<const void*>(backward_weight_split_kernel<ND, 2, S>), WG, 0);
+    const double resident = (double)resident_workgroups(reinterpret_cast<const void*>(split_kernel<ND, S>(c.MT, c.LW, false)), WG, 0);
     const long long nslabs = (long long)P.N * (row_steps(P.outV) / 2);
     const double other = (double)c.igroups * c.mchunks * P.G;
-    if (P.M <= 32 || items < WAVES || (double)items * c.mchunks * P.G * (double)nslabs < 2.5 * WAVES * resident) return c;
+    if ((P.M <= 32 && least > 0.67 * whole) || items < WAVES || (double)whole * c.mchunks * P.G * (double)nslabs < 2.5 * WAVES * resident) return c;
     const size_t one = (size_t)P.kV * P.C_out * P.Cg * sizeof(float);
     long long most = (long long)(room / one);
     if (most > 256) most = 256;
@@ -126,7 +160,7 @@ int launch_bwd_weight(const WeightCall<T, T>& c, const T* off, hipStream_t s) {
 // and deformable groups -- that start at odd channels), where the float32 kernel is the faster one, or
 // where the workspace is too small.
 template <typename T, int ND, typename S>
-int backward_weight_plan(const Params& Pin, const S* in, const S* gout, void* ws, size_t ws_bytes, bool bias, WeightCall<T, S>& c, Prep& prep, bool* declined) {
+int backward_weight_plan(const Params& Pin, const S* in, const S* off, const S* gout, void* ws, size_t ws_bytes, bool bias, WeightCall<T, S>& c, Prep& prep, bool* declined) {
     constexpr bool S16 = !std::is_same<S, T>::value;
     Params& P = c.P;
     P = Pin;
@@ -187,10 +221,10 @@ int backward_weight_plan(const Params& Pin, const S* in, const S* gout, void* ws
     if constexpr (sizeof(S) <= 4) {
         const size_t rbytes = align256(row_operand_bytes<S>(P.N, P.C_out, P.outV));
         const size_t used = ibytes + rbytes + (bias ? (size_t)P.N * last_strips(P.outV) * P.C_out * sizeof(T) : 0) + 256;
-        const SplitPlan sp = split_plan<ND, S>(P, ws && ws_bytes > used ? ws_bytes - used : 0);
+        const SplitPlan sp = split_plan<ND, S>(P, off != nullptr, ws && ws_bytes > used ? ws_bytes - used : 0);
         if (sp.nsplit) {
             obytes = rbytes;
-            c.MT = sp.MT; c.igroups = sp.igroups; P.mchunks = sp.mchunks; P.nsplit = sp.nsplit;
+            c.MT = sp.MT; c.LW = sp.LW; c.igroups = sp.igroups; P.mchunks = sp.mchunks; P.nsplit = sp.nsplit;
         }
     }
     const size_t pbytes = align256((size_t)P.nsplit * P.kV * P.C_out * P.Cg * sizeof(T));
@@ -208,14 +242,11 @@ int backward_weight_plan(const Params& Pin, const S* in, const S* gout, void* ws
     return DCN_OK;
 }
 
-template <int ND, int MT, typename S>
+template <int ND, typename S>
 int launch_bwd_weight_split(const WeightCall<float, S>& c, const S* off, hipStream_t s) {
     const Params& P = c.P;
     const dim3 grid((unsigned)((long long)c.igroups * P.mchunks * P.G * P.nsplit));
-    auto kern = backward_weight_split_kernel<ND, MT, S>;
-    if constexpr (ND == 2 && sizeof(S) == 4)
-        if (!off) kern = backward_weight_split_kernel<ND, MT, S, true>;
-    hipLaunchKernelGGL(kern, grid, dim3(WG), 0, s, P, (const S*)c.in_cl, off, c.gout, reinterpret_cast<const typename Parts<S>::Vec*>(c.gout_cl), c.partial, (unsigned)c.igroups);
+    hipLaunchKernelGGL((split_kernel<ND, S>(c.MT, c.LW, !off)), grid, dim3(WG), 0, s, P, (const S*)c.in_cl, off, c.gout, reinterpret_cast<const typename Parts<S>::Vec*>(c.gout_cl), c.partial, (unsigned)c.igroups);
     return check_launch("backward_weight_split_kernel");
 }
 
@@ -224,7 +255,7 @@ int backward_weight_run(const WeightCall<T, S>& c, const S* off, T* gw, T* gb, b
     const Params& P = c.P;
     if (c.igroups) {
         if constexpr (sizeof(T) == 4)
-            if (int rc = c.MT == 4 ? launch_bwd_weight_split<ND, 4, S>(c, off, s) : launch_bwd_weight_split<ND, 2, S>(c, off, s)) return rc;
+            if (int rc = launch_bwd_weight_split<ND, S>(c, off, s)) return rc;
     } else if constexpr (std::is_same<S, T>::value) {
         int rc;
         switch (c.MT) {
@@ -249,7 +280,7 @@ int backward_weight_run(const WeightCall<T, S>& c, const S* off, T* gw, T* gb, b
 }
 
 #define INSTANTIATE(T, ND, S)                                                                                                                            \
-    template int backward_weight_plan<T, ND, S>(const Params&, const S*, const S*, void*, size_t, bool, WeightCall<T, S>&, Prep&, bool*);           \
+    template int backward_weight_plan<T, ND, S>(const Params&, const S*, const S*, const S*, void*, size_t, bool, WeightCall<T, S>&, Prep&, bool*);           \
     template int backward_weight_run<T, ND, S>(const WeightCall<T, S>&, const S*, T*, T*, bool, hipStream_t);
 INSTANTIATE(float, 2, float) INSTANTIATE(float, 3, float) INSTANTIATE(double, 2, double) INSTANTIATE(double, 3, double)
 INSTANTIATE(float, 2, Bf16) INSTANTIATE(float, 3, Bf16) INSTANTIATE(float, 2, Fp16) INSTANTIATE(float, 3, Fp16)

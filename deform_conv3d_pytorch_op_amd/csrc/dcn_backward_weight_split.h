@@ -1,10 +1,12 @@
-// Backward pass to the weight of the float32 and 16-bit operators, for layers of more than 32 output channels to a group (split_plan).
+// Backward pass to the weight of the float32 and 16-bit operators, for layers of more than 32 output channels to a group or few channels
+// to a segment (split_plan).
 //
 //   gW[g*M+m][cl][tap] += sum_{n,pos} grad_output[n][g*M+m][pos] * sample(in[n][g*Cg+cl], tap, pos)
 //
 // replaces the second deformable_im2col + Sgemm(beta=1) of deform3d/lib/deform_conv3d_cuda.cpp:283-320.
 //
-// The reduction runs over positions.  A wavefront samples 32 channels of one tap (16-bit storage: 64, two to a lane): lane
+// The reduction runs over positions.  A wavefront samples 32 channels of one tap (16-bit storage: 64, two to a lane; few channels: LW lanes
+// to each of 32 / LW taps): lane
 // (j, q) takes channel c0 + j at eight consecutive positions of a step of 16 -- the input is channels-last, so a corner is one
 // coalesced 128-byte read of the lane group -- and those eight samples are the lane's operand of v_mfma_f32_32x32x16_bf16 / _f16
 // as they stand: three bfloat16 parts or one of the storage format (dcn_forward_split.h).  The other operand, the rows of
@@ -40,8 +42,8 @@ constexpr unsigned ROW_SLAB = 32;                       // positions of a slab: 
 __host__ __device__ inline unsigned row_steps(unsigned V) { return (V + ROW_SLAB - 1) / ROW_SLAB * 2; }
 // grad_output in operand order: [n][step][part][q][output channel], 16 bytes (eight positions) each, zero past the volume
 template <typename S> inline size_t row_operand_bytes(int N, int C_out, size_t V) { return (size_t)N * row_steps((unsigned)V) * Parts<S>::NP * 2 * C_out * 16; }
-// channels of a channel tile: those of a 128-byte read by the 32 lanes of a group (16-bit storage: pairs, two columns tiles)
-template <typename S> __host__ __device__ constexpr int tile_channels() { return 128 / (int)sizeof(S); }
+// channels to a lane (16-bit storage: pairs, two column tiles)
+template <typename S> __host__ __device__ constexpr int lane_channels() { return 4 / (int)sizeof(S); }
 
 // channel u of what a lane reads of a corner
 template <typename S> __device__ inline float channel_of(float v, int) { return v; }
@@ -50,9 +52,9 @@ template <typename S> __device__ inline float channel_of(unsigned v, int u) {
     else return (float)__builtin_bit_cast(_Float16, (unsigned short)(u ? v >> 16 : v));
 }
 
-// MT row tiles to a workgroup.  PLAIN: a plain convolution (off is null): samples at integer coordinates are their low corner alone.
-// Grid: igroups * mchunks * G * nsplit workgroups.  An item is a tap of a channel tile of the convolution group, tap fastest.
-template <int ND, int MT, typename S, bool PLAIN = false>
+// MT row tiles to a workgroup.  LW lanes to a tap: an item is 32 / LW taps of LW channels (pairs).  PLAIN: a plain convolution (off is null): samples at integer coordinates are their low corner alone.
+// Grid: igroups * mchunks * G * nsplit workgroups.  The items of a convolution group: taps of a channel tile, taps fastest.
+template <int ND, int MT, int LW, typename S, bool PLAIN = false>
 __global__ __launch_bounds__(WG, (MT == 4 ? 3 : 4) - (sizeof(S) == 2)) void backward_weight_split_kernel(Params P, const S* __restrict__ in_cl, const S* __restrict__ off,
                                                                                          const S* __restrict__ gout,
                                                                                          const typename Parts<S>::Vec* __restrict__ rows,
@@ -61,10 +63,11 @@ __global__ __launch_bounds__(WG, (MT == 4 ? 3 : 4) - (sizeof(S) == 2)) void back
     using MM = Mma<float>;
     using PT = Parts<S>;
     typedef typename PT::Vec Vec;
-    constexpr int TC = tile_channels<S>(), CT = TC / 32;        // CT channels to a lane
+    constexpr int CT = lane_channels<S>(), TC = LW * CT;        // channels of a lane, of a tap
+    constexpr int TP = 32 / LW, GT = TP > 1 ? TP / 2 : 1;       // taps of an item, of a lane that works out geometry
     constexpr int TN = 32, NP = PT::NP, NC = 1 << ND, NR = PLAIN ? 1 : NC;     // corners, corners read
-    __shared__ unsigned sIdx[WAVES][TN];                        // byte offset of the low corner's channel 0 inside the sample
-    __shared__ __align__(16) T sCw[WAVES][TN][NR];              // weight of each corner, 0 where there is no sample
+    __shared__ unsigned sIdx[WAVES][TP][TN];                      // byte offset of the low corner's channel 0 inside the sample
+    __shared__ __align__(16) T sCw[WAVES][TP][TN][NR];            // weight of each corner, 0 where there is no sample
     __shared__ __align__(16) unsigned char sRow[2][MT * NP * 1024];        // rows of a step of grad_output: [part][q][row]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int j = lane % TN, q = lane / TN;
@@ -75,8 +78,8 @@ __global__ __launch_bounds__(WG, (MT == 4 ? 3 : 4) - (sizeof(S) == 2)) void back
     const int mchunk = wg % (unsigned)P.mchunks; wg /= (unsigned)P.mchunks;
     const int g = wg % (unsigned)P.G, split = wg / (unsigned)P.G;
     // the item's channel tile: segments are the intersections of the convolution group with deformable groups
-    const int tap = item % P.kV;
-    int z = item / P.kV, dg, c0 = 0, ce = 0;
+    const int tgroups = (P.kV + TP - 1) / TP, tap0 = item % tgroups * TP, ts = j / LW;      // ts: this lane's tap among them
+    int z = item / tgroups, dg, c0 = 0, ce = 0;
     bool works = false;
     for (dg = g * P.Cg / P.cpg; dg <= ((g + 1) * P.Cg - 1) / P.cpg; ++dg) {
         const int cb = max(g * P.Cg, dg * P.cpg);
@@ -87,13 +90,19 @@ __global__ __launch_bounds__(WG, (MT == 4 ? 3 : 4) - (sizeof(S) == 2)) void back
     }
     if (!works) dg = 0;         // (a wavefront without an item helps with the rows)
 
-    int kk[ND], kd[ND];
-    decode_tap<ND>(P, tap, kk);
+    // taps whose geometry this lane works out (lane groups take turns), clamped to legal ones
+    int gtap[GT], kd[GT][ND];
 #pragma unroll
-    for (int a = 0; a < ND; ++a) kd[a] = kk[a] * P.dil[slot<ND>(a)];
+    for (int u = 0; u < GT; ++u) {
+        gtap[u] = min(tap0 + (TP > 1 ? 2 * u + q : 0), P.kV - 1);
+        int kk[ND];
+        decode_tap<ND>(P, gtap[u], kk);
+#pragma unroll
+        for (int a = 0; a < ND; ++a) kd[u][a] = kk[a] * P.dil[slot<ND>(a)];
+    }
 
     const int m_base = mchunk * MT * TN;
-    const unsigned cj = (unsigned)min(c0 + j * CT, P.C_in - CT);      // clamped: lanes past the segment still load legally
+    const unsigned cj = (unsigned)min(c0 + j % LW * CT, P.C_in - CT);      // clamped: lanes past the segment still load legally
     // 32-bit byte offsets from the sample's base (the host checks that a sample of either tensor stays below 4 GiB)
     const unsigned cjB = cj * (unsigned)sizeof(S), cinB = (unsigned)P.C_in * (unsigned)sizeof(S);
     unsigned strB[ND];                                          // from a corner to the next along an axis
@@ -138,13 +147,15 @@ __global__ __launch_bounds__(WG, (MT == 4 ? 3 : 4) - (sizeof(S) == 2)) void back
         for (int i = 0; i < NA; ++i)
             if ((i + 1) * WG <= NROW || i * WG + threadIdx.x < NROW) *reinterpret_cast<Vec*>(sRow[buf] + (i * WG + threadIdx.x) * 16) = rv[i];
     };
-    T offv[ND];
+    T offv[GT][ND];
     auto load_off = [&](int slab) {
         const int n = slab / slabs_per_sample;
         const unsigned posc = min((unsigned)(slab % slabs_per_sample) * TN + j, P.outV - 1);
-        const S* off_n = PLAIN ? nullptr : off + (((size_t)n * P.DG + dg) * P.kV + tap) * ND * P.outV;
+        const S* off_n = PLAIN ? nullptr : off + ((size_t)n * P.DG + dg) * P.kV * ND * P.outV;
 #pragma unroll
-        for (int a = 0; a < ND; ++a) offv[a] = PLAIN ? 0.f : Store<S>::ld(off_n[(size_t)a * P.outV + posc]);
+        for (int u = 0; u < GT; ++u)
+#pragma unroll
+            for (int a = 0; a < ND; ++a) offv[u][a] = PLAIN ? 0.f : Store<S>::ld(off_n[((size_t)gtap[u] * ND + a) * P.outV + posc]);
     };
     const T sgn = split & 1 ? -1.f : 1.f;               // of this split's samples
     if (first < last) {
@@ -163,38 +174,42 @@ __global__ __launch_bounds__(WG, (MT == 4 ? 3 : 4) - (sizeof(S) == 2)) void back
         const unsigned posc = valid ? pos : P.outV - 1;
         int o[ND];
         decode_pos<ND>(P, posc, o);
-        bool live = valid;
-        T f[ND];
-        unsigned base = 0;
-#pragma unroll
-        for (int a = 0; a < ND; ++a) {
-            const int sa = slot<ND>(a);
-            const T p = (T)(o[a] * P.stride[sa] - P.pad[sa] + kd[a]) + offv[a];
-            const T pc = __builtin_amdgcn_fmed3f(p, 0.f, (T)(P.in[sa] - 1));
-            live = live && fabsf(p - pc) < 1.f;                 // -1 < p < size, false for NaN
-            int lo = (int)pc;
-            if constexpr (!PLAIN) lo = min(lo, max(P.in[sa] - 2, 0));
-            f[a] = pc - (T)lo;
-            base = base * (unsigned)P.in[sa] + (unsigned)lo;
-        }
-        load_off(next_slab);                        // travel through this slab
         // LDS operations of one wavefront execute in order; the fences only pin the compiler
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        if (q == 0) {
-            T cw[NC];                              // multiplied in the reference's order (w_l * w_h * w_w)
-            if constexpr (ND == 3) {
-                const T fl = f[0], gl = 1.f - fl, fh = f[1], gh = 1.f - fh, fw = f[2], gw = 1.f - fw;
-                cw[0] = gl * gh * gw; cw[1] = gl * gh * fw; cw[2] = gl * fh * gw; cw[3] = gl * fh * fw;
-                cw[4] = fl * gh * gw; cw[5] = fl * gh * fw; cw[6] = fl * fh * gw; cw[7] = fl * fh * fw;
-            } else {
-                const T fh = f[0], gh = 1.f - fh, fw = f[1], gw = 1.f - fw;
-                cw[0] = gh * gw; cw[1] = gh * fw; cw[2] = fh * gw; cw[3] = fh * fw;
-            }
-            sIdx[wave][j] = live ? base * cinB : 0u;
 #pragma unroll
-            for (int i = 0; i < NR; ++i) sCw[wave][j][i] = !live ? 0.f : PLAIN ? sgn : sgn * cw[i];
+        for (int u = 0; u < GT; ++u) {
+            bool live = valid;
+            T f[ND];
+            unsigned base = 0;
+#pragma unroll
+            for (int a = 0; a < ND; ++a) {
+                const int sa = slot<ND>(a);
+                const T p = (T)(o[a] * P.stride[sa] - P.pad[sa] + kd[u][a]) + offv[u][a];
+                const T pc = __builtin_amdgcn_fmed3f(p, 0.f, (T)(P.in[sa] - 1));
+                live = live && fabsf(p - pc) < 1.f;                 // -1 < p < size, false for NaN
+                int lo = (int)pc;
+                if constexpr (!PLAIN) lo = min(lo, max(P.in[sa] - 2, 0));
+                f[a] = pc - (T)lo;
+                base = base * (unsigned)P.in[sa] + (unsigned)lo;
+            }
+            if (TP > 1 || q == 0) {
+                const int row = TP > 1 ? 2 * u + q : 0;
+                T cw[NC];                              // multiplied in the reference's order (w_l * w_h * w_w)
+                if constexpr (ND == 3) {
+                    const T fl = f[0], gl = 1.f - fl, fh = f[1], gh = 1.f - fh, fw = f[2], gw = 1.f - fw;
+                    cw[0] = gl * gh * gw; cw[1] = gl * gh * fw; cw[2] = gl * fh * gw; cw[3] = gl * fh * fw;
+                    cw[4] = fl * gh * gw; cw[5] = fl * gh * fw; cw[6] = fl * fh * gw; cw[7] = fl * fh * fw;
+                } else {
+                    const T fh = f[0], gh = 1.f - fh, fw = f[1], gw = 1.f - fw;
+                    cw[0] = gh * gw; cw[1] = gh * fw; cw[2] = fh * gw; cw[3] = fh * fw;
+                }
+                sIdx[wave][row][j] = live ? base * cinB : 0u;
+#pragma unroll
+                for (int i = 0; i < NR; ++i) sCw[wave][row][j][i] = !live ? 0.f : PLAIN ? sgn : sgn * cw[i];
+            }
         }
+        load_off(next_slab);                            // travel through this slab
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
@@ -214,9 +229,9 @@ __global__ __launch_bounds__(WG, (MT == 4 ? 3 : 4) - (sizeof(S) == 2)) void back
         T wn[NR];
         auto fetch = [&](int k) {
             const int pp = (k & 8) * 2 + q * 8 + (k & 7);          // position of the slab this lane group works on
-            const unsigned at = sIdx[wave][pp] + cjB;
+            const unsigned at = sIdx[wave][ts][pp] + cjB;
 #pragma unroll
-            for (int i = 0; i < NR; ++i) wn[i] = sCw[wave][pp][i];
+            for (int i = 0; i < NR; ++i) wn[i] = sCw[wave][ts][pp][i];
 #pragma unroll
             for (int i = 0; i < NR; ++i) cn[i] = *reinterpret_cast<const Word*>(corner[i] + at);
         };
@@ -274,12 +289,17 @@ __global__ __launch_bounds__(WG, (MT == 4 ? 3 : 4) - (sizeof(S) == 2)) void back
     const bool redo = works && __any(!stands);
     // One row tile from the values themselves, two positions at a time, with the reference's corners.  (Its own accumulator, after
     // the loop above: a second loop over `acc` doubled the registers of the kernel.)
+    const int tap = tap0 + ts;                          // of this lane's column
     auto exact_tile = [&](int u, int mt) {
         typename MM::Acc x = acc_zero<T>();
+        int kk[ND], kx[ND];
+        decode_tap<ND>(P, min(tap, P.kV - 1), kk);
+#pragma unroll
+        for (int a = 0; a < ND; ++a) kx[a] = kk[a] * P.dil[slot<ND>(a)];
         for (int slab = first; slab < last; slab += turn) {
             const int n = slab / slabs_per_sample;
             const unsigned p0 = (unsigned)(slab % slabs_per_sample) * TN;
-            const S* off_n = PLAIN ? nullptr : off + (((size_t)n * P.DG + dg) * P.kV + tap) * ND * P.outV;
+            const S* off_n = PLAIN ? nullptr : off + (((size_t)n * P.DG + dg) * P.kV + min(tap, P.kV - 1)) * ND * P.outV;
             const char* in_n = reinterpret_cast<const char*>(in_cl + (size_t)n * P.inV * P.C_in);
 #pragma unroll 1
             for (int ks = 0; ks < TN; ks += 2) {
@@ -288,11 +308,11 @@ __global__ __launch_bounds__(WG, (MT == 4 ? 3 : 4) - (sizeof(S) == 2)) void back
                 decode_pos<ND>(P, posc, o);
 #pragma unroll
                 for (int a = 0; a < ND; ++a) ib[a] = o[a] * P.stride[slot<ND>(a)] - P.pad[slot<ND>(a)];
-                T offv[ND];
+                T ofx[ND];
 #pragma unroll
-                for (int a = 0; a < ND; ++a) offv[a] = PLAIN ? 0.f : Store<S>::ld(off_n[(size_t)a * P.outV + posc]);
+                for (int a = 0; a < ND; ++a) ofx[a] = PLAIN ? 0.f : Store<S>::ld(off_n[(size_t)a * P.outV + posc]);
                 TapGeo<T, ND> t;
-                tap_setup_noidx<T, ND>(P, offv, ib, kd, t);
+                tap_setup_noidx<T, ND>(P, ofx, ib, kx, t);
                 const bool live = pos < P.outV && t.inside;
                 unsigned cb[NC];
                 tap_corner_offsets<T, ND>(P, t, live, cinB, cb);
@@ -315,7 +335,7 @@ __global__ __launch_bounds__(WG, (MT == 4 ? 3 : 4) - (sizeof(S) == 2)) void back
     };
 
     if (!works) return;                                 // (uniform for the wavefront)
-    T* pt = partial + ((size_t)split * P.kV + tap) * P.C_out * P.Cg + (size_t)g * P.M * P.Cg + (c0 + j * CT - g * P.Cg);
+    T* pt = partial + ((size_t)split * P.kV + tap) * P.C_out * P.Cg + (size_t)g * P.M * P.Cg + (c0 + j % LW * CT - g * P.Cg);
 #pragma unroll
     for (int u = 0; u < CT; ++u)
 #pragma unroll
@@ -325,7 +345,7 @@ __global__ __launch_bounds__(WG, (MT == 4 ? 3 : 4) - (sizeof(S) == 2)) void back
 #pragma unroll
         for (int r = 0; r < MM::NACC; ++r) {
             const int m = m_base + mt * TN + MM::row(r, q);
-            if (m < P.M && c0 + j * CT + u < ce) pt[(size_t)m * P.Cg + u] = x[r];
+            if (m < P.M && c0 + j % LW * CT + u < ce && tap < P.kV) pt[(size_t)m * P.Cg + u] = x[r];
         }
     }
 }

@@ -145,7 +145,7 @@ template <typename T> inline size_t backward_weight_need(int N, int C_in, int C_
     long long split_ub = (4096 + tiles_lb - 1) / tiles_lb;
     if (split_ub > 256) split_ub = 256;
     if (split_ub < 1) split_ub = 1;
-    const size_t obytes = (size_t)N * C_out * outV * sizeof(T), rbytes = sizeof(T) == 4 && C_out / G > 32 ? row_operand_bytes<float>(N, C_out, outV) : 0;
+    const size_t obytes = (size_t)N * C_out * outV * sizeof(T), rbytes = sizeof(T) == 4 && kV > 1 || C_out / G > 32 ? row_operand_bytes<float>(N, C_out, outV) : 0;
     return align256((size_t)N * C_in * inV * sizeof(T)) + align256(obytes > rbytes ? obytes : rbytes) +
            align256((size_t)split_ub * kV * C_out * (C_in / G) * sizeof(T)) + align256((size_t)N * last_strips((unsigned)outV) * C_out * sizeof(T));
 }
@@ -537,10 +537,10 @@ template <typename T, typename S> struct WeightCall {
     const S* gout;
     T *partial, *sums;
     int nsums;
-    int igroups;                    // > 0: backward_weight_split_kernel, and gout_cl is grad_output in its operand order
+    int LW, igroups;                  // > 0: backward_weight_split_kernel, and gout_cl is grad_output in its operand order
 };
 template <typename T, int ND, typename S>
-int backward_weight_plan(const Params& P, const S* in, const S* gout, void* ws, size_t ws_bytes, bool bias, WeightCall<T, S>& c, Prep& prep, bool* declined);
+int backward_weight_plan(const Params& P, const S* in, const S* off, const S* gout, void* ws, size_t ws_bytes, bool bias, WeightCall<T, S>& c, Prep& prep, bool* declined);
 template <typename T, int ND, typename S>
 int backward_weight_run(const WeightCall<T, S>& c, const S* off, T* gw, T* gb, bool accumulate, hipStream_t s);
 

@@ -16,6 +16,10 @@ LAYERS = [
     (2, 1, 32, 64, (229, 231), 5, 2, 2, 1, 32, 1, 9.0), (2, 1, 136, 97, (221, 223), 1, 1, 0, 1, 136, 1, 0.9),
     (3, 1, 16, 80, (9, 32, 32), 3, 1, 1, 1, 16, 1, 1.5), (3, 2, 5, 66, (13, 39, 41), 3, (1, 2, 2), 1, 1, 5, 1, 2.5),
     (3, 1, 34, 40, (1, 95, 97), 3, 1, 1, 1, 17, 1, 1.0), (3, 1, 12, 70, (23, 21, 25), 3, 1, 2, 2, 12, 2, 2.0),
+    # two and four taps to an item (segments of up to 16 and 8 channels), up to 32 output channels too
+    (2, 1, 16, 65, (161, 163), 3, 1, 1, 1, 16, 1, 1.5), (2, 2, 42, 130, (97, 73), 3, 1, 1, 1, 14, 1, 3.0), (2, 1, 48, 40, (145, 147), 3, 1, 1, 1, 48, 1, 1.0),
+    (2, 1, 15, 20, (257, 259), 3, 2, 1, 1, 5, 1, 2.0), (2, 1, 8, 34, (229, 231), 5, 2, 2, 1, 8, 1, 9.0), (3, 1, 16, 20, (11, 32, 33), 3, 1, 1, 1, 4, 2, 1.5),
+    (3, 1, 7, 66, (13, 39, 41), 3, 1, 1, 1, 7, 1, 2.5), (3, 1, 16, 33, (17, 33, 35), 3, 1, 1, 1, 16, 1, 2.5), (3, 1, 12, 40, (1, 131, 133), 3, 1, 1, 1, 3, 1, 1.0),
 ]
 IDS = lambda s: "%dd-%d-%d-k%d-g%d" % (s[0], s[2], s[3], s[5], s[10])
 
@@ -56,6 +60,7 @@ LAYERS16 = [
     (2, 1, 34, 70, (129, 161), 3, 1, 1, 1, 34, 1, 1.5), (2, 2, 66, 40, (129, 161), 3, 1, 1, 1, 66, 1, 3.0),
     (2, 1, 24, 120, (141, 99), 3, 1, 1, 1, 8, 2, 2.0), (3, 1, 20, 64, (9, 32, 33), 3, 1, 1, 1, 10, 1, 1.5),
     (3, 1, 40, 97, (7, 31, 32), 3, 1, 1, 1, 40, 1, 2.5), (3, 1, 2, 60, (1, 95, 97), 3, 1, 1, 1, 2, 1, 1.0),
+    (3, 1, 16, 30, (17, 33, 35), 3, 1, 1, 1, 16, 1, 2.5), (2, 1, 60, 64, (129, 161), 3, 1, 1, 1, 30, 1, 1.5), (2, 1, 24, 66, (129, 161), 3, 1, 1, 1, 24, 1, 1.5),
 ]
 
 
