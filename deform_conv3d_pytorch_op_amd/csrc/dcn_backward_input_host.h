@@ -33,21 +33,16 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
     const bool input_only = (flags & FLAG_INPUT_ONLY) != 0;
     if ((!in && !input_only) || !w || !off || !gout || !gin || !goff) return fail(DCN_E_ARGUMENT, "null tensor pointer");
     bwd_data_weight_pad<T>(P.M, P.Cg, P.Mp, P.Cgp);
-    const size_t wbytes = bwd_data_weight_bytes<T>(P.M, P.Cg, P.kV, P.G, P.cpg);
-    const size_t tbytes = align256((size_t)P.N * P.C_in * P.inV * sizeof(T));
-    if (!ws || ws_bytes < wbytes + 2 * tbytes) return fail(DCN_E_WORKSPACE, "workspace too small");
+    DataLayout at = {};
+    if (int rc = data_layout<T, S>(P, ws ? ws_bytes : 0, at)) return rc;
+    const size_t wbytes = at.wbytes, tbytes = at.tbytes;
+    const bool tail_words = at.tail_words;
     S* wt = static_cast<S*>(ws);
     T* in_cl = reinterpret_cast<T*>(static_cast<char*>(ws) + wbytes);
     T* gin_cl = reinterpret_cast<T*>(static_cast<char*>(ws) + wbytes + tbytes);
     const int TN = Mma<T>::TN;
     const int mk = bwd_data_mk<T>(P.M);
-    // weight bounds and, 64 bytes into the block behind them, the plan chosen on the device: in the last whole
-    // 256-byte blocks of the workspace when those lie behind the two channels-last regions (dcn_workspace_bytes counts them),
-    // else at the start of the channels-last gradient, which the LDS paths do not use
-    const size_t tail_at = ws_bytes >= BWD_TAIL ? (ws_bytes - 256) / 256 * 256 - (BWD_TAIL - 256) : 0;
-    const bool tail_words = tail_at >= wbytes + 2 * tbytes;
-    if (!tail_words && tbytes < BWD_TAIL) return fail(DCN_E_WORKSPACE, "workspace too small");
-    float* bounds = tail_words ? reinterpret_cast<float*>(static_cast<char*>(ws) + tail_at) : reinterpret_cast<float*>(gin_cl);
+    float* bounds = reinterpret_cast<float*>(static_cast<char*>(ws) + at.tail_at);
     Prep own;
     Prep& prep = given ? *given : own;
     const dim3 tgrid((P.inV + 31) / 32, (unsigned)(P.C_in + 31) / 32, (unsigned)P.N), tblock(32, 8);
@@ -55,8 +50,6 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
     // 1) one kernel: scatter privatised in LDS + coordinate gradient from an LDS input halo.
     // float32 layers whose LDS cells may be paired and 16-bit storage, of more than one tap: backward_fused_kernel, with
     // grad_output in operand order behind the channels-last regions of the workspace.  Others: backward_input_halo_kernel.
-    const size_t gq_at = wbytes + 2 * tbytes, gq_bytes = fused_gout_need<S>(P.N, P.M, P.G, P.outV);
-    const bool gq_fits = ws_bytes >= gq_at + gq_bytes + (tail_words ? BWD_TAIL + 256 : 0);
     // A halo of up to FUSED_HS cells gets the variant with that compile-time plane stride (the four
     // planes of either kind then lie within the 64 KB reach of an LDS instruction's offset field).
     // Eight wavefronts per workgroup; four (half the positions, in the block shape with the smallest
@@ -89,7 +82,7 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             // a single tap: a chunk is all staging and flush, which the smaller workgroups of backward_input_halo_kernel overlap
             // better, and grad_output is used once per chunk (24 layers of one tap: backward_fused_kernel takes 1.09 times as long).
             // Not where that kernel declines the output channels of a 16-bit layer.
-            const bool split = pair && gq_fits && (P.kV > 1 || (S16 && P.M > 256));
+            const bool split = pair && at.fused && (P.kV > 1 || (S16 && P.M > 256));
             int cch = 0;
             size_t lds = 0;
             Kern kern = nullptr;
@@ -324,7 +317,7 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             job.dst = const_cast<S*>(fp[k].wt);
             any_fused = any_fused || !fp[k].kern;
         }
-        char* gq = static_cast<char*>(ws) + gq_at;
+        char* gq = static_cast<char*>(ws) + at.gq_at;
         if (any_fused) {
             const size_t total = (size_t)P.N * P.G * fused_steps(P.M) * 2 * P.outV;
             PrepJob& job = prep.add(PREP_GOUT, (unsigned)((total + 255) / 256 > 16384 ? 16384 : (total + 255) / 256));

@@ -65,7 +65,7 @@ template <typename T, typename S = T> inline size_t packed_weight_elems(int M, i
 // layout occupies.  cpg = 0: the channels per deformable group are not known (the first workspace
 // query is not told them) and the bound assumes their largest possible number of groups, C_in.
 inline size_t slab_bound(size_t C_in, int G, int cpg, int cch) { return C_in / cch + (cpg > 0 ? C_in / cpg : C_in) + G + 1; }
-// Either weight layout of backward_input_offset fits.
+// Any weight layout of backward_input_offset fits but that of backward_fused_kernel.
 template <typename T> inline size_t bwd_data_weight_bytes(int M, int Cg, int kV, int G, int cpg = 0) {
     int Mp, Cgp;
     bwd_data_weight_pad<T>(M, Cg, Mp, Cgp);
@@ -76,11 +76,16 @@ template <typename T> inline size_t bwd_data_weight_bytes(int M, int Cg, int kV,
     const size_t packed16 = packed_weight_elems<T>(M, kV, slab_bound(C_in, G, cpg, 16), 16);
     size_t packed = packed4 > packed8 ? packed4 : packed8;
     if (packed16 > packed) packed = packed16;
-    size_t bytes = (plain > packed ? plain : packed) * sizeof(T);
-    for (int cch = 4; sizeof(T) == 4 && cch <= 16; cch *= 2) {
-        const size_t parts = slab_bound(C_in, G, cpg, cch) * fused_slab_ops<float>(M, kV, cch) * 16;
-        if (parts > bytes) bytes = parts;
-    }
+    return align256((plain > packed ? plain : packed) * sizeof(T));
+}
+// ... and that one too (float32 and 16-bit storage; float64 has another kernel): S the storage format
+template <typename T, typename S = T> inline size_t bwd_fused_weight_bytes(int M, int Cg, int kV, int G, int cpg = 0) {
+    size_t bytes = bwd_data_weight_bytes<T>(M, Cg, kV, G, cpg);
+    if constexpr (sizeof(T) == 4)
+        for (int cch = 4; cch <= 16; cch *= 2) {
+            const size_t parts = slab_bound((size_t)Cg * G, G, cpg, cch) * fused_slab_ops<S>(M, kV, cch) * 16;
+            if (parts > bytes) bytes = parts;
+        }
     return align256(bytes);
 }
 // Partial outputs of a forward pass that splits the input channels of a position block over several
@@ -134,8 +139,36 @@ template <typename S> inline size_t fused_gout_need(int N, int M, int G, size_t 
 }
 // packed weights, two channels-last tensors, grad_output in operand order (float32 and 16-bit storage), the tail
 template <typename T> inline size_t backward_data_need(int N, int C_in, int C_out, size_t inV, size_t outV, int kV, int G, int cpg = 0) {
-    return bwd_data_weight_bytes<T>(C_out / G, C_in / G, kV, G, cpg) + 2 * align256((size_t)N * C_in * inV * sizeof(T)) +
+    return bwd_fused_weight_bytes<T>(C_out / G, C_in / G, kV, G, cpg) + 2 * align256((size_t)N * C_in * inV * sizeof(T)) +
            fused_gout_need<T>(N, C_out / G, G, outV) + BWD_TAIL + 512;
+}
+// Where the parts of a backward_input_offset workspace lie: [ packed weights | input channels-last | its gradient channels-last |
+// grad_output in operand order | ... | tail ].  A workspace without room for all of it -- what dcn_workspace_bytes asks for has --
+// is laid out for the kernels that use neither the packed parts nor grad_output in operand order (`fused` false), as long as it holds
+// the weights of those and the two channels-last regions.
+struct DataLayout {
+    size_t wbytes, tbytes;      // packed weights; one channels-last region
+    size_t gq_at;
+    bool fused;
+    // Bounds of the weights and, 64 bytes into the block behind them, the plan chosen on the device: in the last whole 256-byte blocks
+    // of the workspace where those lie behind the channels-last regions (tail_words), else at the start of the channels-last
+    // gradient, which the LDS paths do not use.
+    size_t tail_at;
+    bool tail_words;
+};
+template <typename T, typename S> inline int data_layout(const Params& P, size_t ws_bytes, DataLayout& l) {
+    l.tbytes = align256((size_t)P.N * P.C_in * P.inV * sizeof(T));
+    const size_t tail = ws_bytes >= BWD_TAIL ? (ws_bytes - 256) / 256 * 256 - (BWD_TAIL - 256) : 0;
+    for (const bool fused : {true, false}) {
+        l.fused = fused;
+        l.wbytes = fused ? bwd_fused_weight_bytes<T, S>(P.M, P.Cg, P.kV, P.G, P.cpg) : bwd_data_weight_bytes<T>(P.M, P.Cg, P.kV, P.G, P.cpg);
+        l.gq_at = l.wbytes + 2 * l.tbytes;
+        l.tail_words = tail >= l.gq_at;
+        l.tail_at = l.tail_words ? tail : l.wbytes + l.tbytes;
+        if (l.tail_words && ws_bytes >= l.gq_at + fused_gout_need<S>(P.N, P.M, P.G, P.outV) + BWD_TAIL + 256) break;
+    }
+    if (ws_bytes < l.gq_at || (!l.tail_words && l.tbytes < BWD_TAIL)) return fail(DCN_E_WORKSPACE, "workspace too small");
+    return DCN_OK;
 }
 // A channels-last copy of the input, grad_output channels-last or (float32) in operand order + one partial weight per position split (at most 256 splits, and never more
 // than about 4096 workgroups: see bww_plan) + the strips of grad_output's sums

@@ -65,7 +65,8 @@ const char *dcn_last_error(void);   /* message of the last failing call on this 
  * 16-bit formats, elem_size 2, are served by dcn_workspace_bytes_for only and get 0 here;
  * input_volume = input_l * input_h * input_w, output_volume likewise, kernel_volume =
  * kernel_l * kernel_h * kernel_w).  The workspace holds a re-laid-out copy of the weight and, for
- * the backward calls, channels-last copies of the input batch, its gradient and grad_output, and
+ * the backward calls, channels-last copies of the input batch and its gradient, grad_output in the
+ * operand order of the matrix instructions (f32: half as large again as the tensor), and
  * one word in which the device records which of the planned LDS halo sizes it chose for the call
  * from the offsets (so two calls that overlap in time need a workspace each; the forward calls
  * keep it as a 32-bit index, 0 = the narrowest halo, at byte offset (workspace_bytes - 256) rounded

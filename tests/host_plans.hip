@@ -47,6 +47,33 @@ template <int ND> static bool native16(const Params& P, int& hits) {
     return forward16_native<ND>(P) == fits;
 }
 
+// The layout of a backward_input_offset workspace: any size from the packed weights and two channels-last tensors on is taken, the
+// queried size has room for the fused kernel, and no part reaches into another or past the end.
+template <typename T, typename S> static bool layout_holds(const Params& P, size_t ws, bool fused) {
+    DataLayout l = {};
+    if (data_layout<T, S>(P, ws, l) != DCN_OK || l.fused != fused) return false;
+    const size_t weights = fused ? bwd_fused_weight_bytes<T, S>(P.M, P.Cg, P.kV, P.G, P.cpg) : bwd_data_weight_bytes<T>(P.M, P.Cg, P.kV, P.G, P.cpg);
+    const size_t regions = weights + 2 * align256((size_t)P.N * P.C_in * P.inV * sizeof(T)), gout = fused ? fused_gout_need<S>(P.N, P.M, P.G, P.outV) : 0;
+    if (l.wbytes != weights || l.wbytes + 2 * l.tbytes != regions || regions > ws || l.tail_at + BWD_TAIL > ws || l.tail_at % 256) return false;
+    return l.tail_words ? l.gq_at == regions && l.tail_at >= regions + gout : l.tail_at == l.wbytes + l.tbytes && l.tbytes >= BWD_TAIL && !fused;
+}
+template <typename T, typename S> static bool layout(const Params& P, int& hits) {
+    const size_t tbytes = align256((size_t)P.N * P.C_in * P.inV * sizeof(T));
+    const size_t least = bwd_data_weight_bytes<T>(P.M, P.Cg, P.kV, P.G, P.cpg) + 2 * tbytes + (tbytes < BWD_TAIL ? BWD_TAIL : 0);
+    const size_t query = backward_data_need<T>(P.N, P.C_in, P.C_out, P.inV, P.outV, P.kV, P.G, P.cpg);
+    DataLayout l = {};
+    const bool more = sizeof(T) == 4 && fused_gout_need<S>(P.N, P.M, P.G, P.outV) > BWD_TAIL + 512;      // (the fused kernel takes more than the least)
+    hits += more && bwd_fused_weight_bytes<T, S>(P.M, P.Cg, P.kV, P.G, P.cpg) > bwd_data_weight_bytes<T>(P.M, P.Cg, P.kV, P.G, P.cpg);
+    return layout_holds<T, S>(P, query, true) && layout_holds<T, S>(P, query + 77, true) && (!more || layout_holds<T, S>(P, least, false)) &&
+           data_layout<T, S>(P, bwd_data_weight_bytes<T>(P.M, P.Cg, P.kV, P.G, P.cpg) + 2 * tbytes - 1, l) == DCN_E_WORKSPACE;
+}
+static bool layouts(const Params& P, int& hits) {
+    int all[4] = {0, 0, 0, 0};
+    const bool ok = layout<float, float>(P, all[0]) && layout<float, Bf16>(P, all[1]) && layout<float, Fp16>(P, all[2]) && layout<double, double>(P, all[3]);
+    hits += all[0];
+    return ok;
+}
+
 int main(int argc, char** argv) {
     if (argc != 4) return 2;
     const std::string what = argv[1];
@@ -64,7 +91,7 @@ int main(int argc, char** argv) {
         const int nd = pick(2, 3);
         if (!random_layer(nd, P)) continue;
         ++layers;
-        const bool ok = what == "noalloc" ? noalloc(P, hits) : what == "native16" ? (nd == 3 ? native16<3>(P, hits) : native16<2>(P, hits)) : false;
+        const bool ok = what == "noalloc" ? noalloc(P, hits) : what == "layout" ? layouts(P, hits) : what == "native16" ? (nd == 3 ? native16<3>(P, hits) : native16<2>(P, hits)) : false;
         if (!ok) {
             printf("%s: %d-D, C_in %d, C_out %d, G %d, cpg %d, k %d %d %d, stride %d %d %d, dil %d %d %d\n", what.c_str(), nd, P.C_in, P.C_out, P.G, P.cpg, P.k[0],
                    P.k[1], P.k[2], P.stride[0], P.stride[1], P.stride[2], P.dil[0], P.dil[1], P.dil[2]);
