@@ -297,19 +297,18 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
         const float gmax = __uint_as_float(gmaxb), wcol = weight_bound(bounds, 1), wmax = weight_bound(bounds, 0);
         const float bound = 1.001f * wcol * __uint_as_float(nmaxb);    // (0.1 % for the rounding of the norms and of the contraction)
         const float bound_cell = 1.001f * wcol * (float)P.kV * nsum;
-        // Without a finite bound, or where the squares of tiny weights or of a tiny grad_output underflow, the workgroup scatters
-        // through global memory (false for NaN).
-        const bool cells_ok = bound < 3.0e38f && bound_cell < 3.0e38f && !(gmax > 0.f && gmax < 1e-18f) && !(wmax > 0.f && wmax < 1e-18f);
+        // Without a finite bound, where the squares of a tiny grad_output underflow, or where the scale would leave the range of a float,
+        // the workgroup scatters through global memory (false for NaN).
+        const bool cells_ok = bound < 3.0e38f && bound_cell < 3.0e38f && !(gmax > 0.f && gmax < 1e-18f) && !(gmax > 0.f && wcol > 0.f && bound < 1e-30f);
         // operands that bfloat16 parts do not hold: the contraction on the float32 instructions
-        const bool exact_all = sizeof(S) == 4 && !(cells_ok && gmax < 0x1p126f && wmax < 0x1p126f);
+        const bool exact_all = sizeof(S) == 4 && !(cells_ok && gmax < 0x1p126f && wmax < 0x1p126f && !(wmax > 0.f && wmax < 1e-18f));
         float scale = 1.f;
         if (bound > 0.f && cells_ok) {
             // a single term stays below 2^22 (the float conversion of add2), all that a cell can receive below 2^31
             // (half a unit of rounding each for at most NPT * 32 * kV terms fits the one per cent of slack)
             const double s_term = 4194304.0 / (double)bound;
             const double s_cell = bound_cell > 0.f ? 2147483648.0 / (double)bound_cell : s_term;
-            const double sc = 0.99 * (s_term < s_cell ? s_term : s_cell);
-            scale = (float)(sc < 1e30 ? sc : 1e30);                    // (a denormal bound: keep the scale a finite float)
+            scale = (float)(0.99 * (s_term < s_cell ? s_term : s_cell));
         }
         scale = __uint_as_float((unsigned)__builtin_amdgcn_readfirstlane((int)__float_as_uint(scale)));
         const double inv_scale = 1.0 / (double)scale;

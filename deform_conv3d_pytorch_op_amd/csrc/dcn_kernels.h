@@ -1134,9 +1134,11 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
         // the LDS cells need a finite bound; without one this workgroup scatters through the far path
         // (float cells need the exponent; and with either cell type a corner that carries weight zero
         // would receive 0 * inf = NaN where the reference adds nothing)
-        // (and a block whose grad_output is so small that its squares underflow: the bound is then not
-        // trustworthy, and the workgroup takes the far path too rather than rounding its gradient away)
-        const bool cells_ok = bound < 3.0e38f && bound_cell < 3.0e38f && !(PAIR && gmax > 0.f && gmax < 1e-18f);            // false for NaN
+        // (and paired cells of a block whose grad_output is so small that its squares underflow, or whose terms are so small
+        // that their scale leaves the range of a float: the workgroup takes the far path too rather than
+        // rounding its gradient away)
+        const bool cells_ok = bound < 3.0e38f && bound_cell < 3.0e38f &&
+                              !(PAIR && gmax > 0.f && (gmax < 1e-18f || (wbound > 0.f && bound < 1e-30f)));            // false for NaN
         if (bound > 0.f && bound < 3.0e38f) (void)frexpf(bound, &ex);
         double scale = ldexp(1.0, 30 - ex), inv_scale = ldexp(1.0, ex - 30);
         float scale32 = 1.f;
@@ -1150,7 +1152,7 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
                 scale = 0.99 * (s_term < s_cell ? s_term : s_cell);
             } else
                 scale = 1.0;
-            scale32 = (float)(scale < 1e30 ? scale : 1e30);       // (a denormal bound: keep the scale a finite float)
+            scale32 = (float)scale;
             scale = (double)scale32;                 // the flush divides by exactly what the terms were multiplied with
             inv_scale = 1.0 / scale;
         }

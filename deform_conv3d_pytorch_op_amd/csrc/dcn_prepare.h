@@ -34,32 +34,36 @@ __host__ __device__ inline unsigned last_strips(unsigned V) { return (V + LAST_S
 // max |w| and the largest norm over the output channels of a group of an (input channel, tap) column:
 // |grad column| <= that norm times the norm of grad_output over the output channels at the position
 // (Cauchy-Schwarz).  Every block leaves the maxima of its columns as bit patterns, of which NaN is the
-// largest; the readers take the maximum over the blocks (weight_bound).
+// largest; the readers take the maximum over the blocks (weight_bound).  Where the squares of a column may have underflowed (a sum below
+// 2^-100) they are those of 2^96 times its values.
 constexpr int BOUND_BLOCKS = 64;
 template <typename S>
 __device__ inline void prep_bounds(const Params& P, const S* __restrict__ w, float* __restrict__ out, unsigned block) {
     // 64 neighbouring columns of one group x 4 slices of its rows
-    __shared__ float part[4][64];
+    __shared__ float part[2][4][64];
     __shared__ unsigned amax[4];
     const int cx = threadIdx.x & 63, sl = threadIdx.x >> 6;
     const size_t cols = (size_t)P.Cg * P.kV, tiles = (cols + 63) / 64;
     unsigned am = 0u, nm = 0u;
     for (size_t tile = block; tile < tiles * P.G; tile += BOUND_BLOCKS) {
         const size_t g = tile / tiles, col = tile % tiles * 64 + cx;
-        float ss = 0.f;
+        float ss = 0.f, st = 0.f;
         if (col < cols) {
             const S* p = w + g * P.M * cols + col;
 #pragma unroll 8
             for (int r = sl; r < P.M; r += 4) {
                 const float v = offset_value(p[(size_t)r * cols]);
                 ss += v * v;
+                st += (v * 0x1p96f) * (v * 0x1p96f);
                 am = max(am, __float_as_uint(fabsf(v)));
             }
         }
-        part[sl][cx] = ss;
+        part[0][sl][cx] = ss;
+        part[1][sl][cx] = st;
         __syncthreads();
-        ss = (part[0][cx] + part[1][cx]) + (part[2][cx] + part[3][cx]);
-        nm = max(nm, __float_as_uint(fabsf(sqrtf(ss))));
+        ss = (part[0][0][cx] + part[0][1][cx]) + (part[0][2][cx] + part[0][3][cx]);
+        st = (part[1][0][cx] + part[1][1][cx]) + (part[1][2][cx] + part[1][3][cx]);
+        nm = max(nm, __float_as_uint(fabsf(ss < 0x1p-100f ? sqrtf(st) * 0x1p-96f : sqrtf(ss))));      // (false for NaN)
         __syncthreads();
     }
     for (int sh = 1; sh < 64; sh <<= 1) {

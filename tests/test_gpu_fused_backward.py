@@ -69,6 +69,22 @@ def test_small_operands(spec, what, exponent):
         assert err <= tol
 
 
+@pytest.mark.parametrize("spec", [EDGES[5], EDGES[7], EDGES[13], EDGES[16]], ids=["2d", "2d-k1", "3d-strided", "3d-k1"])
+@pytest.mark.parametrize("w,gout", [(62, 0), (66, 0), (90, 0), (98, 0), (101, 0), (120, 10), (140, 30), (55, -55), (30, -58), (58, -30), (0, -58)])
+def test_small_weights(spec, w, gout):
+    """Weights times 2^-w and grad_output times 2^gout, on both sides of the lines between cells and global memory (products of about
+    2^-100) and of squares that underflow (weights below 2^-63): gradients that are normal numbers are as exact as ordinary ones."""
+    print("small weights", spec, w, gout, flush=True)
+    c = make_case(*spec, dtype=torch.float32, seed=35, bias=False)
+    c["w"] = c["w"] * 2.0 ** -w
+    c["gout"] = c["gout"] * 2.0 ** gout
+    for got, want, tol in zip(_gradients(c), _oracle(c), (1e-4, 1e-5)):
+        assert want.abs().max().item() > 2.0 ** -122
+        err = ((got - want).norm() / want.norm()).item()
+        print("  relative 2-norm error %.2e" % err, flush=True)
+        assert err <= tol
+
+
 def test_one_small_position_beside_ordinary_ones():
     """grad_offset of positions whose grad_output alone is tiny."""
     print("small position", flush=True)
