@@ -150,7 +150,7 @@ int backward_weight16(const Geometry& g, const S* in, const S* off, const S* gou
 // The backward pass of a layer in one call: the gradients asked for (null: not wanted), written, not
 // added.  What the operators need beforehand -- cleared buffers, packed weights, channels-last copies,
 // the sums for grad_bias -- is one launch (backward_prepare_kernel).
-// Workspace: [ 16-bit storage: float gradients | backward_input_offset | backward_weight ].
+// Workspace: see LayerNeed.
 template <typename S> struct Wide { typedef float type; };
 template <> struct Wide<double> { typedef double type; };
 template <typename S>
@@ -194,9 +194,10 @@ int layer_backward(const Geometry& g, const S* in, const S* w, const S* off, con
     } else {
         tgin = gin; tgoff = goff; tgw = gw; tgb = gb;
     }
-    const size_t dbytes = backward_data_need<T>(P.N, P.C_in, P.C_out, P.inV, P.outV, P.kV, P.G, P.cpg);
-    const size_t wbytes = backward_weight_need<T>(P.N, P.C_in, P.C_out, P.inV, P.outV, P.kV, P.G);
-    void *dws = data ? take(dbytes) : nullptr, *wws = gw ? take(wbytes) : nullptr;
+    const LayerNeed need = layer_need<T, S>(ND, P.N, P.C_in, P.C_out, P.inV, P.outV, P.kV, P.G, P.cpg);
+    char* const shared = p;                             // (the float copies below lie here, too)
+    const size_t shared_bytes = left;
+    void *dws = data ? take(need.data) : nullptr, *wws = gw ? take(need.weight) : nullptr;
     if ((data && !dws) || (gw && !wws)) return fail(DCN_E_WORKSPACE, "workspace too small");
     Prep prep;
     WeightCall<T, S> call;
@@ -205,33 +206,36 @@ int layer_backward(const Geometry& g, const S* in, const S* w, const S* off, con
     // (16-bit storage: the kernels that read it may decline a layer, which then runs on widened copies)
     bool wdeclined = S16 && !native16(), ddeclined = wdeclined;
     if (gw && !wdeclined)
-        if (int rc = backward_weight_plan<T, ND, S>(P, in, off, gout, wws, wbytes, gb != nullptr, call, prep, S16 ? &wdeclined : nullptr)) return rc;
+        if (int rc = backward_weight_plan<T, ND, S>(P, in, off, gout, wws, need.weight, gb != nullptr, call, prep, S16 ? &wdeclined : nullptr)) return rc;
     if (data && !ddeclined)
-        if (int rc = backward_input_offset<T, ND, S>(g, in, w, off, gout, tgin, tgoff, dws, dbytes, s, flags, S16 ? &ddeclined : nullptr, &prep)) return rc;
+        if (int rc = backward_input_offset<T, ND, S>(g, in, w, off, gout, tgin, tgoff, dws, need.data, s, flags, S16 ? &ddeclined : nullptr, &prep)) return rc;
     if (!data || ddeclined)
         if (int rc = launch_prepare<T, S>(P, none, prep, w, off, 0, s)) return rc;
-    const T *fin = nullptr, *fw = nullptr, *foff = nullptr, *fgout = nullptr;
+    if (gw && !wdeclined)
+        if (int rc = backward_weight_run<T, ND, S>(call, off, tgw, tgb, false, s)) return rc;
     if constexpr (S16) {
-        if ((data && ddeclined) || (gw && wdeclined)) {
+        const bool wide_data = data && ddeclined, wide_weight = gw && wdeclined;
+        if (wide_data || wide_weight) {
+            p = shared;                                 // the kernels above are done with their operands by the time the next ones run
+            left = shared_bytes;
             float* copy[4] = {static_cast<float*>(take(z.in * 4)), static_cast<float*>(take(z.w * 4)), static_cast<float*>(take(z.off * 4)), static_cast<float*>(take(z.out * 4))};
-            if (!copy[0] || !copy[1] || !copy[2] || !copy[3]) return fail(DCN_E_WORKSPACE, "workspace too small");
+            void* ops = take(need.wide);
+            if (!copy[0] || !copy[1] || !copy[2] || !copy[3] || !ops) return fail(DCN_E_WORKSPACE, "workspace too small");
             if (int rc = widen(in, copy[0], z.in, s)) return rc;
             if (int rc = widen(w, copy[1], z.w, s)) return rc;
             if (int rc = widen(off, copy[2], z.off, s)) return rc;
             if (int rc = widen(gout, copy[3], z.out, s)) return rc;
-            fin = copy[0]; fw = copy[1]; foff = copy[2]; fgout = copy[3];
+            const T *fin = copy[0], *fw = copy[1], *foff = copy[2], *fgout = copy[3];
+            if (wide_data)
+                if (int rc = backward_input_offset<T, ND>(g, fin, fw, foff, fgout, tgin, tgoff, ops, need.wide, s, flags)) return rc;
+            if (wide_weight) {
+                WeightCall<T, T> wide;
+                Prep wprep;
+                if (int rc = backward_weight_plan<T, ND, T>(P, fin, foff, fgout, ops, need.weight, gb != nullptr, wide, wprep, nullptr)) return rc;
+                if (int rc = launch_prepare<T, T>(P, none, wprep, fw, foff, 0, s)) return rc;
+                if (int rc = backward_weight_run<T, ND, T>(wide, foff, tgw, tgb, false, s)) return rc;
+            }
         }
-    }
-    if (data && ddeclined)
-        if (int rc = backward_input_offset<T, ND>(g, fin, fw, foff, fgout, tgin, tgoff, dws, dbytes, s, flags)) return rc;
-    if (gw && !wdeclined) {
-        if (int rc = backward_weight_run<T, ND, S>(call, off, tgw, tgb, false, s)) return rc;
-    } else if (gw) {
-        WeightCall<T, T> wide;
-        Prep wprep;
-        if (int rc = backward_weight_plan<T, ND, T>(P, fin, foff, fgout, wws, wbytes, gb != nullptr, wide, wprep, nullptr)) return rc;
-        if (int rc = launch_prepare<T, T>(P, none, wprep, fw, foff, 0, s)) return rc;
-        if (int rc = backward_weight_run<T, ND, T>(wide, foff, tgw, tgb, false, s)) return rc;
     }
     if constexpr (S16) {
         const size_t na = data ? z.in : 0, nb = data ? z.off : 0, nc = gw ? z.w : 0, nd = gb ? (size_t)P.C_out : 0, most = na + nb + nc;
@@ -430,12 +434,9 @@ size_t dcn_layer_backward_workspace_bytes(int elem_size, int nd, int batch, int 
         channel_per_deformable_group <= 0 || input_c % channel_per_deformable_group || input_c % group || output_c % group || nd < 2 || nd > 3)
         return 0;
     const int cpg = channel_per_deformable_group;
-    if (elem_size == 8)
-        return align256(backward_data_need<double>(batch, input_c, output_c, input_volume, output_volume, kernel_volume, group, cpg)) +
-               align256(backward_weight_need<double>(batch, input_c, output_c, input_volume, output_volume, kernel_volume, group));
-    return align256(backward_data_need<float>(batch, input_c, output_c, input_volume, output_volume, kernel_volume, group, cpg)) +
-           align256(backward_weight_need<float>(batch, input_c, output_c, input_volume, output_volume, kernel_volume, group)) +
-           (elem_size == 2 ? copies16_bytes(batch, input_c, output_c, input_volume, output_volume, kernel_volume, group, cpg) : 0);
+#define LAYER_BYTES(T, S) layer_bytes(layer_need<T, S>(nd, batch, input_c, output_c, input_volume, output_volume, kernel_volume, group, cpg))
+    return elem_size == 8 ? LAYER_BYTES(double, double) : elem_size == 2 ? LAYER_BYTES(float, Bf16) : LAYER_BYTES(float, float);
+#undef LAYER_BYTES
 }
 
 int dcn_layer_backward(int nd, int dtype, const void* input, const void* weight, const void* offset, const void* grad_output, void* grad_input, void* grad_offset,

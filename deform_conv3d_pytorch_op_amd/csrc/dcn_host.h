@@ -138,9 +138,9 @@ template <typename S> inline size_t fused_gout_need(int N, int M, int G, size_t 
     else return align256(fused_gout_bytes<S>(N, M, G, outV));
 }
 // packed weights, two channels-last tensors, grad_output in operand order (float32 and 16-bit storage), the tail
-template <typename T> inline size_t backward_data_need(int N, int C_in, int C_out, size_t inV, size_t outV, int kV, int G, int cpg = 0) {
-    return bwd_fused_weight_bytes<T>(C_out / G, C_in / G, kV, G, cpg) + 2 * align256((size_t)N * C_in * inV * sizeof(T)) +
-           fused_gout_need<T>(N, C_out / G, G, outV) + BWD_TAIL + 512;
+template <typename T, typename S = T> inline size_t backward_data_need(int N, int C_in, int C_out, size_t inV, size_t outV, int kV, int G, int cpg = 0) {
+    return bwd_fused_weight_bytes<T, S>(C_out / G, C_in / G, kV, G, cpg) + 2 * align256((size_t)N * C_in * inV * sizeof(T)) +
+           fused_gout_need<S>(N, C_out / G, G, outV) + BWD_TAIL + 512;
 }
 // Where the parts of a backward_input_offset workspace lie: [ packed weights | input channels-last | its gradient channels-last |
 // grad_output in operand order | ... | tail ].  A workspace without room for all of it -- what dcn_workspace_bytes asks for has --
@@ -187,6 +187,28 @@ template <typename T> inline size_t workspace_need(int N, int C_in, int C_out, s
                  bww = backward_weight_need<T>(N, C_in, C_out, inV, outV, kV, G);
     const size_t need = fwd > bwd ? fwd : bwd;
     return need > bww ? need : bww;
+}
+
+// The workspace of a layer's backward pass: [ 16-bit storage: float gradients | backward_input_offset | backward_weight ], and in the place
+// of the last two, once the kernels that read 16-bit tensors have run, [ float copies of the tensors | an operator on them ] for what
+// they decline (the query is not told the strides and dilations that decide it).
+struct LayerNeed { size_t grads, data, weight, copies, wide; };
+template <typename T, typename S> inline LayerNeed layer_need(int nd, int N, int C_in, int C_out, size_t inV, size_t outV, int kV, int G, int cpg) {
+    const size_t in = (size_t)N * C_in * inV, w = (size_t)C_out * (C_in / G) * kV, off = (size_t)N * (C_in / cpg) * kV * nd * outV, out = (size_t)N * C_out * outV;
+    LayerNeed n = {};
+    n.data = align256(backward_data_need<T, S>(N, C_in, C_out, inV, outV, kV, G, cpg));
+    n.weight = align256(backward_weight_need<T>(N, C_in, C_out, inV, outV, kV, G));
+    if (!std::is_same<S, T>::value) {
+        n.grads = align256(in * sizeof(T)) + align256(off * sizeof(T)) + align256(w * sizeof(T)) + align256((size_t)C_out * sizeof(T));
+        n.copies = align256(in * sizeof(T)) + align256(off * sizeof(T)) + align256(w * sizeof(T)) + align256(out * sizeof(T));
+        n.wide = align256(backward_data_need<T>(N, C_in, C_out, inV, outV, kV, G, cpg));
+        if (n.weight > n.wide) n.wide = n.weight;
+    }
+    return n;
+}
+inline size_t layer_bytes(const LayerNeed& n) {
+    const size_t native = n.data + n.weight, wide = n.copies + n.wide;
+    return n.grads + (native > wide ? native : wide);
 }
 
 struct Geometry {   // the reference's argument list, 2-D mapped onto slots 1,2 with a unit length axis

@@ -1,5 +1,7 @@
 """Workspaces smaller than the queried one, down to the least that the operators have always taken: the kernels that need less of it,
 against the oracle, without a write past the end."""
+import ctypes
+
 import pytest
 import torch
 
@@ -106,3 +108,46 @@ def test_backward_weight(spec):
         assert err <= 4e-6
     assert not torch.equal(got[least], got[full])                           # two kernels
     assert _call(L.dcn3d_backward_weight_f32, c, (x, off, gout, torch.zeros_like(w)), copies) == -2
+
+
+# served by the 16-bit kernels; grad_weight on float copies (odd channels); the other gradients (a halo past every block); all of them; a
+# single tap of more output channels than operand registers
+LAYERS = [(3, 1, 24, 40, (6, 9, 17), 3, 1, 1, 1, 24, 1, 1.5), (2, 2, 33, 70, (17, 19), 3, 1, 1, 1, 33, 1, 1.5), (3, 1, 8, 16, (9, 9, 9), 5, 1, 4, 2, 8, 1, 1.0),
+          (3, 2, 7, 12, (9, 9, 9), 5, 1, 4, 2, 7, 1, 1.0), (2, 1, 16, 300, (18, 19), 1, 1, 0, 1, 16, 1, 1.0)]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32, torch.float64], ids=["bf16", "f16", "f32", "f64"])
+@pytest.mark.parametrize("spec", LAYERS, ids=lambda s: "%dd-%d-%d-k%d" % (s[0], s[2], s[3], s[5]))
+def test_layer_backward(spec, dtype):
+    """The one-call backward pass on exactly the queried bytes."""
+    print("layer", spec, dtype, flush=True)
+    L, c = _lib.load(), make_case(*spec, dtype=dtype, seed=53, bias=False)
+    x, w, off, gout = (c[k].cuda() for k in ("x", "w", "off", "gout"))
+    nd, elem = c["nd"], x.element_size()
+    volume = lambda t: t[0, 0].numel()
+    query = L.dcn_layer_backward_workspace_bytes
+    query.restype, query.argtypes = ctypes.c_size_t, [ctypes.c_int] * 5 + [ctypes.c_size_t] * 2 + [ctypes.c_int] * 3
+    ws_bytes = query(elem, nd, x.shape[0], x.shape[1], w.shape[0], volume(x), volume(gout), volume(w), c["groups"], c["cpg"])
+    geom = _geom(nd, x, w, c["outs"], c["stride"], c["pad"], c["dil"], c["cpg"], c["groups"])
+    ws = torch.full((ws_bytes // 4 + 1024,), float("nan"), device="cuda")
+    grads = [torch.full_like(t, 7.0) for t in (x, off, w, w[:, 0, 0, 0].flatten() if nd == 2 else w[:, 0, 0, 0, 0])]
+    pointer = lambda t: ctypes.c_void_p(t.data_ptr())
+    dt = {torch.float32: 0, torch.float64: 1, torch.bfloat16: 2, torch.float16: 3}[dtype]
+
+    def call(size):
+        return L.dcn_layer_backward(nd, dt, *(pointer(t) for t in (x, w, off, gout)), *(pointer(t) for t in grads), (ctypes.c_int * len(geom))(*geom), pointer(ws),
+                                    ctypes.c_size_t(size), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream), ctypes.c_uint(0))
+
+    assert call(ws_bytes) == 0, L.dcn_last_error()
+    torch.cuda.synchronize()
+    assert torch.isnan(ws[ws_bytes // 4:]).all()
+    wide = {k: c[k].to(torch.float64 if dtype == torch.float64 else torch.float32) for k in ("x", "off", "w", "gout")}
+    want = orc.backward(wide["x"], wide["off"], wide["w"], wide["gout"], None, c["stride"], c["pad"], c["dil"], c["cpg"], c["groups"])[:3]
+    want = [t.double() for t in want] + [c["gout"].double().sum(dim=[0] + list(range(2, 2 + nd)))]
+    once = {torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12, torch.float32: 0.0, torch.float64: 0.0}[dtype]
+    tols = [1e-10] * 4 if dtype == torch.float64 else [1e-4 + once, 1e-5 + once, 4e-6 + 2 * once, 4e-6 + once]
+    for name, got, ref, tol in zip(("grad_input", "grad_offset", "grad_weight", "grad_bias"), grads, want, tols):
+        err = ((got.cpu().double() - ref).norm() / ref.norm()).item()
+        print("  %s: relative 2-norm error %.2e" % (name, err), flush=True)
+        assert err <= tol
+    assert call(1024) == -2
