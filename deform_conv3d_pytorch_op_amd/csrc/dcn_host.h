@@ -178,7 +178,7 @@ template <typename T> inline size_t backward_weight_need(int N, int C_in, int C_
     long long split_ub = (4096 + tiles_lb - 1) / tiles_lb;
     if (split_ub > 256) split_ub = 256;
     if (split_ub < 1) split_ub = 1;
-    const size_t obytes = (size_t)N * C_out * outV * sizeof(T), rbytes = sizeof(T) == 4 && kV > 1 || C_out / G > 32 ? row_operand_bytes<float>(N, C_out, outV) : 0;
+    const size_t obytes = (size_t)N * C_out * outV * sizeof(T), rbytes = sizeof(T) == 4 && (kV > 1 || C_out / G > 32) ? row_operand_bytes<float>(N, C_out, outV) : 0;
     return align256((size_t)N * C_in * inV * sizeof(T)) + align256(obytes > rbytes ? obytes : rbytes) +
            align256((size_t)split_ub * kV * C_out * (C_in / G) * sizeof(T)) + align256((size_t)N * last_strips((unsigned)outV) * C_out * sizeof(T));
 }

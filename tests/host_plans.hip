@@ -67,6 +67,14 @@ template <typename T, typename S> static bool layout(const Params& P, int& hits)
     return layout_holds<T, S>(P, query, true) && layout_holds<T, S>(P, query + 77, true) && (!more || layout_holds<T, S>(P, least, false)) &&
            data_layout<T, S>(P, bwd_data_weight_bytes<T>(P.M, P.Cg, P.kV, P.G, P.cpg) + 2 * tbytes - 1, l) == DCN_E_WORKSPACE;
 }
+// float64 has no rows of grad_output in operand order: the workspace of backward_weight is that of its copies, partial tiles and sums.
+static bool weight64(const Params& P, int& hits) {
+    const size_t tiles = (size_t)P.kV * ((P.C_in + 15) / 16), most = (4096 + tiles - 1) / tiles, splits = most < 256 ? most : 256;
+    hits += P.M > 32;
+    return backward_weight_need<double>(P.N, P.C_in, P.C_out, P.inV, P.outV, P.kV, P.G) ==
+           align256((size_t)P.N * P.C_in * P.inV * 8) + align256((size_t)P.N * P.C_out * P.outV * 8) + align256(splits * P.kV * P.C_out * P.Cg * 8) +
+               align256((size_t)P.N * last_strips(P.outV) * P.C_out * 8);
+}
 static bool layouts(const Params& P, int& hits) {
     int all[4] = {0, 0, 0, 0};
     const bool ok = layout<float, float>(P, all[0]) && layout<float, Bf16>(P, all[1]) && layout<float, Fp16>(P, all[2]) && layout<double, double>(P, all[3]);
@@ -91,7 +99,7 @@ int main(int argc, char** argv) {
         const int nd = pick(2, 3);
         if (!random_layer(nd, P)) continue;
         ++layers;
-        const bool ok = what == "noalloc" ? noalloc(P, hits) : what == "layout" ? layouts(P, hits) : what == "native16" ? (nd == 3 ? native16<3>(P, hits) : native16<2>(P, hits)) : false;
+        const bool ok = what == "noalloc" ? noalloc(P, hits) : what == "layout" ? layouts(P, hits) : what == "weight64" ? weight64(P, hits) : what == "native16" ? (nd == 3 ? native16<3>(P, hits) : native16<2>(P, hits)) : false;
         if (!ok) {
             printf("%s: %d-D, C_in %d, C_out %d, G %d, cpg %d, k %d %d %d, stride %d %d %d, dil %d %d %d\n", what.c_str(), nd, P.C_in, P.C_out, P.G, P.cpg, P.k[0],
                    P.k[1], P.k[2], P.stride[0], P.stride[1], P.stride[2], P.dil[0], P.dil[1], P.dil[2]);
