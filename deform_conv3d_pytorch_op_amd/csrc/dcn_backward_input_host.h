@@ -55,7 +55,6 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
     // Eight wavefronts per workgroup; four (half the positions, in the block shape with the smallest
     // halo) where only that fits, e.g. under stride 2.
     constexpr int FUSED_HS = sizeof(T) == 4 ? 2720 : 2112;
-    constexpr int FUSED_HS8 = 2016;     // plane stride of the 8-channel float instantiation with compile-time halo extents
     using Kern = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const S*, const S*, const float*, T*, T*, int, unsigned, int);
     struct FusedPlan {
         Params Ph;
@@ -126,7 +125,7 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             // per chunk keeps the input values bank-swizzled and wants the innermost halo extent a
             // multiple of the four-channel groups per voxel.
             size_t tables = 0;
-            bool fixed = false, special = false;
+            bool fixed = false;
             for (int cand = 16; cand >= 4 && !cch; cand /= 2) {
                 if (cand >= 8 && !((ND == 2 || pair) && nw == 8 && fused_chunk8() && seg >= 8 && passes(8) * 4 < passes(4) * 8)) continue;
                 if (cand == 16 && !(ND == 2 && pair && fused_chunk16() && seg >= 16 && passes(16) * 8 < passes(8) * 16)) continue;
@@ -159,23 +158,15 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             const bool breg = ksteps <= Mma<T>::NACC / slot_regs * ((wide || sixteen) ? 16 : 8) / halve;
             // float, 4-channel chunks: a second set of 32 registers takes the operand of up to 128 output channels (16-bit: 256)
             const bool breg2 = sizeof(T) == 4 && !eight && !breg && ksteps <= 64 / halve && fused_breg2();
-            special = ND == 3 && eight && !sixteen && pair && wide && breg && fused_fixed_stride() && Ph.hext[1] == 14 && Ph.hext[2] == 14 &&
-                      Ph.hstride <= FUSED_HS8;
-            if (special) Ph.hstride = FUSED_HS8;
             lds = (size_t)cch * Ph.hstride * chb + tables;
-#define DCN_FUSED_C(CCH_, BREG_, HS_, NW_, PAIR_) backward_input_halo_kernel<T, ND, CCH_, true, (BREG_) || S16, HS_, NW_, true, PAIR_, 1, 0, 0, S>
-#define DCN_FUSED_B2(HS_, NW_, PAIR_) backward_input_halo_kernel<T, ND, 4, true, true, HS_, NW_, true, PAIR_, 2, 0, 0, S>
+#define DCN_FUSED_C(CCH_, BREG_, HS_, NW_, PAIR_) backward_input_halo_kernel<T, ND, CCH_, true, (BREG_) || S16, HS_, NW_, true, PAIR_, 1, S>
+#define DCN_FUSED_B2(HS_, NW_, PAIR_) backward_input_halo_kernel<T, ND, 4, true, true, HS_, NW_, true, PAIR_, 2, S>
             auto pick = [&](auto pair_tag) {
                 constexpr bool PR = decltype(pair_tag)::value;
                 if (sixteen) {
                     if constexpr (ND == 2 && PR && sizeof(T) == 4) kern = breg ? DCN_FUSED_C(16, true, 0, 8, PR) : DCN_FUSED_C(16, false, 0, 8, PR);
                 } else if (eight) {
                     if constexpr (ND == 2 || PR) kern = breg ? DCN_FUSED_C(8, true, 0, 8, PR) : DCN_FUSED_C(8, false, 0, 8, PR);
-                    // the halo of a 3x3x3 kernel at stride 1 and margin 2 under the default block of positions:
-                    // inner extents 14 x 14 and the plane stride fixed at compile time
-                    if constexpr (ND == 3 && PR && sizeof(T) == 4) {
-                        if (special) kern = backward_input_halo_kernel<T, ND, 8, true, true, FUSED_HS8, 8, true, true, 1, 14, 14, S>;
-                    }
                 } else if (breg2) {
                     if constexpr (sizeof(T) == 4) {
                         if (nw == 8) kern = fixed ? DCN_FUSED_B2(FUSED_HS, 8, PR) : DCN_FUSED_B2(0, 8, PR);

@@ -71,7 +71,7 @@ SplitFn<S> split_kernel(int MT, int LW, bool plain) {
         case 116: return backward_weight_split_kernel<ND, 1, 16, S>;
         case 208: return backward_weight_split_kernel<ND, 2, 8, S>;
         case 216: return backward_weight_split_kernel<ND, 2, 16, S>;
-        case 132: case 232: return backward_weight_split_kernel<ND, 2, 32, S>;
+        case 232: return backward_weight_split_kernel<ND, 2, 32, S>;
         case 408: return backward_weight_split_kernel<ND, 4, 8, S>;
         case 416: return backward_weight_split_kernel<ND, 4, 16, S>;
         default: return backward_weight_split_kernel<ND, 4, 32, S>;
@@ -103,10 +103,11 @@ SplitPlan split_plan(const Params& P, bool off, size_t room) {
     c.MT = P.M > 64 ? 4 : P.M > 32 ? 2 : 1;
     c.mchunks = ((P.M + 31) / 32 + c.MT - 1) / c.MT;
     c.igroups = (items + WAVES - 1) / WAVES;
+    if ((P.M <= 32 && least > 0.67 * whole) || items < WAVES) return c;
     const double resident = (double)resident_workgroups(reinterpret_cast<const void*>(split_kernel<ND, S>(c.MT, c.LW, false)), WG, 0);
     const long long nslabs = (long long)P.N * (row_steps(P.outV) / 2);
     const double other = (double)c.igroups * c.mchunks * P.G;
-    if ((P.M <= 32 && least > 0.67 * whole) || items < WAVES || (double)whole * c.mchunks * P.G * (double)nslabs < 2.5 * WAVES * resident) return c;
+    if ((double)whole * c.mchunks * P.G * (double)nslabs < 2.5 * WAVES * resident) return c;
     const size_t one = (size_t)P.kV * P.C_out * P.Cg * sizeof(float);
     long long most = (long long)(room / one);
     if (most > 256) most = 256;

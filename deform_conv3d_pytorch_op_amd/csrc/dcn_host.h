@@ -413,7 +413,6 @@ static bool fused_breg2() {             // DCN_FUSED_BREG2=0: grad_output operan
     static const int v = [] { const char* e = getenv("DCN_FUSED_BREG2"); return (e && atoi(e) == 0) ? 0 : 1; }();
     return v != 0;
 }
-constexpr size_t FUSED_LDS = 157 * 1024;        // dynamic LDS of backward_fused_kernel at most (160 KB less what it declares)
 static bool native16() {                // DCN_NATIVE16=0: the 16-bit entry points always widen to float32 first
     static const int v = [] { const char* e = getenv("DCN_NATIVE16"); return (e && atoi(e) == 0) ? 0 : 1; }();
     return v != 0;

@@ -910,8 +910,7 @@ __device__ inline float weight_bound(const float* __restrict__ bounds, int which
 // S: storage format of input, offset, weight and grad_output (Bf16 / Fp16 with T = float: the grad-column
 // GEMM then runs on the 16-bit matrix instructions, see GcolGemm; requires BREG and PACKW); the
 // gradients are written as T.
-template <typename T, int ND, int CCH, bool COORD, bool BREG, int HS, int NW, bool PACKW = false, bool PAIR = false, int BS = 1,
-          int HE1 = 0, int HE2 = 0, typename S = T>
+template <typename T, int ND, int CCH, bool COORD, bool BREG, int HS, int NW, bool PACKW = false, bool PAIR = false, int BS = 1, typename S = T>
 __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, PlanSet alts, const unsigned* __restrict__ sel,
                                                                   const S* __restrict__ in,
                                                                   const S* __restrict__ off,
@@ -947,10 +946,7 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
     constexpr int CPL = PAIR ? CCH / 2 : CCH;           // cell planes
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int hs = HS ? HS : H.hstride;
-    // HE1, HE2 > 0 fix the two inner halo extents at compile time (the host then launches this
-    // instantiation only for plans with exactly these extents): the distances between the corners of a
-    // sample become immediate offsets of the LDS instructions instead of per-corner address arithmetic
-    const int he1 = HE1 ? HE1 : H.hext[1], he2 = HE2 ? HE2 : H.hext[2];
+    const int he1 = H.hext[1], he2 = H.hext[2];
     Cell* sG = reinterpret_cast<Cell*>(smem_raw);                                       // [CPL][hstride]
     T* sIn = reinterpret_cast<T*>(sG + (size_t)CPL * hs);                               // [hstride][CCH] if COORD: channels of a voxel side by side
     unsigned* sTab = reinterpret_cast<unsigned*>(sIn + (COORD ? (size_t)CCH * hs : 0));   // [hvol]
