@@ -100,7 +100,11 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
                     if (cand >= 8 && !(fused_chunk8() && seg >= 8 && passes(8) * 4 < passes(4) * 8)) continue;
                     if (cand == 16 && !(ND == 2 && fused_chunk16() && seg >= 16 && passes(16) * 8 < passes(8) * 16)) continue;
                     const size_t vb = fused_voxel_bytes<S>(cand), budget = fused_budget();
-                    // the usual block, or the one with the smallest halo where that is a tenth smaller: zeroing, staging and flushing grow with it
+                    // The usual block, or the one with the smallest halo where that is a tenth smaller: zeroing, staging and flushing grow with
+                    // it.  Backward passes of 60 layers of several taps, the other line's time over this one's: never the smallest halo 1.008 on
+                    // average (34 -> 9, stride 1 2 2, 49 x 54 x 31 positions in binary16 1031 us : 636; 35 -> 94, stride 1 2 2, 603 : 634), where it is
+                    // a fifth smaller 1.001, wherever it is smaller 0.999 (0.78 on one, 32 -> 32, two samples of 19 x 20 x 32, 270 : 346, whose
+                    // blocks then fit its extents; 1.02 to 1.03 on three).
                     Params Pc = P, Ps = P;
                     const bool usual = !smallest && plan_halo<T, ND>(Pc, budget, m, cand, 1, tiles, false, 1, nullptr, 1, false);
                     if (plan_halo<T, ND>(Ps, budget, m, cand, 1, tiles, true, 1, nullptr, 1, false) && (!usual || Ps.hvol * 10 < Pc.hvol * 9)) Pc = Ps;
@@ -195,8 +199,8 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             // every item is split over 1, 2 or 4 workgroups (workgroup cz takes every csplit-th chunk), or
             // the items of the whole rounds stay unsplit and only those of the last round are split, as
             // finely as fills the device; they come last in the launch.  A workgroup's fixed part
-            // (grad_output operand, halo table, offsets) costs about a quarter of a chunk, which the
-            // estimate charges per split.  The workgroups that share an item add their grad_offset parts with
+            // (norms of grad_output, offsets, first loads; grad_output operand and halo table in the kernel with single cells) counts as a quarter of
+            // a chunk (60 layers of several taps: a tenth, a half and a whole one within 0.1 % on average and 2 % on any; none 1.02, at worst 1.41).  The workgroups that share an item add their grad_offset parts with
             // float atomics on a zero-filled buffer; the only owner of an item stores running sums.
             const int nchunks = (seg + cch - 1) / cch;
             const long long items = (long long)Ph.N * Ph.tiles * Ph.DG;

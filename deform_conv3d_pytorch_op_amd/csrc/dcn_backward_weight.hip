@@ -82,6 +82,10 @@ SplitFn<S> split_kernel(int MT, int LW, bool plain) {
 // first threshold counts items of 32 lanes.  50 training layers, us per step, 32 lanes (or the other
 // kernels) : this: 1.058 times as fast on average, at worst 0.994; 16 -> 38 in groups of 4, 3-D, two samples of 16 700 positions in bfloat16 464 : 322; 20 -> 339 in
 // groups of 5, 7200 positions 301 : 245; 16 -> 14, 165 000 positions in bfloat16 734 : 602; 24 -> 36 in groups of 6, 10 600 positions 184 : 162.
+// Estimated time of a split, in us: a wavefront's share of the slabs, 4 to a slab, times the rounds of workgroups -- of less than one, the
+// part a workgroup takes when its CU holds no other, and the rest with what shares the CU -- and the partial tiles.  Backward passes
+// of 60 layers, the other line's time over this one's: 0.2 for 0.4 1.03 (at worst 1.13), 0.6 1.013 (1.07), 1 1.005 (1.04); 1 for 4 1.019 (1.12), 2 1.005,
+// 8 and 16 1.001 (1.03).  A plain convolution is planned by the occupancy of the kernel with offsets (24 layers by its own: 1.0015, at worst 1.02).
 struct SplitPlan { int MT, LW, mchunks, igroups, nsplit; };     // nsplit 0: not a layer for it, or no room
 template <int ND, typename S>
 SplitPlan split_plan(const Params& P, bool off, size_t room) {
