@@ -90,7 +90,17 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
     // worst 1.2 (2-D, 64 -> 64, 75 x 101 positions: 34 / 30).  Limits of half and of twice as many workgroups: the same
     // on average, single layers 0.7 to 0.8 times as fast.  Not for a single tap in 3-D: the halo of 64 positions costs more to
     // stage than it saves (128 -> 32 channels, 16 x 28 x 28: 42 with, 29 without).
+    // And, of any number of positions, 3-D layers whose halo of 256 positions holds no eight channels (3x3x3 at stride 2 along every axis: 5733
+    // voxels): they would take four at a time and leave half of the reduction slots empty.  Those of more than 64 output channels to a
+    // group or at least 32 input channels, without / with, 3x3x3: 176 -> 151, 14 x 27 x 37 positions 1289 / 716; 64 -> 239, three samples of
+    // 14 x 12 x 30 478 / 347; 64 -> 16, four of 17 x 18 x 19 252 / 216; 25 such layers 0.75 of the time on average, at worst 1.09 (16 -> 224 in two
+    // groups, 75 / 81), and 0.6 with offsets that reach past the margins.  Fewer channels lose: 8 -> 24, 88 / 111.
     bool small = false;
+    auto holds_eight = [&](bool smallest) {
+        Params Pt = P;
+        return plan_halo<T, ND>(Pt, MAX_LDS, default_margin(), 1 << 30, sizeof(S), WAVESH, smallest, FG, nullptr, 1, false);
+    };
+    const bool wide_halo = MX && !S16 && ND == 3 && (P.M > 64 || P.Cg >= 32) && !holds_eight(false) && !holds_eight(true);
     // Shared columns only where they can fill half of the device: with a workgroup for every 16 input channels in
     // float32, whose channels can be split, and without in 16-bit storage, whose cannot (256 -> 256 channels, 3x3, 2 x 28 x 28
     // positions in bfloat16: 16 units, 105 us shared and 60 with several wavefronts to a position).
@@ -104,7 +114,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
         Params Pt = P;
         const int mt = mtiles_all > 2 ? 4 : mtiles_all, mc = (mtiles_all + mt - 1) / mt;
         if (plan_halo<T, ND>(Pt, MAX_LDS, default_margin(), 1 << 30, sizeof(S), 2, false, FG, nullptr, 1, false) &&
-            (long long)Pt.N * Pt.tiles * P.G * mc <= (mt == 4 ? 1 : 2) * cu_count()) {
+            (long long)Pt.N * Pt.tiles * P.G * mc <= (wide_halo ? 0x7fffffffLL : (mt == 4 ? 1 : 2) * cu_count())) {
             small = true;
             MT = mt;
             P.mchunks = mc;

@@ -50,6 +50,24 @@ def test_edges_and_accuracy(spec):
     assert err <= 2e-6
 
 
+# 3-D layers whose halo of 256 positions holds no eight channels, of more blocks of 64 positions than the device holds at once: few
+# input channels and several row tiles, one and two row tiles, groups, samples past every halo, 125 taps
+WIDE_HALOS = [(3, 2, 8, 70, (33, 65, 66), 3, 2, 1, 1, 8, 1, 1.5), (3, 1, 32, 20, (41, 66, 67), 3, 2, 1, 1, 16, 1, 2.5), (3, 1, 36, 40, (41, 66, 67), 3, 2, 1, 1, 12, 1, 9.0),
+              (3, 1, 64, 140, (35, 50, 51), 3, 2, 1, 1, 64, 2, 1.0), (3, 1, 8, 66, (25, 66, 67), 5, 2, 2, 1, 4, 1, 1.5)]
+
+
+@pytest.mark.parametrize("spec", WIDE_HALOS, ids=lambda s: "%d-%d-k%d-cpg%d" % (s[2], s[3], s[5], s[9]))
+def test_wide_halos(spec):
+    """2-norm: a chain of float32 roundings (2e-6) and a coordinate rounded by up to 2^-18 (half a unit below 128), which moves a sample
+    of N(0, 1) values by as much."""
+    print("wide halos", spec, flush=True)
+    c = make_case(*spec, dtype=torch.float32, seed=24)
+    got, want = _forward(c).cpu().double(), _oracle(c)
+    err = ((got - want).norm() / want.norm()).item()
+    print("  relative 2-norm error %.2e" % err, flush=True)
+    assert err <= 2e-6 + 2.0 ** -18
+
+
 @pytest.mark.parametrize("spec", [EDGES[2], EDGES[4], EDGES[7]], ids=["2d-split", "2d-shared", "3d"])
 @pytest.mark.parametrize("what", ["input", "weight", "huge"])
 def test_results_that_are_not_finite(spec, what):
