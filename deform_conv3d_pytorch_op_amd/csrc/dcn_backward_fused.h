@@ -523,12 +523,13 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
                         if constexpr (ND == 3) {
                             // out-of-range samples of the 3-D operator: -|gcol| per axis with p <= -1, +|gcol| with p >= the LENGTH extent
                             // (h and w are compared with it too), summed over the channels
-                            // (deform3d/lib/deform_conv3d_cuda_kernel.cu:470-481).  Selected, not multiplied: 0 * inf would be NaN
+                            // (deform3d/lib/deform_conv3d_cuda_kernel.cu:470-481).  Selected, not multiplied: 0 * inf would be NaN, and
+                            // is in the columns past the chunk's channels, whose weights are zeros
                             const bool oor = slot_ok && !inside && !P.oob_zero;
                             if (__any(oor)) {
                                 float asum = 0.f;
 #pragma unroll
-                                for (int e = 0; e < CCH; ++e) asum += fabsf(gv[e]);
+                                for (int e = 0; e < CCH; ++e) asum += e < nch ? fabsf(gv[e]) : 0.f;
                                 if (oor) {
 #pragma unroll
                                     for (int a = 0; a < ND; ++a) ga[a] = pq[a] <= -1.f ? -asum : (pq[a] >= (float)P.in[0] ? asum : 0.f);

@@ -1581,12 +1581,13 @@ __global__ __launch_bounds__(NW * 64) void backward_input_halo_kernel(Params P, 
                         // out-of-range samples of the 3-D operator: -|gcol| per axis with p <= -1, +|gcol|
                         // with p >= the LENGTH extent (h and w are compared with it too), summed over the
                         // channels (deform3d/lib/deform_conv3d_cuda_kernel.cu:470-481).  Selected, not
-                        // multiplied: 0 * inf would be NaN where the reference adds nothing
+                        // multiplied: 0 * inf would be NaN where the reference adds nothing (and is in the rows past the
+                        // chunk's channels, whose packed weights are zeros)
                         const bool oor = slot_ok && !inside && !P.oob_zero;
                         if (__any(oor)) {
                             T asum = 0;
 #pragma unroll
-                            for (int rr = 0; rr < RPS; ++rr) asum += fabs(gv[rr]);
+                            for (int rr = 0; rr < RPS; ++rr) asum += row_ch(ts * RPS + rr, q) < nch ? fabs(gv[rr]) : (T)0;
                             if (oor) {
 #pragma unroll
                                 for (int a = 0; a < ND; ++a)

@@ -312,6 +312,28 @@ def test_non_finite_grad_output_and_weight_propagate(name, dtype, where):
             assert (g[fin] - w[fin]).abs().max().item() <= tol * (scale if scale > 0 else 1.0), nm
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.bfloat16, torch.float16], ids=["f32", "f64", "bf16", "f16"])
+@pytest.mark.parametrize("spec", [(3, 1, 9, 20, (4, 8, 9), 3, 1, 1, 1, 9, 1, 1.0), (3, 1, 13, 33, (9, 17, 15), 3, 2, 1, 1, 13, 1, 1.0),
+                                  (3, 2, 10, 12, (4, 6, 9), 1, 1, 0, 1, 5, 1, 1.0)], ids=["k3", "strided", "k1"])
+def test_non_finite_grad_output_at_samples_outside(spec, dtype):
+    """The gradient that the 3-D operator gives the offsets of a sample outside the volume is the sum of |grad column| over the channels of
+    its deformable group (deform3d/lib/deform_conv3d_cuda_kernel.cu:470-481): infinite where grad_output is, also where the channels do
+    not fill the kernels' chunks; NaN only where grad_output is."""
+    print("non-finite outside", spec, dtype, flush=True)
+    c = make_case(*spec, dtype=dtype, seed=51, bias=False)
+    for at, value in (((2, 3, 1), float("inf")), ((1, 0, 4), -float("inf")), ((0, 3, 3), float("nan"))):
+        at = tuple(min(a, o - 1) for a, o in zip(at, c["outs"]))
+        c["off"][(0, slice(0, None, 3)) + at] = -30
+        c["off"][(0, slice(1, None, 3)) + at] = 40
+        c["gout"][(0, 3) + at] = value
+    got = run_gpu(c)[2].cpu().double()
+    wide = {k: v.float() if torch.is_tensor(v) and dtype != torch.float64 else v for k, v in c.items()}
+    want = run_oracle(wide)[2].double()
+    assert torch.isposinf(want).any() and torch.isneginf(want).any() and torch.isnan(want).any()
+    for special in (torch.isnan, torch.isposinf, torch.isneginf):
+        assert torch.equal(special(got), special(want)), special.__name__
+
+
 @pytest.mark.parametrize("name", ["2d_c3_like", "2d_rect_kernel_stride_dil", "3d_dilation3", "3d_basic"])
 @pytest.mark.parametrize("dtype", [torch.float64, torch.float32], ids=["f64", "f32"])
 def test_standard_output_size_is_a_crop_of_the_reference_layer(name, dtype):
