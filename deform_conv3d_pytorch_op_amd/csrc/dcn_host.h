@@ -7,6 +7,7 @@
 #include "dcn_forward_split.h"
 #include "dcn_prepare.h"
 
+#include <algorithm>
 #include <cstdio>
 #include <cstdlib>
 #include <cstring>
@@ -287,7 +288,8 @@ inline int relayout(const Params& P, const T* w, T* wt, int channel_fastest, hip
 //   DCN_FORWARD_SHARED=0   forward pass, float32 and 16-bit: never share the sampled columns of a block among wavefronts
 //   DCN_FORWARD_SMALL=0    forward pass, float32 and 16-bit: never several wavefronts to a position
 //   DCN_FORWARD_TINY=0     ... never more than four
-//   DCN_SCATTER_BUDGET_KB  LDS per workgroup of the privatised scatter kernels (default 156: backward_fused_kernel, 144: the others)
+//   DCN_SCATTER_BUDGET_KB  dynamic LDS per workgroup of the privatised scatter kernels (default 156, at most 157: backward_fused_kernel, 144, at
+//                          most 159: the others)
 //   DCN_SCATTER=global     scatter grad-input with global atomics instead of the LDS-privatised kernel
 //   DCN_COORD=separate     grad_offset from the channels-last kernel instead of the fused LDS-halo kernel
 //   DCN_FUSED_WAVES=4      fused backward kernel with four wavefronts per workgroup even where eight fit
@@ -306,9 +308,9 @@ static size_t env_kb(const char* name, int dflt) {
     return (size_t)(v > 0 ? v : dflt) * 1024;
 }
 static size_t lds_budget() { static const size_t v = env_kb("DCN_LDS_BUDGET_KB", 72); return v; }
-static size_t scatter_budget() { static const size_t v = env_kb("DCN_SCATTER_BUDGET_KB", 144); return v; }
-// backward_fused_kernel: all that a workgroup can have beside what the kernel declares itself
-static size_t fused_budget() { static const size_t v = env_kb("DCN_SCATTER_BUDGET_KB", 156); return v; }
+// (at most what a CU has beside what the kernels declare themselves: backward_input_halo_kernel 100 bytes, backward_fused_kernel 2120)
+static size_t scatter_budget() { static const size_t v = std::min<size_t>(env_kb("DCN_SCATTER_BUDGET_KB", 144), 159 * 1024); return v; }
+static size_t fused_budget() { static const size_t v = std::min<size_t>(env_kb("DCN_SCATTER_BUDGET_KB", 156), 157 * 1024); return v; }
 static bool fused_coord() {
     static const int v = [] { const char* e = getenv("DCN_COORD"); return (e && strcmp(e, "separate") == 0) ? 0 : 1; }();
     return v != 0;

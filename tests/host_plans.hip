@@ -93,6 +93,12 @@ int main(int argc, char** argv) {
         prep.add(PREP_PLAN, 1);
         return ok && prep.full && prep.jobs.n == MAX_PREP ? 0 : 1;
     }
+    if (what == "budget") {         // of any DCN_SCATTER_BUDGET_KB: what a CU has beside the 2120 and 100 bytes that the kernels declare; 72 stays 72
+        const size_t cu = 160 * 1024, kb72 = 72 * 1024;
+        return fused_budget() + 2120 <= cu && scatter_budget() + 100 <= cu && fused_budget() >= kb72 && scatter_budget() >= kb72 &&
+                       (env_kb("DCN_SCATTER_BUDGET_KB", 0) != kb72 || (fused_budget() == kb72 && scatter_budget() == kb72))
+                   ? 0 : 1;
+    }
     int layers = 0, hits = 0;
     for (const int count = atoi(argv[3]); layers < count;) {
         Params P;

@@ -4,7 +4,8 @@ settings, each in a process of its own (the knobs are read once per process):
   DCN_HALO_MARGIN=0    almost every sample reaches past the LDS halo -> global fallback paths
   DCN_HALO_MARGIN=50   the halo never fits -> kernels that do not use LDS tiling at all
   DCN_SCATTER=global   grad-input through global atomics on the channels-last copy
-  DCN_LDS_BUDGET_KB / DCN_SCATTER_BUDGET_KB small -> smallest channel chunks
+  DCN_LDS_BUDGET_KB / DCN_SCATTER_BUDGET_KB small -> smallest channel chunks; DCN_SCATTER_BUDGET_KB past what a workgroup can
+                       have -> all of that
   DCN_FORWARD_WG=1024  the 1024-thread forward variant also where the grid would be too small for it
   DCN_FORWARD_WG=512   ... and never
   DCN_COORD=separate   grad_offset from the channels-last kernel, grad_input from the scatter-only kernel
@@ -43,6 +44,7 @@ SETTINGS = [
     {"DCN_HALO_MARGIN": "50"},
     {"DCN_SCATTER": "global"},
     {"DCN_LDS_BUDGET_KB": "16", "DCN_SCATTER_BUDGET_KB": "72"},
+    {"DCN_SCATTER_BUDGET_KB": "1000"},
     {"DCN_FORWARD_WG": "1024", "DCN_CSPLIT": "4"},
     {"DCN_FORWARD_WG": "512", "DCN_CSPLIT": "1"},
     {"DCN_COORD": "separate"},

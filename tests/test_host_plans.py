@@ -20,3 +20,13 @@ def probe(tmp_path_factory):
 def test_rule(probe, what):
     r = subprocess.run([probe, what, "7", "20000"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
+
+
+@pytest.mark.parametrize("kb", [None, "72", "156", "158", "160", "100000"])
+def test_lds_budget(probe, kb):
+    """A budget past what a workgroup can have is that: its plans launch."""
+    env = dict(os.environ)
+    env.pop("DCN_SCATTER_BUDGET_KB", None)
+    if kb:
+        env["DCN_SCATTER_BUDGET_KB"] = kb
+    assert subprocess.run([probe, "budget", "7", "1"], env=env, timeout=60).returncode == 0
