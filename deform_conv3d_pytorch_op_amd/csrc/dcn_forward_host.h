@@ -162,10 +162,12 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
         }
         for (int t = 1; t <= 2; ++t) {
             Params Pt = P;
+            const bool forced = forward_tiny() == t;
+            if (forward_tiny() > 0 && !forced) continue;
             if (!plan_halo<T, ND>(Pt, MAX_LDS, default_margin(), 1 << 30, sizeof(S), t, true, FG, nullptr, 1, false)) continue;
-            for (int fs = 1; parts_fit(fs) && (long long)Pt.N * Pt.tiles * P.G * P.mchunks * fs <= cu_count(); fs *= 2) {
+            for (int fs = 1; parts_fit(fs) && ((long long)Pt.N * Pt.tiles * P.G * P.mchunks * fs <= cu_count() || (forced && fs == 1)); fs *= 2) {
                 const double e = estimate(Pt, t, 16 / t, fs);
-                if (e < (tiny ? best : 0.8 * best)) { best = e; tiny = t; fsplit = fs; }
+                if (e < (tiny ? best : 0.8 * best) || (forced && !tiny)) { best = e; tiny = t; fsplit = fs; }
             }
         }
     }
@@ -444,8 +446,8 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             if (wgs > 0x7fffffffLL) return fail(DCN_E_ARGUMENT, "too many workgroups for one launch");
             const dim3 grid((unsigned)wgs);
             if (trace_plans()) {
-                fprintf(stderr, "dcn forward: %d wavefronts, MT %d, grid %u (%lld unsplit, rest x %d), LDS %zu, every unit split x %d\n", nw, MT, grid.x,
-                        tsplit > 1 ? whole : 0LL, tsplit, lds, fsplit);
+                fprintf(stderr, "dcn forward: %d position tiles, %d wavefronts, MT %d, grid %u (%lld unsplit, rest x %d), LDS %zu, every unit split x %d\n", nw,
+                        pairs || tiny ? 16 : shared || small ? 8 : nw, MT, grid.x, tsplit > 1 ? whole : 0LL, tsplit, lds, fsplit);
                 if (ts.splitB) fprintf(stderr, "  of the rest: %u units x %d, the others x %d with %d channels per pass\n", ts.unitsA, tsplit, ts.splitB, ts.cchB);
                 for (int k = 0; k < pc.nplans; ++k)
                     fprintf(stderr, "  plan %d: margin %d, halo %d x %d x %d, %d channels per pass, base cost %.3f\n", k, pc.margin[k],

@@ -287,7 +287,8 @@ inline int relayout(const Params& P, const T* w, T* wt, int channel_fastest, hip
 //   DCN_FORWARD_SLOTS=n    forward pass: plan the launch as if n workgroups ran at once (test hook)
 //   DCN_FORWARD_SHARED=0   forward pass, float32 and 16-bit: never share the sampled columns of a block among wavefronts
 //   DCN_FORWARD_SMALL=0    forward pass, float32 and 16-bit: never several wavefronts to a position
-//   DCN_FORWARD_TINY=0     ... never more than four
+//   DCN_FORWARD_TINY=0     ... never more than four; 1 / 2 (test hook): sixteen to blocks of 32 positions / eight to blocks of 64 on every
+//                          layer with several, of up to two row tiles
 //   DCN_SCATTER_BUDGET_KB  dynamic LDS per workgroup of the privatised scatter kernels (default 156, at most 157: backward_fused_kernel, 144, at
 //                          most 159: the others)
 //   DCN_SCATTER=global     scatter grad-input with global atomics instead of the LDS-privatised kernel
@@ -403,9 +404,9 @@ static bool forward_small() {            // DCN_FORWARD_SMALL=0: the forward pas
     static const int v = [] { const char* e = getenv("DCN_FORWARD_SMALL"); return (e && atoi(e) == 0) ? 0 : 1; }();
     return v != 0;
 }
-static bool forward_tiny() {             // DCN_FORWARD_TINY=0: at most four wavefronts to a position
-    static const int v = [] { const char* e = getenv("DCN_FORWARD_TINY"); return (e && atoi(e) == 0) ? 0 : 1; }();
-    return v != 0;
+static int forward_tiny() {              // DCN_FORWARD_TINY=0: at most four wavefronts to a position; 1, 2: see above; -1: unset
+    static const int v = [] { const char* e = getenv("DCN_FORWARD_TINY"); return e ? atoi(e) : -1; }();
+    return v;
 }
 static bool fused_pair() {              // DCN_FUSED_PAIR=0: float32 LDS cells of the fused backward kernel hold one channel each (64-bit)
     static const int v = [] { const char* e = getenv("DCN_FUSED_PAIR"); return (e && atoi(e) == 0) ? 0 : 1; }();
