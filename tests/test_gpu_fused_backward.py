@@ -1,4 +1,10 @@
 """backward_fused_kernel: edges of its tiles, chunks and block shapes, and the operands that bfloat16 parts do not hold."""
+import ast
+import os
+import re
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -8,8 +14,9 @@ from tests.cases import make_case
 pytestmark = pytest.mark.gpu
 
 # (nd, N, C_in, C_out, ins, k, stride, pad, dil, cpg, groups, reach): steps of 16 output channels and their remainders;
-# chunks of 16, 8 and 4 channels and short ones; one, two and several tiles to a contraction (1, 9, 25 taps); blocks of 128
-# positions (strides in 3-D); wide halos and samples past every halo; a deformable group over two convolution groups
+# chunks of 16, 8 and 4 channels and short ones; two and several tiles to a contraction (9, 25 taps); blocks of 128
+# positions (strides in 3-D); wide halos and samples past every halo; a deformable group over two convolution groups.  Single taps
+# take backward_input_halo_kernel, but for 16-bit storage of more than 256 output channels (EDGES16).
 EDGES = [
     (2, 1, 16, 1, (17, 16), 3, 1, 1, 1, 16, 1, 1.5), (2, 1, 17, 15, (9, 33), 3, 1, 1, 1, 17, 1, 1.5),
     (2, 1, 33, 16, (16, 17), 3, 1, 1, 1, 33, 1, 3.5), (2, 2, 15, 17, (11, 12), 3, 1, 1, 1, 15, 1, 1.0),
@@ -20,6 +27,10 @@ EDGES = [
     (3, 1, 12, 80, (9, 21, 19), 3, 2, 1, 1, 12, 1, 2.0), (3, 1, 16, 130, (6, 15, 17), 3, (1, 2, 2), 1, 1, 8, 1, 2.0),
     (3, 1, 20, 17, (5, 9, 9), 2, 1, 1, 1, 10, 1, 6.0), (3, 1, 8, 24, (9, 9, 9), 3, 1, 2, 2, 4, 2, 2.5),
     (3, 1, 10, 7, (6, 5, 40), 1, 1, 0, 1, 5, 1, 1.5),
+]
+EDGES16 = [
+    (2, 1, 18, 257, (13, 11), 1, 1, 0, 1, 18, 1, 1.5), (2, 1, 9, 264, (17, 16), 1, 2, 0, 1, 9, 1, 1.5), (2, 2, 12, 300, (9, 33), 1, 1, 0, 1, 3, 1, 3.5),
+    (3, 1, 10, 257, (5, 6, 9), 1, 1, 0, 1, 5, 1, 1.5), (3, 1, 13, 272, (4, 9, 20), 1, (1, 2, 2), 0, 1, 13, 1, 6.0), (3, 1, 16, 530, (4, 8, 8), 1, 1, 0, 1, 8, 2, 1.5),
 ]
 
 
@@ -50,6 +61,29 @@ def test_edges(spec, dtype):
         err = ((got - want).norm() / want.norm()).item()
         print("  relative 2-norm error %.2e" % err, flush=True)
         assert err <= tol + once
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("spec", EDGES16, ids=lambda s: "%dd-%d-%d-k%d-cpg%d" % (s[0], s[2], s[3], s[5], s[9]))
+def test_edges_of_single_taps(spec, dtype):
+    test_edges(spec, dtype)
+
+
+def test_kernels_of_the_edges():
+    """backward_fused_kernel runs what these tests are for (the trace of the plans, in a process of its own: the knob is read once)."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    r = subprocess.run([sys.executable, "-u", "-m", "pytest", __file__, "-q", "-x", "-s", "-m", "gpu", "-k", "test_edges", "--timeout", "120",
+                        "--timeout-method", "thread"], cwd=os.path.dirname(here), env=dict(os.environ, DCN_TRACE_PLANS="1"), stdout=subprocess.PIPE,
+                       stderr=subprocess.STDOUT, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout[-3000:]
+    cases = r.stdout.split("edges (")[1:]
+    assert len(cases) == 3 * len(EDGES) + 2 * len(EDGES16)
+    for case in cases:
+        spec = ast.literal_eval("(" + case[:case.index(" torch.")])
+        launches = re.findall(r"dcn backward_input_offset: launch.*", case)
+        print(spec, launches, flush=True)
+        one_tap = spec[5] == 1 and spec not in EDGES16
+        assert launches and all(("(halo kernel)" in l) == one_tap for l in launches), spec
 
 
 @pytest.mark.parametrize("spec", [EDGES[5], EDGES[10], EDGES[13]], ids=["2d", "3d", "3d-strided"])
