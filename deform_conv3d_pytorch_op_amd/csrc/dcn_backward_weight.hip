@@ -185,14 +185,13 @@ int backward_weight_plan(const Params& Pin, const S* in, const S* off, const S* 
         const int TN = Mma<float>::TN, CT = 2 * TN;
         if (P.C_in % 2 || P.cpg % 2 || P.Cg % 2) return DCN_OK;
         const int mtiles = (P.M + TN - 1) / TN;
-        // Two row tiles per workgroup at most (four would take 128 accumulator registers beside the two
-        // channel tiles: one wavefront per SIMD), so more than 64 output channels sample everything once
-        // per 64 of them, and channel segments that fill their 64-channel tiles badly waste the lanes'
-        // loads.  Both kernels are bounded by their corner loads: this one issues half as many per
-        // channel as the float32 kernel (four row tiles, 32-channel tiles), times the re-sampling and the
-        // unused part of the tiles.  Where that comes to more than the float32 kernel's, that kernel on
-        // widened tensors is the faster one (128 -> 128 channels in deformable groups of 32, 3-D: 2.5 ms
-        // here against 1.2 + 0.15 for widening; 256 -> 256 in one group, 2-D: 0.20 here against 0.31).
+        // Which layers the 16-bit kernels take: those for which backward_weight16_kernel reads no more of the corners than the float32
+        // kernels do on widened tensors, five to four.  It has two row tiles per workgroup at most (four would take 128 accumulator
+        // registers beside its two channel tiles: one wavefront per SIMD), so more than 64 output channels sample everything once
+        // per 64 of them, and channel segments that fill their 64-channel tiles badly waste the lanes' loads; it issues half as many per
+        // channel (128 -> 128 channels in deformable groups of 32, 3-D: 2.5 ms against 1.2 + 0.15 for widening; 256 -> 256 in one
+        // group, 2-D: 0.20 against 0.31).  backward_weight_split_kernel samples once for 128 output channels, but rounds the samples to the
+        // storage format, which the widened operator does not: the line stands.
         c.MT = mtiles >= 2 ? 2 : 1;
         P.mchunks = (mtiles + c.MT - 1) / c.MT;
         P.nctiles = 0;
