@@ -526,10 +526,12 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
                             // (deform3d/lib/deform_conv3d_cuda_kernel.cu:470-481).  Selected, not multiplied: 0 * inf would be NaN, and
                             // is in the columns past the chunk's channels, whose weights are zeros
                             const bool oor = slot_ok && !inside && !P.oob_zero;
-                            if (__any(oor)) {
+                            if (__builtin_expect(__any(oor), 0)) {
                                 float asum = 0.f;
+                                int real = nch;
+                                asm volatile("" : "+s"(real));         // (compared here: hoisted, the comparisons spill seven more registers)
 #pragma unroll
-                                for (int e = 0; e < CCH; ++e) asum += e < nch ? fabsf(gv[e]) : 0.f;
+                                for (int e = 0; e < CCH; ++e) asum += e < real ? fabsf(gv[e]) : 0.f;
                                 if (oor) {
 #pragma unroll
                                     for (int a = 0; a < ND; ++a) ga[a] = pq[a] <= -1.f ? -asum : (pq[a] >= (float)P.in[0] ? asum : 0.f);
