@@ -27,7 +27,7 @@
 // What bounds it: the corner reads.  64 -> 64 channels, 3x3x3, 4 x 16 x 56 x 56 positions: 12.2 GB through the vector caches,
 // whose data return is busy 96 % of the time (8.5 GB from L2), the matrix units 20 %, the vector units 40 %.  backward_weight_kernel
 // with the float32 instructions kept the matrix units busy half of the time and read grad_output once per wavefront: with rows
-// straight from L2 this kernel was no faster in 3-D (678 us against 633) and 13 % faster in 2-D.  us, that kernel -> this one: 256 -> 256,
+// straight from L2 this kernel was no faster in 3-D (678 us against 633) and 13 % faster in 2-D.  us of the kernel alone, that one -> this one: 256 -> 256,
 // 3x3, 8 x 56 x 56: 332 -> 240; 512 -> 512 in two groups, 3x3, 4 x 28 x 28: 105 -> 80; 128 -> 128, 3x3x3, 2 x 16 x 56 x 56
 // (stride 2): 1022 -> 860; 64 -> 64 as above: 633 -> 600; 64 -> 64, 3x3, no offsets, 25 088 positions: 33 -> 25.
 // The preparing launch pays 2 to 20 us of it back (three halves of the bytes of a channels-last copy).

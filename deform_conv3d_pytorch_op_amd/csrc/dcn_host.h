@@ -293,14 +293,16 @@ inline int relayout(const Params& P, const T* w, T* wt, int channel_fastest, hip
 //                          most 159: the others)
 //   DCN_SCATTER=global     scatter grad-input with global atomics instead of the LDS-privatised kernel
 //   DCN_COORD=separate     grad_offset from the channels-last kernel instead of the fused LDS-halo kernel
-//   DCN_FUSED_WAVES=4      fused backward kernel with four wavefronts per workgroup even where eight fit
-//   DCN_FUSED_CHUNK=4      fused backward kernel with 4-channel chunks also where it would take 8 or 16; =8: never 16 (2-D layers)
-//   DCN_FUSED_TAIL=0       fused backward kernel: all items split alike, never only those of the last round
-//   DCN_CSPLIT=n           fused backward kernel: every item split over n workgroups
-//   DCN_FUSED_SLOTS=n      fused backward kernel: plan the launch as if n workgroups ran at once (test hook)
-//   DCN_FUSED_FIXED=0      fused backward kernel: runtime plane stride even where the compile-time one fits
-//   DCN_FUSED_PAIR=0       fused backward kernel, float32: one channel per 64-bit LDS cell instead of two 32-bit halves
-//   DCN_FUSED_BREG2=0      fused backward kernel: no second register set for the grad_output operand of 64 < M <= 128
+// Both kernels that form grad_input and grad_offset over a halo, backward_fused_kernel and backward_input_halo_kernel:
+//   DCN_FUSED_WAVES=4      blocks of 128 positions in the shape with the smallest halo even where 256 fit (the second: four wavefronts)
+//   DCN_FUSED_CHUNK=4      4-channel chunks also where they would take 8 or 16; =8: never 16 (2-D layers)
+//   DCN_FUSED_TAIL=0       all items split alike, never only those of the last round
+//   DCN_CSPLIT=n           every item split over n workgroups
+//   DCN_FUSED_SLOTS=n      plan the launch as if n workgroups ran at once (test hook)
+//   DCN_FUSED_PAIR=0       float32: one channel per 64-bit LDS cell instead of two 32-bit halves, and never backward_fused_kernel
+// backward_input_halo_kernel alone:
+//   DCN_FUSED_FIXED=0      runtime plane stride even where the compile-time one fits
+//   DCN_FUSED_BREG2=0      no second register set for the grad_output operand of 64 < M <= 128
 //   DCN_GLOBAL_PLAN=0      backward_input_offset (3-D): the device is not offered the path without LDS tiling
 //   DCN_NATIVE16=0         16-bit entry points: always widen to float32 and run the float32 kernels
 static size_t env_kb(const char* name, int dflt) {
