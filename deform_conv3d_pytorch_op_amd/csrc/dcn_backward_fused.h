@@ -543,48 +543,87 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
                             }
                         }
                         if (__builtin_expect(__any(far), 0)) {         // samples that reach past the halo: global memory
-                            TapGeo<float, ND> t;                       // the reference's corner rule on the same coordinate
-                            t.inside = far;
+                            // 3-D and 16-bit storage: the samples one after the other, a lane for each of a sample's (corner, channel) pairs, one round trip
+                            // to memory each.  A loop over the channels with the samples in their lanes waits for as many round trips as there are
+                            // channels however few the samples, and its spills cost the tap slots (us of a call, that loop -> this: 64 -> 64, 3x3x3, 200 704
+                            // positions, offsets U[-1.5, 1.5] 1311 -> 1272, N(0, 0.7) 1865 -> 1284, at margin 2 N(0, 1) 2932 -> 1682 and U[-3, 3] 5737 -> 3902; in
+                            // bfloat16, 50 176 positions, U[-6, 6] 9591 -> 5783).  float32 in 2-D, where wide halos are cheap and far samples rare: the loop
+                            // (steps of 512 -> 512 in two groups 328 us, 331 with this).
+                            if constexpr (ND == 2 && sizeof(S) == 4) {
+                                TapGeo<float, ND> t;                       // the reference's corner rule on the same coordinate
+                                t.inside = far;
 #pragma unroll
-                            for (int a = 0; a < ND; ++a) {
-                                float pa = pq[a];
-                                asm volatile("" : "+v"(pa));           // (worked out here, not hoisted into the common path)
-                                const int l = far ? (int)pa : 0;
-                                t.p[a] = pa;
-                                t.lo[a] = l;
-                                t.hi[a] = (pa >= (float)(P.in[slot<ND>(a)] - 1) || pa <= 0.f) ? l : l + 1;
-                                t.f[a] = pa - (float)l;
-                            }
-                            tap_corner_idx<float, ND>(P, t);
+                                for (int a = 0; a < ND; ++a) {
+                                    float pa = pq[a];
+                                    asm volatile("" : "+v"(pa));           // (worked out here, not hoisted into the common path)
+                                    const int l = far ? (int)pa : 0;
+                                    t.p[a] = pa;
+                                    t.lo[a] = l;
+                                    t.hi[a] = (pa >= (float)(P.in[slot<ND>(a)] - 1) || pa <= 0.f) ? l : l + 1;
+                                    t.f[a] = pa - (float)l;
+                                }
+                                tap_corner_idx<float, ND>(P, t);
 #pragma unroll 1
-                            for (int e = 0; e < nch; ++e) {
-                                float g1 = 0.f;
+                                for (int e = 0; e < nch; ++e) {
+                                    float g1 = 0.f;
 #pragma unroll
-                                for (int x = 0; x < CCH; ++x) g1 = x == e ? gv[x] : g1;
-                                const size_t chan = ((size_t)n * P.C_in + cc0 + e) * P.inV;
-                                if (far) {
-                                    float* gc = gin + chan;
-                                    const S* ic = in + chan;
-                                    float vv[NC];
+                                    for (int x = 0; x < CCH; ++x) g1 = x == e ? gv[x] : g1;
+                                    const size_t chan = ((size_t)n * P.C_in + cc0 + e) * P.inV;
+                                    if (far) {
+                                        float* gc = gin + chan;
+                                        const S* ic = in + chan;
+                                        float vv[NC];
 #pragma unroll
-                                    for (int i = 0; i < NC; ++i) vv[i] = g1 * Store<S>::ld(ic[t.idx[i]]);
-                                    if constexpr (ND == 3) {
-                                        const float fl = t.f[0], gl = 1.f - fl, fh = t.f[1], gh = 1.f - fh, fw = t.f[2], gw = 1.f - fw;
-                                        const float cw[8] = {gl * gh * gw, gl * gh * fw, gl * fh * gw, gl * fh * fw, fl * gh * gw, fl * gh * fw, fl * fh * gw, fl * fh * fw};
-#pragma unroll
-                                        for (int i = 0; i < NC; ++i) atomic_add(gc + t.idx[i], cw[i] * g1);
-                                        const float c00 = vv[0] * gw + vv[1] * fw, c01 = vv[2] * gw + vv[3] * fw;
-                                        const float c10 = vv[4] * gw + vv[5] * fw, c11 = vv[6] * gw + vv[7] * fw;
-                                        ga[0] += (c10 - c00) * gh + (c11 - c01) * fh;
-                                        ga[1] += (c01 - c00) * gl + (c11 - c10) * fl;
-                                        ga[2] += ((vv[1] - vv[0]) * gh + (vv[3] - vv[2]) * fh) * gl + ((vv[5] - vv[4]) * gh + (vv[7] - vv[6]) * fh) * fl;
-                                    } else {
+                                        for (int i = 0; i < NC; ++i) vv[i] = g1 * Store<S>::ld(ic[t.idx[i]]);
                                         const float fh = t.f[0], gh = 1.f - fh, fw = t.f[1], gw = 1.f - fw;
                                         const float cw[4] = {gh * gw, gh * fw, fh * gw, fh * fw};
 #pragma unroll
                                         for (int i = 0; i < NC; ++i) atomic_add(gc + t.idx[i], cw[i] * g1);
                                         ga[0] += (vv[2] - vv[0]) * gw + (vv[3] - vv[1]) * fw;
                                         ga[1] += (vv[1] - vv[0]) * gh + (vv[3] - vv[2]) * fh;
+                                    }
+                                }
+                            } else {
+                                unsigned long long todo = __ballot(far);
+#pragma unroll 1
+                                while (todo) {                         // (a bit less each time)
+                                    const int src = __builtin_ctzll(todo), me = (int)here((unsigned)lane), i = me % NC, e = me / NC;
+                                    todo &= todo - 1;
+                                    auto from = [&](float v) { return __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(v), src)); };
+                                    float g1 = 0.f, wa[ND], d[ND];
+#pragma unroll
+                                    for (int x = 0; x < CCH; ++x) g1 = x == e ? from(gv[x]) : g1;
+                                    unsigned at = 0;
+#pragma unroll
+                                    for (int a = 0; a < ND; ++a) {     // the reference's corner rule on the same coordinate
+                                        const int size = P.in[slot<ND>(a)];
+                                        const float pa = from(pq[a]);
+                                        const int l = (int)pa, up = (i >> (ND - 1 - a)) & 1;
+                                        at = at * (unsigned)size + (unsigned)(l + (up && !(pa >= (float)(size - 1) || pa <= 0.f) ? 1 : 0));
+                                        wa[a] = up ? pa - (float)l : 1.f - (pa - (float)l);
+                                        d[a] = 0.f;
+                                    }
+                                    if (e < nch) {
+                                        const size_t to = ((size_t)n * P.C_in + cc0 + e) * P.inV + at;
+                                        const float v = g1 * Store<S>::ld(in[to]);
+                                        float cw = wa[0];
+#pragma unroll
+                                        for (int a = 1; a < ND; ++a) cw *= wa[a];
+                                        atomic_add(gin + to, cw * g1);
+#pragma unroll
+                                        for (int a = 0; a < ND; ++a) {
+                                            d[a] = (i >> (ND - 1 - a)) & 1 ? v : -v;
+#pragma unroll
+                                            for (int b = 0; b < ND; ++b)
+                                                if (b != a) d[a] *= wa[b];
+                                        }
+                                    }
+#pragma unroll
+                                    for (int a = 0; a < ND; ++a) {
+                                        d[a] = group_sum(d[a]);        // (its holders: the last lanes of either half)
+                                        const float sum = __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(d[a]), 31)) +
+                                                          __uint_as_float((unsigned)__builtin_amdgcn_readlane((int)__float_as_uint(d[a]), 63));
+                                        ga[a] += me == src ? sum : 0.f;
                                     }
                                 }
                             }

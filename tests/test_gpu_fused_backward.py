@@ -119,6 +119,32 @@ def test_small_weights(spec, w, gout):
         assert err <= tol
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("share", [0.002, 0.3], ids=["few", "many"])
+@pytest.mark.parametrize("spec", [(3, 1, 8, 16, (9, 12, 14), 3, 1, 1, 1, 8, 1, 1.0), (3, 2, 15, 20, (9, 17, 15), 3, 1, 1, 1, 5, 1, 1.0),
+                                  (3, 1, 17, 40, (10, 21, 19), 3, 2, 1, 1, 17, 1, 1.0), (3, 1, 4, 8, (9, 11, 12), 2, 1, 1, 1, 2, 1, 1.0),
+                                  (2, 1, 33, 48, (30, 34), 3, 1, 1, 1, 33, 1, 1.0), (2, 2, 12, 24, (26, 31), 3, 2, 1, 1, 6, 2, 1.0)],
+                         ids=lambda s: "%dd-%d-cpg%d" % (s[0], s[2], s[9]))
+def test_samples_past_the_halo(spec, share, dtype):
+    """Single samples, and most of a tap slot's, that reach past the halo, with full and short chunks of every width: grad_offset of those
+    samples by themselves (bounds as in test_edges), and grad_input."""
+    print("past the halo", spec, share, dtype, flush=True)
+    c = make_case(*spec, dtype=dtype, seed=36, bias=False)
+    g = torch.Generator().manual_seed(37)
+    far = torch.rand(c["off"].shape, generator=g) < share
+    wide = (torch.randint(0, 2, c["off"].shape, generator=g) * 2 - 1) * (7 + 2 * torch.rand(c["off"].shape, generator=g))
+    c["off"] = torch.where(far, wide.to(dtype), c["off"])
+    nd, taps = spec[0], spec[5] ** spec[0]
+    of_sample = far.view(spec[1], -1, taps, nd, *c["outs"]).any(3, keepdim=True).expand(-1, -1, -1, nd, *c["outs"]).reshape(far.shape)
+    once = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -9, torch.float16: 2.0 ** -12}[dtype]
+    (gin, goff), (win, woff) = _gradients(c), _oracle(c)
+    assert woff[of_sample].norm() > 0
+    for got, want, tol in ((gin, win, 1e-4), (goff[of_sample], woff[of_sample], 1e-5), (goff, woff, 1e-5)):
+        err = ((got - want).norm() / want.norm()).item()
+        print("  relative 2-norm error %.2e" % err, flush=True)
+        assert err <= tol + once
+
+
 def test_one_small_position_beside_ordinary_ones():
     """grad_offset of positions whose grad_output alone is tiny."""
     print("small position", flush=True)
