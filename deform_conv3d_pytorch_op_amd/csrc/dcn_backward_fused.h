@@ -125,10 +125,8 @@ template <int ND, int CCH> __host__ __device__ inline constexpr int fused_pt() {
 // LDS bytes per halo voxel: input cells (four float32 or eight 16-bit channels to 16 bytes) and the paired 32-bit sums
 template <typename S> inline size_t fused_voxel_bytes(int cch) { return (size_t)((cch + HaloCell<S>::CH - 1) / HaloCell<S>::CH) * 16 + (size_t)cch * 4; }
 
-// FULL: no chunk has fewer than CCH channels (3-D, where counting the real ones in the sum for samples outside the volume spills one
-// register more: steps of 64 -> 64, 3x3x3, 200 704 positions take 1.012 times as long, of 128 -> 128, stride 1 2 2, 100 352 positions 1.015).
 // Dynamic LDS = hstride * fused_voxel_bytes(CCH).  Work items, csplit, whole and goff_atomic: as at backward_input_halo_kernel.
-template <int ND, int CCH, int NPT, typename S, bool FULL = false>
+template <int ND, int CCH, int NPT, typename S>
 __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params P, PlanSet alts, const unsigned* __restrict__ sel, const S* __restrict__ in,
                                                                           const S* __restrict__ off, const typename Parts<S>::Vec* __restrict__ Wq,
                                                                           const S* __restrict__ W, const S* __restrict__ gout,
@@ -533,9 +531,9 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
                             if (__any(oor)) {
                                 float asum = 0.f;
                                 int real = nch;
-                                if constexpr (!FULL) asm volatile("" : "+s"(real));         // (compared here: hoisted, the comparisons spill seven more registers)
+                                asm volatile("" : "+s"(real));         // (compared here: hoisted, the comparisons spill scalar registers)
 #pragma unroll
-                                for (int e = 0; e < CCH; ++e) asum += FULL || e < real ? fabsf(gv[e]) : 0.f;
+                                for (int e = 0; e < CCH; ++e) asum += e < real ? fabsf(gv[e]) : 0.f;
                                 if (oor) {
 #pragma unroll
                                     for (int a = 0; a < ND; ++a) ga[a] = pq[a] <= -1.f ? -asum : (pq[a] >= (float)P.in[0] ? asum : 0.f);

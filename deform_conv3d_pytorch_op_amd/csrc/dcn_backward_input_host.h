@@ -4,13 +4,11 @@
 
 namespace dcn {
 
-// The instantiations of backward_fused_kernel: channels per chunk, position tiles per block, and whether every chunk is a full one.
+// The instantiations of backward_fused_kernel: channels per chunk and position tiles per block.
 template <int ND, typename S>
 using FusedKern = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const typename Parts<S>::Vec*, const S*, const S*, const typename Parts<S>::Vec*,
                            const float*, float*, float*, int, unsigned, int);
-template <int ND, typename S> inline FusedKern<ND, S> fused_kernel(int cch, int tiles, bool full) {
-    if constexpr (ND == 3)
-        if (full && cch == 8) return tiles == 4 ? backward_fused_kernel<3, 8, 4, S, true> : backward_fused_kernel<3, 8, 8, S, true>;
+template <int ND, typename S> inline FusedKern<ND, S> fused_kernel(int cch, int tiles) {
     if (tiles == 4) return cch == 8 ? backward_fused_kernel<ND, 8, 4, S> : cch == 4 ? backward_fused_kernel<ND, 4, 4, S> : nullptr;
     if constexpr (ND == 2)
         if (cch == 16) return backward_fused_kernel<2, 16, 8, S>;
@@ -69,7 +67,6 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
         const S* wt;
     };
     const int seg = P.cpg < P.Cg ? P.cpg : P.Cg;
-    auto full_chunks = [&](int cch) { return P.cpg % cch == 0 && P.Cg % cch == 0; };
     // Plans the fused kernel for a halo of margin m; false when none of its shapes fits.
     // (attempts: eight wavefronts on the default block, eight on the block shape with the smallest
     // halo, four on the block shape with the smallest halo)
@@ -117,7 +114,7 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
                     cch = cand;
                     nw = tiles;
                     lds = (size_t)Ph.hstride * vb;
-                    entry = reinterpret_cast<const void*>(fused_kernel<ND, S>(cand, tiles, full_chunks(cand)));
+                    entry = reinterpret_cast<const void*>(fused_kernel<ND, S>(cand, tiles));
                 }
             }
             if (split && !cch) continue;
@@ -365,7 +362,7 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             } else {
                 if constexpr (sizeof(T) == 4) {
                     typedef const typename Parts<S>::Vec* Ops;
-                    hipLaunchKernelGGL((fused_kernel<ND, S>(fp[k].cch, fp[k].nw, full_chunks(fp[k].cch))), grid, dim3(FUSED_WAVES * 64), lds, s, fp[k].Ph, alts, (const unsigned*)sel, in, off,
+                    hipLaunchKernelGGL((fused_kernel<ND, S>(fp[k].cch, fp[k].nw)), grid, dim3(FUSED_WAVES * 64), lds, s, fp[k].Ph, alts, (const unsigned*)sel, in, off,
                                        reinterpret_cast<Ops>(fp[k].wt), w, gout, reinterpret_cast<Ops>(gq), (const float*)bounds, gin, goff, fp[k].csplit,
                                        (unsigned)fp[k].whole, fp[k].goff_atomic);
                 }
