@@ -251,8 +251,10 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
         pc.nd = ND;
         pc.margin[0] = margins[0];
         pc.base[0] = 1.f;
-        pc.far_sample = ND == 3 ? 4.5f : 1.f;       // a sample beyond the halo scatters with global atomics
-        pc.far_steep = ND == 3 ? 25.f : 0.f;        // (64 -> 64 channels, 4 x 16 x 56 x 56, margin 2: 3.0, 4.1, 10.4, 26.6 times the time at 49, 70, 87.5, 96 % of the samples beyond the halo)
+        // A sample beyond the halo scatters with global atomics.  backward_fused_kernel, 64 -> 64 channels, 4 x 16 x 56 x 56, margin 2: 1.5, 2.1, 3.1, 13,
+        // 25 times the time at 25, 49, 70, 94, 98 % of the samples beyond the halo (offsets U[-r, r]; normal ones reach further: 1.2, 2.8 at 13, 45 %).
+        pc.far_sample = ND == 2 ? 1.f : fp[0].kern ? 4.5f : 2.f;
+        pc.far_steep = ND == 3 ? 25.f : 0.f;
         // 3-D: when most samples leave even the widest halo, the path without LDS tiling (coalesced
         // atomics on a channels-last copy; about 6.5 times the fused kernel's time on small offsets,
         // whatever the offsets) is the cheaper one: offered as a fourth choice, its kernels launched
@@ -273,14 +275,16 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
                 ++copies;
             }
             pc.margin[pc.nplans] = margins[k];
-            // Flush, staging and the per-chunk passes grow with the halo.  3-D: with its voxels per position r, as 1 + 0.068 r, a tenth more
-            // with narrower chunks (backward_fused_kernel, 64 -> 64 channels, 4 x 16 x 56 x 56: r = 7.7, 18 and 17.7 with 4-channel
-            // chunks at the margins 2, 3, 4 take 1, 1.46 and 1.60); the kernel with single cells as fitted when it served them all.
-            // Little in 2-D.
+            // Flush, staging and the per-chunk passes grow with the halo.  backward_fused_kernel in 3-D: with its voxels per position r, as
+            // 1 + 0.008 r, a fifth more with narrower chunks (64 -> 64 channels, 4 x 16 x 56 x 56: r = 7.7, 12 and 17.7, the latter two with
+            // 4-channel chunks, take 1, 1.35 and 1.36; in bfloat16 with 8-channel chunks at 12 1, 1.07 and 1.34).  With the costs above and the
+            // 6.5 below, over 8 layers under 17 distributions of offsets from U[-1.5, 1.5] to U[-10, 10] the chosen plan takes 1.025 times the best one's
+            // time on average; with 0.068 r, a tenth and 4.5, fitted to the loop over channels that far samples took before, 1.044.  The
+            // kernel with single cells as fitted when it served them all.  Little in 2-D.
             const Params &H0 = fp[0].Ph, &Hk = c.Ph;
             const float r0 = (float)H0.hvol / (float)(fp[0].nw * TN), rk = (float)Hk.hvol / (float)(c.nw * TN);
             if (ND == 3 && !c.kern && !fp[0].kern)
-                pc.base[pc.nplans] = (1.f + 0.068f * rk) / (1.f + 0.068f * r0) * (c.cch < fp[0].cch ? 1.1f : 1.f);
+                pc.base[pc.nplans] = (1.f + 0.008f * rk) / (1.f + 0.008f * r0) * (c.cch < fp[0].cch ? 1.2f : 1.f);
             else
                 pc.base[pc.nplans] = (1.f + (ND == 3 ? 0.9f : 0.05f) * ((float)Hk.hvol / (float)H0.hvol - 1.f)) * (c.nw < fp[0].nw ? 1.25f : 1.f);
             ++pc.nplans;
