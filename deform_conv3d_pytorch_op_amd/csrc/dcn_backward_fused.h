@@ -23,13 +23,13 @@
 // chunk's contraction and input loads go out before a chunk's flush, whose atomics they would otherwise wait for (64 -> 64
 // channels, 3x3x3, 200 704 positions: 1.41 -> 1.31 ms).
 // Against the eight wavefronts, grad_output in registers and float32 matrix instructions that float32 layers had before, ms per call of
-// backward_input_offset with its preparation: that layer 1.35 -> 1.35, in bfloat16 1.28 -> 1.11; 128 -> 128 in deformable groups of 32,
-// stride 1 2 2, 100 352 positions 2.91 -> 2.61, in bfloat16 2.26 -> 2.32; 2-D 256 -> 256, 25 088 positions 0.61 -> 0.43, in binary16
-// 0.65 (on widened tensors) -> 0.27; 512 -> 512 in two groups, 3136 positions 0.195 -> 0.145.  It pays for it with traffic: grad_output in
+// backward_input_offset with its preparation: that layer 1.34 -> 1.31, in bfloat16 1.29 -> 1.10; 128 -> 128 in deformable groups of 32,
+// stride 1 2 2, 100 352 positions 2.93 -> 2.49, in bfloat16 2.26 -> 2.09; 2-D 256 -> 256, 25 088 positions 0.61 -> 0.42, in binary16
+// 0.64 (on widened tensors) -> 0.23; 512 -> 512 in two groups, 3136 positions 0.193 -> 0.145.  It pays for it with traffic: grad_output in
 // operand order, half as much again as the tensor, is written once and read past the L2 by every block, for each chunk and as far as the
-// L2 lets go of it for each tile (2-D 256 -> 256 0.20 -> 0.84 GB a call, 64 -> 64 in 3-D 2.4 -> 4.7 GB).  Tried and slower or no faster: the weights of a step shared through the LDS (the wavefronts then multiply
-// together and scatter together), two workgroups of eight wavefronts per CU (2-D: 1 to 5 % faster on large layers, 13 % slower on
-// 3600 positions), two tiles to a contraction in 3-D.
+// L2 lets go of it for each tile (2-D 256 -> 256 0.20 -> 0.84 GB a call, 64 -> 64 in 3-D 2.4 -> 4.6 GB).  Tried and slower or no
+// faster: the weights of a step shared through the LDS (the wavefronts then multiply together and scatter together), two workgroups of
+// eight wavefronts per CU (2-D: 1 to 5 % faster on large layers, 13 % slower on 3600 positions), two tiles to a contraction in 3-D.
 #pragma once
 #include "dcn_forward_split.h"
 
