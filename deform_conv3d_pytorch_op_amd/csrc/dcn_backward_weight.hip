@@ -66,6 +66,8 @@ template <int ND, typename S>
 SplitFn<S> split_kernel(int MT, int LW, bool plain) {
     if constexpr (ND == 2 && sizeof(S) == 4)
         if (plain) return MT == 4 ? backward_weight_split_kernel<ND, 4, 32, S, true> : backward_weight_split_kernel<ND, 2, 32, S, true>;
+    if constexpr (sizeof(S) == 4)
+        if (MT == 8) return backward_weight_split_kernel<ND, 8, 32, S>;
     switch (MT * 100 + LW) {
         case 108: return backward_weight_split_kernel<ND, 1, 8, S>;
         case 116: return backward_weight_split_kernel<ND, 1, 16, S>;
@@ -108,10 +110,22 @@ SplitPlan split_plan(const Params& P, bool off, size_t room) {
     c.mchunks = ((P.M + 31) / 32 + c.MT - 1) / c.MT;
     c.igroups = (items + WAVES - 1) / WAVES;
     if ((P.M <= 32 && least > 0.67 * whole) || items < WAVES) return c;
-    const double resident = (double)resident_workgroups(reinterpret_cast<const void*>(split_kernel<ND, S>(c.MT, c.LW, false)), WG, 0);
+    double resident = (double)resident_workgroups(reinterpret_cast<const void*>(split_kernel<ND, S>(c.MT, c.LW, false)), WG, 0);
     const long long nslabs = (long long)P.N * (row_steps(P.outV) / 2);
-    const double other = (double)c.igroups * c.mchunks * P.G;
+    double other = (double)c.igroups * c.mchunks * P.G;
     if ((double)whole * c.mchunks * P.G * (double)nslabs < 2.5 * WAVES * resident) return c;
+    // Eight row tiles in float32 where they hold no more padding than fours do and leave work for the wavefronts that then fit (single taps and
+    // few channels: the corner reads are not what bounds them).
+    const int mtiles = (P.M + 31) / 32, fewer = (mtiles + 7) / 8;
+    if (sizeof(S) == 4 && off && c.LW == 32 && fewer * 8 == c.mchunks * 4) {
+        const double fit = (double)resident_workgroups(reinterpret_cast<const void*>(split_kernel<ND, S>(8, 32, false)), WG, 0);
+        if ((double)whole * fewer * P.G * (double)nslabs >= 2.5 * WAVES * fit) {
+            c.MT = 8;
+            c.mchunks = fewer;
+            resident = fit;
+            other = (double)c.igroups * fewer * P.G;
+        }
+    }
     const size_t one = (size_t)P.kV * P.C_out * P.Cg * sizeof(float);
     long long most = (long long)(room / one);
     if (most > 256) most = 256;

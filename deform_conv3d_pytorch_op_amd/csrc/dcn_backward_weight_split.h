@@ -31,6 +31,9 @@
 // 3x3, 8 x 56 x 56: 332 -> 240; 512 -> 512 in two groups, 3x3, 4 x 28 x 28: 105 -> 80; 128 -> 128, 3x3x3, 2 x 16 x 56 x 56
 // (stride 2): 1022 -> 860; 64 -> 64 as above: 633 -> 600; 64 -> 64, 3x3, no offsets, 25 088 positions: 33 -> 25.
 // The preparing launch pays 2 to 20 us of it back (three halves of the bytes of a channels-last copy).
+// float32 layers of more than 128 output channels to a group: eight row tiles, so that 256 of them share the corner reads of a sample, at two
+// wavefronts per SIMD instead of three: 256 -> 256 as above 228 -> 208 (steps of the layer 900 -> 889 us), 512 -> 512 in two groups 91 -> 80 (327 -> 323).  In 16-bit
+// storage a lane holds two column tiles and eight row tiles leave one wavefront per SIMD: steps of 256 -> 256 in binary16 497 -> 514 us, so it keeps four.
 // 16-bit storage, against backward_weight16_kernel, which samples once for every 64 output channels: 256 -> 256 in float16 150 -> 116,
 // 64 -> 64 in 3-D in bfloat16 361 -> 326.
 #pragma once
@@ -55,7 +58,7 @@ template <typename S> __device__ inline float channel_of(unsigned v, int u) {
 // MT row tiles to a workgroup.  LW lanes to a tap: an item is 32 / LW taps of LW channels (pairs).  PLAIN: a plain convolution (off is null): samples at integer coordinates are their low corner alone.
 // Grid: igroups * mchunks * G * nsplit workgroups.  The items of a convolution group: taps of a channel tile, taps fastest.
 template <int ND, int MT, int LW, typename S, bool PLAIN = false>
-__global__ __launch_bounds__(WG, (MT == 4 ? 3 : 4) - (sizeof(S) == 2)) void backward_weight_split_kernel(Params P, const S* __restrict__ in_cl, const S* __restrict__ off,
+__global__ __launch_bounds__(WG, MT == 8 ? 2 : (MT == 4 ? 3 : 4) - (sizeof(S) == 2)) void backward_weight_split_kernel(Params P, const S* __restrict__ in_cl, const S* __restrict__ off,
                                                                                          const S* __restrict__ gout,
                                                                                          const typename Parts<S>::Vec* __restrict__ rows,
                                                                                          float* __restrict__ partial, unsigned igroups) {

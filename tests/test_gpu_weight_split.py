@@ -20,6 +20,9 @@ LAYERS = [
     (2, 1, 16, 65, (161, 163), 3, 1, 1, 1, 16, 1, 1.5), (2, 2, 42, 130, (97, 73), 3, 1, 1, 1, 14, 1, 3.0), (2, 1, 48, 40, (145, 147), 3, 1, 1, 1, 48, 1, 1.0),
     (2, 1, 15, 20, (257, 259), 3, 2, 1, 1, 5, 1, 2.0), (2, 1, 8, 34, (229, 231), 5, 2, 2, 1, 8, 1, 9.0), (3, 1, 16, 20, (11, 32, 33), 3, 1, 1, 1, 4, 2, 1.5),
     (3, 1, 7, 66, (13, 39, 41), 3, 1, 1, 1, 7, 1, 2.5), (3, 1, 16, 33, (17, 33, 35), 3, 1, 1, 1, 16, 1, 2.5), (3, 1, 12, 40, (1, 131, 133), 3, 1, 1, 1, 3, 1, 1.0),
+    # eight row tiles (129 to 256 output channels to a group): their least and their most, two groups; nine tiles take chunks of four
+    (2, 1, 33, 129, (97, 101), 3, 1, 1, 1, 33, 1, 1.5), (2, 1, 40, 256, (97, 97), 3, 1, 1, 1, 40, 1, 2.5), (2, 1, 40, 420, (101, 99), 3, 1, 1, 1, 20, 2, 9.0),
+    (3, 1, 33, 161, (9, 21, 35), 3, 1, 1, 1, 33, 1, 1.5), (2, 1, 160, 250, (223, 225), 1, 1, 0, 1, 160, 1, 0.9), (2, 1, 33, 288, (97, 101), 3, 1, 1, 1, 33, 1, 1.5),
 ]
 IDS = lambda s: "%dd-%d-%d-k%d-g%d" % (s[0], s[2], s[3], s[5], s[10])
 
