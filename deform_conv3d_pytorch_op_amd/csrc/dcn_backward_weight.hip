@@ -62,22 +62,29 @@ inline int split_items(const Params& P, int TC, int TP) {
 // workgroups, as long as the tiles (written and read at about 8 TB/s) cost less than the longer runs of slabs.
 template <typename S> using RowOps = typename Parts<S>::Vec;
 template <typename S> using SplitFn = void (*)(Params, const S*, const S*, const S*, const RowOps<S>*, float*, unsigned);
-template <int ND, typename S>
-SplitFn<S> split_kernel(int MT, int LW, bool plain) {
+template <int ND, typename S, bool QUAD>
+SplitFn<S> split_kernel_of(int MT, int LW, bool plain) {
     if constexpr (ND == 2 && sizeof(S) == 4)
-        if (plain) return MT == 4 ? backward_weight_split_kernel<ND, 4, 32, S, true> : backward_weight_split_kernel<ND, 2, 32, S, true>;
+        if (plain) return MT == 4 ? backward_weight_split_kernel<ND, 4, 32, S, QUAD, true> : backward_weight_split_kernel<ND, 2, 32, S, QUAD, true>;
     if constexpr (sizeof(S) == 4)
-        if (MT == 8) return backward_weight_split_kernel<ND, 8, 32, S>;
+        if (MT == 8) return backward_weight_split_kernel<ND, 8, 32, S, QUAD>;
     switch (MT * 100 + LW) {
-        case 108: return backward_weight_split_kernel<ND, 1, 8, S>;
-        case 116: return backward_weight_split_kernel<ND, 1, 16, S>;
-        case 208: return backward_weight_split_kernel<ND, 2, 8, S>;
-        case 216: return backward_weight_split_kernel<ND, 2, 16, S>;
-        case 232: return backward_weight_split_kernel<ND, 2, 32, S>;
-        case 408: return backward_weight_split_kernel<ND, 4, 8, S>;
-        case 416: return backward_weight_split_kernel<ND, 4, 16, S>;
-        default: return backward_weight_split_kernel<ND, 4, 32, S>;
+        case 108: return backward_weight_split_kernel<ND, 1, 8, S, QUAD>;
+        case 116: return backward_weight_split_kernel<ND, 1, 16, S, QUAD>;
+        case 208: return backward_weight_split_kernel<ND, 2, 8, S, QUAD>;
+        case 216: return backward_weight_split_kernel<ND, 2, 16, S, QUAD>;
+        case 232: return backward_weight_split_kernel<ND, 2, 32, S, QUAD>;
+        case 408: return backward_weight_split_kernel<ND, 4, 8, S, QUAD>;
+        case 416: return backward_weight_split_kernel<ND, 4, 16, S, QUAD>;
+        default: return backward_weight_split_kernel<ND, 4, 32, S, QUAD>;
     }
+}
+// 16-byte loads where every lane's channels of a voxel are aligned to them, but not for float32 in 3-D (see the kernel).
+template <int ND, typename S>
+SplitFn<S> split_kernel(const Params& P, int MT, int LW, bool plain) {
+    constexpr int CL = 16 / sizeof(S);
+    if constexpr (ND == 3 && sizeof(S) == 4) return split_kernel_of<ND, S, false>(MT, LW, plain);
+    else return P.C_in % CL == 0 && P.cpg % CL == 0 && P.Cg % CL == 0 ? split_kernel_of<ND, S, true>(MT, LW, plain) : split_kernel_of<ND, S, false>(MT, LW, plain);
 }
 // Lanes to a tap: 16 or 8 where a segment fits them and that makes fewer items, at 1.05 and 1.2 items for one of 32: eight lanes read 32
 // bytes of a corner.  (Longer segments read their cache lines in parts then: 80 -> 96, 3-D, 23 600 positions 406 us a step with 32, 431 with 16.)  Layers of up to 32 output channels, too, if it takes a third off them; the
@@ -110,7 +117,7 @@ SplitPlan split_plan(const Params& P, bool off, size_t room) {
     c.mchunks = ((P.M + 31) / 32 + c.MT - 1) / c.MT;
     c.igroups = (items + WAVES - 1) / WAVES;
     if ((P.M <= 32 && least > 0.67 * whole) || items < WAVES) return c;
-    double resident = (double)resident_workgroups(reinterpret_cast<const void*>(split_kernel<ND, S>(c.MT, c.LW, false)), WG, 0);
+    double resident = (double)resident_workgroups(reinterpret_cast<const void*>(split_kernel<ND, S>(P, c.MT, c.LW, false)), WG, 0);
     const long long nslabs = (long long)P.N * (row_steps(P.outV) / 2);
     double other = (double)c.igroups * c.mchunks * P.G;
     if ((double)whole * c.mchunks * P.G * (double)nslabs < 2.5 * WAVES * resident) return c;
@@ -118,7 +125,7 @@ SplitPlan split_plan(const Params& P, bool off, size_t room) {
     // few channels: the corner reads are not what bounds them).
     const int mtiles = (P.M + 31) / 32, fewer = (mtiles + 7) / 8;
     if (sizeof(S) == 4 && off && c.LW == 32 && fewer * 8 == c.mchunks * 4) {
-        const double fit = (double)resident_workgroups(reinterpret_cast<const void*>(split_kernel<ND, S>(8, 32, false)), WG, 0);
+        const double fit = (double)resident_workgroups(reinterpret_cast<const void*>(split_kernel<ND, S>(P, 8, 32, false)), WG, 0);
         if ((double)whole * fewer * P.G * (double)nslabs >= 2.5 * WAVES * fit) {
             c.MT = 8;
             c.mchunks = fewer;
@@ -264,7 +271,7 @@ template <int ND, typename S>
 int launch_bwd_weight_split(const WeightCall<float, S>& c, const S* off, hipStream_t s) {
     const Params& P = c.P;
     const dim3 grid((unsigned)((long long)c.igroups * P.mchunks * P.G * P.nsplit));
-    hipLaunchKernelGGL((split_kernel<ND, S>(c.MT, c.LW, !off)), grid, dim3(WG), 0, s, P, (const S*)c.in_cl, off, c.gout, reinterpret_cast<const typename Parts<S>::Vec*>(c.gout_cl), c.partial, (unsigned)c.igroups);
+    hipLaunchKernelGGL((split_kernel<ND, S>(P, c.MT, c.LW, !off)), grid, dim3(WG), 0, s, P, (const S*)c.in_cl, off, c.gout, reinterpret_cast<const typename Parts<S>::Vec*>(c.gout_cl), c.partial, (unsigned)c.igroups);
     return check_launch("backward_weight_split_kernel");
 }
 

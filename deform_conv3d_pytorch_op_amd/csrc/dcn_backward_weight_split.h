@@ -34,6 +34,12 @@
 // float32 layers of more than 128 output channels to a group: eight row tiles, so that 256 of them share the corner reads of a sample, at two
 // wavefronts per SIMD instead of three: 256 -> 256 as above 228 -> 208 (steps of the layer 900 -> 889 us), 512 -> 512 in two groups 91 -> 80 (327 -> 323).  In 16-bit
 // storage a lane holds two column tiles and eight row tiles leave one wavefront per SIMD: steps of 256 -> 256 in binary16 497 -> 514 us, so it keeps four.
+// Where every lane's channels are aligned to it (QUAD), eight lanes read 16 bytes of a corner each and the wavefront eight positions at a time: a
+// quarter of the load instructions -- of a line or a half to a lane group, one that hits the L1 takes 7.5 ns a CU for 1 KB, of 4 bytes to a lane 2.9 for 256
+// bytes -- and of the records, and the weighted sums change places with the positions (swap_lanes_registers) before the
+// contraction.  2-D and 16-bit storage: us of the kernel alone, 4 bytes -> 16: 256 -> 256 in binary16 118 -> 95 (step 466 -> 433),
+// in float32 208 -> 193, 512 -> 512 in two groups 80 -> 77, without offsets 26.7 -> 23.7, 64 -> 64 in 3-D in bfloat16 333 -> 289 (step 1752 -> 1717).  Not float32 in 3-D, where the lines of eight positions with eight corners each, of every wavefront, turn the L1 over before their
+// neighbours come back to them: steps of 64 -> 64 2478 -> 2598 us, of 128 -> 128 4525 -> 5058.
 // 16-bit storage, against backward_weight16_kernel, which samples once for every 64 output channels: 256 -> 256 in float16 150 -> 116,
 // 64 -> 64 in 3-D in bfloat16 361 -> 326.
 #pragma once
@@ -48,17 +54,44 @@ template <typename S> inline size_t row_operand_bytes(int N, int C_out, size_t V
 // channels to a lane (16-bit storage: pairs, two column tiles)
 template <typename S> __host__ __device__ constexpr int lane_channels() { return 4 / (int)sizeof(S); }
 
+// wavefronts to a SIMD
+template <typename S> __host__ __device__ constexpr int split_waves(int MT) { return MT == 8 ? 2 : (MT == 4 ? 3 : 4) - (sizeof(S) == 2); }
+
 // channel u of what a lane reads of a corner
 template <typename S> __device__ inline float channel_of(float v, int) { return v; }
 template <typename S> __device__ inline float channel_of(unsigned v, int u) {
     if constexpr (std::is_same<S, Bf16>::value) return __uint_as_float(u ? v & 0xffff0000u : v << 16);
     else return (float)__builtin_bit_cast(_Float16, (unsigned short)(u ? v >> 16 : v));
 }
+typedef unsigned Quad __attribute__((ext_vector_type(4)));
+template <typename S> __device__ inline float channel_of(const Quad& v, int u) {
+    if constexpr (sizeof(S) == 4) return __uint_as_float(v[u]);
+    else return channel_of<S>(v[u / 2], u % 2);
+}
+
+// Where bit `lane bit 4` of a lane's number and one of the two registers trade places, then bit 3: registers v[k1 * 2 + k0] of lanes (.., p1, p0, ...)
+// become v[p1 * 2 + p0] of lanes (.., k1, k0, ...).
+__device__ inline void swap_lanes_registers(float v[4]) {
+    auto bits = [](float x) { return __float_as_uint(x); };
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const auto r = __builtin_amdgcn_permlane16_swap(bits(v[k]), bits(v[2 + k]), false, false);      // odd rows of the first with even rows of the second
+        v[k] = __uint_as_float(r[0]);
+        v[2 + k] = __uint_as_float(r[1]);
+    }
+#pragma unroll
+    for (int k = 0; k < 4; k += 2) {                    // row_ror:8, written to the upper eight lanes of a row or to the lower
+        const unsigned a = bits(v[k]), b = bits(v[k + 1]);
+        v[k] = __uint_as_float(__builtin_amdgcn_update_dpp(a, b, 0x128, 0xF, 0xC, false));
+        v[k + 1] = __uint_as_float(__builtin_amdgcn_update_dpp(b, a, 0x128, 0xF, 0x3, false));
+    }
+}
 
 // MT row tiles to a workgroup.  LW lanes to a tap: an item is 32 / LW taps of LW channels (pairs).  PLAIN: a plain convolution (off is null): samples at integer coordinates are their low corner alone.
 // Grid: igroups * mchunks * G * nsplit workgroups.  The items of a convolution group: taps of a channel tile, taps fastest.
-template <int ND, int MT, int LW, typename S, bool PLAIN = false>
-__global__ __launch_bounds__(WG, MT == 8 ? 2 : (MT == 4 ? 3 : 4) - (sizeof(S) == 2)) void backward_weight_split_kernel(Params P, const S* __restrict__ in_cl, const S* __restrict__ off,
+// QUAD: 16 bytes of a corner to a lane -- see the top of the file; channels and segments in multiples of four (16-bit storage: eight).
+template <int ND, int MT, int LW, typename S, bool QUAD, bool PLAIN = false>
+__global__ __launch_bounds__(WG, split_waves<S>(MT)) void backward_weight_split_kernel(Params P, const S* __restrict__ in_cl, const S* __restrict__ off,
                                                                                          const S* __restrict__ gout,
                                                                                          const typename Parts<S>::Vec* __restrict__ rows,
                                                                                          float* __restrict__ partial, unsigned igroups) {
@@ -81,7 +114,7 @@ __global__ __launch_bounds__(WG, MT == 8 ? 2 : (MT == 4 ? 3 : 4) - (sizeof(S) ==
     const int mchunk = wg % (unsigned)P.mchunks; wg /= (unsigned)P.mchunks;
     const int g = wg % (unsigned)P.G, split = wg / (unsigned)P.G;
     // the item's channel tile: segments are the intersections of the convolution group with deformable groups
-    const int tgroups = (P.kV + TP - 1) / TP, tap0 = item % tgroups * TP, ts = j / LW;      // ts: this lane's tap among them
+    const int tgroups = (P.kV + TP - 1) / TP, tap0 = item % tgroups * TP, ts = QUAD ? j % 8 / (LW / 4) : j / LW;      // ts: this lane's tap among them
     int z = item / tgroups, dg, c0 = 0, ce = 0;
     bool works = false;
     for (dg = g * P.Cg / P.cpg; dg <= ((g + 1) * P.Cg - 1) / P.cpg; ++dg) {
@@ -105,7 +138,10 @@ __global__ __launch_bounds__(WG, MT == 8 ? 2 : (MT == 4 ? 3 : 4) - (sizeof(S) ==
     }
 
     const int m_base = mchunk * MT * TN;
-    const unsigned cj = (unsigned)min(c0 + j % LW * CT, P.C_in - CT);      // clamped: lanes past the segment still load legally
+    constexpr int CL = QUAD ? 4 * CT : CT;                      // channels that a lane loads
+    const int cq = QUAD ? j % 8 % (LW / 4) : j % LW;
+    const unsigned cj = (unsigned)min(c0 + cq * CL, P.C_in - CL);          // clamped: lanes past the segment still load legally
+    auto column = [&](int u) { return QUAD ? cq * CL + u * 4 + j / 8 : cq * CT + u; };      // channel of this lane's column of tile u
     // 32-bit byte offsets from the sample's base (the host checks that a sample of either tensor stays below 4 GiB)
     const unsigned cjB = cj * (unsigned)sizeof(S), cinB = (unsigned)P.C_in * (unsigned)sizeof(S);
     unsigned strB[ND];                                          // from a corner to the next along an axis
@@ -226,17 +262,21 @@ __global__ __launch_bounds__(WG, MT == 8 ? 2 : (MT == 4 ? 3 : 4) - (sizeof(S) ==
                 if ((i >> (ND - 1 - a)) & 1) d += strB[a];
             corner[i] = in_n + d;
         }
-        // position by position; the next one's record and corner values are on their way while this one is added up
-        typedef typename std::conditional<CT == 1, T, unsigned>::type Word;
-        Word cn[NR];
-        T wn[NR];
+        // one position (QUAD: four of the lane group's eight, one to every eight lanes) after the other; the next one's record and corner values are
+        // on their way while this one is added up
+        constexpr int PB = QUAD ? 2 : 8;            // such turns to a step
+        constexpr int NB = QUAD && NR > 4 ? 4 : NR, HB = NR / NB;       // corners at a time, for the registers
+        typedef typename std::conditional<QUAD, Quad, typename std::conditional<CT == 1, T, unsigned>::type>::type Word;
+        Word cn[NB];
+        T wn[NB];
         auto fetch = [&](int k) {
-            const int pp = (k & 8) * 2 + q * 8 + (k & 7);          // position of the slab this lane group works on
+            const int h = k % HB, e = k / HB % PB;
+            const int pp = k / HB / PB * 16 + q * 8 + (QUAD ? e * 4 + j / 8 : e);          // position of the slab this lane works on
             const unsigned at = sIdx[wave][ts][pp] + cjB;
 #pragma unroll
-            for (int i = 0; i < NR; ++i) wn[i] = sCw[wave][ts][pp][i];
+            for (int i = 0; i < NB; ++i) wn[i] = sCw[wave][ts][pp][h * NB + i];
 #pragma unroll
-            for (int i = 0; i < NR; ++i) cn[i] = *reinterpret_cast<const Word*>(corner[i] + at);
+            for (int i = 0; i < NB; ++i) cn[i] = *reinterpret_cast<const Word*>(corner[h * NB + i] + at);
         };
         if (works) fetch(0);
 #pragma unroll
@@ -245,21 +285,30 @@ __global__ __launch_bounds__(WG, MT == 8 ? 2 : (MT == 4 ? 3 : 4) - (sizeof(S) ==
             if (works) {
                 float val[CT][8];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) {
-                    Word cc[NR];
-                    T wc[NR];
+                for (int e = 0; e < PB; ++e) {
 #pragma unroll
-                    for (int i = 0; i < NR; ++i) { cc[i] = cn[i]; wc[i] = wn[i]; }
-                    if (st * 8 + e + 1 < 16) fetch(st * 8 + e + 1);
-                    __builtin_amdgcn_sched_barrier(0);      // the next position's loads are issued before this one's arithmetic
+                    for (int h = 0; h < HB; ++h) {
+                        const int k = (st * PB + e) * HB + h;
+                        Word cc[NB];
+                        T wc[NB];
 #pragma unroll
-                    for (int u = 0; u < CT; ++u) {          // weighted corner sum, as the reference's sampler forms it
-                        T v = wc[0] * channel_of<S>(cc[0], u);
+                        for (int i = 0; i < NB; ++i) { cc[i] = cn[i]; wc[i] = wn[i]; }
+                        if (k + 1 < 2 * PB * HB) fetch(k + 1);
+                        __builtin_amdgcn_sched_barrier(0);      // the next loads are issued before this turn's arithmetic
+                        // weighted corner sum, as the reference's sampler forms it
 #pragma unroll
-                        for (int i = 1; i < NR; ++i) v += wc[i] * channel_of<S>(cc[i], u);
-                        val[u][e] = v;
+                        for (int u = 0; u < CL; ++u) {
+                            T& v = QUAD ? val[u / 4][e * 4 + u % 4] : val[u][e];
+                            v = h ? v + wc[0] * channel_of<S>(cc[0], u) : wc[0] * channel_of<S>(cc[0], u);
+#pragma unroll
+                            for (int i = 1; i < NB; ++i) v += wc[i] * channel_of<S>(cc[i], u);
+                        }
+                        __builtin_amdgcn_sched_barrier(0);
                     }
-                    __builtin_amdgcn_sched_barrier(0);
+                    if constexpr (QUAD) {
+#pragma unroll
+                        for (int u = 0; u < CT; ++u) swap_lanes_registers(val[u] + e * 4);
+                    }
                 }
                 // B[k = position][col = channel j]: weight 0 where there is no sample and past the end.  A row of A only reaches
                 // its own row of the tile and a column of B its own column, and rows past M / columns past the segment are not stored.
@@ -325,7 +374,7 @@ __global__ __launch_bounds__(WG, MT == 8 ? 2 : (MT == 4 ? 3 : 4) - (sizeof(S) ==
                     T w = 1.f;
 #pragma unroll
                     for (int a = 0; a < ND; ++a) w *= PLAIN ? 1.f : (i >> (ND - 1 - a)) & 1 ? t.f[a] : 1.f - t.f[a];
-                    v += w * Store<S>::ld(*reinterpret_cast<const S*>(in_n + (cb[i] + cjB + u * (unsigned)sizeof(S))));
+                    v += w * Store<S>::ld(*reinterpret_cast<const S*>(in_n + (cb[i] + (unsigned)min(c0 + column(u), P.C_in - 1) * (unsigned)sizeof(S))));
                 }
                 if constexpr (CT > 1) v = (T)(typename PT::Elem)v;         // rounded like the operand
                 const T b = live ? v : 0.f;
@@ -338,7 +387,7 @@ __global__ __launch_bounds__(WG, MT == 8 ? 2 : (MT == 4 ? 3 : 4) - (sizeof(S) ==
     };
 
     if (!works) return;                                 // (uniform for the wavefront)
-    T* pt = partial + ((size_t)split * P.kV + tap) * P.C_out * P.Cg + (size_t)g * P.M * P.Cg + (c0 + j % LW * CT - g * P.Cg);
+    T* pt = partial + ((size_t)split * P.kV + tap) * P.C_out * P.Cg + (size_t)g * P.M * P.Cg + (c0 - g * P.Cg);
 #pragma unroll
     for (int u = 0; u < CT; ++u)
 #pragma unroll
@@ -348,7 +397,7 @@ __global__ __launch_bounds__(WG, MT == 8 ? 2 : (MT == 4 ? 3 : 4) - (sizeof(S) ==
 #pragma unroll
         for (int r = 0; r < MM::NACC; ++r) {
             const int m = m_base + mt * TN + MM::row(r, q);
-            if (m < P.M && c0 + j % LW * CT + u < ce && tap < P.kV) pt[(size_t)m * P.Cg + u] = x[r];
+            if (m < P.M && c0 + column(u) < ce && tap < P.kV) pt[(size_t)m * P.Cg + column(u)] = x[r];
         }
     }
 }

@@ -23,6 +23,9 @@ LAYERS = [
     # eight row tiles (129 to 256 output channels to a group): their least and their most, two groups; nine tiles take chunks of four
     (2, 1, 33, 129, (97, 101), 3, 1, 1, 1, 33, 1, 1.5), (2, 1, 40, 256, (97, 97), 3, 1, 1, 1, 40, 1, 2.5), (2, 1, 40, 420, (101, 99), 3, 1, 1, 1, 20, 2, 9.0),
     (3, 1, 33, 161, (9, 21, 35), 3, 1, 1, 1, 33, 1, 1.5), (2, 1, 160, 250, (223, 225), 1, 1, 0, 1, 160, 1, 0.9), (2, 1, 33, 288, (97, 101), 3, 1, 1, 1, 33, 1, 1.5),
+    # 16 bytes of a corner to a lane: segments that end one lane into a tile, also two and four taps to an item; one over two convolution groups
+    (2, 1, 36, 70, (97, 161), 3, 1, 1, 1, 36, 1, 1.5), (2, 1, 40, 130, (161, 99), 3, 1, 1, 1, 40, 2, 3.0), (2, 1, 12, 65, (161, 163), 3, 1, 1, 1, 12, 1, 9.0),
+    (2, 1, 4, 66, (229, 231), 3, 1, 1, 1, 4, 1, 1.5), (2, 1, 68, 66, (1, 9001), 3, 1, 1, 1, 68, 1, 1.5),
 ]
 IDS = lambda s: "%dd-%d-%d-k%d-g%d" % (s[0], s[2], s[3], s[5], s[10])
 
@@ -64,6 +67,8 @@ LAYERS16 = [
     (2, 1, 24, 120, (141, 99), 3, 1, 1, 1, 8, 2, 2.0), (3, 1, 20, 64, (9, 32, 33), 3, 1, 1, 1, 10, 1, 1.5),
     (3, 1, 40, 97, (7, 31, 32), 3, 1, 1, 1, 40, 1, 2.5), (3, 1, 2, 60, (1, 95, 97), 3, 1, 1, 1, 2, 1, 1.0),
     (3, 1, 16, 30, (17, 33, 35), 3, 1, 1, 1, 16, 1, 2.5), (2, 1, 60, 64, (129, 161), 3, 1, 1, 1, 30, 1, 1.5), (2, 1, 24, 66, (129, 161), 3, 1, 1, 1, 24, 1, 1.5),
+    (2, 1, 72, 70, (129, 161), 3, 1, 1, 1, 72, 1, 1.5), (3, 1, 48, 64, (7, 31, 33), 3, 1, 1, 1, 24, 1, 2.5), (3, 1, 80, 64, (1, 95, 97), 3, 1, 1, 1, 80, 2, 1.0),
+    (2, 1, 16, 130, (129, 161), 3, 1, 1, 1, 16, 1, 9.0), (2, 1, 8, 66, (229, 231), 3, 1, 1, 1, 8, 1, 1.5),
 ]
 
 
