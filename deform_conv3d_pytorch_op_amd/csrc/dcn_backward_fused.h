@@ -50,34 +50,35 @@ template <typename S> inline size_t fused_gout_bytes(int N, int M, int G, size_t
 }
 
 // Weights: lane (q, j) of step k in tile t holds the parts of W[m = 16 * k + 8 * q + e][channel = first + fused_row_channel(j)]
-// [tap = t * 32 / CCH + fused_row_tap(j)], zero past M, the last tap and the segment.  One thread per lane and step.
+// [tap = t * 32 / CCH + fused_row_tap(j)], zero past M, the last tap and the segment.  A wavefront per tile and step.
 template <int CCH, typename S>
 __device__ inline void pack_fused_weight(const Params& P, const S* __restrict__ W, typename Parts<S>::Vec* __restrict__ Wq, unsigned block, unsigned blocks) {
     using PT = Parts<S>;
     constexpr int NP = PT::NP;
     const int steps = fused_steps(P.M), tiles = fused_tiles(P.kV, CCH);
-    const unsigned per_slab = (unsigned)(tiles * steps * 64);
-    const size_t total = (size_t)chunk_candidates<CCH>(P.cpg, P.Cg, P.C_in) * per_slab;
-    for (size_t i = (size_t)block * 256 + threadIdx.x; i < total; i += (size_t)blocks * 256) {
-        const int c0 = chunk_candidate<CCH>(P.cpg, P.Cg, (int)(i / per_slab));
-        const int seg_b = max(c0 / P.cpg * P.cpg, c0 / P.Cg * P.Cg);
+    const unsigned per_slab = (unsigned)(tiles * steps), total = (unsigned)chunk_candidates<CCH>(P.cpg, P.Cg, P.C_in) * per_slab;      // wavefronts
+    const int lane = threadIdx.x & 63, j = lane % 32;
+    for (unsigned w = (unsigned)__builtin_amdgcn_readfirstlane(block * 4 + (threadIdx.x >> 6)); w < total; w += blocks * 4) {      // uniform for a wavefront
+        const unsigned cand = w / per_slab, r = w - cand * per_slab;
+        const int c0 = chunk_candidate<CCH>(P.cpg, P.Cg, (int)cand);
+        const int g = c0 / P.Cg, dg = c0 / P.cpg, seg_b = max(dg * P.cpg, g * P.Cg), seg_e = min((dg + 1) * P.cpg, (g + 1) * P.Cg);
         if ((c0 - seg_b) % CCH) continue;
-        const int seg_e = min((c0 / P.cpg + 1) * P.cpg, (c0 / P.Cg + 1) * P.Cg);
-        const unsigned r = (unsigned)(i % per_slab);
-        const int lane = r % 64, k = (int)(r / 64) % steps, t = (int)(r / 64) / steps;
-        const int j = lane % 32, tap = t * (32 / CCH) + fused_row_tap<CCH>(j), c = c0 + fused_row_channel<CCH>(j), g = c0 / P.Cg;
+        const int t = (int)(r / (unsigned)steps), k = (int)r - t * steps;
+        const int tap = t * (32 / CCH) + fused_row_tap<CCH>(j), c = c0 + fused_row_channel<CCH>(j), m0 = k * 16 + lane / 32 * 8;
+        // (no load is masked: a masked one is waited for on its own)
+        const S* src = W + ((size_t)g * P.M * P.Cg + (min(c, seg_e - 1) - g * P.Cg)) * P.kV + min(tap, P.kV - 1);
+        S v[8];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = src[(size_t)min(m0 + e, P.M - 1) * P.Cg * P.kV];
         typename PT::Vec part[NP];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
-            const int m = k * 16 + lane / 32 * 8 + e;
-            S v = S();
-            if (m < P.M && tap < P.kV && c < seg_e) v = W[(((size_t)g * P.M + m) * P.Cg + (c - g * P.Cg)) * P.kV + tap];
             typename PT::Elem p[NP];
-            PT::split1(v, p);
+            PT::split1(m0 + e < P.M && tap < P.kV && c < seg_e ? v[e] : S(), p);
 #pragma unroll
             for (int x = 0; x < NP; ++x) part[x][e] = p[x];
         }
-        typename PT::Vec* dst = Wq + ((size_t)chunk_slot<CCH>(P.cpg, P.Cg, c0) * per_slab + (size_t)(t * steps + k) * 64) * NP + lane;
+        typename PT::Vec* dst = Wq + ((size_t)chunk_slot<CCH>(P.cpg, P.Cg, c0) * per_slab + r) * NP * 64 + lane;
 #pragma unroll
         for (int x = 0; x < NP; ++x) dst[x * 64] = part[x];
     }
@@ -92,18 +93,25 @@ __device__ inline void split_grad_output(const Params& P, const S* __restrict__ 
     const int steps = fused_steps(P.M);
     const size_t total = (size_t)P.N * P.G * steps * 2 * P.outV;
     for (size_t i = (size_t)block * 256 + threadIdx.x; i < total; i += (size_t)blocks * 256) {
-        const unsigned pos = (unsigned)(i % P.outV);
-        const size_t row = i / P.outV;                                  // (n, group, step, lane group)
-        const int q = (int)(row & 1), k = (int)((row >> 1) % steps);
-        const size_t ng = (row >> 1) / steps;                           // n * G + g
-        const S* src = gout + (ng * P.M + (size_t)(k * 16 + q * 8)) * P.outV + pos;
-        const int left = P.M - (k * 16 + q * 8);
-        S v[8];
+        unsigned pos;                                                   // of (n, group, step, lane group)
+        int q, k;
+        size_t ng;                                                      // n * G + g
+        auto decode = [&](auto at) {
+            const auto row = at / P.outV;
+            pos = (unsigned)(at - row * P.outV);
+            q = (int)(row & 1);
+            ng = (row >> 1) / (unsigned)steps;
+            k = (int)((row >> 1) - (decltype(at))ng * (unsigned)steps);
+        };
+        if (total <= ~0u) decode((unsigned)i);                          // (uniform; a 64-bit division is a hundred instructions)
+        else decode(i);
+        const int m0 = k * 16 + q * 8, left = P.M - m0;
+        const S* src = gout + ng * P.M * P.outV + pos;
+        S v[8];                                                         // (no load is masked: a masked one is waited for on its own)
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            v[e] = S();
-            if (e < left) v[e] = src[(size_t)e * P.outV];
-        }
+        for (int e = 0; e < 8; ++e) v[e] = src[(size_t)min(m0 + e, P.M - 1) * P.outV];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = e < left ? v[e] : S();
         typename PT::Vec part[NP];
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
@@ -133,6 +141,7 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
                                                                           const typename Parts<S>::Vec* __restrict__ gq, const float* __restrict__ bounds,
                                                                           float* __restrict__ gin, float* __restrict__ goff, int csplit, unsigned whole,
                                                                           int goff_atomic) {
+    touch_arguments<sizeof(Params) + sizeof(PlanSet) + 88>();
     HaloPlan H;
     if (!chosen_halo(P, alts, sel, H)) return;          // another launch runs the chosen plan
     using PS = Parts<S>;
@@ -165,8 +174,8 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
         item = whole + r / (unsigned)cs;
         cz = (int)(r % (unsigned)cs);
     }
-    const unsigned nt = (unsigned)P.N * P.tiles;
-    const int dg = item / nt;
+    const unsigned nt = (unsigned)P.N * (unsigned)P.tiles.d;
+    const int dg = (int)(item / nt);
     goff_atomic = cs > 1 ? 1 : goff_atomic;
 
     TileGeo<ND> tg;
@@ -182,7 +191,7 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
         for (int a = 0; a < ND; ++a) ib[a] = o[a] * P.stride[slot<ND>(a)] - P.pad[slot<ND>(a)];
     }
     const unsigned row = (unsigned)H.hext[2], plane = ND == 3 ? (unsigned)(H.hext[1] * H.hext[2]) : 0u;
-    const float inv2 = 1.f / (float)H.hext[2], inv1 = 1.f / (float)H.hext[1], invV = 1.f / (float)H.hvol;
+    const float inv2 = __builtin_amdgcn_rcpf((float)H.hext[2]), inv1 = __builtin_amdgcn_rcpf((float)H.hext[1]), invV = __builtin_amdgcn_rcpf((float)H.hvol);
 
     const int c_lo = dg * P.cpg, c_hi = c_lo + P.cpg;
     const S* off_dg = off + ((size_t)n * P.DG + dg) * P.kV * ND * P.outV;
@@ -247,7 +256,9 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
         }
     };
 
-    for (int g = c_lo / P.Cg; g <= (c_hi - 1) / P.Cg; ++g) {
+    const int g_last = (c_hi - 1) / P.Cg;
+#pragma unroll 1
+    for (int g = c_lo / P.Cg; g <= g_last; ++g) {
         const int rb = max(c_lo, g * P.Cg), re = min(c_hi, (g + 1) * P.Cg);
         const int chunks = (re - rb + CCH - 1) / CCH, mine = (cz - chunk_no % cs + cs) % cs;      // this workgroup's: mine, mine + cs, ...
         chunk_no += chunks;

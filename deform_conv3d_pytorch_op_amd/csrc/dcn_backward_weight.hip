@@ -198,9 +198,11 @@ int backward_weight_plan(const Params& Pin, const S* in, const S* off, const S* 
     if ((unsigned long long)P.inV * P.C_in * sizeof(S) >= (1ull << 32) || (unsigned long long)P.outV * P.C_out * sizeof(S) >= (1ull << 32))
         return refuse(DCN_E_ARGUMENT, "one sample of the input or of grad_output reaches 4 GiB");
     if constexpr (!S16) {
-        bww_plan<T>(P, c.MT, P.mchunks, P.nctiles, P.nsplit);
+        int mchunks;
+        bww_plan<T>(P, c.MT, mchunks, P.nctiles, P.nsplit);
         const long long resident = c.MT == 1 ? bww_resident<T, ND, 1>() : c.MT == 2 ? bww_resident<T, ND, 2>() : bww_resident<T, ND, 4>();
-        bww_plan<T>(P, c.MT, P.mchunks, P.nctiles, P.nsplit, resident);
+        bww_plan<T>(P, c.MT, mchunks, P.nctiles, P.nsplit, resident);
+        P.mchunks = mchunks;
         if ((long long)P.nsplit * P.kV * P.nctiles * P.mchunks > 0x7fffffffLL) return fail(DCN_E_ARGUMENT, "too many workgroups for one launch");
     } else {
         const int TN = Mma<float>::TN, CT = 2 * TN;

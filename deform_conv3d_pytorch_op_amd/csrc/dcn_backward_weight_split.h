@@ -102,6 +102,7 @@ __global__ __launch_bounds__(WG, split_waves<S>(MT)) void backward_weight_split_
     constexpr int CT = lane_channels<S>(), TC = LW * CT;        // channels of a lane, of a tap
     constexpr int TP = 32 / LW, GT = TP > 1 ? TP / 2 : 1;       // taps of an item, of a lane that works out geometry
     constexpr int TN = 32, NP = PT::NP, NC = 1 << ND, NR = PLAIN ? 1 : NC;     // corners, corners read
+    touch_arguments<sizeof(Params) + 40>();
     __shared__ unsigned sIdx[WAVES][TP][TN];                      // byte offset of the low corner's channel 0 inside the sample
     __shared__ __align__(16) T sCw[WAVES][TP][TN][NR];            // weight of each corner, 0 where there is no sample
     __shared__ __align__(16) unsigned char sRow[2][MT * NP * 1024];        // rows of a step of grad_output: [part][q][row]
@@ -111,8 +112,8 @@ __global__ __launch_bounds__(WG, split_waves<S>(MT)) void backward_weight_split_
     // XCD-contiguous order with the items fastest: the workgroups that gather around the same positions share an L2
     unsigned wg = xcd_contiguous(blockIdx.x, gridDim.x);
     const int item = (int)(wg % igroups) * WAVES + wave; wg /= igroups;
-    const int mchunk = wg % (unsigned)P.mchunks; wg /= (unsigned)P.mchunks;
-    const int g = wg % (unsigned)P.G, split = wg / (unsigned)P.G;
+    const int mchunk = wg % P.mchunks; wg /= P.mchunks;
+    const int g = wg % P.G, split = wg / P.G;
     // the item's channel tile: segments are the intersections of the convolution group with deformable groups
     const int tgroups = (P.kV + TP - 1) / TP, tap0 = item % tgroups * TP, ts = QUAD ? j % 8 / (LW / 4) : j / LW;      // ts: this lane's tap among them
     int z = item / tgroups, dg, c0 = 0, ce = 0;

@@ -108,7 +108,8 @@ __global__ __launch_bounds__(NW * 64, 1) void forward_quad_kernel(Params P, Plan
                                                            const T* __restrict__ in,
                                                            const T* __restrict__ off, const T* __restrict__ Wq,
                                                            const T* __restrict__ bias, T* __restrict__ out,
-                                                           T* __restrict__ part, int csplit, unsigned whole, TailSplit ts) {
+                                                           T* __restrict__ part, Div csplit, unsigned whole, TailSplit ts) {
+    touch_arguments<sizeof(Params) + sizeof(PlanSet) + 80>();
     HaloPlan H;
     if (!chosen_halo(P, alts, sel, H)) return;          // another launch runs the chosen plan
     using MM = Mma<T>;
@@ -124,31 +125,30 @@ __global__ __launch_bounds__(NW * 64, 1) void forward_quad_kernel(Params P, Plan
     unsigned wg, pslot = 0;                             // pslot: which partial sum of the split runs
     int cz = 0;
     int cch = H.cchunk;                                 // channels per LDS pass
-    const bool split = csplit > 1 && blockIdx.x >= whole;
-    if (!split) wg = xcd_contiguous(blockIdx.x, csplit > 1 ? whole : gridDim.x);
+    const bool split = csplit.d > 1 && blockIdx.x >= whole;
+    if (!split) wg = xcd_contiguous(blockIdx.x, csplit.d > 1 ? whole : gridDim.x);
     else {
         const unsigned rel = blockIdx.x - whole, all = gridDim.x - whole;
-        const unsigned wgsA = ts.splitB ? ts.unitsA * (unsigned)csplit : all;
+        const unsigned wgsA = ts.splitB.d ? ts.unitsA * (unsigned)csplit.d : all;
         if (rel < wgsA) {
             const unsigned r = xcd_contiguous(rel, wgsA);
-            wg = whole + r / (unsigned)csplit;
-            cz = r % (unsigned)csplit;
+            wg = whole + r / csplit;
+            cz = r % csplit;
             pslot = r;
         } else {
             const unsigned r = xcd_contiguous(rel - wgsA, all - wgsA);
             csplit = ts.splitB;
-            wg = whole + ts.unitsA + r / (unsigned)csplit;
-            cz = r % (unsigned)csplit;
+            wg = whole + ts.unitsA + r / csplit;
+            cz = r % csplit;
             pslot = wgsA + r;
             cch = min(cch, ts.cchB);
         }
     }
-    if (!split) csplit = 1;
-    const unsigned gm = wg % (unsigned)(P.G * P.mchunks);
-    const int g = gm / P.mchunks, mchunk = gm % P.mchunks;
+    const unsigned rest = wg / P.mchunks;
+    const int g = rest % P.G, mchunk = wg - rest * P.mchunks;
 
     TileGeo<ND> tg_;
-    tile_decode<ND>(P, H, wg / (unsigned)(P.G * P.mchunks), tg_);
+    tile_decode<ND>(P, H, rest / P.G, tg_);
     const int n = tg_.n;
     int o[ND];
     unsigned pos;
@@ -181,11 +181,14 @@ __global__ __launch_bounds__(NW * 64, 1) void forward_quad_kernel(Params P, Plan
     const int cg0 = g * P.Cg, cg1 = cg0 + P.Cg;
     int chunk_no = 0;
     if (threadIdx.x == 0) sNonFinite = 0;               // (stays set for the chunks that follow, see forward_split_kernel)
-    for (int dg = cg0 / P.cpg; dg <= (cg1 - 1) / P.cpg; ++dg) {
+    const int dg_last = (cg1 - 1) / P.cpg;
+#pragma unroll 1
+    for (int dg = cg0 / P.cpg; dg <= dg_last; ++dg) {
         const int cb = max(cg0, dg * P.cpg), ce = min(cg1, (dg + 1) * P.cpg);
         const T* off_dg = off + ((size_t)n * P.DG + dg) * P.kV * ND * P.outV;
         for (int cc0 = cb; cc0 < ce; cc0 += cch) {
-            if ((chunk_no++) % csplit != cz) continue;                     // another workgroup's chunk (uniform)
+            const int turn = chunk_no++;
+            if (split && turn % csplit != cz) continue;                     // another workgroup's chunk (uniform)
             const int nch = min(cch, ce - cc0);
             const int ngrp = (nch + FQ - 1) / FQ;
             const T* chan0 = in + ((size_t)n * P.C_in + cc0) * P.inV;      // workgroup-uniform
@@ -401,10 +404,10 @@ __global__ __launch_bounds__(NW * 64) void forward_join_tail_kernel(Params P, Pl
     if (threadIdx.x >= NW * TN) return;
     const unsigned unit = blockIdx.x / SLICES, ml0 = (blockIdx.x % SLICES) * JOIN_ROWS;
     const unsigned wg = whole + unit;
-    const unsigned gm = wg % (unsigned)(P.G * P.mchunks);
-    const int g = gm / P.mchunks, mchunk = gm % P.mchunks;
+    const unsigned rest = wg / P.mchunks;
+    const int g = rest % P.G, mchunk = wg - rest * P.mchunks;
     TileGeo<ND> tg_;
-    tile_decode<ND>(P, H, wg / (unsigned)(P.G * P.mchunks), tg_);
+    tile_decode<ND>(P, H, rest / P.G, tg_);
     int o[ND];
     unsigned pos;
     if (!tile_position<ND>(P, tg_, (int)threadIdx.x, o, pos)) return;

@@ -58,8 +58,9 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
     if (int rc = device_info(nullptr)) return rc;
     if constexpr (S16)
         if (!forward16_native<ND>(P)) { *declined = true; return DCN_OK; }
-    int MT;
-    fwd_weight_pad<T>(P.M, P.Cg, MT, P.mchunks, P.Mp, P.Cgp);
+    int MT, mchunks;
+    fwd_weight_pad<T>(P.M, P.Cg, MT, mchunks, P.Mp, P.Cgp);
+    P.mchunks = mchunks;
     if (!ws || (!S16 && ws_bytes < (size_t)P.G * P.kV * P.Mp * P.Cgp * sizeof(T))) return fail(DCN_E_WORKSPACE, "workspace too small");
     const int TN = Mma<T>::TN;
     // Too few position blocks to give every CU a workgroup.  First the input channels of a block are
@@ -206,7 +207,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
     // still leaves 8 channels per LDS pass, else one large one.  Returns the wavefronts per
     // workgroup, 0 when no halo of margin m fits.
     // channels per LDS pass: multiples of eight for forward_split_kernel, where they fit
-    auto plan_shape = [&](Params& Ph, size_t budget, int m, int waves, bool smallest, const int* blocks = nullptr) {
+    auto plan_shape = [&](Params& Ph, size_t budget, int m, int waves, bool smallest, const Div* blocks = nullptr) {
         if constexpr (MX)
             if (plan_halo<T, ND>(Ph, budget, m, 1 << 30, sizeof(S), waves, smallest, FG, blocks, 1, false)) return true;
         return !S16 && plan_halo<T, ND>(Ph, budget, m, MX ? 4 : 1 << 30, sizeof(T), waves, smallest, FQ, blocks, 1, !MX);
@@ -353,8 +354,8 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                 if (l > lds) lds = l;
             }
             const Params& Ph = plans[0];
-            using KernMx = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const WE*, const S*, const S*, S*, T*, int, unsigned, TailSplit);
-            using KernQuad = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const WE*, const S*, S*, T*, int, unsigned, TailSplit);
+            using KernMx = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const WE*, const S*, const S*, S*, T*, Div, unsigned, TailSplit);
+            using KernQuad = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const WE*, const S*, S*, T*, Div, unsigned, TailSplit);
             typename std::conditional<MX, KernMx, KernQuad>::type kern = nullptr;
             if constexpr (MX) {
                 if (pairs) kern = MT == 1 ? forward_split_kernel<ND, 1, 16, 2, S> : forward_split_kernel<ND, 2, 16, 2, S>;
@@ -382,7 +383,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             const long long units = (long long)Ph.N * Ph.tiles * Ph.G * Ph.mchunks;
             int tsplit = 1;
             long long whole = 0;
-            TailSplit ts = {0u, 0, 0};
+            TailSplit ts = {0u, Div(0), 0};
             if (fsplit == 1 && !tiny && forward_tail_split()) {
                 const long long slots = forward_slots() ? forward_slots() : resident_workgroups(reinterpret_cast<const void*>(kern), (pairs || tiny ? 16 : shared || small ? 8 : nw) * 64, lds);
                 const long long rest = units % slots;
@@ -417,7 +418,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                             const double t = (double)rounds * ta;
                             const size_t bytes = (size_t)rest * cs * per_wg;
                             if ((t < best || forward_tail_split() > 1) && bytes <= room && bytes <= FWD_PARTIAL_CAP) {
-                                best = t; tsplit = cs; ts = TailSplit{0u, 0, 0};
+                                best = t; tsplit = cs; ts = TailSplit{0u, Div(0), 0};
                             }
                         }
                         // two runs: nb units cs + 1 ways, the others cs ways, rounds * slots workgroups in all;
@@ -435,7 +436,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
                         const double t = ta + (double)(rounds - 1) * tb;
                         const size_t bytes = (size_t)(rounds * slots) * per_wg;
                         if (t < best && bytes <= room && bytes <= FWD_PARTIAL_CAP) {
-                            best = t; tsplit = cs; ts = TailSplit{(unsigned)(rest - nb), cs + 1, cchb};
+                            best = t; tsplit = cs; ts = TailSplit{(unsigned)(rest - nb), Div((int)cs + 1), cchb};
                         }
                     }
                     if (tsplit > 1) whole = units - rest;
@@ -448,7 +449,7 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             if (trace_plans()) {
                 fprintf(stderr, "dcn forward: %d position tiles, %d wavefronts, MT %d, grid %u (%lld unsplit, rest x %d), LDS %zu, every unit split x %d\n", nw,
                         pairs || tiny ? 16 : shared || small ? 8 : nw, MT, grid.x, tsplit > 1 ? whole : 0LL, tsplit, lds, fsplit);
-                if (ts.splitB) fprintf(stderr, "  of the rest: %u units x %d, the others x %d with %d channels per pass\n", ts.unitsA, tsplit, ts.splitB, ts.cchB);
+                if (ts.splitB) fprintf(stderr, "  of the rest: %u units x %d, the others x %d with %d channels per pass\n", ts.unitsA, tsplit, (int)ts.splitB, ts.cchB);
                 for (int k = 0; k < pc.nplans; ++k)
                     fprintf(stderr, "  plan %d: margin %d, halo %d x %d x %d, %d channels per pass, base cost %.3f\n", k, pc.margin[k],
                             plans[k].hext[0], plans[k].hext[1], plans[k].hext[2], plans[k].cchunk, pc.base[k]);
@@ -456,8 +457,8 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
             const unsigned* sel = pc.sel;
             const int threads = (pairs || tiny ? 16 : shared || small ? 8 : nw) * 64, splits = tsplit > 1 ? tsplit : fsplit;
             int rc;
-            if constexpr (MX) rc = launch_halo(kern, "forward halo kernel", grid, threads, lds, s, Ph, alts, sel, in, off, (const WE*)ws, w, bias, out, part, splits, (unsigned)whole, ts);
-            else rc = launch_halo(kern, "forward halo kernel", grid, threads, lds, s, Ph, alts, sel, in, off, (const WE*)ws, bias, out, part, splits, (unsigned)whole, ts);
+            if constexpr (MX) rc = launch_halo(kern, "forward halo kernel", grid, threads, lds, s, Ph, alts, sel, in, off, (const WE*)ws, w, bias, out, part, Div(splits), (unsigned)whole, ts);
+            else rc = launch_halo(kern, "forward halo kernel", grid, threads, lds, s, Ph, alts, sel, in, off, (const WE*)ws, bias, out, part, Div(splits), (unsigned)whole, ts);
             if (rc) return rc;
             if (fsplit == 1 && tsplit == 1) return DCN_OK;
             if (tsplit > 1) {

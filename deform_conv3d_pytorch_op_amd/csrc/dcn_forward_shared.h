@@ -28,8 +28,9 @@ template <int ND, int RT, typename S>
 __global__ __launch_bounds__(SHARED_WAVES * 64, 2) void forward_shared_kernel(Params P, PlanSet alts, const unsigned* __restrict__ sel,
                                                            const S* __restrict__ in, const S* __restrict__ off,
                                                            const typename Parts<S>::Elem* __restrict__ Wq, const S* __restrict__ W,
-                                                           const S* __restrict__ bias, S* __restrict__ out, float* __restrict__ part, int csplit,
+                                                           const S* __restrict__ bias, S* __restrict__ out, float* __restrict__ part, Div csplit,
                                                            unsigned whole, TailSplit ts) {
+    touch_arguments<sizeof(Params) + sizeof(PlanSet) + 96>();
     HaloPlan H;
     if (!chosen_halo(P, alts, sel, H)) return;          // another launch runs the chosen plan
     using PT = Parts<S>;
@@ -48,10 +49,10 @@ __global__ __launch_bounds__(SHARED_WAVES * 64, 2) void forward_shared_kernel(Pa
     const int rw = wave & 3, cwv = wave >> 2;           // this wavefront's row tiles and column tiles of the product
     const int ct = wave & 3, half = wave >> 2;          // what it samples: column tile, group of the phase
     const ForwardUnit U = forward_unit(H.cchunk, csplit, whole, ts);
-    const unsigned gm = U.wg % (unsigned)(P.G * P.mchunks);
-    const int g = gm / P.mchunks, mchunk = gm % P.mchunks;
+    const unsigned rest = U.wg / P.mchunks;
+    const int g = rest % P.G, mchunk = U.wg - rest * P.mchunks;
     TileGeo<ND> tg;
-    tile_decode<ND>(P, H, U.wg / (unsigned)(P.G * P.mchunks), tg);
+    tile_decode<ND>(P, H, rest / P.G, tg);
     const int n = tg.n;
     int ib[ND];
     unsigned pos;
@@ -76,11 +77,14 @@ __global__ __launch_bounds__(SHARED_WAVES * 64, 2) void forward_shared_kernel(Pa
 #pragma unroll
         for (int i = 0; i < CW * RW; ++i) acc[i] = acc_zero<float>();
         int chunk_no = 0;
-        for (int dg = cg0 / P.cpg; dg <= (cg1 - 1) / P.cpg; ++dg) {
+        const int dg_last = (cg1 - 1) / P.cpg;          // (in the loop's condition, with its loop unrolled, it sends the accumulators through scratch memory)
+#pragma unroll 1
+        for (int dg = cg0 / P.cpg; dg <= dg_last; ++dg) {
             const int cb = max(cg0, dg * P.cpg), ce = min(cg1, (dg + 1) * P.cpg);
             const S* off_dg = off + ((size_t)n * P.DG + dg) * P.kV * ND * P.outV;
             for (int cc0 = cb; cc0 < ce; cc0 += U.cch) {
-                if ((chunk_no++) % U.cs != U.cz) continue;                     // another workgroup's chunk (uniform)
+                const int turn = chunk_no++;
+                if (U.split && turn % U.cs != U.cz) continue;                  // another workgroup's chunk (uniform)
                 const int nch = min(U.cch, ce - cc0);
                 const int ngrp = (nch + FG - 1) / FG, npair = (ngrp + 1) / 2;
                 const S* chan0 = in + ((size_t)n * P.C_in + cc0) * P.inV;      // workgroup-uniform

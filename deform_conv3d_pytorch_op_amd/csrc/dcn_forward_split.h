@@ -128,11 +128,12 @@ template <typename S> __device__ inline S weight_at(const Params& P, const S* __
     return P.transposed ? W[(((size_t)g * P.Cg + cl) * P.M + m) * P.kV + (P.kV - 1 - tap)] : W[(((size_t)g * P.M + m) * P.Cg + cl) * P.kV + tap];
 }
 
-// One thread per operand of a lane.  With pc.sel set the launch has one block more, which chooses the
+// A wavefront per operand.  With pc.sel set the launch has one block more, which chooses the
 // halo plan from the offsets.
 template <typename S>
 __global__ __launch_bounds__(256) void pack_split_weight_kernel(Params P, const S* __restrict__ W, typename Parts<S>::Elem* __restrict__ Wq,
                                                                 PlanChoice pc, const S* __restrict__ off, size_t n_off) {
+    touch_arguments<sizeof(Params) + sizeof(PlanChoice) + 24>();
     using PT = Parts<S>;
     constexpr int TN = 32, NP = PT::NP;
     const unsigned pack_blocks = pc.sel ? gridDim.x - 1 : gridDim.x;
@@ -140,37 +141,37 @@ __global__ __launch_bounds__(256) void pack_split_weight_kernel(Params P, const 
         choose_plan(pc, off, n_off);
         return;
     }
-    const unsigned mtiles = P.Mp / TN, ntg = (P.kV + 1) / 2;
-    const unsigned per_slab = ntg * mtiles * 64;                                    // threads of a slab
-    const size_t total = (size_t)chunk_candidates<FG>(P.cpg, P.Cg, P.C_in) * per_slab;
-    for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < total; i += (size_t)pack_blocks * blockDim.x) {
-        const int c0 = chunk_candidate<FG>(P.cpg, P.Cg, (int)(i / per_slab));       // candidate first channel of a group
-        const int seg_b = max(c0 / P.cpg * P.cpg, c0 / P.Cg * P.Cg);
+    const unsigned mtiles = P.Mp / TN, ntg = (P.kV + 1) / 2, per_slab = ntg * mtiles;       // wavefronts of a slab
+    const unsigned total = (unsigned)chunk_candidates<FG>(P.cpg, P.Cg, P.C_in) * per_slab;
+    const unsigned lane = threadIdx.x & 63;
+    for (unsigned w = (unsigned)__builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6)); w < total; w += pack_blocks * 4) {      // uniform for a wavefront
+        const unsigned cand = w / per_slab, r = w - cand * per_slab;
+        const int c0 = chunk_candidate<FG>(P.cpg, P.Cg, (int)cand);                 // candidate first channel of a group
+        const int g = c0 / P.Cg, dg = c0 / P.cpg, seg_b = max(dg * P.cpg, g * P.Cg), seg_e = min((dg + 1) * P.cpg, (g + 1) * P.Cg);
         if ((c0 - seg_b) % FG) continue;
-        const int seg_e = min((c0 / P.cpg + 1) * P.cpg, (c0 / P.Cg + 1) * P.Cg);
-        unsigned r = (unsigned)(i % per_slab);
-        const int lane = r % 64; r /= 64;
-        const int tile = (int)(r % mtiles), tg = (int)(r / mtiles);
-        const int m = tile * TN + lane % TN, tap = tg * 2 + lane / TN, g = c0 / P.Cg;
+        const int tg = (int)(r / mtiles), tile = (int)r - tg * (int)mtiles;
+        const int m = tile * TN + lane % TN, tap = tg * 2 + lane / TN;
+        // (no load is masked: a masked one is waited for on its own)
+        S v[FG];
+#pragma unroll
+        for (int e = 0; e < FG; ++e) v[e] = weight_at<S>(P, W, g, min(m, P.M - 1), (size_t)(min(c0 + e, seg_e - 1) - g * P.Cg), min(tap, P.kV - 1));
         typename PT::Vec part[NP];
 #pragma unroll
         for (int e = 0; e < FG; ++e) {
-            S v = S();
-            if (m < P.M && tap < P.kV && c0 + e < seg_e) v = weight_at<S>(P, W, g, m, (size_t)(c0 + e - g * P.Cg), tap);
             typename PT::Elem p[NP];
-            PT::split1(v, p);
+            PT::split1(m < P.M && tap < P.kV && c0 + e < seg_e ? v[e] : S(), p);
 #pragma unroll
             for (int k = 0; k < NP; ++k) part[k][e] = p[k];
         }
-        typename PT::Vec* dst = reinterpret_cast<typename PT::Vec*>(Wq) + (size_t)chunk_slot<FG>(P.cpg, P.Cg, c0) * per_slab * NP +
-                                ((size_t)tg * mtiles + tile) * NP * 64 + lane;
+        typename PT::Vec* dst = reinterpret_cast<typename PT::Vec*>(Wq) + ((size_t)chunk_slot<FG>(P.cpg, P.Cg, c0) * per_slab + r) * NP * 64 + lane;
 #pragma unroll
         for (int k = 0; k < NP; ++k) dst[k * 64] = part[k];
     }
 }
 
 // Offset of halo voxel v inside a channel of the input, ~0u outside the volume.  The two divisions
-// are float multiplications: exact for the few thousand voxels of a halo.
+// are float multiplications by a reciprocal: half a voxel of slack is far more than their rounding for the few
+// thousand voxels of a halo.
 template <int ND>
 __device__ inline unsigned halo_voxel(const Params& P, const HaloPlan& H, const TileGeo<ND>& tg, int v, float inv1, float inv2) {
     const int r = (int)(((float)v + 0.5f) * inv2);
@@ -199,24 +200,26 @@ __device__ inline unsigned halo_voxel(const Params& P, const HaloPlan& H, const 
 struct ForwardUnit {
     unsigned wg;                // unit
     unsigned pslot;             // which partial sum of the split runs
-    int cz, cs;                 // this workgroup takes every cs-th channel pass, from the cz-th on
+    int cz;                     // this workgroup takes every cs-th channel pass, from the cz-th on
+    Div cs;
     int cch;                    // channels per LDS pass
     bool split;
 };
-__device__ inline ForwardUnit forward_unit(int cchunk, int csplit, unsigned whole, const TailSplit& ts) {
+__device__ inline ForwardUnit forward_unit(int cchunk, const Div& csplit, unsigned whole, const TailSplit& ts) {
     ForwardUnit u;
     u.pslot = 0;
     u.cz = 0;
     u.cs = csplit;
     u.cch = cchunk;
-    u.split = csplit > 1 && blockIdx.x >= whole;
+    u.split = csplit.d > 1 && blockIdx.x >= whole;
     if (!u.split) {
-        u.wg = xcd_contiguous(blockIdx.x, csplit > 1 ? whole : gridDim.x);
-        u.cs = 1;
+        u.wg = xcd_contiguous(blockIdx.x, csplit.d > 1 ? whole : gridDim.x);
+        u.cs = Div{};                                      // (not divided by: one workgroup takes every pass)
+        u.cs.d = 1;
         return u;
     }
     const unsigned rel = blockIdx.x - whole, all = gridDim.x - whole;
-    const unsigned wgsA = ts.splitB ? ts.unitsA * (unsigned)csplit : all;
+    const unsigned wgsA = ts.splitB.d ? ts.unitsA * (unsigned)csplit.d : all;
     unsigned first = whole, r;
     if (rel < wgsA) {
         r = xcd_contiguous(rel, wgsA);
@@ -228,8 +231,9 @@ __device__ inline ForwardUnit forward_unit(int cchunk, int csplit, unsigned whol
         u.pslot = wgsA + r;
         u.cch = min(cchunk, ts.cchB);
     }
-    u.wg = first + r / (unsigned)u.cs;
-    u.cz = (int)(r % (unsigned)u.cs);
+    const unsigned unit = r / u.cs;
+    u.wg = first + unit;
+    u.cz = (int)(r - unit * (unsigned)u.cs.d);
     return u;
 }
 
@@ -251,7 +255,7 @@ __device__ inline bool stage_halo(const Params& P, const HaloPlan& H, const Tile
     constexpr int CH = HaloCell<S>::CH;
     // an item is a cell: consecutive threads take consecutive voxels, several items of a thread are in flight
     const int items = (nch + CH - 1) / CH * H.hvol;
-    const float inv2 = 1.f / (float)H.hext[2], inv1 = 1.f / (float)H.hext[1], inv = 1.f / (float)H.hvol;
+    const float inv2 = __builtin_amdgcn_rcpf((float)H.hext[2]), inv1 = __builtin_amdgcn_rcpf((float)H.hext[1]), inv = __builtin_amdgcn_rcpf((float)H.hvol);
     const size_t step = (size_t)P.inV * sizeof(S);
     bool bad = false;
     auto stage = [&](int it, auto full_tag) {
@@ -528,8 +532,9 @@ template <int ND, int MT, int NW, int TS, typename S>
 __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel(Params P, PlanSet alts, const unsigned* __restrict__ sel,
                                                            const S* __restrict__ in, const S* __restrict__ off,
                                                            const typename Parts<S>::Elem* __restrict__ Wq, const S* __restrict__ W,
-                                                           const S* __restrict__ bias, S* __restrict__ out, float* __restrict__ part, int csplit,
+                                                           const S* __restrict__ bias, S* __restrict__ out, float* __restrict__ part, Div csplit,
                                                            unsigned whole, TailSplit ts) {
+    touch_arguments<sizeof(Params) + sizeof(PlanSet) + 96>();
     HaloPlan H;
     if (!chosen_halo(P, alts, sel, H)) return;          // another launch runs the chosen plan
     using PT = Parts<S>;
@@ -545,11 +550,11 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
     const int lane = threadIdx.x & 63, wave = TS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : threadIdx.x >> 6;
     const int j = lane % TN, q = lane / TN;
     const ForwardUnit U = forward_unit(H.cchunk, csplit, whole, ts);
-    const unsigned gm = U.wg % (unsigned)(P.G * P.mchunks);
-    const int g = gm / P.mchunks, mchunk = gm % P.mchunks;
+    const unsigned rest = U.wg / P.mchunks;
+    const int g = rest % P.G, mchunk = U.wg - rest * P.mchunks;
 
     TileGeo<ND> tg;
-    tile_decode<ND>(P, H, U.wg / (unsigned)(P.G * P.mchunks), tg);
+    tile_decode<ND>(P, H, rest / P.G, tg);
     const int n = tg.n;
     int ib[ND];
     unsigned pos;
@@ -580,17 +585,22 @@ __global__ __launch_bounds__(NW * 64, MT <= 2 ? 4 : 2) void forward_split_kernel
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[mt] = acc_zero<float>();
         int chunk_no = 0;
-        for (int dg = cg0 / P.cpg; dg <= (cg1 - 1) / P.cpg; ++dg) {
+        const int dg_last = (cg1 - 1) / P.cpg;          // (in the loop's condition, with its loop unrolled, it sends the accumulators through scratch memory)
+#pragma unroll 1
+        for (int dg = cg0 / P.cpg; dg <= dg_last; ++dg) {
             const int cb = max(cg0, dg * P.cpg), ce = min(cg1, (dg + 1) * P.cpg);
             const S* off_dg = off + ((size_t)n * P.DG + dg) * P.kV * ND * P.outV;
             for (int cc0 = cb; cc0 < ce; cc0 += U.cch) {
-                if ((chunk_no++) % U.cs != U.cz) continue;                     // another workgroup's chunk (uniform)
+                const int turn = chunk_no++;
+                if (U.split && turn % U.cs != U.cz) continue;                  // another workgroup's chunk (uniform)
                 const int nch = min(U.cch, ce - cc0);
                 const int ngrp = (nch + FG - 1) / FG;
                 const S* chan0 = in + ((size_t)n * P.C_in + cc0) * P.inV;      // workgroup-uniform
                 // this wavefront's steps of the pass: [first, last) of the (tap pair, group) list
                 const int steps = ntg * ngrp, first = TS > 1 ? steps * (wave % TS) / TS : 0, last = TS > 1 ? steps * (wave % TS + 1) / TS : steps;
-                const int tg_first = TS > 1 ? __builtin_amdgcn_readfirstlane(first / ngrp) : 0, tg_end = TS > 1 ? __builtin_amdgcn_readfirstlane((last + ngrp - 1) / ngrp) : ntg;
+                const float per = __builtin_amdgcn_rcpf((float)ngrp);                 // (floor((x + 0.5) / ngrp) for the few thousand steps of a pass)
+                const int tg_first = TS > 1 ? __builtin_amdgcn_readfirstlane((int)(((float)first + 0.5f) * per)) : 0;
+                const int tg_end = TS > 1 ? __builtin_amdgcn_readfirstlane((int)(((float)(last + ngrp - 1) + 0.5f) * per)) : ntg;
                 float ofs[ND];
                 load_pair_offsets<ND, S>(P, off_dg, min(tg_first, ntg - 1), q, pos, ofs, off == nullptr);
                 __syncthreads();                                               // readers of the previous chunk are done

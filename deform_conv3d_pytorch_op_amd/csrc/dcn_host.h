@@ -463,7 +463,7 @@ static int forced_csplit() {    // DCN_CSPLIT=n: workgroups per (tile, deformabl
 
 template <typename T, int ND>
 inline bool plan_halo(Params& P, size_t budget, int m, int max_chunk = 1 << 30, size_t cell_bytes = sizeof(T), int waves = WAVESH,
-               bool smallest_halo = false, int chunk_mult = 0, const int* blocks = nullptr, int wmult = 1, bool table = true) {
+               bool smallest_halo = false, int chunk_mult = 0, const Div* blocks = nullptr, int wmult = 1, bool table = true) {
     const int npos = waves * Mma<T>::TN;        // positions per workgroup, one column tile per wavefront
     int td[3] = {1, 1, 1};
     if (ND == 3) { td[1] = td[2] = npos >= 64 ? 8 : 4; td[0] = npos / (td[1] * td[2]); }

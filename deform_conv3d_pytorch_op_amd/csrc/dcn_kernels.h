@@ -107,8 +107,8 @@ __global__ void relayout_weight_kernel(Params P, const T* __restrict__ W, T* __r
 // A chunk that starts at channel c0 owns slab chunk_slot(c0): increasing in c0, by at least one per
 // chunk (c0 / CCH steps within a segment, one of the other terms at every segment start), so no two
 // chunks share a slab; some slabs stay unused.
-template <int CCH>
-__host__ __device__ inline int chunk_slot(int cpg, int Cg, int c0) { return c0 / CCH + c0 / cpg + c0 / Cg; }
+template <int CCH, typename D>
+__host__ __device__ inline int chunk_slot(const D& cpg, const D& Cg, int c0) { return c0 / CCH + c0 / cpg + c0 / Cg; }
 // The pack kernels walk over candidate chunk starts.  Where one of cpg and Cg divides the other
 // (nearly every layer) the segments all have the length of the smaller and the y-th chunk start
 // is known in closed form; otherwise every channel is a candidate and non-starts are skipped.
@@ -356,8 +356,8 @@ struct TileGeo {
 
 template <int ND>
 __device__ inline void tile_decode(const Params& P, const HaloPlan& H, unsigned bid, TileGeo<ND>& tg) {
-    unsigned t = bid % (unsigned)P.tiles;
-    tg.n = bid / (unsigned)P.tiles;
+    tg.n = (int)(bid / P.tiles);
+    unsigned t = bid - (unsigned)tg.n * (unsigned)P.tiles;
 #pragma unroll
     for (int a = ND - 1; a >= 0; --a) {
         const int s = slot<ND>(a);

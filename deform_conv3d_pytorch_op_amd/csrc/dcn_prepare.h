@@ -182,6 +182,7 @@ __device__ inline void prep_rows(const PrepJob& job, unsigned block) {
 template <typename T, typename S>
 __global__ __launch_bounds__(256) void backward_prepare_kernel(Params P, PlanChoice pc, PrepJobs jobs, const S* __restrict__ W,
                                                                const S* __restrict__ off, size_t n_off) {
+    touch_arguments<sizeof(Params) + sizeof(PlanChoice) + sizeof(PrepJobs) + 16>();
     // this block's job (selected field by field from constant argument offsets: a dynamic index would
     // put the whole list into scratch memory)
     PrepJob job = jobs.job[0];

@@ -93,6 +93,18 @@ int main(int argc, char** argv) {
         prep.add(PREP_PLAN, 1);
         return ok && prep.full && prep.jobs.n == MAX_PREP ? 0 : 1;
     }
+    if (what == "div") {            // what the device does with a Div is a division: up to 2^31, around multiples of every small divisor and of random ones
+        auto divides = [](int d, unsigned n) {
+            const Div D(d);
+            return (((unsigned)((unsigned long long)D.m * n >> 32) + n) >> D.l) == n / (unsigned)d;
+        };
+        for (int i = 0; i < 1000 * atoi(argv[3]); ++i) {
+            const int d = i < 5000 ? i + 1 : (int)(rng() % (i & 1 ? 0x7fffffffu : 100000u)) + 1;
+            const unsigned n = rng() & 0x7fffffffu, m = n / d * d;
+            if (!divides(d, n) || !divides(d, m) || (m && !divides(d, m - 1)) || !divides(d, 0) || !divides(d, 0x7fffffffu)) return printf("%u / %d\n", n, d), 1;
+        }
+        return 0;
+    }
     if (what == "budget") {         // of any DCN_SCATTER_BUDGET_KB: what a CU has beside the 2120 and 100 bytes that the kernels declare; 72 stays 72
         const size_t cu = 160 * 1024, kb72 = 72 * 1024;
         return fused_budget() + 2120 <= cu && scatter_budget() + 100 <= cu && fused_budget() >= kb72 && scatter_budget() >= kb72 &&
@@ -107,8 +119,8 @@ int main(int argc, char** argv) {
         ++layers;
         const bool ok = what == "noalloc" ? noalloc(P, hits) : what == "layout" ? layouts(P, hits) : what == "weight64" ? weight64(P, hits) : what == "native16" ? (nd == 3 ? native16<3>(P, hits) : native16<2>(P, hits)) : false;
         if (!ok) {
-            printf("%s: %d-D, C_in %d, C_out %d, G %d, cpg %d, k %d %d %d, stride %d %d %d, dil %d %d %d\n", what.c_str(), nd, P.C_in, P.C_out, P.G, P.cpg, P.k[0],
-                   P.k[1], P.k[2], P.stride[0], P.stride[1], P.stride[2], P.dil[0], P.dil[1], P.dil[2]);
+            printf("%s: %d-D, C_in %d, C_out %d, G %d, cpg %d, k %d %d %d, stride %d %d %d, dil %d %d %d\n", what.c_str(), nd, P.C_in, P.C_out, (int)P.G, (int)P.cpg, (int)P.k[0],
+                   (int)P.k[1], (int)P.k[2], P.stride[0], P.stride[1], P.stride[2], P.dil[0], P.dil[1], P.dil[2]);
             return 1;
         }
     }

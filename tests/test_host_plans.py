@@ -22,6 +22,11 @@ def test_rule(probe, what):
     assert r.returncode == 0, r.stdout
 
 
+def test_divisors(probe):
+    r = subprocess.run([probe, "div", "7", "2000"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
+
+
 @pytest.mark.parametrize("kb", [None, "72", "156", "158", "160", "100000"])
 def test_lds_budget(probe, kb):
     """A budget past what a workgroup can have is that: its plans launch."""
