@@ -34,6 +34,40 @@ inline int even_chunk(const Params& P, int cchunk, int step, int fsplit) {
     return cchunk;
 }
 
+// The plain convolution on a kernel of its own; *done says whether it took the layer.
+inline int plain_forward(Params P, const float* in, const float* w, const float* bias, float* out, void* ws, size_t ws_bytes, hipStream_t s, bool* done) {
+    *done = false;
+    const int mtiles = (P.M + 31) / 32;
+    int mw = mtiles > 2 ? 4 : mtiles, rw = mtiles > 4 ? 2 : 1;
+    P.mchunks = (mtiles + mw * rw - 1) / (mw * rw);
+    P.Mp = P.mchunks * mw * rw * 32;
+    if (!plan_halo<float, 2>(P, (size_t)1 << 30, 0, 64, 1, PLAIN_COLS, false, FG, nullptr, 1, false)) return DCN_OK;
+    // Channels at a time: two workgroups to a CU.
+    while (P.cchunk > FG && plain_lds(P.hvol, P.cchunk) > MAX_FORWARD_LDS / 2) P.cchunk -= FG;
+    const size_t lds = plain_lds(P.hvol, P.cchunk);
+    const long long wgs = (long long)P.N * P.tiles * P.G * P.mchunks;
+    if (lds > MAX_FORWARD_LDS || ws_bytes < split_weight_bytes<float>(P, P.Mp) || wgs > 0x7fffffffLL || !plain_conv()) return DCN_OK;
+    // A wavefront takes some 0.26 us to a step of sixteen reduction slots, whatever the others do: long chains want enough wavefronts for the
+    // device, short ones three to four CUs.  Others keep the kernels that share a position or its channels among wavefronts.  us of
+    // the forward call, those kernels : this one, 43 layers: with fewer than 1400 wavefronts and more than 40 steps -- 512 -> 32, 3x3, 25 x 24 x 24 (450,
+    // 320 steps) 68 : 118; 128 -> 128, 28 x 28, four samples (512, 80) 30 : 39; 256 -> 64, 56 x 56, four (784, 160) 55 : 61 --, above either line 64 -> 64,
+    // 56 x 56 (196, 40) 21.9 : 20.4; 16 -> 128, 40 x 40, two (400, 10) 20.3 : 13.8; 256 -> 128, 28 x 28, sixteen (2048, 160) 108 : 79; 100 -> 100, 5x5, 60 x 60,
+    // four (2048, 169) 139 : 77; at worst 11.3 : 12.7 (24 -> 24, 60 x 60, two samples).
+    const int steps = (P.Cg + FG - 1) / FG * ((P.kV + 1) / 2);
+    const long long waves = wgs * PLAIN_COLS * mw;
+    if (plain_conv() != 2 && waves * 2 < 11 * cu_count() && (steps > 40 || waves * 4 < 3 * cu_count())) return DCN_OK;
+    *done = true;
+    const unsigned items = (unsigned)chunk_candidates<FG>(P.cpg, P.Cg, P.C_in) * (unsigned)((P.kV + 1) / 2) * (unsigned)(P.Mp / 32), blocks = (items + 3) / 4;
+    const PlanChoice none = {};
+    hipLaunchKernelGGL(pack_split_weight_kernel<float>, dim3(blocks > 8192 ? 8192 : blocks), dim3(256), 0, s, P, w, static_cast<Parts<float>::Elem*>(ws), none,
+                       static_cast<const float*>(nullptr), (size_t)0);
+    if (int rc = check_launch("forward weight packing")) return rc;
+    if (trace_plans())
+        fprintf(stderr, "dcn plain convolution: %d wavefronts along the rows, %d row tiles each, %d channels at a time, grid %lld, LDS %zu\n", mw, rw, P.cchunk, wgs, lds);
+    auto kern = rw == 2 ? plain_conv_kernel<2> : plain_conv_kernel<1>;
+    return launch_halo(kern, "plain_conv_kernel", dim3((unsigned)wgs), PLAIN_COLS * mw * 64, lds, s, P, in, reinterpret_cast<const Parts<float>::Vec*>(ws), w, bias, out);
+}
+
 // S = T: the float32 / float64 operator.  S = Bf16 / Fp16 (T = float): the tensors are in that
 // storage format and only the LDS-halo kernel serves them; where it cannot (halo too large, a layer
 // that wants the input-channel split), *declined is set and nothing is launched: the caller then
@@ -58,6 +92,12 @@ int forward(const Geometry& g, const S* in, const S* w, const S* off, const S* b
     if (int rc = device_info(nullptr)) return rc;
     if constexpr (S16)
         if (!forward16_native<ND>(P)) { *declined = true; return DCN_OK; }
+    if constexpr (ND == 2 && sizeof(S) == 4)
+        if (!off) {
+            bool done = false;
+            if (int rc = plain_forward(P, in, w, bias, out, ws, ws ? ws_bytes : 0, s, &done)) return rc;
+            if (done) return DCN_OK;
+        }
     int MT, mchunks;
     fwd_weight_pad<T>(P.M, P.Cg, MT, mchunks, P.Mp, P.Cgp);
     P.mchunks = mchunks;

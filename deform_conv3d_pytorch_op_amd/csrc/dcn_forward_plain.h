@@ -1,0 +1,178 @@
+// Plain convolution of float32 in 2-D (offsets that are all zero): forward pass, and backward pass to the input at stride 1.
+//
+//   out[n][g*M + m][pos] = sum_{cl,tap} W[g*M+m][cl][tap] * in[n][g*Cg+cl][pos * stride - pad + tap * dil]  (+ bias)
+//
+// replaces im2col + the per-group Sgemm of the reference (conv2d/lib/conv2d_cuda.cpp:77-290, conv2d/lib/conv2d_cuda_kernel.cu:25-169).
+//
+// forward_split_kernel with a null offset works out the geometry of every (tap, position), weighs four corners of which three have weight
+// zero, and splits every sample into its bfloat16 parts once per tap.  Here a value is split once, on its way into LDS, where a voxel's
+// parts lie as the operands want them -- [part][voxel][channel] -- so that a step of the contraction is three 16-byte LDS reads at a tap's
+// fixed distance, the weights from L2 (a few steps ahead, in the order of pack_split_weight_kernel) and six matrix instructions a row tile.
+// A workgroup has two position tiles (a block of 64 positions) and MW wavefronts along the rows, RW row tiles each.
+// Small layers: the matrix instructions of 64 -> 64 channels, 3x3, 8 x 56 x 56 take 5 us of the device, a workgroup's first instructions and
+// loads as long again.  us of a forward call with the packing of its weights, on the former kernels -> here: that layer 35 -> 27 (a training step 103 -> 93),
+// 100 -> 100, 5x5, 4 x 60 x 60: 139 -> 77; 512 -> 512, 8 x 28 x 28: 297 -> 273.  One sum to a result tile (every instruction waits for the one
+// before it) and operands read in their own step: 30.
+#pragma once
+#include "dcn_forward_split.h"
+
+namespace dcn {
+
+constexpr int PLAIN_COLS = 2;                           // position tiles of a workgroup
+// operands of a voxel in a part's plane: an odd number, so that eight voxels in a row lie in different LDS banks
+__host__ __device__ inline constexpr int plain_row(int channels) { return (channels / FG) | 1; }
+__host__ inline size_t plain_lds(int hvol, int channels) { return (size_t)Parts<float>::NP * hvol * plain_row(channels) * 16; }
+
+// Grid: N * tiles * G * mchunks workgroups of PLAIN_COLS * MW wavefronts; P.cchunk a multiple of eight.
+template <int RW>
+__global__ __launch_bounds__(512) void plain_conv_kernel(Params P, const float* __restrict__ in, const Parts<float>::Vec* __restrict__ Wq,
+                                                         const float* __restrict__ W, const float* __restrict__ bias, float* __restrict__ out) {
+    touch_arguments<sizeof(Params) + 32>();
+    using PT = Parts<float>;
+    using MM = Mma<float>;
+    typedef PT::Vec Vec;
+    constexpr int TN = 32, NP = PT::NP, AHEAD = RW == 1 ? 4 : 2;
+    constexpr int CH = RW == 1 ? 2 : 1;                 // sums of a result tile, in turn: a matrix instruction does not wait for the one before it
+    extern __shared__ __align__(16) unsigned char smem_raw[];
+    Vec* sX = reinterpret_cast<Vec*>(smem_raw);         // [part][voxel][slab of eight channels]
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), WGS = (int)blockDim.x;
+    const int j = lane % TN, q = lane / TN;
+    const int pt = wave % PLAIN_COLS, mw = wave / PLAIN_COLS, MW = WGS / (64 * PLAIN_COLS);
+    const unsigned unit = xcd_contiguous(blockIdx.x, gridDim.x), rest = unit / P.mchunks;
+    const int g = rest % P.G, mchunk = (int)(unit - rest * (unsigned)P.mchunks.d);
+    HaloPlan H;
+    H.mlo[1] = H.mlo[2] = 0;
+    TileGeo<2> tg;
+    tile_decode<2>(P, H, rest / P.G, tg);
+    int o[2];
+    unsigned pos;
+    const bool valid = tile_position<2>(P, tg, pt * TN + j, o, pos);
+    const int row = P.hext[2], hvol = P.hvol;
+    const int at = (o[0] * P.stride[1] - P.pad[1] - tg.hb[0]) * row + o[1] * P.stride[2] - P.pad[2] - tg.hb[1];      // the position's voxel at tap 0
+    const int cg0 = g * P.Cg, cg1 = cg0 + P.Cg, ntg = (P.kV + 1) / 2;
+    const unsigned mtiles = P.Mp / TN, tile0 = (unsigned)(mchunk * MW + mw) * RW;
+    const unsigned a_tg = mtiles * NP * 64, per_slab = (unsigned)ntg * a_tg;      // operands
+    const float inv = __builtin_amdgcn_rcpf((float)hvol), inv_row = __builtin_amdgcn_rcpf((float)row);
+    const int rs = plain_row(P.cchunk);
+
+    MM::Acc part[CH][RW];
+#pragma unroll
+    for (int h = 0; h < CH; ++h)
+#pragma unroll
+        for (int r = 0; r < RW; ++r) part[h][r] = acc_zero<float>();
+#pragma unroll 1
+    for (int cc0 = cg0; cc0 < cg1; cc0 += P.cchunk) {
+        const int nch = min(P.cchunk, cg1 - cc0), nsl = (nch + FG - 1) / FG;
+        const float* chan0 = in + ((size_t)P.C_in * tg.n + cc0) * P.inV;
+        // Steps: tap pairs, and the slabs of each.  Weights of this wavefront's row tiles, AHEAD steps ahead.
+        const Vec* wp = Wq + (size_t)chunk_slot<FG>(P.cpg, P.Cg, cc0) * per_slab + tile0 * (NP * 64) + lane;
+        const int steps = nsl * ntg;
+        Vec a8[AHEAD][RW][NP];
+        int asl = 0, atg = 0;
+        unsigned lat = 0;
+        auto load_a = [&](int u) {
+#pragma unroll
+            for (int r = 0; r < RW; ++r)
+#pragma unroll
+                for (int k = 0; k < NP; ++k) a8[u][r][k] = wp[lat + (r * NP + k) * 64];
+            lat += per_slab;
+            if (++asl == nsl) {
+                asl = 0;
+                atg = min(atg + 1, ntg - 1);            // (past the last step the last pair again, for nothing)
+                lat = (unsigned)atg * a_tg;
+            }
+        };
+        if (cc0 > cg0) __syncthreads();                 // readers of the last channels are done
+#pragma unroll
+        for (int u = 0; u < AHEAD; ++u) load_a(u);
+        const int items = nsl * hvol;
+#pragma unroll 2
+        for (int it = (int)threadIdx.x; it < items; it += WGS) {
+            const int sl = (int)(((float)it + 0.5f) * inv), v = it - __mul24(sl, hvol);
+            const int vh = (int)(((float)v + 0.5f) * inv_row), ch = vh + tg.hb[0], cw = v - __mul24(vh, row) + tg.hb[1];
+            const bool there = (unsigned)ch < (unsigned)P.in[1] && (unsigned)cw < (unsigned)P.in[2];
+            const unsigned to = there ? (unsigned)ch * (unsigned)P.in[2] + (unsigned)cw : 0u;
+            float x[FG];
+#pragma unroll
+            for (int e = 0; e < FG; ++e) x[e] = chan0[(size_t)min(sl * FG + e, nch - 1) * P.inV + to];
+#pragma unroll
+            for (int e = 0; e < FG; ++e) x[e] = there && sl * FG + e < nch ? x[e] : 0.f;
+            Vec p[NP];
+            PT::split(x, p);
+#pragma unroll
+            for (int k = 0; k < NP; ++k) sX[((size_t)k * hvol + v) * rs + sl] = p[k];
+        }
+        __syncthreads();
+        Vec b8[2][NP];
+        int k0[2] = {0, 0}, bsl = 0, btg = 0;
+        const Vec* bp = nullptr;
+        auto pair = [&]() {                             // this lane's voxel at tap pair btg
+            int k1[2] = {k0[0], k0[1]};
+            next_tap<2>(P, k1);
+            int t0 = k0[0] * P.dil[1] * row + k0[1] * P.dil[2], t1 = k1[0] * P.dil[1] * row + k1[1] * P.dil[2];
+            t1 = 2 * btg + 1 < P.kV ? t1 : t0;          // (its weights are zero)
+            bp = sX + (size_t)(at + (q ? t1 : t0)) * rs;
+            next_tap<2>(P, k1);
+            k0[0] = k1[0]; k0[1] = k1[1];
+        };
+        const size_t plane = (size_t)hvol * rs;
+        auto load_b = [&](int u) {
+#pragma unroll
+            for (int k = 0; k < NP; ++k) b8[u][k] = bp[k * plane];
+            ++bp;
+            if (++bsl == nsl) {
+                bsl = 0;
+                if (++btg < ntg) pair();
+                else bp -= nsl;
+            }
+        };
+        pair();
+        load_b(0);
+        for (int s = 0; s < steps; s += AHEAD) {
+#pragma unroll
+            for (int u = 0; u < AHEAD; ++u)
+                if (s + u < steps) {                    // (uniform)
+                    load_b((u + 1) & 1);
+                    mma_parts<float, RW>(a8[u], b8[u & 1], part[u % CH]);
+                    load_a(u);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+        }
+    }
+    MM::Acc acc[RW];
+#pragma unroll
+    for (int r = 0; r < RW; ++r) {
+        acc[r] = part[0][r];
+        if constexpr (CH > 1) acc[r] += part[1][r];
+    }
+    // Results that the parts may have cost bits (see dcn_forward_split.h): once more on the float32 instructions, from the values themselves.
+    if (__builtin_expect(__any(valid && !results_stand<RW, float>(acc)), 0)) {
+#pragma unroll
+        for (int r = 0; r < RW; ++r) acc[r] = acc_zero<float>();
+        int kk[2] = {0, 0};
+#pragma unroll 1
+        for (int tap = 0; tap < P.kV; ++tap) {
+            const int ch = o[0] * P.stride[1] - P.pad[1] + kk[0] * P.dil[1], cw = o[1] * P.stride[2] - P.pad[2] + kk[1] * P.dil[2];
+            const bool there = valid && (unsigned)ch < (unsigned)P.in[1] && (unsigned)cw < (unsigned)P.in[2];
+            const float* x = in + (size_t)P.C_in * P.inV * tg.n + (there ? (unsigned)ch * (unsigned)P.in[2] + (unsigned)cw : 0u);
+#pragma unroll 1
+            for (int cl = 0; cl < P.Cg; cl += 2) {
+                const int c = min(cl + q, P.Cg - 1);
+                const float xv = x[(size_t)(cg0 + c) * P.inV], b = there && cl + q < P.Cg ? xv : 0.f;
+#pragma unroll
+                for (int r = 0; r < RW; ++r) {
+                    const int m = (int)(tile0 + r) * TN + j;
+                    const float wv = weight_at<float>(P, W, g, min(m, P.M - 1), (size_t)c, tap);
+                    acc[r] = MM::mma(m < P.M && cl + q < P.Cg ? wv : 0.f, b, acc[r]);
+                }
+            }
+            next_tap<2>(P, kk);
+        }
+    }
+    if (!valid) return;
+#pragma unroll
+    for (int r = 0; r < RW; ++r)
+        store_tile<float, float>(P, out + (size_t)P.C_out * P.outV * tg.n, bias, g, (int)(tile0 + r) * TN, q, pos, acc[r]);
+}
+
+}  // namespace dcn

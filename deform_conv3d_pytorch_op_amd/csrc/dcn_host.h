@@ -5,6 +5,7 @@
 #include "dcn_kernels.h"
 #include "dcn_forward.h"
 #include "dcn_forward_split.h"
+#include "dcn_forward_plain.h"
 #include "dcn_prepare.h"
 
 #include <algorithm>
@@ -289,6 +290,7 @@ inline int relayout(const Params& P, const T* w, T* wt, int channel_fastest, hip
 //   DCN_FORWARD_SMALL=0    forward pass, float32 and 16-bit: never several wavefronts to a position
 //   DCN_FORWARD_TINY=0     ... never more than four; 1 / 2 (test hook): sixteen to blocks of 32 positions / eight to blocks of 64 on every
 //                          layer with several, of up to two row tiles
+//   DCN_PLAIN=0            the plain convolution of float32 on the kernels of the deformable layer; =2 (test hook): of any size on its own
 //   DCN_SCATTER_BUDGET_KB  dynamic LDS per workgroup of the privatised scatter kernels (default 156, at most 157: backward_fused_kernel, 144, at
 //                          most 159: the others)
 //   DCN_SCATTER=global     scatter grad-input with global atomics instead of the LDS-privatised kernel
@@ -397,6 +399,10 @@ static int forward_tail_split() {       // DCN_FORWARD_TAIL=0: the forward pass 
 static bool forward_tail_two_runs() {    // DCN_FORWARD_TAIL2=0: the split units of the forward pass's last round are all split the same number of ways
     static const int v = [] { const char* e = getenv("DCN_FORWARD_TAIL2"); return (e && atoi(e) == 0) ? 0 : 1; }();
     return v != 0;
+}
+static int plain_conv() {                // DCN_PLAIN=0, 2: see above
+    static const int v = [] { const char* e = getenv("DCN_PLAIN"); return e ? atoi(e) : 1; }();
+    return v;
 }
 static bool forward_shared() {           // DCN_FORWARD_SHARED=0: the forward pass always samples in every wavefront (forward_split_kernel)
     static const int v = [] { const char* e = getenv("DCN_FORWARD_SHARED"); return (e && atoi(e) == 0) ? 0 : 1; }();

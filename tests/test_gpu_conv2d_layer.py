@@ -33,3 +33,46 @@ def test_gradients(spec, dtype):
     for name, got, ref in (("y", y, want), ("x", x.grad, x64.grad), ("w", m.weight.grad, w64.grad), ("b", m.bias.grad, b64.grad)):
         err = (got.detach().cpu().double() - ref.detach()).norm() / ref.detach().norm()
         assert err.item() <= tol, (name, err.item())
+
+
+# The kernel of the plain convolution at the edges of its shapes -- one, two, four and eight row tiles, passes of eight to sixty-four channels
+# with remainders, one, two and three tap pairs and a lone tap, strides and dilations, groups, positions that fill no block -- whatever the
+# layer's size (DCN_PLAIN=2, read once per process).
+PLAIN = [(1, 8, 1, (9, 9), 3, 1, 1, 1, 1), (2, 5, 33, (8, 17), 1, 1, 0, 1, 1), (1, 70, 64, (7, 24), 3, 2, 1, 1, 1), (1, 24, 130, (11, 9), (3, 2), 1, (1, 0), (2, 3), 1),
+         (1, 136, 260, (10, 12), 2, 1, 1, 1, 1), (2, 18, 36, (13, 8), 5, (1, 2), 2, 1, 2), (1, 64, 96, (30, 31), 3, 1, 8, 7, 1), (1, 200, 40, (16, 16), 3, 1, 1, 1, 1),
+         (1, 12, 300, (9, 10), 3, 1, 2, 2, 4), (3, 1, 1, (1, 1), 1, 1, 0, 1, 1), (1, 40, 16, (20, 22), 7, 1, 3, 1, 1)]
+
+
+def plain_cases():
+    import deform_conv3d_pytorch_op_amd as dcn
+    for spec in PLAIN:
+        test_gradients(spec, torch.float32)
+    # values without bfloat16 parts, and values that are not finite: next to them no result but those that they belong to
+    torch.manual_seed(5)
+    x = torch.randn(3, 20, 18, 19)
+    x[0, 3, 4, 5], x[0, 7, 0, 0] = float("inf"), float("nan")
+    x[1] *= 1e-36
+    w = torch.randn(40, 20, 3, 3)
+    m = dcn.Conv2d(20, 40, 3, 1, 1, bias=False, device="cuda", dtype=torch.float32)
+    with torch.no_grad():
+        m.weight.copy_(w)
+        got = m(x.cuda()).cpu().double()
+    want = F.conv2d(x.double(), w.double(), None, 1, 1)
+    assert torch.equal(torch.isfinite(got), torch.isfinite(want))
+    for n in (1, 2):
+        assert ((got[n] - want[n]).norm() / want[n].norm()).item() <= 1e-6
+    print("plain cases passed", flush=True)
+
+
+def test_plain_kernel():
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-u", "-c", "from tests.test_gpu_conv2d_layer import plain_cases; plain_cases()"], cwd=root,
+                       env=dict(os.environ, DCN_PLAIN="2", DCN_TRACE_PLANS="1"), stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert r.returncode == 0 and "plain cases passed" in r.stdout, r.stdout[-3000:]
+    assert r.stdout.count("dcn plain convolution") >= 2 * len(PLAIN) - 4      # (grad_input of layers with a stride or more padding than span is no convolution)
+    assert "dcn forward:" not in r.stdout
+    for rows in ("1 wavefronts along the rows, 1 row", "2 wavefronts along the rows, 1 row", "4 wavefronts along the rows, 1 row", "4 wavefronts along the rows, 2 row"):
+        assert rows in r.stdout
