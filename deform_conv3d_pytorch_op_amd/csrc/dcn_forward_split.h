@@ -253,37 +253,46 @@ template <int ND, int WGS, bool CHECK, typename S>
 __device__ inline bool stage_halo(const Params& P, const HaloPlan& H, const TileGeo<ND>& tg, const S* __restrict__ chan0, int nch,
                                   typename HaloCell<S>::Vec* __restrict__ sIn) {
     constexpr int CH = HaloCell<S>::CH;
-    // an item is a cell: consecutive threads take consecutive voxels, several items of a thread are in flight
+    // an item is a cell: consecutive threads take consecutive voxels
     const int items = (nch + CH - 1) / CH * H.hvol;
     const float inv2 = __builtin_amdgcn_rcpf((float)H.hext[2]), inv1 = __builtin_amdgcn_rcpf((float)H.hext[1]), inv = __builtin_amdgcn_rcpf((float)H.hvol);
     const size_t step = (size_t)P.inV * sizeof(S);
+    // Items of a thread in flight, the last ones too: a pass waits for memory ceil(items / U) times.  (Four in a loop unrolled so, and the remainder one by
+    // one: 256 -> 256, 2-D, steps 880 -> 858 us, the ragged 48 -> 80 in 3-D 398 -> 390.  Of 128 -> 128 at stride 1 2 2, eight wavefronts, 17 items: 2, 3, 4, 6
+    // in flight 4535, 4497, 4511, 4476; 64 -> 64 in 3-D, sixteen wavefronts, inference: 469, 471, 481, 471.)
+    constexpr int U = WGS >= 1024 ? 3 : 6;
     bool bad = false;
-    auto stage = [&](int it, auto full_tag) {
-        const int grp = (int)(((float)it + 0.5f) * inv), v = it - __mul24(grp, H.hvol);
-        const unsigned t = halo_voxel<ND>(P, H, tg, v, inv1, inv2);
-        const char* cp = reinterpret_cast<const char*>(chan0) + (size_t)(t == ~0u ? 0u : t) * sizeof(S) + (size_t)(grp * CH) * step;
-        const int last = nch - 1 - grp * CH;                    // >= CH - 1 but in a short last group
-        typename HaloCell<S>::Vec cell;
+    // (no load is masked: a masked one is waited for on its own; past the last item and past the last channel a load is repeated)
+    auto stage = [&](int it0, auto count) {
+        constexpr int C = decltype(count)::value;
+        typename HaloCell<S>::Vec cell[C];
+        int grp[C], v[C];
+        bool there[C];
 #pragma unroll
-        for (int e = 0; e < CH; ++e) {
-            cell[e] = (typename HaloCell<S>::V)0.f;
-            if (decltype(full_tag)::value || e < nch) {         // (uniform)
-                const S x = *reinterpret_cast<const S*>(cp + (size_t)min(e, last) * step);
-                if constexpr (CHECK) bad = bad || !(fabsf(Store<S>::ld(x)) <= std::numeric_limits<float>::max());
-                cell[e] = HaloCell<S>::raw(x);
-            }
+        for (int u = 0; u < C; ++u) {
+            const int it = min(it0 + u * WGS, items - 1);
+            grp[u] = (int)(((float)it + 0.5f) * inv);
+            v[u] = it - __mul24(grp[u], H.hvol);
+            const unsigned t = halo_voxel<ND>(P, H, tg, v[u], inv1, inv2);
+            there[u] = t != ~0u;
+            const char* cp = reinterpret_cast<const char*>(chan0) + (size_t)(there[u] ? t : 0u) * sizeof(S) + (size_t)(grp[u] * CH) * step;
+            const int last = nch - 1 - grp[u] * CH;             // >= CH - 1 but in a short last group
+#pragma unroll
+            for (int e = 0; e < CH; ++e) cell[u][e] = HaloCell<S>::raw(*reinterpret_cast<const S*>(cp + (size_t)min(e, last) * step));
         }
 #pragma unroll
-        for (int e = 0; e < CH; ++e) cell[e] = (e <= last && t != ~0u) ? cell[e] : (typename HaloCell<S>::V)0.f;
-        sIn[(size_t)grp * H.hstride + v] = cell;
+        for (int u = 0; u < C; ++u) {
+            const int last = nch - 1 - grp[u] * CH;
+            if constexpr (CHECK) {
+#pragma unroll
+                for (int e = 0; e < CH; ++e) bad = bad || !(fabsf((float)cell[u][e]) <= std::numeric_limits<float>::max());
+            }
+#pragma unroll
+            for (int e = 0; e < CH; ++e) cell[u][e] = (e <= last && there[u]) ? cell[u][e] : (typename HaloCell<S>::V)0.f;
+            if (it0 + u * WGS < items) sIn[(size_t)grp[u] * H.hstride + v[u]] = cell[u];
+        }
     };
-    if (nch >= CH) {
-#pragma unroll 4
-        for (int it = threadIdx.x; it < items; it += WGS) stage(it, std::true_type{});
-    } else {                                                    // a segment shorter than a cell loads what it has
-#pragma unroll 4
-        for (int it = threadIdx.x; it < items; it += WGS) stage(it, std::false_type{});
-    }
+    for (int it = threadIdx.x; it < items; it += U * WGS) stage(it, std::integral_constant<int, U>{});
     return bad;
 }
 
