@@ -49,7 +49,7 @@ namespace dcn {
 
 constexpr unsigned ROW_SLAB = 32;                       // positions of a slab: two steps
 __host__ __device__ inline unsigned row_steps(unsigned V) { return (V + ROW_SLAB - 1) / ROW_SLAB * 2; }
-// grad_output in operand order: [n][step][part][q][output channel], 16 bytes (eight positions) each, zero past the volume
+// grad_output in operand order: [n][octet of positions][part][output channel], 16 bytes (eight positions) each, zero past the volume
 template <typename S> inline size_t row_operand_bytes(int N, int C_out, size_t V) { return (size_t)N * row_steps((unsigned)V) * Parts<S>::NP * 2 * C_out * 16; }
 // channels to a lane (16-bit storage: pairs, two column tiles)
 template <typename S> __host__ __device__ constexpr int lane_channels() { return 4 / (int)sizeof(S); }
@@ -156,11 +156,12 @@ __global__ __launch_bounds__(WG, split_waves<S>(MT)) void backward_weight_split_
     }
     // what this thread copies of a step's rows: 16 bytes each, rows past M as row M - 1
     constexpr int NROW = MT * NP * 64, NA = (NROW + WG - 1) / WG;
-    unsigned r_at[NA];
+    unsigned r_at[NA], r_q[NA];
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
         const int x = i * WG + threadIdx.x, m = x % (MT * TN), pq = min(x / (MT * TN), NP * 2 - 1);
-        r_at[i] = ((unsigned)pq * P.C_out + g * P.M + min(m_base + m, P.M - 1)) * 16u;
+        r_at[i] = ((unsigned)(pq / 2) * P.C_out + g * P.M + min(m_base + m, P.M - 1)) * 16u;
+        r_q[i] = pq & 1;
     }
 
     typename MM::Acc acc[CT][MT];
@@ -174,13 +175,32 @@ __global__ __launch_bounds__(WG, split_waves<S>(MT)) void backward_weight_split_
     for (int u = 0; u < CT; ++u)
 #pragma unroll
         for (int mt = 0; mt < MT; ++mt) acc[u][mt] = acc_zero<T>();
-    const size_t step_bytes = (size_t)NP * 2 * P.C_out * 16;
+    // A slab's positions are four octets.  In 3-D of float32, which reads a corner's channels dword by dword and waits for the L1: of a run of 4 * S octets
+    // -- about four rows of the output -- slab r takes octets r, r + S, r + 2 S, r + 3 S, a block of positions, whose samples share more lines than
+    // those of 32 positions in a row; the octets behind the last whole run in order.  (Steps of 64 -> 64, rows of 56: 2436 -> 2406 us, 128 -> 128
+    // at stride 1 2 2 4484 -> 4461.  2-D waits less for the L1 and loses the arithmetic: 256 -> 256 861 -> 870, no offsets 90 -> 92.)
+    constexpr bool BLOCKS = ND == 3 && sizeof(S) == 4 && !PLAIN;
+    const int S4 = BLOCKS ? max((P.out[2].d + 4) / 8, 1) : 1, runs4 = BLOCKS ? slabs_per_sample / S4 * S4 : 0;
+    auto first_octet = [&](int slab, int& stride) {     // of a slab of a sample
+        stride = BLOCKS && slab < runs4 ? S4 : 1;
+        return BLOCKS && slab < runs4 ? slab / S4 * S4 * 4 + slab % S4 : slab * 4;
+    };
+    const unsigned octet_bytes = (unsigned)(NP * P.C_out * 16);
     const char* const row0 = reinterpret_cast<const char*>(rows);
     Vec rv[NA];
-    auto load_rows = [&](size_t step) {                 // of all samples
-        const char* ap = row0 + step * step_bytes;
+    auto load_rows = [&](int slab, int st) {
+        const int n = slab / slabs_per_sample;
+        int stride;
+        const int oct = first_octet(slab - n * slabs_per_sample, stride);
+        const char* ap = row0 + ((size_t)n * slabs_per_sample * 4 + oct + 2 * st * stride) * octet_bytes;
+        const unsigned next = (unsigned)stride * octet_bytes;
 #pragma unroll
-        for (int i = 0; i < NA; ++i) rv[i] = *reinterpret_cast<const Vec*>(ap + r_at[i]);
+        for (int i = 0; i < NA; ++i) rv[i] = *reinterpret_cast<const Vec*>(ap + (r_at[i] + (r_q[i] ? next : 0u)));
+    };
+    auto slab_position = [&](int slab, int at) {        // position `at` (0 .. 31) of a slab of all samples, in its sample
+        int stride;
+        const int oct = first_octet(slab % slabs_per_sample, stride);
+        return (unsigned)(oct + at / 8 * stride) * 8u + (unsigned)(at % 8);
     };
     auto put_rows = [&](int buf) {
 #pragma unroll
@@ -190,7 +210,7 @@ __global__ __launch_bounds__(WG, split_waves<S>(MT)) void backward_weight_split_
     T offv[GT][ND];
     auto load_off = [&](int slab) {
         const int n = slab / slabs_per_sample;
-        const unsigned posc = min((unsigned)(slab % slabs_per_sample) * TN + j, P.outV - 1);
+        const unsigned posc = min(slab_position(slab, j), P.outV - 1);
         const S* off_n = PLAIN ? nullptr : off + ((size_t)n * P.DG + dg) * P.kV * ND * P.outV;
 #pragma unroll
         for (int u = 0; u < GT; ++u)
@@ -200,16 +220,15 @@ __global__ __launch_bounds__(WG, split_waves<S>(MT)) void backward_weight_split_
     const T sgn = split & 1 ? -1.f : 1.f;               // of this split's samples
     if (first < last) {
         load_off(first);
-        load_rows((size_t)first * 2);
+        load_rows(first, 0);
         put_rows(0);
     }
     __syncthreads();
     for (int slab = first; slab < last; slab += turn) {
         const int n = slab / slabs_per_sample;
-        const unsigned p0 = (unsigned)(slab % slabs_per_sample) * TN;
         const char* in_n = reinterpret_cast<const char*>(in_cl + (size_t)n * P.inV * P.C_in);        // scalar bases
         const int next_slab = min(slab + turn, last - 1);
-        const unsigned pos = p0 + j;
+        const unsigned pos = slab_position(slab, j);
         const bool valid = pos < P.outV;
         const unsigned posc = valid ? pos : P.outV - 1;
         int o[ND];
@@ -282,7 +301,7 @@ __global__ __launch_bounds__(WG, split_waves<S>(MT)) void backward_weight_split_
         if (works) fetch(0);
 #pragma unroll
         for (int st = 0; st < 2; ++st) {
-            load_rows(st == 0 ? (size_t)slab * 2 + 1 : (size_t)next_slab * 2);
+            load_rows(st == 0 ? slab : next_slab, st ^ 1);
             if (works) {
                 float val[CT][8];
 #pragma unroll
@@ -351,12 +370,11 @@ __global__ __launch_bounds__(WG, split_waves<S>(MT)) void backward_weight_split_
         for (int a = 0; a < ND; ++a) kx[a] = kk[a] * P.dil[slot<ND>(a)];
         for (int slab = first; slab < last; slab += turn) {
             const int n = slab / slabs_per_sample;
-            const unsigned p0 = (unsigned)(slab % slabs_per_sample) * TN;
             const S* off_n = PLAIN ? nullptr : off + (((size_t)n * P.DG + dg) * P.kV + min(tap, P.kV - 1)) * ND * P.outV;
             const char* in_n = reinterpret_cast<const char*>(in_cl + (size_t)n * P.inV * P.C_in);
 #pragma unroll 1
             for (int ks = 0; ks < TN; ks += 2) {
-                const unsigned pos = p0 + ks + q, posc = min(pos, P.outV - 1);
+                const unsigned pos = slab_position(slab, ks + q), posc = min(pos, P.outV - 1);
                 int o[ND], ib[ND];
                 decode_pos<ND>(P, posc, o);
 #pragma unroll

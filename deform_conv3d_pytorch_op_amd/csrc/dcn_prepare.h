@@ -164,7 +164,7 @@ __device__ inline void prep_rows(const PrepJob& job, unsigned block) {
                 for (int x = 0; x < PT::NP; ++x) p8[x][e] = p[x];
             }
 #pragma unroll
-            for (int x = 0; x < PT::NP; ++x) dst[((size_t)(step * PT::NP + x) * 2 + (oct & 1)) * job.C + c] = p8[x];
+            for (int x = 0; x < PT::NP; ++x) dst[((size_t)(step * 2 + (oct & 1)) * PT::NP + x) * job.C + c] = p8[x];
         }
         __syncthreads();
     }

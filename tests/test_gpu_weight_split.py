@@ -26,6 +26,8 @@ LAYERS = [
     # 16 bytes of a corner to a lane: segments that end one lane into a tile, also two and four taps to an item; one over two convolution groups
     (2, 1, 36, 70, (97, 161), 3, 1, 1, 1, 36, 1, 1.5), (2, 1, 40, 130, (161, 99), 3, 1, 1, 1, 40, 2, 3.0), (2, 1, 12, 65, (161, 163), 3, 1, 1, 1, 12, 1, 9.0),
     (2, 1, 4, 66, (229, 231), 3, 1, 1, 1, 4, 1, 1.5), (2, 1, 68, 66, (1, 9001), 3, 1, 1, 1, 68, 1, 1.5),
+    # slabs of four octets apart, 3-D: rows of several octets with slabs left over, rows shorter than an octet, two samples
+    (3, 1, 17, 66, (3, 41, 75), 3, 1, 1, 1, 17, 1, 1.5), (3, 1, 9, 70, (203, 16, 3), 3, 1, 1, 1, 9, 1, 1.5), (3, 2, 16, 129, (5, 31, 47), 3, 1, 1, 1, 16, 1, 9.0),
 ]
 IDS = lambda s: "%dd-%d-%d-k%d-g%d" % (s[0], s[2], s[3], s[5], s[10])
 
