@@ -156,9 +156,12 @@ template <> struct Wide<double> { typedef double type; };
 template <typename S>
 __global__ __launch_bounds__(256) void narrow_gradients_kernel(const float* __restrict__ a, S* __restrict__ da, size_t na, const float* __restrict__ b,
                                                                S* __restrict__ db, size_t nb, const float* __restrict__ c, S* __restrict__ dc, size_t nc,
-                                                               const float* __restrict__ d, S* __restrict__ dd, size_t nd) {
+                                                               const float* __restrict__ d, S* __restrict__ dd, size_t nd, bool octets, int N, int C,
+                                                               unsigned V) {
     const size_t step = (size_t)gridDim.x * 256, first = (size_t)blockIdx.x * 256 + threadIdx.x;
-    for (size_t i = first; i < na; i += step) da[i] = S::narrow(a[i]);
+    if (octets) octets_to_planes(a, N, C, V, false, first, step, [&](size_t to, float v) { da[to] = S::narrow(v); });
+    else
+        for (size_t i = first; i < na; i += step) da[i] = S::narrow(a[i]);
     for (size_t i = first; i < nb; i += step) db[i] = S::narrow(b[i]);
     for (size_t i = first; i < nc; i += step) dc[i] = S::narrow(c[i]);
     for (size_t i = first; i < nd; i += step) dd[i] = S::narrow(d[i]);
@@ -202,19 +205,28 @@ int layer_backward(const Geometry& g, const S* in, const S* w, const S* off, con
     Prep prep;
     WeightCall<T, S> call;
     const PlanChoice none = {};
-    if (data) prep.zero(tgin, z.in * sizeof(T));
     // (16-bit storage: the kernels that read it may decline a layer, which then runs on widened copies)
     bool wdeclined = S16 && !native16(), ddeclined = wdeclined;
     if (gw && !wdeclined)
         if (int rc = backward_weight_plan<T, ND, S>(P, in, off, gout, wws, need.weight, gb != nullptr, call, prep, S16 ? &wdeclined : nullptr)) return rc;
     if (data && !ddeclined)
         if (int rc = backward_input_offset<T, ND, S>(g, in, w, off, gout, tgin, tgoff, dws, need.data, s, flags, S16 ? &ddeclined : nullptr, &prep)) return rc;
+    if (data && ddeclined) prep.zero(tgin, z.in * sizeof(T));      // (else the operator sees to it)
     if (!data || ddeclined)
         if (int rc = launch_prepare<T, S>(P, none, prep, w, off, 0, s)) return rc;
     if (gw && !wdeclined)
         if (int rc = backward_weight_run<T, ND, S>(call, off, tgw, tgb, false, s)) return rc;
+    bool narrowed = false;                              // grad_input
     if constexpr (S16) {
         const bool wide_data = data && ddeclined, wide_weight = gw && wdeclined;
+        if (wide_weight && prep.octets) {               // they lie where the copies go
+            const unsigned blocks = (unsigned)((z.in + 1023) / 1024 > 8192 ? 8192 : (z.in + 1023) / 1024);
+            hipLaunchKernelGGL(narrow_gradients_kernel<S>, dim3(blocks), dim3(256), 0, s, prep.octets, gin, z.in, nullptr, nullptr, 0, nullptr, nullptr, 0, nullptr,
+                               nullptr, 0, true, P.N, P.C_in, P.inV);
+            if (int rc = check_launch("narrow_gradients_kernel")) return rc;
+            prep.octets = nullptr;
+            narrowed = true;
+        }
         if (wide_data || wide_weight) {
             p = shared;                                 // the kernels above are done with their operands by the time the next ones run
             left = shared_bytes;
@@ -238,10 +250,10 @@ int layer_backward(const Geometry& g, const S* in, const S* w, const S* off, con
         }
     }
     if constexpr (S16) {
-        const size_t na = data ? z.in : 0, nb = data ? z.off : 0, nc = gw ? z.w : 0, nd = gb ? (size_t)P.C_out : 0, most = na + nb + nc;
+        const size_t na = data && !narrowed ? z.in : 0, nb = data ? z.off : 0, nc = gw ? z.w : 0, nd = gb ? (size_t)P.C_out : 0, most = na + nb + nc;
         const unsigned blocks = (unsigned)((most + 1023) / 1024 > 8192 ? 8192 : (most + 1023) / 1024 + 1);
-        hipLaunchKernelGGL(narrow_gradients_kernel<S>, dim3(blocks), dim3(256), 0, s, (const float*)tgin, gin, na, (const float*)tgoff, goff, nb, (const float*)tgw, gw,
-                           nc, (const float*)tgb, gb, nd);
+        hipLaunchKernelGGL(narrow_gradients_kernel<S>, dim3(blocks), dim3(256), 0, s, prep.octets ? prep.octets : (const float*)tgin, gin, na, (const float*)tgoff, goff, nb, (const float*)tgw, gw,
+                           nc, (const float*)tgb, gb, nd, prep.octets != nullptr, P.N, P.C_in, P.inV);
         return check_launch("narrow_gradients_kernel");
     }
     return DCN_OK;

@@ -133,6 +133,36 @@ template <int ND, int CCH> __host__ __device__ inline constexpr int fused_pt() {
 // LDS bytes per halo voxel: input cells (four float32 or eight 16-bit channels to 16 bytes) and the paired 32-bit sums
 template <typename S> inline size_t fused_voxel_bytes(int cch) { return (size_t)((cch + HaloCell<S>::CH - 1) / HaloCell<S>::CH) * 16 + (size_t)cch * 4; }
 
+// grad_input in octets, [n][channel / 8][voxel][8], where every chunk of channels is an octet or half of one: collected there, and brought to
+// the layout of the tensor by octets_to_planes.  The float atomics of a flush go to memory by the line: 1.0e8 of them from halos of 9 x 15 x 15
+// voxels take 545 us with the lanes along the rows of eight planes (14 voxels: 56 bytes), 283 in octets (448), 462 channels-last (32).
+// Steps of 128 -> 128 in deformable groups of 32, stride 1 2 2, 2 x 16 x 112 x 112: 4460 -> 4202 us (the kernel 2.40 -> 2.24 ms, 59 us for
+// the tensor), of 64 -> 64, 4 x 16 x 56 x 56: 2403 -> 2372, in bfloat16 1659 -> 1648, whose flushes are a third as long beside the rest.
+// put(index in the tensor, value), one thread per voxel of an octet.  last: the source is channels-last instead.
+template <typename Put>
+__device__ inline void octets_to_planes(const float* __restrict__ src, int N, int C, unsigned V, bool last, size_t first, size_t step, Put put) {
+    typedef float F4 __attribute__((ext_vector_type(4)));
+    const size_t items = (size_t)N * (unsigned)(C / 8) * V;
+    for (size_t i = first; i < items; i += step) {
+        const size_t row = items <= ~0u ? (size_t)((unsigned)i / V) : i / V;      // (uniform; a 64-bit division is a hundred instructions)
+        const unsigned v = (unsigned)(i - row * V);
+        const size_t n = row / (unsigned)(C / 8);
+        const F4* from = reinterpret_cast<const F4*>(src + (last ? (n * V + v) * C + (row - n * (unsigned)(C / 8)) * 8 : i * 8));
+        const F4 a = from[0], b = from[1];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) put((row * 8 + e) * V + v, e < 4 ? a[e & 3] : b[e & 3]);
+    }
+}
+// ADD: the tensor is added to.  *gate == gate_last: the source is channels-last.
+template <bool ADD>
+__global__ __launch_bounds__(256) void octets_to_planes_kernel(const float* __restrict__ src, float* __restrict__ dst, int N, int C, unsigned V,
+                                                               const unsigned* __restrict__ gate, unsigned gate_last) {
+    octets_to_planes(src, N, C, V, gate && *gate == gate_last, (size_t)blockIdx.x * 256 + threadIdx.x, (size_t)gridDim.x * 256, [&](size_t to, float v) {
+        if (ADD) dst[to] += v;
+        else dst[to] = v;
+    });
+}
+
 // Dynamic LDS = hstride * fused_voxel_bytes(CCH).  Work items, csplit, whole and goff_atomic: as at backward_input_halo_kernel.
 template <int ND, int CCH, int NPT, typename S>
 __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params P, PlanSet alts, const unsigned* __restrict__ sel, const S* __restrict__ in,
@@ -140,7 +170,7 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
                                                                           const S* __restrict__ W, const S* __restrict__ gout,
                                                                           const typename Parts<S>::Vec* __restrict__ gq, const float* __restrict__ bounds,
                                                                           float* __restrict__ gin, float* __restrict__ goff, int csplit, unsigned whole,
-                                                                          int goff_atomic) {
+                                                                          int goff_atomic, int octets) {
     touch_arguments<sizeof(Params) + sizeof(PlanSet) + 88>();
     HaloPlan H;
     if (!chosen_halo(P, alts, sel, H)) return;          // another launch runs the chosen plan
@@ -254,6 +284,11 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
             load_cell(chan0, nch, u, cell);
             store_cell(nch, u, cell);
         }
+    };
+
+    // where the gradient of a voxel of this sample is collected
+    auto gin_at = [&](int c, unsigned at) {
+        return gin + (ND == 3 && octets ? ((size_t)n * P.C_in + (c & ~7)) * P.inV + (size_t)at * 8 + (c & 7) : ((size_t)n * P.C_in + c) * P.inV + at);
     };
 
     const int g_last = (c_hi - 1) / P.Cg;
@@ -579,7 +614,6 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
                                     for (int x = 0; x < CCH; ++x) g1 = x == e ? gv[x] : g1;
                                     const size_t chan = ((size_t)n * P.C_in + cc0 + e) * P.inV;
                                     if (far) {
-                                        float* gc = gin + chan;
                                         const S* ic = in + chan;
                                         float vv[NC];
 #pragma unroll
@@ -587,7 +621,7 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
                                         const float fh = t.f[0], gh = 1.f - fh, fw = t.f[1], gw = 1.f - fw;
                                         const float cw[4] = {gh * gw, gh * fw, fh * gw, fh * fw};
 #pragma unroll
-                                        for (int i = 0; i < NC; ++i) atomic_add(gc + t.idx[i], cw[i] * g1);
+                                        for (int i = 0; i < NC; ++i) atomic_add(gin_at(cc0 + e, t.idx[i]), cw[i] * g1);
                                         ga[0] += (vv[2] - vv[0]) * gw + (vv[3] - vv[1]) * fw;
                                         ga[1] += (vv[1] - vv[0]) * gh + (vv[3] - vv[2]) * fh;
                                     }
@@ -613,12 +647,11 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
                                         d[a] = 0.f;
                                     }
                                     if (e < nch) {
-                                        const size_t to = ((size_t)n * P.C_in + cc0 + e) * P.inV + at;
-                                        const float v = g1 * Store<S>::ld(in[to]);
+                                        const float v = g1 * Store<S>::ld(in[((size_t)n * P.C_in + cc0 + e) * P.inV + at]);
                                         float cw = wa[0];
 #pragma unroll
                                         for (int a = 1; a < ND; ++a) cw *= wa[a];
-                                        atomic_add(gin + to, cw * g1);
+                                        atomic_add(gin_at(cc0 + e, at), cw * g1);
 #pragma unroll
                                         for (int a = 0; a < ND; ++a) {
                                             d[a] = (i >> (ND - 1 - a)) & 1 ? v : -v;
@@ -664,27 +697,54 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
                 load_x(chunk_input(cn), nchn);
             }
             __syncthreads();                                           // all LDS adds of this chunk have landed
-            // up to four cell planes of a voxel to a thread
-            const int pairs = (nch + 1) / 2, cells = (pairs + 3) / 4 * H.hvol;
-            for (int it = (int)here(threadIdx.x); it < cells; it += WGS) {
-                const int pg = CCH > 8 ? (int)(((float)it + 0.5f) * invV) : 0, vox = it - __mul24(pg, H.hvol);
-                const unsigned at = halo_voxel<ND>(P, H, tg, vox, inv1, inv2);
-                float* gp = gin + ((size_t)n * P.C_in + cc0 + pg * 8) * P.inV + (at == ~0u ? 0u : at);
-                Sum* cp = sG + (size_t)(pg * 4) * hs + vox;
-                const int planes = min(4, pairs - pg * 4);
-                for (int x = 0; x < planes; ++x) {
-                    const Sum cell = *cp;
-                    if (cell != 0) {
-                        *cp = 0;
-                        if (at != ~0u) {                               // (a cell outside the volume holds zero)
-                            float v0, v1;
-                            Cells::value2(cell, inv_scale, v0, v1);
-                            if (v0 != 0.f) atomic_add(gp, v0);
-                            if (pg * 8 + x * 2 + 1 < nch && v1 != 0.f) atomic_add(gp + P.inV, v1);
-                        }
+            constexpr int FE = CCH < 8 ? CCH : 8, FP = FE / 2;         // channels, cell planes flushed together
+            if (ND == 3 && octets) {
+                // 64 voxels to a wavefront: each works one out, then FE lanes share a voxel, whose sums go to neighbouring addresses
+                const unsigned l = here((unsigned)lane), e = l % FE;
+                float* const ge = gin + ((size_t)n * P.C_in + (cc0 & ~7)) * P.inV + (cc0 & 7) + e;
+                for (int v0 = wave * 64; v0 < H.hvol; v0 += WGS) {
+                    const int vox = v0 + (int)l;
+                    const unsigned at = vox < H.hvol ? halo_voxel<ND>(P, H, tg, vox, inv1, inv2) : ~0u;
+                    Sum* const cp = sG + (size_t)(e / 2) * hs;
+                    int from[FE];
+                    unsigned to[FE];
+                    Sum cell[FE];
+#pragma unroll
+                    for (int u = 0; u < FE; ++u) {
+                        to[u] = (unsigned)__shfl((int)at, u * (64 / FE) + (int)(l / FE));
+                        from[u] = min(v0 + u * (64 / FE) + (int)(l / FE), H.hvol - 1);
+                        cell[u] = cp[from[u]];
                     }
-                    cp += hs;
-                    gp += 2 * (size_t)P.inV;
+                    __builtin_amdgcn_sched_barrier(0);                 // all of them on their way
+#pragma unroll
+                    for (int u = 0; u < FE; ++u)
+                        if (to[u] != ~0u) {                            // (a cell outside the volume holds zero)
+                            reinterpret_cast<unsigned*>(cp + from[u])[e & 1] = 0;
+                            const float v = Cells::value_of_pair(cell[u], e & 1, inv_scale);
+                            if (v != 0.f) atomic_add(ge + (size_t)to[u] * 8, v);
+                        }
+                }
+            } else {
+                const int pairs = (nch + 1) / 2, cells = (pairs + FP - 1) / FP * H.hvol;
+                for (int it = (int)here(threadIdx.x); it < cells; it += WGS) {
+                    const int pg = CCH > 8 ? (int)(((float)it + 0.5f) * invV) : 0, vox = it - __mul24(pg, H.hvol);
+                    const unsigned at = halo_voxel<ND>(P, H, tg, vox, inv1, inv2);
+                    float* gp = gin + ((size_t)n * P.C_in + cc0 + pg * 8) * P.inV + (at == ~0u ? 0u : at);
+                    Sum* cp = sG + (size_t)(pg * 4) * hs + vox;
+                    Sum cell[FP];
+#pragma unroll
+                    for (int x = 0; x < FP; ++x) cell[x] = cp[(size_t)x * hs];
+#pragma unroll
+                    for (int x = 0; x < FP; ++x) cp[(size_t)x * hs] = 0;
+                    if (at == ~0u) continue;                           // (a cell outside the volume holds zero)
+#pragma unroll
+                    for (int x = 0; x < FP; ++x) {                     // (planes past the chunk's channels hold zeros)
+                        float v0, v1;
+                        Cells::value2(cell[x], inv_scale, v0, v1);
+                        if (v0 != 0.f) atomic_add(gp, v0);
+                        if (pg * 8 + x * 2 + 1 < nch && v1 != 0.f) atomic_add(gp + P.inV, v1);
+                        gp += 2 * (size_t)P.inV;
+                    }
                 }
             }
             if (more) {

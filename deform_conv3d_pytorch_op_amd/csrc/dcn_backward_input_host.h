@@ -7,7 +7,7 @@ namespace dcn {
 // The instantiations of backward_fused_kernel: channels per chunk and position tiles per block.
 template <int ND, typename S>
 using FusedKern = void (*)(Params, PlanSet, const unsigned*, const S*, const S*, const typename Parts<S>::Vec*, const S*, const S*, const typename Parts<S>::Vec*,
-                           const float*, float*, float*, int, unsigned, int);
+                           const float*, float*, float*, int, unsigned, int, int);
 template <int ND, typename S> inline FusedKern<ND, S> fused_kernel(int cch, int tiles) {
     if (tiles == 4) return cch == 8 ? backward_fused_kernel<ND, 8, 4, S> : cch == 4 ? backward_fused_kernel<ND, 4, 4, S> : nullptr;
     if constexpr (ND == 2)
@@ -327,6 +327,15 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
         bool any_atomic = false;
         for (int k = 0; k < pc.nplans; ++k) any_atomic = any_atomic || fp[k].zero_goff;
         if (any_atomic) prep.zero(goff, n_off * sizeof(T));
+        // Where the fused kernel collects grad_input: in octets of channels in the place of the channels-last gradient, or in the tensor itself.  In 3-D
+        // the last launch of the path without LDS tiling, or the rounding of a 16-bit layer's gradients, brings them to the tensor, and a halo
+        // has 8 to 18 voxels to a position.  In 2-D it has two: steps of 256 -> 256, 3x3, 8 x 56 x 56 874 us in the tensor, 883 in octets (one launch more),
+        // in binary16 435 and 436.
+        bool octets = ND == 3 && sizeof(T) == 4 && at.fused && tail_words && P.cpg % 8 == 0 && P.Cg % 8 == 0;
+        for (int k = 0; k < pc.nplans; ++k) octets = octets && !fp[k].kern;
+        if (octets) prep.zero(gin_cl, (size_t)P.N * P.C_in * P.inV * sizeof(T));
+        else if (given) prep.zero(gin, (size_t)P.N * P.C_in * P.inV * sizeof(T));
+        float* const collect = reinterpret_cast<float*>(octets ? gin_cl : gin);
         if (int rc = launch_prepare<T, S>(P, pc, prep, w, off, n_off, s)) return rc;
         // one launch per set of plans that differ in nothing but the halo
         unsigned launched = 0;
@@ -367,8 +376,8 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
                 if constexpr (sizeof(T) == 4) {
                     typedef const typename Parts<S>::Vec* Ops;
                     hipLaunchKernelGGL((fused_kernel<ND, S>(fp[k].cch, fp[k].nw)), grid, dim3(FUSED_WAVES * 64), lds, s, fp[k].Ph, alts, (const unsigned*)sel, in, off,
-                                       reinterpret_cast<Ops>(fp[k].wt), w, gout, reinterpret_cast<Ops>(gq), (const float*)bounds, gin, goff, fp[k].csplit,
-                                       (unsigned)fp[k].whole, fp[k].goff_atomic);
+                                       reinterpret_cast<Ops>(fp[k].wt), w, gout, reinterpret_cast<Ops>(gq), (const float*)bounds, collect, goff, fp[k].csplit,
+                                       (unsigned)fp[k].whole, fp[k].goff_atomic, octets ? 1 : 0);
                 }
             }
             if (int rc = check_launch(fp[k].kern ? "backward_input_halo_kernel" : "backward_fused_kernel")) return rc;
@@ -391,10 +400,24 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             hipLaunchKernelGGL((backward_data_kernel<T, ND, true, 0>), dim3((unsigned)Pg.N * Pg.tiles, (unsigned)P.DG), dim3(WG), 0, s, Pg,
                                (const T*)in_cl, off, (const T*)wt, gout, gin_cl, goff, (const unsigned*)sel, (unsigned)MAX_PLANS);
             if (int rc = check_launch("backward_data_kernel")) return rc;
-            hipLaunchKernelGGL(add_from_channels_last_kernel<T>, tgrid, tblock, 0, s, (const T*)gin_cl, gin, P.C_in, P.inV,
-                               (const unsigned*)sel, (unsigned)MAX_PLANS);
-            if (int rc = check_launch("add_from_channels_last_kernel")) return rc;
+            if (!octets) {
+                hipLaunchKernelGGL(add_from_channels_last_kernel<T>, tgrid, tblock, 0, s, (const T*)gin_cl, gin, P.C_in, P.inV,
+                                   (const unsigned*)sel, (unsigned)MAX_PLANS);
+                if (int rc = check_launch("add_from_channels_last_kernel")) return rc;
+            }
         }
+        if constexpr (sizeof(T) == 4)
+            if (octets) {
+                if (S16 && given) {                     // (the caller rounds them)
+                    given->octets = reinterpret_cast<const float*>(gin_cl);
+                    return DCN_OK;
+                }
+                const size_t blocks = ((size_t)P.N * (P.C_in / 8) * P.inV + 255) / 256;
+                auto kernel = given ? octets_to_planes_kernel<false> : octets_to_planes_kernel<true>;
+                hipLaunchKernelGGL(kernel, dim3((unsigned)(blocks < 65536 ? blocks : 65536)), dim3(256), 0, s, (const float*)gin_cl, gin, P.N, P.C_in, P.inV,
+                                   (const unsigned*)(offer_global ? sel : nullptr), (unsigned)MAX_PLANS);
+                return check_launch("octets_to_planes_kernel");
+            }
         return DCN_OK;
     }
     if constexpr (S16) {
@@ -404,6 +427,7 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
 
     // 2) grad_offset from the channels-last kernel, grad_input from the LDS-privatised scatter
     {
+        if (given) prep.zero(gin, (size_t)P.N * P.C_in * P.inV * sizeof(T));
         prep.add(PREP_BOUNDS, BOUND_BLOCKS).dst = bounds;
         PlanChoice none = {};
         if (int rc = launch_prepare<T, S>(P, none, prep, w, off, 0, s)) return rc;

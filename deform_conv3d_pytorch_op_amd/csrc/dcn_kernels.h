@@ -849,6 +849,10 @@ template <> struct LdsCell<float> {
         v0 = (float)((double)a * inv_scale);
         v1 = (float)((double)b * inv_scale);
     }
+    __device__ static inline float value_of_pair(type c, unsigned second, double inv_scale) {      // one of the two
+        const int a = (int)(unsigned)c, b = (int)(unsigned)(c >> 32) - (a >> 31);
+        return (float)((double)(second ? b : a) * inv_scale);
+    }
 };
 template <> struct LdsCell<double> {
     typedef double type;

@@ -244,6 +244,7 @@ __global__ __launch_bounds__(256) void backward_prepare_kernel(Params P, PlanCho
 struct Prep {
     PrepJobs jobs;
     unsigned blocks = 0;
+    const float* octets = nullptr;              // where a 16-bit layer's grad_input was collected, if in octets (see dcn_backward_fused.h)
     bool full = false;                          // a job too many was added: launch_prepare then refuses
     Prep() { jobs.n = 0; }
     PrepJob& add(int kind, unsigned nblocks) {

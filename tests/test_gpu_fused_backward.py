@@ -145,6 +145,32 @@ def test_samples_past_the_halo(spec, share, dtype):
         assert err <= tol + once
 
 
+# grad_input collected in octets of channels: several deformable and convolution groups, halves of octets (the 4-channel chunks of wide halos),
+# stride 2, the path without LDS tiling behind it, and a weight gradient that 16-bit storage computes on widened tensors in the same workspace
+OCTETS = [(3, 2, 24, 20, (5, 9, 10), 3, 1, 1, 1, 8, 1, 1.5), (3, 1, 16, 12, (4, 8, 9), 3, 1, 1, 1, 16, 2, 3.5), (3, 1, 16, 33, (9, 21, 19), 3, 2, 1, 1, 16, 1, 2.0),
+          (3, 2, 8, 16, (6, 9, 9), 3, 1, 1, 1, 8, 1, 12.0), (3, 1, 64, 128, (4, 9, 10), 3, 1, 1, 1, 32, 1, 1.5)]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("spec", OCTETS, ids=lambda s: "%d-%d-cpg%d-reach%g" % (s[2], s[3], s[9], s[11]))
+def test_octets(spec, dtype):
+    """Every gradient of a layer in one call; the same call with grad_input alone wanted besides grad_offset.  Bounds as in test_edges; grad_weight in
+    bfloat16: its samples are rounded too."""
+    import deform_conv3d_pytorch_op_amd as dcn
+    print("octets", spec, dtype, flush=True)
+    c = make_case(*spec, dtype=dtype, seed=38, bias=False)
+    x, off, w = (c[k].cuda().requires_grad_() for k in ("x", "off", "w"))
+    dcn.ConvOffset3dFunction.apply(x, off, w, None, c["stride"], c["pad"], c["dil"], c["cpg"], c["groups"]).backward(c["gout"].cuda())
+    d = {k: c[k].float() for k in ("x", "off", "w", "gout")}
+    want = [t.double() for t in orc.backward(d["x"], d["off"], d["w"], d["gout"], None, c["stride"], c["pad"], c["dil"], c["cpg"], c["groups"])[:3]]
+    once = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -9}[dtype]
+    got = [t.grad.cpu().double() for t in (x, off, w)] + list(_gradients(c))
+    for g, t, tol in zip(got, want + want[:2], (1e-4, 1e-5, 1e-5 + 2 * once, 1e-4, 1e-5)):
+        err = ((g - t).norm() / t.norm()).item()
+        print("  relative 2-norm error %.2e" % err, flush=True)
+        assert err <= tol + once
+
+
 def test_one_small_position_beside_ordinary_ones():
     """grad_offset of positions whose grad_output alone is tiny."""
     print("small position", flush=True)
