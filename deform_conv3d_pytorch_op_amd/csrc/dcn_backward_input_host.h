@@ -15,6 +15,14 @@ template <int ND, typename S> inline FusedKern<ND, S> fused_kernel(int cch, int 
     return cch == 8 ? backward_fused_kernel<ND, 8, 8, S> : cch == 4 ? backward_fused_kernel<ND, 4, 8, S> : nullptr;
 }
 
+// The first element of grad_offset that belongs to an item from `whole` on: items are (deformable group, sample, block), blocks fastest, the
+// tensor is [sample][deformable group].
+template <int ND> inline size_t first_split_offset(const Params& P, long long whole) {
+    const long long per_group = (long long)P.N * P.tiles, dg = whole / per_group, n = whole % per_group / P.tiles;
+    if (dg >= P.DG) return (size_t)P.N * P.DG * P.kV * ND * P.outV;
+    return (size_t)(dg == P.DG - 1 ? n * P.DG + dg : dg) * P.kV * ND * P.outV;
+}
+
 // S = T: the float32 / float64 operator.  S = Bf16 / Fp16 (T = float): input, weight, offset and
 // grad_output are in that storage format (the gradients are float), and only the fused kernels serve
 // them; where they cannot, *declined is set and nothing is launched: the caller then widens the tensors and
@@ -324,9 +332,14 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
             job.dst = gq;
         }
         prep.add(PREP_BOUNDS, BOUND_BLOCKS).dst = bounds;
-        bool any_atomic = false;
-        for (int k = 0; k < pc.nplans; ++k) any_atomic = any_atomic || fp[k].zero_goff;
-        if (any_atomic) prep.zero(goff, n_off * sizeof(T));
+        // grad_offset is cleared from the first element that is added to: where only the last round's items are split, the last samples of the last
+        // deformable group.
+        size_t added = n_off;
+        for (int k = 0; k < pc.nplans; ++k) {
+            const size_t from = !fp[k].zero_goff ? n_off : fp[k].goff_atomic ? 0 : first_split_offset<ND>(fp[k].Ph, fp[k].whole);
+            if (from < added) added = from;
+        }
+        if (added < n_off) prep.zero(goff + added, (n_off - added) * sizeof(T));
         // Where the fused kernel collects grad_input: in octets of channels in the place of the channels-last gradient, or in the tensor itself.  In 3-D
         // the last launch of the path without LDS tiling, or the rounding of a 16-bit layer's gradients, brings them to the tensor, and a halo
         // has 8 to 18 voxels to a position.  In 2-D it has two: steps of 256 -> 256, 3x3, 8 x 56 x 56 874 us in the tensor, 883 in octets (one launch more),

@@ -1,6 +1,7 @@
 // Host code of the library's planning, run on the CPU by test_host_plans.py (no GPU, nothing is launched):
 //   host_plans <what> <seed> <count>     exit status 0 when the property holds for `count` random layers
 #include "../deform_conv3d_pytorch_op_amd/csrc/dcn_forward_host.h"
+#include "../deform_conv3d_pytorch_op_amd/csrc/dcn_backward_input_host.h"
 
 #include <random>
 
@@ -75,6 +76,21 @@ static bool weight64(const Params& P, int& hits) {
            align256((size_t)P.N * P.C_in * P.inV * 8) + align256((size_t)P.N * P.C_out * P.outV * 8) + align256(splits * P.kV * P.C_out * P.Cg * 8) +
                align256((size_t)P.N * last_strips(P.outV) * P.C_out * 8);
 }
+// What is cleared of grad_offset reaches every item that is added to, and starts with one of them where they lie in the last deformable group.
+static bool added(const Params& Pin, int& hits) {
+    Params P = Pin;
+    P.tiles = pick(1, 5);
+    const long long per_group = (long long)P.N * P.tiles, items = per_group * P.DG, whole = pick(0, (int)items);
+    const size_t slab = (size_t)P.kV * 3 * P.outV, all = slab * P.N * P.DG, from = first_split_offset<3>(P, whole);
+    size_t least = all;
+    for (long long i = whole; i < items; ++i) {
+        const size_t at = slab * (size_t)(i % per_group / P.tiles * P.DG + i / per_group);
+        if (at < least) least = at;
+    }
+    const bool last = whole >= per_group * (P.DG - 1);
+    hits += last && whole < items;
+    return from <= least && (!last || from == least);
+}
 static bool layouts(const Params& P, int& hits) {
     int all[4] = {0, 0, 0, 0};
     const bool ok = layout<float, float>(P, all[0]) && layout<float, Bf16>(P, all[1]) && layout<float, Fp16>(P, all[2]) && layout<double, double>(P, all[3]);
@@ -117,7 +133,7 @@ int main(int argc, char** argv) {
         const int nd = pick(2, 3);
         if (!random_layer(nd, P)) continue;
         ++layers;
-        const bool ok = what == "noalloc" ? noalloc(P, hits) : what == "layout" ? layouts(P, hits) : what == "weight64" ? weight64(P, hits) : what == "native16" ? (nd == 3 ? native16<3>(P, hits) : native16<2>(P, hits)) : false;
+        const bool ok = what == "noalloc" ? noalloc(P, hits) : what == "layout" ? layouts(P, hits) : what == "weight64" ? weight64(P, hits) : what == "added" ? added(P, hits) : what == "native16" ? (nd == 3 ? native16<3>(P, hits) : native16<2>(P, hits)) : false;
         if (!ok) {
             printf("%s: %d-D, C_in %d, C_out %d, G %d, cpg %d, k %d %d %d, stride %d %d %d, dil %d %d %d\n", what.c_str(), nd, P.C_in, P.C_out, (int)P.G, (int)P.cpg, (int)P.k[0],
                    (int)P.k[1], (int)P.k[2], P.stride[0], P.stride[1], P.stride[2], P.dil[0], P.dil[1], P.dil[2]);

@@ -16,7 +16,7 @@ def probe(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("what", ["noalloc", "native16", "jobs", "layout", "weight64"])
+@pytest.mark.parametrize("what", ["noalloc", "native16", "jobs", "layout", "weight64", "added"])
 def test_rule(probe, what):
     r = subprocess.run([probe, what, "7", "20000"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
