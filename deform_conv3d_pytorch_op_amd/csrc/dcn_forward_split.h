@@ -259,8 +259,10 @@ __device__ inline bool stage_halo(const Params& P, const HaloPlan& H, const Tile
     const size_t step = (size_t)P.inV * sizeof(S);
     // Items of a thread in flight, the last ones too: a pass waits for memory ceil(items / U) times.  (Four in a loop unrolled so, and the remainder one by
     // one: 256 -> 256, 2-D, steps 880 -> 858 us, the ragged 48 -> 80 in 3-D 398 -> 390.  Of 128 -> 128 at stride 1 2 2, eight wavefronts, 17 items: 2, 3, 4, 6
-    // in flight 4535, 4497, 4511, 4476; 64 -> 64 in 3-D, sixteen wavefronts, inference: 469, 471, 481, 471.)
-    constexpr int U = WGS >= 1024 ? 3 : 6;
+    // in flight 4535, 4497, 4511, 4476; 64 -> 64 in 3-D, sixteen wavefronts, inference: 469, 471, 481, 471.  With six, layers of few channels repeat more loads
+    // than they have: inference of 10 -> 41 in groups of 5, 3x3, 4 x 174 x 138, 53.4 us before any of this, 58.8 with six, 53.3 with three; 44 -> 43 in groups of 11,
+    // 1x1x1, 8 x 30 x 28 x 53, 166, 182, 167; 70 drawn layers 1.046 times as fast as before with six, 1.058 with three.)
+    constexpr int U = 3;
     bool bad = false;
     // (no load is masked: a masked one is waited for on its own; past the last item and past the last channel a load is repeated)
     auto stage = [&](int it0, auto count) {
