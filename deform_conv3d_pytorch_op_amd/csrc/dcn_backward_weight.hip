@@ -68,23 +68,22 @@ SplitFn<S> split_kernel_of(int MT, int LW, bool plain) {
         if (plain) return MT == 4 ? backward_weight_split_kernel<ND, 4, 32, S, QUAD, true> : backward_weight_split_kernel<ND, 2, 32, S, QUAD, true>;
     if constexpr (sizeof(S) == 4)
         if (MT == 8) return backward_weight_split_kernel<ND, 8, 32, S, QUAD>;
+    constexpr bool QUAD8 = QUAD && !(ND == 3 && std::is_same<S, Bf16>::value);      // (see split_quad)
     switch (MT * 100 + LW) {
         case 108: return backward_weight_split_kernel<ND, 1, 8, S, QUAD>;
         case 116: return backward_weight_split_kernel<ND, 1, 16, S, QUAD>;
-        case 208: return backward_weight_split_kernel<ND, 2, 8, S, QUAD>;
+        case 208: return backward_weight_split_kernel<ND, 2, 8, S, QUAD8>;
         case 216: return backward_weight_split_kernel<ND, 2, 16, S, QUAD>;
         case 232: return backward_weight_split_kernel<ND, 2, 32, S, QUAD>;
-        case 408: return backward_weight_split_kernel<ND, 4, 8, S, QUAD>;
+        case 408: return backward_weight_split_kernel<ND, 4, 8, S, QUAD8>;
         case 416: return backward_weight_split_kernel<ND, 4, 16, S, QUAD>;
         default: return backward_weight_split_kernel<ND, 4, 32, S, QUAD>;
     }
 }
-// 16-byte loads where every lane's channels of a voxel are aligned to them, but not for float32 in 3-D (see the kernel).
 template <int ND, typename S>
 SplitFn<S> split_kernel(const Params& P, int MT, int LW, bool plain) {
-    constexpr int CL = 16 / sizeof(S);
     if constexpr (ND == 3 && sizeof(S) == 4) return split_kernel_of<ND, S, false>(MT, LW, plain);
-    else return P.C_in % CL == 0 && P.cpg % CL == 0 && P.Cg % CL == 0 ? split_kernel_of<ND, S, true>(MT, LW, plain) : split_kernel_of<ND, S, false>(MT, LW, plain);
+    else return split_quad<ND, S>(P, MT, LW) ? split_kernel_of<ND, S, true>(MT, LW, plain) : split_kernel_of<ND, S, false>(MT, LW, plain);
 }
 // Lanes to a tap: 16 or 8 where a segment fits them and that makes fewer items, at 1.05 and 1.2 items for one of 32: eight lanes read 32
 // bytes of a corner.  (Longer segments read their cache lines in parts then: 80 -> 96, 3-D, 23 600 positions 406 us a step with 32, 431 with 16.)  Layers of up to 32 output channels, too, if it takes a third off them; the

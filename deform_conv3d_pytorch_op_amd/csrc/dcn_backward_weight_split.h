@@ -89,7 +89,7 @@ __device__ inline void swap_lanes_registers(float v[4]) {
 
 // MT row tiles to a workgroup.  LW lanes to a tap: an item is 32 / LW taps of LW channels (pairs).  PLAIN: a plain convolution (off is null): samples at integer coordinates are their low corner alone.
 // Grid: igroups * mchunks * G * nsplit workgroups.  The items of a convolution group: taps of a channel tile, taps fastest.
-// QUAD: 16 bytes of a corner to a lane -- see the top of the file; channels and segments in multiples of four (16-bit storage: eight).
+// QUAD: 16 bytes of a corner to a lane -- see the top of the file and split_quad; channels and segments in multiples of four (16-bit storage: eight).
 template <int ND, int MT, int LW, typename S, bool QUAD, bool PLAIN = false>
 __global__ __launch_bounds__(WG, split_waves<S>(MT)) void backward_weight_split_kernel(Params P, const S* __restrict__ in_cl, const S* __restrict__ off,
                                                                                          const S* __restrict__ gout,
@@ -419,6 +419,20 @@ __global__ __launch_bounds__(WG, split_waves<S>(MT)) void backward_weight_split_
             if (m < P.M && c0 + column(u) < ce && tap < P.kV) pt[(size_t)m * P.Cg + column(u)] = x[r];
         }
     }
+}
+
+// 16-byte loads (QUAD) where every lane's channels of a voxel are aligned to them, but not for
+// - float32 in 3-D (see the top of the file),
+// - bfloat16 in 3-D with eight lanes to a tap and more than one row tile, which spills 69 registers with them: backward passes to the weight of 16 such layers, us with 4 bytes
+//   to a lane : 16 -- 64 -> 64 in groups of 8, 4 x 16 x 28 x 28, 268 : 384; 16 -> 48 in groups of 8, 4 x 16 x 56 x 56, 210 : 351; never less than 1.19 times as long.  (One
+//   row tile 1.02 to 1.25 times as fast with 16, binary16 1.00 to 1.22.)
+// float32 in 2-D with fewer than 32 lanes to a tap, 680 layers: 0.95 to 1.28 times as fast with them, 1.01 on average, one row tile 1.08; no line by channels or
+// row tiles does better.  16-bit storage in 2-D with fewer than 32 lanes: 1.00 to 1.30, 1.05 on average.
+template <int ND, typename S>
+inline bool split_quad(const Params& P, int MT, int LW) {
+    constexpr int CL = 16 / sizeof(S);
+    if (P.C_in % CL || P.cpg % CL || P.Cg % CL || (ND == 3 && sizeof(S) == 4)) return false;
+    return !(ND == 3 && std::is_same<S, Bf16>::value && LW == 8 && MT > 1);
 }
 
 }  // namespace dcn

@@ -2,6 +2,7 @@
 //   host_plans <what> <seed> <count>     exit status 0 when the property holds for `count` random layers
 #include "../deform_conv3d_pytorch_op_amd/csrc/dcn_forward_host.h"
 #include "../deform_conv3d_pytorch_op_amd/csrc/dcn_backward_input_host.h"
+#include "../deform_conv3d_pytorch_op_amd/csrc/dcn_backward_weight_split.h"
 
 #include <random>
 
@@ -98,6 +99,19 @@ static bool layouts(const Params& P, int& hits) {
     return ok;
 }
 
+// Where the weight gradient reads 16 bytes of a corner to a lane.
+static bool quads() {
+    auto layer = [](int c_in, int cpg, int c_out) {
+        Params P = {};
+        P.N = 1; P.C_in = c_in; P.C_out = c_out; P.G = 1; P.cpg = cpg; P.DG = c_in / cpg; P.M = c_out; P.Cg = c_in;
+        return P;
+    };
+    const Params g8 = layer(64, 8, 64), c64 = layer(64, 64, 64), odd = layer(20, 20, 64);
+    return !split_quad<3, Bf16>(g8, 2, 8) && !split_quad<3, Bf16>(layer(16, 16, 48), 2, 8) && split_quad<3, Bf16>(layer(64, 8, 24), 1, 8) && split_quad<3, Fp16>(g8, 2, 8) &&
+           split_quad<2, Bf16>(g8, 2, 8) && split_quad<3, Bf16>(c64, 2, 32) && split_quad<3, Bf16>(layer(32, 32, 64), 2, 16) && !split_quad<3, Bf16>(odd, 2, 16) &&
+           !split_quad<3, float>(c64, 2, 32) && split_quad<2, float>(c64, 2, 32) && split_quad<2, float>(layer(256, 256, 256), 8, 32) && split_quad<2, float>(g8, 2, 8) &&
+           split_quad<2, float>(odd, 2, 32) && !split_quad<2, float>(layer(42, 14, 64), 2, 16);
+}
 int main(int argc, char** argv) {
     if (argc != 4) return 2;
     const std::string what = argv[1];
@@ -121,6 +135,7 @@ int main(int argc, char** argv) {
         }
         return 0;
     }
+    if (what == "quad") return quads() ? 0 : 1;
     if (what == "budget") {         // of any DCN_SCATTER_BUDGET_KB: what a CU has beside the 2120 and 100 bytes that the kernels declare; 72 stays 72
         const size_t cu = 160 * 1024, kb72 = 72 * 1024;
         return fused_budget() + 2120 <= cu && scatter_budget() + 100 <= cu && fused_budget() >= kb72 && scatter_budget() >= kb72 &&

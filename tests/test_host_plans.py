@@ -22,6 +22,13 @@ def test_rule(probe, what):
     assert r.returncode == 0, r.stdout
 
 
+@pytest.mark.parametrize("what", ["quad"])
+def test_measured_line(probe, what):
+    """Which variant of a kernel a layer takes, where the times with either are known."""
+    r = subprocess.run([probe, what, "7", "1"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
+    assert r.returncode == 0, r.stdout
+
+
 def test_divisors(probe):
     r = subprocess.run([probe, "div", "7", "2000"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
     assert r.returncode == 0, r.stdout
