@@ -90,10 +90,6 @@ SplitFn<S> split_kernel(const Params& P, int MT, int LW, bool plain) {
 // first threshold counts items of 32 lanes.  50 training layers, us per step, 32 lanes (or the other
 // kernels) : this: 1.058 times as fast on average, at worst 0.994; 16 -> 38 in groups of 4, 3-D, two samples of 16 700 positions in bfloat16 464 : 322; 20 -> 339 in
 // groups of 5, 7200 positions 301 : 245; 16 -> 14, 165 000 positions in bfloat16 734 : 602; 24 -> 36 in groups of 6, 10 600 positions 184 : 162.
-// Estimated time of a split, in us: a wavefront's share of the slabs, 4 to a slab, times the rounds of workgroups -- of less than one, the
-// part a workgroup takes when its CU holds no other, and the rest with what shares the CU -- and the partial tiles.  Backward passes
-// of 60 layers, the other line's time over this one's: 0.2 for 0.4 1.03 (at worst 1.13), 0.6 1.013 (1.07), 1 1.005 (1.04); 1 for 4 1.019 (1.12), 2 1.005,
-// 8 and 16 1.001 (1.03).  A plain convolution is planned by the occupancy of the kernel with offsets (24 layers by its own: 1.0015, at worst 1.02).
 struct SplitPlan { int MT, LW, mchunks, igroups, nsplit; };     // nsplit 0: not a layer for it, or no room
 template <int ND, typename S>
 SplitPlan split_plan(const Params& P, bool off, size_t room) {
@@ -116,35 +112,28 @@ SplitPlan split_plan(const Params& P, bool off, size_t room) {
     c.mchunks = ((P.M + 31) / 32 + c.MT - 1) / c.MT;
     c.igroups = (items + WAVES - 1) / WAVES;
     if ((P.M <= 32 && least > 0.67 * whole) || items < WAVES) return c;
-    double resident = (double)resident_workgroups(reinterpret_cast<const void*>(split_kernel<ND, S>(P, c.MT, c.LW, false)), WG, 0);
+    auto resident = [&](int MT) { return (double)resident_workgroups(reinterpret_cast<const void*>(split_kernel<ND, S>(P, MT, c.LW, false)), WG, 0); };
     const long long nslabs = (long long)P.N * (row_steps(P.outV) / 2);
-    double other = (double)c.igroups * c.mchunks * P.G;
-    if ((double)whole * c.mchunks * P.G * (double)nslabs < 2.5 * WAVES * resident) return c;
-    // Eight row tiles in float32 where they hold no more padding than fours do and leave work for the wavefronts that then fit (single taps and
-    // few channels: the corner reads are not what bounds them).
+    const double fit = resident(c.MT), other = (double)c.igroups * P.G;
+    if ((double)whole * c.mchunks * P.G * (double)nslabs < 2.5 * WAVES * fit) return c;
+    const size_t one = (size_t)P.kV * P.C_out * P.Cg * sizeof(float);
+    const long long most = (long long)(room / one);
+    SplitCost best = split_cost(other * c.mchunks, fit, nslabs, most, one);
+    // Eight row tiles in float32, where they hold no more padding than fours do and leave work for the wavefronts that then fit, if that is faster by the estimate.
     const int mtiles = (P.M + 31) / 32, fewer = (mtiles + 7) / 8;
     if (sizeof(S) == 4 && off && c.LW == 32 && fewer * 8 == c.mchunks * 4) {
-        const double fit = (double)resident_workgroups(reinterpret_cast<const void*>(split_kernel<ND, S>(P, 8, 32, false)), WG, 0);
-        if ((double)whole * fewer * P.G * (double)nslabs >= 2.5 * WAVES * fit) {
-            c.MT = 8;
-            c.mchunks = fewer;
-            resident = fit;
-            other = (double)c.igroups * fewer * P.G;
+        const double fit8 = resident(8);
+        if ((double)whole * fewer * P.G * (double)nslabs >= 2.5 * WAVES * fit8) {
+            const SplitCost eight = split_cost(other * fewer, fit8, nslabs, most, one);
+            if (eight_tiles_pay(ND, best, eight)) {
+                best = eight;
+                c.MT = 8;
+                c.mchunks = fewer;
+            }
         }
     }
-    const size_t one = (size_t)P.kV * P.C_out * P.Cg * sizeof(float);
-    long long most = (long long)(room / one);
-    if (most > 256) most = 256;
-    if (most > nslabs) most = nslabs;
-    double best = 0;
-    for (long long s = 1; s <= most; ++s) {
-        const double load = other * (double)s / resident, rounds = load > 1 ? ceil(load) : 0.4 + 0.6 * load;
-        const double t = (double)((nslabs + s - 1) / s) * rounds * 4 + (double)s * (double)one * 2 / 8e6;
-        if (s > 1 && t >= best) continue;
-        best = t;
-        c.nsplit = (int)s;
-    }
-    if (other * c.nsplit > 2147483647.0) c.nsplit = 0;
+    c.nsplit = best.nsplit;
+    if (other * c.mchunks * c.nsplit > 2147483647.0) c.nsplit = 0;
     return c;
 }
 

@@ -31,18 +31,19 @@
 // 3x3, 8 x 56 x 56: 332 -> 240; 512 -> 512 in two groups, 3x3, 4 x 28 x 28: 105 -> 80; 128 -> 128, 3x3x3, 2 x 16 x 56 x 56
 // (stride 2): 1022 -> 860; 64 -> 64 as above: 633 -> 600; 64 -> 64, 3x3, no offsets, 25 088 positions: 33 -> 25.
 // The preparing launch pays 2 to 20 us of it back (three halves of the bytes of a channels-last copy).
-// float32 layers of more than 128 output channels to a group: eight row tiles, so that 256 of them share the corner reads of a sample, at two
-// wavefronts per SIMD instead of three: 256 -> 256 as above 228 -> 208 (steps of the layer 900 -> 889 us), 512 -> 512 in two groups 91 -> 80 (327 -> 323).  In 16-bit
+// float32 layers of more than 128 output channels to a group, where they pay (eight_tiles_pay): eight row tiles, so that 256 of them share the corner reads
+// of a sample, at two wavefronts per SIMD instead of three: 256 -> 256 as above 228 -> 208 (steps of the layer 900 -> 889 us).  In 16-bit
 // storage a lane holds two column tiles and eight row tiles leave one wavefront per SIMD: steps of 256 -> 256 in binary16 497 -> 514 us, so it keeps four.
 // Where every lane's channels are aligned to it (QUAD), eight lanes read 16 bytes of a corner each and the wavefront eight positions at a time: a
 // quarter of the load instructions -- of a line or a half to a lane group, one that hits the L1 takes 7.5 ns a CU for 1 KB, of 4 bytes to a lane 2.9 for 256
 // bytes -- and of the records, and the weighted sums change places with the positions (swap_lanes_registers) before the
 // contraction.  2-D and 16-bit storage: us of the kernel alone, 4 bytes -> 16: 256 -> 256 in binary16 118 -> 95 (step 466 -> 433),
-// in float32 208 -> 193, 512 -> 512 in two groups 80 -> 77, without offsets 26.7 -> 23.7, 64 -> 64 in 3-D in bfloat16 333 -> 289 (step 1752 -> 1717).  Not float32 in 3-D, where the lines of eight positions with eight corners each, of every wavefront, turn the L1 over before their
+// in float32 208 -> 193, without offsets 26.7 -> 23.7, 64 -> 64 in 3-D in bfloat16 333 -> 289 (step 1752 -> 1717).  Not float32 in 3-D, where the lines of eight positions with eight corners each, of every wavefront, turn the L1 over before their
 // neighbours come back to them: steps of 64 -> 64 2478 -> 2598 us, of 128 -> 128 4525 -> 5058.
 // 16-bit storage, against backward_weight16_kernel, which samples once for every 64 output channels: 256 -> 256 in float16 150 -> 116,
 // 64 -> 64 in 3-D in bfloat16 361 -> 326.
 #pragma once
+#include <cmath>
 #include "dcn_forward_split.h"
 
 namespace dcn {
@@ -433,6 +434,30 @@ inline bool split_quad(const Params& P, int MT, int LW) {
     constexpr int CL = 16 / sizeof(S);
     if (P.C_in % CL || P.cpg % CL || P.Cg % CL || (ND == 3 && sizeof(S) == 4)) return false;
     return !(ND == 3 && std::is_same<S, Bf16>::value && LW == 8 && MT > 1);
+}
+
+// Estimated time of a split, in us: a wavefront's share of the slabs, 4 to a slab, times the rounds of workgroups -- of less than one, the
+// part a workgroup takes when its CU holds no other, and the rest with what shares the CU -- and the partial tiles (of `one` bytes a split).  Backward passes
+// of 60 layers, the other line's time over this one's: 0.2 for 0.4 1.03 (at worst 1.13), 0.6 1.013 (1.07), 1 1.005 (1.04); 1 for 4 1.019 (1.12), 2 1.005,
+// 8 and 16 1.001 (1.03).  A plain convolution is planned by the occupancy of the kernel with offsets (24 layers by its own: 1.0015, at worst 1.02).
+struct SplitCost { double slabs, tiles; int nsplit; };  // nsplit 0: no room
+inline SplitCost split_cost(double workgroups, double resident, long long nslabs, long long most, size_t one) {
+    SplitCost best = {0, 0, 0};
+    if (most > 256) most = 256;
+    if (most > nslabs) most = nslabs;
+    for (long long s = 1; s <= most; ++s) {
+        const double load = workgroups * (double)s / resident, rounds = load > 1 ? ceil(load) : 0.4 + 0.6 * load;
+        const SplitCost c = {(double)((nslabs + s - 1) / s) * rounds * 4, (double)s * (double)one * 2 / 8e6, (int)s};
+        if (s == 1 || c.slabs + c.tiles < best.slabs + best.tiles) best = c;
+    }
+    return best;
+}
+// Whether eight row tiles to a workgroup are faster than four, by the estimates of either: a slab of eight, two wavefronts to a SIMD, takes 1.18 times as long as one of four, three to a
+// SIMD, in 3-D and 1.22 times in 2-D, where the corner reads are a smaller part.  Backward passes to the weight of 504 layers of more than 128 output channels: by this line 1.0022
+// times the time of the better one on average, always eight 1.013 (at worst 1.22: 950 -> 415 to each of two groups, 3x3, two samples of 26 x 20, 233 us : 284; 86 -> 249, 3x3, two of 67 x 99,
+// 77 : 91; 128 -> 256, 1x1x1, 4 x 16 x 56 x 56, 384 : 406), always four 1.08 (64 -> 256, 3x3x3, 4 x 16 x 56 x 56, 1727 : 1415).
+inline bool eight_tiles_pay(int nd, const SplitCost& four, const SplitCost& eight) {
+    return eight.nsplit > 0 && eight.slabs * (nd == 3 ? 1.18 : 1.22) + eight.tiles < four.slabs + four.tiles;
 }
 
 }  // namespace dcn

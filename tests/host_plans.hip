@@ -112,6 +112,24 @@ static bool quads() {
            !split_quad<3, float>(c64, 2, 32) && split_quad<2, float>(c64, 2, 32) && split_quad<2, float>(layer(256, 256, 256), 8, 32) && split_quad<2, float>(g8, 2, 8) &&
            split_quad<2, float>(odd, 2, 32) && !split_quad<2, float>(layer(42, 14, 64), 2, 16);
 }
+// Eight row tiles to a workgroup of the weight gradient or four: what the estimate says of layers whose times with either are known.
+static bool row_tiles() {
+    struct Layer { int nd, c_in, c_out, G, taps, N, positions; bool eight; };      // channels of one group, one segment each
+    const Layer layers[] = {
+        {3, 64, 256, 1, 27, 4, 50176, true},   {3, 64, 256, 1, 27, 2, 12544, true},  {3, 128, 256, 1, 27, 1, 6272, true},  {3, 256, 256, 1, 1, 4, 50176, true},
+        {3, 135, 142, 1, 27, 1, 81700, true},  {3, 256, 256, 1, 27, 1, 1568, false}, {3, 128, 256, 1, 27, 1, 1568, false}, {3, 114, 253, 1, 27, 4, 693, false},
+        {2, 256, 256, 1, 9, 8, 3136, true},    {2, 128, 256, 1, 9, 8, 3136, true},   {2, 512, 256, 2, 9, 8, 3136, true},   {2, 256, 256, 1, 9, 4, 784, false},
+        {2, 128, 256, 1, 9, 2, 3136, false},   {2, 256, 256, 1, 1, 8, 3136, false},  {2, 950, 415, 2, 9, 2, 520, false},   {2, 86, 249, 1, 9, 2, 6633, false},
+    };
+    for (const Layer& l : layers) {
+        const int items = (l.c_in + 31) / 32 * l.taps, groups = (items + 3) / 4 * l.G, tiles = (l.c_out + 31) / 32;
+        const long long slabs = (long long)l.N * ((l.positions + 31) / 32);
+        const size_t one = (size_t)l.taps * l.c_out * l.G * l.c_in * sizeof(float);
+        const SplitCost four = split_cost((double)groups * ((tiles + 3) / 4), 768, slabs, 256, one), eight = split_cost((double)groups * ((tiles + 7) / 8), 512, slabs, 256, one);
+        if (eight_tiles_pay(l.nd, four, eight) != l.eight) return printf("%d-D, %d -> %d: %g %g\n", l.nd, l.c_in, l.c_out, four.slabs + four.tiles, eight.slabs + eight.tiles), false;
+    }
+    return true;
+}
 int main(int argc, char** argv) {
     if (argc != 4) return 2;
     const std::string what = argv[1];
@@ -136,6 +154,7 @@ int main(int argc, char** argv) {
         return 0;
     }
     if (what == "quad") return quads() ? 0 : 1;
+    if (what == "rows") return row_tiles() ? 0 : 1;
     if (what == "budget") {         // of any DCN_SCATTER_BUDGET_KB: what a CU has beside the 2120 and 100 bytes that the kernels declare; 72 stays 72
         const size_t cu = 160 * 1024, kb72 = 72 * 1024;
         return fused_budget() + 2120 <= cu && scatter_budget() + 100 <= cu && fused_budget() >= kb72 && scatter_budget() >= kb72 &&
