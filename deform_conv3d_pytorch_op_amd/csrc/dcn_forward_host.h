@@ -37,10 +37,10 @@ inline int even_chunk(const Params& P, int cchunk, int step, int fsplit) {
 // The plain convolution on a kernel of its own; *done says whether it took the layer.
 inline int plain_forward(Params P, const float* in, const float* w, const float* bias, float* out, void* ws, size_t ws_bytes, hipStream_t s, bool* done) {
     *done = false;
-    const int mtiles = (P.M + 31) / 32;
-    int mw = mtiles > 2 ? 4 : mtiles, rw = mtiles > 4 ? 2 : 1;
-    P.mchunks = (mtiles + mw * rw - 1) / (mw * rw);
-    P.Mp = P.mchunks * mw * rw * 32;
+    const PlainRows rows = plain_rows(P.M, P.kV);
+    const int mw = rows.mw, rw = rows.rw;
+    P.mchunks = rows.mchunks;
+    P.Mp = rows.mchunks * mw * rw * 32;
     if (!plan_halo<float, 2>(P, (size_t)1 << 30, 0, 64, 1, PLAIN_COLS, false, FG, nullptr, 1, false)) return DCN_OK;
     // Channels at a time: two workgroups to a CU.
     while (P.cchunk > FG && plain_lds(P.hvol, P.cchunk) > MAX_FORWARD_LDS / 2) P.cchunk -= FG;

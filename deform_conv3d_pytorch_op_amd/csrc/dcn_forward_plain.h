@@ -23,6 +23,20 @@ constexpr int PLAIN_COLS = 2;                           // position tiles of a w
 __host__ __device__ inline constexpr int plain_row(int channels) { return (channels / FG) | 1; }
 __host__ inline size_t plain_lds(int hvol, int channels) { return (size_t)Parts<float>::NP * hvol * plain_row(channels) * 16; }
 
+// Wavefronts along the rows, row tiles of each, chunks of rows.  Two row tiles to a wavefront, for half the staging and half the reads of values, where that makes no more
+// rows than one does, and of a single tap, which is all staging, up to a quarter more.  293 layers of nine to twelve and of seventeen to twenty row tiles, us of the forward call
+// with two : one -- 92 -> 339, 3x3, 82 x 112, 88 : 53; 225 -> 379, 3x3, two samples of 18 x 210, 195 : 113; 20 -> 591, 3x3, 16 x 17 x 16, 31 : 21; on average 1.22 : 1 and, from
+// seventeen on, 1.07 : 1, at worst 0.90 : 1; single taps 1.09 : 1 up to twelve, from seventeen on 0.95 : 1 (13 -> 592, four of 106 x 219, 76 : 88).
+struct PlainRows { int mw, rw, mchunks; };
+inline PlainRows plain_rows(int M, int taps) {
+    const int tiles = (M + 31) / 32, four = (tiles + 3) / 4 * 4, eight = (tiles + 7) / 8 * 8;
+    PlainRows r;
+    r.mw = tiles > 2 ? 4 : tiles;
+    r.rw = tiles > 4 && (eight == four || (taps == 1 && eight * 4 <= four * 5)) ? 2 : 1;
+    r.mchunks = (tiles + r.mw * r.rw - 1) / (r.mw * r.rw);
+    return r;
+}
+
 // Grid: N * tiles * G * mchunks workgroups of PLAIN_COLS * MW wavefronts; P.cchunk a multiple of eight.
 template <int RW>
 __global__ __launch_bounds__(512) void plain_conv_kernel(Params P, const float* __restrict__ in, const Parts<float>::Vec* __restrict__ Wq,

@@ -130,6 +130,16 @@ static bool row_tiles() {
     }
     return true;
 }
+// Rows of the plain convolution: chunks hold them all, with two row tiles to a wavefront only where that is no more padding (single taps: a quarter more).
+static bool plain_row_chunks() {
+    for (int M = 1; M <= 2000; ++M)
+        for (int taps : {1, 9}) {
+            const PlainRows r = plain_rows(M, taps);
+            const int tiles = (M + 31) / 32, held = r.mw * r.rw * r.mchunks, one = tiles > 2 ? (tiles + 3) / 4 * 4 : tiles;
+            if (held < tiles || (taps > 1 && held != one) || held * 4 > one * 5 || r.mw * r.rw > 8) return printf("%d rows, %d taps\n", M, taps), false;
+        }
+    return plain_rows(256, 9).rw == 2 && plain_rows(257, 9).rw == 1 && plain_rows(339, 1).rw == 1 && plain_rows(591, 9).rw == 1 && plain_rows(591, 1).rw == 2;
+}
 int main(int argc, char** argv) {
     if (argc != 4) return 2;
     const std::string what = argv[1];
@@ -154,6 +164,7 @@ int main(int argc, char** argv) {
         return 0;
     }
     if (what == "quad") return quads() ? 0 : 1;
+    if (what == "plain_rows") return plain_row_chunks() ? 0 : 1;
     if (what == "rows") return row_tiles() ? 0 : 1;
     if (what == "budget") {         // of any DCN_SCATTER_BUDGET_KB: what a CU has beside the 2120 and 100 bytes that the kernels declare; 72 stays 72
         const size_t cu = 160 * 1024, kb72 = 72 * 1024;

@@ -40,7 +40,7 @@ def test_gradients(spec, dtype):
 # layer's size (DCN_PLAIN=2, read once per process).
 PLAIN = [(1, 8, 1, (9, 9), 3, 1, 1, 1, 1), (2, 5, 33, (8, 17), 1, 1, 0, 1, 1), (1, 70, 64, (7, 24), 3, 2, 1, 1, 1), (1, 24, 130, (11, 9), (3, 2), 1, (1, 0), (2, 3), 1),
          (1, 136, 260, (10, 12), 2, 1, 1, 1, 1), (2, 18, 36, (13, 8), 5, (1, 2), 2, 1, 2), (1, 64, 96, (30, 31), 3, 1, 8, 7, 1), (1, 200, 40, (16, 16), 3, 1, 1, 1, 1),
-         (1, 12, 300, (9, 10), 3, 1, 2, 2, 4), (3, 1, 1, (1, 1), 1, 1, 0, 1, 1), (1, 40, 16, (20, 22), 7, 1, 3, 1, 1)]
+         (1, 12, 300, (9, 10), 3, 1, 2, 2, 4), (3, 1, 1, (1, 1), 1, 1, 0, 1, 1), (1, 40, 16, (20, 22), 7, 1, 3, 1, 1), (1, 16, 520, (9, 9), 1, 1, 0, 1, 1)]
 
 
 def plain_cases():
