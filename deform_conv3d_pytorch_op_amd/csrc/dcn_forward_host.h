@@ -51,15 +51,7 @@ inline int plain_forward(Params P, const float* in, const float* w, const float*
         while (P.cchunk > 3 * FG && plain_lds(P.hvol, P.cchunk) > MAX_FORWARD_LDS / 4) P.cchunk -= FG;
     const size_t lds = plain_lds(P.hvol, P.cchunk);
     if (lds > MAX_FORWARD_LDS || ws_bytes < split_weight_bytes<float>(P, P.Mp) || wgs > 0x7fffffffLL || !plain_conv()) return DCN_OK;
-    // A wavefront takes some 0.26 us to a step of sixteen reduction slots, whatever the others do: long chains want enough wavefronts for the
-    // device, short ones three to four CUs.  Others keep the kernels that share a position or its channels among wavefronts.  us of
-    // the forward call, those kernels : this one, 43 layers: with fewer than 1400 wavefronts and more than 40 steps -- 512 -> 32, 3x3, 25 x 24 x 24 (450,
-    // 320 steps) 68 : 118; 128 -> 128, 28 x 28, four samples (512, 80) 30 : 39; 256 -> 64, 56 x 56, four (784, 160) 55 : 61 --, above either line 64 -> 64,
-    // 56 x 56 (196, 40) 21.9 : 20.4; 16 -> 128, 40 x 40, two (400, 10) 20.3 : 13.8; 256 -> 128, 28 x 28, sixteen (2048, 160) 108 : 79; 100 -> 100, 5x5, 60 x 60,
-    // four (2048, 169) 139 : 77; at worst 11.3 : 12.7 (24 -> 24, 60 x 60, two samples).
-    const int steps = (P.Cg + FG - 1) / FG * ((P.kV + 1) / 2);
-    const long long waves = wgs * PLAIN_COLS * mw;
-    if (plain_conv() != 2 && waves * 2 < 11 * cu_count() && (steps > 40 || waves * 4 < 3 * cu_count())) return DCN_OK;
+    if (plain_conv() != 2 && !plain_pays(rows, wgs, P.Cg, P.kV, P.hvol, cu_count())) return DCN_OK;
     *done = true;
     const unsigned items = (unsigned)chunk_candidates<FG>(P.cpg, P.Cg, P.C_in) * (unsigned)((P.kV + 1) / 2) * (unsigned)(P.Mp / 32), blocks = (items + 3) / 4;
     const PlanChoice none = {};

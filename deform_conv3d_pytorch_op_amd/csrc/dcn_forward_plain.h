@@ -37,6 +37,27 @@ inline PlainRows plain_rows(int M, int taps) {
     return r;
 }
 
+// Which layers take it.  A wavefront goes through the steps of sixteen reduction slots one after the other, 0.23 us to each (0.33 beside three others along the rows, 0.66 with
+// two row tiles) whatever the device does, and 0.5 to 0.8 us to each of its thread's cells of the halo, of eight channels; the kernels of the deformable layer share a
+// position or its channels among up to sixteen wavefronts.  So enough workgroups take it always and fewer only short chains: `steps` and 2.5 for every cell, up to a line that
+// rises with the workgroups.  2400 layers, us of the forward call on those kernels : here, always here 1.26 times as fast on average, by these lines and by the faster of the two
+// 1.28.  Refused: one row tile -- 256 -> 16, 1x1, two samples of 60 x 60, 14.1 : 22.1; 64 -> 32, 3x3, two of 60 x 60, 13.7 : 19.3 --, two -- 64 -> 64, 3x3, two
+// of 60 x 60, 16.5 : 19.1; 129 -> 56, 1x1, stride 2, sixteen of 29 x 18, 15.1 : 21.0 --, eight -- 24 -> 256, 5x5, 56 x 56, 30.7 : 34.9; 64 -> 273, 3x3, 28.8 : 44.4 --, long chains of few
+// wavefronts -- 512 -> 32, 3x3, 25 x 24 x 24, 68 : 118.  Taken: 64 -> 64, 3x3, 56 x 56, 21.9 : 20.4; 16 -> 128, 3x3, two of 40 x 40, 20.3 : 13.8; 256 -> 128, sixteen of 28 x 28, 108 : 79;
+// 59 -> 131, 3x3, eight of 24 x 23, 63 : 35; at worst 38 : 42 (251 -> 196, 1x1, stride 2, eight of 44 x 51).
+inline bool plain_pays(const PlainRows& r, long long workgroups, int channels, int taps, int hvol, int cus) {
+    const int slabs = (channels + FG - 1) / FG, steps = slabs * ((taps + 1) / 2);
+    const long long waves = workgroups * PLAIN_COLS * r.mw;
+    if (waves * 2 >= 11 * (long long)cus) return true;
+    if (steps > 40 || waves * 4 < 3 * (long long)cus) return false;
+    const double load = steps + 2.5 * slabs * hvol / (64.0 * PLAIN_COLS * r.mw), per_cu = (double)workgroups / cus;
+    if (r.mw == 1) return load <= 10 + 20 * per_cu;
+    // (from 64 channels on the other kernels split those of so few blocks into eight parts, which a further launch joins)
+    if (r.mw == 2) return load <= 26 || load <= 10 + 50 * per_cu || (channels >= 64 && taps > 1 && per_cu <= 0.25);
+    if (r.rw == 1) return load <= 60;
+    return steps <= 20 || (per_cu >= 0.25 && slabs > 3);
+}
+
 // Grid: N * tiles * G * mchunks workgroups of PLAIN_COLS * MW wavefronts; P.cchunk a multiple of eight.
 template <int RW>
 __global__ __launch_bounds__(512) void plain_conv_kernel(Params P, const float* __restrict__ in, const Parts<float>::Vec* __restrict__ Wq,

@@ -140,6 +140,25 @@ static bool plain_row_chunks() {
         }
     return plain_rows(256, 9).rw == 2 && plain_rows(257, 9).rw == 1 && plain_rows(339, 1).rw == 1 && plain_rows(591, 9).rw == 1 && plain_rows(591, 1).rw == 2;
 }
+// Which layers the kernel of the plain convolution takes: some whose times with it and with the others are known.
+static bool plain_layers() {
+    struct Layer { int N, h, w, c_in, c_out, k, stride, dil, G; bool faster; };
+    const Layer layers[] = {
+        {2, 60, 60, 256, 16, 1, 1, 1, 1, false}, {2, 60, 60, 64, 32, 3, 1, 1, 1, false}, {2, 60, 60, 64, 64, 3, 1, 1, 1, false}, {2, 60, 60, 24, 24, 5, 1, 1, 1, false},
+        {2, 60, 60, 24, 24, 3, 1, 1, 1, false},  {1, 112, 112, 64, 16, 3, 1, 1, 1, false}, {16, 29, 18, 129, 56, 1, 2, 1, 1, false}, {1, 56, 56, 24, 256, 5, 1, 1, 1, false},
+        {25, 24, 24, 512, 32, 3, 1, 1, 1, false}, {4, 28, 28, 128, 128, 3, 1, 1, 1, false}, {8, 24, 23, 59, 131, 3, 1, 1, 1, true}, {1, 56, 56, 64, 64, 3, 1, 1, 1, true},
+        {2, 60, 60, 16, 24, 3, 1, 1, 1, true},   {2, 40, 40, 16, 128, 3, 1, 1, 1, true},  {16, 28, 28, 256, 128, 3, 1, 1, 1, true}, {8, 56, 56, 64, 64, 3, 1, 1, 1, true},
+        {2, 60, 60, 8, 8, 3, 1, 1, 1, true},     {1, 82, 112, 92, 339, 3, 1, 1, 1, true},
+    };
+    for (const Layer& l : layers) {
+        const int M = l.c_out / l.G, pad = l.k / 2 * l.dil, span = (l.k - 1) * l.dil + 1, ext = 7 * l.stride + span;
+        const int oh = (l.h + 2 * pad - span) / l.stride + 1, ow = (l.w + 2 * pad - span) / l.stride + 1;
+        const PlainRows r = plain_rows(M, l.k * l.k);
+        if (plain_pays(r, (long long)l.N * ((oh + 7) / 8) * ((ow + 7) / 8) * l.G * r.mchunks, l.c_in / l.G, l.k * l.k, ext * ext, 256) != l.faster)
+            return printf("%d -> %d, %d taps, %d of %d x %d\n", l.c_in, l.c_out, l.k * l.k, l.N, l.h, l.w), false;
+    }
+    return true;
+}
 int main(int argc, char** argv) {
     if (argc != 4) return 2;
     const std::string what = argv[1];
@@ -164,6 +183,7 @@ int main(int argc, char** argv) {
         return 0;
     }
     if (what == "quad") return quads() ? 0 : 1;
+    if (what == "plain") return plain_layers() ? 0 : 1;
     if (what == "plain_rows") return plain_row_chunks() ? 0 : 1;
     if (what == "rows") return row_tiles() ? 0 : 1;
     if (what == "budget") {         // of any DCN_SCATTER_BUDGET_KB: what a CU has beside the 2120 and 100 bytes that the kernels declare; 72 stays 72
