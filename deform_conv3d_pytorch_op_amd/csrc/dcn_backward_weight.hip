@@ -261,6 +261,9 @@ template <int ND, typename S>
 int launch_bwd_weight_split(const WeightCall<float, S>& c, const S* off, hipStream_t s) {
     const Params& P = c.P;
     const dim3 grid((unsigned)((long long)c.igroups * P.mchunks * P.G * P.nsplit));
+    if (trace_plans())
+        fprintf(stderr, "dcn backward_weight, %s: %d row tiles, %d lanes to a tap, %d bytes of a corner to a lane, %d splits, grid %u\n",
+                sizeof(S) == 4 ? "float32" : std::is_same<S, Bf16>::value ? "bfloat16" : "binary16", c.MT, c.LW, split_quad<ND, S>(P, c.MT, c.LW) ? 16 : 4, P.nsplit, grid.x);
     hipLaunchKernelGGL((split_kernel<ND, S>(P, c.MT, c.LW, !off)), grid, dim3(WG), 0, s, P, (const S*)c.in_cl, off, c.gout, reinterpret_cast<const typename Parts<S>::Vec*>(c.gout_cl), c.partial, (unsigned)c.igroups);
     return check_launch("backward_weight_split_kernel");
 }

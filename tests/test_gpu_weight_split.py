@@ -1,4 +1,10 @@
 """backward_weight_split_kernel: layers just large enough for it, with the edges of its tiles, slabs, segments and volumes."""
+import ast
+import os
+import re
+import subprocess
+import sys
+
 import pytest
 import torch
 
@@ -29,6 +35,17 @@ LAYERS = [
     # slabs of four octets apart, 3-D: rows of several octets with slabs left over, rows shorter than an octet, two samples
     (3, 1, 17, 66, (3, 41, 75), 3, 1, 1, 1, 17, 1, 1.5), (3, 1, 9, 70, (203, 16, 3), 3, 1, 1, 1, 9, 1, 1.5), (3, 2, 16, 129, (5, 31, 47), 3, 1, 1, 1, 16, 1, 9.0),
 ]
+# (row tiles, lanes to a tap, bytes of a corner to a lane) of layers whose variant is one of few: eight row tiles, 16 bytes to a lane with 32, 16 and 8 lanes
+VARIANTS = {
+    (2, 1, 33, 129, (97, 101), 3, 1, 1, 1, 33, 1, 1.5): (8, 32, 4), (2, 1, 40, 256, (193, 195), 3, 1, 1, 1, 40, 1, 2.5): (8, 32, 16),
+    (2, 1, 40, 420, (131, 133), 3, 1, 1, 1, 20, 2, 9.0): (8, 32, 16), (3, 1, 33, 161, (9, 21, 35), 3, 1, 1, 1, 33, 1, 1.5): (8, 32, 4),
+    (2, 1, 160, 250, (223, 225), 1, 1, 0, 1, 160, 1, 0.9): (8, 32, 16), (2, 1, 36, 70, (97, 161), 3, 1, 1, 1, 36, 1, 1.5): (4, 32, 16),
+    (2, 1, 68, 66, (1, 9301), 3, 1, 1, 1, 68, 1, 1.5): (4, 32, 16), (2, 1, 32, 65, (161, 163), 3, 1, 1, 1, 16, 1, 1.5): (4, 16, 16),
+    (2, 1, 24, 65, (161, 163), 3, 1, 1, 1, 12, 1, 9.0): (4, 16, 16), (2, 1, 16, 66, (161, 163), 3, 1, 1, 1, 8, 1, 1.5): (4, 8, 16),
+    (2, 1, 16, 40, (161, 163), 3, 1, 1, 1, 4, 1, 1.5): (2, 8, 16), (2, 1, 33, 65, (97, 161), 3, 1, 1, 1, 33, 1, 1.5): (4, 32, 4),
+    (3, 1, 17, 66, (3, 41, 75), 3, 1, 1, 1, 17, 1, 1.5): (4, 32, 4),
+}
+LAYERS += [s for s in VARIANTS if s not in LAYERS]
 IDS = lambda s: "%dd-%d-%d-k%d-g%d" % (s[0], s[2], s[3], s[5], s[10])
 
 
@@ -72,6 +89,14 @@ LAYERS16 = [
     (2, 1, 72, 70, (129, 161), 3, 1, 1, 1, 72, 1, 1.5), (3, 1, 48, 64, (7, 31, 33), 3, 1, 1, 1, 24, 1, 2.5), (3, 1, 80, 64, (1, 95, 97), 3, 1, 1, 1, 80, 2, 1.0),
     (2, 1, 16, 130, (129, 161), 3, 1, 1, 1, 16, 1, 9.0), (2, 1, 8, 66, (229, 231), 3, 1, 1, 1, 8, 1, 1.5),
 ]
+# ... of the kernel that reads 16-bit storage; where two are given, bfloat16's and binary16's
+VARIANTS16 = {
+    (2, 1, 72, 64, (129, 161), 3, 1, 1, 1, 72, 1, 1.5): (2, 32, 16), (3, 1, 40, 97, (7, 31, 32), 3, 1, 1, 1, 40, 1, 2.5): (4, 32, 16),
+    (3, 1, 160, 128, (1, 95, 97), 3, 1, 1, 1, 160, 2, 1.0): (2, 32, 16), (3, 1, 48, 64, (7, 31, 33), 3, 1, 1, 1, 24, 1, 2.5): (2, 16, 16),
+    (2, 1, 32, 64, (129, 161), 3, 1, 1, 1, 16, 1, 9.0): (2, 8, 16), (2, 1, 16, 40, (161, 163), 3, 1, 1, 1, 8, 1, 1.5): (2, 8, 16),
+    (3, 1, 32, 64, (9, 32, 33), 3, 1, 1, 1, 16, 1, 1.5): ((2, 8, 4), (2, 8, 16)), (3, 1, 16, 30, (17, 33, 35), 3, 1, 1, 1, 16, 1, 2.5): (1, 8, 16),
+}
+LAYERS16 += [s for s in VARIANTS16 if s not in LAYERS16]
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
@@ -96,7 +121,33 @@ def test_layers_16bit(spec, dtype):
     assert ((got - want)[fin].norm() / want[fin].norm()).item() <= 2 * once
 
 
-@pytest.mark.parametrize("spec", [LAYERS[0], LAYERS[6]], ids=IDS)
+EXACT = [LAYERS[0], LAYERS[6]] + [s for s in VARIANTS if s[3] in (129, 256) or s[2:4] in ((36, 70), (24, 65))]
+
+
+def test_variants_of_the_layers():
+    """The layers take the variants that they are here for (the trace of the plans, in a process of its own: the knob is read once)."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    r = subprocess.run([sys.executable, "-u", "-m", "pytest", __file__, "-q", "-x", "-s", "-m", "gpu", "-k", "test_layers", "--timeout", "120", "--timeout-method", "thread"],
+                       cwd=os.path.dirname(here), env=dict(os.environ, DCN_TRACE_PLANS="1"), stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout[-3000:]
+    seen = 0
+    for case in r.stdout.split("weight gradient (")[1:]:
+        what = case[:case.index("\n")]
+        spec, dtype = ast.literal_eval("(" + what[:what.rindex(")") + 1]), what[what.rindex(")") + 1:].strip() or "torch.float32"
+        want = (VARIANTS if dtype == "torch.float32" else VARIANTS16).get(spec)
+        if want is None:
+            continue
+        if isinstance(want[0], tuple):
+            want = want[dtype == "torch.float16"]
+        got = re.findall(r"dcn backward_weight, (\w+): (\d+) row tiles, (\d+) lanes to a tap, (\d+) bytes", case)
+        print(spec, dtype, got, flush=True)
+        storage = {"torch.float32": "float32", "torch.bfloat16": "bfloat16", "torch.float16": "binary16"}[dtype]
+        assert got and set(got) == {(storage,) + tuple(map(str, want))}, spec
+        seen += 1
+    assert seen == len(VARIANTS) + 2 * len(VARIANTS16)
+
+
+@pytest.mark.parametrize("spec", EXACT, ids=IDS)
 @pytest.mark.parametrize("what,exponent", [("gout", 90), ("gout", 120), ("x", 100), ("x", 126)])
 def test_small_operands(spec, what, exponent):
     """Operands whose bfloat16 parts leave the range of normal numbers: the results are formed from the values themselves."""
@@ -111,7 +162,7 @@ def test_small_operands(spec, what, exponent):
         assert ((got - want).norm() / want.norm()).item() <= 4e-6
 
 
-@pytest.mark.parametrize("spec", [LAYERS[0], LAYERS[6]], ids=IDS)
+@pytest.mark.parametrize("spec", EXACT, ids=IDS)
 @pytest.mark.parametrize("what", ["x", "gout", "off"])
 def test_non_finite(spec, what):
     """Not finite where the oracle's gradient is not, equal to it elsewhere."""
