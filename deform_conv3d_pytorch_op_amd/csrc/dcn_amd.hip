@@ -224,6 +224,7 @@ int layer_backward(const Geometry& g, const S* in, const S* w, const S* off, con
             hipLaunchKernelGGL(narrow_gradients_kernel<S>, dim3(blocks), dim3(256), 0, s, prep.octets, gin, z.in, nullptr, nullptr, 0, nullptr, nullptr, 0, nullptr,
                                nullptr, 0, true, P.N, P.C_in, P.inV);
             if (int rc = check_launch("narrow_gradients_kernel")) return rc;
+            if (trace_plans()) fprintf(stderr, "dcn layer_backward: grad_input rounded ahead of the widened copies\n");
             prep.octets = nullptr;
             narrowed = true;
         }

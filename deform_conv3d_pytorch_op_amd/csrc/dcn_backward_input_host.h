@@ -343,12 +343,15 @@ int backward_input_offset(const Geometry& g, const S* in, const S* w, const S* o
         // Where the fused kernel collects grad_input: in octets of channels in the place of the channels-last gradient, or in the tensor itself.  In 3-D
         // the last launch of the path without LDS tiling, or the rounding of a 16-bit layer's gradients, brings them to the tensor, and a halo
         // has 8 to 18 voxels to a position.  In 2-D it has two: steps of 256 -> 256, 3x3, 8 x 56 x 56 874 us in the tensor, 883 in octets (one launch more),
-        // in binary16 435 and 436.
+        // in binary16 435 and 436.  Halos so large that float32 chunks are half octets flush a line twice: backward passes to input and offset of 132 such layers 0.93 to 1.18 times
+        // as fast as in the tensor, 1.02 on average (2x2x2 at stride 2, 64 -> 64, two samples of 16 x 56 x 56, 193 us in the tensor, 203 in octets; 4x4x4 at stride 2, 64 -> 64, one
+        // sample, samples within 1.5 voxels 261 and 270, within 3 483 and 412: the corners of a sample past the halo are a line in octets).
         bool octets = ND == 3 && sizeof(T) == 4 && at.fused && tail_words && P.cpg % 8 == 0 && P.Cg % 8 == 0;
         for (int k = 0; k < pc.nplans; ++k) octets = octets && !fp[k].kern;
         if (octets) prep.zero(gin_cl, (size_t)P.N * P.C_in * P.inV * sizeof(T));
         else if (given) prep.zero(gin, (size_t)P.N * P.C_in * P.inV * sizeof(T));
         float* const collect = reinterpret_cast<float*>(octets ? gin_cl : gin);
+        if (trace_plans() && ND == 3) fprintf(stderr, "dcn backward_input_offset: grad_input collected in %s\n", octets ? "octets" : "the tensor");
         if (int rc = launch_prepare<T, S>(P, pc, prep, w, off, n_off, s)) return rc;
         // one launch per set of plans that differ in nothing but the halo
         unsigned launched = 0;

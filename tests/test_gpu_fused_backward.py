@@ -145,10 +145,10 @@ def test_samples_past_the_halo(spec, share, dtype):
         assert err <= tol + once
 
 
-# grad_input collected in octets of channels: several deformable and convolution groups, halves of octets (the 4-channel chunks of wide halos),
-# stride 2, the path without LDS tiling behind it, and a weight gradient that 16-bit storage computes on widened tensors in the same workspace
+# grad_input collected in octets of channels: several deformable and convolution groups, halves of octets (the 4-channel chunks of stride 2, and, beside whole
+# ones, of wide halos), the path without LDS tiling behind it, and a weight gradient that 16-bit storage computes on widened tensors in the same workspace
 OCTETS = [(3, 2, 24, 20, (5, 9, 10), 3, 1, 1, 1, 8, 1, 1.5), (3, 1, 16, 12, (4, 8, 9), 3, 1, 1, 1, 16, 2, 3.5), (3, 1, 16, 33, (9, 21, 19), 3, 2, 1, 1, 16, 1, 2.0),
-          (3, 2, 8, 16, (6, 9, 9), 3, 1, 1, 1, 8, 1, 12.0), (3, 1, 64, 128, (4, 9, 10), 3, 1, 1, 1, 32, 1, 1.5)]
+          (3, 2, 8, 16, (6, 9, 9), 3, 1, 1, 1, 8, 1, 12.0), (3, 1, 64, 128, (4, 9, 10), 3, 1, 1, 1, 32, 1, 1.5), (3, 2, 16, 12, (8, 17, 19), 3, 1, 1, 1, 16, 1, 3.3)]
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
@@ -169,6 +169,47 @@ def test_octets(spec, dtype):
         err = ((g - t).norm() / t.norm()).item()
         print("  relative 2-norm error %.2e" % err, flush=True)
         assert err <= tol + once
+
+
+def test_octets_are_taken():
+    """What the layers above are for (the trace of the plans, in a process of its own: the knob is read once)."""
+    here = os.path.dirname(os.path.abspath(__file__))
+    r = subprocess.run([sys.executable, "-u", "-m", "pytest", __file__, "-q", "-x", "-s", "-m", "gpu", "-k", "test_octets and not taken and not behind", "--timeout", "120",
+                        "--timeout-method", "thread"], cwd=os.path.dirname(here), env=dict(os.environ, DCN_TRACE_PLANS="1"), stdout=subprocess.PIPE,
+                       stderr=subprocess.STDOUT, text=True, timeout=300)
+    assert r.returncode == 0, r.stdout[-3000:]
+    cases = r.stdout.split("octets (")[1:]
+    assert len(cases) == 2 * len(OCTETS)
+    for case in cases:
+        what = case[:case.index("\n")]
+        spec, f32 = ast.literal_eval("(" + what[:what.rindex(")") + 1]), what.endswith("torch.float32")
+        collected = re.findall(r"grad_input collected in (.*)", case)
+        chunks = set(re.findall(r"dcn backward_input_offset: launch.* (\d+) channels per chunk, ", case))
+        print(spec, what, collected, chunks, flush=True)
+        assert collected and set(collected) == {"octets"}, spec
+        assert chunks == ({"4"} if spec == OCTETS[2] else {"8", "4"} if spec == OCTETS[5] else {"8"}), spec
+        assert ("grad_input rounded ahead" in case) == (spec == OCTETS[4] and not f32), spec
+        assert ("path without LDS tiling offered" in case) == f32, spec
+
+
+def test_octets_behind_the_path_without_lds():
+    """The device takes the path without LDS tiling for the layer of far offsets (the plan is recorded in the workspace, include/dcn_amd.h), whose channels-last
+    gradients the octets' last launch then adds to what grad_input holds."""
+    from deform_conv3d_pytorch_op_amd import _lib
+    from deform_conv3d_pytorch_op_amd.functions import _geom, _workspace_bytes
+    print("octets, global", flush=True)
+    L, c = _lib.load(), make_case(*OCTETS[3], dtype=torch.float32, seed=38, bias=False)
+    x, off, w, gout = (c[k].cuda() for k in ("x", "off", "w", "gout"))
+    nbytes = _workspace_bytes(x, w, c["groups"], c["outs"], c["cpg"])
+    ws = torch.full((nbytes,), 0xFF, dtype=torch.uint8, device="cuda")
+    gin, goff = torch.ones_like(x), torch.empty_like(off)
+    geom = _geom(3, x, w, c["outs"], c["stride"], c["pad"], c["dil"], c["cpg"], c["groups"])
+    assert L.dcn3d_backward_input_offset_f32(*(t.data_ptr() for t in (x, w, off, gout, gin, goff)), *geom, ws.data_ptr(), nbytes, torch.cuda.current_stream().cuda_stream) == 0
+    torch.cuda.synchronize()
+    at = (nbytes - 256) // 256 * 256 + 64
+    assert int.from_bytes(bytes(ws[at:at + 4].cpu().tolist()), "little") == 3
+    for got, want, tol in zip((gin - 1, goff), _oracle(c), (1e-4, 1e-5)):
+        assert ((got.cpu().double() - want).norm() / want.norm()).item() <= tol
 
 
 def test_one_small_position_beside_ordinary_ones():
