@@ -43,14 +43,9 @@ inline int plain_forward(Params P, const float* in, const float* w, const float*
     P.Mp = rows.mchunks * mw * rw * 32;
     if (!plan_halo<float, 2>(P, (size_t)1 << 30, 0, 64, 1, PLAIN_COLS, false, FG, nullptr, 1, false)) return DCN_OK;
     const long long wgs = (long long)P.N * P.tiles * P.G * P.mchunks;
-    // Channels at a time: two workgroups to a CU.  Those of one row tile are two wavefronts each: four, if there are so many, unless it leaves less than 24 channels.  81 such layers,
-    // us of the forward call with two : with four, 1.22 : 1 on average: 276 -> 15, 3x3, dilation 2, eight samples of 81 x 62, 140 : 86; 157 -> 8, 5x5, sixteen of 89 x 29, 153 : 95; 62 -> 25, 5x5,
-    // dilation 2, sixteen of 181 x 9, 76 : 47.
-    while (P.cchunk > FG && plain_lds(P.hvol, P.cchunk) > MAX_FORWARD_LDS / 2) P.cchunk -= FG;
-    if (mw == 1 && wgs > 2 * (long long)cu_count())
-        while (P.cchunk > 3 * FG && plain_lds(P.hvol, P.cchunk) > MAX_FORWARD_LDS / 4) P.cchunk -= FG;
+    P.cchunk = plain_channels(rows, wgs, P.cchunk, P.hvol, cu_count());
     const size_t lds = plain_lds(P.hvol, P.cchunk);
-    if (lds > MAX_FORWARD_LDS || ws_bytes < split_weight_bytes<float>(P, P.Mp) || wgs > 0x7fffffffLL || !plain_conv()) return DCN_OK;
+    if (lds > MAX_PLAIN_LDS || ws_bytes < split_weight_bytes<float>(P, P.Mp) || wgs > 0x7fffffffLL || !plain_conv()) return DCN_OK;
     if (plain_conv() != 2 && !plain_pays(rows, wgs, P.Cg, P.kV, P.hvol, cu_count())) return DCN_OK;
     *done = true;
     const unsigned items = (unsigned)chunk_candidates<FG>(P.cpg, P.Cg, P.C_in) * (unsigned)((P.kV + 1) / 2) * (unsigned)(P.Mp / 32), blocks = (items + 3) / 4;

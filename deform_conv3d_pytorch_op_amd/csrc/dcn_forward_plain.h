@@ -19,6 +19,7 @@
 namespace dcn {
 
 constexpr int PLAIN_COLS = 2;                           // position tiles of a workgroup
+constexpr size_t MAX_PLAIN_LDS = 160 * 1024 - 256;      // dynamic LDS of a workgroup
 // operands of a voxel in a part's plane: an odd number, so that eight voxels in a row lie in different LDS banks
 __host__ __device__ inline constexpr int plain_row(int channels) { return (channels / FG) | 1; }
 __host__ inline size_t plain_lds(int hvol, int channels) { return (size_t)Parts<float>::NP * hvol * plain_row(channels) * 16; }
@@ -35,6 +36,17 @@ inline PlainRows plain_rows(int M, int taps) {
     r.rw = tiles > 4 && (eight == four || (taps == 1 && eight * 4 <= four * 5)) ? 2 : 1;
     r.mchunks = (tiles + r.mw * r.rw - 1) / (r.mw * r.rw);
     return r;
+}
+
+// Channels at a time, `most` of them at most: two workgroups to a CU.  Those of one row tile are two wavefronts each: four, if there are so many, unless it leaves less than 24 channels.
+// 81 such layers, us of the forward call with two : with four, 1.22 : 1 on average: 276 -> 15, 3x3, dilation 2, eight samples of 81 x 62, 140 : 86; 157 -> 8, 5x5, sixteen of 89 x 29,
+// 153 : 95; 62 -> 25, 5x5, dilation 2, sixteen of 181 x 9, 76 : 47.
+inline int plain_channels(const PlainRows& r, long long workgroups, int most, int hvol, int cus) {
+    int c = most;
+    while (c > FG && plain_lds(hvol, c) > MAX_PLAIN_LDS / 2) c -= FG;
+    if (r.mw == 1 && workgroups > 2 * (long long)cus)
+        while (c > 3 * FG && plain_lds(hvol, c) > MAX_PLAIN_LDS / 4) c -= FG;
+    return c;
 }
 
 // Which layers take it.  A wavefront goes through the steps of sixteen reduction slots one after the other, 0.23 us to each (0.33 beside three others along the rows, 0.66 with

@@ -140,6 +140,21 @@ static bool plain_row_chunks() {
         }
     return plain_rows(256, 9).rw == 2 && plain_rows(257, 9).rw == 1 && plain_rows(339, 1).rw == 1 && plain_rows(591, 9).rw == 1 && plain_rows(591, 1).rw == 2;
 }
+// Channels at a time of the plain convolution: they fit, two workgroups to a CU or one at the least channels; of one row tile, where there are many, four down to 24 channels.
+static bool plain_chunks() {
+    for (int i = 0; i < 20000; ++i) {
+        const PlainRows r = plain_rows(pick(1, 300), 9);
+        const int most = pick(1, 8) * 8, hvol = pick(1, 40) * pick(1, 40), wgs = pick(1, 4000), c = plain_channels(r, wgs, most, hvol, 256);
+        const bool four = r.mw == 1 && wgs > 512;
+        const size_t room = MAX_PLAIN_LDS / (four && c >= 24 && c + 8 <= most && plain_lds(hvol, c + 8) * 2 <= MAX_PLAIN_LDS ? 4 : 2);
+        if (c < 8 || c > most || c % 8 || (c > 8 && plain_lds(hvol, c) > MAX_PLAIN_LDS / 2) || (four && c > 24 && plain_lds(hvol, c) > MAX_PLAIN_LDS / 4) ||
+            (c < most && plain_lds(hvol, c + 8) <= room))
+            return printf("%d of %d channels, %d voxels, %d workgroups\n", c, most, hvol, wgs), false;
+    }
+    const PlainRows one = plain_rows(15, 9), two = plain_rows(64, 9);
+    return plain_channels(one, 600, 64, 144, 256) == 40 && plain_channels(one, 500, 64, 144, 256) == 64 && plain_channels(two, 600, 64, 144, 256) == 64 &&
+           plain_channels(one, 600, 24, 361, 256) == 24;
+}
 // Which layers the kernel of the plain convolution takes: some whose times with it and with the others are known.
 static bool plain_layers() {
     struct Layer { int N, h, w, c_in, c_out, k, stride, dil, G; bool faster; };
@@ -183,6 +198,7 @@ int main(int argc, char** argv) {
         return 0;
     }
     if (what == "quad") return quads() ? 0 : 1;
+    if (what == "plain_chunks") return plain_chunks() ? 0 : 1;
     if (what == "plain") return plain_layers() ? 0 : 1;
     if (what == "plain_rows") return plain_row_chunks() ? 0 : 1;
     if (what == "rows") return row_tiles() ? 0 : 1;

@@ -22,7 +22,7 @@ def test_rule(probe, what):
     assert r.returncode == 0, r.stdout
 
 
-@pytest.mark.parametrize("what", ["quad", "rows", "plain_rows", "plain"])
+@pytest.mark.parametrize("what", ["quad", "rows", "plain_rows", "plain_chunks", "plain"])
 def test_measured_line(probe, what):
     """Which variant of a kernel a layer takes, where the times with either are known."""
     r = subprocess.run([probe, what, "7", "1"], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=60)
