@@ -1,8 +1,9 @@
 """The reference's plain convolution package: `Conv2dFunction`
 (conv2d/conv2d_functions/conv2d_function.py:7-67) and `Conv2d`
-(conv2d/conv2d_modules/conv2d_model.py:11-46), on the kernels of the 2-D deformable layer with every
-offset zero (C ABI: conv2d_forward / conv2d_backward_input / conv2d_backward_weight in
-include/dcn_amd.h, in place of conv2d/lib/conv2d_cuda.h:17-39).
+(conv2d/conv2d_modules/conv2d_model.py:11-46).  The float32 forward pass, and the backward pass to the
+input at stride 1, have a kernel of their own; the rest, and layers that it is not faster on, run on the
+kernels of the 2-D deformable layer with every offset zero (C ABI: conv2d_forward / conv2d_backward_input /
+conv2d_backward_weight in include/dcn_amd.h, in place of conv2d/lib/conv2d_cuda.h:17-39).
 
 Same call shape, `Conv2dFunction.apply(inputs, weight, bias=None, stride=(1, 1), padding=(0, 0),
 dilation=(1, 1), group=1)`, and the reference's dilation-aware output size

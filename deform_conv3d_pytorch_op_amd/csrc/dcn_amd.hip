@@ -264,10 +264,11 @@ int layer_backward(const Geometry& g, const S* in, const S* w, const S* off, con
 // Plain 2-D convolution: the reference's conv2d package (conv2d/lib/conv2d_cuda.cpp:77-290, kernels
 // conv2d/lib/conv2d_cuda_kernel.cu:25-169: im2col / col2im with integer taps and one GEMM per sample
 // and group).  It is the 2-D deformable layer with every offset zero, one deformable group and the
-// dilation-aware output size (conv2d/lib/conv2d_cuda.cpp:20-22), so it runs on the same kernels: a
-// null offset means zeros to the float32 forward pass and to the backward pass to the weight; the others
-// get a zero offset tensor at the front of the workspace, behind it scratch for the grad_offset that
-// one fallback kernel of backward-to-input writes, then the deformable layer's own workspace.
+// dilation-aware output size (conv2d/lib/conv2d_cuda.cpp:20-22).  The float32 forward pass, which is also the
+// backward pass to the input at stride 1, has a kernel of its own where that is faster (plain_conv_kernel); the rest
+// runs on the deformable layer's: a null offset means zeros to the float32 forward pass and to the backward
+// pass to the weight; the others get a zero offset tensor at the front of the workspace, behind it scratch for the
+// grad_offset that one fallback kernel of backward-to-input writes, then the deformable layer's own workspace.
 template <typename T> size_t conv2d_zero_bytes(int N, int kV, size_t outV) { return align256((size_t)N * 2 * kV * outV * sizeof(T)); }
 template <typename T>
 int conv2d_offsets(const Geometry& g, void* ws, size_t ws_bytes, hipStream_t s, T** off, T** scratch, void** rest, size_t* rest_bytes) {
@@ -309,7 +310,7 @@ int conv2d_backward_weight(Geometry g, const T* in, const T* gout, T* gw, void* 
 }
 // The gradients asked for (null: not wanted), written.  grad_input of a layer of stride 1 is a
 // convolution itself -- grad_output with the weight's channels exchanged and its taps in reverse, padded
-// by dilation * (k - 1) - pad -- and runs as a forward pass: no scatter (64 -> 64 channels, 8 x 56 x 56: 34 us
+// by dilation * (k - 1) - pad -- and runs as a forward pass: no scatter (64 -> 64 channels, 8 x 56 x 56: 27 us
 // against 146 for the kernel that adds up grad_input in LDS).
 template <typename T>
 int conv2d_layer_backward(Geometry g, const T* in, const T* w, const T* gout, T* gin, T* gw, T* gb, void* ws, size_t ws_bytes, hipStream_t s) {

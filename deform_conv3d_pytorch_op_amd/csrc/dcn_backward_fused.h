@@ -137,8 +137,8 @@ template <typename S> inline size_t fused_voxel_bytes(int cch) { return (size_t)
 // grad_input in octets, [n][channel / 8][voxel][8], where every chunk of channels is an octet or half of one: collected there, and brought to
 // the layout of the tensor by octets_to_planes.  The float atomics of a flush go to memory by the line: 1.0e8 of them from halos of 9 x 15 x 15
 // voxels take 545 us with the lanes along the rows of eight planes (14 voxels: 56 bytes), 283 in octets (448), 462 channels-last (32).
-// Steps of 128 -> 128 in deformable groups of 32, stride 1 2 2, 2 x 16 x 112 x 112: 4460 -> 4202 us (the kernel 2.40 -> 2.24 ms, 59 us for
-// the tensor), of 64 -> 64, 4 x 16 x 56 x 56: 2403 -> 2372, in bfloat16 1659 -> 1648, whose flushes are a third as long beside the rest.
+// Steps of 128 -> 128 in deformable groups of 32, stride 1 2 2, 2 x 16 x 112 x 112, in the tensor -> in octets: 4453 -> 4208 us (the kernel 2.40 -> 2.24 ms,
+// 59 us for the tensor), of 64 -> 64, 4 x 16 x 56 x 56: 2398 -> 2358, in bfloat16 1618 -> 1606, whose flushes are a third as long beside the rest.
 // put(index in the tensor, value), one thread per voxel of an octet.  last: the source is channels-last instead.
 template <typename Put>
 __device__ inline void octets_to_planes(const float* __restrict__ src, int N, int C, unsigned V, bool last, size_t first, size_t step, Put put) {
@@ -186,7 +186,7 @@ __global__ __launch_bounds__(FUSED_WAVES * 64) void backward_fused_kernel(Params
     constexpr int XP = (CCH + CH - 1) / CH;                             // planes of input cells
     constexpr int CR = PT > 1 && NC > 4 ? 4 : NC;                        // corners read at a time
     constexpr int XR = 4;                                               // input cells of a thread in flight
-    // The adds of a tap slot go ahead of what other wavefronts have to issue: 64 -> 64 channels, 3x3x3, 4 x 16 x 56 x 56, in bfloat16 a step 1634 -> 1608 us.
+    // The adds of a tap slot go ahead of what other wavefronts have to issue: 64 -> 64 channels, 3x3x3, 4 x 16 x 56 x 56, in bfloat16 a step 1630 -> 1595 us.
     // In float32, where the contraction has six times the instructions, 2371 -> 2364, at stride 1 2 2 4190 -> 4210, 2-D 877 -> 895.
     constexpr bool FIRST = ND == 3 && sizeof(S) == 2;
     extern __shared__ __align__(16) unsigned char smem_raw[];

@@ -10,7 +10,7 @@
 // fixed distance, the weights from L2 (a few steps ahead, in the order of pack_split_weight_kernel) and six matrix instructions a row tile.
 // A workgroup has two position tiles (a block of 64 positions) and MW wavefronts along the rows, RW row tiles each.
 // Small layers: the matrix instructions of 64 -> 64 channels, 3x3, 8 x 56 x 56 take 5 us of the device, a workgroup's first instructions and
-// loads as long again.  us of a forward call with the packing of its weights, on the former kernels -> here: that layer 35 -> 27 (a training step 103 -> 93),
+// loads as long again.  us of a forward call with the packing of its weights, on the former kernels -> here: that layer 35 -> 27 (a training step 102 -> 90),
 // 100 -> 100, 5x5, 4 x 60 x 60: 139 -> 77; 512 -> 512, 8 x 28 x 28: 297 -> 273.  One sum to a result tile (every instruction waits for the one
 // before it) and operands read in their own step: 30.
 #pragma once

@@ -180,9 +180,10 @@ int dcn2d_backward_weight_f64(const double *input, const double *offset, const d
  * (input + 2 pad - dilation (kernel - 1) - 1) / stride + 1.  `bias` ([output_c] or NULL) is added in
  * the epilogue (the reference adds it from Python, conv2d/conv2d_functions/conv2d_function.py:34-35);
  * grad_input and grad_weight are accumulated into (the caller zero-fills them, as the reference's
- * Function does).  backward_input is not given the input, like the reference's.  The layer runs on
- * the kernels of the 2-D deformable layer with every offset zero; the workspace (conv2d_workspace_bytes) has
- * room for that zero offset tensor, which the calls that read one put in front of the deformable layer's own. */
+ * Function does).  backward_input is not given the input, like the reference's.  The float32 forward pass has a
+ * kernel of its own for the layers that are faster on it; the rest runs on the kernels of the 2-D deformable
+ * layer with every offset zero, and the workspace (conv2d_workspace_bytes) has room for that zero offset tensor,
+ * which the calls that read one put in front of the deformable layer's own. */
 #define CONV2D_GEOMETRY                                                                          \
     int batch, int input_c, int output_c, int input_h, int input_w, int output_h, int output_w,  \
     int kernel_h, int kernel_w, int pad_h, int pad_w, int stride_h, int stride_w,                \
