@@ -55,8 +55,7 @@ inline int plain_forward(Params P, const float* in, const float* w, const float*
     if (int rc = check_launch("forward weight packing")) return rc;
     if (trace_plans())
         fprintf(stderr, "dcn plain convolution: %d wavefronts along the rows, %d row tiles each, %d channels at a time, grid %lld, LDS %zu\n", mw, rw, P.cchunk, wgs, lds);
-    auto kern = rw == 2 ? plain_conv_kernel<2> : plain_conv_kernel<1>;
-    return launch_halo(kern, "plain_conv_kernel", dim3((unsigned)wgs), PLAIN_COLS * mw * 64, lds, s, P, in, reinterpret_cast<const Parts<float>::Vec*>(ws), w, bias, out);
+    return launch_halo(plain_kernel(rows), "plain_conv_kernel", dim3((unsigned)wgs), PLAIN_COLS * mw * 64, lds, s, P, in, reinterpret_cast<const Parts<float>::Vec*>(ws), w, bias, out);
 }
 
 // S = T: the float32 / float64 operator.  S = Bf16 / Fp16 (T = float): the tensors are in that

@@ -10,9 +10,14 @@
 // fixed distance, the weights from L2 (a few steps ahead, in the order of pack_split_weight_kernel) and six matrix instructions a row tile.
 // A workgroup has two position tiles (a block of 64 positions) and MW wavefronts along the rows, RW row tiles each.
 // Small layers: the matrix instructions of 64 -> 64 channels, 3x3, 8 x 56 x 56 take 5 us of the device, a workgroup's first instructions and
-// loads as long again.  us of a forward call with the packing of its weights, on the former kernels -> here: that layer 35 -> 27 (a training step 102 -> 90),
-// 100 -> 100, 5x5, 4 x 60 x 60: 139 -> 77; 512 -> 512, 8 x 28 x 28: 297 -> 273.  One sum to a result tile (every instruction waits for the one
-// before it) and operands read in their own step: 30.
+// loads as long again.  us of a forward call with the packing of its weights, on the former kernels -> here: that layer 36 -> 26 (a training step 102 -> 90),
+// 100 -> 100, 5x5, 4 x 60 x 60: 131 -> 69; 512 -> 512, 8 x 28 x 28: 272 -> 237.
+// Sums: every matrix instruction rounds what it adds to, and cuts products off towards minus infinity below its last places; a result that went through six of them in
+// each of some hundred steps was up to twice as far from float64 as that of the kernels before, whose chains are shorter where they share a position.  Here the products of
+// a step start from zero, and their sum is added to the result while the next one's are formed; every second slab of channels lies in LDS with its sign turned round, and so
+// do the sums that come of it.  Error against float64, 2-norm, of 260 layers over the kernels before: 0.41 on average, at worst 0.81, where the sum through all steps had
+// 0.99 and 1.98.  The additions are placed between the matrix instructions (the scheduler's own order, all of them after the first, cost layers of two row tiles to a
+// wavefront 5 %): 150 layers 0.986 of the time of the sum through all steps, at worst 1.066.
 #pragma once
 #include "dcn_forward_split.h"
 
@@ -70,16 +75,17 @@ inline bool plain_pays(const PlainRows& r, long long workgroups, int channels, i
     return steps <= 20 || (per_cu >= 0.25 && slabs > 3);
 }
 
-// Grid: N * tiles * G * mchunks workgroups of PLAIN_COLS * MW wavefronts; P.cchunk a multiple of eight.
-template <int RW>
-__global__ __launch_bounds__(512) void plain_conv_kernel(Params P, const float* __restrict__ in, const Parts<float>::Vec* __restrict__ Wq,
+// Grid: N * tiles * G * mchunks workgroups of PLAIN_COLS * MW wavefronts; P.cchunk a multiple of eight.  AHEAD: steps that weights are read ahead by, as many as leave
+// two workgroups to a CU (eight wavefronts each, of 128 registers, where four are along the rows): see plain_kernel.
+template <int RW, int AHEAD>
+__global__ __launch_bounds__(AHEAD == 4 ? 256 : 512, AHEAD == 4 ? 2 : 4) void plain_conv_kernel(Params P, const float* __restrict__ in, const Parts<float>::Vec* __restrict__ Wq,
                                                          const float* __restrict__ W, const float* __restrict__ bias, float* __restrict__ out) {
     touch_arguments<sizeof(Params) + 32>();
     using PT = Parts<float>;
     using MM = Mma<float>;
     typedef PT::Vec Vec;
-    constexpr int TN = 32, NP = PT::NP, AHEAD = RW == 1 ? 4 : 2;
-    constexpr int CH = RW == 1 ? 2 : 1;                 // sums of a result tile, in turn: a matrix instruction does not wait for the one before it
+    constexpr int TN = 32, NP = PT::NP, UN = AHEAD > 2 ? AHEAD : 2;
+    constexpr int NA = AHEAD == 4 ? 2 : RW;             // results being summed up: of one row tile, two where there are registers for them
     extern __shared__ __align__(16) unsigned char smem_raw[];
     Vec* sX = reinterpret_cast<Vec*>(smem_raw);         // [part][voxel][slab of eight channels]
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), WGS = (int)blockDim.x;
@@ -93,7 +99,7 @@ __global__ __launch_bounds__(512) void plain_conv_kernel(Params P, const float* 
     tile_decode<2>(P, H, rest / P.G, tg);
     int o[2];
     unsigned pos;
-    const bool valid = tile_position<2>(P, tg, pt * TN + j, o, pos);
+    bool valid = tile_position<2>(P, tg, pt * TN + j, o, pos);
     const int row = P.hext[2], hvol = P.hvol;
     const int at = (o[0] * P.stride[1] - P.pad[1] - tg.hb[0]) * row + o[1] * P.stride[2] - P.pad[2] - tg.hb[1];      // the position's voxel at tap 0
     const int cg0 = g * P.Cg, cg1 = cg0 + P.Cg, ntg = (P.kV + 1) / 2;
@@ -102,11 +108,13 @@ __global__ __launch_bounds__(512) void plain_conv_kernel(Params P, const float* 
     const float inv = __builtin_amdgcn_rcpf((float)hvol), inv_row = __builtin_amdgcn_rcpf((float)row);
     const int rs = plain_row(P.cchunk);
 
-    MM::Acc part[CH][RW];
+    MM::Acc acc[NA], part[2] = {acc_zero<float>(), acc_zero<float>()};      // results; sums of a step, one being formed and one to be added
 #pragma unroll
-    for (int h = 0; h < CH; ++h)
+    for (int r = 0; r < NA; ++r) acc[r] = acc_zero<float>();
+    auto add = [&](int r, const MM::Acc& sum, float sign) {
 #pragma unroll
-        for (int r = 0; r < RW; ++r) part[h][r] = acc_zero<float>();
+        for (int i = 0; i < MM::NACC; ++i) acc[r][i] = fmaf(sum[i], sign, acc[r][i]);
+    };
 #pragma unroll 1
     for (int cc0 = cg0; cc0 < cg1; cc0 += P.cchunk) {
         const int nch = min(P.cchunk, cg1 - cc0), nsl = (nch + FG - 1) / FG;
@@ -143,7 +151,7 @@ __global__ __launch_bounds__(512) void plain_conv_kernel(Params P, const float* 
 #pragma unroll
             for (int e = 0; e < FG; ++e) x[e] = chan0[(size_t)min(sl * FG + e, nch - 1) * P.inV + to];
 #pragma unroll
-            for (int e = 0; e < FG; ++e) x[e] = there && sl * FG + e < nch ? x[e] : 0.f;
+            for (int e = 0; e < FG; ++e) x[e] = __uint_as_float(__float_as_uint(there && sl * FG + e < nch ? x[e] : 0.f) ^ (unsigned)sl << 31);
             Vec p[NP];
             PT::split(x, p);
 #pragma unroll
@@ -151,6 +159,7 @@ __global__ __launch_bounds__(512) void plain_conv_kernel(Params P, const float* 
         }
         __syncthreads();
         Vec b8[2][NP];
+        float sign[2], last = 1.f;                      // of the sums of a step
         int k0[2] = {0, 0}, bsl = 0, btg = 0;
         const Vec* bp = nullptr;
         auto pair = [&]() {                             // this lane's voxel at tap pair btg
@@ -167,6 +176,7 @@ __global__ __launch_bounds__(512) void plain_conv_kernel(Params P, const float* 
 #pragma unroll
             for (int k = 0; k < NP; ++k) b8[u][k] = bp[k * plane];
             ++bp;
+            sign[u] = bsl & 1 ? -1.f : 1.f;
             if (++bsl == nsl) {
                 bsl = 0;
                 if (++btg < ntg) pair();
@@ -175,23 +185,38 @@ __global__ __launch_bounds__(512) void plain_conv_kernel(Params P, const float* 
         };
         pair();
         load_b(0);
-        for (int s = 0; s < steps; s += AHEAD) {
+        for (int s = 0; s < steps; s += UN) {
 #pragma unroll
-            for (int u = 0; u < AHEAD; ++u)
+            for (int u = 0; u < UN; ++u)
                 if (s + u < steps) {                    // (uniform)
                     load_b((u + 1) & 1);
-                    mma_parts<float, RW>(a8[u], b8[u & 1], part[u % CH]);
-                    load_a(u);
+#pragma unroll
+                    for (int r = 0; r < RW; ++r) {
+                        const int i = u * RW + r;
+                        part[i & 1] = acc_zero<float>();
+                        mma_parts<float, 1>(a8[u % AHEAD] + r, b8[u & 1], part + (i & 1));
+                        add(RW == 1 ? u / 2 % NA : 1 - r, part[(i + 1) & 1], r ? sign[u & 1] : last);
+                    }
+                    last = sign[u & 1];
+                    load_a(u % AHEAD);
+#pragma unroll
+                    for (int i = 0; i < 6 * RW; ++i) {  // a matrix instruction, three others, ...
+                        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
+                    }
                     __builtin_amdgcn_sched_barrier(0);
                 }
         }
+        add(RW - 1, RW == 1 && (steps & 1) ? part[0] : part[1], last);
+        part[1] = acc_zero<float>();
     }
-    MM::Acc acc[RW];
 #pragma unroll
-    for (int r = 0; r < RW; ++r) {
-        acc[r] = part[0][r];
-        if constexpr (CH > 1) acc[r] += part[1][r];
-    }
+    for (int r = RW; r < NA; ++r) acc[0] += acc[r];
+    // (lane and position once more: kept through the steps they are spilled)
+    int me = (int)__builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0u));
+    asm volatile("" : "+v"(me));
+    const int mj = me % TN, mq = me / TN;
+    valid = tile_position<2>(P, tg, pt * TN + mj, o, pos);
     // Results that the parts may have cost bits (see dcn_forward_split.h): once more on the float32 instructions, from the values themselves.
     if (__builtin_expect(__any(valid && !results_stand<RW, float>(acc)), 0)) {
 #pragma unroll
@@ -204,13 +229,13 @@ __global__ __launch_bounds__(512) void plain_conv_kernel(Params P, const float* 
             const float* x = in + (size_t)P.C_in * P.inV * tg.n + (there ? (unsigned)ch * (unsigned)P.in[2] + (unsigned)cw : 0u);
 #pragma unroll 1
             for (int cl = 0; cl < P.Cg; cl += 2) {
-                const int c = min(cl + q, P.Cg - 1);
-                const float xv = x[(size_t)(cg0 + c) * P.inV], b = there && cl + q < P.Cg ? xv : 0.f;
+                const int c = min(cl + mq, P.Cg - 1);
+                const float xv = x[(size_t)(cg0 + c) * P.inV], b = there && cl + mq < P.Cg ? xv : 0.f;
 #pragma unroll
                 for (int r = 0; r < RW; ++r) {
-                    const int m = (int)(tile0 + r) * TN + j;
+                    const int m = (int)(tile0 + r) * TN + mj;
                     const float wv = weight_at<float>(P, W, g, min(m, P.M - 1), (size_t)c, tap);
-                    acc[r] = MM::mma(m < P.M && cl + q < P.Cg ? wv : 0.f, b, acc[r]);
+                    acc[r] = MM::mma(m < P.M && cl + mq < P.Cg ? wv : 0.f, b, acc[r]);
                 }
             }
             next_tap<2>(P, kk);
@@ -219,7 +244,10 @@ __global__ __launch_bounds__(512) void plain_conv_kernel(Params P, const float* 
     if (!valid) return;
 #pragma unroll
     for (int r = 0; r < RW; ++r)
-        store_tile<float, float>(P, out + (size_t)P.C_out * P.outV * tg.n, bias, g, (int)(tile0 + r) * TN, q, pos, acc[r]);
+        store_tile<float, float>(P, out + (size_t)P.C_out * P.outV * tg.n, bias, g, (int)(tile0 + r) * TN, mq, pos, acc[r]);
 }
+
+using PlainKern = void (*)(Params, const float*, const Parts<float>::Vec*, const float*, const float*, float*);
+inline PlainKern plain_kernel(const PlainRows& r) { return r.rw == 2 ? plain_conv_kernel<2, 1> : r.mw == 4 ? plain_conv_kernel<1, 2> : plain_conv_kernel<1, 4>; }
 
 }  // namespace dcn

@@ -76,3 +76,37 @@ def test_plain_kernel():
     assert "dcn forward:" not in r.stdout
     for rows in ("1 wavefronts along the rows, 1 row", "2 wavefronts along the rows, 1 row", "4 wavefronts along the rows, 1 row", "4 wavefronts along the rows, 2 row"):
         assert rows in r.stdout
+
+
+# Layers of long sums that the kernel takes, of each variant; the other kernels share most of their positions among wavefronts or workgroups.  The last one's values are all positive.
+LONG = [(1, 47, 256, 69, 86, 3), (8, 19, 256, 14, 63, 3), (2, 45, 128, 40, 89, 3), (2, 21, 64, 67, 75, 5), (16, 440, 64, 50, 25, 3), (16, 23, 15, 78, 66, 3), (8, 374, 37, 33, 89, 1)]
+
+
+def long_sums():
+    import deform_conv3d_pytorch_op_amd as dcn
+    for n, (N, cin, cout, h, w, k) in enumerate(LONG):
+        torch.manual_seed(n)
+        x, wt = torch.randn(N, cin, h, w), torch.randn(cout, cin, k, k)
+        if n == len(LONG) - 1:
+            x, wt = x.abs(), wt.abs()
+        got = dcn.Conv2dFunction.apply(x.cuda(), wt.cuda(), None, 1, k // 2, 1, 1).cpu().double()
+        want = F.conv2d(x.double(), wt.double(), None, 1, k // 2)
+        print("error %.4e" % ((got - want).norm() / want.norm()).item(), flush=True)
+
+
+def test_plain_kernel_is_as_exact_as_the_others():
+    """2-norm against float64, at most that of the kernels of the deformable layer (DCN_PLAIN=0), whose sums are those of the float32 operator."""
+    import os
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    errors = {}
+    for knob in ("0", "1"):
+        r = subprocess.run([sys.executable, "-u", "-c", "from tests.test_gpu_conv2d_layer import long_sums; long_sums()"], cwd=root,
+                           env=dict(os.environ, DCN_PLAIN=knob, DCN_TRACE_PLANS="1"), stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+        assert r.returncode == 0, r.stdout[-3000:]
+        errors[knob] = [float(l.split()[1]) for l in r.stdout.splitlines() if l.startswith("error ")]
+        assert len(errors[knob]) == len(LONG) and r.stdout.count("dcn plain convolution") == (len(LONG) if knob == "1" else 0)
+    print(errors, flush=True)
+    for spec, other, own in zip(LONG, errors["0"], errors["1"]):
+        assert own <= other, (spec, own, other)
